@@ -5,12 +5,14 @@
 // the natural operand order of v_mfma_f32_32x32x16_f16: every lane feeds 8 consecutive k of one
 // row of lhs (A) and of one row of W (B).
 //
-// Two kernels:
-//   gemm_dl_kernel (K a multiple of 128, every shape of the model family): both operands travel
+// Three kernels:
+//   gemm_tile_kernel (gemm_tile.hpp): 256-row tiles of 128, 192 or 256 columns where these fill most of the
+//     chip, and 256x128 with the K range split over workgroups; fp16 and bfloat16 operands
+//   gemm_dl_kernel (K a multiple of 128, every other shape of the model family): both operands travel
 //     from global memory straight into a ring of 2-3 LDS stages with global_load_lds_dwordx4 (no
 //     staging registers, no LDS store instructions); rows are unpadded and the 16-byte chunks of a
 //     row are permuted so that neither the requests nor the fragment reads meet in a bank; tiles
-//     of 256x128, 128x128 or 128x64 with 4 or 8 wavefronts (a second group of four may take the
+//     of 256x128 (uint8), 128x128 or 128x64 with 4 or 8 wavefronts (a second group of four may take the
 //     other half of a 128-wide K stage), chosen by how many tiles the product has; uint8 weights
 //     add a ring of codes and of scales and are turned into fp16 -- exactly fp16((q - 127.5) *
 //     scale), llama_cu.cu:287-289 -- once per block tile; with 2..64 rows, and with few large tiles
@@ -25,6 +27,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemm_tile.hpp"
 #include "linear.hpp"
 
 using namespace lcu;
@@ -39,16 +42,6 @@ namespace {
 
 constexpr int BK = 64;        // K extent one group of four wavefronts multiplies per stage
 constexpr int NUM_XCD = 8;
-
-// Up to three products lhs * W_g^T with weight matrices of one shape in a single launch (Wq, Wk,
-// Wv; W1, W3): the tile index along N runs through matrix 0, then 1, then 2, `tiles_n_per` tiles
-// each.  Matrix 0 travels in the kernel's ordinary arguments, the others here.
-struct more_matrices_t {
-  half_t* out[2];
-  const void* W[2];
-  const half_t* S[2];
-  int tiles_n_per;  // tiles along N of one matrix; 0: a single matrix
-};
 
 __device__ __forceinline__ half2_t dequant2(uint32_t spread, half2_t scale2x) {
   const uint32_t bits = (spread << 2) | 0x58005800u;                                  // 128 + q/2
@@ -332,11 +325,6 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(
 // Per iteration: wait until this wavefront's loads of stage t have landed, barrier (so everybody's
 // have), request stage t+NS-1 into the slot whose reads ended before that barrier, multiply
 // stage t.  The compiler does not track these loads against LDS reads; the waits are explicit.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // WM x WN wavefronts tile the block (each a (BM/WM) x (BN/WN) sub-tile of 32x32 matrix-instruction
 // tiles), times KS groups along K.
 //
@@ -360,10 +348,6 @@ __device__ __forceinline__ void wait_vmcnt() {
 // epilogues (linear.hpp) take bfloat16 operands, which travel exactly like the fp16 ones, through
 // v_mfma_f32_32x32x16_bf16, and end in a bias, a GELU, or a clamped gate; GROUPED ones take the
 // rows of a tile and its weight matrix from a tile list on the device (lcu_experts_plan).
-struct f16_epilogue {
-  static constexpr bool BF16 = false, GROUPED = false;
-};
-
 template <int BM, int BN, int WM, int WN, int KS, int NS, bool U8, bool SPLIT = false, class EP = f16_epilogue>
 __global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS <= 4 ? 2 : 1) void gemm_dl_kernel(
     half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0,
@@ -911,6 +895,52 @@ int launch_dl(operands_t op, const half_t* A, int M, int K, int N, int block, fl
   return LCU_OK;
 }
 
+// A launch of gemm_tile_kernel; splits > 1: the K stages of every tile dealt to that many workgroups, fp32 sums to part.
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, class EP>
+int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N, float beta, hipStream_t st, int splits = 1,
+                float* part = nullptr) {
+  using shape = tile_shape<BM, BN, WM, WN, NS, SPLIT, EP>;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n_per = (N + BN - 1) / BN, tiles_n = tiles_n_per * op.n_mats;
+  op.more.tiles_n_per = op.n_mats > 1 ? tiles_n_per : 0;
+  auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NS, SPLIT, EP>;
+  static bool raised[16] = {};  // per device, once
+  int dev = 0;
+  LCU_HIP(hipGetDevice(&dev));
+  if (!raised[dev & 15]) {
+    LCU_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, shape::LDS));
+    raised[dev & 15] = true;
+  }
+  kernel<<<tiles_m * tiles_n * splits, 64 * WM * WN, shape::LDS, st>>>(op.out, (const half_t*)A, op.W, M, K, N, beta, tiles_m, tiles_n, part,
+                                                                       splits, op.more, ep);
+  LCU_LAUNCH_CHECK();
+  return LCU_OK;
+}
+
+// Columns of the 256-row tile of a product that fills most of the chip with them: the one whose rounds of workgroups
+// cost least, a round of 128 / 192 / 256 columns taking 57 / 88 / 106 us at K = 4096 (512 rows, W1 and W3 of 11008
+// columns in one launch: 230 tiles of 192 columns 88 us, 172 of 256 94 us, 344 of 128 108 us; 1987 rows: 303 us with 256
+// columns, 330 us with 128).  Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts.
+inline int large_tile_columns(int M, int N, int n_mats, long cus, bool gated) {
+  const auto cost = [&](int columns, int round) {
+    const long tiles = (long)((M + 255) / 256) * ((N + columns - 1) / columns) * n_mats;
+    return (tiles + cus - 1) / cus * round;
+  };
+  const long c128 = cost(128, 57), c192 = gated ? c128 : cost(192, 88), c256 = cost(256, 106);
+  if (c256 < c128 && c256 <= c192) return 256;
+  return c192 < c128 ? 192 : 128;
+}
+
+template <class EP>
+int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N, float beta, hipStream_t st) {
+  device_state* ds = current_device_state();
+  const int columns = large_tile_columns(M, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
+  if (columns == 256) return launch_tile<256, 256, 2, 2, 2, false>(ep, op, A, M, K, N, beta, st);
+  if constexpr (!EP::GATED) {
+    if (columns == 192) return launch_tile<256, 192, 2, 2, 2, false>(ep, op, A, M, K, N, beta, st);
+  }
+  return launch_tile<256, 128, 4, 2, 3, false>(ep, op, A, M, K, N, beta, st);
+}
+
 // where a split-K launch left its partial sums: part[matrix][split][M][N] fp32
 struct partial_sums_t {
   const float* part;
@@ -1004,6 +1034,16 @@ inline int large_tile_splits(int M, int K, int N, int n_mats, long cus, size_t w
     return 0;
   }
   return (int)splits;
+}
+
+int launch_large_split(operands_t op, const half_t* A, int M, int K, int N, float beta, hipStream_t st, int splits, float* part) {
+  const int rc = launch_tile<256, 128, 4, 2, 3, true>(f16_epilogue{}, op, A, M, K, N, beta, st, splits, part);
+  if (rc != LCU_OK) return rc;
+  const size_t mn = (size_t)M * N;
+  splitk_reduce_kernel<<<dim3((unsigned)((mn + 1023) / 1024), op.n_mats), 256, 0, st>>>(op.out, op.more.out[0], op.more.out[1], part, mn,
+                                                                                        splits, beta);
+  LCU_LAUNCH_CHECK();
+  return LCU_OK;
 }
 
 // The direct-to-LDS kernels fetch a thread's fp16 scale as the aligned 4-byte word that holds it:
@@ -1232,12 +1272,11 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
   // with two groups of four wavefronts splitting the K stage, because then the grid cannot give a
   // compute unit a second workgroup (M = 512, N = 4096: 35 us against 41 us, K = 11008: 100 us
   // against 135 us with the register-staged kernel).
-  // Several matrices of one shape (op.n_mats > 1) count as one product with n_mats * N columns --
-  // unless each of them already fills the chip with 256x128 tiles and fusing saves no round of
-  // workgroups (W1 + W3 at M = 512, N = 11008: 344 tiles take two rounds either way, and the fused
-  // launch measured 132 us against 2 x 63 us).
+  // Several matrices of one shape (op.n_mats > 1) count as one product with n_mats * N columns -- with
+  // uint8 weights unless each of them already fills the chip with 256x128 tiles and fusing saves no
+  // round of workgroups (fp16 weights choose a wider tile there, large_tile_columns).
   const bool whole_stages = K % 128 == 0 && scale_words_ok<U8>(op, K, N, block);
-  if (op.n_mats > 1 && M > 64 && whole_stages) {
+  if (U8 && op.n_mats > 1 && M > 64 && whole_stages) {
     device_state* ds = current_device_state();
     const long cus = ds && ds->compute_units > 0 ? ds->compute_units : 256;
     const long per = (long)((M + 255) / 256) * ((N + 127) / 128);
@@ -1271,14 +1310,24 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
   }
   if (whole_stages) {  // whole stages: the direct-to-LDS kernels
     const long tiles256 = (long)((M + 255) / 256) * ((N + 127) / 128) * nm;
-    if (tiles256 >= 160) return launch_dl<256, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+    if (tiles256 >= 160) {
+      if constexpr (U8) {
+        return launch_dl<256, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+      } else {
+        return launch_large(f16_epilogue{}, op, A, M, K, N, beta, st);
+      }
+    }
     {
       device_state* ds = current_device_state();
       const workspace_t ws = workspace_for(st);
       if (ds != nullptr && ws.ptr != nullptr) {
         const int splits = large_tile_splits(M, K, N, op.n_mats, ds->compute_units > 0 ? ds->compute_units : 256, ws.bytes);
         if (splits > 0) {
-          return launch_split<256, 128, 4, 2, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
+          if constexpr (U8) {
+            return launch_split<256, 128, 4, 2, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
+          } else {
+            return launch_large_split(op, A, M, K, N, beta, st, splits, (float*)ws.ptr);
+          }
         }
       }
     }
@@ -1398,7 +1447,7 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     if (rc != LCU_OK || done) return rc;
     return launch_bf16<64, 64, 2, GATED ? 1 : 2, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   }
-  if (tm(256) * tn(128) >= 160) return launch_bf16<256, 128, 4, 2, 1, 3>(ep, A, W, tm(256), M, K, N, st);
+  if (tm(256) * tn(128) >= 160) return launch_large(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0.0f, st);
   if (tm(128) * tn(128) > 256) return launch_bf16<128, 128, 2, 2, 1, 2>(ep, A, W, tm(128), M, K, N, st);
   if (tm(128) * tn(128) >= 160) return launch_bf16<128, 128, 4, 2, 1, 3>(ep, A, W, tm(128), M, K, N, st);
   if constexpr (GATED) {

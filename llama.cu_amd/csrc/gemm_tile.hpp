@@ -1,0 +1,304 @@
+// Large tiles of a matrix product with many rows: out[M,N] = lhs[M,K] * W[N,K]^T, fp16 or bfloat16 operands, sums
+// in fp32 over ascending k.
+//
+// What bounds it: the chip's power, and behind it the way from L2 into LDS.  On random operands the matrix
+// cores alone, fed from registers, reach 1.64 PFLOP/s (4096^3: 84 us; 70 us on zeros); with the operands on
+// their way through LDS this kernel takes 106 us there (1.30 PFLOP/s; 81 us on zeros).  So the design saves
+// what costs energy or makes a wavefront wait:
+//  * v_mfma_f32_16x16x32 instead of 32x32x16: half the accumulator traffic per multiply-add (4096^3 with 256x128
+//    tiles 133 -> 119 us).  Both take their products eight at a time in ascending k, so the bits are the same.
+//  * neighbouring instructions share an operand, also where the row of tiles changes (boustrophedon order).
+//  * a half stage (32 of K) of fragments is read from LDS while the half before it is multiplied, one read
+//    between two matrix instructions; requests for the stage NS ahead go out the same way.
+//  * requests are buffer loads straight into LDS whose stage offset is a scalar.  Behind the last stage the
+//    resource holds no records: the request counts as any other but touches no memory, so that the loop has one
+//    form up to the end and its registers are never copied.
+//  * outputs go through LDS and leave in 16-byte pieces.
+// LDS stage: rows of 128 bytes, lhs tile then W tile, 16-byte chunk g of row r at position g ^ (r / 2) % 8, so that
+// neither requests (1 KB per instruction, dense) nor fragment reads (16 rows, one chunk) meet in a bank.
+#pragma once
+#include <type_traits>
+
+#include "linear.hpp"
+
+namespace lcu {
+
+// Up to three products lhs * W_g^T with weight matrices of one shape in a single launch (Wq, Wk,
+// Wv; W1, W3): the tile index along N runs through matrix 0, then 1, then 2, `tiles_n_per` tiles
+// each.  Matrix 0 travels in the kernel's ordinary arguments, the others here.
+struct more_matrices_t {
+  half_t* out[2];
+  const void* W[2];
+  const half_t* S[2];
+  int tiles_n_per;  // tiles along N of one matrix; 0: a single matrix
+};
+
+struct f16_epilogue {
+  static constexpr bool BF16 = false, GROUPED = false, GATED = false;
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// the buffer resource of an operand below 4 GiB
+__device__ __forceinline__ uint4_t operand_resource(const void* p) {
+  const uintptr_t a = (uintptr_t)p;
+  uint4_t r;
+  r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
+  r[2] = 0xffffffffu;
+  r[3] = 0x00020000u;
+  return r;
+}
+
+// WM x WN wavefronts of (BM / WM) x (BN / WN) outputs each, a ring of NS stages of 64 along K.
+// SPLIT: the grid holds `splits` workgroups per tile, each taking a contiguous run of the K stages and writing its
+// fp32 sums to part[split][M][N].
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, class EP>
+struct tile_shape {
+  static constexpr int NW = WM * WN, WR = BM / WM, WC = BN / WN;
+  static constexpr int STAGE = (BM + BN) * 128;
+  static constexpr int OUT_LD = WC + 4;                  // floats per row of a wavefront's 64 output rows in LDS
+  static constexpr int RING = NS * STAGE, OUT = NW * 64 * OUT_LD * 4;
+  static constexpr int LDS = RING > OUT ? RING : OUT;
+  static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 32 == 0, "tile");
+};
+
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, class EP>
+__global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
+    half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, int M, int K, int N, float beta, int tiles_m,
+    int tiles_n, float* __restrict__ part, int splits, more_matrices_t more, EP ep) {
+  using shape = tile_shape<BM, BN, WM, WN, NS, SPLIT, EP>;
+  static_assert(!EP::GROUPED, "one matrix for all rows");
+  constexpr int NW = shape::NW;
+  constexpr int TM = shape::WR / 16, TN = shape::WC / 16;        // 16x16 tiles of a wavefront
+  constexpr int PA = BM / 8 / NW, PB = BN / 8 / NW, P = PA + PB;  // requests of a wavefront per stage
+  constexpr int A_BYTES = BM * 128, STAGE = shape::STAGE;
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && NS >= 2 && P * (NS - 1) < 64, "requests");
+  extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
+
+  // consecutive workgroups go round the eight XCDs: each gets one run of the M-fastest tile sequence, so that
+  // tiles that share a slice of W share an L2
+  const int nb = tiles_m * tiles_n;
+  const int split = SPLIT ? blockIdx.x / nb : 0;
+  const int bx = SPLIT ? blockIdx.x - split * nb : blockIdx.x;
+  const int q = nb / 8, r = nb % 8, xcd = bx % 8;
+  const int logical = xcd * q + min(xcd, r) + bx / 8;
+  const int tm = logical % tiles_m;
+  int tn = logical / tiles_m;
+  half_t* out = out0;
+  const void* W = W0;
+  if (more.tiles_n_per > 0) {
+    const int g = tn / more.tiles_n_per;
+    tn -= g * more.tiles_n_per;
+    out = g == 0 ? out0 : (g == 1 ? more.out[0] : more.out[1]);
+    W = g == 0 ? W0 : (g == 1 ? more.W[0] : more.W[1]);
+    if constexpr (SPLIT) part += (size_t)g * splits * M * N;  // each matrix has its own partial sums
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave % WM) * shape::WR, wn = (wave / WM) * shape::WC;
+
+  // this workgroup's K stages
+  const int nt_all = K / 64;
+  const int stage0 = SPLIT ? (int)((long)split * nt_all / splits) : 0;
+  const int nt = SPLIT ? (int)((long)(split + 1) * nt_all / splits) - stage0 : nt_all;
+
+  // request j of this wavefront fills LDS bytes [(wave + j * NW) * 1024, + 1024) of an operand's part of a stage.
+  // Rows past M or N are clamped to the last one: their sums are never stored.
+  uint32_t a_off[PA], b_off[PB];
+#pragma unroll
+  for (int j = 0; j < PA; ++j) {
+    const int c = (wave + j * NW) * 64 + lane, row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
+    a_off[j] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)K + g * 8) * 2u;
+  }
+#pragma unroll
+  for (int j = 0; j < PB; ++j) {
+    const int c = (wave + j * NW) * 64 + lane, row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
+    b_off[j] = ((uint32_t)min(n0 + row, N - 1) * (uint32_t)K + g * 8) * 2u;
+  }
+  uint4_t ra = operand_resource(A), rw = operand_resource(W);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)tile_lds;
+  // Inline assembly, so that the compiler does not know about the LDS writes: knowing, it waits for every LDS read
+  // in front of each matrix instruction.  There is no output register; the waits are the explicit ones below.
+  const auto request = [&](uint4_t resource, uint32_t stage_bytes, uint32_t offset, uint32_t at) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(offset), "s"(resource), "s"(stage_bytes),
+                 "s"(lds0 + at)
+                 : "memory", "m0");
+  };
+  const auto issue = [&](int stage, int slot, int i) {
+    const uint32_t along = (uint32_t)(stage0 + stage) * 128u;
+    if (i < PA) {
+      request(ra, along, a_off[i], slot * STAGE + (wave + i * NW) * 1024);
+    } else {
+      request(rw, along, b_off[i - PA], slot * STAGE + A_BYTES + (wave + (i - PA) * NW) * 1024);
+    }
+  };
+
+  float4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = (float4_t)(0.0f);
+  }
+  const int frag_row = lane & 15, frag_chunk = lane >> 4, turn = (frag_row / 2) % 8;
+  uint32_t pos[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) pos[h] = (uint32_t)(((frag_chunk + 4 * h) ^ turn) * 16);
+  const uint32_t a_row = (uint32_t)(wm + frag_row) * 128, b_row = (uint32_t)A_BYTES + (uint32_t)(wn + frag_row) * 128;
+  half8_t fa[2][TM], fb[2][TN];
+  constexpr int READS = TM + TN, PRODUCTS = TM * TN;
+  const auto read = [&](int slot, int h, int i) {
+    const unsigned char* p = tile_lds + slot * STAGE + pos[h];
+    if (i < TN) {
+      fb[h][i] = *reinterpret_cast<const half8_t*>(p + b_row + i * 2048);
+    } else {
+      fa[h][i - TN] = *reinterpret_cast<const half8_t*>(p + a_row + (i - TN) * 2048);
+    }
+  };
+  const auto multiply = [&](int h, int i) {
+    const int a = i / TN, b = (a & 1) ? TN - 1 - i % TN : i % TN;
+    if constexpr (EP::BF16) {
+      acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fa[h][a]), __builtin_bit_cast(bf16x8_t, fb[h][b]),
+                                                          acc[a][b], 0, 0, 0);
+    } else {
+      acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[h][a], fb[h][b], acc[a][b], 0, 0, 0);
+    }
+  };
+  // the products of half h, with the reads spread over the first five eighths and the requests over all of them
+  const auto half_stage = [&](int h, auto n_reads, auto&& do_read, auto n_requests, auto&& do_request) {
+    constexpr int NR = decltype(n_reads)::value, NQ = decltype(n_requests)::value, SPREAD = PRODUCTS * 5 / 8;
+#pragma unroll
+    for (int i = 0; i < PRODUCTS; ++i) {
+      multiply(h, i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i < SPREAD) {
+#pragma unroll
+        for (int k = i * NR / SPREAD; k < (i + 1) * NR / SPREAD; ++k) do_read(k);
+      }
+#pragma unroll
+      for (int k = i * NQ / PRODUCTS; k < (i + 1) * NQ / PRODUCTS; ++k) do_request(k);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // One stage in ring slot `slot`: multiply its first half while the second is read; this wavefront has then read
+  // the whole stage, and once its own requests of the next stage have landed (at most those of NS - 2 later stages
+  // outstanding) the barrier says both for everybody.  Then the second half, with the next stage's first half on its
+  // way from slot `next_slot` and the stage NS ahead requested into `slot`.
+  const auto stage = [&](int slot, int next_slot, int ahead, auto more_follow) {
+    constexpr bool MORE = decltype(more_follow)::value;
+    half_stage(0, std::integral_constant<int, READS>{}, [&](int k) { read(slot, 1, k); }, std::integral_constant<int, 0>{}, [](int) {});
+    if constexpr (MORE) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      wait_vmcnt<(NS - 2) * P>();
+      asm volatile("s_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      half_stage(1, std::integral_constant<int, READS>{}, [&](int k) { read(next_slot, 0, k); }, std::integral_constant<int, P>{},
+                 [&](int k) { issue(ahead, slot, k); });
+    } else {
+      half_stage(1, std::integral_constant<int, 0>{}, [](int) {}, std::integral_constant<int, 0>{}, [](int) {});
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if (s == nt) ra[2] = rw[2] = 0;  // no records: a request brings zeros and reads nothing
+#pragma unroll
+    for (int i = 0; i < P; ++i) issue(s, s, i);
+  }
+  wait_vmcnt<(NS - 1) * P>();
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < READS; ++i) read(0, 0, i);
+  __builtin_amdgcn_sched_barrier(0);
+  int slot = 0;
+  for (int t = 0; t < nt - 1; ++t) {
+    if (t + NS == nt) ra[2] = rw[2] = 0;
+    const int next_slot = slot + 1 == NS ? 0 : slot + 1;
+    stage(slot, next_slot, t + NS, std::true_type{});
+    slot = next_slot;
+  }
+  stage(slot, 0, 0, std::false_type{});
+  wait_vmcnt<0>();  // the requests behind the last stage have written their zeros
+  __syncthreads();  // LDS is free
+
+  // ---- epilogue, 64 rows of the wavefront's tile at a time.  Register v of lane l holds row 4 (l / 16) + v, column
+  // l % 16 of a 16x16 tile.
+  float* rows = reinterpret_cast<float*>(tile_lds) + wave * 64 * shape::OUT_LD;
+  constexpr int OC = EP::GATED ? shape::WC / 2 : shape::WC;  // output columns of the wavefront
+  constexpr int PIECES = OC / 8;                             // pieces of eight columns per row, and per lane
+  const int out_n0 = EP::GATED ? (n0 + wn) / 2 : n0 + wn, out_n = EP::GATED ? N / 2 : N;
+  const bool whole = !EP::BF16 && !SPLIT && N % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;  // 16-byte rows
+  const auto pass = [&](auto which) {
+    constexpr int p = decltype(which)::value;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float* to = rows + (i * 16 + (lane >> 4) * 4 + v) * shape::OUT_LD + (lane & 15);
+        if constexpr (EP::GATED) {
+          // 64 columns are 32 gate rows of the matrix, then the 32 up rows that they belong to
+          static_assert(TN % 4 == 0, "whole gate / up pairs");
+#pragma unroll
+          for (int j = 0; j < TN; j += 4) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) to[(j / 2 + e) * 16] = ep.gate(acc[p * 4 + i][j + e][v], acc[p * 4 + i][j + 2 + e][v]);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) to[j * 16] = acc[p * 4 + i][j][v];
+        }
+      }
+    }
+    constexpr int AT_ONCE = PIECES % 4 == 0 ? 4 : 2;
+#pragma unroll 1
+    for (int k0 = 0; k0 < PIECES; k0 += AT_ONCE) {
+      half8_t old[AT_ONCE];
+      if constexpr (!EP::BF16 && !SPLIT) {
+        if (beta != 0.0f && whole) {
+#pragma unroll
+          for (int k = 0; k < AT_ONCE; ++k) {
+            const int c = lane + 64 * (k0 + k), gm = m0 + wm + p * 64 + c / PIECES, gn = out_n0 + c % PIECES * 8;
+            if (gm < M && gn < N) old[k] = *reinterpret_cast<const half8_t*>(out + (size_t)gm * N + gn);
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) {
+        const int c = lane + 64 * (k0 + k), gm = m0 + wm + p * 64 + c / PIECES, gn = out_n0 + c % PIECES * 8;
+        const float* from = rows + (c / PIECES) * shape::OUT_LD + c % PIECES * 8;
+        const float4_t lo = *reinterpret_cast<const float4_t*>(from), hi = *reinterpret_cast<const float4_t*>(from + 4);
+        const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        if (gm >= M || gn >= out_n) continue;
+        if constexpr (SPLIT) {
+          float* to = part + ((size_t)split * M + gm) * N + gn;
+          if (N % 4 == 0 && gn + 8 <= N) {
+            *reinterpret_cast<float4_t*>(to) = lo;
+            *reinterpret_cast<float4_t*>(to + 4) = hi;
+          } else {
+            for (int e = 0; e < 8 && gn + e < N; ++e) to[e] = x[e];
+          }
+        } else if constexpr (EP::BF16) {
+          ep.store8(gm, gn, x, out_n);
+        } else {
+          half_t* to = out + (size_t)gm * N + gn;
+          if (whole) {  // llama_cu.cu:208-215: fp16(acc + beta * old)
+            half8_t y;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = round_f16(beta != 0.0f ? fmaf(beta, (float)old[k][e], x[e]) : x[e]);
+            *reinterpret_cast<half8_t*>(to) = y;
+          } else {
+            for (int e = 0; e < 8 && gn + e < N; ++e) to[e] = round_f16(beta != 0.0f ? fmaf(beta, (float)to[e], x[e]) : x[e]);
+          }
+        }
+      }
+    }
+  };
+  pass(std::integral_constant<int, 0>{});
+  if constexpr (shape::WR > 64) pass(std::integral_constant<int, 1>{});
+  static_assert(shape::WR <= 128, "passes");
+}
+
+}  // namespace lcu

@@ -68,6 +68,41 @@ struct linear_epilogue {
     }
     put(m, n, v);
   }
+  // eight neighbouring columns of `columns`, from a multiple of eight on: in 16-byte pieces where rows allow them
+  __device__ __forceinline__ void store8(int m, int n, const float (&x)[8], int columns) const {
+    const bool wide = n + 8 <= columns && (!tail || n + 8 <= tail_from) && ldo % (out_f32 ? 4 : 8) == 0 &&
+                      (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    if (!wide) {
+      for (int e = 0; e < 8 && n + e < columns; ++e) {
+        if constexpr (GATED) {
+          put(m, n + e, x[e]);
+        } else {
+          store(m, n + e, x[e]);
+        }
+      }
+      return;
+    }
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      y[e] = x[e];
+      if constexpr (!GATED) {
+        if (bias) y[e] += bias[n + e];
+        if (n + e < gelu_cols) y[e] = gelu_tanh(y[e]);
+      }
+    }
+    const size_t at = (size_t)m * ldo + n;
+    if (out_f32) {
+      float4_t* to = reinterpret_cast<float4_t*>(reinterpret_cast<float*>(out) + at);
+      to[0] = float4_t{y[0], y[1], y[2], y[3]};
+      to[1] = float4_t{y[4], y[5], y[6], y[7]};
+    } else {
+      bf16x8_t v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = (bf16_t)y[e];
+      *reinterpret_cast<bf16x8_t*>(reinterpret_cast<bf16_t*>(out) + at) = v;
+    }
+  }
   __device__ __forceinline__ void store_gated(int m, int n, float g, float u) const {
     const float s = row_scale ? row_scale[m] : 1.0f;
     put(m, n, gate(g * s, u * s));

@@ -36,6 +36,44 @@ def test_linear_with_bias_and_gelu_columns(gpu, dt, M, K, N):
     gpu.release()
 
 
+# tiles of 256 rows in bfloat16: 192 columns with ragged rows and columns, 256 columns and a single K stage, 128 columns;
+# the last four columns as fp32 of their own
+@pytest.mark.parametrize("M,K,N", [(2049, 192, 4100), (4096, 64, 4096), (300, 320, 12804)])
+def test_linear_large_tiles(gpu, M, K, N):
+    rng = np.random.default_rng(N)
+    x, w, b = rounded(rng.standard_normal((M, K))), rounded(rng.standard_normal((N, K)) / K ** 0.5), rng.standard_normal(N)
+    xd, wd, ldo, tail = put(gpu, x, BF16), put(gpu, w, BF16), up64(N), 4
+    want = x @ w.T + b
+    want[:, :100] = S.gelu_tanh(want[:, :100])
+    out = zeros(gpu, (M, ldo), BF16)
+    call(gpu, "lcu_linear", out, 0, ldo, xd, wd, put(gpu, b), 100, BF16, M, K, N)
+    got = get(gpu, out, (M, ldo), BF16)
+    close(got[:, :N], want, BF16)
+    assert (got[:, N:] == 0).all()
+    last = zeros(gpu, (M, tail))
+    out = zeros(gpu, (M, ldo), BF16)
+    call(gpu, "lcu_linear_tail", out, ldo, last, tail, N - tail, xd, wd, BF16, M, K, N)
+    close(get(gpu, out, (M, ldo), BF16)[:, :N - tail], (x @ w.T)[:, :-tail], BF16)
+    close(get(gpu, last, (M, tail)), (x @ w.T)[:, -tail:], F32)
+    out = zeros(gpu, (M, N + 1))
+    call(gpu, "lcu_linear", out, 1, N + 1, xd, wd, None, 0, BF16, M, K, N)   # rows off any 16-byte boundary
+    close(get(gpu, out, (M, N + 1))[:, :N], x @ w.T, F32)
+    gpu.release()
+
+
+@pytest.mark.parametrize("M,K,ff", [(4096, 64, 2048), (2050, 128, 4100)])
+def test_gated_linear_large_tiles(gpu, M, K, ff):
+    rng = np.random.default_rng(ff)
+    x, gw, uw = rounded(rng.standard_normal((M, K))), rounded(rng.standard_normal((ff, K)) / K ** 0.5), \
+        rounded(rng.standard_normal((ff, K)) / K ** 0.5)
+    ld = up64(ff)
+    out = zeros(gpu, (M, ld), BF16)
+    gate = gpu.B.GateParams(0.75, 1.702, 1.0)
+    call(gpu, "lcu_linear_gated", out, ld, put(gpu, x, BF16), put(gpu, pack_gated(gw, uw, ld), BF16), C.byref(gate), BF16, M, K, 2 * ld)
+    close(get(gpu, out, (M, ld), BF16)[:, :ff], S.expert(x, gw, uw, np.eye(ff), 0.75), BF16)
+    gpu.release()
+
+
 @BOTH
 @pytest.mark.parametrize("M,K,ff", [(1, 64, 32), (5, 128, 40), (66, 192, 100), (200, 128, 640), (700, 64, 1000), (2, 1024, 70), (40, 768, 500)])
 def test_gated_linear_clamps(gpu, dt, M, K, ff):

@@ -200,6 +200,18 @@ def test_gemm_f16(gpu, M, K, N):
     G.release()
 
 
+# tiles of 256 rows at their edges: 192 columns with rows of 4 halves past a 16-byte boundary, 256 columns, 128 columns of one
+# row and column beyond a tile, and K split over workgroups with rows of 2 floats past one; a single K stage pair and many
+@pytest.mark.parametrize("M,K,N", [(2049, 128, 4100), (4096, 256, 4090), (257, 384, 12929), (300, 5120, 1030)])
+def test_gemm_f16_large_tiles_ragged(gpu, M, K, N):
+    G = gpu
+    x, w, old = normal((M, K), 0, 320, 1.0), normal((N, K), 0, 321, 0.02), normal((M, N), 0, 322, 1.0)
+    assert G.ulp_mismatch(G.gemm_f16(x, w), O.matmul_nt(x, w, flavour=2)) == 0.0, O.gemm_plan(M, K, N)
+    got = G.gemm_f16(x, w, beta=1.0, out=old)
+    assert G.ulp_mismatch(got, O.matmul_nt(x, w, beta=1.0, out=old, flavour=2)) == 0.0
+    G.release()
+
+
 def test_gemm_residual_into_an_output_that_is_not_16_byte_aligned(gpu):
     """beta = 1 with the output tile 8 bytes off a 16-byte boundary: the tile that fetches its old values in 16-byte
     pieces (512 x 4096 x 4096, the Wo product) must fall back to 2-byte reads; same bits as the aligned call."""
