@@ -1054,6 +1054,279 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   }
 }
 
+// ---- prompts -------------------------------------------------------------------------------------
+// exp_ieee for x <= 0 (and NaN): the scaling by 2^k in one step, k's bits taken from the sum that rounds to it.
+// The same bits for every x in [-104, 0] and below, in two thirds of the instructions.
+__device__ __forceinline__ float exp_ieee_nonpositive(float x) {
+  const float magic = x * 1.44269504f + 12582912.0f;
+  const float kf = magic - 12582912.0f;
+  float r = fmaf(kf, -0.693359375f, x);
+  r = fmaf(kf, 2.12194440e-4f, r);
+  float p = 1.9875691500e-4f;
+  p = fmaf(p, r, 1.3981999507e-3f);
+  p = fmaf(p, r, 8.3334519073e-3f);
+  p = fmaf(p, r, 4.1665795894e-2f);
+  p = fmaf(p, r, 1.6666665459e-1f);
+  p = fmaf(p, r, 5.0000001201e-1f);
+  p = fmaf(p * r, r, r) + 1.0f;
+  const float scale = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, magic) << 23) + 0x3f800000u);
+  return x < -87.33654f ? 0.0f : p * scale;
+}
+
+// x / d from the correctly rounded reciprocal of d: quotient, exact remainder, correction.  Correctly rounded
+// for finite x and normal results; what is below the normal numbers is 0 in fp16 either way.
+__device__ __forceinline__ float divide_by(float x, float d, float reciprocal) {
+  const float q = x * reciprocal;
+  return fmaf(fmaf(-q, d, x), reciprocal, q);
+}
+
+// Attention of many rows: NW wavefronts of 16 rows each share the K and V of their head in chunks of 64 cache rows,
+// which travel into a ring of four 16 KB LDS slots, three ahead.
+//
+// What bounds it is vector instructions: a score that is rounded to fp16, exponentiated and divided where the
+// reference does takes about 50 of them.  So scores are never stored: they are computed three times (the matrix
+// cores have room), for the maximum, for the sum and for the probabilities, and LDS holds no strip of scores, which at
+// 2000 rows left four wavefronts to a compute unit.  Scores are computed with cache rows as rows of the tile, in an
+// order that leaves a lane eight consecutive ones of its query: the operand of the product with V as it stands, V
+// itself being transposed on its way out of LDS.
+// The sums are those of a wavefront per row: pair p = (column % 128) / 2 adds its two exponentials per 128 columns, then the
+// 64 pairs meet as in wave_sum (llama_cu.cu:433-499); the products with V are a chain over ascending cache rows.
+// 32 heads, n = T = 1987: 502 -> 154 us; 52 heads, n = T = 2048: 837 -> 242 us.
+template <int NW>
+__global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_t* __restrict__ out, const half_t* __restrict__ q,
+                                                                           const half_t* __restrict__ k, const half_t* __restrict__ v,
+                                                                           int n_new, int T, int start_pos, int dim, int n_tiles) {
+  constexpr int ROWS = 16 * NW, SLOT = 64 * HD * 2, R = 16 / NW;  // rows of a workgroup, bytes of a chunk, requests per wavefront
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  // the tiles that see most columns first
+  const int n_heads = gridDim.x / n_tiles;
+  const int tile = n_tiles - 1 - blockIdx.x / n_heads, h = blockIdx.x % n_heads;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = tile * ROWS, w0 = r0 + wave * 16;
+  const int chunks = (min(r0 + ROWS, n_new) + start_pos + 63) / 64;
+  // chunks that this wavefront's rows see, and from which one on columns have to be masked
+  const int own_chunks = w0 < n_new ? (min(w0 + 16, n_new) + start_pos + 63) / 64 : 0;
+  const int masked_from = (w0 + start_pos + 1) / 64;
+  const int row = lane & 15, group = lane >> 4;  // this lane's query, and which eight of 32 columns
+  const int limit = w0 + row + start_pos;        // last column it sees (llama_cu.cu:415)
+
+  half8_t qf[4];
+  // ---- the ring.  Items are K chunks (maximum), K chunks again (sum), then K and V chunks in turn.  A row of a chunk
+  // is 256 bytes; its 16-byte pieces are permuted by row so that neither fragment reads nor transposed reads of rows
+  // eight apart meet in a bank.
+  const int items = 4 * chunks;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  const auto turn_k = [](int r) { return (r & 3) | (((r >> 3) & 3) << 2); };
+  const auto turn_v = [](int r) { return ((r & 3) | (((r >> 3) & 1) << 2)) << 1; };
+  const auto issue = [&](int item) {
+    const bool is_v = item >= 2 * chunks && (item & 1) != 0;
+    const int c = item < chunks ? item : (item < 2 * chunks ? item - chunks : item / 2 - chunks);
+    const half_t* src = (is_v ? v : k) + h * HD;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int r = (wave + j * NW) * 4 + (lane >> 4);
+      const int piece = (lane & 15) ^ (is_v ? turn_v(r) : turn_k(r));
+      // rows past T are never used: their scores are masked, their probabilities 0
+      const half_t* from = src + (size_t)min(c * 64 + r, T - 1) * dim + piece * 8;
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from),
+                   "s"(lds0 + (item & 3) * SLOT + (wave + j * NW) * 1024)
+                   : "memory", "m0");
+    }
+  };
+  // item i is there for everybody, and item i + 3 on its way into the slot of item i - 1, which everybody has read
+  const auto acquire = [&](int item) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int behind = items - 1 - item;
+    if (behind >= 2) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * R) : "memory");
+    } else if (behind == 1) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    asm volatile("s_barrier" ::: "memory");
+    if (item + 3 < items) issue(item + 3);
+  };
+
+  // scores of chunk c: s[b][t][e] is column 64 c + 32 b + 8 group + 4 t + e of the lane's query.  Row m of tile (b, t) is
+  // cache row 32 b + 8 (m / 4) + 4 t + m % 4, and a lane's registers are rows 4 group + e.
+  const int key_row = 8 * (row >> 2) + (row & 3);
+  const uint32_t k_base = (uint32_t)key_row * 256;
+  const int k_turn = turn_k(key_row);
+  const auto products = [&](float4_t (&s)[2][2], int item) {
+    const unsigned char* slot = smem + (item & 3) * SLOT + k_base;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        s[b][t] = (float4_t)(0.0f);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const half8_t kf = *reinterpret_cast<const half8_t*>(slot + (32 * b + 4 * t) * 256 + (((d * 4 + group) ^ k_turn) * 16));
+          s[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[d], s[b][t], 0, 0, 0);
+        }
+      }
+    }
+  };
+  // the lowest finite value: scaled and rounded to fp16 it is the reference's -infinity
+  constexpr float MASKED = -3.402823466e38f;
+  const auto mask = [&](float4_t (&s)[2][2], int c) {
+    if (c < masked_from) return;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (c * 64 + 32 * b + 8 * group + 4 * t + e > limit) s[b][t][e] = MASKED;
+        }
+      }
+    }
+  };
+
+#pragma unroll
+  for (int i = 0; i < 3; ++i) issue(i);  // a tile has four items at least
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    qf[s] = *reinterpret_cast<const half8_t*>(q + (size_t)min(w0 + row, n_new - 1) * dim + h * HD + s * 32 + group * 8);
+  }
+  // arrived before the loops: a wait inside them would be for the chunks requested meanwhile too
+#pragma unroll
+  for (int s = 0; s < 4; ++s) asm volatile("" : "+v"(qf[s]));
+
+  // ---- maximum.  Rounding and division keep the order, so the largest product gives the largest score.
+  float m = -INFINITY, size = 0.0f;
+  for (int c = 0; c < chunks; ++c) {
+    acquire(c);
+    if (c >= own_chunks) continue;
+    float4_t s[2][2];
+    products(s, c);
+    mask(s, c);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      m = fmaxf(m, s[i >> 3][(i >> 2) & 1][i & 3]);
+      size = fmaxf(size, fabsf(s[i >> 3][(i >> 2) & 1][i & 3]));
+    }
+  }
+  m = fmaxf(m, __shfl_xor(m, 16, WAVE));
+  m = fmaxf(m, __shfl_xor(m, 32, WAVE));
+  const float denom = sqrtf((float)HD), inverse = 1.0f / denom;
+  // an infinite product (infinite operands) would leave NaN in the remainder: such rows are divided the long way
+  const bool plain = __ballot(size > -MASKED) == 0;
+  const auto scaled = [&](float x) { return (float)round_f16(plain ? divide_by(x, denom, inverse) : x / denom); };
+  m = scaled(m);
+  const auto scale = [&](float4_t (&s)[2][2]) {  // products to scores, which are fp16 values; one branch for all of them
+    if (plain) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float4_t& x = s[i >> 3][(i >> 2) & 1];
+        x[i & 3] = (float)round_f16(divide_by(x[i & 3], denom, inverse));
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float4_t& x = s[i >> 3][(i >> 2) & 1];
+        x[i & 3] = (float)round_f16(x[i & 3] / denom);
+      }
+    }
+  };
+
+  // ---- sum
+  float pairs[2][2][4] = {};  // [chunk & 1][b][pair]: pair index 32 (chunk & 1) + 16 b + 4 group + pair of 64
+  const auto add_chunk = [&](int c, float (&sum)[2][4]) {
+    acquire(chunks + c);
+    if (c >= own_chunks) return;
+    float4_t s[2][2];
+    products(s, chunks + c);
+    mask(s, c);
+    scale(s);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const float4_t x = s[b][p >> 1];
+        sum[b][p] += exp_ieee_nonpositive(x[2 * (p & 1)] - m) + exp_ieee_nonpositive(x[2 * (p & 1) + 1] - m);
+      }
+    }
+  };
+  for (int c = 0; c < chunks; c += 2) {
+    add_chunk(c, pairs[0]);
+    if (c + 1 < chunks) add_chunk(c + 1, pairs[1]);
+  }
+  float quarter[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const float(&p)[4] = pairs[b >> 1][b & 1];
+    float x = (p[0] + p[1]) + (p[2] + p[3]);
+    x += __shfl_xor(x, 16, WAVE);
+    x += __shfl_xor(x, 32, WAVE);
+    quarter[b] = x;
+  }
+  const float total = (quarter[0] + quarter[1]) + (quarter[2] + quarter[3]), share = 1.0f / total;
+
+  // ---- probabilities and their product with V: o[d] is columns 16 d + 4 group + e of the lane's query
+  float4_t o[HD / 16];
+#pragma unroll
+  for (int d = 0; d < HD / 16; ++d) o[d] = (float4_t)(0.0f);
+  // transposed read: lane i of sixteen gives four neighbouring columns of row i / 4 and receives column i of the four rows
+  const int v_row = 8 * group + (row >> 2), v_turn = turn_v(v_row);
+  const uint32_t v_base = (uint32_t)v_row * 256 + (row & 1) * 8;
+  typedef short short4_t __attribute__((ext_vector_type(4)));
+  for (int c = 0; c < chunks; ++c) {
+    const int item = 2 * chunks + 2 * c;
+    half8_t pf[2];
+    acquire(item);
+    if (c < own_chunks) {
+      float4_t s[2][2];
+      products(s, item);
+      mask(s, c);
+      scale(s);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pf[b][e] = round_f16(divide_by(exp_ieee_nonpositive(s[b][e >> 2][e & 3] - m), total, share));
+      }
+    }
+    acquire(item + 1);
+    if (c < own_chunks) {
+      const unsigned char* slot = smem + ((item + 1) & 3) * SLOT + v_base;
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+#pragma unroll
+        for (int d = 0; d < HD / 16; ++d) {
+          const unsigned char* at = slot + 32 * b * 256 + (((2 * d + ((row >> 1) & 1)) ^ v_turn) * 16);
+          union {
+            short4_t half[2];
+            half8_t all;
+          } vf;
+          vf.half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)at);
+          vf.half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(at + 4 * 256));
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf.all, pf[b], o[d], 0, 0, 0);
+        }
+      }
+    }
+  }
+  if (w0 + row < n_new) {
+    half_t* to = out + (size_t)(w0 + row) * dim + h * HD + 4 * group;
+#pragma unroll
+    for (int d = 0; d < HD / 16; ++d) {
+      half4_t y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = round_f16(o[d][e]);  // llama_cu.cu:529
+      *reinterpret_cast<half4_t*>(to + 16 * d) = y;
+    }
+  }
+}
+
+template <int NW>
+int launch_prompt_attention(half_t* out, const half_t* q, const half_t* k, const half_t* v, int n_new, int T, int start_pos, int dim,
+                            int n_heads, hipStream_t s) {
+  const int n_tiles = (n_new + 16 * NW - 1) / (16 * NW);
+  prompt_attention_kernel<NW><<<n_tiles * n_heads, 64 * NW, 4 * 64 * HD * 2, s>>>(out, q, k, v, n_new, T, start_pos, dim, n_tiles);
+  LCU_LAUNCH_CHECK();
+  return LCU_OK;
+}
+
 // ---- scores of long decode rows for callers that may not allocate --------------------------------
 // lcu_attention_decode_static keeps the fp16 scores of dec_scores_kernel in this array instead of
 // a workspace from hipMalloc: MAX_HEADS x MAX_T_DECODE halves = 512 KiB per GPU, held until the
@@ -1119,6 +1392,21 @@ int lcu_attention(void* out_dev, const void* q_dev, const void* k_dev, const voi
                                    nullptr, T, dim, n_heads, (half_t*)ws.ptr, s);
   }
   LCU_REQUIRE(T <= MAX_T_PREFILL, "lcu_attention: T %d exceeds %d for n_new > 1", T, MAX_T_PREFILL);
+  // Many scores: the kernel that computes them three times and stores none.  A wavefront of it walks all T columns
+  // alone, 3.9 us per 64 of them, while the kernel below shares a tile's columns among four wavefronts but is bound by
+  // what LDS holds from about 0.17 M scores per us on; the lines cross where the call has 11 000 scores per column
+  // (heads, n = T, us here against below: 32 heads 512 rows 35 / 24, 700 rows 47 / 44, 1024 rows 70 / 144, 1987 rows 154 / 502;
+  // 52 heads 512 rows 36 / 38; 4 heads 1500 rows 95 / 90; 32 heads 64 rows of 1000 66 / 39, 512 rows of 2048 129 / 214).
+  const double scores = (double)n_heads * n_new * (start_pos + 0.5 * n_new);
+  if (scores >= 11000.0 * T) {
+    // 128 rows to a workgroup read K and V half as often, if two workgroups per compute unit are left
+    if ((long)((n_new + 127) / 128) * n_heads >= 512) {
+      return launch_prompt_attention<8>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T,
+                                        start_pos, dim, n_heads, s);
+    }
+    return launch_prompt_attention<4>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T,
+                                      start_pos, dim, n_heads, s);
+  }
   // 16-row tiles when 32-row tiles would leave the grid under four workgroups per compute unit
   // and the rows are short (T <= 1024: 22 us against 29 us at n = T = 512, dim 4096); with long
   // rows the per-chunk overhead of the extra workgroups costs more than the balance gains.

@@ -659,6 +659,46 @@ def test_attention_llama7b_heads(gpu, n, T):
     G.release()
 
 
+# calls with enough scores for the kernel that stores none: ragged rows and columns, 64- and 128-row tiles, rows behind cached ones
+@pytest.mark.parametrize("heads,n,T", [(40, 601, 601), (64, 350, 385), (64, 900, 931), (52, 449, 450)])
+def test_attention_of_many_scores(gpu, heads, n, T):
+    G = gpu
+    dim, start = heads * 128, T - n
+    q, k, v = normal((n, dim), 0, 1020, 1.0), normal((T, dim), 0, 1021, 1.0), normal((T, dim), 0, 1022, 1.0)
+    out_d = G.empty((n, dim))
+    G.B.check(G.L().lcu_attention(out_d.ptr, G.dev_keep(q).ptr, G.dev_keep(k).ptr, G.dev_keep(v).ptr, n, T, start, dim, heads, None))
+    assert G.ulp_mismatch(G.host(out_d, (n, dim)), O.attention_prefill_kernel_order(q, k, v, heads, start)) == 0.0
+    G.release()
+
+
+def test_attention_of_many_scores_equals_portions(gpu):
+    """One call against portions of 16 rows, which take the other kernel: the same bits, also with scores past the
+    range of fp16, products past that of fp32 (infinite operands), NaN, and rows that see equal scores only."""
+    G = gpu
+    heads, n = 48, 520
+    dim = heads * 128
+    q, k, v = normal((n, dim), 0, 1030, 1.0), normal((n, dim), 0, 1031, 1.0), normal((n, dim), 0, 1032, 1.0)
+    q[:, :128] *= 0                       # head 0: equal scores
+    q[:, 128:256] *= 60                   # head 1: one score takes all, exponentials underflow
+    k[100, 256:384] = 60000               # head 2: a score of +-infinity in fp16 from row 100 on
+    q[:, 256:384] = 60000
+    k[200, 384], k[300, 512] = np.inf, np.nan
+    kd, vd = G.dev_keep(k), G.dev_keep(v)
+    out_d = G.empty((n, dim))
+    G.B.check(G.L().lcu_attention(out_d.ptr, G.dev_keep(q).ptr, kd.ptr, vd.ptr, n, n, 0, dim, heads, None))
+    got = G.host(out_d, (n, dim))
+    part = G.empty((16, dim))
+    for r in range(0, n, 16):
+        rows = min(16, n - r)
+        G.B.check(G.L().lcu_attention(part.ptr, G.dev_keep(q[r:r + rows]).ptr, kd.ptr, vd.ptr, rows, r + rows, r, dim, heads, None))
+        want = G.host(part, (16, dim))[:rows]
+        assert (np.isnan(got[r:r + rows]) == np.isnan(want)).all(), r
+        same = got[r:r + rows].view(np.uint16) == want.view(np.uint16)
+        assert (same | np.isnan(want)).all(), r
+    assert np.isnan(got[250:, 384:512]).any() and not np.isnan(got[:200, 384:512]).any()
+    G.release()
+
+
 def test_attention_decode_twice_reuses_workspace(gpu):
     # the split-T decode path keeps arrival counters in a workspace; back-to-back calls must agree
     G = gpu
