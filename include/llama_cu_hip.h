@@ -54,6 +54,9 @@ int lcu_set_device(int device);
 int lcu_malloc(void** out_dev, size_t bytes);                                   /* gpu_buffer ctor, 712-715 */
 int lcu_free(void* dev);                                                        /* gpu_buffer dtor, 732-736 */
 int lcu_memset(void* dev, int byte_value, size_t bytes, void* stream);          /* llama_cu.h:239-241 */
+/* the first `bytes` (a multiple of 16) of `count` buffers in one launch: buffers_dev is a device array of their
+ * addresses, each on a 16-byte boundary */
+int lcu_memset_many(const void* buffers_dev, int count, int byte_value, size_t bytes, void* stream);
 int lcu_h2d(void* dst_dev, const void* src_host, size_t bytes, void* stream);   /* copy_from, 699-706; async */
 int lcu_d2h(void* dst_host, const void* src_dev, size_t bytes, void* stream);   /* copy_to, 707-710; blocks */
 int lcu_d2d(void* dst_dev, const void* src_dev, size_t bytes, void* stream);

@@ -37,6 +37,7 @@ SIGNATURES = {
     "lcu_malloc": (i32, [C.POINTER(vp), sz]),
     "lcu_free": (i32, [vp]),
     "lcu_memset": (i32, [vp, i32, sz, vp]),
+    "lcu_memset_many": (i32, [vp, i32, i32, sz, vp]),
     "lcu_h2d": (i32, [vp, vp, sz, vp]),
     "lcu_d2h": (i32, [vp, vp, sz, vp]),
     "lcu_d2d": (i32, [vp, vp, sz, vp]),

@@ -1,6 +1,8 @@
 // Row-wise and element-wise kernels of the forward pass, the int8 absmax quantiser, and the
 // synthetic-tensor fill.  Each kernel keeps the reference's fp16 rounding points; reference
 // lines are cited per kernel.
+#include <algorithm>
+
 #include "common.hpp"
 
 using namespace lcu;
@@ -731,6 +733,13 @@ __global__ void fill_bytes_kernel(uint8_t* out, size_t bytes, uint8_t value) {
   for (size_t i = tail_start + tid; i < bytes; i += stride) out[i] = value;
 }
 
+// the first `pieces` 16-byte pieces of buffer blockIdx.y
+__global__ __launch_bounds__(256) void fill_many_kernel(uint4* const* __restrict__ buffers, size_t pieces, uint8_t value) {
+  const uint32_t w = value * 0x01010101u;
+  uint4* to = buffers[blockIdx.y];
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (size_t)gridDim.x * 256) to[i] = make_uint4(w, w, w, w);
+}
+
 inline int grid_for(size_t n, int threads, int cap = 1 << 16) {
   size_t g = (n + threads - 1) / threads;
   return (int)(g < 1 ? 1 : (g > (size_t)cap ? cap : g));
@@ -795,6 +804,18 @@ int lcu_memset(void* dev, int byte_value, size_t bytes, void* stream) {
   LCU_REQUIRE(dev != nullptr, "lcu_memset: null pointer");
   fill_bytes_kernel<<<grid_for(bytes / 16 + 1, 256, 4096), 256, 0, as_stream(stream)>>>((uint8_t*)dev, bytes,
                                                                                          (uint8_t)byte_value);
+  LCU_LAUNCH_CHECK();
+  return LCU_OK;
+}
+
+int lcu_memset_many(const void* buffers_dev, int count, int byte_value, size_t bytes, void* stream) {
+  LCU_REQUIRE(count >= 0 && count <= 65535 && bytes % 16 == 0, "lcu_memset_many: %d buffers of %zu bytes (multiples of 16)", count, bytes);
+  if (bytes == 0 || count == 0) return LCU_OK;
+  LCU_REQUIRE(buffers_dev != nullptr, "lcu_memset_many: null pointer");
+  // a few thousand workgroups in all, whatever their number per buffer
+  const int per = grid_for(bytes / 16, 256, std::max(1, 4096 / count));
+  fill_many_kernel<<<dim3((unsigned)per, (unsigned)count), 256, 0, as_stream(stream)>>>((uint4* const*)buffers_dev, bytes / 16,
+                                                                                       (uint8_t)byte_value);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }

@@ -51,9 +51,7 @@ struct llama_batch_context_impl final : public llama_batch_context {
 
   void clear_tokens(int sequence) override {
     LCU_CHECK(lcu_sync(stream_));
-    seqs_[sequence]->clear_tokens();  // fresh caches: other addresses
-    upload_cache_pointers();
-    drop_graph();
+    seqs_[sequence]->clear_tokens();  // the caches stay where they are
   }
 
   size_t tokens_left(int sequence) override { return seqs_[sequence]->tokens_left(); }

@@ -89,6 +89,33 @@ def test_prefill_and_decode_vs_oracle(gpu, cfg, q_type):
     assert gc.tokens_left() == 64 - T
 
 
+def test_a_cleared_context_is_a_fresh_one(gpu):
+    """clear_tokens keeps the caches and the captured step: zeroed rows, and the tokens, logits and cache rows of the
+    next sequence are those of a context that never held another, across the bound of the captured step too."""
+    P = gpu.P
+    m = P.Model(dim=512, multiple_of=128, n_heads=4, n_layers=2, n_vocab=512, seed=5, weight_std=0.05)
+    rng = np.random.default_rng(8)
+    used, fresh = P.Context(m, 1536, 0.8), P.Context(m, 1536, 0.8)
+    for n in (1010, 40):
+        tok = used.next_token(rng.integers(0, 512, n).astype(np.int16))
+        for _ in range(30):               # the first sequence passes 1024 rows
+            tok = used.next_token([tok])
+        used.clear_tokens()
+        assert used.tokens_left() == 1536
+        for layer in range(2):
+            k, v = used.kv(layer, 1536)
+            assert not k.view(np.uint16).any() and not v.view(np.uint16).any()
+    prompt = rng.integers(0, 512, 23).astype(np.int16)
+    a, b = used.next_token(prompt), fresh.next_token(prompt)
+    for _ in range(5):
+        assert a == b and (used.logits().view(np.uint16) == fresh.logits().view(np.uint16)).all()
+        a, b = used.next_token([a]), fresh.next_token([b])
+    for x, y in zip(used.kv(1, 1536), fresh.kv(1, 1536)):
+        assert (x.view(np.uint16) == y.view(np.uint16)).all()
+    for c in (used, fresh, m):
+        c.close()
+
+
 def test_prefill_chunks_and_decode_agree(gpu):
     # KV-cache consistency on the device: one 24-token prefill == 10 + 9 prefill then 5 decode steps
     G = gpu
