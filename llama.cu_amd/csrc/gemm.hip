@@ -43,12 +43,6 @@ namespace {
 constexpr int BK = 64;        // K extent one group of four wavefronts multiplies per stage
 constexpr int NUM_XCD = 8;
 
-__device__ __forceinline__ half2_t dequant2(uint32_t spread, half2_t scale2x) {
-  const uint32_t bits = (spread << 2) | 0x58005800u;                                  // 128 + q/2
-  const half2_t t = __builtin_bit_cast(half2_t, bits) - (half2_t)((half_t)191.75f);   // (q - 127.5)/2
-  return t * scale2x;                                                                 // one rounding
-}
-
 // KS: groups of four wavefronts per workgroup.  A stage holds KS * 64 of K; group g multiplies
 // columns g*64 .. g*64+63 of it into its own accumulators, and the groups' accumulators are added
 // through LDS at the end (group 0 + group 1, a fixed order).  With KS = 2 every SIMD holds two
@@ -895,14 +889,22 @@ int launch_dl(operands_t op, const half_t* A, int M, int K, int N, int block, fl
   return LCU_OK;
 }
 
+// 64 << shift = block, -1 for blocks that gemm_tile_kernel does not take (0: no codes)
+inline int block_shift(int block) {
+  for (int shift = 0; shift < 16; ++shift) {
+    if (block == 64 << shift) return shift;
+  }
+  return -1;
+}
+
 // A launch of gemm_tile_kernel; splits > 1: the K stages of every tile dealt to that many workgroups, fp32 sums to part.
-template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, class EP>
-int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N, float beta, hipStream_t st, int splits = 1,
+template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
+int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits = 1,
                 float* part = nullptr) {
-  using shape = tile_shape<BM, BN, WM, WN, NS, SPLIT, EP>;
+  using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
   const int tiles_m = (M + BM - 1) / BM, tiles_n_per = (N + BN - 1) / BN, tiles_n = tiles_n_per * op.n_mats;
   op.more.tiles_n_per = op.n_mats > 1 ? tiles_n_per : 0;
-  auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NS, SPLIT, EP>;
+  auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -910,35 +912,47 @@ int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N,
     LCU_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, shape::LDS));
     raised[dev & 15] = true;
   }
-  kernel<<<tiles_m * tiles_n * splits, 64 * WM * WN, shape::LDS, st>>>(op.out, (const half_t*)A, op.W, M, K, N, beta, tiles_m, tiles_n, part,
-                                                                       splits, op.more, ep);
+  kernel<<<tiles_m * tiles_n * splits, 64 * WM * WN, shape::LDS, st>>>(op.out, (const half_t*)A, op.W, op.S, block_shift(block), M, K, N, beta,
+                                                                       tiles_m, tiles_n, part, splits, op.more, ep);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
 
 // Columns of the 256-row tile of a product that fills most of the chip with them: the one whose rounds of workgroups
-// cost least, a round of 128 / 192 / 256 columns taking 57 / 88 / 106 us at K = 4096 (512 rows, W1 and W3 of 11008
-// columns in one launch: 230 tiles of 192 columns 88 us, 172 of 256 94 us, 344 of 128 108 us; 1987 rows: 303 us with 256
-// columns, 330 us with 128).  Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts.
-inline int large_tile_columns(int M, int N, int n_mats, long cus, bool gated) {
+// cost least.  fp16 and bfloat16: a round of 128 / 192 / 256 columns takes 57 / 88 / 106 us at K = 4096 (512 rows, W1 and W3
+// of 11008 columns in one launch: 230 tiles of 192 columns 88 us, 172 of 256 94 us, 344 of 128 108 us; 1987 rows: 303 us
+// with 256 columns, 330 us with 128).  uint8: 128 / 256 columns 65 / 113 us (512 rows, K 6656, three times 6656 columns:
+// 156 tiles of 256 168 us, 312 of 128 187 us; 1987 rows, twice 11008 columns 346 / 374 us, three times 4096 226 / 196 us).
+// Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts there.
+template <bool U8>
+int large_tile_columns(int M, int N, int n_mats, long cus, bool gated) {
   const auto cost = [&](int columns, int round) {
     const long tiles = (long)((M + 255) / 256) * ((N + columns - 1) / columns) * n_mats;
     return (tiles + cus - 1) / cus * round;
   };
-  const long c128 = cost(128, 57), c192 = gated ? c128 : cost(192, 88), c256 = cost(256, 106);
-  if (c256 < c128 && c256 <= c192) return 256;
-  return c192 < c128 ? 192 : 128;
+  if constexpr (U8) {
+    return cost(256, 113) < cost(128, 65) ? 256 : 128;
+  } else {
+    const long c128 = cost(128, 57), c192 = gated ? c128 : cost(192, 88), c256 = cost(256, 106);
+    if (c256 < c128 && c256 <= c192) return 256;
+    return c192 < c128 ? 192 : 128;
+  }
 }
 
-template <class EP>
-int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N, float beta, hipStream_t st) {
+template <bool U8, class EP>
+int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st) {
   device_state* ds = current_device_state();
-  const int columns = large_tile_columns(M, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
-  if (columns == 256) return launch_tile<256, 256, 2, 2, 2, false>(ep, op, A, M, K, N, beta, st);
-  if constexpr (!EP::GATED) {
-    if (columns == 192) return launch_tile<256, 192, 2, 2, 2, false>(ep, op, A, M, K, N, beta, st);
+  const int columns = large_tile_columns<U8>(M, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
+  if constexpr (U8) {
+    if (columns == 256) return launch_tile<256, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
+    return launch_tile<256, 128, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
+  } else {
+    if (columns == 256) return launch_tile<256, 256, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st);
+    if constexpr (!EP::GATED) {
+      if (columns == 192) return launch_tile<256, 192, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st);
+    }
+    return launch_tile<256, 128, 4, 2, 3, false, false>(ep, op, A, M, K, N, 0, beta, st);
   }
-  return launch_tile<256, 128, 4, 2, 3, false>(ep, op, A, M, K, N, beta, st);
 }
 
 // where a split-K launch left its partial sums: part[matrix][split][M][N] fp32
@@ -1036,8 +1050,9 @@ inline int large_tile_splits(int M, int K, int N, int n_mats, long cus, size_t w
   return (int)splits;
 }
 
-int launch_large_split(operands_t op, const half_t* A, int M, int K, int N, float beta, hipStream_t st, int splits, float* part) {
-  const int rc = launch_tile<256, 128, 4, 2, 3, true>(f16_epilogue{}, op, A, M, K, N, beta, st, splits, part);
+template <bool U8>
+int launch_large_split(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits, float* part) {
+  const int rc = launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, beta, st, splits, part);
   if (rc != LCU_OK) return rc;
   const size_t mn = (size_t)M * N;
   splitk_reduce_kernel<<<dim3((unsigned)((mn + 1023) / 1024), op.n_mats), 256, 0, st>>>(op.out, op.more.out[0], op.more.out[1], part, mn,
@@ -1276,7 +1291,7 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
   // uint8 weights unless each of them already fills the chip with 256x128 tiles and fusing saves no
   // round of workgroups (fp16 weights choose a wider tile there, large_tile_columns).
   const bool whole_stages = K % 128 == 0 && scale_words_ok<U8>(op, K, N, block);
-  if (U8 && op.n_mats > 1 && M > 64 && whole_stages) {
+  if (U8 && block_shift(block) < 0 && op.n_mats > 1 && M > 64 && whole_stages) {
     device_state* ds = current_device_state();
     const long cus = ds && ds->compute_units > 0 ? ds->compute_units : 256;
     const long per = (long)((M + 255) / 256) * ((N + 127) / 128);
@@ -1312,10 +1327,9 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
     const long tiles256 = (long)((M + 255) / 256) * ((N + 127) / 128) * nm;
     if (tiles256 >= 160) {
       if constexpr (U8) {
-        return launch_dl<256, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
-      } else {
-        return launch_large(f16_epilogue{}, op, A, M, K, N, beta, st);
+        if (block_shift(block) < 0) return launch_dl<256, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
       }
+      return launch_large<U8>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
     }
     {
       device_state* ds = current_device_state();
@@ -1324,10 +1338,9 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         const int splits = large_tile_splits(M, K, N, op.n_mats, ds->compute_units > 0 ? ds->compute_units : 256, ws.bytes);
         if (splits > 0) {
           if constexpr (U8) {
-            return launch_split<256, 128, 4, 2, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
-          } else {
-            return launch_large_split(op, A, M, K, N, beta, st, splits, (float*)ws.ptr);
+            if (block_shift(block) < 0) return launch_split<256, 128, 4, 2, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
           }
+          return launch_large_split<U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
         }
       }
     }
@@ -1447,7 +1460,7 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     if (rc != LCU_OK || done) return rc;
     return launch_bf16<64, 64, 2, GATED ? 1 : 2, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   }
-  if (tm(256) * tn(128) >= 160) return launch_large(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0.0f, st);
+  if (tm(256) * tn(128) >= 160) return launch_large<false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
   if (tm(128) * tn(128) > 256) return launch_bf16<128, 128, 2, 2, 1, 2>(ep, A, W, tm(128), M, K, N, st);
   if (tm(128) * tn(128) >= 160) return launch_bf16<128, 128, 4, 2, 1, 3>(ep, A, W, tm(128), M, K, N, st);
   if constexpr (GATED) {

@@ -18,6 +18,7 @@
 // neither requests (1 KB per instruction, dense) nor fragment reads (16 rows, one chunk) meet in a bank.
 #pragma once
 #include <type_traits>
+#include <utility>
 
 #include "linear.hpp"
 
@@ -53,30 +54,55 @@ __device__ __forceinline__ uint4_t operand_resource(const void* p) {
   return r;
 }
 
+// f of 0 .. N - 1 as constants: loops whose bodies are too long for the compiler to unroll when asked
+template <class F, int... I>
+__device__ __forceinline__ void static_for_each(F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_each(f, std::make_integer_sequence<int, N>{});
+}
+
+// two codes, spread to the low bytes of two halves, to fp16((q - 127.5) * scale) each (llama_cu.cu:287-289)
+__device__ __forceinline__ half2_t dequant2(uint32_t spread, half2_t scale2x) {
+  const uint32_t bits = (spread << 2) | 0x58005800u;                                  // 128 + q/2
+  const half2_t t = __builtin_bit_cast(half2_t, bits) - (half2_t)((half_t)191.75f);   // (q - 127.5)/2
+  return t * scale2x;                                                                 // one rounding
+}
+
 // WM x WN wavefronts of (BM / WM) x (BN / WN) outputs each, a ring of NS stages of 64 along K.
-// SPLIT: the grid holds `splits` workgroups per tile, each taking a contiguous run of the K stages and writing its
-// fp32 sums to part[split][M][N].
-template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, class EP>
+// U8: W is codes with one fp16 scale per `block` of a row, block = 64 << block_shift.  Codes lie in LDS as they are, 64
+// bytes a row with the 16-byte pieces of every second group of four rows turned by two, so that sixteen rows' halves meet in
+// no bank; a wavefront turns the eight codes of each of its fragments into fp16 itself, four instructions at a time
+// between the matrix instructions of the half stage before.  The wavefronts stand side by side (WM = 1), so that every code
+// is converted once; with the lhs read from LDS by all four that leaves vector instructions, LDS and matrix cores about
+// equally busy.  512 rows, (N, K) = (11008, 4096): 64 us; two rows of two wavefronts (every code twice) 64-66, four of two
+// 88; converted once into an fp16 tile in LDS, with its own ring, 87 us.  1987 rows, twice (11008, 4096): 346 / 432 / 492 / 475 us.
+template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
 struct tile_shape {
   static constexpr int NW = WM * WN, WR = BM / WM, WC = BN / WN;
-  static constexpr int STAGE = (BM + BN) * 128;
+  static constexpr int A_BYTES = BM * 128, B_BYTES = BN * (U8 ? 64 : 128), SW = (WC + 63) / 64 * 64, S_BYTES = U8 ? NW * SW * 4 : 0;
+  static constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES;  // S: one word per column of every wavefront, of its own
   static constexpr int OUT_LD = WC + 4;                  // floats per row of a wavefront's 64 output rows in LDS
   static constexpr int RING = NS * STAGE, OUT = NW * 64 * OUT_LD * 4;
   static constexpr int LDS = RING > OUT ? RING : OUT;
   static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 32 == 0, "tile");
 };
 
-template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, class EP>
+template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
-    half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, int M, int K, int N, float beta, int tiles_m,
-    int tiles_n, float* __restrict__ part, int splits, more_matrices_t more, EP ep) {
-  using shape = tile_shape<BM, BN, WM, WN, NS, SPLIT, EP>;
+    half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0, int block_shift,
+    int M, int K, int N, float beta, int tiles_m, int tiles_n, float* __restrict__ part, int splits, more_matrices_t more, EP ep) {
+  using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
   static_assert(!EP::GROUPED, "one matrix for all rows");
   constexpr int NW = shape::NW;
   constexpr int TM = shape::WR / 16, TN = shape::WC / 16;        // 16x16 tiles of a wavefront
-  constexpr int PA = BM / 8 / NW, PB = BN / 8 / NW, P = PA + PB;  // requests of a wavefront per stage
-  constexpr int A_BYTES = BM * 128, STAGE = shape::STAGE;
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && NS >= 2 && P * (NS - 1) < 64, "requests");
+  constexpr int A_BYTES = shape::A_BYTES, B_BYTES = shape::B_BYTES, STAGE = shape::STAGE;
+  constexpr int PA = A_BYTES / 1024 / NW, PB = B_BYTES / 1024 / NW, PS = U8 ? shape::SW / 64 : 0;
+  constexpr int P = PA + PB + PS;  // requests of a wavefront per stage
+  static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0 && NS >= 2 && P * (NS - 1) < 64, "requests");
+  static_assert(!U8 || !EP::BF16, "codes");
   extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
 
   // consecutive workgroups go round the eight XCDs: each gets one run of the M-fastest tile sequence, so that
@@ -90,11 +116,13 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   int tn = logical / tiles_m;
   half_t* out = out0;
   const void* W = W0;
+  const half_t* S = S0;
   if (more.tiles_n_per > 0) {
     const int g = tn / more.tiles_n_per;
     tn -= g * more.tiles_n_per;
     out = g == 0 ? out0 : (g == 1 ? more.out[0] : more.out[1]);
     W = g == 0 ? W0 : (g == 1 ? more.W[0] : more.W[1]);
+    if constexpr (U8) S = g == 0 ? S0 : (g == 1 ? more.S[0] : more.S[1]);
     if constexpr (SPLIT) part += (size_t)g * splits * M * N;  // each matrix has its own partial sums
   }
   const int m0 = tm * BM, n0 = tn * BN;
@@ -116,10 +144,25 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   }
 #pragma unroll
   for (int j = 0; j < PB; ++j) {
-    const int c = (wave + j * NW) * 64 + lane, row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
-    b_off[j] = ((uint32_t)min(n0 + row, N - 1) * (uint32_t)K + g * 8) * 2u;
+    const int c = (wave + j * NW) * 64 + lane;
+    if constexpr (U8) {
+      const int row = c / 4, g = (c % 4) ^ (2 * ((row / 4) % 2));
+      b_off[j] = (uint32_t)min(n0 + row, N - 1) * (uint32_t)K + g * 16;
+    } else {
+      const int row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
+      b_off[j] = ((uint32_t)min(n0 + row, N - 1) * (uint32_t)K + g * 8) * 2u;
+    }
   }
-  uint4_t ra = operand_resource(A), rw = operand_resource(W);
+  // first scale of the rows whose scales this lane requests, and of those of its fragments
+  uint32_t s_first[U8 ? PS : 1], f_first[U8 ? TN : 1];
+  if constexpr (U8) {
+    const uint32_t blocks = (uint32_t)K >> (6 + block_shift);
+#pragma unroll
+    for (int j = 0; j < PS; ++j) s_first[j] = (uint32_t)min(n0 + wn + j * 64 + lane, N - 1) * blocks;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) f_first[j] = (uint32_t)min(n0 + wn + j * 16 + (lane & 15), N - 1) * blocks;
+  }
+  uint4_t ra = operand_resource(A), rw = operand_resource(W), rs = operand_resource(U8 ? (const void*)S : (const void*)A);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)tile_lds;
   // Inline assembly, so that the compiler does not know about the LDS writes: knowing, it waits for every LDS read
   // in front of each matrix instruction.  There is no output register; the waits are the explicit ones below.
@@ -132,8 +175,13 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     const uint32_t along = (uint32_t)(stage0 + stage) * 128u;
     if (i < PA) {
       request(ra, along, a_off[i], slot * STAGE + (wave + i * NW) * 1024);
-    } else {
-      request(rw, along, b_off[i - PA], slot * STAGE + A_BYTES + (wave + (i - PA) * NW) * 1024);
+    } else if (i < PA + PB) {
+      request(rw, U8 ? along / 2 : along, b_off[i - PA], slot * STAGE + A_BYTES + (wave + (i - PA) * NW) * 1024);
+    } else if constexpr (U8) {  // the word that holds the row's scale of this stage
+      const uint32_t at = s_first[i - PA - PB] + ((uint32_t)(stage0 + stage) >> block_shift);
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"((at & ~1u) * 2u), "s"(rs),
+                   "s"(lds0 + slot * STAGE + A_BYTES + B_BYTES + wave * shape::SW * 4 + (i - PA - PB) * 256)
+                   : "memory", "m0");
     }
   };
 
@@ -149,13 +197,48 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   for (int h = 0; h < 2; ++h) pos[h] = (uint32_t)(((frag_chunk + 4 * h) ^ turn) * 16);
   const uint32_t a_row = (uint32_t)(wm + frag_row) * 128, b_row = (uint32_t)A_BYTES + (uint32_t)(wn + frag_row) * 128;
   half8_t fa[2][TM], fb[2][TN];
-  constexpr int READS = TM + TN, PRODUCTS = TM * TN;
+  // U8: the eight codes behind a fragment, and twice their scale
+  uint2_t codes[2][U8 ? TN : 1];
+  uint32_t words[U8 ? TN : 1];
+  half2_t scales[U8 ? TN : 1];
+  // reads of half 0: (scales, codes,) W and lhs fragments of half 0(, codes of half 1); of half 1 the fragments that are left
+  constexpr int READS0 = U8 ? 3 * TN + TM : TN + TM, READS1 = U8 ? TM : TN + TM, PRODUCTS = TM * TN;
   const auto read = [&](int slot, int h, int i) {
-    const unsigned char* p = tile_lds + slot * STAGE + pos[h];
-    if (i < TN) {
-      fb[h][i] = *reinterpret_cast<const half8_t*>(p + b_row + i * 2048);
+    const unsigned char* p = tile_lds + slot * STAGE;
+    if constexpr (U8) {
+      const unsigned char* c = p + A_BYTES + (wn + frag_row) * 64 + frag_chunk * 8;
+      const int half_turn = (frag_row / 4) % 2 * 32;  // pieces turned by two: the halves change places
+      if (h == 1) {
+        fa[1][i] = *reinterpret_cast<const half8_t*>(p + pos[1] + a_row + i * 2048);
+      } else if (i < TN) {
+        words[i] = *reinterpret_cast<const uint32_t*>(p + A_BYTES + B_BYTES + wave * shape::SW * 4 + (i * 16 + frag_row) * 4);
+      } else if (i < 2 * TN) {
+        codes[0][i - TN] = *reinterpret_cast<const uint2_t*>(c + (i - TN) * 1024 + half_turn);
+      } else if (i < 2 * TN + TM) {
+        fa[0][i - 2 * TN] = *reinterpret_cast<const half8_t*>(p + pos[0] + a_row + (i - 2 * TN) * 2048);
+      } else {
+        codes[1][i - 2 * TN - TM] = *reinterpret_cast<const uint2_t*>(c + (i - 2 * TN - TM) * 1024 + (32 - half_turn));
+      }
+    } else if (i < TN) {
+      fb[h][i] = *reinterpret_cast<const half8_t*>(p + pos[h] + b_row + i * 2048);
     } else {
-      fa[h][i - TN] = *reinterpret_cast<const half8_t*>(p + a_row + (i - TN) * 2048);
+      fa[h][i - TN] = *reinterpret_cast<const half8_t*>(p + pos[h] + a_row + (i - TN) * 2048);
+    }
+  };
+  // two of the eight values of a fragment of half h from their codes, which belong to stage `st`; four instructions, as
+  // many as go out while a matrix instruction runs
+  constexpr int CONVERTS = U8 ? 4 * TN : 0;
+  const auto convert = [&](int h, int k, int st) {
+    if constexpr (U8) {
+      const int j = k / 4, w = k / 2 % 2, high = k % 2;
+      if (h == 0 && k % 4 == 0) {
+        const uint32_t at = f_first[j] + ((uint32_t)(stage0 + st) >> block_shift);
+        const half_t x = __builtin_bit_cast(half_t, (uint16_t)((at & 1) ? words[j] >> 16 : words[j])) * (half_t)2.0f;
+        scales[j] = half2_t{x, x};
+      }
+      const half2_t y = dequant2(__builtin_amdgcn_perm(0u, codes[h][j][w], high ? 0x0c030c02u : 0x0c010c00u), scales[j]);
+      fb[h][j][4 * w + 2 * high] = y.x;
+      fb[h][j][4 * w + 2 * high + 1] = y.y;
     }
   };
   const auto multiply = [&](int h, int i) {
@@ -167,60 +250,71 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
       acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[h][a], fb[h][b], acc[a][b], 0, 0, 0);
     }
   };
-  // the products of half h, with the reads spread over the first five eighths and the requests over all of them
-  const auto half_stage = [&](int h, auto n_reads, auto&& do_read, auto n_requests, auto&& do_request) {
+  // the products of half h, with the reads spread over the first five eighths, the requests over all of them, and the
+  // conversions of the next half (U8) over the last half (of half 1, whose codes are read first) or all (of half 0)
+  const auto half_stage = [&](int h, auto n_reads, auto&& do_read, auto n_requests, auto&& do_request, auto n_converts, int convert_stage) {
     constexpr int NR = decltype(n_reads)::value, NQ = decltype(n_requests)::value, SPREAD = PRODUCTS * 5 / 8;
-#pragma unroll
-    for (int i = 0; i < PRODUCTS; ++i) {
+    constexpr int NC = decltype(n_converts)::value;
+    static_for<PRODUCTS>([&](auto at) {
+      constexpr int i = decltype(at)::value;
       multiply(h, i);
       __builtin_amdgcn_sched_barrier(0);
-      if (i < SPREAD) {
+      if constexpr (i < SPREAD) {
 #pragma unroll
         for (int k = i * NR / SPREAD; k < (i + 1) * NR / SPREAD; ++k) do_read(k);
       }
 #pragma unroll
       for (int k = i * NQ / PRODUCTS; k < (i + 1) * NQ / PRODUCTS; ++k) do_request(k);
+      const int from = h == 1 ? PRODUCTS / 2 : 0;
+      if (NC > 0 && i >= from) {
+#pragma unroll
+        for (int k = (i - from) * NC / (PRODUCTS - from); k < (i - from + 1) * NC / (PRODUCTS - from); ++k) convert(1 - h, k, convert_stage);
+      }
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
   };
   // One stage in ring slot `slot`: multiply its first half while the second is read; this wavefront has then read
   // the whole stage, and once its own requests of the next stage have landed (at most those of NS - 2 later stages
   // outstanding) the barrier says both for everybody.  Then the second half, with the next stage's first half on its
   // way from slot `next_slot` and the stage NS ahead requested into `slot`.
-  const auto stage = [&](int slot, int next_slot, int ahead, auto more_follow) {
+  const auto stage = [&](int t, int slot, int next_slot, int ahead, auto more_follow) {
     constexpr bool MORE = decltype(more_follow)::value;
-    half_stage(0, std::integral_constant<int, READS>{}, [&](int k) { read(slot, 1, k); }, std::integral_constant<int, 0>{}, [](int) {});
+    half_stage(0, std::integral_constant<int, READS1>{}, [&](int k) { read(slot, 1, k); }, std::integral_constant<int, 0>{}, [](int) {},
+               std::integral_constant<int, CONVERTS>{}, t);
     if constexpr (MORE) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       wait_vmcnt<(NS - 2) * P>();
       asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      half_stage(1, std::integral_constant<int, READS>{}, [&](int k) { read(next_slot, 0, k); }, std::integral_constant<int, P>{},
-                 [&](int k) { issue(ahead, slot, k); });
+      half_stage(1, std::integral_constant<int, READS0>{}, [&](int k) { read(next_slot, 0, k); }, std::integral_constant<int, P>{},
+                 [&](int k) { issue(ahead, slot, k); }, std::integral_constant<int, CONVERTS>{}, t + 1);
     } else {
-      half_stage(1, std::integral_constant<int, 0>{}, [](int) {}, std::integral_constant<int, 0>{}, [](int) {});
+      half_stage(1, std::integral_constant<int, 0>{}, [](int) {}, std::integral_constant<int, 0>{}, [](int) {},
+                 std::integral_constant<int, 0>{}, 0);
     }
   };
 
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    if (s == nt) ra[2] = rw[2] = 0;  // no records: a request brings zeros and reads nothing
+    if (s == nt) ra[2] = rw[2] = rs[2] = 0;  // no records: a request brings zeros and reads nothing
 #pragma unroll
     for (int i = 0; i < P; ++i) issue(s, s, i);
   }
   wait_vmcnt<(NS - 1) * P>();
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < READS; ++i) read(0, 0, i);
+  for (int i = 0; i < READS0; ++i) read(0, 0, i);
+#pragma unroll
+  for (int k = 0; k < CONVERTS; ++k) convert(0, k, 0);
   __builtin_amdgcn_sched_barrier(0);
   int slot = 0;
   for (int t = 0; t < nt - 1; ++t) {
-    if (t + NS == nt) ra[2] = rw[2] = 0;
+    if (t + NS == nt) ra[2] = rw[2] = rs[2] = 0;
     const int next_slot = slot + 1 == NS ? 0 : slot + 1;
-    stage(slot, next_slot, t + NS, std::true_type{});
+    stage(t, slot, next_slot, t + NS, std::true_type{});
     slot = next_slot;
   }
-  stage(slot, 0, 0, std::false_type{});
+  stage(nt - 1, slot, 0, 0, std::false_type{});
   wait_vmcnt<0>();  // the requests behind the last stage have written their zeros
   __syncthreads();  // LDS is free
 
@@ -253,6 +347,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
       }
     }
     constexpr int AT_ONCE = PIECES % 4 == 0 ? 4 : 2;
+    static_assert(PIECES % AT_ONCE == 0, "pieces");
 #pragma unroll 1
     for (int k0 = 0; k0 < PIECES; k0 += AT_ONCE) {
       half8_t old[AT_ONCE];
@@ -296,9 +391,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
       }
     }
   };
-  pass(std::integral_constant<int, 0>{});
-  if constexpr (shape::WR > 64) pass(std::integral_constant<int, 1>{});
-  static_assert(shape::WR <= 128, "passes");
+  static_for<shape::WR / 64>(pass);
 }
 
 }  // namespace lcu

@@ -268,6 +268,21 @@ def test_gemm_u8(gpu, M, K, N):
     G.release()
 
 
+# uint8 tiles of 256 rows at their edges: 128 and 256 columns, K split over workgroups, blocks of one, two and four K
+# stages, and a block that takes the other kernel
+@pytest.mark.parametrize("M,K,N,block", [(2049, 256, 4100, 64), (4096, 128, 4090, 128), (2300, 512, 6000, 256), (300, 5120, 1030, 128),
+                                         (2049, 128, 4100, 32)])
+def test_gemm_u8_large_tiles_ragged(gpu, M, K, N, block):
+    G = gpu
+    x, w = normal((M, K), 0, 420, 1.0), normal((N, K), 0, 421, 0.02)
+    w[3] *= np.float16(2.0 ** -7)             # subnormal scales, and a row of zeros
+    w[5] = 0
+    codes, scales = O.quantize_absmax_u8(w, block)
+    got = G.gemm_u8(x, codes, scales, block)
+    assert G.ulp_mismatch(got, O.matmul_nt_u8(x, codes, scales, block, flavour=2)) == 0.0, O.gemm_plan(M, K, N, True)
+    G.release()
+
+
 @pytest.mark.parametrize("M,K,N,count", [(512, 512, 4096, 3), (8, 4096, 4096, 3), (40, 1024, 11008, 2), (300, 256, 700, 2),
                                           (33, 200, 70, 3), (1, 512, 300, 3)])
 def test_gemm_multi_matches_separate_calls(gpu, M, K, N, count):
