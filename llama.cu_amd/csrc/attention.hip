@@ -1073,13 +1073,6 @@ __device__ __forceinline__ float exp_ieee_nonpositive(float x) {
   return x < -87.33654f ? 0.0f : p * scale;
 }
 
-// x / d from the correctly rounded reciprocal of d: quotient, exact remainder, correction.  Correctly rounded
-// for finite x and normal results; what is below the normal numbers is 0 in fp16 either way.
-__device__ __forceinline__ float divide_by(float x, float d, float reciprocal) {
-  const float q = x * reciprocal;
-  return fmaf(fmaf(-q, d, x), reciprocal, q);
-}
-
 // Attention of many rows: NW wavefronts of 16 rows each share the K and V of their head in chunks of 64 cache rows,
 // which travel into a ring of four 16 KB LDS slots, three ahead.
 //

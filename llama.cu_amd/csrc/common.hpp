@@ -117,6 +117,13 @@ __device__ __forceinline__ float exp_ieee(float x) {
   return res < 1.17549435e-38f ? 0.0f : res;
 }
 
+// x / d from the correctly rounded reciprocal of d: quotient, exact remainder, correction.  Correctly rounded
+// for finite x and normal results; what is below the normal numbers is 0 in fp16 either way.
+__device__ __forceinline__ float divide_by(float x, float d, float reciprocal) {
+  const float q = x * reciprocal;
+  return fmaf(fmaf(-q, d, x), reciprocal, q);
+}
+
 // ---- wavefront reductions (all 64 lanes end with the result) ----
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {

@@ -54,6 +54,25 @@ def test_quantize_bit_exact(gpu, rows, cols, block):
     assert (G.host(out_d, (rows, cols)).view(np.uint16) == O.dequantize_absmax_u8(ec, es, block).view(np.uint16)).all()
 
 
+# one to sixty-four lanes a block, block sizes and places that take the general kernel, counts that end inside a workgroup
+@pytest.mark.parametrize("rows,cols,block,shift", [(3, 8, 8, 0), (67, 112, 16, 0), (5, 96, 32, 0), (129, 64, 64, 0), (41, 256, 128, 0),
+                                                   (9, 512, 256, 0), (3, 1536, 512, 0), (5, 72, 24, 0), (4, 100, 20, 0), (37, 256, 128, 1)])
+def test_quantize_block_sizes_and_places(gpu, rows, cols, block, shift):
+    G = gpu
+    w = normal((rows, cols), 3, 6, 0.02)
+    w[0, :block] = np.float16(np.inf)
+    w[-1, -1] = np.float16(np.nan)
+    w[1, :block] *= np.float16(2.0 ** -9)     # subnormal scale
+    w[2, :block] = 0
+    wd = G.dev_keep(np.concatenate([np.zeros(shift, np.float16), w.reshape(-1)]))
+    codes_d, scales_d = G.empty((rows, cols), np.uint8), G.empty((rows, cols // block))
+    G.B.check(G.L().lcu_quantize_absmax_u8(codes_d.ptr, scales_d.ptr, wd.ptr + 2 * shift, rows, cols, block, None))
+    ec, es = O.quantize_absmax_u8(w, block)
+    assert (G.host(scales_d, (rows, cols // block)).view(np.uint16) == es.view(np.uint16)).all()
+    assert (G.host(codes_d, (rows, cols), np.uint8) == ec).all()
+    G.release()
+
+
 @pytest.mark.parametrize("rows,cols", [(4096, 4096), (11008, 4096), (4096, 11008)])
 def test_quantize_bit_exact_at_llama7b_shapes(gpu, rows, cols):
     """the weight matrices of the int8 benchmark configuration, W ~ N(0, 0.02), block 128: every code and scale"""
