@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemm_stream.hpp"
 #include "gemm_tile.hpp"
 #include "linear.hpp"
 
@@ -1000,6 +1001,50 @@ int launch_split(operands_t op, const half_t* A, int M, int K, int N, int block,
   return LCU_OK;
 }
 
+// Wavefronts (of 16 columns) per workgroup of gemm_stream_kernel: one workgroup runs per compute unit, so the longest
+// compute unit has rounds * wavefronts of them to stream; below four a compute unit has too little in flight.
+inline int stream_waves(int N, int n_mats, int splits, long cus, int most) {
+  const long groups = (N + 15) / 16;
+  int best = 1;
+  long least = 0;
+  for (int w = 1; w <= most; ++w) {
+    const long wgs = (groups + w - 1) / w * n_mats * splits;
+    const long cost = (wgs + cus - 1) / cus * std::max(w, 4);
+    if (w == 1 || cost <= least) {
+      least = cost;
+      best = w;
+    }
+  }
+  return best;
+}
+
+template <int TM, bool U8, bool BF16>
+int launch_stream_rows(operands_t op, const void* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, long cus) {
+  const int waves = stream_waves(N, op.n_mats, splits, cus, stream_max_waves(U8)), tiles = ((N + 15) / 16 + waves - 1) / waves;
+  op.more.tiles_n_per = op.n_mats;
+  auto kernel = gemm_stream_kernel<TM, U8, BF16>;
+  static bool raised[16] = {};  // per device, once
+  int dev = 0;
+  LCU_HIP(hipGetDevice(&dev));
+  if (!raised[dev & 15]) {
+    LCU_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, stream_lds(U8, stream_max_waves(U8))));
+    raised[dev & 15] = true;
+  }
+  const int kc = stream_chunk(M, K / BK, splits);
+  kernel<<<tiles * op.n_mats * splits, 64 * waves, stream_lds(U8, waves), st>>>((const half_t*)A, op.W, op.S, block_shift(block), M, K, N, tiles,
+                                                                                kc, part, splits, op.more);
+  LCU_LAUNCH_CHECK();
+  return LCU_OK;
+}
+
+// 1 .. 64 rows, K a multiple of 64: fp32 sums of every split's K stages to part[matrix][split][M][N]
+template <bool U8, bool BF16>
+int launch_stream(operands_t op, const void* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, long cus) {
+  if (M <= 16) return launch_stream_rows<1, U8, BF16>(op, A, M, K, N, block, st, splits, part, cus);
+  if (M <= 32) return launch_stream_rows<2, U8, BF16>(op, A, M, K, N, block, st, splits, part, cus);
+  return launch_stream_rows<4, U8, BF16>(op, A, M, K, N, block, st, splits, part, cus);
+}
+
 // Few rows (2 .. 64: short prompts, where the reference takes its 16-row tile, llama_cu.cu:1481-1484):
 // BM x 128 tiles with four wavefronts, the K stages split over enough workgroups to give every
 // compute unit one.  Returns LCU_OK with *done = false when the shape does not suit it.
@@ -1028,7 +1073,23 @@ int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block
       (long)tiles_m * tiles_n * splits < ds->compute_units / 2) {
     return LCU_OK;
   }
-  const int rc = launch_split<BM, BN, 1, 4, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
+  int rc;
+  if constexpr (U8) {
+    if (block_shift(block) < 0) {
+      rc = launch_split<BM, BN, 1, 4, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
+      *done = rc == LCU_OK;
+      return rc;
+    }
+  }
+  rc = launch_stream<U8, false>(op, A, M, K, N, block, st, splits, (float*)ws.ptr, ds->compute_units);
+  if (rc == LCU_OK && leave) {
+    leave->part = (float*)ws.ptr;
+    leave->splits = splits;
+  } else if (rc == LCU_OK) {
+    splitk_reduce_kernel<<<dim3((unsigned)((mn + 1023) / 1024), op.n_mats), 256, 0, st>>>(op.out, op.more.out[0], op.more.out[1],
+                                                                                          (const float*)ws.ptr, mn, splits, beta);
+    LCU_LAUNCH_CHECK();
+  }
   *done = rc == LCU_OK;
   return rc;
 }
@@ -1434,8 +1495,7 @@ int bf16_skinny(linear_epilogue<false, GATED> const& ep, const void* A, const vo
   while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws.bytes) --splits;
   if (splits < 2) return LCU_OK;
   float* part = (float*)ws.ptr;
-  const int rc = M <= 32 ? launch_bf16<32, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part)
-                         : launch_bf16<64, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part);
+  const int rc = launch_stream<false, true>(single_matrix(nullptr, W, nullptr), A, M, K, N, 0, st, splits, part, ds->compute_units);
   if (rc != LCU_OK) return rc;
   const int outs = M * (GATED ? N / 2 : N);
   splitk_epilogue_kernel<GATED><<<(outs + 255) / 256, 256, 0, st>>>(ep, part, M, N, splits);

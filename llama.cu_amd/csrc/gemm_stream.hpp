@@ -1,0 +1,200 @@
+// Matrix products of 2 to 64 rows: the weight stream is what counts.  fp16 or bfloat16 weights, or uint8 codes; fp32 sums
+// of a run of K stages (64 of K) per output to part[matrix][split][M][N].
+//
+// What bounds it: a compute unit has so many cache lines on their way, 24 to 28 GB/s of cold ones, so each has
+// to be given the same number of bytes, in whole lines, and asked for them without a pause.  A wavefront owns 16
+// columns of W and brings 128 bytes of each of its rows at a time into an LDS ring of its own, three ahead, with no
+// barrier; it shares nothing but lhs, which lies in LDS in one piece or in chunks.  One workgroup runs per compute unit, with
+// as many wavefronts as give every compute unit one (stream_waves): 128-column tiles with a common ring left 288 workgroups
+// of Wq, Wk, Wv for 256 compute units.  (Loaded into registers as the matrix instructions want them, sixteen rows
+// per 16 lanes, a line takes four requests: slower for fp16 than the common ring.)
+// M = 8 with the launch that adds the splits, fp16 three times (4096, 4096) 26.0 -> 22.7 us, twice (N, K) = (11008, 4096) 45 -> 42,
+// (4096, 4096) 12.1 -> 12.4; uint8 three times (6656, 6656) 61 -> 35, twice (17920, 6656) 104 -> 57, (6656, 17920) 62 -> 37.  Rows of
+// 8 KB meet in the same memory channels: K = 4224 takes a tenth less than 4096.
+#pragma once
+#include <algorithm>
+
+#include "gemm_tile.hpp"
+
+namespace lcu {
+
+constexpr int STREAM_RING = 4;
+constexpr int STREAM_LHS = 64 * 1024;  // bytes of lhs in LDS: one chunk, or two of half of it
+// a unit is 16 rows of 128 bytes; uint8: and a word with the scales of each row
+constexpr int stream_unit(bool u8) { return 2048 + (u8 ? 256 : 0); }
+constexpr int stream_max_waves(bool u8) { return u8 ? 10 : 12; }  // LDS: 160 KB
+constexpr int stream_lds(bool u8, int waves) { return STREAM_LHS + waves * STREAM_RING * stream_unit(u8); }
+// K extent of a chunk of lhs: the longest run, counted from the 128 of K that it begins in, or what two chunks leave
+inline int stream_chunk(int rows, int stages_in_all, int splits) {
+  long longest = 0;
+  for (long i = 0; i < splits; ++i) longest = std::max(longest, (i + 1) * stages_in_all / splits - (i * stages_in_all / splits & ~1L));
+  const int whole = (int)(longest + 1) / 2 * 128;
+  return rows * whole * 2 <= STREAM_LHS ? whole : STREAM_LHS / 4 / rows / 128 * 128;
+}
+
+template <int TM, bool U8, bool BF16>
+__global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kernel(const half_t* __restrict__ A, const void* __restrict__ W0,
+                                                                               const half_t* __restrict__ S0, int block_shift, int M, int K,
+                                                                               int N, int tiles, int kc, float* __restrict__ part, int splits,
+                                                                               more_matrices_t more) {
+  constexpr int RING = STREAM_RING, UNIT = stream_unit(U8), P = U8 ? 3 : 2;  // requests per unit
+  constexpr int PER = U8 ? 2 : 1;                                           // stages per unit
+  extern __shared__ __attribute__((aligned(16))) unsigned char stream_mem[];
+  const int waves = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // tiles of one matrix, then of the next, then the same of the next split
+  const int mats = more.tiles_n_per;
+  const int split = blockIdx.x / (tiles * mats), rest = blockIdx.x % (tiles * mats), g = rest / tiles;
+  const void* W = g == 0 ? W0 : (g == 1 ? more.W[0] : more.W[1]);
+  const half_t* S = g == 0 ? S0 : (g == 1 ? more.S[0] : more.S[1]);
+  const int n0 = ((rest % tiles) * waves + wave) * 16;
+  const bool mine = n0 < N;
+  const int nt_all = K / 64;
+  const int stage0 = (int)((long)split * nt_all / splits), stage1 = (int)((long)(split + 1) * nt_all / splits);
+  // stages are counted from an even one, so that units of two are whole lines of codes
+  const int base = stage0 & ~1, first = stage0 - base, end = stage1 - base;
+  const int units = (end + PER - 1) / PER;
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)stream_mem;
+  // lhs: rows of kc, 16-byte piece p of row r at p ^ r % 16 (within 16 pieces), so that the sixteen rows of a
+  // fragment meet in no bank.
+  const uint32_t row_bytes = (uint32_t)kc * 2, chunk_bytes = (uint32_t)(M * row_bytes + 1023) / 1024 * 1024;
+  const auto request_chunk = [&](int chunk) {
+    const int pieces = kc / 8;
+    for (int u = wave; u * 64 < M * pieces; u += waves) {
+      const int piece = min(u * 64 + lane, M * pieces - 1), row = piece / pieces, at = piece - row * pieces;
+      const int k = min((base * 64 + chunk * kc) + ((at & ~15) | ((at ^ row) & 15)) * 8, K - 8);
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(A + (size_t)row * K + k),
+                   "s"(lds0 + (chunk & 1) * chunk_bytes + u * 1024)
+                   : "memory", "m0");
+    }
+  };
+
+  // this wavefront's columns: rows of 128 bytes, 16-byte piece p of row r at p ^ (r / 2) % 8
+  const uint32_t ring0 = lds0 + STREAM_LHS + wave * RING * UNIT;
+  uint4_t rw = operand_resource(W), rs = operand_resource(U8 ? (const void*)S : W);
+  uint32_t w_off[2], s_first = 0;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = j * 8 + (lane >> 3), piece = (lane & 7) ^ ((row / 2) % 8);
+    w_off[j] = (uint32_t)min(n0 + row, N - 1) * (uint32_t)K * (U8 ? 1u : 2u) + piece * 16;
+  }
+  const int col = lane & 15, group = lane >> 4;
+  if constexpr (U8) s_first = (uint32_t)min(n0 + col, N - 1) * ((uint32_t)K >> (6 + block_shift));
+  const auto request = [&](int u) {
+    if (u == units) rw[2] = rs[2] = 0;  // behind the last unit: requests that count and touch no memory
+    const uint32_t slot = ring0 + (u % RING) * UNIT, along = (uint32_t)(base * (U8 ? 64 : 128) + u * 128);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(w_off[j]), "s"(rw), "s"(along),
+                   "s"(slot + j * 1024)
+                   : "memory", "m0");
+    }
+    if constexpr (U8) {  // the word that holds the row's scales of both stages
+      const uint32_t at = s_first + ((uint32_t)(base + 2 * u) >> block_shift);
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"((at & ~1u) * 2u), "s"(rs), "s"(slot + 2048)
+                   : "memory", "m0");
+    }
+  };
+
+  float4_t acc[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) acc[i] = (float4_t)(0.0f);
+  const int turn = (col / 2) % 8;
+  uint32_t lhs_row[TM];  // rows past M: the last one, whose sums nobody stores there
+  int lhs_turn[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int row = min(i * 16 + col, M - 1);
+    lhs_row[i] = (uint32_t)row * row_bytes;
+    lhs_turn[i] = row & 15;
+  }
+  // stage s, whose columns lie in `slot` (U8: in its first or second half)
+  const auto multiply = [&](const unsigned char* slot, int s) {
+    half8_t w[2];
+    const unsigned char* row = slot + col * 128;
+    if constexpr (U8) {
+      const uint32_t at = s_first + ((uint32_t)(base + s) >> block_shift);
+      const uint32_t word = *reinterpret_cast<const uint32_t*>(slot + 2048 + lane * 4);
+      const half_t s2 = __builtin_bit_cast(half_t, (uint16_t)((at & 1) ? word >> 16 : word)) * (half_t)2.0f;
+      const half2_t s2v = {s2, s2};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int byte = (s & 1) * 64 + h * 32 + group * 8;
+        const uint2_t q = *reinterpret_cast<const uint2_t*>(row + (((byte >> 4) ^ turn) << 4) + (byte & 8));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const half2_t lo = dequant2(__builtin_amdgcn_perm(0u, q[i], 0x0c010c00u), s2v);
+          const half2_t hi = dequant2(__builtin_amdgcn_perm(0u, q[i], 0x0c030c02u), s2v);
+          w[h][4 * i] = lo.x, w[h][4 * i + 1] = lo.y, w[h][4 * i + 2] = hi.x, w[h][4 * i + 3] = hi.y;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) w[h] = *reinterpret_cast<const half8_t*>(row + (((4 * h + group) ^ turn) << 4));
+    }
+    const int chunk = s * 64 / kc, p0 = (s * 64 - chunk * kc) / 8;
+    const unsigned char* lhs = stream_mem + (chunk & 1) * chunk_bytes;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int p = p0 + 4 * h + group;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const half8_t a = *reinterpret_cast<const half8_t*>(lhs + lhs_row[i] + ((p & ~15) | ((p ^ lhs_turn[i]) & 15)) * 16);
+        if constexpr (BF16) {
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, w[h]), acc[i], 0, 0, 0);
+        } else {
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, w[h], acc[i], 0, 0, 0);
+        }
+      }
+    }
+  };
+
+  const int chunk_units = kc / 64 / PER, u0 = first / PER;
+  request_chunk(0);
+  if (mine) {
+#pragma unroll
+    for (int j = 0; j < RING - 1; ++j) request(u0 + j);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P * (RING - 1)) : "memory");  // lhs, but not yet the columns
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  asm volatile("s_barrier" ::: "memory");
+  for (int c = 0; c * chunk_units < units; ++c) {
+    if (c > 0) {
+      // chunk c was requested a chunk of units ago: before all that may still be out, if that is as long as the ring
+      if (mine && chunk_units >= RING) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(P * (RING - 1)) : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      }
+      asm volatile("s_barrier" ::: "memory");
+    }
+    if ((c + 1) * chunk_units < units) request_chunk(c + 1);  // into the half that was read before the barrier
+    if (!mine) continue;
+    for (int u = max(u0, c * chunk_units); u < min(units, (c + 1) * chunk_units); ++u) {
+      // unit u has landed, and the unit before it has been read: the ring may take another in its place
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(P * (RING - 2)) : "memory");
+      request(u + RING - 1);
+      const unsigned char* slot = stream_mem + STREAM_LHS + (wave * RING + u % RING) * UNIT;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int s = u * PER + e;
+        if (PER == 1 || (s >= first && s < end)) multiply(slot, s);
+      }
+    }
+  }
+  if (!mine) return;
+  // register e of a lane is row 4 group + e, column col of its tile
+  part += ((size_t)g * splits + split) * M * N;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int m = i * 16 + group * 4 + e;
+      if (m < M && n0 + col < N) part[(size_t)m * N + n0 + col] = acc[i][e];
+    }
+  }
+}
+
+}  // namespace lcu

@@ -276,20 +276,6 @@ void llama_context_impl::clear_tokens() {
   llama_params const& p = model_->params;
   const size_t ctx = (size_t)context_len_, dim = p.dim, ffn = p.ffn_dim();
   LCU_CHECK(lcu_sync(stream_));
-  if (kv_.empty() && p.n_layers > 0) {
-    kv_.resize(p.n_layers);
-    std::vector<void*> buffers;
-    for (auto& kv : kv_) {
-      kv.k = gpu_buffer(ctx * dim * 2);
-      kv.v = gpu_buffer(ctx * dim * 2);
-      buffers.insert(buffers.end(), {kv.k.data(), kv.v.data()});
-    }
-    t_caches_ = gpu_buffer(buffers.size() * sizeof(void*));
-    t_caches_.copy_from(buffers.data(), t_caches_.size());
-    LCU_CHECK(lcu_sync(nullptr));
-    start_pos_ = context_len_;  // fresh memory: every row
-  }
-  LCU_CHECK(lcu_memset_many(t_caches_.data(), 2 * (int)kv_.size(), 0, (size_t)start_pos_ * dim * 2, stream_));
   if (!t_embed_.is_ok()) {
     t_embed_ = gpu_buffer(ctx * dim * 2);
     t_norm_ = gpu_buffer(ctx * dim * 2);
@@ -302,8 +288,20 @@ void llama_context_impl::clear_tokens() {
     t_logits_ = gpu_buffer((size_t)p.n_vocab * 2);
     t_probs_ = gpu_buffer((size_t)p.n_vocab * 2);
     t_argmax_ = gpu_buffer(2 * sizeof(int));  // {token, count of hand-overs that did not arrive}
-    t_step_ = gpu_buffer(sizeof(step_state));
+    t_step_ = gpu_buffer(sizeof(step_state) + 2 * p.n_layers * sizeof(void*));  // and the addresses of the caches
   }
+  std::vector<void*> caches;
+  if (kv_.empty()) {
+    kv_.resize(p.n_layers);
+    for (auto& kv : kv_) {
+      kv.k = gpu_buffer(ctx * dim * 2);
+      kv.v = gpu_buffer(ctx * dim * 2);
+      caches.insert(caches.end(), {kv.k.data(), kv.v.data()});
+    }
+    LCU_CHECK(lcu_h2d((char*)t_step_.data() + sizeof(step_state), caches.data(), caches.size() * sizeof(void*), stream_));
+    start_pos_ = context_len_;  // fresh memory: every row
+  }
+  LCU_CHECK(lcu_memset_many((char*)t_step_.data() + sizeof(step_state), 2 * (int)kv_.size(), 0, (size_t)start_pos_ * dim * 2, stream_));
   LCU_CHECK(lcu_sync(stream_));
   start_pos_ = 0;
   last_n_ = 0;
@@ -315,10 +313,10 @@ size_t llama_context_impl::context_memory_usage() {
     count += kv.k.size() + kv.v.size();
   }
   for (gpu_buffer const* b : {&t_embed_, &t_norm_, &t_xq_, &t_out_, &t_w1_, &t_w3_, &t_silu_, &t_tokens_, &t_logits_,
-                              &t_probs_, &t_argmax_, &t_step_}) {
+                              &t_probs_, &t_argmax_}) {
     count += b->size();
   }
-  return count;
+  return count + sizeof(step_state);
 }
 
 void llama_context_impl::matmul(void* out, const void* lhs, weight_tensor const& w, int M, float beta) {

@@ -85,12 +85,12 @@ struct llama_context_impl final : public llama_context {
   void enqueue_head(int n);
   void drop_graph();
   std::vector<kv_cache_layer> kv_;
-  gpu_buffer t_caches_;  // addresses of every layer's k and v
   gpu_buffer t_embed_, t_norm_, t_xq_, t_out_, t_w1_, t_w3_, t_silu_;
   gpu_buffer t_tokens_, t_logits_, t_probs_, t_argmax_;
   // step state on the device: {int32 position, int16 token, 64 random bits, uint32 step counter};
   // the decode kernels and the sampler read it from here, so one captured graph replays for every
   // step (the counter differs from step to step: the epoch of the attention kernel's hand-over)
+  // (behind it: the addresses of every layer's k and v, for clear_tokens)
   gpu_buffer t_step_;
   struct step_state {
     int32_t pos;

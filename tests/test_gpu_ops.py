@@ -287,6 +287,29 @@ def test_gemm_u8(gpu, M, K, N):
     G.release()
 
 
+# few rows, codes: runs of K stages that begin in the middle of 128 codes, one to four row tiles, lhs in one piece and in
+# chunks, one and two scales in 128 codes, and a block that takes the other kernel
+@pytest.mark.parametrize("M,K,N,block", [(2, 1152, 520, 64), (16, 1152, 4100, 128), (17, 2560, 1000, 256), (33, 1152, 5000, 64),
+                                         (64, 5888, 4100, 128), (64, 1152, 3000, 384), (7, 17920, 6656, 128)])
+def test_gemm_u8_few_rows(gpu, M, K, N, block):
+    G = gpu
+    x, w = normal((M, K), 0, 430, 1.0), normal((N, K), 0, 431, 0.02)
+    codes, scales = O.quantize_absmax_u8(w, block)
+    got = G.gemm_u8(x, codes, scales, block)
+    assert G.ulp_mismatch(got, O.matmul_nt_u8(x, codes, scales, block, flavour=2)) == 0.0, O.gemm_plan(M, K, N, True)
+    G.release()
+
+
+# few rows, fp16: odd runs, rows past the last whole tile, columns past the last whole wavefront, lhs in chunks
+@pytest.mark.parametrize("M,K,N", [(3, 1152, 520), (16, 1408, 4099), (31, 2944, 1000), (48, 5888, 4100), (64, 4096, 24000)])
+def test_gemm_f16_few_rows(gpu, M, K, N):
+    G = gpu
+    x, w, old = normal((M, K), 0, 440, 1.0), normal((N, K), 0, 441, 0.02), normal((M, N), 0, 442, 1.0)
+    assert G.ulp_mismatch(G.gemm_f16(x, w), O.matmul_nt(x, w, flavour=2)) == 0.0, O.gemm_plan(M, K, N)
+    assert G.ulp_mismatch(G.gemm_f16(x, w, beta=1.0, out=old), O.matmul_nt(x, w, beta=1.0, out=old, flavour=2)) == 0.0
+    G.release()
+
+
 # uint8 tiles of 256 rows at their edges: 128 and 256 columns, K split over workgroups, blocks of one, two and four K
 # stages, and a block that takes the other kernel
 @pytest.mark.parametrize("M,K,N,block", [(2049, 256, 4100, 64), (4096, 128, 4090, 128), (2300, 512, 6000, 256), (300, 5120, 1030, 128),
