@@ -925,12 +925,15 @@ int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N,
 // with 256 columns, 330 us with 128).  uint8: 128 / 256 columns 65 / 113 us (512 rows, K 6656, three times 6656 columns:
 // 156 tiles of 256 168 us, 312 of 128 187 us; 1987 rows, twice 11008 columns 346 / 374 us, three times 4096 226 / 196 us).
 // Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts there.
+// Up to 128 rows: tiles of 128 rows, a round of 128 / 256 columns taking 52 / 66 us in fp16 and 42 / 62 in uint8 (100
+// rows, twice 11008 columns 61 -> 52 us and 55 -> 42 against tiles of 256 rows; twice 17920 of K 6656 140 -> 118 and 170 -> 109).
 template <bool U8>
 int large_tile_columns(int M, int N, int n_mats, long cus, bool gated) {
   const auto cost = [&](int columns, int round) {
     const long tiles = (long)((M + 255) / 256) * ((N + columns - 1) / columns) * n_mats;
     return (tiles + cus - 1) / cus * round;
   };
+  if (M <= 128) return cost(256, U8 ? 62 : 66) < cost(128, U8 ? 42 : 52) ? 256 : 128;
   if constexpr (U8) {
     return cost(256, 113) < cost(128, 65) ? 256 : 128;
   } else {
@@ -944,6 +947,15 @@ template <bool U8, class EP>
 int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st) {
   device_state* ds = current_device_state();
   const int columns = large_tile_columns<U8>(M, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
+  if (M <= 128) {
+    if constexpr (U8) {
+      if (columns == 256) return launch_tile<128, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
+      return launch_tile<128, 128, 1, 4, 4, true, false>(ep, op, A, M, K, N, block, beta, st);
+    } else {
+      if (columns == 256) return launch_tile<128, 256, 2, 4, 3, false, false>(ep, op, A, M, K, N, 0, beta, st);
+      return launch_tile<128, 128, 2, 2, 4, false, false>(ep, op, A, M, K, N, 0, beta, st);
+    }
+  }
   if constexpr (U8) {
     if (columns == 256) return launch_tile<256, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
     return launch_tile<256, 128, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
@@ -1113,7 +1125,8 @@ inline int large_tile_splits(int M, int K, int N, int n_mats, long cus, size_t w
 
 template <bool U8>
 int launch_large_split(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits, float* part) {
-  const int rc = launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, beta, st, splits, part);
+  const int rc = M <= 128 ? launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, U8, true>(f16_epilogue{}, op, A, M, K, N, block, beta, st, splits, part)
+                          : launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, beta, st, splits, part);
   if (rc != LCU_OK) return rc;
   const size_t mn = (size_t)M * N;
   splitk_reduce_kernel<<<dim3((unsigned)((mn + 1023) / 1024), op.n_mats), 256, 0, st>>>(op.out, op.more.out[0], op.more.out[1], part, mn,

@@ -32,6 +32,18 @@ inline int stream_chunk(int rows, int stages_in_all, int splits) {
   return rows * whole * 2 <= STREAM_LHS ? whole : STREAM_LHS / 4 / rows / 128 * 128;
 }
 
+// at most BASE requests outstanding, and `more` (0 .. 4) younger ones of another kind besides; this wavefront's LDS reads done
+template <int BASE>
+__device__ __forceinline__ void wait_requests(int more) {
+  switch (more) {
+    case 1: asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BASE + 1) : "memory"); break;
+    case 2: asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BASE + 2) : "memory"); break;
+    case 3: asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BASE + 3) : "memory"); break;
+    case 4: asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BASE + 4) : "memory"); break;
+    default: asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BASE) : "memory"); break;
+  }
+}
+
 template <int TM, bool U8, bool BF16>
 __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kernel(const half_t* __restrict__ A, const void* __restrict__ W0,
                                                                                const half_t* __restrict__ S0, int block_shift, int M, int K,
@@ -68,6 +80,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
                    "s"(lds0 + (chunk & 1) * chunk_bytes + u * 1024)
                    : "memory", "m0");
     }
+    return (M * pieces - wave * 64 + waves * 64 - 1) / (waves * 64);
   };
 
   // this wavefront's columns: rows of 128 bytes, 16-byte piece p of row r at p ^ (r / 2) % 8
@@ -170,11 +183,13 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
       }
       asm volatile("s_barrier" ::: "memory");
     }
-    if ((c + 1) * chunk_units < units) request_chunk(c + 1);  // into the half that was read before the barrier
+    const int from = max(u0, c * chunk_units);
+    int lhs_out = 0;  // requests of the next chunk, behind those of the RING - 1 units that are out
+    if ((c + 1) * chunk_units < units) lhs_out = request_chunk(c + 1);  // into the half that was read before the barrier
     if (!mine) continue;
-    for (int u = max(u0, c * chunk_units); u < min(units, (c + 1) * chunk_units); ++u) {
+    for (int u = from; u < min(units, (c + 1) * chunk_units); ++u) {
       // unit u has landed, and the unit before it has been read: the ring may take another in its place
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(P * (RING - 2)) : "memory");
+      wait_requests<P*(RING - 2)>(u - from < RING - 1 ? lhs_out : 0);
       request(u + RING - 1);
       const unsigned char* slot = stream_mem + STREAM_LHS + (wave * RING + u % RING) * UNIT;
 #pragma unroll
