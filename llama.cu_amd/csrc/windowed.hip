@@ -131,11 +131,14 @@ constexpr int QT = 64, KT = 64;
 // where key r of a tile lies in a row of transposed values
 __device__ __forceinline__ int key_place(int r) { return (r & ~31) + ((r >> 2) & 3) * 8 + ((r >> 4) & 1) * 4 + (r & 3); }
 
-template <int DV, bool BIAS>
-__global__ __launch_bounds__(256) void attention_tile_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
+// KP: 32-column pieces of a key.  With registers for keys of 256 whatever their size, one wavefront per SIMD was all that
+// fits at values of 128; two or three do now.  2048 tokens, 32 heads, values of 128: keys of 192 over all and keys of 128 in a window
+// of 1024 took 216 us on average, 167 and 86 now.
+template <int DV, bool BIAS, int KP>
+__global__ __launch_bounds__(256, DV <= 128 && KP <= 6 ? 2 : 1) void attention_tile_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                                                              const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, int n,
                                                              int start, window_args p) {
-  constexpr int NT = DV / 16, LDP = KT + 8, KP = 8, VP = (DV + 63) / 64;  // KP, VP: pieces of a tile per thread
+  constexpr int NT = DV / 16, LDP = KT + 8, VP = (DV + 63) / 64;  // KP, VP: pieces of a tile per thread
   extern __shared__ __attribute__((aligned(16))) unsigned char attn_lds[];
   const int ldk = p.dk + 8;
   bf16_t* Ks = reinterpret_cast<bf16_t*>(attn_lds);   // [KT][ldk]
@@ -292,11 +295,11 @@ __global__ __launch_bounds__(256) void attention_tile_kernel(bf16_t* __restrict_
 
 size_t tile_lds(int dk, int dv) { return ((size_t)KT * (dk + 8) + (size_t)dv * (KT + 8)) * 2; }
 
-template <int DV, bool BIAS>
-int launch_tiles(void* out, const void* q, const void* k, const void* v, int n, int start, const window_args& p, hipStream_t st) {
+template <int DV, bool BIAS, int KP>
+int launch_tiles_of(void* out, const void* q, const void* k, const void* v, int n, int start, const window_args& p, hipStream_t st) {
   const size_t lds = tile_lds(p.dk, DV);
   LCU_REQUIRE(lds <= 160 * 1024, "lcu_attention_windowed: head size %d with value size %d", p.dk, DV);
-  auto kernel = attention_tile_kernel<DV, BIAS>;
+  auto kernel = attention_tile_kernel<DV, BIAS, KP>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -308,6 +311,13 @@ int launch_tiles(void* out, const void* q, const void* k, const void* v, int n, 
                                                               start, p);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
+}
+
+template <int DV, bool BIAS>
+int launch_tiles(void* out, const void* q, const void* k, const void* v, int n, int start, const window_args& p, hipStream_t st) {
+  if (p.dk <= 128) return launch_tiles_of<DV, BIAS, 4>(out, q, k, v, n, start, p, st);
+  if (p.dk <= 192) return launch_tiles_of<DV, BIAS, 6>(out, q, k, v, n, start, p, st);
+  return launch_tiles_of<DV, BIAS, 8>(out, q, k, v, n, start, p, st);
 }
 
 // ---- one new token, bfloat16 ----------------------------------------------------------------------------

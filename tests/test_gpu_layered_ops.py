@@ -289,6 +289,14 @@ def test_windowed_attention_in_portions(gpu, dt, heads, kv, dim, vdim, window, k
     gpu.release()
 
 
+# key sizes on both sides of what the tile kernel keeps registers for
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (129, 64), (192, 128), (193, 200), (256, 32)])
+def test_windowed_attention_key_sizes(gpu, dim, vdim):
+    c = attention_case(gpu, BF16, 4, 2, dim, vdim, 90, 3, 150, dim)
+    close(run_attention(gpu, c, BF16, (150,)), c["want"], BF16, bf16=2.0 ** -7)
+    gpu.release()
+
+
 @BOTH
 @pytest.mark.parametrize("window,keep,edge", [(48, 0, "window"), (64, 6, "window"), (65, 0, "window"), (32, 0, "window"), (20, 70, "keep")])
 def test_attention_edges(gpu, dt, window, keep, edge):
