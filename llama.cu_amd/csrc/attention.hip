@@ -1084,7 +1084,7 @@ __device__ __forceinline__ float exp_ieee_nonpositive(float x) {
 // itself being transposed on its way out of LDS.
 // The sums are those of a wavefront per row: pair p = (column % 128) / 2 adds its two exponentials per 128 columns, then the
 // 64 pairs meet as in wave_sum (llama_cu.cu:433-499); the products with V are a chain over ascending cache rows.
-// 32 heads, n = T = 1987: 502 -> 154 us; 52 heads, n = T = 2048: 837 -> 242 us.
+// 32 heads, n = T = 1987: 502 -> 155 us, 512 rows of 2048: 214 -> 122 us; 52 heads, n = T = 2048: 839 -> 246 us.
 template <int NW>
 __global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_t* __restrict__ out, const half_t* __restrict__ q,
                                                                            const half_t* __restrict__ k, const half_t* __restrict__ v,
@@ -1148,16 +1148,15 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_
   const int k_turn = turn_k(key_row);
   const auto products = [&](float4_t (&s)[2][2], int item) {
     const unsigned char* slot = smem + (item & 3) * SLOT + k_base;
+    // four sums in turn: each matrix instruction's result is wanted four instructions later
+    // (32 heads, n = T = 1024: 70 us with one sum after the other, 67 us so)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int d = 0; d < 4; ++d) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        s[b][t] = (float4_t)(0.0f);
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          const half8_t kf = *reinterpret_cast<const half8_t*>(slot + (32 * b + 4 * t) * 256 + (((d * 4 + group) ^ k_turn) * 16));
-          s[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[d], s[b][t], 0, 0, 0);
-        }
+      for (int i = 0; i < 4; ++i) {
+        const int b = i >> 1, t = i & 1;
+        const half8_t kf = *reinterpret_cast<const half8_t*>(slot + (32 * b + 4 * t) * 256 + (((d * 4 + group) ^ k_turn) * 16));
+        s[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[d], d == 0 ? (float4_t)(0.0f) : s[b][t], 0, 0, 0);
       }
     }
   };
@@ -1386,10 +1385,10 @@ int lcu_attention(void* out_dev, const void* q_dev, const void* k_dev, const voi
   }
   LCU_REQUIRE(T <= MAX_T_PREFILL, "lcu_attention: T %d exceeds %d for n_new > 1", T, MAX_T_PREFILL);
   // Many scores: the kernel that computes them three times and stores none.  A wavefront of it walks all T columns
-  // alone, 3.9 us per 64 of them, while the kernel below shares a tile's columns among four wavefronts but is bound by
+  // alone, 3.75 us per 64 of them, while the kernel below shares a tile's columns among four wavefronts but is bound by
   // what LDS holds from about 0.17 M scores per us on; the lines cross where the call has 11 000 scores per column
-  // (heads, n = T, us here against below: 32 heads 512 rows 35 / 24, 700 rows 47 / 44, 1024 rows 70 / 144, 1987 rows 154 / 502;
-  // 52 heads 512 rows 36 / 38; 4 heads 1500 rows 95 / 90; 32 heads 64 rows of 1000 66 / 39, 512 rows of 2048 129 / 214).
+  // (heads, n = T, us here against below: 32 heads 512 rows 35 / 25, 700 rows 46 / 47, 1024 rows 67 / 143, 1987 rows 155 / 502;
+  // 52 heads 512 rows 35 / 37; 4 heads 1500 rows 89 / 90; 32 heads 64 rows of 1000 62 / 38, 512 rows of 2048 122 / 214).
   const double scores = (double)n_heads * n_new * (start_pos + 0.5 * n_new);
   if (scores >= 11000.0 * T) {
     // 128 rows to a workgroup read K and V half as often, if two workgroups per compute unit are left
