@@ -5,22 +5,24 @@
 // the natural operand order of v_mfma_f32_32x32x16_f16: every lane feeds 8 consecutive k of one
 // row of lhs (A) and of one row of W (B).
 //
-// Three kernels:
+// Four kernels:
 //   gemm_tile_kernel (gemm_tile.hpp): 256-row tiles of 128, 192 or 256 columns where these fill most of the
-//     chip, and 256x128 with the K range split over workgroups; fp16 and bfloat16 operands
+//     chip, 256x128 with the K range split over workgroups, 128-row tiles of up to 128 rows and where only
+//     those of 128x128 fill most of the chip; fp16, uint8 (codes in blocks of 64 << n) and bfloat16 weights
+//   gemm_stream_kernel (gemm_stream.hpp): 2..64 rows, the K range split over workgroups
 //   gemm_dl_kernel (K a multiple of 128, every other shape of the model family): both operands travel
 //     from global memory straight into a ring of 2-3 LDS stages with global_load_lds_dwordx4 (no
 //     staging registers, no LDS store instructions); rows are unpadded and the 16-byte chunks of a
 //     row are permuted so that neither the requests nor the fragment reads meet in a bank; tiles
-//     of 256x128 (uint8), 128x128 or 128x64 with 4 or 8 wavefronts (a second group of four may take the
+//     of 128x64 (other blocks of codes: 256x128 and 128x128 too) with 4 or 8 wavefronts (a second group of four may take the
 //     other half of a 128-wide K stage), chosen by how many tiles the product has; uint8 weights
 //     add a ring of codes and of scales and are turned into fp16 -- exactly fp16((q - 127.5) *
-//     scale), llama_cu.cu:287-289 -- once per block tile; with 2..64 rows, and with few large tiles
-//     and a long K, the K range is split over workgroups and a second launch adds the fp32 partial
-//     sums in split order (launch_skinny, large_tile_splits)
+//     scale), llama_cu.cu:287-289 -- once per block tile
+//   Where the K range is split -- 2..64 rows, few large tiles and a long K -- a second launch adds the
+//     fp32 partial sums in split order (launch_skinny, large_tile_splits)
 //   gemm_kernel (ragged K): global -> registers -> padded LDS with two LDS buffers and two
 //     register stages, uint8 weights dequantised between the load and the LDS store
-// Both: the K loop carries no vector address arithmetic and no predication; the block index ->
+// All: the K loop carries no vector address arithmetic and no predication; the block index ->
 // tile mapping keeps the tiles that share a slice of W on one XCD (one L2); rows >= M and columns
 // >= N are masked instead of the reference's zeroed "gutter" rows (llama_cu.h:236-242).
 #include <algorithm>
@@ -1058,8 +1060,8 @@ int launch_stream(operands_t op, const void* A, int M, int K, int N, int block, 
 }
 
 // Few rows (2 .. 64: short prompts, where the reference takes its 16-row tile, llama_cu.cu:1481-1484):
-// BM x 128 tiles with four wavefronts, the K stages split over enough workgroups to give every
-// compute unit one.  Returns LCU_OK with *done = false when the shape does not suit it.
+// the K stages split as BM x 128 tiles would need to give every compute unit one workgroup; gemm_stream_kernel
+// walks the splits (blocks of codes other than 64 << n: such tiles with four wavefronts).  Returns LCU_OK with *done = false when the shape does not suit it.
 template <int BM, bool U8>
 int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st,
                   bool* done, partial_sums_t* leave = nullptr) {
@@ -1353,14 +1355,11 @@ int launch_gemm(half_t* out, const half_t* A, const void* W, const half_t* S, in
 template <bool U8>
 int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st) {
   // Tile choice.  Large tiles read fewer operand bytes per multiply-add, and the per-CU load path
-  // is what these kernels run against; but a compute unit needs two wavefronts per SIMD to overlap
-  // LDS waits with matrix work.  So: 256x128 tiles with eight wavefronts when that still gives 160
-  // workgroups (fp16 path); 128x128 with four when every compute unit gets one (two fit and
-  // desynchronise: 344 such tiles at N = 11008 beat 344 workgroups of eight wavefronts); 128x64
-  // with four wavefronts when there are more of them than compute units (two fit); else 128x64
-  // with two groups of four wavefronts splitting the K stage, because then the grid cannot give a
-  // compute unit a second workgroup (M = 512, N = 4096: 35 us against 41 us, K = 11008: 100 us
-  // against 135 us with the register-staged kernel).
+  // is what these kernels run against.  So: tiles of 256 rows when those of 256x128 still give 160
+  // workgroups; 128x128 when these do; 128x64 with four wavefronts when there are more of them than
+  // compute units (two fit); else 128x64 with two groups of four wavefronts splitting the K stage,
+  // because then the grid cannot give a compute unit a second workgroup (M = 512, N = 4096: 35 us
+  // against 41 us, K = 11008: 100 us against 135 us with the register-staged kernel).
   // Several matrices of one shape (op.n_mats > 1) count as one product with n_mats * N columns -- with
   // uint8 weights unless each of them already fills the chip with 256x128 tiles and fusing saves no
   // round of workgroups (fp16 weights choose a wider tile there, large_tile_columns).
@@ -1418,11 +1417,21 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         }
       }
     }
-    if constexpr (!U8) {  // uint8 needs a code ring and two W tiles besides: too much LDS for two workgroups
-      if (tiles128 >= 256) return launch_dl<128, 128, 2, 2, 1, 2, false>(op, A, M, K, N, block, beta, st);
-    }
-    if (tiles128 < 256) {
-      if (tiles128 >= 160) return launch_dl<128, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+    // Tiles of 128x128, the ring of four stages filled by address-free requests: us here against a two-stage ring with two
+    // workgroups per compute unit (from 256 tiles up) or eight wavefronts and three stages (below), M x K x N: 256 tiles
+    // 1000x4096x4096 71 -> 41, 1024x2048x4096 39 -> 24; 288 tiles 1100x4096x4096 55 -> 47; 160 and 192 tiles the same
+    // (512x4096x5120 40, 384x4096x4096 twice 42).  uint8, against eight wavefronts with a
+    // ring of codes or, from 256 tiles up, the register-staged kernel: 1000x4096x4096 67 -> 44, 1100 rows 69 -> 56, 200 rows of
+    // three matrices 55 -> 41, 512x4096x5120 54 -> 39.
+    if (tiles128 >= 160) {
+      if constexpr (U8) {
+        const bool one_chain = tiles128 < 256 || tiles128 / nm >= 256 || tiles64 / nm > 256;  // else half stages are summed apart, below
+        if (block_shift(block) >= 0 && one_chain) return launch_tile<128, 128, 1, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        if (tiles128 < 256) return launch_dl<128, 128, 4, 2, 1, 3, true>(op, A, M, K, N, block, beta, st);
+      } else {
+        return launch_tile<128, 128, 2, 2, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
+      }
+    } else {
       if (tiles64 > 256) return launch_dl<128, 64, 2, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
       return launch_dl<128, 64, 2, 2, 2, 3, U8>(op, A, M, K, N, block, beta, st);
     }
@@ -1534,8 +1543,7 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     return launch_bf16<64, 64, 2, GATED ? 1 : 2, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   }
   if (tm(256) * tn(128) >= 160) return launch_large<false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
-  if (tm(128) * tn(128) > 256) return launch_bf16<128, 128, 2, 2, 1, 2>(ep, A, W, tm(128), M, K, N, st);
-  if (tm(128) * tn(128) >= 160) return launch_bf16<128, 128, 4, 2, 1, 3>(ep, A, W, tm(128), M, K, N, st);
+  if (tm(128) * tn(128) >= 160) return launch_tile<128, 128, 2, 2, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
   if constexpr (GATED) {
     if (tm(128) * tn(64) > 128) return launch_bf16<128, 64, 4, 1, 1, 3>(ep, A, W, tm(128), M, K, N, st);
     return launch_bf16<64, 64, 2, 1, 1, 3>(ep, A, W, tm(64), M, K, N, st);

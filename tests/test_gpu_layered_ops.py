@@ -38,7 +38,8 @@ def test_linear_with_bias_and_gelu_columns(gpu, dt, M, K, N):
 
 # tiles of 256 rows in bfloat16: 192 columns with ragged rows and columns, 256 columns and a single K stage, 128 columns;
 # the last four columns as fp32 of their own
-@pytest.mark.parametrize("M,K,N", [(2049, 192, 4100), (4096, 64, 4096), (300, 320, 12804), (100, 192, 20484), (127, 64, 35000)])
+@pytest.mark.parametrize("M,K,N", [(2049, 192, 4100), (4096, 64, 4096), (300, 320, 12804), (100, 192, 20484), (127, 64, 35000),
+                                   (257, 64, 6790), (1100, 320, 3684)])
 def test_linear_large_tiles(gpu, M, K, N):
     rng = np.random.default_rng(N)
     x, w, b = rounded(rng.standard_normal((M, K))), rounded(rng.standard_normal((N, K)) / K ** 0.5), rng.standard_normal(N)
@@ -61,7 +62,7 @@ def test_linear_large_tiles(gpu, M, K, N):
     gpu.release()
 
 
-@pytest.mark.parametrize("M,K,ff", [(4096, 64, 2048), (2050, 128, 4100), (100, 64, 10250), (70, 128, 17000)])
+@pytest.mark.parametrize("M,K,ff", [(4096, 64, 2048), (2050, 128, 4100), (100, 64, 10250), (70, 128, 17000), (300, 64, 4000)])
 def test_gated_linear_large_tiles(gpu, M, K, ff):
     rng = np.random.default_rng(ff)
     x, gw, uw = rounded(rng.standard_normal((M, K))), rounded(rng.standard_normal((ff, K)) / K ** 0.5), \

@@ -222,7 +222,8 @@ def test_gemm_f16(gpu, M, K, N):
 # tiles of 256 rows at their edges: 192 columns with rows of 4 halves past a 16-byte boundary, 256 columns, 128 columns of one
 # row and column beyond a tile, and K split over workgroups with rows of 2 floats past one; a single K stage pair and many
 @pytest.mark.parametrize("M,K,N", [(2049, 128, 4100), (4096, 256, 4090), (257, 384, 12929), (300, 5120, 1030),
-                                   (65, 128, 20500), (127, 256, 35000), (100, 5120, 1030)])  # and of 128 rows: 128 and 256 columns, K split
+                                   (65, 128, 20500), (127, 256, 35000), (100, 5120, 1030),  # and of 128 rows: 128 and 256 columns, K split
+                                   (257, 128, 6790), (1100, 384, 3690)])  # with more rows: 160 tiles, 261
 def test_gemm_f16_large_tiles_ragged(gpu, M, K, N):
     G = gpu
     x, w, old = normal((M, K), 0, 320, 1.0), normal((N, K), 0, 321, 0.02), normal((M, N), 0, 322, 1.0)
@@ -314,7 +315,8 @@ def test_gemm_f16_few_rows(gpu, M, K, N):
 # uint8 tiles of 256 rows at their edges: 128 and 256 columns, K split over workgroups, blocks of one, two and four K
 # stages, and a block that takes the other kernel
 @pytest.mark.parametrize("M,K,N,block", [(2049, 256, 4100, 64), (4096, 128, 4090, 128), (2300, 512, 6000, 256), (300, 5120, 1030, 128),
-                                         (2049, 128, 4100, 32), (65, 128, 20500, 64), (127, 256, 35000, 128), (100, 5120, 1030, 128)])
+                                         (2049, 128, 4100, 32), (65, 128, 20500, 64), (127, 256, 35000, 128), (100, 5120, 1030, 128),
+                                         (257, 128, 6790, 64), (1100, 384, 3690, 128), (1100, 384, 3690, 32)])
 def test_gemm_u8_large_tiles_ragged(gpu, M, K, N, block):
     G = gpu
     x, w = normal((M, K), 0, 420, 1.0), normal((N, K), 0, 421, 0.02)
