@@ -85,18 +85,19 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
 
   // this wavefront's columns: rows of 128 bytes, 16-byte piece p of row r at p ^ (r / 2) % 8
   const uint32_t ring0 = lds0 + STREAM_LHS + wave * RING * UNIT;
-  uint4_t rw = operand_resource(W), rs = operand_resource(U8 ? (const void*)S : W);
+  uint4_t rw = operand_resource(W, (uint32_t)N * (uint32_t)K * (U8 ? 1u : 2u)), rs = rw;
+  if constexpr (U8) rs = operand_resource(S, (uint32_t)N * ((uint32_t)K >> (6 + block_shift)) * 2u);
   uint32_t w_off[2], s_first = 0;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int row = j * 8 + (lane >> 3), piece = (lane & 7) ^ ((row / 2) % 8);
-    w_off[j] = (uint32_t)min(n0 + row, N - 1) * (uint32_t)K * (U8 ? 1u : 2u) + piece * 16;
+    w_off[j] = row_piece(n0 + row, N, (uint32_t)K * (U8 ? 1u : 2u), piece);
   }
   const int col = lane & 15, group = lane >> 4;
   if constexpr (U8) s_first = (uint32_t)min(n0 + col, N - 1) * ((uint32_t)K >> (6 + block_shift));
   const auto request = [&](int u) {
-    if (u == units) rw[2] = rs[2] = 0;  // behind the last unit: requests that count and touch no memory
-    const uint32_t slot = ring0 + (u % RING) * UNIT, along = (uint32_t)(base * (U8 ? 64 : 128) + u * 128);
+    if (u == units) rw[2] = rs[2] = 0;  // behind the last unit: requests that count and touch no memory (stage_offset)
+    const uint32_t slot = ring0 + (u % RING) * UNIT, along = stage_offset(rw[2], (uint32_t)(base * (U8 ? 64 : 128) + u * 128));
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(w_off[j]), "s"(rw), "s"(along),
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
     }
     if constexpr (U8) {  // the word that holds the row's scales of both stages
       const uint32_t at = s_first + ((uint32_t)(base + 2 * u) >> block_shift);
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"((at & ~1u) * 2u), "s"(rs), "s"(slot + 2048)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(scale_word(at)), "s"(rs), "s"(slot + 2048)
                    : "memory", "m0");
     }
   };

@@ -11,8 +11,8 @@
 //  * a half stage (32 of K) of fragments is read from LDS while the half before it is multiplied, one read
 //    between two matrix instructions; requests for the stage NS ahead go out the same way.
 //  * requests are buffer loads straight into LDS whose stage offset is a scalar.  Behind the last stage the
-//    resource holds no records: the request counts as any other but touches no memory, so that the loop has one
-//    form up to the end and its registers are never copied.
+//    resource holds no records and the offset is 0 (operand_range.hpp): the request counts as any other but touches
+//    no memory, so that the loop has one form up to the end and its registers are never copied.
 //  * outputs go through LDS and leave in 16-byte pieces.
 // LDS stage: rows of 128 bytes, lhs tile then W tile, 16-byte chunk g of row r at position g ^ (r / 2) % 8, so that
 // neither requests (1 KB per instruction, dense) nor fragment reads (16 rows, one chunk) meet in a bank.
@@ -21,6 +21,7 @@
 #include <utility>
 
 #include "linear.hpp"
+#include "operand_range.hpp"
 
 namespace lcu {
 
@@ -43,13 +44,13 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// the buffer resource of an operand below 4 GiB
-__device__ __forceinline__ uint4_t operand_resource(const void* p) {
+// the buffer resource of an operand of `bytes` (below 4 GiB)
+__device__ __forceinline__ uint4_t operand_resource(const void* p, uint32_t bytes) {
   const uintptr_t a = (uintptr_t)p;
   uint4_t r;
   r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
   r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
-  r[2] = 0xffffffffu;
+  r[2] = __builtin_amdgcn_readfirstlane(bytes);
   r[3] = 0x00020000u;
   return r;
 }
@@ -140,17 +141,17 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 #pragma unroll
   for (int j = 0; j < PA; ++j) {
     const int c = (wave + j * NW) * 64 + lane, row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
-    a_off[j] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)K + g * 8) * 2u;
+    a_off[j] = row_piece(m0 + row, M, (uint32_t)K * 2u, g);
   }
 #pragma unroll
   for (int j = 0; j < PB; ++j) {
     const int c = (wave + j * NW) * 64 + lane;
     if constexpr (U8) {
       const int row = c / 4, g = (c % 4) ^ (2 * ((row / 4) % 2));
-      b_off[j] = (uint32_t)min(n0 + row, N - 1) * (uint32_t)K + g * 16;
+      b_off[j] = row_piece(n0 + row, N, (uint32_t)K, g);
     } else {
       const int row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
-      b_off[j] = ((uint32_t)min(n0 + row, N - 1) * (uint32_t)K + g * 8) * 2u;
+      b_off[j] = row_piece(n0 + row, N, (uint32_t)K * 2u, g);
     }
   }
   // first scale of the rows whose scales this lane requests, and of those of its fragments
@@ -162,7 +163,8 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 #pragma unroll
     for (int j = 0; j < TN; ++j) f_first[j] = (uint32_t)min(n0 + wn + j * 16 + (lane & 15), N - 1) * blocks;
   }
-  uint4_t ra = operand_resource(A), rw = operand_resource(W), rs = operand_resource(U8 ? (const void*)S : (const void*)A);
+  uint4_t ra = operand_resource(A, (uint32_t)M * (uint32_t)K * 2u), rw = operand_resource(W, (uint32_t)N * (uint32_t)K * (U8 ? 1u : 2u)), rs = ra;
+  if constexpr (U8) rs = operand_resource(S, (uint32_t)N * ((uint32_t)K >> (6 + block_shift)) * 2u);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)tile_lds;
   // Inline assembly, so that the compiler does not know about the LDS writes: knowing, it waits for every LDS read
   // in front of each matrix instruction.  There is no output register; the waits are the explicit ones below.
@@ -172,14 +174,14 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
                  : "memory", "m0");
   };
   const auto issue = [&](int stage, int slot, int i) {
-    const uint32_t along = (uint32_t)(stage0 + stage) * 128u;
+    const uint32_t along = stage_offset(ra[2], (uint32_t)(stage0 + stage) * 128u);
     if (i < PA) {
       request(ra, along, a_off[i], slot * STAGE + (wave + i * NW) * 1024);
     } else if (i < PA + PB) {
       request(rw, U8 ? along / 2 : along, b_off[i - PA], slot * STAGE + A_BYTES + (wave + (i - PA) * NW) * 1024);
     } else if constexpr (U8) {  // the word that holds the row's scale of this stage
       const uint32_t at = s_first[i - PA - PB] + ((uint32_t)(stage0 + stage) >> block_shift);
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"((at & ~1u) * 2u), "s"(rs),
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(scale_word(at)), "s"(rs),
                    "s"(lds0 + slot * STAGE + A_BYTES + B_BYTES + wave * shape::SW * 4 + (i - PA - PB) * 256)
                    : "memory", "m0");
     }
@@ -296,7 +298,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    if (s == nt) ra[2] = rw[2] = rs[2] = 0;  // no records: a request brings zeros and reads nothing
+    if (s == nt) ra[2] = rw[2] = rs[2] = 0;  // no records: a request brings zeros and reads nothing (stage_offset)
 #pragma unroll
     for (int i = 0; i < P; ++i) issue(s, s, i);
   }
