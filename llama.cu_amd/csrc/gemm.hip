@@ -1425,8 +1425,12 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
     // three matrices 55 -> 41, 512x4096x5120 54 -> 39.
     if (tiles128 >= 160) {
       if constexpr (U8) {
-        const bool one_chain = tiles128 < 256 || tiles128 / nm >= 256 || tiles64 / nm > 256;  // else half stages are summed apart, below
-        if (block_shift(block) >= 0 && one_chain) return launch_tile<128, 128, 1, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        // Several matrices, each with so few tiles that a call of its own would sum the half stages apart: so does their common
+        // launch, on the kernel that such a call takes (512 rows, three times 3072x3072: 86 us on the register-staged
+        // kernel, 75 in separate calls, 71 here; blocks of 32 96 / 77 / 73; 1000 rows, twice 2048 columns of K 4608 85 / 76 / 74).
+        const bool one_chain = tiles128 < 256 || tiles128 / nm >= 256 || tiles64 / nm > 256;
+        if (!one_chain) return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);
+        if (block_shift(block) >= 0) return launch_tile<128, 128, 1, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
         if (tiles128 < 256) return launch_dl<128, 128, 4, 2, 1, 3, true>(op, A, M, K, N, block, beta, st);
       } else {
         return launch_tile<128, 128, 2, 2, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);

@@ -329,7 +329,9 @@ def test_gemm_u8_large_tiles_ragged(gpu, M, K, N, block):
 
 
 @pytest.mark.parametrize("M,K,N,count", [(512, 512, 4096, 3), (8, 4096, 4096, 3), (40, 1024, 11008, 2), (300, 256, 700, 2),
-                                          (33, 200, 70, 3), (1, 512, 300, 3)])
+                                          (33, 200, 70, 3), (1, 512, 300, 3),
+                                          # uint8: each alone has few tiles, together they have many
+                                          (512, 256, 3072, 3), (1000, 384, 1990, 2)])
 def test_gemm_multi_matches_separate_calls(gpu, M, K, N, count):
     """Several weight matrices of one shape in one launch (Wq, Wk, Wv; W1, W3): what separate calls give
     (to the matmul tolerance: the fused launch may pick another tile shape, hence another summation order)
