@@ -1055,24 +1055,6 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
 }
 
 // ---- prompts -------------------------------------------------------------------------------------
-// exp_ieee for x <= 0 (and NaN): the scaling by 2^k in one step, k's bits taken from the sum that rounds to it.
-// The same bits for every x in [-104, 0] and below, in two thirds of the instructions.
-__device__ __forceinline__ float exp_ieee_nonpositive(float x) {
-  const float magic = x * 1.44269504f + 12582912.0f;
-  const float kf = magic - 12582912.0f;
-  float r = fmaf(kf, -0.693359375f, x);
-  r = fmaf(kf, 2.12194440e-4f, r);
-  float p = 1.9875691500e-4f;
-  p = fmaf(p, r, 1.3981999507e-3f);
-  p = fmaf(p, r, 8.3334519073e-3f);
-  p = fmaf(p, r, 4.1665795894e-2f);
-  p = fmaf(p, r, 1.6666665459e-1f);
-  p = fmaf(p, r, 5.0000001201e-1f);
-  p = fmaf(p * r, r, r) + 1.0f;
-  const float scale = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, magic) << 23) + 0x3f800000u);
-  return x < -87.33654f ? 0.0f : p * scale;
-}
-
 // Attention of many rows: NW wavefronts of 16 rows each share the K and V of their head in chunks of 64 cache rows,
 // which travel into a ring of four 16 KB LDS slots, three ahead.
 //

@@ -96,7 +96,7 @@ __device__ __forceinline__ half_t round_f16(float f) {
 // ln 2 split in two; a degree-7 polynomial in r (Cephes' coefficients); the result scaled by 2^k in
 // two steps.  Results below the smallest normal number are returned as 0 and arguments above
 // 88.72283 as infinity, whatever the denormal mode of the machine.
-__device__ __forceinline__ float exp_ieee(float x) {
+__host__ __device__ __forceinline__ float exp_ieee(float x) {
   if (x > 88.72283f) return __builtin_inff();
   if (x < -87.33654f) return 0.0f;
   const float kf = __builtin_rintf(x * 1.44269504f);
@@ -117,9 +117,32 @@ __device__ __forceinline__ float exp_ieee(float x) {
   return res < 1.17549435e-38f ? 0.0f : res;
 }
 
-// x / d from the correctly rounded reciprocal of d: quotient, exact remainder, correction.  Correctly rounded
-// for finite x and normal results; what is below the normal numbers is 0 in fp16 either way.
-__device__ __forceinline__ float divide_by(float x, float d, float reciprocal) {
+// exp_ieee for x <= 0 (and NaN): the scaling by 2^k in one step, k's bits taken from the sum that rounds to it.
+// The same bits for every x <= 0 in two thirds of the instructions, provided that no multiply-add is contracted
+// (tests/cxx/kernel_arithmetic.hip goes through all x in [-104, 0]; below -87.33654 both are 0).
+__host__ __device__ __forceinline__ float exp_ieee_nonpositive(float x) {
+  const float magic = x * 1.44269504f + 12582912.0f;
+  const float kf = magic - 12582912.0f;
+  float r = fmaf(kf, -0.693359375f, x);
+  r = fmaf(kf, 2.12194440e-4f, r);
+  float p = 1.9875691500e-4f;
+  p = fmaf(p, r, 1.3981999507e-3f);
+  p = fmaf(p, r, 8.3334519073e-3f);
+  p = fmaf(p, r, 4.1665795894e-2f);
+  p = fmaf(p, r, 1.6666665459e-1f);
+  p = fmaf(p, r, 5.0000001201e-1f);
+  p = fmaf(p * r, r, r) + 1.0f;
+  const float scale = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, magic) << 23) + 0x3f800000u);
+  return x < -87.33654f ? 0.0f : p * scale;
+}
+
+// x / d from the correctly rounded reciprocal of d: quotient, remainder, correction (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990).  Where the remainder is exact the result is
+// the correctly rounded quotient; the remainder loses bits when it falls among the subnormals, which takes an x below
+// 2^-100: rounded to fp16 the quotients are equal all the same.  For finite x: an infinite one leaves NaN.
+// (tests/cxx/kernel_arithmetic.hip: every x with the attention's divisor, every pair of halves that the quantiser
+// divides, samples of the probabilities.)
+__host__ __device__ __forceinline__ float divide_by(float x, float d, float reciprocal) {
   const float q = x * reciprocal;
   return fmaf(fmaf(-q, d, x), reciprocal, q);
 }

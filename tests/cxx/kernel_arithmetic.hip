@@ -1,0 +1,107 @@
+// The kernels' shortened exponential and division (csrc/common.hpp), compiled for the host, against what they stand for.
+// Each part prints how many of its inputs differ; the exit code says whether any does that must not.
+#include <math.h>
+#include <stdint.h>
+#include <stdio.h>
+#include <string.h>
+
+#include <atomic>
+#include <functional>
+#include <random>
+#include <thread>
+#include <vector>
+
+#include "common.hpp"
+
+namespace {
+
+float of_bits(uint32_t u) { return __builtin_bit_cast(float, u); }
+uint32_t bits(float f) { return __builtin_bit_cast(uint32_t, f); }
+uint16_t half_bits(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
+
+// f(first, last) over pieces of [0, n); the sum of what it returns
+long in_pieces(uint64_t n, const std::function<long(uint64_t, uint64_t)>& f) {
+  std::atomic<uint64_t> next{0};
+  std::atomic<long> sum{0};
+  std::vector<std::thread> threads;
+  const uint64_t piece = n / 256 + 1;
+  for (int t = 0; t < 8; ++t) {
+    threads.emplace_back([&] {
+      for (uint64_t at; (at = next.fetch_add(piece)) < n;) sum += f(at, at + piece < n ? at + piece : n);
+    });
+  }
+  for (auto& t : threads) t.join();
+  return sum;
+}
+
+int failed = 0;
+void report(const char* what, long differ) {
+  printf("%s: %ld differ\n", what, differ);
+  failed |= differ != 0;
+}
+
+}  // namespace
+
+int main() {
+  // the exponential: every float in [-104, -0], steps of 16 values from there to -infinity, and NaN
+  const uint32_t far = bits(-104.0f), low = bits(-INFINITY);
+  report("exp of all x in [-104, 0]", in_pieces(far - 0x80000000u + 1, [](uint64_t a, uint64_t b) {
+           long n = 0;
+           for (uint64_t i = a; i < b; ++i) {
+             const float x = of_bits(0x80000000u + (uint32_t)i);
+             n += bits(lcu::exp_ieee(x)) != bits(lcu::exp_ieee_nonpositive(x));
+           }
+           return n;
+         }));
+  long rest = lcu::exp_ieee_nonpositive(0.0f) != 1.0f || !isnan(lcu::exp_ieee_nonpositive(NAN));
+  for (uint64_t u = far; u <= low; u += 16) rest += lcu::exp_ieee_nonpositive(of_bits((uint32_t)u)) != 0.0f;
+  report("exp below", rest + (lcu::exp_ieee_nonpositive(-INFINITY) != 0.0f));
+
+  // scores: every finite x over sqrt(128) (the operation is odd in x)
+  const float denom = sqrtf(128.0f), inverse = 1.0f / denom;
+  std::atomic<long> small{0};
+  report("x / sqrt(128), fp16, or fp32 for x of 2^-100 and more", in_pieces(0x7f800000u, [&](uint64_t a, uint64_t b) {
+           long n = 0, s = 0;
+           for (uint64_t i = a; i < b; ++i) {
+             const float x = of_bits((uint32_t)i), want = x / denom, got = lcu::divide_by(x, denom, inverse);
+             if (bits(got) == bits(want)) continue;
+             ++s;
+             n += x >= 0x1p-100f || half_bits(got) != half_bits(want);
+           }
+           small += s;
+           return n;
+         }));
+  printf("  (%ld smaller ones differ in fp32)\n", small.load());
+
+  // the quantiser: every pair of a normal fp16 scale and an fp16 value with a quotient of up to 300
+  report("halves over fp16 scales", in_pieces(0x7c00 - 0x0400, [](uint64_t a, uint64_t b) {
+           long n = 0;
+           for (uint64_t i = a; i < b; ++i) {
+             const float s = (float)__builtin_bit_cast(_Float16, (uint16_t)(0x0400 + i)), inverse = 1.0f / s;
+             for (uint32_t h = 0; h < 0x7c00; ++h) {
+               const float x = (float)__builtin_bit_cast(_Float16, (uint16_t)h), want = x / s;
+               if (want > 300.0f) break;
+               n += bits(lcu::divide_by(x, s, inverse)) != bits(want);
+             }
+           }
+           return n;
+         }));
+
+  // probabilities: exponentials (0 and 2^-126 .. 1) over sums in [1, 4096], with significands at both ends among the sums
+  report("samples of e / sum, fp16, or fp32 for e of 2^-100 and more", in_pieces(4096, [](uint64_t a, uint64_t b) {
+           long n = 0;
+           for (uint64_t t = a; t < b; ++t) {
+             std::mt19937 random((uint32_t)t);
+             float s = of_bits(0x3f800000u + random() % (12u << 23));
+             if (t < 400) s = of_bits((bits(s) & 0xff800000u) | (t < 200 ? (uint32_t)t : 0x7fffffu - (uint32_t)(t - 200)));
+             const float share = 1.0f / s;
+             for (int i = 0; i < 50000; ++i) {
+               const float e = i == 0 ? 0.0f : of_bits(0x00800000u + random() % (0x3f800001u - 0x00800000u));
+               const float want = e / s, got = lcu::divide_by(e, s, share);
+               n += bits(got) != bits(want) && (e >= 0x1p-100f || half_bits(got) != half_bits(want));
+             }
+           }
+           return n;
+         }));
+  return failed;
+}

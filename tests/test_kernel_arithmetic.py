@@ -1,4 +1,5 @@
-"""Arithmetic of the kernels that can be checked whole without a GPU: the addresses their requests ask for."""
+"""Arithmetic of the kernels that can be checked whole without a GPU: the addresses their requests ask for, and the
+exponential and the division in fewer instructions."""
 import os
 import subprocess
 
@@ -24,3 +25,12 @@ def test_requests_stay_in_their_operands(operand_range):
 def test_a_scalar_offset_without_a_length_would_be_found(operand_range):
     res = subprocess.run([operand_range, "offset"], capture_output=True, text=True)
     assert res.returncode == 1 and " 0 reach" not in res.stdout, res.stdout
+
+
+def test_short_exponential_and_division(tmp_path):
+    """exp_ieee_nonpositive has exp_ieee's bits, and divide_by the quotient's where the kernels use it."""
+    exe = str(tmp_path / "kernel_arithmetic")
+    subprocess.run(["hipcc", "-x", "hip", "--offload-host-only", "-O2", "-std=c++17", "-ffp-contract=off", "-mfma", "-mf16c", "-I", CSRC,
+                    "-I", os.path.join(ROOT, "include"), os.path.join(CXX, "kernel_arithmetic.hip"), "-o", exe], check=True)
+    res = subprocess.run([exe], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
