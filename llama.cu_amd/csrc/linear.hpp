@@ -27,12 +27,26 @@ struct clamped_gate {
   }
 };
 
-// GROUPED: rows are sorted by group (expert); row tile t belongs to group tile_group[t], starts at row
+// Rows that are sorted by group (expert): row tile t belongs to group tile_group[t], starts at row
 // tile_row[t] and ends at the group's end; group g multiplies matrix W + g * group_stride bytes; row r of lhs
-// is row row_index[r] of the array when row_index is given.
+// is row row_index[r] of the array when row_index is given.  Products of ungrouped rows have none of this.
+template <bool GROUPED>
+struct row_groups {};
+template <>
+struct row_groups<true> {
+  const float* row_scale;  // factor of row r of lhs, or nullptr (gated products only)
+  const int* tile_group;
+  const int* tile_row;
+  const int* group_end;
+  const int* n_tiles;
+  const int* row_index;
+  size_t group_stride;
+  int tile_rows;
+};
+
 // GATED: the matrix holds, in blocks of 64 rows, 32 gate rows and the 32 up rows of the same hidden columns.
 template <bool GROUPED_, bool GATED_>
-struct linear_epilogue {
+struct linear_epilogue : row_groups<GROUPED_> {
   static constexpr bool BF16 = true, GROUPED = GROUPED_, GATED = GATED_;
   void* out;
   int ldo;
@@ -42,14 +56,6 @@ struct linear_epilogue {
   float* tail;               // fp32 rows [ld_tail] of the columns from tail_from on, or nullptr
   int tail_from, ld_tail;
   clamped_gate gate;
-  const float* row_scale;    // factor of row r of lhs, or nullptr (gated products only)
-  const int* tile_group;
-  const int* tile_row;
-  const int* group_end;
-  const int* n_tiles;
-  const int* row_index;
-  size_t group_stride;
-  int tile_rows;
 
   __device__ __forceinline__ void put(int m, int n, float v) const {
     const size_t at = (size_t)m * ldo + n;
@@ -104,8 +110,11 @@ struct linear_epilogue {
     }
   }
   __device__ __forceinline__ void store_gated(int m, int n, float g, float u) const {
-    const float s = row_scale ? row_scale[m] : 1.0f;
-    put(m, n, gate(g * s, u * s));
+    if constexpr (GROUPED) {
+      const float s = this->row_scale ? this->row_scale[m] : 1.0f;
+      g *= s, u *= s;
+    }
+    put(m, n, gate(g, u));
   }
 };
 

@@ -9,9 +9,18 @@
 #include <functional>
 #include <random>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
-#include "common.hpp"
+#include "linear.hpp"
+
+// the factor of a row belongs to grouped products: other kernels do not apply it, so no other epilogue can carry it
+template <class EP, class = void>
+constexpr bool has_row_scale = false;
+template <class EP>
+constexpr bool has_row_scale<EP, std::void_t<decltype(EP::row_scale)>> = true;
+static_assert(has_row_scale<lcu::linear_epilogue<true, true>> && !has_row_scale<lcu::linear_epilogue<false, true>> &&
+              !has_row_scale<lcu::linear_epilogue<false, false>>);
 
 namespace {
 
