@@ -54,12 +54,15 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
   extern __shared__ __attribute__((aligned(16))) unsigned char stream_mem[];
   const int waves = blockDim.x >> 6;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // tiles of one matrix, then of the next, then the same of the next split
-  const int mats = more.tiles_n_per;
-  const int split = blockIdx.x / (tiles * mats), rest = blockIdx.x % (tiles * mats), g = rest / tiles;
+  // Tiles of one matrix, then of the next; the same for the next split.  Consecutive workgroups go round the eight XCDs: each
+  // gets one run of the tiles, the same of every split, so that what adds the splits up may find them in one L2 (bfloat16,
+  // 8 rows, 4096x2048, both launches: 11.9 us with the tiles dealt one by one, 8.3 so; fp16 4096x32000 66 / 61).
+  const int mats = more.tiles_n_per, nb = tiles * mats;
+  const int split = blockIdx.x / nb, bx = blockIdx.x - split * nb, xcd = bx % 8;
+  const int rest = xcd * (nb / 8) + min(xcd, nb % 8) + bx / 8, g = rest / tiles;
   const void* W = g == 0 ? W0 : (g == 1 ? more.W[0] : more.W[1]);
   const half_t* S = g == 0 ? S0 : (g == 1 ? more.S[0] : more.S[1]);
-  const int n0 = ((rest % tiles) * waves + wave) * 16;
+  const int n0 = ((rest - g * tiles) * waves + wave) * 16;
   const bool mine = n0 < N;
   const int nt_all = K / 64;
   const int stage0 = (int)((long)split * nt_all / splits), stage1 = (int)((long)(split + 1) * nt_all / splits);
