@@ -921,10 +921,13 @@ int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N,
 // with 256 columns, 330 us with 128).  uint8: 128 / 256 columns 65 / 113 us (512 rows, K 6656, three times 6656 columns:
 // 156 tiles of 256 168 us, 312 of 128 187 us; 1987 rows, twice 11008 columns 346 / 374 us, three times 4096 226 / 196 us).
 // Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts there.
+// Up to 512 of K what a tile pays beside its stages counts: 256 columns leave by four wavefronts, and the rounds are no measure of
+// them (1441 rows of K 256, three times 2944 columns: 216 tiles of 256 20.1 us, 414 of 128 16.5; bfloat16 1027x512x11840 28.7 / 23.4),
+// and 192 no gain below 256.
 // Up to 128 rows: tiles of 128 rows, a round of 128 / 256 columns taking 52 / 66 us in fp16 and 42 / 62 in uint8 (100
 // rows, twice 11008 columns 61 -> 52 us and 55 -> 42 against tiles of 256 rows; twice 17920 of K 6656 140 -> 118 and 170 -> 109).
 template <bool U8>
-int large_tile_columns(int M, int N, int n_mats, long cus, bool gated) {
+int large_tile_columns(int M, int K, int N, int n_mats, long cus, bool gated) {
   const auto cost = [&](int columns, int round) {
     const long tiles = (long)((M + 255) / 256) * ((N + columns - 1) / columns) * n_mats;
     return (tiles + cus - 1) / cus * round;
@@ -934,15 +937,15 @@ int large_tile_columns(int M, int N, int n_mats, long cus, bool gated) {
     return cost(256, 113) < cost(128, 65) ? 256 : 128;
   } else {
     const long c128 = cost(128, 57), c192 = gated ? c128 : cost(192, 88), c256 = cost(256, 106);
-    if (c256 < c128 && c256 <= c192) return 256;
-    return c192 < c128 ? 192 : 128;
+    if (K >= 640 && c256 < c128 && c256 <= c192) return 256;
+    return K >= 256 && c192 < c128 ? 192 : 128;
   }
 }
 
 template <bool U8, class EP>
 int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st) {
   device_state* ds = current_device_state();
-  const int columns = large_tile_columns<U8>(M, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
+  const int columns = large_tile_columns<U8>(M, K, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
   if (M <= 128) {
     if constexpr (U8) {
       if (columns == 256) return launch_tile<128, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
@@ -1349,15 +1352,17 @@ int launch_gemm(half_t* out, const half_t* A, const void* W, const half_t* S, in
 
 template <bool U8>
 int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st) {
-  // Tile choice.  Large tiles read fewer operand bytes per multiply-add, and the per-CU load path
-  // is what these kernels run against.  So: tiles of 256 rows when those of 256x128 still give 160
-  // workgroups; 128x128 when these do; 128x64 with four wavefronts when there are more of them than
-  // compute units (two fit); else 128x64 with two groups of four wavefronts splitting the K stage,
-  // because then the grid cannot give a compute unit a second workgroup (M = 512, N = 4096: 35 us
-  // against 41 us, K = 11008: 100 us against 135 us with the register-staged kernel).
-  // Several matrices of one shape (op.n_mats > 1) count as one product with n_mats * N columns -- with
-  // uint8 weights unless each of them already fills the chip with 256x128 tiles and fusing saves no
-  // round of workgroups (fp16 weights choose a wider tile there, large_tile_columns).
+  // Tile choice.  Large tiles read fewer operand bytes per multiply-add and pay per output for fewer
+  // barriers.  So: tiles of 256 rows when those of 256x128 still give 160 workgroups, or with few of them
+  // and a long K the splits of each (large_tile_splits); 128x128 when these give 160; 128x64 with four
+  // wavefronts when there are more of them than compute units (two fit); else 128x64 with two groups of four
+  // wavefronts splitting the K stage, because then the grid cannot give a compute unit a second workgroup
+  // (512x4096x4096 29 us, with one group 34, on the register-staged kernel 36.5; 400x2048x2048 13.6, 17.5, 19.1).
+  // gemm_tile_kernel pays about 1 us more per tile before its first and behind its last stage than gemm_dl_kernel (a longer ring
+  // to fill, outputs through LDS) and less per stage: over a short K the other kernels stay, by the lines below.
+  // Several matrices of one shape (op.n_mats > 1) count as one product with n_mats * N columns; only uint8
+  // weights in blocks other than 64 << n, whose kernel has one width of large tiles, take a launch each where
+  // a matrix fills the chip with 256x128 tiles and fusing saves no round of workgroups.
   const bool whole_stages = K % 128 == 0 && scale_words_ok<U8>(op, K, N, block);
   if (U8 && block_shift(block) < 0 && op.n_mats > 1 && M > 64 && whole_stages) {
     device_state* ds = current_device_state();
@@ -1395,7 +1400,14 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
     const long tiles256 = (long)((M + 255) / 256) * ((N + 127) / 128) * nm;
     if (tiles256 >= 160) {
       if constexpr (U8) {
-        if (block_shift(block) < 0) return launch_dl<256, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+        // over a short K gemm_dl_kernel is done sooner (us, it / gemm_tile_kernel, K 256, 512, 768: 512 rows of 12288 columns 11.2 / 12.4,
+        // 15.1 / 16.2, 18.7 / 18.3; several rounds of workgroups, 1015 rows, three times 4096 columns of K 256 20.2 / 22.0, 1805
+        // rows, three times 8256 of K 384 85.6 / 90.3, 1987 rows, three times 4096 of K 512 52.2 / 46.9)
+        device_state* ds = current_device_state();
+        const bool one_round = tiles256 <= (ds && ds->compute_units > 0 ? ds->compute_units : 256);
+        if (block_shift(block) < 0 || (M > 128 && K < (one_round ? 640 : 448))) {
+          return launch_dl<256, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+        }
       }
       return launch_large<U8>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
     }
@@ -1425,9 +1437,17 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         // kernel, 75 in separate calls, 71 here; blocks of 32 96 / 77 / 73; 1000 rows, twice 2048 columns of K 4608 85 / 76 / 74).
         const bool one_chain = tiles128 < 256 || tiles128 / nm >= 256 || tiles64 / nm > 256;
         if (!one_chain) return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);
-        if (block_shift(block) >= 0) return launch_tile<128, 128, 1, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        // us, the older kernel / here, K 256, 512, 1024, 2048: 512 rows of 5120 columns 7.6 / 7.8, 10.5 / 9.8, 16.3 / 13.7; one matrix with
+        // more tiles than compute units, which the register-staged kernel puts two to a compute unit, 1000 rows of 4608 columns
+        // 11.4 / 14.0, 15.8 / 17.8, 24.5 / 25.6, 41.9 / 41.6
+        const bool long_enough = tiles128 < 256 ? K >= 384 : tiles128 / nm <= 256 || K >= 1536;
+        if (block_shift(block) >= 0 && long_enough) return launch_tile<128, 128, 1, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
         if (tiles128 < 256) return launch_dl<128, 128, 4, 2, 1, 3, true>(op, A, M, K, N, block, beta, st);
       } else {
+        // us, K 256, 512, 1024, 1536, 2048: eight wavefronts / here, 512 rows of 5120 columns 6.2 / 7.1, 7.8 / 8.5, 10.9 / 11.2, 16.1 / 15.2, 22.0 / 22.3;
+        // two workgroups per compute unit / here, 1000 rows of 4608 columns 9.6 / 12.4, 13.2 / 15.7, 20.8 / 21.4, 29.3 / 27.9, 39.5 / 35.1
+        if (K < 1280 && tiles128 < 256) return launch_dl<128, 128, 4, 2, 1, 3, false>(op, A, M, K, N, block, beta, st);
+        if (K < 1280 && tiles128 > 256) return launch_dl<128, 128, 2, 2, 1, 2, false>(op, A, M, K, N, block, beta, st);
         return launch_tile<128, 128, 2, 2, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
       }
     } else {
@@ -1540,6 +1560,9 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     return launch_bf16<64, 64, 2, GATED ? 1 : 2, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   }
   if (tm(256) * tn(128) >= 160) return launch_large<false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
+  if constexpr (GATED) {  // 1000 rows of 4608 columns, K 512, 1024, 2048: 17.2 us, 24.5, 43.1 with two workgroups per compute unit, else 17.8, 24.8, 39.7
+    if (K < 1280 && tm(128) * tn(128) > 256) return launch_bf16<128, 128, 2, 2, 1, 2>(ep, A, W, tm(128), M, K, N, st);
+  }
   if (tm(128) * tn(128) >= 160) return launch_tile<128, 128, 2, 2, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
   if constexpr (GATED) {
     if (tm(128) * tn(64) > 128) return launch_bf16<128, 64, 4, 1, 1, 3>(ep, A, W, tm(128), M, K, N, st);

@@ -75,6 +75,17 @@ def test_gated_linear_large_tiles(gpu, M, K, ff):
     gpu.release()
 
 
+# 128 or 256 columns by the length of K; gated tiles of 128x128 that outnumber the compute units, on both sides of theirs
+@pytest.mark.parametrize("M,K,N", [(1441, 512, 8900), (1441, 640, 8900)])
+def test_linear_large_tiles_by_length(gpu, M, K, N):
+    test_linear_large_tiles(gpu, M, K, N)
+
+
+@pytest.mark.parametrize("M,K,ff", [(1100, 1216, 1850), (1100, 1280, 1850), (1441, 640, 4400)])
+def test_gated_linear_tiles_by_length(gpu, M, K, ff):
+    test_gated_linear_large_tiles(gpu, M, K, ff)
+
+
 @BOTH
 @pytest.mark.parametrize("M,K,ff", [(1, 64, 32), (5, 128, 40), (66, 192, 100), (200, 128, 640), (700, 64, 1000), (2, 1024, 70), (40, 768, 500)])
 def test_gated_linear_clamps(gpu, dt, M, K, ff):

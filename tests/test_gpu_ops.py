@@ -233,6 +233,34 @@ def test_gemm_f16_large_tiles_ragged(gpu, M, K, N):
     G.release()
 
 
+# both sides of the lengths of K that decide between the kernels: fp16 with 160 .. 255 tiles of 128x128 and more, 128 or 256 columns
+# of large tiles; the cases above whose K is short, with a long one
+@pytest.mark.parametrize("M,K,N,count", [(257, 1152, 6790, 1), (257, 1280, 6790, 1), (1100, 1152, 3690, 1), (1100, 1280, 3690, 1),
+                                         (1441, 512, 2900, 3), (1441, 640, 2900, 3), (2049, 640, 4100, 1), (300, 640, 12930, 1)])
+def test_gemm_f16_short_and_long_k(gpu, M, K, N, count):
+    G = gpu
+    VP = G.B.vp
+    x, ws = normal((M, K), 0, 330, 1.0), [normal((N, K), 0, 331 + g, 0.02) for g in range(count)]
+    wd, outs = [G.dev_keep(w) for w in ws], [G.empty((M, N)) for _ in ws]
+    G.B.check(G.L().lcu_gemm_f16_nt_multi((VP * count)(*[o.ptr for o in outs]), G.dev_keep(x).ptr, (VP * count)(*[w.ptr for w in wd]), count,
+                                          M, K, N, 0.0, None))
+    for o, w in zip(outs, ws):
+        assert G.ulp_mismatch(G.host(o, (M, N)), O.matmul_nt_kernel_order(x, w, n_mats=count)) == 0.0, O.gemm_plan(M, K, N)
+    G.release()
+
+
+# the same for codes: 160 .. 255 tiles of 128x128, more, one round of large tiles and several
+@pytest.mark.parametrize("M,K,N,block", [(257, 256, 6790, 128), (257, 384, 6790, 64), (1100, 1408, 3690, 128), (1100, 1536, 3690, 128),
+                                         (1030, 512, 4100, 128), (1030, 640, 4100, 128), (2049, 384, 4100, 64), (2049, 512, 4100, 256)])
+def test_gemm_u8_short_and_long_k(gpu, M, K, N, block):
+    G = gpu
+    x, w = normal((M, K), 0, 340, 1.0), normal((N, K), 0, 341, 0.02)
+    codes, scales = O.quantize_absmax_u8(w, block)
+    got = G.gemm_u8(x, codes, scales, block)
+    assert G.ulp_mismatch(got, O.matmul_nt_u8(x, codes, scales, block, flavour=2)) == 0.0, O.gemm_plan(M, K, N, True)
+    G.release()
+
+
 def test_gemm_residual_into_an_output_that_is_not_16_byte_aligned(gpu):
     """beta = 1 with the output tile 8 bytes off a 16-byte boundary: the tile that fetches its old values in 16-byte
     pieces (512 x 4096 x 4096, the Wo product) must fall back to 2-byte reads; same bits as the aligned call."""
