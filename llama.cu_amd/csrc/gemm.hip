@@ -337,8 +337,8 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(
 // dequantised once per block tile and the fragment path is the fp16 one.  The chunk's scale comes
 // by an ordinary 2-byte load one stage earlier.
 //
-// SPLIT (few tiles; uint8 weights in blocks other than 64 << n): the grid holds `splits` workgroups per
-// tile, each taking a contiguous run of the K stages and writing its fp32 sums to part[split][M][N];
+// SPLIT (few rows, so few tiles): the grid holds `splits` workgroups per tile, each taking a
+// contiguous run of the K stages and writing its fp32 sums to part[split][M][N];
 // splitk_reduce_kernel adds them in split order and applies the epilogue.
 //
 // EP: what the accumulators become.  f16_epilogue is the fp16 output described above.  The bfloat16
@@ -749,7 +749,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS <= 4 ? 2 : 1) void 
     }
   }
   if constexpr (EP::BF16) {
-    static_assert(!U8 && !SPLIT, "bfloat16 operands are neither quantised nor split here");
+    static_assert(!U8, "bfloat16 operands are not quantised");
     if (group == 0) {
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
@@ -757,7 +757,13 @@ __global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS <= 4 ? 2 : 1) void 
         for (int v = 0; v < 16; ++v) {
           const int gm = m0 + wm + i * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
           if (gm >= M) continue;
-          if constexpr (EP::GATED) {
+          if constexpr (SPLIT) {  // the epilogue belongs to the launch that adds the splits
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+              const int gn = n0 + wn + j * 32 + (lane & 31);
+              if (gn < N) part[((size_t)split * M + gm) * N + gn] = acc[i][j][v];
+            }
+          } else if constexpr (EP::GATED) {
             // 32 columns of gate rows, then the 32 of the up rows they belong to: one lane holds both
             static_assert(TN == 2, "a wavefront's columns are one gate / up pair of blocks");
             const int hc = (n0 + wn) / 2 + (lane & 31);
@@ -973,21 +979,22 @@ struct partial_sums_t {
   int splits;
 };
 
-// uint8 weights in blocks other than 64 << n: BM x BN tiles of WM x WN wavefronts, the K stages of every
-// tile dealt to `splits` workgroups (gemm_dl_kernel<.., SPLIT = true>), fp32 partial sums in the stream's
-// workspace, then splitk_reduce_kernel -- or the caller's own kernel when `leave` is given.
-template <int BM, int BN, int WM, int WN>
+// BM x BN tiles of WM x WN wavefronts, the K stages of every tile dealt to `splits` workgroups
+// (gemm_dl_kernel<.., SPLIT = true>), fp32 partial sums in the stream's workspace, then
+// splitk_reduce_kernel -- or the caller's own kernel when `leave` is given.
+template <int BM, int BN, int WM, int WN, bool U8>
 int launch_split(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits,
                  float* part, partial_sums_t* leave = nullptr) {
   constexpr int KS = 1, NS = 3;
   constexpr int ROWB = BK * KS * 2;
-  constexpr int DCH = BN * (BK * KS / 16) / (64 * WM * WN * KS);
-  constexpr size_t lds = (size_t)NS * BM * ROWB + (size_t)2 * BN * ROWB + (size_t)NS * (BN * BK * KS + 64 * WM * WN * KS * 4 * DCH);
+  constexpr int DCH = U8 ? BN * (BK * KS / 16) / (64 * WM * WN * KS) : 0;
+  constexpr size_t lds = (size_t)NS * BM * ROWB + (size_t)(U8 ? 2 : NS) * BN * ROWB +
+                         (U8 ? (size_t)NS * (BN * BK * KS + 64 * WM * WN * KS * 4 * DCH) : 0);
   static_assert(lds <= 160 * 1024, "LDS");
   const int tiles_m = (M + BM - 1) / BM, tiles_n_per = (N + BN - 1) / BN, tiles_n = tiles_n_per * op.n_mats;
   op.more.tiles_n_per = op.n_mats > 1 ? tiles_n_per : 0;
   const size_t mn = (size_t)M * N;
-  auto kernel = gemm_dl_kernel<BM, BN, WM, WN, KS, NS, true, true>;
+  auto kernel = gemm_dl_kernel<BM, BN, WM, WN, KS, NS, U8, true>;
   if constexpr (lds > 64 * 1024) {
     static bool raised[16] = {};  // per device, once
     int dev = 0;
@@ -1012,8 +1019,7 @@ int launch_split(operands_t op, const half_t* A, int M, int K, int N, int block,
 }
 
 // Wavefronts (of 16 columns) per workgroup of gemm_stream_kernel: one workgroup runs per compute unit, so the longest
-// compute unit has rounds * wavefronts of them to stream; below four a compute unit has too little in flight (8 rows, three
-// times 2048x2048: nine rounds of single wavefronts 19.6 us, one of ten 10.7).
+// compute unit has rounds * wavefronts of them to stream; below four a compute unit has too little in flight.
 inline int stream_waves(int N, int n_mats, int splits, long cus, int most) {
   const long groups = (N + 15) / 16;
   int best = 1;
@@ -1058,8 +1064,7 @@ int launch_stream(operands_t op, const void* A, int M, int K, int N, int block, 
 
 // Few rows (2 .. 64: short prompts, where the reference takes its 16-row tile, llama_cu.cu:1481-1484):
 // the K stages split as BM x 128 tiles would need to give every compute unit one workgroup; gemm_stream_kernel
-// walks the splits (blocks of codes other than 64 << n: such tiles with four wavefronts).  Returns LCU_OK with
-// *done = false when the shape does not suit it.
+// walks the splits (blocks of codes other than 64 << n: such tiles with four wavefronts).  Returns LCU_OK with *done = false when the shape does not suit it.
 template <int BM, bool U8>
 int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st,
                   bool* done, partial_sums_t* leave = nullptr) {
@@ -1088,7 +1093,7 @@ int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block
   int rc;
   if constexpr (U8) {
     if (block_shift(block) < 0) {
-      rc = launch_split<BM, BN, 1, 4>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
+      rc = launch_split<BM, BN, 1, 4, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
       *done = rc == LCU_OK;
       return rc;
     }
@@ -1418,7 +1423,7 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         const int splits = large_tile_splits(M, K, N, op.n_mats, ds->compute_units > 0 ? ds->compute_units : 256, ws.bytes);
         if (splits > 0) {
           if constexpr (U8) {
-            if (block_shift(block) < 0) return launch_split<256, 128, 4, 2>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
+            if (block_shift(block) < 0) return launch_split<256, 128, 4, 2, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
           }
           return launch_large_split<U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr);
         }
@@ -1477,13 +1482,15 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
 }
 
 // ---- bfloat16 operands ----
-template <int BM, int BN, int WM, int WN, int KS, int NS, class EP>
-int launch_bf16(EP const& ep, const void* A, const void* W, int tiles_m, int M, int K, int N, hipStream_t st) {
+// splits > 1: the K stages of every tile dealt to that many workgroups, fp32 sums to part (no epilogue)
+template <int BM, int BN, int WM, int WN, int KS, int NS, bool SPLIT = false, class EP>
+int launch_bf16(EP const& ep, const void* A, const void* W, int tiles_m, int M, int K, int N, hipStream_t st, int splits = 1,
+                float* part = nullptr) {
   constexpr int ROWB = BK * KS * 2;
   constexpr size_t lds = (size_t)NS * (BM + BN) * ROWB;
   static_assert(lds <= 160 * 1024, "rings do not fit LDS");
   static_assert(KS == 1 || lds >= (size_t)BM * BN * 4 / 2, "LDS must hold one group's accumulators");
-  auto kernel = gemm_dl_kernel<BM, BN, WM, WN, KS, NS, false, false, EP>;
+  auto kernel = gemm_dl_kernel<BM, BN, WM, WN, KS, NS, false, SPLIT, EP>;
   if constexpr (lds > 64 * 1024) {
     static bool raised[16] = {};  // per device, once
     int dev = 0;
@@ -1495,8 +1502,8 @@ int launch_bf16(EP const& ep, const void* A, const void* W, int tiles_m, int M, 
   }
   const int tiles_n = (N + BN - 1) / BN;
   const more_matrices_t none{{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}, 0};
-  kernel<<<tiles_m * tiles_n, 64 * WM * WN * KS, lds, st>>>(nullptr, (const half_t*)A, W, nullptr, M, K, N, 0, 0.0f, tiles_m,
-                                                            tiles_n, nullptr, 1, none, ep);
+  kernel<<<tiles_m * tiles_n * splits, 64 * WM * WN * KS, lds, st>>>(nullptr, (const half_t*)A, W, nullptr, M, K, N, 0, 0.0f,
+                                                                     tiles_m, tiles_n, part, splits, none, ep);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
