@@ -337,9 +337,9 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(
 // dequantised once per block tile and the fragment path is the fp16 one.  The chunk's scale comes
 // by an ordinary 2-byte load one stage earlier.
 //
-// SPLIT (few rows, so few tiles): the grid holds `splits` workgroups per tile, each taking a
-// contiguous run of the K stages and writing its fp32 sums to part[split][M][N];
-// splitk_reduce_kernel adds them in split order and applies the epilogue.
+// SPLIT (few rows that gemm_stream_kernel leaves, blocks of codes other than 64 << n): the grid holds
+// `splits` workgroups per tile, each taking a contiguous run of the K stages and writing its fp32 sums to
+// part[split][M][N]; splitk_reduce_kernel adds them in split order and applies the epilogue.
 //
 // EP: what the accumulators become.  f16_epilogue is the fp16 output described above.  The bfloat16
 // epilogues (linear.hpp) take bfloat16 operands, which travel exactly like the fp16 ones, through
@@ -1019,8 +1019,9 @@ int launch_split(operands_t op, const half_t* A, int M, int K, int N, int block,
 }
 
 // Wavefronts (of 16 columns) per workgroup of gemm_stream_kernel: one workgroup runs per compute unit, so the longest
-// compute unit has rounds * wavefronts of them to stream; below four a compute unit has too little in flight.
-inline int stream_waves(int N, int n_mats, int splits, long cus, int most) {
+// compute unit has rounds * wavefronts of them to stream; below four a compute unit has too little in flight (8 rows, three
+// times 2048x2048: nine rounds of single wavefronts 19.6 us, one of ten 10.7).  *rounds: how many they are.
+inline int stream_waves(int N, int n_mats, int splits, long cus, int most, long* rounds) {
   const long groups = (N + 15) / 16;
   int best = 1;
   long least = 0;
@@ -1030,14 +1031,27 @@ inline int stream_waves(int N, int n_mats, int splits, long cus, int most) {
     if (w == 1 || cost <= least) {
       least = cost;
       best = w;
+      *rounds = (wgs + cus - 1) / cus;
     }
   }
   return best;
 }
 
+// Whether a product of few rows is one of gemm_stream_kernel, or of BM x 128 tiles of four wavefronts.  Of those several share a
+// compute unit; a workgroup here has it alone, so that a second round fills lhs and ring again with nothing beside it.  us, tiles /
+// here, 8 and 32 rows: fp16 2048x32000 (two rounds) 27.7 / 33.9, 30.7 / 37.6, 4096x32000 56.0 / 56.4, 58.5 / 58.6, 5888x9664 three
+// times (three) 62 / 67, 67 / 77; one round 4096x11008 twice 43.8 / 41.9, 46.5 / 42.9 (45 rows).  uint8 gains more in a round: 4096x11008
+// twice (two) 36.6 / 32.7 with 16 rows, 37.6 / 40.4 with 32, 4096x32000 37.2 / 32.9, 39.8 / 42.8, 5888x9664 three times 56 / 61, 56 / 81.
+inline bool streams(int M, int N, int n_mats, int splits, long cus, bool u8) {
+  long rounds = 1;
+  stream_waves(N, n_mats, splits, cus, stream_max_waves(u8), &rounds);
+  return rounds == 1 || (u8 && M <= 16 && rounds == 2);
+}
+
 template <int TM, bool U8, bool BF16>
 int launch_stream_rows(operands_t op, const void* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, long cus) {
-  const int waves = stream_waves(N, op.n_mats, splits, cus, stream_max_waves(U8)), tiles = ((N + 15) / 16 + waves - 1) / waves;
+  long rounds = 1;
+  const int waves = stream_waves(N, op.n_mats, splits, cus, stream_max_waves(U8), &rounds), tiles = ((N + 15) / 16 + waves - 1) / waves;
   op.more.tiles_n_per = op.n_mats;
   auto kernel = gemm_stream_kernel<TM, U8, BF16>;
   static bool raised[16] = {};  // per device, once
@@ -1064,7 +1078,8 @@ int launch_stream(operands_t op, const void* A, int M, int K, int N, int block, 
 
 // Few rows (2 .. 64: short prompts, where the reference takes its 16-row tile, llama_cu.cu:1481-1484):
 // the K stages split as BM x 128 tiles would need to give every compute unit one workgroup; gemm_stream_kernel
-// walks the splits (blocks of codes other than 64 << n: such tiles with four wavefronts).  Returns LCU_OK with *done = false when the shape does not suit it.
+// walks the splits, or such tiles with four wavefronts do (`streams`; blocks of codes other than 64 << n).
+// Returns LCU_OK with *done = false when the shape does not suit it.
 template <int BM, bool U8>
 int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st,
                   bool* done, partial_sums_t* leave = nullptr) {
@@ -1091,12 +1106,10 @@ int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block
     return LCU_OK;
   }
   int rc;
-  if constexpr (U8) {
-    if (block_shift(block) < 0) {
-      rc = launch_split<BM, BN, 1, 4, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
-      *done = rc == LCU_OK;
-      return rc;
-    }
+  if ((U8 && block_shift(block) < 0) || !streams(M, N, op.n_mats, splits, ds->compute_units, U8)) {
+    rc = launch_split<BM, BN, 1, 4, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
+    *done = rc == LCU_OK;
+    return rc;
   }
   rc = launch_stream<U8, false>(op, A, M, K, N, block, st, splits, (float*)ws.ptr, ds->compute_units);
   if (rc == LCU_OK && leave) {
@@ -1541,7 +1554,13 @@ int bf16_skinny(linear_epilogue<false, GATED> const& ep, const void* A, const vo
   while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws.bytes) --splits;
   if (splits < 2) return LCU_OK;
   float* part = (float*)ws.ptr;
-  const int rc = launch_stream<false, true>(single_matrix(nullptr, W, nullptr), A, M, K, N, 0, st, splits, part, ds->compute_units);
+  int rc;
+  if (streams(M, N, 1, splits, ds->compute_units, false)) {
+    rc = launch_stream<false, true>(single_matrix(nullptr, W, nullptr), A, M, K, N, 0, st, splits, part, ds->compute_units);
+  } else {
+    rc = M <= 32 ? launch_bf16<32, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part)
+                 : launch_bf16<64, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part);
+  }
   if (rc != LCU_OK) return rc;
   const int outs = M * (GATED ? N / 2 : N);
   splitk_epilogue_kernel<GATED><<<(outs + 255) / 256, 256, 0, st>>>(ep, part, M, N, splits);

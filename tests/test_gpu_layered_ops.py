@@ -76,12 +76,13 @@ def test_gated_linear_large_tiles(gpu, M, K, ff):
 
 
 # 128 or 256 columns by the length of K; gated tiles of 128x128 that outnumber the compute units, on both sides of theirs
-@pytest.mark.parametrize("M,K,N", [(1441, 512, 8900), (1441, 640, 8900)])
+@pytest.mark.parametrize("M,K,N", [(1441, 512, 8900), (1441, 640, 8900),
+                                   (8, 512, 30000), (40, 640, 25000)])  # few rows in two rounds of workgroups
 def test_linear_large_tiles_by_length(gpu, M, K, N):
     test_linear_large_tiles(gpu, M, K, N)
 
 
-@pytest.mark.parametrize("M,K,ff", [(1100, 1216, 1850), (1100, 1280, 1850), (1441, 640, 4400)])
+@pytest.mark.parametrize("M,K,ff", [(1100, 1216, 1850), (1100, 1280, 1850), (1441, 640, 4400), (20, 512, 13000), (6, 2816, 1020)])
 def test_gated_linear_tiles_by_length(gpu, M, K, ff):
     test_gated_linear_large_tiles(gpu, M, K, ff)
 

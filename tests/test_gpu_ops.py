@@ -320,7 +320,8 @@ def test_gemm_u8(gpu, M, K, N):
 # few rows, codes: runs of K stages that begin in the middle of 128 codes, one to four row tiles, lhs in one piece and in
 # chunks, one and two scales in 128 codes, and a block that takes the other kernel
 @pytest.mark.parametrize("M,K,N,block", [(2, 1152, 520, 64), (16, 1152, 4100, 128), (17, 2560, 1000, 256), (33, 1152, 5000, 64),
-                                         (64, 5888, 4100, 128), (64, 1152, 3000, 384), (7, 17920, 6656, 128)])
+                                         (64, 5888, 4100, 128), (64, 1152, 3000, 384), (7, 17920, 6656, 128),
+                                         (16, 512, 32000, 128), (17, 512, 32000, 64)])  # two rounds of workgroups, both kernels
 def test_gemm_u8_few_rows(gpu, M, K, N, block):
     G = gpu
     x, w = normal((M, K), 0, 430, 1.0), normal((N, K), 0, 431, 0.02)
@@ -331,7 +332,8 @@ def test_gemm_u8_few_rows(gpu, M, K, N, block):
 
 
 # few rows, fp16: odd runs, rows past the last whole tile, columns past the last whole wavefront, lhs in chunks
-@pytest.mark.parametrize("M,K,N", [(3, 1152, 520), (16, 1408, 4099), (31, 2944, 1000), (48, 5888, 4100), (64, 4096, 24000)])
+@pytest.mark.parametrize("M,K,N", [(3, 1152, 520), (16, 1408, 4099), (31, 2944, 1000), (48, 5888, 4100), (64, 4096, 24000),
+                                   (8, 512, 32000), (40, 640, 31000)])  # two rounds of workgroups: the other kernel
 def test_gemm_f16_few_rows(gpu, M, K, N):
     G = gpu
     x, w, old = normal((M, K), 0, 440, 1.0), normal((N, K), 0, 441, 0.02), normal((M, N), 0, 442, 1.0)
@@ -359,7 +361,9 @@ def test_gemm_u8_large_tiles_ragged(gpu, M, K, N, block):
 @pytest.mark.parametrize("M,K,N,count", [(512, 512, 4096, 3), (8, 4096, 4096, 3), (40, 1024, 11008, 2), (300, 256, 700, 2),
                                           (33, 200, 70, 3), (1, 512, 300, 3),
                                           # uint8: each alone has few tiles, together they have many
-                                          (512, 256, 3072, 3), (1000, 384, 1990, 2)])
+                                          (512, 256, 3072, 3), (1000, 384, 1990, 2),
+                                          # few rows whose columns take two and three rounds of one workgroup per compute unit
+                                          (8, 640, 9664, 3), (33, 512, 9664, 3), (9, 512, 31990, 2)])
 def test_gemm_multi_matches_separate_calls(gpu, M, K, N, count):
     """Several weight matrices of one shape in one launch (Wq, Wk, Wv; W1, W3): what separate calls give
     (to the matmul tolerance: the fused launch may pick another tile shape, hence another summation order)
