@@ -133,9 +133,11 @@ __device__ __forceinline__ int key_place(int r) { return (r & ~31) + ((r >> 2) &
 
 // KP: 32-column pieces of a key.  With registers for keys of 256 whatever their size, one wavefront per SIMD was all that
 // fits at values of 128; two or three do now.  2048 tokens, 32 heads, values of 128: keys of 192 over all and keys of 128 in a window
-// of 1024 took 216 us on average, 167 and 86 now.
-template <int DV, bool BIAS, int KP>
-__global__ __launch_bounds__(256, DV <= 128 && KP <= 6 ? 2 : 1) void attention_tile_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
+// of 1024 took 233 and 157 us, 134 and 80 now.
+// OCC: wavefronts per SIMD that the registers are cut to.  Asked for two, the compiler puts the sums among the other registers and may
+// fit another wavefront, but each takes longer for a tile: launch_tiles.
+template <int DV, bool BIAS, int KP, int OCC>
+__global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                                                              const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, int n,
                                                              int start, window_args p) {
   constexpr int NT = DV / 16, LDP = KT + 8, VP = (DV + 63) / 64;  // KP, VP: pieces of a tile per thread
@@ -295,11 +297,11 @@ __global__ __launch_bounds__(256, DV <= 128 && KP <= 6 ? 2 : 1) void attention_t
 
 size_t tile_lds(int dk, int dv) { return ((size_t)KT * (dk + 8) + (size_t)dv * (KT + 8)) * 2; }
 
-template <int DV, bool BIAS, int KP>
+template <int DV, bool BIAS, int KP, int OCC>
 int launch_tiles_of(void* out, const void* q, const void* k, const void* v, int n, int start, const window_args& p, hipStream_t st) {
   const size_t lds = tile_lds(p.dk, DV);
   LCU_REQUIRE(lds <= 160 * 1024, "lcu_attention_windowed: head size %d with value size %d", p.dk, DV);
-  auto kernel = attention_tile_kernel<DV, BIAS, KP>;
+  auto kernel = attention_tile_kernel<DV, BIAS, KP, OCC>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -313,11 +315,24 @@ int launch_tiles_of(void* out, const void* q, const void* k, const void* v, int 
   return LCU_OK;
 }
 
+// us, registers cut to two wavefronts / to one, where more fit all the same.  Keys of 192 are done sooner with one at every size (32 heads,
+// values of 128, 100 rows behind 1500 109 / 90, 2048 rows 150 / 134; values of 64 92 / 73).  Keys of 128 with values of 128 fit three
+// wavefronts in place of two when cut, which pays where the grid has more than that for every SIMD (32 heads, 2048 rows in a window of
+// 1024 80 / 106, 3000 rows 196 / 245) and costs where it has not (32 heads, 100 rows behind 3000 185 / 151; 64 heads, 500 behind 1000
+// 89 / 78; 16 heads, 3000 rows 166 / 143).  With values of 64 keys of 64 gain by the cut (512 rows 16.6 / 17.4), keys of 128 lose (32
+// heads, 100 rows behind 3000 144 / 119).
 template <int DV, bool BIAS>
 int launch_tiles(void* out, const void* q, const void* k, const void* v, int n, int start, const window_args& p, hipStream_t st) {
-  if (p.dk <= 128) return launch_tiles_of<DV, BIAS, 4>(out, q, k, v, n, start, p, st);
-  if (p.dk <= 192) return launch_tiles_of<DV, BIAS, 6>(out, q, k, v, n, start, p, st);
-  return launch_tiles_of<DV, BIAS, 8>(out, q, k, v, n, start, p, st);
+  if (p.dk <= 128) {
+    if constexpr (DV <= 128) {
+      device_state* ds = current_device_state();
+      const long cus = ds && ds->compute_units > 0 ? ds->compute_units : 256;
+      if (DV == 128 ? (long)((n + QT - 1) / QT) * p.heads > 3 * cus : p.dk <= 64) return launch_tiles_of<DV, BIAS, 4, 2>(out, q, k, v, n, start, p, st);
+    }
+    return launch_tiles_of<DV, BIAS, 4, 1>(out, q, k, v, n, start, p, st);
+  }
+  if (p.dk <= 192) return launch_tiles_of<DV, BIAS, 6, 1>(out, q, k, v, n, start, p, st);
+  return launch_tiles_of<DV, BIAS, 8, 1>(out, q, k, v, n, start, p, st);
 }
 
 // ---- one new token, bfloat16 ----------------------------------------------------------------------------

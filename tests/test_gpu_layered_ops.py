@@ -303,10 +303,18 @@ def test_windowed_attention_in_portions(gpu, dt, heads, kv, dim, vdim, window, k
 
 
 # key sizes on both sides of what the tile kernel keeps registers for
-@pytest.mark.parametrize("dim,vdim", [(128, 128), (129, 64), (192, 128), (193, 200), (256, 32)])
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (129, 64), (192, 128), (193, 200), (256, 32), (64, 64), (65, 33)])
 def test_windowed_attention_key_sizes(gpu, dim, vdim):
     c = attention_case(gpu, BF16, 4, 2, dim, vdim, 90, 3, 150, dim)
     close(run_attention(gpu, c, BF16, (150,)), c["want"], BF16, bf16=2.0 ** -7)
+    gpu.release()
+
+
+# 768 workgroups and more: the form that fits three to a compute unit
+@pytest.mark.parametrize("heads,T", [(128, 384), (112, 390), (112, 449)])
+def test_windowed_attention_many_workgroups(gpu, heads, T):
+    c = attention_case(gpu, BF16, heads, 4, 120, 128, 90, 3, T, heads)
+    close(run_attention(gpu, c, BF16, (T,)), c["want"], BF16, bf16=2.0 ** -7)
     gpu.release()
 
 
