@@ -673,53 +673,51 @@ __global__ __launch_bounds__(256) void quantize_kernel(uint8_t* __restrict__ cod
   }
 }
 
-// The same for blocks of 8 L elements, L a power of two up to 64: a lane holds eight neighbouring elements, L lanes a block, and
-// every lane asks for four such pieces at once.  Bound by HBM: 4096 x 11008 (136 MB) 117 -> 30 us, against 2-byte loads and a
-// wavefront per block.  Where the scale is a normal number the quotient is taken from its reciprocal and the exact
-// remainder (divide_by), which gives the correctly rounded one for every pair of halves with a quotient below 300.
+// The same for blocks of 8 L elements, L a power of two up to 64: a lane holds eight neighbouring elements, L lanes a block.  Bound
+// by HBM: 4096 x 11008 (136 MB) 117 -> 29 us, against 2-byte loads and a wavefront per block.  Where the scale is a normal number the
+// quotient is taken from its reciprocal and the exact remainder (divide_by), which gives the correctly rounded one for every
+// pair of halves with a quotient below 300.  (Four pieces to a lane, asked for together: 0.2 to 0.8 us slower in all sizes, 4096 x 4096
+// 14.0 / 11.7 us.)
 template <int L>
 __global__ __launch_bounds__(256) void quantize_pieces_kernel(uint8_t* __restrict__ codes, half_t* __restrict__ scales,
                                                               const half_t* __restrict__ in, size_t pieces) {
-  constexpr int AT_ONCE = 4;
-  const size_t first = (size_t)blockIdx.x * 256 * AT_ONCE + threadIdx.x;
-  half8_t x[AT_ONCE];
+  const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const half8_t x = at < pieces ? *reinterpret_cast<const half8_t*>(in + at * 8) : (half8_t)(0.0f);
+  float top = 0.0f;
 #pragma unroll
-  for (int i = 0; i < AT_ONCE; ++i) {
-    const size_t at = first + i * 256;
-    x[i] = at < pieces ? *reinterpret_cast<const half8_t*>(in + at * 8) : (half8_t)(0.0f);
-  }
-#pragma unroll
-  for (int i = 0; i < AT_ONCE; ++i) {
-    const size_t at = first + i * 256;
-    float top = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf((float)x[i][e]));
-    if constexpr (L > 1) top = fmaxf(top, dpp_f32<0xB1>(top));   // lanes 1 apart, 2 apart, then mirrored within 8 and 16
-    if constexpr (L > 2) top = fmaxf(top, dpp_f32<0x4E>(top));
-    if constexpr (L > 4) top = fmaxf(top, dpp_f32<0x141>(top));
-    if constexpr (L > 8) top = fmaxf(top, dpp_f32<0x140>(top));
-    if constexpr (L > 16) top = fmaxf(top, __shfl_xor(top, 16, WAVE));
-    if constexpr (L > 32) top = fmaxf(top, __shfl_xor(top, 32, WAVE));
-    if (at >= pieces) continue;  // whole blocks: the lanes of one go the same way
-    const half_t sh = round_f16(top / 127.5f);
-    if (threadIdx.x % L == 0) scales[at / L] = sh;
-    const float s = (float)sh;
-    const bool normal = s >= 6.103515625e-5f && s < 65536.0f;
+  for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf((float)x[e]));
+  if constexpr (L > 1) top = fmaxf(top, dpp_f32<0xB1>(top));   // lanes 1 apart, 2 apart, then mirrored within 8 and 16
+  if constexpr (L > 2) top = fmaxf(top, dpp_f32<0x4E>(top));
+  if constexpr (L > 4) top = fmaxf(top, dpp_f32<0x141>(top));
+  if constexpr (L > 8) top = fmaxf(top, dpp_f32<0x140>(top));
+  if constexpr (L > 16) top = fmaxf(top, __shfl_xor(top, 16, WAVE));
+  if constexpr (L > 32) top = fmaxf(top, __shfl_xor(top, 32, WAVE));
+  if (at >= pieces) return;  // whole blocks: the lanes of one go the same way
+  const half_t sh = round_f16(top / 127.5f);
+  if (threadIdx.x % L == 0) scales[at / L] = sh;
+  const float s = (float)sh;
+  float quotient[8];
+  if (s >= 6.103515625e-5f && s < 65536.0f) {
     const float inverse = 1.0f / s;
-    uint32_t word[2] = {0, 0};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float v = roundf(127.5f + (normal ? divide_by((float)x[i][e], s, inverse) : (float)x[i][e] / s));
-      const uint32_t code = v >= 255.0f ? 255u : (v > 0.0f ? (uint32_t)v : 0u);
-      word[e / 4] |= code << (e % 4 * 8);
-    }
-    *reinterpret_cast<uint2_t*>(codes + at * 8) = uint2_t{word[0], word[1]};
+    for (int e = 0; e < 8; ++e) quotient[e] = divide_by((float)x[e], s, inverse);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) quotient[e] = (float)x[e] / s;
   }
+  uint32_t word[2] = {0, 0};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = roundf(127.5f + quotient[e]);
+    const uint32_t code = v >= 255.0f ? 255u : (v > 0.0f ? (uint32_t)v : 0u);
+    word[e / 4] |= code << (e % 4 * 8);
+  }
+  *reinterpret_cast<uint2_t*>(codes + at * 8) = uint2_t{word[0], word[1]};
 }
 
 template <int L>
 int launch_quantize_pieces(uint8_t* codes, half_t* scales, const half_t* in, size_t pieces, hipStream_t st) {
-  quantize_pieces_kernel<L><<<(unsigned)((pieces + 1023) / 1024), 256, 0, st>>>(codes, scales, in, pieces);
+  quantize_pieces_kernel<L><<<(unsigned)((pieces + 255) / 256), 256, 0, st>>>(codes, scales, in, pieces);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
@@ -1110,7 +1108,7 @@ int lcu_quantize_absmax_u8(void* codes_dev, void* scales_dev, const void* in_dev
   LCU_REQUIRE((n_blocks + 3) / 4 < ((size_t)1 << 31), "lcu_quantize_absmax_u8: tensor too large");
   const size_t pieces = n_blocks * (size_t)(block / 8);
   if (block % 8 == 0 && reinterpret_cast<uintptr_t>(in_dev) % 16 == 0 && reinterpret_cast<uintptr_t>(codes_dev) % 8 == 0 &&
-      (pieces + 1023) / 1024 < ((size_t)1 << 31)) {
+      (pieces + 255) / 256 < ((size_t)1 << 31)) {
     uint8_t* codes = (uint8_t*)codes_dev;
     half_t* scales = (half_t*)scales_dev;
     const half_t* in = (const half_t*)in_dev;
