@@ -1371,8 +1371,10 @@ int lcu_attention(void* out_dev, const void* q_dev, const void* k_dev, const voi
   // what LDS holds from about 0.17 M scores per us on; the lines cross where the call has 11 000 scores per column
   // (heads, n = T, us here against below: 32 heads 512 rows 35 / 25, 700 rows 46 / 47, 1024 rows 67 / 143, 1987 rows 155 / 502;
   // 52 heads 512 rows 35 / 37; 4 heads 1500 rows 89 / 90; 32 heads 64 rows of 1000 62 / 38, 512 rows of 2048 122 / 214).
+  // Its requests and stores are of 16 and 8 bytes: operands that are not so aligned stay with the kernel below.
   const double scores = (double)n_heads * n_new * (start_pos + 0.5 * n_new);
-  if (scores >= 11000.0 * T) {
+  const bool aligned = (((uintptr_t)q_dev | (uintptr_t)k_dev | (uintptr_t)v_dev) & 15) == 0 && ((uintptr_t)out_dev & 7) == 0;
+  if (scores >= 11000.0 * T && aligned) {
     // 128 rows to a workgroup read K and V half as often, if two workgroups per compute unit are left
     if ((long)((n_new + 127) / 128) * n_heads >= 512) {
       return launch_prompt_attention<8>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T,

@@ -765,6 +765,22 @@ def test_attention_of_many_scores(gpu, heads, n, T):
     G.release()
 
 
+@pytest.mark.parametrize("shift", [1, 4])
+def test_attention_of_many_scores_into_an_output_off_16_bytes(gpu, shift):
+    """An output 2 bytes off any boundary goes to the kernel that stores 2 bytes at a time, one of 8 bytes need not; same bits."""
+    G = gpu
+    heads, n, dim = 40, 601, 5120
+    q, k, v = normal((n, dim), 0, 1023, 1.0), normal((n, dim), 0, 1024, 1.0), normal((n, dim), 0, 1025, 1.0)
+    qd, kd, vd = G.dev_keep(q), G.dev_keep(k), G.dev_keep(v)
+    flat, out = G.dev(np.full(n * dim + 8, 9.0, np.float16)), G.empty((n, dim))
+    G.B.check(G.L().lcu_attention(out.ptr, qd.ptr, kd.ptr, vd.ptr, n, n, 0, dim, heads, None))
+    G.B.check(G.L().lcu_attention(flat.ptr + 2 * shift, qd.ptr, kd.ptr, vd.ptr, n, n, 0, dim, heads, None))
+    got = G.host(flat, (n * dim + 8,))
+    assert G.ulp_mismatch(got[shift:shift + n * dim].reshape(n, dim), G.host(out, (n, dim))) == 0.0
+    assert (got[:shift] == 9.0).all() and (got[shift + n * dim:] == 9.0).all()
+    G.release()
+
+
 def test_attention_of_many_scores_equals_portions(gpu):
     """One call against portions of 16 rows, which take the other kernel: the same bits, also with scores past the
     range of fp16, products past that of fp32 (infinite operands), NaN, and rows that see equal scores only."""
