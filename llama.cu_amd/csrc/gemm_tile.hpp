@@ -326,7 +326,10 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   constexpr int OC = EP::GATED ? shape::WC / 2 : shape::WC;  // output columns of the wavefront
   constexpr int PIECES = OC / 8;                             // pieces of eight columns per row, and per lane
   const int out_n0 = EP::GATED ? (n0 + wn) / 2 : n0 + wn, out_n = EP::GATED ? N / 2 : N;
-  const bool whole = !EP::BF16 && !SPLIT && N % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;  // 16-byte rows
+  // Pieces of eight columns leave as 16 bytes wherever a row begins, its last ones one by one (fp16 1401x384x16515: 39 us so,
+  // 75 with single stores for rows off 16 bytes).
+  typedef half8_t any_half8_t __attribute__((aligned(2)));
+  typedef float4_t any_float4_t __attribute__((aligned(4)));
   const auto pass = [&](auto which) {
     constexpr int p = decltype(which)::value;
 #pragma unroll
@@ -354,11 +357,11 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     for (int k0 = 0; k0 < PIECES; k0 += AT_ONCE) {
       half8_t old[AT_ONCE];
       if constexpr (!EP::BF16 && !SPLIT) {
-        if (beta != 0.0f && whole) {
+        if (beta != 0.0f) {
 #pragma unroll
           for (int k = 0; k < AT_ONCE; ++k) {
             const int c = lane + 64 * (k0 + k), gm = m0 + wm + p * 64 + c / PIECES, gn = out_n0 + c % PIECES * 8;
-            if (gm < M && gn < N) old[k] = *reinterpret_cast<const half8_t*>(out + (size_t)gm * N + gn);
+            if (gm < M && gn + 8 <= N) old[k] = *reinterpret_cast<const any_half8_t*>(out + (size_t)gm * N + gn);
           }
         }
       }
@@ -371,9 +374,9 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
         if (gm >= M || gn >= out_n) continue;
         if constexpr (SPLIT) {
           float* to = part + ((size_t)split * M + gm) * N + gn;
-          if (N % 4 == 0 && gn + 8 <= N) {
-            *reinterpret_cast<float4_t*>(to) = lo;
-            *reinterpret_cast<float4_t*>(to + 4) = hi;
+          if (gn + 8 <= N) {
+            *reinterpret_cast<any_float4_t*>(to) = lo;
+            *reinterpret_cast<any_float4_t*>(to + 4) = hi;
           } else {
             for (int e = 0; e < 8 && gn + e < N; ++e) to[e] = x[e];
           }
@@ -381,11 +384,11 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
           ep.store8(gm, gn, x, out_n);
         } else {
           half_t* to = out + (size_t)gm * N + gn;
-          if (whole) {  // llama_cu.cu:208-215: fp16(acc + beta * old)
+          if (gn + 8 <= N) {  // llama_cu.cu:208-215: fp16(acc + beta * old)
             half8_t y;
 #pragma unroll
             for (int e = 0; e < 8; ++e) y[e] = round_f16(beta != 0.0f ? fmaf(beta, (float)old[k][e], x[e]) : x[e]);
-            *reinterpret_cast<half8_t*>(to) = y;
+            *reinterpret_cast<any_half8_t*>(to) = y;
           } else {
             for (int e = 0; e < 8 && gn + e < N; ++e) to[e] = round_f16(beta != 0.0f ? fmaf(beta, (float)to[e], x[e]) : x[e]);
           }

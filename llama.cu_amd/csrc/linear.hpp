@@ -74,11 +74,9 @@ struct linear_epilogue : row_groups<GROUPED_> {
     }
     put(m, n, v);
   }
-  // eight neighbouring columns of `columns`, from a multiple of eight on: in 16-byte pieces where rows allow them
+  // eight neighbouring columns of `columns`, from a multiple of eight on: in 16-byte pieces, wherever the row begins, but at its end and in the tail
   __device__ __forceinline__ void store8(int m, int n, const float (&x)[8], int columns) const {
-    const bool wide = n + 8 <= columns && (!tail || n + 8 <= tail_from) && ldo % (out_f32 ? 4 : 8) == 0 &&
-                      (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    if (!wide) {
+    if (n + 8 > columns || (tail && n + 8 > tail_from)) {
       for (int e = 0; e < 8 && n + e < columns; ++e) {
         if constexpr (GATED) {
           put(m, n + e, x[e]);
@@ -99,14 +97,16 @@ struct linear_epilogue : row_groups<GROUPED_> {
     }
     const size_t at = (size_t)m * ldo + n;
     if (out_f32) {
-      float4_t* to = reinterpret_cast<float4_t*>(reinterpret_cast<float*>(out) + at);
+      typedef float4_t any_float4_t __attribute__((aligned(4)));
+      any_float4_t* to = reinterpret_cast<any_float4_t*>(reinterpret_cast<float*>(out) + at);
       to[0] = float4_t{y[0], y[1], y[2], y[3]};
       to[1] = float4_t{y[4], y[5], y[6], y[7]};
     } else {
       bf16x8_t v;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = (bf16_t)y[e];
-      *reinterpret_cast<bf16x8_t*>(reinterpret_cast<bf16_t*>(out) + at) = v;
+      typedef bf16x8_t any_bf16x8_t __attribute__((aligned(2)));
+      *reinterpret_cast<any_bf16x8_t*>(reinterpret_cast<bf16_t*>(out) + at) = v;
     }
   }
   __device__ __forceinline__ void store_gated(int m, int n, float g, float u) const {

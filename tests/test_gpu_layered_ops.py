@@ -59,6 +59,10 @@ def test_linear_large_tiles(gpu, M, K, N):
     out = zeros(gpu, (M, N + 1))
     call(gpu, "lcu_linear", out, 1, N + 1, xd, wd, None, 0, BF16, M, K, N)   # rows off any 16-byte boundary
     close(get(gpu, out, (M, N + 1))[:, :N], x @ w.T, F32)
+    out = zeros(gpu, (M, N + 1), BF16)
+    call(gpu, "lcu_linear", out, 0, N + 1, xd, wd, None, 0, BF16, M, K, N)
+    close(get(gpu, out, (M, N + 1), BF16)[:, :N], x @ w.T, BF16)
+    assert (get(gpu, out, (M, N + 1), BF16)[:, N:] == 0).all()
     gpu.release()
 
 
