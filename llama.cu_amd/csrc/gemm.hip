@@ -1041,11 +1041,20 @@ inline int stream_waves(int N, int n_mats, int splits, long cus, int most, long*
 // compute unit; a workgroup here has it alone, so that a second round fills lhs and ring again with nothing beside it.  us, tiles /
 // here, 8 and 32 rows: fp16 2048x32000 (two rounds) 27.7 / 33.9, 30.7 / 37.6, 4096x32000 56.0 / 56.4, 58.5 / 58.6, 5888x9664 three
 // times (three) 62 / 67, 67 / 77; one round 4096x11008 twice 43.8 / 41.9, 46.5 / 42.9 (45 rows).  uint8 gains more in a round: 4096x11008
-// twice (two) 36.6 / 32.7 with 16 rows, 37.6 / 40.4 with 32, 4096x32000 37.2 / 32.9, 39.8 / 42.8, 5888x9664 three times 56 / 61, 56 / 81.
-inline bool streams(int M, int N, int n_mats, int splits, long cus, bool u8) {
+// twice (two) 36.6 / 32.7 with 16 rows, 37.6 / 40.4 with 32, 4096x32000 37.2 / 32.9, 39.8 / 42.8, 5888x9664 three times 56 / 61, 56 / 81; over short runs it does not (15x512x10304
+// twice 10.3 / 11.4).
+// One round: fp16 gains where the tiles (`tiles` in all, with their splits) do not come out even, or up to 16 rows over runs of 8 stages and
+// more; else it is done no sooner with weights from memory and later with weights from a cache (tiles / here, memory and cache:
+// 10x1024x7304 8.6 / 9.2, 7.4 / 8.3; 24x4096x4096 12.4 / 12.7, 11.0 / 11.7; but 13x2048x2048 three times 12.0 / 11.6, 9.1 / 10.0, 27x17920x6656
+// 62 / 47).  bfloat16 gains at every count (4x512x3264 9.2 / 7.9, 46x17920x6656 68 / 50).  Neither does for more than 16 rows over the
+// shortest runs (28x512x16840 10.5 / 11.1, bfloat16 56x512x16576 13.8 / 14.8).
+inline bool streams(int M, int N, int n_mats, int splits, int stages, long tiles, long cus, bool u8, bool bf16) {
   long rounds = 1;
   stream_waves(N, n_mats, splits, cus, stream_max_waves(u8), &rounds);
-  return rounds == 1 || (u8 && M <= 16 && rounds == 2);
+  const int run = stages / splits;
+  if (u8) return rounds == 1 || (M <= 16 && rounds == 2 && run >= 12);
+  const bool short_runs = M > 16 && run <= 4;
+  return rounds == 1 && (bf16 ? !short_runs || 4 * tiles <= 3 * cus : (tiles > cus && !short_runs) || (M <= 16 && run >= 8));
 }
 
 template <int TM, bool U8, bool BF16>
@@ -1106,7 +1115,7 @@ int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block
     return LCU_OK;
   }
   int rc;
-  if ((U8 && block_shift(block) < 0) || !streams(M, N, op.n_mats, splits, ds->compute_units, U8)) {
+  if ((U8 && block_shift(block) < 0) || !streams(M, N, op.n_mats, splits, nt_all, (long)tiles_m * tiles_n * splits, ds->compute_units, U8, false)) {
     rc = launch_split<BM, BN, 1, 4, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
     *done = rc == LCU_OK;
     return rc;
@@ -1555,7 +1564,7 @@ int bf16_skinny(linear_epilogue<false, GATED> const& ep, const void* A, const vo
   if (splits < 2) return LCU_OK;
   float* part = (float*)ws.ptr;
   int rc;
-  if (streams(M, N, 1, splits, ds->compute_units, false)) {
+  if (streams(M, N, 1, splits, K / BK, (long)tiles * splits, ds->compute_units, false, true)) {
     rc = launch_stream<false, true>(single_matrix(nullptr, W, nullptr), A, M, K, N, 0, st, splits, part, ds->compute_units);
   } else {
     rc = M <= 32 ? launch_bf16<32, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part)

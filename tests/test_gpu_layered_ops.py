@@ -81,7 +81,8 @@ def test_gated_linear_large_tiles(gpu, M, K, ff):
 
 # 128 or 256 columns by the length of K; gated tiles of 128x128 that outnumber the compute units, on both sides of theirs
 @pytest.mark.parametrize("M,K,N", [(1441, 512, 8900), (1441, 640, 8900),
-                                   (8, 512, 30000), (40, 640, 25000)])  # few rows in two rounds of workgroups
+                                   (8, 512, 30000), (40, 640, 25000),  # few rows in two rounds of workgroups
+                                   (56, 512, 16580), (56, 640, 16580), (56, 512, 5000)])  # runs of 4 and of 5, more and fewer tiles
 def test_linear_large_tiles_by_length(gpu, M, K, N):
     test_linear_large_tiles(gpu, M, K, N)
 

@@ -333,6 +333,7 @@ def test_gemm_u8_few_rows(gpu, M, K, N, block):
 
 # few rows, fp16: odd runs, rows past the last whole tile, columns past the last whole wavefront, lhs in chunks
 @pytest.mark.parametrize("M,K,N", [(3, 1152, 520), (16, 1408, 4099), (31, 2944, 1000), (48, 5888, 4100), (64, 4096, 24000),
+                                   (16, 5760, 4099), (31, 5760, 4099), (24, 4096, 4096), (28, 512, 16840),  # 264, 264, 256 and 264 tiles
                                    (8, 512, 32000), (40, 640, 31000)])  # two rounds of workgroups: the other kernel
 def test_gemm_f16_few_rows(gpu, M, K, N):
     G = gpu
