@@ -1041,8 +1041,8 @@ inline int stream_waves(int N, int n_mats, int splits, long cus, int most, long*
 // compute unit; a workgroup here has it alone, so that a second round fills lhs and ring again with nothing beside it.  us, tiles /
 // here, 8 and 32 rows: fp16 2048x32000 (two rounds) 27.7 / 33.9, 30.7 / 37.6, 4096x32000 56.0 / 56.4, 58.5 / 58.6, 5888x9664 three
 // times (three) 62 / 67, 67 / 77; one round 4096x11008 twice 43.8 / 41.9, 46.5 / 42.9 (45 rows).  uint8 gains more in a round: 4096x11008
-// twice (two) 36.6 / 32.7 with 16 rows, 37.6 / 40.4 with 32, 4096x32000 37.2 / 32.9, 39.8 / 42.8, 5888x9664 three times 56 / 61, 56 / 81; over short runs it does not (15x512x10304
-// twice 10.3 / 11.4).
+// twice (two) 36.6 / 32.7 with 16 rows, 37.6 / 40.4 with 32, 4096x32000 37.2 / 32.9, 39.8 / 42.8, 5888x9664 three times 56 / 61, 56 / 81;
+// over short runs it does not (15x512x10304 twice 10.3 / 11.4).
 // One round: fp16 gains where the tiles (`tiles` in all, with their splits) do not come out even, or up to 16 rows over runs of 8 stages and
 // more; else it is done no sooner with weights from memory and later with weights from a cache (tiles / here, memory and cache:
 // 10x1024x7304 8.6 / 9.2, 7.4 / 8.3; 24x4096x4096 12.4 / 12.7, 11.0 / 11.7; but 13x2048x2048 three times 12.0 / 11.6, 9.1 / 10.0, 27x17920x6656

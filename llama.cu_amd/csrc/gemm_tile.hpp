@@ -2,7 +2,7 @@
 // in fp32 over ascending k.
 //
 // What bounds it: the chip's power, and behind it the way from L2 into LDS.  On random operands the matrix
-// cores alone, fed from registers, reach 1.64 PFLOP/s (4096^3: 84 us; 70 us on zeros); with the operands on
+// cores alone, fed from registers, reach 1.6 to 1.9 PFLOP/s (4096^3: 71 to 84 us by the loop; 60 to 70 us on zeros); with the operands on
 // their way through LDS this kernel takes 106 us there (1.30 PFLOP/s; 81 us on zeros).  So the design saves
 // what costs energy or makes a wavefront wait:
 //  * v_mfma_f32_16x16x32 instead of 32x32x16: half the accumulator traffic per multiply-add (4096^3 with 256x128
@@ -13,9 +13,10 @@
 //  * requests are buffer loads straight into LDS whose stage offset is a scalar.  Behind the last stage the
 //    resource holds no records and the offset is 0 (operand_range.hpp): the request counts as any other but touches
 //    no memory, so that the loop has one form up to the end and its registers are never copied.
-//  * outputs go through LDS and leave in 16-byte pieces.
+//  * outputs go through LDS and leave in 16-byte pieces, wherever a row begins.
 // LDS stage: rows of 128 bytes, lhs tile then W tile, 16-byte chunk g of row r at position g ^ (r / 2) % 8, so that
-// neither requests (1 KB per instruction, dense) nor fragment reads (16 rows, one chunk) meet in a bank.
+// neither requests (1 KB per instruction, dense) nor fragment reads (16 rows, one chunk) meet in a bank (counted: 512x4096x12288 98 304
+// conflict cycles of 6.7 M; they grow with the outputs, not with K).
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -74,9 +75,10 @@ __device__ __forceinline__ half2_t dequant2(uint32_t spread, half2_t scale2x) {
 
 // WM x WN wavefronts of (BM / WM) x (BN / WN) outputs each, a ring of NS stages of 64 along K.
 // U8: W is codes with one fp16 scale per `block` of a row, block = 64 << block_shift.  Codes lie in LDS as they are, 64
-// bytes a row with the 16-byte pieces of every second group of four rows turned by two, so that sixteen rows' halves meet in
-// no bank; a wavefront turns the eight codes of each of its fragments into fp16 itself, four instructions at a time
-// between the matrix instructions of the half stage before.  The wavefronts stand side by side (WM = 1), so that every code
+// bytes a row with the 16-byte pieces of every second group of four rows turned by two (a sixth of LDS's cycles still go to conflicts of
+// their 8-byte reads, a ninth with 256 columns: counted on 512x6656x35840 and 512x6656x19968); a wavefront turns
+// the eight codes of each of its fragments into fp16 itself, four instructions at a time between the matrix instructions of the half
+// stage before.  The wavefronts stand side by side (WM = 1), so that every code
 // is converted once; with the lhs read from LDS by all four that leaves vector instructions, LDS and matrix cores about
 // equally busy.  512 rows, (N, K) = (11008, 4096): 64 us; two rows of two wavefronts (every code twice) 64-66, four of two
 // 88; converted once into an fp16 tile in LDS, with its own ring, 87 us.  1987 rows, twice (11008, 4096): 346 / 432 / 492 / 475 us.
