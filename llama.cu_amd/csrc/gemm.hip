@@ -1474,7 +1474,9 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         // us, K 256, 512, 1024, 1536, 2048: eight wavefronts / here, 512 rows of 5120 columns 6.2 / 7.1, 7.8 / 8.5, 10.9 / 11.2, 16.1 / 15.2, 22.0 / 22.3;
         // two workgroups per compute unit / here, 1000 rows of 4608 columns 9.6 / 12.4, 13.2 / 15.7, 20.8 / 21.4, 29.3 / 27.9, 39.5 / 35.1
         if (K < 1280 && tiles128 < 256) return launch_dl<128, 128, 4, 2, 1, 3, false>(op, A, M, K, N, block, beta, st);
-        if (K < 1280 && tiles128 > 256) return launch_dl<128, 128, 2, 2, 1, 2, false>(op, A, M, K, N, block, beta, st);
+        // with weights from memory the second workgroup also hides the second round's first requests: K 1280, 1536, 1792, 512 rows of
+        // 10000 columns 30.3 / 34.4, 34.2 / 38.2, 38.9 / 42.0, 896 rows of 4992 26.6 / 28.3, 30.4 / 31.0, 34.6 / 34.1
+        if (K < 1536 && tiles128 > 256) return launch_dl<128, 128, 2, 2, 1, 2, false>(op, A, M, K, N, block, beta, st);
         return launch_tile<128, 128, 2, 2, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
       }
     } else {

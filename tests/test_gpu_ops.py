@@ -235,7 +235,7 @@ def test_gemm_f16_large_tiles_ragged(gpu, M, K, N):
 
 # both sides of the lengths of K that decide between the kernels: fp16 with 160 .. 255 tiles of 128x128 and more, 128 or 256 columns
 # of large tiles; the cases above whose K is short, with a long one
-@pytest.mark.parametrize("M,K,N,count", [(257, 1152, 6790, 1), (257, 1280, 6790, 1), (1100, 1152, 3690, 1), (1100, 1280, 3690, 1),
+@pytest.mark.parametrize("M,K,N,count", [(257, 1152, 6790, 1), (257, 1280, 6790, 1), (1100, 1152, 3690, 1), (1100, 1408, 3690, 1), (1100, 1536, 3690, 1),
                                          (1441, 512, 2900, 3), (1441, 640, 2900, 3), (2049, 640, 4100, 1), (300, 640, 12930, 1)])
 def test_gemm_f16_short_and_long_k(gpu, M, K, N, count):
     G = gpu
