@@ -446,6 +446,12 @@ def test_experts(gpu, dt, n, K, ff, experts, top, tile):
     gpu.release()
 
 
+@pytest.mark.parametrize("n,K,ff,experts,top,tile", [(4700, 64, 64, 3, 2, 64), (190, 64, 130, 100, 1, 64), (90, 128, 70, 65, 1, 128)])
+def test_experts_lists_of_many_tiles(gpu, n, K, ff, experts, top, tile):
+    """Lists of row tiles that 64 entries do not hold: runs of one expert across their edge, and many of one tile each."""
+    test_experts(gpu, BF16, n, K, ff, experts, top, tile)
+
+
 @pytest.mark.parametrize("n", [1, 7, 640, 32000, 50257])
 def test_argmax_and_softmax(gpu, n):
     rng = np.random.default_rng(n)
