@@ -882,6 +882,10 @@ inline operands_t single_matrix(half_t* out, const void* W, const half_t* S) {
   return operands_t{out, W, S, more_matrices_t{{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}, 0}, 1};
 }
 
+inline operands_t last_matrix(operands_t op) {
+  return op.n_mats == 1 ? op : single_matrix(op.more.out[op.n_mats - 2], op.more.W[op.n_mats - 2], op.more.S[op.n_mats - 2]);
+}
+
 template <int BM, int BN, int WM, int WN, int KS, int NS, bool U8>
 int launch_dl(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st) {
   constexpr int ROWB = BK * KS * 2;
@@ -916,12 +920,20 @@ inline int block_shift(int block) {
   return -1;
 }
 
+// Which columns of a product a launch of gemm_tile_kernel takes: the first `tiles` tiles along N, counted through the matrices
+// (0: all of them), or those from column `from` of the last matrix on.
+struct columns_t {
+  int tiles = 0, from = 0;
+};
+
 // A launch of gemm_tile_kernel; splits > 1: the K stages of every tile dealt to that many workgroups, fp32 sums to part.
 template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
 int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits = 1,
-                float* part = nullptr) {
+                float* part = nullptr, columns_t which = {}) {
   using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
-  const int tiles_m = (M + BM - 1) / BM, tiles_n_per = (N + BN - 1) / BN, tiles_n = tiles_n_per * op.n_mats;
+  const int tiles_m = (M + BM - 1) / BM;
+  if (which.from > 0) op = last_matrix(op);
+  const int tiles_n_per = (N - which.from + BN - 1) / BN, tiles_n = which.tiles > 0 ? which.tiles : tiles_n_per * op.n_mats;
   op.more.tiles_n_per = op.n_mats > 1 ? tiles_n_per : 0;
   auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
   static bool raised[16] = {};  // per device, once
@@ -932,16 +944,26 @@ int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N,
     raised[dev & 15] = true;
   }
   kernel<<<tiles_m * tiles_n * splits, 64 * WM * WN, shape::LDS, st>>>(op.out, (const half_t*)A, op.W, op.S, block_shift(block), M, K, N, beta,
-                                                                       tiles_m, tiles_n, part, splits, op.more, ep);
+                                                                       tiles_m, tiles_n, which.from, part, splits, op.more, ep);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
 
-// Columns of the 256-row tile of a product that fills most of the chip with them: the one whose rounds of workgroups
-// cost least.  fp16 and bfloat16: a round of 128 / 192 / 256 columns takes 57 / 88 / 106 us at K = 4096 (512 rows, W1 and W3
-// of 11008 columns in one launch: 230 tiles of 192 columns 88 us, 172 of 256 94 us, 344 of 128 108 us; 1987 rows: 303 us
-// with 256 columns, 330 us with 128).  uint8: 128 / 256 columns 65 / 113 us (512 rows, K 6656, three times 6656 columns:
-// 156 tiles of 256 168 us, 312 of 128 187 us; 1987 rows, twice 11008 columns 346 / 374 us, three times 4096 226 / 196 us).
+// Tiles of a product that fills most of the chip with those of 256x128: `columns` wide, of 256 rows (128 up to 128 rows); from column `from` of
+// the last matrix on, where that is not 0, tiles of rest_rows x rest_columns in a launch of their own.
+struct large_tiles_t {
+  int columns;
+  columns_t first, rest;
+  int rest_rows, rest_columns;
+};
+
+// The tiles whose rounds of workgroups cost least.  fp16 and bfloat16: a round of 128 / 192 / 256 columns takes 57 / 88 / 106 us at K = 4096 (512
+// rows, W1 and W3 of 11008 columns in one launch: 230 tiles of 192 columns 88 us, 172 of 256 94 us, 344 of 128 108 us; 1987 rows: 303 us
+// with 256 columns, 330 us with 128), one of 128x128 tiles 41.  uint8: 59 / 79 / 104 and 40 (512 rows, K 6656, three times 6656 columns: 156 tiles of
+// 256 191 us, 208 of 192 148, 312 of 128 208; K 4096, twice 11008: 107 / 86 / 118; 1987 rows 341 / 346 / 381).
+// A last round that is nearly empty goes to smaller tiles: whole rounds of one width, then the columns that are left in those tiles that cost least
+// (us, the best single width / so: 512 rows, K 6656, twice 17920 columns uint8 254 / 234, fp16 266 / 234; K 4096, 700 rows, twice 11008 fp16
+// 143 / 136, 1000 rows 164 / 158, 1987 rows 300 / 290).  The second launch costs 3 us more; below 1024 of K that is what it gains.
 // Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts there.
 // Up to 512 of K what a tile pays beside its stages counts: 256 columns leave by four wavefronts, and the rounds are no measure of
 // them (1441 rows of K 256, three times 2944 columns: 216 tiles of 256 20.1 us, 414 of 128 16.5; bfloat16 1027x512x11840 28.7 / 23.4),
@@ -949,44 +971,77 @@ int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N,
 // Up to 128 rows: tiles of 128 rows, a round of 128 / 256 columns taking 52 / 66 us in fp16 and 42 / 62 in uint8 (100
 // rows, twice 11008 columns 61 -> 52 us and 55 -> 42 against tiles of 256 rows; twice 17920 of K 6656 140 -> 118 and 170 -> 109).
 template <bool U8>
-int large_tile_columns(int M, int K, int N, int n_mats, long cus, bool gated) {
-  const auto cost = [&](int columns, int round) {
-    const long tiles = (long)((M + 255) / 256) * ((N + columns - 1) / columns) * n_mats;
-    return (tiles + cus - 1) / cus * round;
-  };
-  if (M <= 128) return cost(256, U8 ? 62 : 66) < cost(128, U8 ? 42 : 52) ? 256 : 128;
+large_tiles_t plan_large(int M, int K, int N, int n_mats, long cus, bool gated) {
+  const auto tiles = [&](int rows, int columns, int n) { return (long)((M + rows - 1) / rows) * ((n + columns - 1) / columns); };
+  const auto rounds = [&](long n) { return (n + cus - 1) / cus; };
+  if (M <= 128) {
+    const long c128 = rounds(tiles(128, 128, N) * n_mats) * (U8 ? 42 : 52), c256 = rounds(tiles(128, 256, N) * n_mats) * (U8 ? 62 : 66);
+    return {c256 < c128 ? 256 : 128, {}, {}, 0, 0};
+  }
+  const auto round = [&](int columns) -> long { return columns == 128 ? (U8 ? 59 : 57) : columns == 192 ? (U8 ? 79 : 88) : (U8 ? 104 : 106); };
+  const auto allowed = [&](int columns) { return columns == 128 || (columns == 192 ? K >= 256 && !gated : K >= 640); };
+  large_tiles_t best{128, {}, {}, 0, 0};
+  long least = rounds(tiles(256, 128, N) * n_mats) * round(128);
+  for (int columns : {256, 192}) {
+    const long cost = rounds(tiles(256, columns, N) * n_mats) * round(columns);
+    if (allowed(columns) && cost < least) {
+      least = cost;
+      best.columns = columns;
+    }
+  }
+  if (K < 1024) return best;
+  const int tiles_m = (M + 255) / 256;
+  for (int columns : {256, 192, 128}) {
+    const long per = (N + columns - 1) / columns, whole = per * n_mats * tiles_m / cus, first = whole * cus / tiles_m;
+    const int from = (int)(first - per * (n_mats - 1)) * columns;
+    if (!allowed(columns) || whole == 0 || from <= 0 || from >= N) continue;  // what is left lies in the last matrix
+    for (int rest : {0, 128, 192}) {                                          // 0: tiles of 128x128
+      if (rest == 192 && !allowed(192)) continue;
+      const long last = rest == 0 ? rounds(tiles(128, 128, N - from)) * (U8 ? 40 : 41) : rounds(tiles(256, rest, N - from)) * round(rest);
+      const long cost = whole * round(columns) + last + 3 * 4096 / K;
+      if (cost < least) {
+        least = cost;
+        best = {columns, {(int)first, 0}, {0, from}, rest == 0 ? 128 : 256, rest == 0 ? 128 : rest};
+      }
+    }
+  }
+  return best;
+}
+
+// tiles of 256 rows
+template <bool U8, class EP>
+int launch_columns(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st, int columns,
+                   columns_t which) {
   if constexpr (U8) {
-    return cost(256, 113) < cost(128, 65) ? 256 : 128;
+    if (columns == 256) return launch_tile<256, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
+    if (columns == 192) return launch_tile<256, 192, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
+    return launch_tile<256, 128, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
   } else {
-    const long c128 = cost(128, 57), c192 = gated ? c128 : cost(192, 88), c256 = cost(256, 106);
-    if (K >= 640 && c256 < c128 && c256 <= c192) return 256;
-    return K >= 256 && c192 < c128 ? 192 : 128;
+    if (columns == 256) return launch_tile<256, 256, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
+    if constexpr (!EP::GATED) {
+      if (columns == 192) return launch_tile<256, 192, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
+    }
+    return launch_tile<256, 128, 4, 2, 3, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
   }
 }
 
 template <bool U8, class EP>
 int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st) {
   device_state* ds = current_device_state();
-  const int columns = large_tile_columns<U8>(M, K, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
+  const large_tiles_t plan = plan_large<U8>(M, K, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
   if (M <= 128) {
     if constexpr (U8) {
-      if (columns == 256) return launch_tile<128, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
+      if (plan.columns == 256) return launch_tile<128, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
       return launch_tile<128, 128, 1, 4, 4, true, false>(ep, op, A, M, K, N, block, beta, st);
     } else {
-      if (columns == 256) return launch_tile<128, 256, 2, 4, 3, false, false>(ep, op, A, M, K, N, 0, beta, st);
+      if (plan.columns == 256) return launch_tile<128, 256, 2, 4, 3, false, false>(ep, op, A, M, K, N, 0, beta, st);
       return launch_tile<128, 128, 2, 2, 4, false, false>(ep, op, A, M, K, N, 0, beta, st);
     }
   }
-  if constexpr (U8) {
-    if (columns == 256) return launch_tile<256, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
-    return launch_tile<256, 128, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
-  } else {
-    if (columns == 256) return launch_tile<256, 256, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st);
-    if constexpr (!EP::GATED) {
-      if (columns == 192) return launch_tile<256, 192, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st);
-    }
-    return launch_tile<256, 128, 4, 2, 3, false, false>(ep, op, A, M, K, N, 0, beta, st);
-  }
+  const int rc = launch_columns<U8>(ep, op, A, M, K, N, block, beta, st, plan.columns, plan.first);
+  if (rc != LCU_OK || plan.rest.from == 0) return rc;
+  if (plan.rest_rows == 256) return launch_columns<U8>(ep, op, A, M, K, N, block, beta, st, plan.rest_columns, plan.rest);
+  return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, U8, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, plan.rest);
 }
 
 // where a split-K launch left its partial sums: part[matrix][split][M][N] fp32

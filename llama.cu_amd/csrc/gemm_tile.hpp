@@ -90,13 +90,13 @@ struct tile_shape {
   static constexpr int OUT_LD = WC + 4;                  // floats per row of a wavefront's 64 output rows in LDS
   static constexpr int RING = NS * STAGE, OUT = NW * 64 * OUT_LD * 4;
   static constexpr int LDS = RING > OUT ? RING : OUT;
-  static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 32 == 0, "tile");
+  static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 16 == 0, "tile");
 };
 
 template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0, int block_shift,
-    int M, int K, int N, float beta, int tiles_m, int tiles_n, float* __restrict__ part, int splits, more_matrices_t more, EP ep) {
+    int M, int K, int N, float beta, int tiles_m, int tiles_n, int from, float* __restrict__ part, int splits, more_matrices_t more, EP ep) {
   using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
   static_assert(!EP::GROUPED, "one matrix for all rows");
   constexpr int NW = shape::NW;
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     if constexpr (U8) S = g == 0 ? S0 : (g == 1 ? more.S[0] : more.S[1]);
     if constexpr (SPLIT) part += (size_t)g * splits * M * N;  // each matrix has its own partial sums
   }
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * BM, n0 = from + tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave % WM) * shape::WR, wn = (wave / WM) * shape::WC;
 

@@ -87,6 +87,13 @@ def test_linear_large_tiles_by_length(gpu, M, K, N):
     test_linear_large_tiles(gpu, M, K, N)
 
 
+# whole rounds of 256 columns and what is left of them in tiles of 128x128
+@pytest.mark.parametrize("M,K,N", [(1100, 1024, 13900)])
+def test_linear_columns_left_of_whole_rounds(gpu, M, K, N):
+    test_linear_large_tiles(gpu, M, K, N)
+    test_gated_linear_large_tiles(gpu, M, K, N // 2)
+
+
 @pytest.mark.parametrize("M,K,ff", [(1100, 1216, 1850), (1100, 1280, 1850), (1441, 640, 4400), (20, 512, 13000), (6, 2816, 1020)])
 def test_gated_linear_tiles_by_length(gpu, M, K, ff):
     test_gated_linear_large_tiles(gpu, M, K, ff)

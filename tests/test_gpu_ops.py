@@ -297,6 +297,38 @@ def test_gemm_exact_cases(gpu):
     G.release()
 
 
+# whole rounds of large tiles and the columns behind them in smaller ones: 128x128, 128 and 192 columns of 256 rows, ragged ones, one to
+# three matrices; codes: and 192 columns alone.  512 rows at a time take other tiles; the sums are one ascending chain in both
+@pytest.mark.parametrize("u8,M,K,N,count", [(False, 1100, 1024, 14000, 1), (False, 1000, 2048, 11008, 2), (False, 1987, 1024, 11008, 2),
+                                            (False, 700, 1024, 11003, 2), (True, 1100, 1024, 14000, 1), (True, 1987, 1024, 11008, 2),
+                                            (True, 1500, 1152, 6652, 3), (True, 512, 1024, 17924, 2), (True, 300, 1024, 6656, 3)])
+def test_gemm_columns_left_of_whole_rounds(gpu, u8, M, K, N, count):
+    G = gpu
+    VP, check, L = G.B.vp, G.B.check, G.L()
+    x, ws = normal((M, K), 0, 350, 1.0), [normal((N, K), 0, 351 + g, 0.02) for g in range(count)]
+    w = [O.quantize_absmax_u8(v, 128) for v in ws] if u8 else [(v,) for v in ws]
+    wd = [[G.dev_keep(part) for part in v] for v in w]
+    ptrs = [(VP * count)(*[v[i].ptr for v in wd]) for i in range(len(w[0]))]
+
+    def product(rows, beta, old):
+        assert O.gemm_plan(len(rows), K, N, u8, 128, count) == O.gemm_plan(M, K, N, u8, 128, count)
+        outs = [G.dev_keep(o) for o in old]
+        args = ((VP * count)(*[o.ptr for o in outs]), G.dev_keep(rows).ptr, *ptrs, count, len(rows), K, N)
+        check(L.lcu_gemm_f16u8_nt_multi(*args, 128, beta, None) if u8 else L.lcu_gemm_f16_nt_multi(*args, beta, None))
+        return [G.host(o, (len(rows), N)) for o in outs]
+
+    old = [normal((M, N), 0, 360 + g, 1.0) for g in range(count)]
+    for beta in (0.0, 1.0):
+        got = product(x, beta, old)
+        at = list(range(0, M, 512))
+        if len(at) > 1 and M - at[-1] < 257:  # so that the last piece has enough tiles for one chain
+            at.pop()
+        for a, b in zip(at, at[1:] + [M]):
+            for g, part in zip(got, product(x[a:b], beta, [o[a:b] for o in old])):
+                assert G.ulp_mismatch(g[a:b], part) == 0.0, (a, b)
+    G.release()
+
+
 @pytest.mark.parametrize("M,K,N", [(512, 4096, 4096), (512, 4096, 11008), (512, 11008, 4096), (16, 256, 128),
                                    (130, 384, 70), (512, 256, 5120), (512, 384, 4160), (1024, 256, 4096),
                                    (500, 128, 5100), (40, 384, 300), (4096, 128, 4096), (512, 256, 17920),
