@@ -249,8 +249,9 @@ int lcu_attention_decode_batch(void* out_dev, const void* q_dev, const void* k_c
                                const void* v_cache_ptrs_dev, const void* pos_dev, int n_seq, int max_T, int dim,
                                int n_heads, void* stream);
 /* The products of a batched step fused with what follows them (for 2..64 sequences the partial sums
- * of the split-K product are added up by the kernel that goes on with them; any other shape runs
- * the separate operators above).  w_dev / scales_dev: host arrays of device pointers (scales NULL
+ * of the split-K product are added up by the kernel that goes on with them, and so they are in
+ * lcu_batch_proj_norm for more rows where their product is split; any other shape runs the separate
+ * operators above).  w_dev / scales_dev: host arrays of device pointers (scales NULL
  * and block 0 for fp16 weights); *_tmp_dev: [n_seq][dim] / [n_seq][ffn] fp16 scratch.
  *   lcu_batch_qkv: Wq, Wk, Wv products of lhs [n_seq][dim], then lcu_rope_store_batch (1144-1156)
  *   lcu_batch_ffn_up: W1, W3 products, then fp16(silu(w1) * w3) (1180-1183)

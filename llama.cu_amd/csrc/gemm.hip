@@ -929,7 +929,7 @@ struct columns_t {
 // A launch of gemm_tile_kernel; splits > 1: the K stages of every tile dealt to that many workgroups, fp32 sums to part.
 template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
 int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits = 1,
-                float* part = nullptr, columns_t which = {}) {
+                float* part = nullptr, columns_t which = {}, int step = 1) {
   using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
   const int tiles_m = (M + BM - 1) / BM;
   if (which.from > 0) op = last_matrix(op);
@@ -944,7 +944,7 @@ int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N,
     raised[dev & 15] = true;
   }
   kernel<<<tiles_m * tiles_n * splits, 64 * WM * WN, shape::LDS, st>>>(op.out, (const half_t*)A, op.W, op.S, block_shift(block), M, K, N, beta,
-                                                                       tiles_m, tiles_n, which.from, part, splits, op.more, ep);
+                                                                       tiles_m, tiles_n, which.from, part, splits, step, op.more, ep);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
@@ -1221,10 +1221,18 @@ inline int large_tile_splits(int M, int K, int N, int n_mats, long cus, size_t w
   return (int)splits;
 }
 
+// tiles of 256x128 (128x128 up to 128 rows or where `small`), sums of every split to part
+template <bool U8>
+int launch_partial(operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, bool small, int step) {
+  if (small || M <= 128) {
+    return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+  }
+  return launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+}
+
 template <bool U8>
 int launch_large_split(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits, float* part) {
-  const int rc = M <= 128 ? launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, U8, true>(f16_epilogue{}, op, A, M, K, N, block, beta, st, splits, part)
-                          : launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, beta, st, splits, part);
+  const int rc = launch_partial<U8>(op, A, M, K, N, block, st, splits, part, false, 1);
   if (rc != LCU_OK) return rc;
   const size_t mn = (size_t)M * N;
   splitk_reduce_kernel<<<dim3((unsigned)((mn + 1023) / 1024), op.n_mats), 256, 0, st>>>(op.out, op.more.out[0], op.more.out[1], part, mn,
@@ -1271,15 +1279,52 @@ int skinny_partial(operands_t op, const half_t* A, int M, int K, int N, int bloc
   }
 }
 
+// The same for more than 64 rows of one matrix, where dispatch_gemm has more than one chain per output: the splits of large tiles, or the even and
+// the odd 64-blocks of K of its 128x64 tiles, here dealt to workgroups of 128x128 tiles.  The latter where K is long enough for what the sums
+// cost on their way through memory (product, residual and norm, separate / here, us: fp16 80x4096x4096 30 / 24, 256 rows 33 / 29, 512 rows 35.5 / 34.7,
+// 700x2048x2048 19.6 / 20.0, 1000x512x2048 14.7 / 21.6; uint8 512x4096x4096 45 / 39, 700x2048x2048 25.1 / 23.1, 1000x512x2048 16.1 / 22.5).
+template <bool U8>
+int many_rows_partial(operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, bool* done, partial_sums_t* res) {
+  *done = false;
+  device_state* ds = current_device_state();
+  const workspace_t ws = workspace_for(st);
+  if (K % 128 != 0 || M <= 64 || ds == nullptr || ws.ptr == nullptr || !scale_words_ok<U8>(op, K, N, block) || (U8 && block_shift(block) < 0) ||
+      (size_t)M * K * 2 >= (size_t)1 << 32 || (size_t)N * K * (U8 ? 1 : 2) >= (size_t)1 << 32) {
+    return LCU_OK;
+  }
+  const auto tiles = [&](int rows, int columns) { return (long)((M + rows - 1) / rows) * ((N + columns - 1) / columns); };
+  const long cus = ds->compute_units > 0 ? ds->compute_units : 256;
+  if (tiles(256, 128) >= 160) return LCU_OK;
+  int splits = large_tile_splits(M, K, N, 1, cus, ws.bytes), step = 1;
+  if (splits == 0) {
+    if (tiles(128, 128) >= 160 || tiles(128, 64) > 256 || (size_t)2 * M * N * sizeof(float) > ws.bytes) return LCU_OK;
+    if ((size_t)M * N > (size_t)K * (U8 ? 1024 : 512)) return LCU_OK;
+    splits = step = 2;
+  }
+  const int rc = launch_partial<U8>(op, A, M, K, N, block, st, splits, (float*)ws.ptr, step == 2, step);
+  res->part = (float*)ws.ptr;
+  res->splits = splits;
+  *done = rc == LCU_OK;
+  return rc;
+}
+
 // ---- kernels that add the partial sums up and go on with what follows the product in a batched
 // decode step (llama_cu.cu:1144-1156, 1174-1176, 1180-1185), one row per sequence ----
 
+// In split order, four splits asked for at a time: with a runtime count the compiler waits for each before the next.
 __device__ __forceinline__ float2 sum_pair(const float* __restrict__ part, size_t at, size_t mn, int splits) {
   float2 v = *reinterpret_cast<const float2*>(part + at);
-  for (int s = 1; s < splits; ++s) {
-    const float2 w = *reinterpret_cast<const float2*>(part + (size_t)s * mn + at);
-    v.x += w.x;
-    v.y += w.y;
+  for (int s = 1; s < splits; s += 4) {
+    float2 w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) w[u] = *reinterpret_cast<const float2*>(part + (size_t)min(s + u, splits - 1) * mn + at);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (s + u < splits) {
+        v.x += w[u].x;
+        v.y += w[u].y;
+      }
+    }
   }
   return v;
 }
@@ -1337,7 +1382,10 @@ __global__ __launch_bounds__(256) void reduce_silu_kernel(half_t* __restrict__ o
 // (up to 8192 columns: four pairs per thread, every partial sum requested before the first is
 // used -- the launch is a handful of workgroups and nothing but latency); the norm as in
 // rmsnorm_kernel, its sum of squares taken by the first 256 threads in the reference's association.
+// 8 rows of 4096, eight splits: 7.4 us with a wait per split, 6.0 with four asked for at a time; 512 rows, four splits 9.1 (the sums' 46 MB),
+// where the sum and the norm took 9.5 and 5.5 in launches of their own.
 constexpr int RN_THREADS = 1024, RN_PAIRS = 4;
+template <int PAIRS>
 __global__ __launch_bounds__(RN_THREADS) void reduce_residual_norm_kernel(half_t* __restrict__ x,
                                                                           half_t* __restrict__ norm_out,
                                                                           const float* __restrict__ part, int splits,
@@ -1348,27 +1396,38 @@ __global__ __launch_bounds__(RN_THREADS) void reduce_residual_norm_kernel(half_t
   const int b = blockIdx.x, tid = threadIdx.x;
   const size_t mn = (size_t)n_seq * cols;
   half_t* xr = x + (size_t)b * cols;
-  float2 acc[RN_PAIRS];
-  half2_t old[RN_PAIRS], wv[RN_PAIRS];
+  float2 acc[PAIRS];
+  half2_t old[PAIRS], wv[PAIRS];
 #pragma unroll
-  for (int j = 0; j < RN_PAIRS; ++j) {
+  for (int j = 0; j < PAIRS; ++j) {
     const int c = min((tid + j * RN_THREADS) * 2, cols - 2);
     acc[j] = *reinterpret_cast<const float2*>(part + (size_t)b * cols + c);
     old[j] = *reinterpret_cast<const half2_t*>(xr + c);
     wv[j] = *reinterpret_cast<const half2_t*>(norm_w + c);
   }
-  for (int s = 1; s < splits; ++s) {
+  for (int s = 1; s < splits; s += 4) {
+    float2 w[4][PAIRS];
 #pragma unroll
-    for (int j = 0; j < RN_PAIRS; ++j) {
-      const int c = min((tid + j * RN_THREADS) * 2, cols - 2);
-      const float2 w = *reinterpret_cast<const float2*>(part + (size_t)s * mn + (size_t)b * cols + c);
-      acc[j].x += w.x;
-      acc[j].y += w.y;
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+      for (int j = 0; j < PAIRS; ++j) {
+        const int c = min((tid + j * RN_THREADS) * 2, cols - 2);
+        w[u][j] = *reinterpret_cast<const float2*>(part + (size_t)min(s + u, splits - 1) * mn + (size_t)b * cols + c);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (s + u >= splits) break;
+#pragma unroll
+      for (int j = 0; j < PAIRS; ++j) {
+        acc[j].x += w[u][j].x;
+        acc[j].y += w[u][j].y;
+      }
     }
   }
-  half2_t val[RN_PAIRS];
+  half2_t val[PAIRS];
 #pragma unroll
-  for (int j = 0; j < RN_PAIRS; ++j) {
+  for (int j = 0; j < PAIRS; ++j) {
     const int c = (tid + j * RN_THREADS) * 2;
     val[j].x = round_f16(fmaf(1.0f, (float)old[j].x, acc[j].x));
     val[j].y = round_f16(fmaf(1.0f, (float)old[j].y, acc[j].y));
@@ -1402,7 +1461,7 @@ __global__ __launch_bounds__(RN_THREADS) void reduce_residual_norm_kernel(half_t
   const float rms_inv = 1.0f / sqrtf(total / (float)cols + eps);
   half_t* y = norm_out + (size_t)b * cols;
 #pragma unroll
-  for (int j = 0; j < RN_PAIRS; ++j) {
+  for (int j = 0; j < PAIRS; ++j) {
     const int c = (tid + j * RN_THREADS) * 2;
     if (c < cols) {
       half2_t r;
@@ -1887,13 +1946,19 @@ int lcu_batch_proj_norm(void* x_dev, void* norm_out_dev, const void* lhs_dev, co
   partial_sums_t ps{};
   if (n_seq > 1 && dim <= RN_THREADS * RN_PAIRS * 2) {
     const operands_t op = single_matrix((half_t*)x_dev, w_dev, (const half_t*)(block ? scales_dev : nullptr));
-    const int rc = block ? skinny_partial<true>(op, (const half_t*)lhs_dev, n_seq, K, dim, block, st, &done, &ps)
-                         : skinny_partial<false>(op, (const half_t*)lhs_dev, n_seq, K, dim, 0, st, &done, &ps);
+    const half_t* lhs = (const half_t*)lhs_dev;
+    int rc;
+    if (n_seq > 64) {
+      rc = block ? many_rows_partial<true>(op, lhs, n_seq, K, dim, block, st, &done, &ps) : many_rows_partial<false>(op, lhs, n_seq, K, dim, 0, st, &done, &ps);
+    } else {
+      rc = block ? skinny_partial<true>(op, lhs, n_seq, K, dim, block, st, &done, &ps) : skinny_partial<false>(op, lhs, n_seq, K, dim, 0, st, &done, &ps);
+    }
     if (rc != LCU_OK) return rc;
   }
   if (done) {
-    reduce_residual_norm_kernel<<<n_seq, RN_THREADS, (size_t)dim * 2, st>>>(
-        (half_t*)x_dev, (half_t*)norm_out_dev, ps.part, ps.splits, n_seq, dim, (const half_t*)norm_w_dev, eps);
+    auto kernel = dim <= RN_THREADS * 2 ? reduce_residual_norm_kernel<1> : dim <= RN_THREADS * 4 ? reduce_residual_norm_kernel<2> : reduce_residual_norm_kernel<RN_PAIRS>;
+    kernel<<<n_seq, RN_THREADS, (size_t)dim * 2, st>>>((half_t*)x_dev, (half_t*)norm_out_dev, ps.part, ps.splits, n_seq, dim,
+                                                       (const half_t*)norm_w_dev, eps);
     LCU_LAUNCH_CHECK();
     return LCU_OK;
   }

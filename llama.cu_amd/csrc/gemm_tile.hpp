@@ -96,7 +96,7 @@ struct tile_shape {
 template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0, int block_shift,
-    int M, int K, int N, float beta, int tiles_m, int tiles_n, int from, float* __restrict__ part, int splits, more_matrices_t more, EP ep) {
+    int M, int K, int N, float beta, int tiles_m, int tiles_n, int from, float* __restrict__ part, int splits, int step, more_matrices_t more, EP ep) {
   using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
   static_assert(!EP::GROUPED, "one matrix for all rows");
   constexpr int NW = shape::NW;
@@ -134,8 +134,12 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 
   // this workgroup's K stages
   const int nt_all = K / 64;
-  const int stage0 = SPLIT ? (int)((long)split * nt_all / splits) : 0;
-  const int nt = SPLIT ? (int)((long)(split + 1) * nt_all / splits) - stage0 : nt_all;
+  int stage0 = 0, nt = nt_all;
+  if constexpr (SPLIT) {  // a run of them, or with step = splits every so many
+    stage0 = step > 1 ? split : (int)((long)split * nt_all / splits);
+    nt = step > 1 ? nt_all / step : (int)((long)(split + 1) * nt_all / splits) - stage0;
+  }
+  const auto stage_of = [&](int t) { return (uint32_t)(SPLIT ? stage0 + t * step : t); };
 
   // request j of this wavefront fills LDS bytes [(wave + j * NW) * 1024, + 1024) of an operand's part of a stage.
   // Rows past M or N are clamped to the last one: their sums are never stored.
@@ -176,13 +180,13 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
                  : "memory", "m0");
   };
   const auto issue = [&](int stage, int slot, int i) {
-    const uint32_t along = stage_offset(ra[2], (uint32_t)(stage0 + stage) * 128u);
+    const uint32_t along = stage_offset(ra[2], stage_of(stage) * 128u);
     if (i < PA) {
       request(ra, along, a_off[i], slot * STAGE + (wave + i * NW) * 1024);
     } else if (i < PA + PB) {
       request(rw, U8 ? along / 2 : along, b_off[i - PA], slot * STAGE + A_BYTES + (wave + (i - PA) * NW) * 1024);
     } else if constexpr (U8) {  // the word that holds the row's scale of this stage
-      const uint32_t at = s_first[i - PA - PB] + ((uint32_t)(stage0 + stage) >> block_shift);
+      const uint32_t at = s_first[i - PA - PB] + (stage_of(stage) >> block_shift);
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(scale_word(at)), "s"(rs),
                    "s"(lds0 + slot * STAGE + A_BYTES + B_BYTES + wave * shape::SW * 4 + (i - PA - PB) * 256)
                    : "memory", "m0");
@@ -236,7 +240,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     if constexpr (U8) {
       const int j = k / 4, w = k / 2 % 2, high = k % 2;
       if (h == 0 && k % 4 == 0) {
-        const uint32_t at = f_first[j] + ((uint32_t)(stage0 + st) >> block_shift);
+        const uint32_t at = f_first[j] + (stage_of(st) >> block_shift);
         const half_t x = __builtin_bit_cast(half_t, (uint16_t)((at & 1) ? words[j] >> 16 : words[j])) * (half_t)2.0f;
         scales[j] = half2_t{x, x};
       }

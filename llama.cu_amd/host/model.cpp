@@ -329,6 +329,17 @@ void llama_context_impl::matmul(void* out, const void* lhs, weight_tensor const&
   }
 }
 
+// x += lhs * W^T, then the norm of x to t_norm_
+void llama_context_impl::matmul_norm(void* x, const void* lhs, weight_tensor const& w, int M, gpu_buffer const& norm) {
+  if (w.cols % 16 != 0 || w.rows > 24576) {  // a feed-forward of an odd number of eights
+    matmul(x, lhs, w, M, 1.0f);
+    LCU_CHECK(lcu_rmsnorm(t_norm_.data(), x, norm.data(), M, (int)w.rows, model_->params.norm_eps, stream_));
+    return;
+  }
+  LCU_CHECK(lcu_batch_proj_norm(x, t_norm_.data(), lhs, w.data.data(), w.scales.data(), w.quantised ? w.block : 0, M, (int)w.cols, (int)w.rows,
+                                norm.data(), model_->params.norm_eps, stream_));
+}
+
 // products of one lhs with several weight matrices of one shape (Wq, Wk, Wv; W1, W3) in one launch
 void llama_context_impl::matmul_multi(void* const* outs, const void* lhs, weight_tensor const* const* ws, int count,
                                       int M) {
@@ -390,7 +401,8 @@ void llama_context_impl::enqueue_layers(int n, bool first_norm_ready) {
     } else {
       char* k_new = kc + (size_t)sp * dim * 2;
       char* v_new = vc + (size_t)sp * dim * 2;
-      LCU_CHECK(lcu_rmsnorm(t_norm_.data(), x, L.attn_norm.data(), n, dim, p.norm_eps, stream_));            // 1129
+      if (!norm_ready) LCU_CHECK(lcu_rmsnorm(t_norm_.data(), x, L.attn_norm.data(), n, dim, p.norm_eps, stream_));  // 1129
+      norm_ready = false;
       void* const qkv_out[3] = {t_xq_.data(), k_new, v_new};
       weight_tensor const* const qkv_w[3] = {&L.wq, &L.wk, &L.wv};
       matmul_multi(qkv_out, t_norm_.data(), qkv_w, 3, n);                                                    // 1144, 1150, 1156
@@ -403,18 +415,17 @@ void llama_context_impl::enqueue_layers(int n, bool first_norm_ready) {
                                      dim, L.ffn_norm.data(), p.norm_eps,
                                      (char*)t_step_.data() + offsetof(step_state, seq), (int)((2 * l) & 1023), stream_));
     } else if (!fused_wo) {
-      matmul(x, t_out_.data(), L.wo, n, 1.0f);                                                               // 1174
-      LCU_CHECK(lcu_rmsnorm(t_norm_.data(), x, L.ffn_norm.data(), n, dim, p.norm_eps, stream_));             // 1176
+      matmul_norm(x, t_out_.data(), L.wo, n, L.ffn_norm);                                                    // 1174, 1176
     }
     if (n == 1) {
       // 1180-1183 in one launch
       LCU_CHECK(lcu_decode_ffn_up(t_silu_.data(), t_norm_.data(), nullptr, L.w1.data.data(), L.w3.data.data(),
                                   L.w1.scales.data(), L.w3.scales.data(), block, dim, ffn, p.norm_eps, stream_));
     } else {
-      void* const up_out[2] = {t_w1_.data(), t_w3_.data()};
-      weight_tensor const* const up_w[2] = {&L.w1, &L.w3};
-      matmul_multi(up_out, t_norm_.data(), up_w, 2, n);                                                      // 1180, 1181
-      LCU_CHECK(lcu_silu_mul(t_silu_.data(), t_w1_.data(), t_w3_.data(), (size_t)n * ffn, stream_));         // 1183
+      const void* const up_w[2] = {L.w1.data.data(), L.w3.data.data()};
+      const void* const up_s[2] = {L.w1.scales.data(), L.w3.scales.data()};
+      LCU_CHECK(lcu_batch_ffn_up(t_silu_.data(), t_w1_.data(), t_w3_.data(), t_norm_.data(), up_w, up_s, L.w1.quantised ? L.w1.block : 0, n,
+                                 dim, ffn, stream_));                                                        // 1180-1183
     }
     if (n == 1 && hand_overs_ && l + 1 < model_->layers.size() && dim <= 8192) {
       // 1185 and the next layer's 1129 in one launch
@@ -422,6 +433,9 @@ void llama_context_impl::enqueue_layers(int n, bool first_norm_ready) {
       LCU_CHECK(lcu_decode_proj_norm(x, t_norm_.data(), t_silu_.data(), L.w2.data.data(), L.w2.scales.data(), block,
                                      ffn, dim, next.attn_norm.data(), p.norm_eps,
                                      (char*)t_step_.data() + offsetof(step_state, seq), (int)((2 * l + 1) & 1023), stream_));
+      norm_ready = true;
+    } else if (n > 1 && l + 1 < model_->layers.size()) {
+      matmul_norm(x, t_silu_.data(), L.w2, n, model_->layers[l + 1].attn_norm);                              // 1185, 1129
       norm_ready = true;
     } else {
       matmul(x, t_silu_.data(), L.w2, n, 1.0f);                                                              // 1185

@@ -1262,3 +1262,27 @@ def test_softmax_argmax_fused(gpu, n, temp):
     assert int(G.host(idx_d, (1,), np.int32)[0]) == O.argmax_first(got) == int(np.flatnonzero(got[0] == got.max())[0])
     assert G.L().lcu_softmax_argmax(probs_d.ptr, idx_d.ptr, probs_d.ptr, n, temp, None) == -2
     G.release()
+
+
+# more rows than the kernel of few rows takes: even and odd 64-blocks of K apart (one stage each, odd counts, ragged rows and columns, blocks of 64
+# and 256 codes), too short a K for that, splits of large tiles and of 128 rows, a single chain, and a K that is no whole number of stages
+@pytest.mark.parametrize("M,K,N,block", [(512, 4096, 4096, 0), (65, 128, 130, 0), (130, 384, 1030, 0), (511, 384, 2050, 0), (300, 1152, 1030, 64), (200, 2304, 4094, 256),
+                                         (512, 11008, 4096, 0), (100, 11008, 4096, 128), (300, 5120, 8192, 128), (1000, 256, 8192, 0),
+                                         (70, 320, 512, 0), (90, 256, 9000, 128)])
+def test_product_residual_norm_of_many_rows(gpu, M, K, N, block):
+    """lcu_batch_proj_norm against the product and the norm by themselves, bit for bit."""
+    G = gpu
+    check, L = G.B.check, G.L()
+    x, lhs, w, nw = normal((M, N), 0, 1800, 1.0), normal((M, K), 0, 1801, 1.0), normal((N, K), 0, 1802, 0.02), normal((N,), 0, 1803, 1.0)
+    wd = [G.dev_keep(part) for part in (O.quantize_absmax_u8(w, block) if block else (w,))]
+    ld, nd = G.dev_keep(lhs), G.dev_keep(nw)
+    xa, xb, na, nb = G.dev(x), G.dev(x), G.empty((M, N)), G.empty((M, N))
+    check(L.lcu_batch_proj_norm(xa.ptr, na.ptr, ld.ptr, wd[0].ptr, wd[1].ptr if block else None, block, M, K, N, nd.ptr, 1e-6, None))
+    if block:
+        check(L.lcu_gemm_f16u8_nt(xb.ptr, ld.ptr, wd[0].ptr, wd[1].ptr, M, K, N, block, 1.0, None))
+    else:
+        check(L.lcu_gemm_f16_nt(xb.ptr, ld.ptr, wd[0].ptr, M, K, N, 1.0, None))
+    check(L.lcu_rmsnorm(nb.ptr, xb.ptr, nd.ptr, M, N, 1e-6, None))
+    assert (G.host(xa, (M, N)).view(np.uint16) == G.host(xb, (M, N)).view(np.uint16)).all()
+    assert (G.host(na, (M, N)).view(np.uint16) == G.host(nb, (M, N)).view(np.uint16)).all()
+    G.release()
