@@ -927,15 +927,15 @@ struct columns_t {
 };
 
 // A launch of gemm_tile_kernel; splits > 1: the K stages of every tile dealt to that many workgroups, fp32 sums to part.
-template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
+template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP>
 int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits = 1,
                 float* part = nullptr, columns_t which = {}, int step = 1) {
-  using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
+  using shape = tile_shape<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP>;
   const int tiles_m = (M + BM - 1) / BM;
   if (which.from > 0) op = last_matrix(op);
   const int tiles_n_per = (N - which.from + BN - 1) / BN, tiles_n = which.tiles > 0 ? which.tiles : tiles_n_per * op.n_mats;
   op.more.tiles_n_per = op.n_mats > 1 ? tiles_n_per : 0;
-  auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
+  auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -957,13 +957,13 @@ struct large_tiles_t {
   int rest_rows, rest_columns;
 };
 
-// The tiles whose rounds of workgroups cost least.  fp16 and bfloat16: a round of 128 / 192 / 256 columns takes 57 / 88 / 106 us at K = 4096 (512
-// rows, W1 and W3 of 11008 columns in one launch: 230 tiles of 192 columns 88 us, 172 of 256 94 us, 344 of 128 108 us; 1987 rows: 303 us
-// with 256 columns, 330 us with 128), one of 128x128 tiles 41.  uint8: 59 / 79 / 104 and 40 (512 rows, K 6656, three times 6656 columns: 156 tiles of
+// The tiles whose rounds of workgroups cost least.  fp16 and bfloat16: a round of 128 / 192 / 256 columns takes 57 / 73 / 94 us at K = 4096 (512
+// rows, W1 and W3 of 11008 columns in one launch: 230 tiles of 192 columns 82 us, 172 of 256 92, 344 of 128 110; 1987 rows: 307, 293 and
+// 332 us), one of 128x128 tiles 41.  uint8: 59 / 79 / 104 and 40 (512 rows, K 6656, three times 6656 columns: 156 tiles of
 // 256 191 us, 208 of 192 148, 312 of 128 208; K 4096, twice 11008: 107 / 86 / 118; 1987 rows 341 / 346 / 381).
 // A last round that is nearly empty goes to smaller tiles: whole rounds of one width, then the columns that are left in those tiles that cost least
-// (us, the best single width / so: 512 rows, K 6656, twice 17920 columns uint8 254 / 234, fp16 266 / 234; K 4096, 700 rows, twice 11008 fp16
-// 143 / 136, 1000 rows 164 / 158, 1987 rows 300 / 290).  The second launch costs 3 us more; below 1024 of K that is what it gains.
+// (us, the best single width / so: uint8 512 rows, K 6656, twice 17920 columns 254 / 234; fp16 K 4096, twice 11008 columns, 700 rows 143 / 136,
+// 1000 rows 164 / 158, 1987 rows 300 / 290).  The second launch costs 3 us more; below 1024 of K that is what it gains.
 // Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts there.
 // Up to 512 of K what a tile pays beside its stages counts: 256 columns leave by four wavefronts, and the rounds are no measure of
 // them (1441 rows of K 256, three times 2944 columns: 216 tiles of 256 20.1 us, 414 of 128 16.5; bfloat16 1027x512x11840 28.7 / 23.4),
@@ -978,7 +978,7 @@ large_tiles_t plan_large(int M, int K, int N, int n_mats, long cus, bool gated) 
     const long c128 = rounds(tiles(128, 128, N) * n_mats) * (U8 ? 42 : 52), c256 = rounds(tiles(128, 256, N) * n_mats) * (U8 ? 62 : 66);
     return {c256 < c128 ? 256 : 128, {}, {}, 0, 0};
   }
-  const auto round = [&](int columns) -> long { return columns == 128 ? (U8 ? 59 : 57) : columns == 192 ? (U8 ? 79 : 88) : (U8 ? 104 : 106); };
+  const auto round = [&](int columns) -> long { return columns == 128 ? (U8 ? 59 : 57) : columns == 192 ? (U8 ? 79 : 73) : (U8 ? 104 : 94); };
   const auto allowed = [&](int columns) { return columns == 128 || (columns == 192 ? K >= 256 && !gated : K >= 640); };
   large_tiles_t best{128, {}, {}, 0, 0};
   long least = rounds(tiles(256, 128, N) * n_mats) * round(128);
@@ -1013,15 +1013,15 @@ template <bool U8, class EP>
 int launch_columns(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st, int columns,
                    columns_t which) {
   if constexpr (U8) {
-    if (columns == 256) return launch_tile<256, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
-    if (columns == 192) return launch_tile<256, 192, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
-    return launch_tile<256, 128, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
+    if (columns == 256) return launch_tile<256, 256, 1, 4, 3, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
+    if (columns == 192) return launch_tile<256, 192, 1, 4, 3, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
+    return launch_tile<256, 128, 1, 4, 3, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
   } else {
-    if (columns == 256) return launch_tile<256, 256, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
+    if (columns == 256) return launch_tile<256, 256, 2, 2, 2, 3, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
     if constexpr (!EP::GATED) {
-      if (columns == 192) return launch_tile<256, 192, 2, 2, 2, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
+      if (columns == 192) return launch_tile<256, 192, 2, 2, 2, 4, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
     }
-    return launch_tile<256, 128, 4, 2, 3, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
+    return launch_tile<256, 128, 4, 2, 3, 3, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
   }
 }
 
@@ -1031,17 +1031,17 @@ int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N
   const large_tiles_t plan = plan_large<U8>(M, K, N, op.n_mats, ds && ds->compute_units > 0 ? ds->compute_units : 256, EP::GATED);
   if (M <= 128) {
     if constexpr (U8) {
-      if (plan.columns == 256) return launch_tile<128, 256, 1, 4, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
-      return launch_tile<128, 128, 1, 4, 4, true, false>(ep, op, A, M, K, N, block, beta, st);
+      if (plan.columns == 256) return launch_tile<128, 256, 1, 4, 3, 3, true, false>(ep, op, A, M, K, N, block, beta, st);
+      return launch_tile<128, 128, 1, 4, 4, 4, true, false>(ep, op, A, M, K, N, block, beta, st);
     } else {
-      if (plan.columns == 256) return launch_tile<128, 256, 2, 4, 3, false, false>(ep, op, A, M, K, N, 0, beta, st);
-      return launch_tile<128, 128, 2, 2, 4, false, false>(ep, op, A, M, K, N, 0, beta, st);
+      if (plan.columns == 256) return launch_tile<128, 256, 2, 4, 3, 3, false, false>(ep, op, A, M, K, N, 0, beta, st);
+      return launch_tile<128, 128, 2, 2, 4, 4, false, false>(ep, op, A, M, K, N, 0, beta, st);
     }
   }
   const int rc = launch_columns<U8>(ep, op, A, M, K, N, block, beta, st, plan.columns, plan.first);
   if (rc != LCU_OK || plan.rest.from == 0) return rc;
   if (plan.rest_rows == 256) return launch_columns<U8>(ep, op, A, M, K, N, block, beta, st, plan.rest_columns, plan.rest);
-  return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, U8, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, plan.rest);
+  return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, 4, U8, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, plan.rest);
 }
 
 // where a split-K launch left its partial sums: part[matrix][split][M][N] fp32
@@ -1225,9 +1225,9 @@ inline int large_tile_splits(int M, int K, int N, int n_mats, long cus, size_t w
 template <bool U8>
 int launch_partial(operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, bool small, int step) {
   if (small || M <= 128) {
-    return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+    return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, 4, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
   }
-  return launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+  return launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
 }
 
 template <bool U8>
@@ -1598,7 +1598,7 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         // more tiles than compute units, which the register-staged kernel puts two to a compute unit, 1000 rows of 4608 columns
         // 11.4 / 14.0, 15.8 / 17.8, 24.5 / 25.6, 41.9 / 41.6
         const bool long_enough = tiles128 < 256 ? K >= 384 : tiles128 / nm <= 256 || K >= 1536;
-        if (block_shift(block) >= 0 && long_enough) return launch_tile<128, 128, 1, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        if (block_shift(block) >= 0 && long_enough) return launch_tile<128, 128, 1, 4, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
         if (tiles128 < 256) return launch_dl<128, 128, 4, 2, 1, 3, true>(op, A, M, K, N, block, beta, st);
       } else {
         // us, K 256, 512, 1024, 1536, 2048: eight wavefronts / here, 512 rows of 5120 columns 6.2 / 7.1, 7.8 / 8.5, 10.9 / 11.2, 16.1 / 15.2, 22.0 / 22.3;
@@ -1607,7 +1607,7 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         // with weights from memory the second workgroup also hides the second round's first requests: K 1280, 1536, 1792, 512 rows of
         // 10000 columns 30.3 / 34.4, 34.2 / 38.2, 38.9 / 42.0, 896 rows of 4992 26.6 / 28.3, 30.4 / 31.0, 34.6 / 34.1
         if (K < 1536 && tiles128 > 256) return launch_dl<128, 128, 2, 2, 1, 2, false>(op, A, M, K, N, block, beta, st);
-        return launch_tile<128, 128, 2, 2, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
+        return launch_tile<128, 128, 2, 2, 4, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
       }
     } else {
       if (tiles64 > 256) return launch_dl<128, 64, 2, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
@@ -1730,7 +1730,7 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
   if constexpr (GATED) {  // 1000 rows of 4608 columns, K 512, 1024, 2048: 17.2 us, 24.5, 43.1 with two workgroups per compute unit, else 17.8, 24.8, 39.7
     if (K < 1280 && tm(128) * tn(128) > 256) return launch_bf16<128, 128, 2, 2, 1, 2>(ep, A, W, tm(128), M, K, N, st);
   }
-  if (tm(128) * tn(128) >= 160) return launch_tile<128, 128, 2, 2, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
+  if (tm(128) * tn(128) >= 160) return launch_tile<128, 128, 2, 2, 4, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
   if constexpr (GATED) {
     if (tm(128) * tn(64) > 128) return launch_bf16<128, 64, 4, 1, 1, 3>(ep, A, W, tm(128), M, K, N, st);
     return launch_bf16<64, 64, 2, 1, 1, 3>(ep, A, W, tm(64), M, K, N, st);

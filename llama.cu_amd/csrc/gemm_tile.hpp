@@ -9,7 +9,7 @@
 //    tiles 133 -> 119 us).  Both take their products eight at a time in ascending k, so the bits are the same.
 //  * neighbouring instructions share an operand, also where the row of tiles changes (boustrophedon order).
 //  * a half stage (32 of K) of fragments is read from LDS while the half before it is multiplied, one read
-//    between two matrix instructions; requests for the stage NS ahead go out the same way.
+//    between two matrix instructions; requests for the stages ahead go out the same way.
 //  * requests are buffer loads straight into LDS whose stage offset is a scalar.  Behind the last stage the
 //    resource holds no records and the offset is 0 (operand_range.hpp): the request counts as any other but touches
 //    no memory, so that the loop has one form up to the end and its registers are never copied.
@@ -73,7 +73,10 @@ __device__ __forceinline__ half2_t dequant2(uint32_t spread, half2_t scale2x) {
   return t * scale2x;                                                                 // one rounding
 }
 
-// WM x WN wavefronts of (BM / WM) x (BN / WN) outputs each, a ring of NS stages of 64 along K.
+// WM x WN wavefronts of (BM / WM) x (BN / WN) outputs each, rings of NA stages of 64 along K of lhs and NB of W.  The lhs comes from L2, W
+// from memory: where LDS does not hold three stages of both, W's ring takes what two of lhs leave (fp16, 512 rows of K 4096, a round of 192
+// columns 82 -> 67 us with rings of two and two -> two and four, of 256 columns 93 -> 84; 1987 rows, twice 11008 columns 304 -> 293.  From
+// three stages on longer rings of W measured equal or slower, in uint8 too.)
 // U8: W is codes with one fp16 scale per `block` of a row, block = 64 << block_shift.  Codes lie in LDS as they are, 64
 // bytes a row with the 16-byte pieces of every second group of four rows turned by two (a sixth of LDS's cycles still go to conflicts of
 // their 8-byte reads, a ninth with 256 columns: counted on 512x6656x35840 and 512x6656x19968); a wavefront turns
@@ -82,29 +85,30 @@ __device__ __forceinline__ half2_t dequant2(uint32_t spread, half2_t scale2x) {
 // is converted once; with the lhs read from LDS by all four that leaves vector instructions, LDS and matrix cores about
 // equally busy.  512 rows, (N, K) = (11008, 4096): 64 us; two rows of two wavefronts (every code twice) 64-66, four of two
 // 88; converted once into an fp16 tile in LDS, with its own ring, 87 us.  1987 rows, twice (11008, 4096): 346 / 432 / 492 / 475 us.
-template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
+template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP>
 struct tile_shape {
   static constexpr int NW = WM * WN, WR = BM / WM, WC = BN / WN;
   static constexpr int A_BYTES = BM * 128, B_BYTES = BN * (U8 ? 64 : 128), SW = (WC + 63) / 64 * 64, S_BYTES = U8 ? NW * SW * 4 : 0;
-  static constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES;  // S: one word per column of every wavefront, of its own
+  static constexpr int W_BYTES = B_BYTES + S_BYTES;      // S: one word per column of every wavefront, of its own
   static constexpr int OUT_LD = WC + 4;                  // floats per row of a wavefront's 64 output rows in LDS
-  static constexpr int RING = NS * STAGE, OUT = NW * 64 * OUT_LD * 4;
+  static constexpr int RING = NA * A_BYTES + NB * W_BYTES, OUT = NW * 64 * OUT_LD * 4;
   static constexpr int LDS = RING > OUT ? RING : OUT;
   static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 16 == 0, "tile");
 };
 
-template <int BM, int BN, int WM, int WN, int NS, bool U8, bool SPLIT, class EP>
+template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0, int block_shift,
     int M, int K, int N, float beta, int tiles_m, int tiles_n, int from, float* __restrict__ part, int splits, int step, more_matrices_t more, EP ep) {
-  using shape = tile_shape<BM, BN, WM, WN, NS, U8, SPLIT, EP>;
+  using shape = tile_shape<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP>;
   static_assert(!EP::GROUPED, "one matrix for all rows");
   constexpr int NW = shape::NW;
   constexpr int TM = shape::WR / 16, TN = shape::WC / 16;        // 16x16 tiles of a wavefront
-  constexpr int A_BYTES = shape::A_BYTES, B_BYTES = shape::B_BYTES, STAGE = shape::STAGE;
+  constexpr int A_BYTES = shape::A_BYTES, B_BYTES = shape::B_BYTES, W_BYTES = shape::W_BYTES, W_RING = NA * A_BYTES;
   constexpr int PA = A_BYTES / 1024 / NW, PB = B_BYTES / 1024 / NW, PS = U8 ? shape::SW / 64 : 0;
-  constexpr int P = PA + PB + PS;  // requests of a wavefront per stage
-  static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0 && NS >= 2 && P * (NS - 1) < 64, "requests");
+  constexpr int PW = PB + PS, P = PA + PW;  // requests of a wavefront per stage
+  constexpr int BEHIND = NB > NA ? PW : 0;  // of a stage's requests, those behind its lhs that lhs's turn need not wait for
+  static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0 && NA >= 2 && NB >= NA && PA * NA + PW * NB < 64, "requests");
   static_assert(!U8 || !EP::BF16, "codes");
   extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
 
@@ -179,16 +183,16 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
                  "s"(lds0 + at)
                  : "memory", "m0");
   };
-  const auto issue = [&](int stage, int slot, int i) {
-    const uint32_t along = stage_offset(ra[2], stage_of(stage) * 128u);
+  // request i of a wavefront's P: lhs of stage `a` into its ring's slot, then the columns (and scales) of stage `b` into theirs
+  const auto issue = [&](int a, int a_slot, int b, int b_slot, int i) {
     if (i < PA) {
-      request(ra, along, a_off[i], slot * STAGE + (wave + i * NW) * 1024);
+      request(ra, stage_offset(ra[2], stage_of(a) * 128u), a_off[i], a_slot * A_BYTES + (wave + i * NW) * 1024);
     } else if (i < PA + PB) {
-      request(rw, U8 ? along / 2 : along, b_off[i - PA], slot * STAGE + A_BYTES + (wave + (i - PA) * NW) * 1024);
+      request(rw, stage_offset(rw[2], stage_of(b) * (U8 ? 64u : 128u)), b_off[i - PA], W_RING + b_slot * W_BYTES + (wave + (i - PA) * NW) * 1024);
     } else if constexpr (U8) {  // the word that holds the row's scale of this stage
-      const uint32_t at = s_first[i - PA - PB] + (stage_of(stage) >> block_shift);
+      const uint32_t at = s_first[i - PA - PB] + (stage_of(b) >> block_shift);
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(scale_word(at)), "s"(rs),
-                   "s"(lds0 + slot * STAGE + A_BYTES + B_BYTES + wave * shape::SW * 4 + (i - PA - PB) * 256)
+                   "s"(lds0 + W_RING + b_slot * W_BYTES + B_BYTES + wave * shape::SW * 4 + (i - PA - PB) * 256)
                    : "memory", "m0");
     }
   };
@@ -203,7 +207,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   uint32_t pos[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) pos[h] = (uint32_t)(((frag_chunk + 4 * h) ^ turn) * 16);
-  const uint32_t a_row = (uint32_t)(wm + frag_row) * 128, b_row = (uint32_t)A_BYTES + (uint32_t)(wn + frag_row) * 128;
+  const uint32_t a_row = (uint32_t)(wm + frag_row) * 128, b_row = (uint32_t)W_RING + (uint32_t)(wn + frag_row) * 128;
   half8_t fa[2][TM], fb[2][TN];
   // U8: the eight codes behind a fragment, and twice their scale
   uint2_t codes[2][U8 ? TN : 1];
@@ -211,26 +215,26 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   half2_t scales[U8 ? TN : 1];
   // reads of half 0: (scales, codes,) W and lhs fragments of half 0(, codes of half 1); of half 1 the fragments that are left
   constexpr int READS0 = U8 ? 3 * TN + TM : TN + TM, READS1 = U8 ? TM : TN + TM, PRODUCTS = TM * TN;
-  const auto read = [&](int slot, int h, int i) {
-    const unsigned char* p = tile_lds + slot * STAGE;
+  const auto read = [&](int a_slot, int b_slot, int h, int i) {
+    const unsigned char *pa = tile_lds + a_slot * A_BYTES + a_row, *pw = tile_lds + b_slot * W_BYTES;
     if constexpr (U8) {
-      const unsigned char* c = p + A_BYTES + (wn + frag_row) * 64 + frag_chunk * 8;
+      const unsigned char* c = pw + W_RING + (wn + frag_row) * 64 + frag_chunk * 8;
       const int half_turn = (frag_row / 4) % 2 * 32;  // pieces turned by two: the halves change places
       if (h == 1) {
-        fa[1][i] = *reinterpret_cast<const half8_t*>(p + pos[1] + a_row + i * 2048);
+        fa[1][i] = *reinterpret_cast<const half8_t*>(pa + pos[1] + i * 2048);
       } else if (i < TN) {
-        words[i] = *reinterpret_cast<const uint32_t*>(p + A_BYTES + B_BYTES + wave * shape::SW * 4 + (i * 16 + frag_row) * 4);
+        words[i] = *reinterpret_cast<const uint32_t*>(pw + W_RING + B_BYTES + wave * shape::SW * 4 + (i * 16 + frag_row) * 4);
       } else if (i < 2 * TN) {
         codes[0][i - TN] = *reinterpret_cast<const uint2_t*>(c + (i - TN) * 1024 + half_turn);
       } else if (i < 2 * TN + TM) {
-        fa[0][i - 2 * TN] = *reinterpret_cast<const half8_t*>(p + pos[0] + a_row + (i - 2 * TN) * 2048);
+        fa[0][i - 2 * TN] = *reinterpret_cast<const half8_t*>(pa + pos[0] + (i - 2 * TN) * 2048);
       } else {
         codes[1][i - 2 * TN - TM] = *reinterpret_cast<const uint2_t*>(c + (i - 2 * TN - TM) * 1024 + (32 - half_turn));
       }
     } else if (i < TN) {
-      fb[h][i] = *reinterpret_cast<const half8_t*>(p + pos[h] + b_row + i * 2048);
+      fb[h][i] = *reinterpret_cast<const half8_t*>(pw + pos[h] + b_row + i * 2048);
     } else {
-      fa[h][i - TN] = *reinterpret_cast<const half8_t*>(p + pos[h] + a_row + (i - TN) * 2048);
+      fa[h][i - TN] = *reinterpret_cast<const half8_t*>(pa + pos[h] + (i - TN) * 2048);
     }
   };
   // two of the eight values of a fragment of half h from their codes, which belong to stage `st`; four instructions, as
@@ -281,48 +285,54 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
       __builtin_amdgcn_sched_barrier(0);
     });
   };
-  // One stage in ring slot `slot`: multiply its first half while the second is read; this wavefront has then read
-  // the whole stage, and once its own requests of the next stage have landed (at most those of NS - 2 later stages
-  // outstanding) the barrier says both for everybody.  Then the second half, with the next stage's first half on its
-  // way from slot `next_slot` and the stage NS ahead requested into `slot`.
-  const auto stage = [&](int t, int slot, int next_slot, int ahead, auto more_follow) {
+  // One stage: multiply its first half while the second is read; this wavefront has then read the whole stage, and once its own
+  // requests of the next stage have landed the barrier says both for everybody.  Then the second half, with the next stage's first half
+  // on its way and the stages NA and NB ahead requested into this one's slots.  Of a stage's requests the lhs goes first: when that of
+  // stage t + 1 has to be there, the columns asked for behind it and all of the NA - 2 stages since may still be out.
+  const auto stage = [&](int t, int a_slot, int b_slot, int a_next, int b_next, auto more_follow) {
     constexpr bool MORE = decltype(more_follow)::value;
-    half_stage(0, std::integral_constant<int, READS1>{}, [&](int k) { read(slot, 1, k); }, std::integral_constant<int, 0>{}, [](int) {},
+    half_stage(0, std::integral_constant<int, READS1>{}, [&](int k) { read(a_slot, b_slot, 1, k); }, std::integral_constant<int, 0>{}, [](int) {},
                std::integral_constant<int, CONVERTS>{}, t);
     if constexpr (MORE) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      wait_vmcnt<(NS - 2) * P>();
+      wait_vmcnt<(NA - 2) * P + BEHIND>();
       asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      half_stage(1, std::integral_constant<int, READS0>{}, [&](int k) { read(next_slot, 0, k); }, std::integral_constant<int, P>{},
-                 [&](int k) { issue(ahead, slot, k); }, std::integral_constant<int, CONVERTS>{}, t + 1);
+      half_stage(1, std::integral_constant<int, READS0>{}, [&](int k) { read(a_next, b_next, 0, k); }, std::integral_constant<int, P>{},
+                 [&](int k) { issue(t + NA, a_slot, t + NB, b_slot, k); }, std::integral_constant<int, CONVERTS>{}, t + 1);
     } else {
       half_stage(1, std::integral_constant<int, 0>{}, [](int) {}, std::integral_constant<int, 0>{}, [](int) {},
                  std::integral_constant<int, 0>{}, 0);
     }
   };
 
+  // no records behind the last stage: a request brings zeros and reads nothing (stage_offset)
+  const auto end_at = [&](int a, int b) {
+    if (a == nt) ra[2] = 0;
+    if (b == nt) rw[2] = rs[2] = 0;
+  };
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    if (s == nt) ra[2] = rw[2] = rs[2] = 0;  // no records: a request brings zeros and reads nothing (stage_offset)
+  for (int s = 0; s < NB; ++s) {  // what the stages before stage 0 would have asked for
+    end_at(s - (NB - NA), s);
 #pragma unroll
-    for (int i = 0; i < P; ++i) issue(s, s, i);
+    for (int i = s < NB - NA ? PA : 0; i < P; ++i) issue(s - (NB - NA), max(s - (NB - NA), 0), s, s, i);
   }
-  wait_vmcnt<(NS - 1) * P>();
+  wait_vmcnt<(NA - 1) * P + BEHIND>();
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < READS0; ++i) read(0, 0, i);
+  for (int i = 0; i < READS0; ++i) read(0, 0, 0, i);
 #pragma unroll
   for (int k = 0; k < CONVERTS; ++k) convert(0, k, 0);
   __builtin_amdgcn_sched_barrier(0);
-  int slot = 0;
+  int a_slot = 0, b_slot = 0;
   for (int t = 0; t < nt - 1; ++t) {
-    if (t + NS == nt) ra[2] = rw[2] = rs[2] = 0;
-    const int next_slot = slot + 1 == NS ? 0 : slot + 1;
-    stage(t, slot, next_slot, t + NS, std::true_type{});
-    slot = next_slot;
+    end_at(t + NA, t + NB);
+    const int a_next = a_slot + 1 == NA ? 0 : a_slot + 1, b_next = b_slot + 1 == NB ? 0 : b_slot + 1;
+    stage(t, a_slot, b_slot, a_next, b_next, std::true_type{});
+    a_slot = a_next;
+    b_slot = b_next;
   }
-  stage(nt - 1, slot, 0, 0, std::false_type{});
+  stage(nt - 1, a_slot, b_slot, 0, 0, std::false_type{});
   wait_vmcnt<0>();  // the requests behind the last stage have written their zeros
   __syncthreads();  // LDS is free
 

@@ -32,38 +32,42 @@ struct shape {
   int M, K, N, block, splits;  // block 0: fp16
 };
 
-// gemm_tile.hpp: tiles of BM x BN, a ring of NS stages
-void walk_tile(const shape& s, int BM, int BN, int NS) {
+// gemm_tile.hpp: tiles of BM x BN, a ring of NS stages, or of NS for lhs and NB for W; step > 1: every so many of the stages
+void walk_tile(const shape& s, int BM, int BN, int NS, int NB = 0, int step = 1) {
+  if (NB == 0) NB = NS;
   const bool u8 = s.block != 0;
   int shift = 0;
   while (u8 && (64 << shift) < s.block) ++shift;
   const uint32_t K = s.K, blocks = u8 ? K >> (6 + shift) : 0, wbytes = u8 ? 1 : 2;
   const uint64_t a_size = (uint64_t)s.M * K * 2, w_size = (uint64_t)s.N * K * wbytes, s_size = (uint64_t)s.N * blocks * 2;
-  const int nt_all = s.K / 64;
+  const int nt_all = s.K / 64, splits = step > 1 ? step : s.splits;
   // a tile in the middle asks for what one of the first tile asks for, shifted: the first and the last of each direction
   for (int m0 : {0, (s.M - 1) / BM * BM}) {
     for (int n0 : {0, (s.N - 1) / BN * BN}) {
-      for (int split : {0, s.splits / 2, s.splits - 1}) {
-        const int stage0 = (int)((long)split * nt_all / s.splits), nt = (int)((long)(split + 1) * nt_all / s.splits) - stage0;
+      for (int split : {0, splits / 2, splits - 1}) {
+        const int stage0 = step > 1 ? split : (int)((long)split * nt_all / splits);
+        const int nt = step > 1 ? nt_all / step : (int)((long)(split + 1) * nt_all / splits) - stage0;
         uint32_t la = (uint32_t)a_size, lw = (uint32_t)w_size, ls = (uint32_t)s_size;
-        const auto issue = [&](int stage) {
-          const uint32_t along = along_of(la, (uint32_t)(stage0 + stage) * 128u);
+        const auto issue_lhs = [&](int stage) {
+          const uint32_t along = along_of(la, (uint32_t)(stage0 + stage * step) * 128u);
           for (int row = 0; row < BM; ++row)
             for (int g = 0; g < 8; ++g) request(la, lcu::row_piece(m0 + row, s.M, K * 2, g), along, 16, a_size);
+        };
+        const auto issue_w = [&](int stage) {
+          const uint32_t along = along_of(lw, (uint32_t)(stage0 + stage * step) * (u8 ? 64u : 128u));
           for (int row = 0; row < BN; ++row) {
-            for (int g = 0; g < (u8 ? 4 : 8); ++g)
-              request(lw, lcu::row_piece(n0 + row, s.N, K * wbytes, g), u8 ? along / 2 : along, 16, w_size);
-            if (u8) request(ls, lcu::scale_word((uint32_t)std::min(n0 + row, s.N - 1) * blocks + ((uint32_t)(stage0 + stage) >> shift)), 0, 4, s_size);
+            for (int g = 0; g < (u8 ? 4 : 8); ++g) request(lw, lcu::row_piece(n0 + row, s.N, K * wbytes, g), along, 16, w_size);
+            if (u8) request(ls, lcu::scale_word((uint32_t)std::min(n0 + row, s.N - 1) * blocks + ((uint32_t)(stage0 + stage * step) >> shift)), 0, 4, s_size);
           }
         };
-        for (int st = 0; st < NS; ++st) {
-          if (st == nt) la = lw = ls = 0;
-          issue(st);
-        }
-        for (int t = 0; t < nt - 1; ++t) {
-          if (t + NS == nt) la = lw = ls = 0;
-          issue(t + NS);
-        }
+        const auto issue = [&](int a, int b) {
+          if (a == nt) la = 0;
+          if (b == nt) lw = ls = 0;
+          if (a >= 0) issue_lhs(a);
+          issue_w(b);
+        };
+        for (int st = 0; st < NB; ++st) issue(st - (NB - NS), st);
+        for (int t = 0; t < nt - 1; ++t) issue(t + NS, t + NB);
       }
     }
   }
@@ -109,6 +113,9 @@ int main(int argc, char** argv) {
     walk_tile(s, 256, 128, 3);
     walk_tile(s, 128, 256, 3);
     walk_tile(s, 128, 128, 4);
+    walk_tile(s, 256, 192, s.block ? 3 : 2, s.block ? 3 : 4);
+    walk_tile(s, 256, 256, 2, 3);
+    if (s.K % 128 == 0) walk_tile(s, 128, 128, 4, 4, 2);
   }
   const shape rows[] = {{3, 1152, 520, 0, 4},     {16, 1408, 4099, 0, 5},  {48, 5888, 4100, 0, 2},  {7, 64, 40, 0, 1},
                         {2, 1152, 520, 64, 4},    {17, 2560, 1000, 256, 7}, {64, 5888, 4101, 128, 3}, {7, 17920, 6656, 128, 5},
