@@ -467,7 +467,8 @@ int lcu_latent_rows(const lcu_latent_rows_args* rows, const lcu_latent_params* p
 /* Few tokens, bfloat16, without keys and values multiplied out.  lcu_latent_queries: out [n][heads * ldc], head h =
  * uk_t[h] [ldc][dn] times the unrotated part of the query; with rows, lcu_latent_rows in the same launch (the
  * unrotated parts do not depend on it).  lcu_latent_attention: scores and softmax over the latents (sink as above,
- * NULL: none), then uv [heads * dv][ldc] and the gate (NULL: none).  scratch: lcu_latent_attention_scratch bytes;
+ * NULL: none), then uv [heads * dv][ldc] and the gate (NULL: none); one token that sees at most 512 positions
+ * (max_positions or the window) in one launch.  scratch: lcu_latent_attention_scratch bytes;
  * lcu_latent_attention_fits: 0 where the sizes are too large for its kernels (ldc above 512). */
 int lcu_latent_queries(void* out_dev, const void* q_dev, int ldq, const void* uk_t_dev, const lcu_latent_params* p,
                        const lcu_latent_rows_args* rows, int n, void* stream);

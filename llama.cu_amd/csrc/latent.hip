@@ -354,6 +354,199 @@ __global__ __launch_bounds__(256) void latent_value_kernel(latent_value_args p) 
   }
 }
 
+// ---- one token ------------------------------------------------------------------------------------------
+// Scores, weighted sums and value matrix of a head in one launch.  Workgroup: a head and a part of its values; its eight
+// wavefronts take eight neighbouring keys at a time, a lane eight columns of the latent, with a maximum, a sum and weighted
+// columns of their own until the end, where they meet in LDS.  Probabilities and the weighted latent stay in fp32.
+//
+// What bounds it: round trips to memory, one after another (the launches above: position, queries into LDS, latents, scores,
+// transposed latents in LDS, sums to memory and back, 11.5 + 6.6 us for 130 keys and 16 heads, three of 256 compute units at
+// work in the first).  Here everything the first 256 keys need is asked for at the start, value matrix and gate too, and nothing
+// goes back to memory: 9.2 us.  Every workgroup goes through all keys, 2.1 us per hundred of them (25.5 us at 915), so beyond
+// LATENT_TOKEN_KEYS the slices above are sooner done.  (Sixteen wavefronts and a sum over the wavefront per key spilled: 20 us.)
+constexpr int TOKEN_WAVES = 8, TOKEN_KEYS = 8, LATENT_TOKEN_KEYS = 512;
+
+// a . b of eight bfloat16 pairs in fp32
+__device__ __forceinline__ float bf16_dot(bf16x8_t a, bf16x8_t b) {
+  float s = 0.0f;
+  const uint4_t x = __builtin_bit_cast(uint4_t, a), y = __builtin_bit_cast(uint4_t, b);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s = fmaf(__builtin_bit_cast(float, x[e] << 16), __builtin_bit_cast(float, y[e] << 16), s);
+    s = fmaf(__builtin_bit_cast(float, x[e] & 0xffff0000u), __builtin_bit_cast(float, y[e] & 0xffff0000u), s);
+  }
+  return s;
+}
+// the halves of the wavefront, and the rows of 16 lanes in each half, change places between two values
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  const uint32_t first = r[0], second = r[1];  // a bit cast of r[1] itself takes r[0]
+  a = __builtin_bit_cast(float, first);
+  b = __builtin_bit_cast(float, second);
+}
+__device__ __forceinline__ void swap_rows(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  const uint32_t first = r[0], second = r[1];  // a bit cast of r[1] itself takes r[0]
+  a = __builtin_bit_cast(float, first);
+  b = __builtin_bit_cast(float, second);
+}
+// lanes 8 i .. 8 i + 7: sum of x[i] over all lanes
+__device__ __forceinline__ float sums_of_eight(float (&x)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    swap_halves(x[i], x[i + 4]);
+    x[i] += x[i + 4];
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    swap_rows(x[i], x[i + 2]);
+    x[i] += x[i + 2];
+  }
+  const bool upper = threadIdx.x & 8;
+  float v = (upper ? x[1] : x[0]) + dpp_f32<0x128>(upper ? x[0] : x[1]);  // turned by eight lanes of sixteen
+  v += dpp_f32<0xB1>(v);
+  v += dpp_f32<0x4E>(v);
+  return v + dpp_f32<0x141>(v);
+}
+// over the eight groups of eight lanes, whose lanes are equal
+template <class F>
+__device__ __forceinline__ float over_eights(float v, F&& f) {
+  v = f(v, dpp_f32<0x128>(v));
+  float w = v;
+  swap_rows(v, w);
+  v = w = f(v, w);
+  swap_halves(v, w);
+  return f(v, w);
+}
+
+__global__ __launch_bounds__(64 * TOKEN_WAVES) void latent_token_kernel(latent_args p, latent_value_args v) {
+  __shared__ __attribute__((aligned(16))) float O[TOKEN_WAVES][512];
+  __shared__ float ml[TOKEN_WAVES][2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.x;
+  const int rows = (v.dv + gridDim.y - 1) / gridDim.y, r0 = blockIdx.y * rows, r1 = min(r0 + rows, v.dv);
+  const int column = min(lane * 8, p.ldc - 8), turned = min((lane & 7) * 8, p.dr - 8);  // this lane's piece of a latent, of a rotated part
+  const bool live = lane * 8 < p.ldc, turns = (lane & 7) * 8 < p.dr;
+  const bf16x8_t none = (bf16x8_t)(bf16_t)0.0f;
+  const int hi = min(max(*p.start, 0), p.max_pos - 1), lo = max(0, hi - p.window + 1);
+  // the queries; zero where the lane has no piece
+  const bf16x8_t q = live ? *reinterpret_cast<const bf16x8_t*>(p.q + (size_t)h * p.ldc + column) : none;
+  const bf16x8_t qr = turns ? *reinterpret_cast<const bf16x8_t*>(p.q_rot + (size_t)h * p.head_ld + turned) : none;
+  const float sink = v.sink ? v.sink[h] : -1e30f;
+  // keys base .. base + 7, those behind the last one as the last one; lanes 8 i .. 8 i + 7 hold the rotated part of key i
+  const auto ask = [&](int base, bf16x8_t (&c)[TOKEN_KEYS], bf16x8_t (&kr)[TOKEN_KEYS / 8]) {
+#pragma unroll
+    for (int i = 0; i < TOKEN_KEYS; ++i) c[i] = *reinterpret_cast<const bf16x8_t*>(p.c + (size_t)min(base + i, hi) * p.ldc + column);
+#pragma unroll
+    for (int g = 0; g < TOKEN_KEYS / 8; ++g) {
+      kr[g] = none;
+      if (turns) kr[g] = *reinterpret_cast<const bf16x8_t*>(p.keys + (size_t)min(base + 8 * g + (lane >> 3), hi) * p.dr + turned);
+    }
+  };
+  constexpr int STEP = TOKEN_WAVES * TOKEN_KEYS, DEPTH = 4;  // groups of keys on their way
+  bf16x8_t c[DEPTH][TOKEN_KEYS], kr[DEPTH][TOKEN_KEYS / 8];
+  int base = lo + wave * TOKEN_KEYS;
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) ask(base + d * STEP, c[d], kr[d]);
+  const bf16_t* const w = v.w + (size_t)h * v.dv * v.ldc + column;
+  constexpr int AHEAD = 4;  // rows of the value matrix asked for before the first is used
+  bf16x8_t wv[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) wv[i] = *reinterpret_cast<const bf16x8_t*>(w + (size_t)min(r0 + i * TOKEN_WAVES + wave, v.dv - 1) * v.ldc);
+  float o[8], m = -1e30f, l = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = 0.0f;
+  const auto take = [&](const bf16x8_t (&c)[TOKEN_KEYS], const bf16x8_t (&kr)[TOKEN_KEYS / 8], int base) {
+    float s[TOKEN_KEYS / 8], now = m;
+#pragma unroll
+    for (int g = 0; g < TOKEN_KEYS / 8; ++g) {
+      float x[8], turn = bf16_dot(kr[g], qr);  // of the eight lanes of a key
+      turn += dpp_f32<0xB1>(turn);
+      turn += dpp_f32<0x4E>(turn);
+      turn += dpp_f32<0x141>(turn);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = live ? bf16_dot(c[8 * g + i], q) : 0.0f;
+      s[g] = (sums_of_eight(x) + turn) * p.scale;
+      if (base + 8 * g + (lane >> 3) > hi) s[g] = -1e30f;
+      now = fmaxf(now, s[g]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    now = over_eights(now, [](float a, float b) { return fmaxf(a, b); });
+    const float shrink = __expf(m - now);
+    m = now;
+    float sum = 0.0f;
+#pragma unroll
+    for (int g = 0; g < TOKEN_KEYS / 8; ++g) {
+      s[g] = base + 8 * g + (lane >> 3) > hi ? 0.0f : __expf(s[g] - now);
+      sum += s[g];
+    }
+    l = fmaf(l, shrink, over_eights(sum, [](float a, float b) { return a + b; }));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= shrink;
+#pragma unroll
+    for (int i = 0; i < TOKEN_KEYS; ++i) {
+      const float pr = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[i / 8]), i % 8 * 8));
+      const uint4_t x = __builtin_bit_cast(uint4_t, c[i]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t pair = x[e];
+        asm volatile("" : "+v"(pair));  // or the 128 values of the scores above are kept, in scratch memory
+        o[2 * e] = fmaf(pr, __builtin_bit_cast(float, pair << 16), o[2 * e]);
+        o[2 * e + 1] = fmaf(pr, __builtin_bit_cast(float, pair & 0xffff0000u), o[2 * e + 1]);
+      }
+    }
+  };
+  for (; base <= hi; base += DEPTH * STEP) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      if (base + d * STEP > hi) break;
+      take(c[d], kr[d], base + d * STEP);
+      if (base + (DEPTH + d) * STEP <= hi) ask(base + (DEPTH + d) * STEP, c[d], kr[d]);
+    }
+  }
+  if (live) {
+    *reinterpret_cast<float4_t*>(&O[wave][lane * 8]) = float4_t{o[0], o[1], o[2], o[3]};
+    *reinterpret_cast<float4_t*>(&O[wave][lane * 8 + 4]) = float4_t{o[4], o[5], o[6], o[7]};
+  }
+  if (lane == 0) {
+    ml[wave][0] = m;
+    ml[wave][1] = l;
+  }
+  __syncthreads();
+  if (tid < p.ldc) {
+    float top = sink;
+#pragma unroll
+    for (int x = 0; x < TOKEN_WAVES; ++x) top = fmaxf(top, ml[x][0]);
+    float total = v.sink ? __expf(sink - top) : 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int x = 0; x < TOKEN_WAVES; ++x) {
+      const float f = ml[x][1] > 0.0f ? __expf(ml[x][0] - top) : 0.0f;
+      total = fmaf(f, ml[x][1], total);
+      sum = fmaf(f, O[x][tid], sum);
+    }
+    O[0][tid] = sum / total;  // nobody else reads column tid
+  }
+  __syncthreads();
+  const float4_t lo4 = *reinterpret_cast<const float4_t*>(&O[0][column]), hi4 = *reinterpret_cast<const float4_t*>(&O[0][column + 4]);
+  for (int r = r0 + wave, i = 0; r < r1; r += TOKEN_WAVES * AHEAD, ++i) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int row = r + u * TOKEN_WAVES;
+      if (row >= r1) break;
+      if (i > 0) wv[u] = *reinterpret_cast<const bf16x8_t*>(w + (size_t)row * v.ldc);
+      const uint4_t x = __builtin_bit_cast(uint4_t, wv[u]);
+      float sum = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sum = fmaf(__builtin_bit_cast(float, x[e] << 16), e < 2 ? lo4[2 * e] : hi4[2 * e - 4], sum);
+        sum = fmaf(__builtin_bit_cast(float, x[e] & 0xffff0000u), e < 2 ? lo4[2 * e + 1] : hi4[2 * e - 3], sum);
+      }
+      sum = wave_sum(live ? sum : 0.0f);
+      if (v.gate) sum *= sigmoid_f32((float)v.gate[(size_t)h * v.dv + row]);
+      if (lane == 0) v.out[(size_t)h * v.dv + row] = (bf16_t)sum;
+    }
+  }
+}
+
 int check_latent(const char* who, const lcu_latent_params* p) {
   LCU_REQUIRE(p, "%s: null pointer", who);
   LCU_REQUIRE(p->heads > 0 && p->heads <= 4096 && p->dn > 0 && p->dn % 32 == 0 && p->dr >= 0 && p->dr % 32 == 0 && p->rot >= 0 &&
@@ -456,10 +649,15 @@ int lcu_latent_attention(void* out_dev, int ldo, const void* q_latent_dev, const
   float* ml = part + (size_t)slices * rows * p->ldc;
   const latent_args a{p->heads, n, p->ldc, p->dr, p->window, slices, p->scale, (const bf16_t*)q_latent_dev, (const bf16_t*)q_rot_dev, ldq,
                       p->dn + p->dr, (const bf16_t*)latents_dev, (const bf16_t*)keys_dev, (const int*)start_dev, max_positions, part, ml};
-  hipStream_t st = as_stream(stream);
-  const size_t lds = attention_lds(p->ldc, p->dr);
   const latent_value_args v{p->heads, n, p->ldc, p->dv, slices, part, ml, (const float*)sink_dev, (const bf16_t*)uv_dev,
                             (const bf16_t*)gate_dev, ldg, (bf16_t*)out_dev, ldo};
+  hipStream_t st = as_stream(stream);
+  if (n == 1 && p->dr <= 64 && std::min(p->window, max_positions) <= LATENT_TOKEN_KEYS) {
+    latent_token_kernel<<<dim3(p->heads, std::min(4, p->dv / 32)), 64 * TOKEN_WAVES, 0, st>>>(a, v);
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+  }
+  const size_t lds = attention_lds(p->ldc, p->dr);
   const auto go = [&](auto nt) -> int {
     auto kernel = latent_attention_kernel<decltype(nt)::value>;
     static bool raised[16] = {};  // per device, once

@@ -16,6 +16,7 @@ constexpr int MAX_ROWS = 2048;  // tokens of one pass: bounds the activations, n
 // Calls of at most this many tokens attend over the latents; longer ones multiply keys and values out, which
 // costs the visible keys once but makes every row's sums several times shorter.
 constexpr int FEW_ROWS = 32;
+constexpr int SHORT_CONTEXT = 512;
 
 lcu_latent_params latent_shape(latent_weights const& w, latent_params const& p) {
   return lcu_latent_params{p.heads, w.dn, w.dr, p.rot.dims, w.dv, p.kv_rank, w.ldc, p.window > 0 ? p.window : std::numeric_limits<int>::max(),
@@ -137,7 +138,7 @@ layered_context_impl::layered_context_impl(layered_model_impl* model, int contex
 layered_context_impl::~layered_context_impl() {
   lcu_sync(stream_);
   device_structure_lock lock(device_structure_mutex());
-  lcu_graph_destroy(decode_graph_);
+  for (auto& d : decode_) lcu_graph_destroy(d.graph);
   lcu_stream_destroy(stream_);
 }
 
@@ -242,7 +243,7 @@ void layered_context_impl::latent(latent_weights const& w, latent_params const& 
   if (few) {
     LCU_CHECK(lcu_latent_queries(t_latent_queries_.data(), q, ldq, w.uk_t.data(), &lp, low ? nullptr : &rows, n, stream_));
     LCU_CHECK(lcu_latent_attention(t_rec_.data(), w.ldo, t_latent_queries_.data(), q + (size_t)w.dn * m.elem, ldq, s.k.data(), s.v.data(),
-                                   start(), context_len_, values, p.sink ? w.sink.data() : nullptr, gate, w.ldw, &lp, t_scratch_.data(), n,
+                                   start(), fused ? decode_positions_ : context_len_, values, p.sink ? w.sink.data() : nullptr, gate, w.ldw, &lp, t_scratch_.data(), n,
                                    stream_));
   } else {
     // keys and values of every position the call sees
@@ -444,25 +445,30 @@ void layered_context_impl::enqueue_one() {
 void layered_context_impl::step_one() {
   device_structure_lock lock(device_structure_mutex());  // capture, instantiation, launch: see host_common.hpp
   static const bool no_graph = getenv("LLAMA_CU_NO_GRAPH") != nullptr && atoi(getenv("LLAMA_CU_NO_GRAPH")) != 0;
-  if (!decode_graph_ && ++decode_calls_ >= 2 && !no_graph) {
+  const bool few = start_pos_ < SHORT_CONTEXT;
+  decode_positions_ = few ? std::min(SHORT_CONTEXT, context_len_) : context_len_;
+  auto& d = decode_[few ? 0 : 1];
+  if (!d.graph && ++d.calls >= 2 && !no_graph) {
     LCU_CHECK(lcu_graph_begin_capture(stream_));
     enqueue_one();
-    LCU_CHECK(lcu_graph_end_capture(stream_, &decode_graph_));
+    LCU_CHECK(lcu_graph_end_capture(stream_, &d.graph));
   }
-  if (decode_graph_) {
-    LCU_CHECK(lcu_graph_launch(decode_graph_, stream_));
+  if (d.graph) {
+    LCU_CHECK(lcu_graph_launch(d.graph, stream_));
   } else {
     enqueue_one();
   }
 }
 
 void layered_context_impl::drop_graph() {
-  if (decode_graph_) {
-    device_structure_lock lock(device_structure_mutex());
-    LCU_CHECK(lcu_graph_destroy(decode_graph_));
-    decode_graph_ = nullptr;
+  for (auto& d : decode_) {
+    if (d.graph) {
+      device_structure_lock lock(device_structure_mutex());
+      LCU_CHECK(lcu_graph_destroy(d.graph));
+      d.graph = nullptr;
+    }
+    d.calls = 0;
   }
-  decode_calls_ = 0;
 }
 
 int layered_context_impl::read_residual(int layer, float* out, int rows) const {

@@ -64,8 +64,12 @@ struct layered_context_impl final : public llama_context {
   std::vector<std::vector<float>> residual_;
   bool sampling_{false};
   uint64_t sample_seed_{0}, samples_drawn_{0};
-  void* decode_graph_{nullptr};
-  int decode_calls_{0};
+  // one-token steps of up to SHORT_CONTEXT positions, for which lcu_latent_attention has a launch of its own, and of more
+  struct {
+    void* graph{nullptr};
+    int calls{0};
+  } decode_[2];
+  int decode_positions_{0};                        // what latent() says it may see in such a step
   gpu_buffer t_arrived_;                           // counters of the attention step, zero between launches
   void* stream_{nullptr};
 };

@@ -286,6 +286,19 @@ def test_attention_over_latents(gpu, shape):
         gpu.release()
 
 
+# one token: eight keys to a wavefront, eight wavefronts, four such groups asked for at once, the longest context and one key more
+# (which is the slices' again); rotated parts of 0, 32, 64 and of 96, latents of 64 to 512, 1 to 4 workgroups for the values
+@pytest.mark.parametrize("shape", [(2, 32, 64, 32, 512, None, True, True), (3, 40, 30, 70, 190, None, False, False), (2, 64, 0, 128, 64, 512, True, False),
+                                   (1, 32, 96, 200, 256, None, False, True), (4, 32, 64, 128, 450, 140, True, True)],
+                         ids=lambda s: "x".join(map(str, s[:5])))
+def test_one_token_over_latents(gpu, shape):
+    H, dim, rot, vdim, rank, window, sink, gate = shape
+    x = attention_case(H + rank, H, dim, rot, vdim, rank, 1030, window, sink, gate, far=None if window else 5)
+    for start in (0, 6, 7, 8, 62, 63, 64, 127, 128, 255, 256, 319, 320, 510, 511, 512, 513, 1029):
+        close(over_latents(gpu, x, start, 1, max(512, start + 1)), expected(x, start, 1), BF16, bf16=BF16_ATTENTION)
+        gpu.release()
+
+
 @BOTH
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s[:5])))
 def test_attention_over_keys(gpu, dt, shape):
