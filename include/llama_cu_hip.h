@@ -265,6 +265,12 @@ int lcu_batch_ffn_up(void* out_dev, void* w1_tmp_dev, void* w3_tmp_dev, const vo
                      const void* const* scales_dev, int block, int n_seq, int dim, int ffn, void* stream);
 int lcu_batch_proj_norm(void* x_dev, void* norm_out_dev, const void* lhs_dev, const void* w_dev, const void* scales_dev,
                         int block, int n_seq, int K, int dim, const void* norm_w_dev, float eps, void* stream);
+/* Wq, Wk, Wv products of a prompt's rows [rows][dim], q and k rotated at positions first_position + row (llama_cu.cu:1144-1156); k_out and
+ * v_out are the caches' rows from first_position on.  The bits of lcu_gemm_*_multi and lcu_rope_pair; the rotation goes with the
+ * product where that is one launch, or with the sums of a split one for up to 64 rows. */
+int lcu_prompt_qkv(void* q_out_dev, void* k_out_dev, void* v_out_dev, const void* lhs_dev, const void* const* w_dev,
+                   const void* const* scales_dev, int block, int rows, int dim, int n_heads, int first_position,
+                   const void* table_dev, int table_positions, void* stream);
 /* lcu_softmax_argmax on `rows` rows of n logits (n a multiple of 8): probabilities [rows][n],
  * one int32 index per row */
 int lcu_softmax_argmax_rows(void* probs_dev, void* out_index_dev, const void* logits_dev, int rows, int n, float temp,

@@ -1025,6 +1025,13 @@ int launch_columns(EP const& ep, operands_t op, const void* A, int M, int K, int
   }
 }
 
+// the columns of the last matrix that whole rounds of large tiles leave
+template <bool U8, class EP>
+int launch_rest(EP const& ep, large_tiles_t const& plan, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st) {
+  if (plan.rest_rows == 256) return launch_columns<U8>(ep, op, A, M, K, N, block, beta, st, plan.rest_columns, plan.rest);
+  return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, 4, U8, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, plan.rest);
+}
+
 template <bool U8, class EP>
 int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st) {
   device_state* ds = current_device_state();
@@ -1040,8 +1047,14 @@ int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N
   }
   const int rc = launch_columns<U8>(ep, op, A, M, K, N, block, beta, st, plan.columns, plan.first);
   if (rc != LCU_OK || plan.rest.from == 0) return rc;
-  if (plan.rest_rows == 256) return launch_columns<U8>(ep, op, A, M, K, N, block, beta, st, plan.rest_columns, plan.rest);
-  return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, 4, U8, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, plan.rest);
+  if constexpr (EP::ROTARY) {  // the last matrix, by itself
+    if (ep.matrices < op.n_mats) return launch_rest<U8>(f16_epilogue{}, plan, op, A, M, K, N, block, beta, st);
+    EP last = ep;
+    last.matrices = 1;
+    return launch_rest<U8>(last, plan, op, A, M, K, N, block, beta, st);
+  } else {
+    return launch_rest<U8>(ep, plan, op, A, M, K, N, block, beta, st);
+  }
 }
 
 // where a split-K launch left its partial sums: part[matrix][split][M][N] fp32
@@ -1329,20 +1342,34 @@ __device__ __forceinline__ float2 sum_pair(const float* __restrict__ part, size_
   return v;
 }
 
-// Wq, Wk, Wv products -> fp16 -> rotary of q (to q_out) and k at pos[b]; rotated k and v into row
-// pos[b] of sequence b's caches (what splitk_reduce_kernel + rope_store_batch_kernel do)
-__global__ __launch_bounds__(256) void reduce_rope_store_kernel(half_t* __restrict__ q_out, const float* __restrict__ part,
-                                                                int splits, int n_seq, int dim,
-                                                                half_t* const* __restrict__ k_ptrs,
-                                                                half_t* const* __restrict__ v_ptrs,
-                                                                const int* __restrict__ pos_dev, int head_dim,
-                                                                const float2* __restrict__ table, int max_pos) {
+// Wq, Wk, Wv products -> fp16 -> rotary of q (to q_out) and k.  Sequences: at pos[b], rotated k and v into row
+// pos[b] of sequence b's caches (what splitk_reduce_kernel + rope_store_batch_kernel do).  A prompt: at first + row, into the rows of k_out, v_out.
+struct sequence_rows {
+  half_t* const* __restrict__ k_ptrs;
+  half_t* const* __restrict__ v_ptrs;
+  const int* __restrict__ pos_dev;
+  int max_pos;
+  __device__ __forceinline__ int position(int b) const { return min(max(pos_dev[b], 0), max_pos); }
+  __device__ __forceinline__ half_t* k(int b, int pos, int dim) const { return k_ptrs[b] + (size_t)pos * dim; }
+  __device__ __forceinline__ half_t* v(int b, int pos, int dim) const { return v_ptrs[b] + (size_t)pos * dim; }
+};
+struct prompt_rows {
+  half_t* k_out;
+  half_t* v_out;
+  int first;
+  __device__ __forceinline__ int position(int row) const { return first + row; }
+  __device__ __forceinline__ half_t* k(int row, int, int dim) const { return k_out + (size_t)row * dim; }
+  __device__ __forceinline__ half_t* v(int row, int, int dim) const { return v_out + (size_t)row * dim; }
+};
+template <class ROWS>
+__global__ __launch_bounds__(256) void reduce_rope_store_kernel(half_t* __restrict__ q_out, const float* __restrict__ part, int splits, int n_seq,
+                                                                int dim, ROWS rows, int head_dim, const float2* __restrict__ table) {
   const int pair = blockIdx.x * 256 + threadIdx.x;
   const int b = blockIdx.y;
   if (pair * 2 >= dim) return;
   const int c = pair * 2;
   const size_t mn = (size_t)n_seq * dim, at = (size_t)b * dim + c;
-  const int pos = min(max(pos_dev[b], 0), max_pos);
+  const int pos = rows.position(b);
   const float2 cs = table[(size_t)pos * (head_dim / 2) + (c % head_dim) / 2];
   const float2 qf = sum_pair(part, at, mn, splits);
   const float2 kf = sum_pair(part + (size_t)splits * mn, at, mn, splits);
@@ -1354,13 +1381,12 @@ __global__ __launch_bounds__(256) void reduce_rope_store_kernel(half_t* __restri
   w.x = round_f16(fmaf(qr, cs.x, -(qi * cs.y)));
   w.y = round_f16(fmaf(qr, cs.y, qi * cs.x));
   *reinterpret_cast<half2_t*>(q_out + at) = w;
-  const size_t dst = (size_t)pos * dim + c;
   w.x = round_f16(fmaf(kr, cs.x, -(ki * cs.y)));
   w.y = round_f16(fmaf(kr, cs.y, ki * cs.x));
-  *reinterpret_cast<half2_t*>(k_ptrs[b] + dst) = w;
+  *reinterpret_cast<half2_t*>(rows.k(b, pos, dim) + c) = w;
   w.x = round_f16(vf.x);
   w.y = round_f16(vf.y);
-  *reinterpret_cast<half2_t*>(v_ptrs[b] + dst) = w;
+  *reinterpret_cast<half2_t*>(rows.v(b, pos, dim) + c) = w;
 }
 
 // W1, W3 products -> fp16 each -> fp16(silu(w1) * w3)  (1180-1183, 533-539)
@@ -1507,8 +1533,10 @@ int launch_gemm(half_t* out, const half_t* A, const void* W, const half_t* S, in
   return launch_one<BM, BN, U8, true, KS>(out, A, W, S, M, K, N, block, beta, tiles_m, tiles_n, st);
 }
 
+// rotary: rotates the outputs where the product takes gemm_tile_kernel without a split; *rotated then says so.
 template <bool U8>
-int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st) {
+int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st,
+                  const rotary_epilogue* rotary = nullptr, bool* rotated = nullptr) {
   // Tile choice.  Large tiles read fewer operand bytes per multiply-add and pay per output for fewer
   // barriers.  So: tiles of 256 rows when those of 256x128 still give 160 workgroups, or with few of them
   // and a long K the splits of each (large_tile_splits); 128x128 when these give 160; 128x64 with four
@@ -1566,6 +1594,10 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
           return launch_dl<256, 128, 4, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
         }
       }
+      if (rotary && N % 8 == 0) {
+        *rotated = true;
+        return launch_large<U8>(*rotary, op, A, M, K, N, block, beta, st);
+      }
       return launch_large<U8>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
     }
     {
@@ -1598,7 +1630,13 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         // more tiles than compute units, which the register-staged kernel puts two to a compute unit, 1000 rows of 4608 columns
         // 11.4 / 14.0, 15.8 / 17.8, 24.5 / 25.6, 41.9 / 41.6
         const bool long_enough = tiles128 < 256 ? K >= 384 : tiles128 / nm <= 256 || K >= 1536;
-        if (block_shift(block) >= 0 && long_enough) return launch_tile<128, 128, 1, 4, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        if (block_shift(block) >= 0 && long_enough) {
+          if (rotary && N % 8 == 0) {
+            *rotated = true;
+            return launch_tile<128, 128, 1, 4, 4, 4, true, false>(*rotary, op, A, M, K, N, block, beta, st);
+          }
+          return launch_tile<128, 128, 1, 4, 4, 4, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        }
         if (tiles128 < 256) return launch_dl<128, 128, 4, 2, 1, 3, true>(op, A, M, K, N, block, beta, st);
       } else {
         // us, K 256, 512, 1024, 1536, 2048: eight wavefronts / here, 512 rows of 5120 columns 6.2 / 7.1, 7.8 / 8.5, 10.9 / 11.2, 16.1 / 15.2, 22.0 / 22.3;
@@ -1607,6 +1645,10 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         // with weights from memory the second workgroup also hides the second round's first requests: K 1280, 1536, 1792, 512 rows of
         // 10000 columns 30.3 / 34.4, 34.2 / 38.2, 38.9 / 42.0, 896 rows of 4992 26.6 / 28.3, 30.4 / 31.0, 34.6 / 34.1
         if (K < 1536 && tiles128 > 256) return launch_dl<128, 128, 2, 2, 1, 2, false>(op, A, M, K, N, block, beta, st);
+        if (rotary && N % 8 == 0) {
+          *rotated = true;
+          return launch_tile<128, 128, 2, 2, 4, 4, false, false>(*rotary, op, A, M, K, N, 0, beta, st);
+        }
         return launch_tile<128, 128, 2, 2, 4, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
       }
     } else {
@@ -1888,10 +1930,9 @@ int lcu_batch_qkv(void* q_out_dev, void* k_tmp_dev, void* v_tmp_dev, const void*
     if (rc != LCU_OK) return rc;
   }
   if (done) {
-    reduce_rope_store_kernel<<<dim3((dim / 2 + 255) / 256, n_seq), 256, 0, st>>>(
-        (half_t*)q_out_dev, ps.part, ps.splits, n_seq, dim, (half_t* const*)k_cache_ptrs_dev,
-        (half_t* const*)v_cache_ptrs_dev, (const int*)pos_dev, dim / n_heads, (const float2*)table_dev,
-        table_positions - 1);
+    const sequence_rows rows{(half_t* const*)k_cache_ptrs_dev, (half_t* const*)v_cache_ptrs_dev, (const int*)pos_dev, table_positions - 1};
+    reduce_rope_store_kernel<<<dim3((dim / 2 + 255) / 256, n_seq), 256, 0, st>>>((half_t*)q_out_dev, ps.part, ps.splits, n_seq, dim, rows,
+                                                                                 dim / n_heads, (const float2*)table_dev);
     LCU_LAUNCH_CHECK();
     return LCU_OK;
   }
@@ -1901,6 +1942,47 @@ int lcu_batch_qkv(void* q_out_dev, void* k_tmp_dev, void* v_tmp_dev, const void*
   if (rc != LCU_OK) return rc;
   return lcu_rope_store_batch(q_out_dev, k_tmp_dev, v_tmp_dev, k_cache_ptrs_dev, v_cache_ptrs_dev, pos_dev, n_seq, dim,
                               n_heads, table_dev, table_positions, stream);
+}
+
+int lcu_prompt_qkv(void* q_out_dev, void* k_out_dev, void* v_out_dev, const void* lhs_dev, const void* const* w_dev, const void* const* scales_dev,
+                   int block, int rows, int dim, int n_heads, int first_position, const void* table_dev, int table_positions, void* stream) {
+  LCU_REQUIRE(q_out_dev && k_out_dev && v_out_dev && lhs_dev && w_dev && w_dev[0] && w_dev[1] && w_dev[2] && table_dev, "lcu_prompt_qkv: null pointer");
+  LCU_REQUIRE(rows >= 0 && rows <= 65535 && dim > 0 && n_heads > 0 && dim % n_heads == 0 && (dim / n_heads) % 2 == 0 && dim % 16 == 0,
+              "lcu_prompt_qkv: bad shape rows %d dim %d heads %d", rows, dim, n_heads);
+  LCU_REQUIRE(first_position >= 0 && first_position + rows <= table_positions, "lcu_prompt_qkv: positions %d..%d outside the table of %d",
+              first_position, first_position + rows, table_positions);
+  LCU_REQUIRE(block == 0 || (scales_dev && scales_dev[0] && scales_dev[1] && scales_dev[2] && block % 16 == 0 && dim % block == 0),
+              "lcu_prompt_qkv: quantised weights need scales and a block dividing dim");
+  LCU_REQUIRE((size_t)rows * dim * 2 < ((size_t)1 << 32) && (size_t)dim * dim * (block ? 1 : 2) < ((size_t)1 << 32),
+              "lcu_prompt_qkv: operands of 4 GiB or more are not supported");
+  if (rows == 0) return LCU_OK;
+  hipStream_t st = as_stream(stream);
+  void* const outs[3] = {q_out_dev, k_out_dev, v_out_dev};
+  const half_t* lhs = (const half_t*)lhs_dev;
+  const int head_dim = dim / n_heads;
+  bool done = false;
+  if (rows > 1) {
+    const operands_t op = make_operands(outs, w_dev, block ? scales_dev : nullptr, 3);
+    partial_sums_t ps{};
+    int rc = block ? skinny_partial<true>(op, lhs, rows, dim, dim, block, st, &done, &ps) : skinny_partial<false>(op, lhs, rows, dim, dim, 0, st, &done, &ps);
+    if (rc != LCU_OK) return rc;
+    if (done) {
+      const prompt_rows to{(half_t*)k_out_dev, (half_t*)v_out_dev, first_position};
+      reduce_rope_store_kernel<<<dim3((dim / 2 + 255) / 256, rows), 256, 0, st>>>((half_t*)q_out_dev, ps.part, ps.splits, rows, dim, to, head_dim,
+                                                                                  (const float2*)table_dev);
+      LCU_LAUNCH_CHECK();
+      return LCU_OK;
+    }
+    const rotary_epilogue turn{(const float2*)table_dev, head_dim, first_position, 2};
+    const rotary_epilogue* rotary = head_dim % 8 == 0 && (reinterpret_cast<uintptr_t>(table_dev) & 15) == 0 ? &turn : nullptr;
+    rc = block ? dispatch_gemm<true>(op, lhs, rows, dim, dim, block, 0.0f, st, rotary, &done) : dispatch_gemm<false>(op, lhs, rows, dim, dim, 0, 0.0f, st, rotary, &done);
+    if (rc != LCU_OK) return rc;
+  } else {
+    const int rc = block ? lcu_gemm_f16u8_nt_multi(outs, lhs_dev, w_dev, scales_dev, 3, rows, dim, dim, block, 0.0f, stream)
+                         : lcu_gemm_f16_nt_multi(outs, lhs_dev, w_dev, 3, rows, dim, dim, 0.0f, stream);
+    if (rc != LCU_OK) return rc;
+  }
+  return done ? LCU_OK : lcu_rope_pair(q_out_dev, k_out_dev, rows, dim, n_heads, first_position, table_dev, table_positions, stream);
 }
 
 int lcu_batch_ffn_up(void* out_dev, void* w1_tmp_dev, void* w3_tmp_dev, const void* lhs_dev, const void* const* w_dev,

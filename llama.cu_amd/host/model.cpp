@@ -340,24 +340,6 @@ void llama_context_impl::matmul_norm(void* x, const void* lhs, weight_tensor con
                                 norm.data(), model_->params.norm_eps, stream_));
 }
 
-// products of one lhs with several weight matrices of one shape (Wq, Wk, Wv; W1, W3) in one launch
-void llama_context_impl::matmul_multi(void* const* outs, const void* lhs, weight_tensor const* const* ws, int count,
-                                      int M) {
-  const void* values[3];
-  const void* scales[3];
-  for (int g = 0; g < count; ++g) {
-    values[g] = ws[g]->data.data();
-    scales[g] = ws[g]->scales.data();
-  }
-  weight_tensor const& w = *ws[0];
-  if (w.quantised) {
-    LCU_CHECK(lcu_gemm_f16u8_nt_multi(outs, lhs, values, scales, count, M, (int)w.cols, (int)w.rows, w.block, 0.0f,
-                                      stream_));
-  } else {
-    LCU_CHECK(lcu_gemm_f16_nt_multi(outs, lhs, values, count, M, (int)w.cols, (int)w.rows, 0.0f, stream_));
-  }
-}
-
 // The layer loop for n new rows sitting in t_embed_; positions start_pos_ .. start_pos_ + n - 1.
 // n == 1 takes the fused decode kernels, which read the position from t_step_ on the device.
 void llama_context_impl::enqueue_layers(int n, bool first_norm_ready) {
@@ -403,10 +385,10 @@ void llama_context_impl::enqueue_layers(int n, bool first_norm_ready) {
       char* v_new = vc + (size_t)sp * dim * 2;
       if (!norm_ready) LCU_CHECK(lcu_rmsnorm(t_norm_.data(), x, L.attn_norm.data(), n, dim, p.norm_eps, stream_));  // 1129
       norm_ready = false;
-      void* const qkv_out[3] = {t_xq_.data(), k_new, v_new};
-      weight_tensor const* const qkv_w[3] = {&L.wq, &L.wk, &L.wv};
-      matmul_multi(qkv_out, t_norm_.data(), qkv_w, 3, n);                                                    // 1144, 1150, 1156
-      LCU_CHECK(lcu_rope_pair(t_xq_.data(), k_new, n, dim, heads, sp, rope_table_, context_len_, stream_));  // 1146, 1152 (new rows only)
+      const void* const qkv_w[3] = {L.wq.data.data(), L.wk.data.data(), L.wv.data.data()};
+      const void* const qkv_s[3] = {L.wq.scales.data(), L.wk.scales.data(), L.wv.scales.data()};
+      LCU_CHECK(lcu_prompt_qkv(t_xq_.data(), k_new, v_new, t_norm_.data(), qkv_w, qkv_s, L.wq.quantised ? L.wq.block : 0, n, dim, heads, sp,
+                               rope_table_, context_len_, stream_));                                         // 1144-1156 (new rows only)
       LCU_CHECK(lcu_attention(t_out_.data(), t_xq_.data(), kc, vc, n, T, sp, dim, heads, stream_));          // 1161-1171
     }
     if (n == 1 && hand_overs_ && !fused_wo && dim <= 8192) {

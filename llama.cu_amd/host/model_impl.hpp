@@ -81,7 +81,6 @@ struct llama_context_impl final : public llama_context {
   void enqueue_logits(int row);
   void matmul(void* out, const void* lhs, weight_tensor const& w, int M, float beta);
   void matmul_norm(void* x, const void* lhs, weight_tensor const& w, int M, gpu_buffer const& norm);
-  void matmul_multi(void* const* outs, const void* lhs, weight_tensor const* const* ws, int count, int M);
   void enqueue_layers(int n, bool first_norm_ready = false);
   void enqueue_head(int n);
   void drop_graph();

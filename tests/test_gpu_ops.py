@@ -1286,3 +1286,33 @@ def test_product_residual_norm_of_many_rows(gpu, M, K, N, block):
     assert (G.host(xa, (M, N)).view(np.uint16) == G.host(xb, (M, N)).view(np.uint16)).all()
     assert (G.host(na, (M, N)).view(np.uint16) == G.host(nb, (M, N)).view(np.uint16)).all()
     G.release()
+
+
+# split sums of few rows (two kernels), tiles of 128 and 256 rows, columns left of whole rounds, ragged rows; kernels without a rotation of their
+# own (half stages apart, K no whole number of stages, blocks of 96 codes), one row
+@pytest.mark.parametrize("rows,dim,heads,first,block", [(24, 512, 4, 0, 0), (45, 4096, 32, 7, 0), (64, 1024, 8, 3, 128), (512, 4096, 32, 0, 0), (301, 4096, 32, 100, 0),
+                                                        (700, 2048, 16, 9, 0), (1000, 4096, 32, 20, 0), (512, 6656, 52, 0, 128), (1500, 6656, 52, 11, 128),
+                                                        (1500, 5120, 40, 0, 0), (200, 4096, 32, 1, 128), (100, 4096, 32, 5, 0), (90, 320, 2, 4, 0),
+                                                        (300, 1152, 9, 2, 96), (1, 512, 4, 6, 0), (260, 3200, 100, 2, 128)])
+def test_prompt_qkv(gpu, rows, dim, heads, first, block):
+    """lcu_prompt_qkv against the products and lcu_rope_pair, bit for bit."""
+    G = gpu
+    check, L, VP = G.B.check, G.L(), G.B.vp
+    table = VP()
+    check(L.lcu_rope_table_create(G.B.C.byref(table), first + rows, dim // heads, 10000.0))
+    x, ws = G.dev_keep(normal((rows, dim), 0, 1900, 1.0)), [normal((dim, dim), 0, 1901 + g, 0.02) for g in range(3)]
+    wd = [[G.dev_keep(part) for part in (O.quantize_absmax_u8(w, block) if block else (w,))] for w in ws]
+    w_arr, s_arr = (VP * 3)(*[w[0].ptr for w in wd]), (VP * 3)(*[w[1].ptr for w in wd]) if block else None
+    outs, seps = [G.empty((rows, dim)) for _ in range(3)], [G.empty((rows, dim)) for _ in range(3)]
+    check(L.lcu_prompt_qkv(outs[0].ptr, outs[1].ptr, outs[2].ptr, x.ptr, w_arr, s_arr, block, rows, dim, heads, first, table, first + rows, None))
+    arr = (VP * 3)(*[o.ptr for o in seps])
+    if block:
+        check(L.lcu_gemm_f16u8_nt_multi(arr, x.ptr, w_arr, s_arr, 3, rows, dim, dim, block, 0.0, None))
+    else:
+        check(L.lcu_gemm_f16_nt_multi(arr, x.ptr, w_arr, 3, rows, dim, dim, 0.0, None))
+    check(L.lcu_rope_pair(seps[0].ptr, seps[1].ptr, rows, dim, heads, first, table, first + rows, None))
+    for a, b in zip(outs, seps):
+        assert (G.host(a, (rows, dim)).view(np.uint16) == G.host(b, (rows, dim)).view(np.uint16)).all()
+    assert L.lcu_prompt_qkv(outs[0].ptr, outs[1].ptr, outs[2].ptr, x.ptr, w_arr, s_arr, block, rows, dim, heads, first + 1, table, first + rows, None) == -2
+    G.release()
+    L.lcu_free(table)
