@@ -16,6 +16,7 @@
 // v_mfma_f32_16x16x32_f16 into an LDS score strip [rows][T], softmax in LDS, P.V by MFMA with V
 // staged row-major in LDS; the next 64-row chunk of K or V is in flight while the current one is
 // multiplied.
+#include <type_traits>
 #include <atomic>
 
 #include "common.hpp"
@@ -853,21 +854,24 @@ int launch_decode_attention(half_t* out, const half_t* q, const half_t* k, const
 // ---------------------------------------------------------------------------------------------
 constexpr int CW = 64;         // cache rows per staged chunk
 constexpr int QLD = HD + 8;    // LDS row stride (halves) of the Q and K tiles
-constexpr int MAX_T_PREFILL = 4096;    // 16-row tiles: a strip of 16 x 4096 fp16 scores fits LDS; 32-row tiles reach 2048
-constexpr int MAX_T_PREFILL_32 = 2048;
+constexpr int VLD = HD + 16;   // and of V chunks
+// four halves of a column; see prefill_attention_kernel
+__device__ __forceinline__ half4_t read_transposed(const half_t* at) {
+  typedef short short4_t __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)at));
+}
+constexpr int BR = 16;                 // query rows per workgroup
+constexpr int MAX_T_PREFILL = 4096;    // a strip of 16 x 4096 fp16 scores fits LDS
 
-// BR: query rows per workgroup (16 or 32)
 // LDS row of position p of a V chunk (a permutation inside every block of 32 positions)
 __device__ __forceinline__ int v_row(int p) {
   const int e = p & 7, g = (p >> 3) & 3;
   return (p & ~31) + 4 * g + (e & 3) + 16 * (e >> 2);
 }
 
-template <int BR>
 __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restrict__ out, const half_t* __restrict__ q,
                                                                 const half_t* __restrict__ k, const half_t* __restrict__ v,
                                                                 int n_new, int T, int start_pos, int dim, int n_tiles) {
-  constexpr int RT = BR / 16;  // 16-row matrix-instruction tiles per workgroup
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // Heaviest work first over the whole grid (a later row tile has the longer causal span): the
   // heads' last tiles, then their second-to-last ones, and so on, so that compute units pick up
@@ -884,8 +888,8 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   const int SLD = Tc + 8;
 
   half_t* Qs = reinterpret_cast<half_t*>(smem);             // [BR][QLD]
-  half_t* KVs = Qs + BR * QLD;                              // K or V chunk [CW][QLD]
-  half_t* Ss = KVs + CW * QLD;                              // [BR][SLD]
+  half_t* KVs = Qs + BR * QLD;                              // K chunk [CW][QLD] or V chunk [CW][VLD]
+  half_t* Ss = KVs + CW * VLD;                              // [BR][SLD]
 
   // Q tile
   for (int c = tid; c < BR * HD / 8; c += 256) {
@@ -896,7 +900,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
     *reinterpret_cast<half8_t*>(&Qs[row * QLD + col]) = val;
   }
 
-  const float denom = sqrtf((float)HD);
+  const float denom = sqrtf((float)HD), inverse = 1.0f / denom;
   const int frow = lane & 15, fk = (lane >> 4) * 8;
   // A chunk of 64 cache rows is 64 x 128 halves = 4 x 16 bytes per thread.  The next chunk is
   // requested into registers before the current one is multiplied, so its latency hides behind
@@ -918,7 +922,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
       const int c = tid + i * 256;
       const int p = c >> 4;
       const int row = permute_rows ? v_row(p) : p;
-      *reinterpret_cast<half8_t*>(&KVs[row * QLD + (c & 15) * 8]) = reg[i];
+      *reinterpret_cast<half8_t*>(&KVs[row * (permute_rows ? VLD : QLD) + (c & 15) * 8]) = reg[i];
     }
   };
 
@@ -951,105 +955,142 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   // ---- scores: S[BR][Tc] = Q . K^T, wave w owns the 16 columns w*16.. of every 64-column chunk
   prefetch_first(k);
   for_chunks(k, [&](int c0) {
-    float4_t acc[RT];
-#pragma unroll
-    for (int i = 0; i < RT; ++i) acc[i] = (float4_t)(0.0f);
+    float4_t acc = (float4_t)(0.0f);
 #pragma unroll
     for (int ks = 0; ks < HD; ks += 32) {
       const half8_t fb = *reinterpret_cast<const half8_t*>(&KVs[(wave * 16 + frow) * QLD + ks + fk]);
-#pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        const half8_t fa = *reinterpret_cast<const half8_t*>(&Qs[(i * 16 + frow) * QLD + ks + fk]);
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb, acc[i], 0, 0, 0);
-      }
+      const half8_t fa = *reinterpret_cast<const half8_t*>(&Qs[frow * QLD + ks + fk]);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb, acc, 0, 0, 0);
     }
     // accumulator register e of lane l is (row 4*(l/16) + e, column l%16)
     const int col = c0 + wave * 16 + (lane & 15);
+    float size = 0.0f;
 #pragma unroll
-    for (int i = 0; i < RT; ++i) {
+    for (int e = 0; e < 4; ++e) size = fmaxf(size, fabsf(acc[e]));
+    const bool plain = __ballot(size > 3.402823466e38f) == 0;  // infinite products are divided the long way (divide_by)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = i * 16 + (lane >> 4) * 4 + e;
-        const bool masked = col > r0 + row + start_pos || col >= T;  // llama_cu.cu:415
-        Ss[row * SLD + col] = masked ? (half_t)(-INFINITY) : round_f16(acc[i][e] / denom);
-      }
+    for (int e = 0; e < 4; ++e) {
+      const int row = (lane >> 4) * 4 + e;
+      const bool masked = col > r0 + row + start_pos || col >= T;  // llama_cu.cu:415
+      acc[e] = plain ? divide_by(acc[e], denom, inverse) : acc[e] / denom;
+      Ss[row * SLD + col] = masked ? (half_t)(-INFINITY) : round_f16(acc[e]);
     }
   });
   // the first V chunks travel while the softmax runs
   prefetch_first(v);
   __syncthreads();
 
-  // ---- softmax over each row of the strip (llama_cu.cu:433-499): wave w owns rows w*8 .. w*8+7;
-  // exp_ieee and a true division, as in every other softmax here
-  for (int rr = 0; rr < BR / 4; ++rr) {
-    // two neighbouring scores per lane and access (4 bytes: whole LDS words)
-    half2_t* srow = reinterpret_cast<half2_t*>(Ss + (wave * (BR / 4) + rr) * SLD);
-    const int pairs = Tc / 2;
-    float m = -INFINITY;
-    for (int i = lane; i < pairs; i += WAVE) {
-      const half2_t v = srow[i];
-      m = fmaxf(m, fmaxf((float)v.x, (float)v.y));
+  // ---- softmax over each row of the strip (llama_cu.cu:433-499): wave w owns rows w * BR / 4 on, two at a time; the bits of
+  // exp_ieee and a true division, as in every other softmax here.  Vector instructions are what it takes: up to 1024 columns a lane
+  // keeps its pairs of neighbouring scores and takes each exponential once (32 heads, n = T = 512: 25.5 us with exponentials twice and
+  // general divisions, 19.8 so, 17.8 with V turned on its way out of LDS below).
+  const int pairs = Tc / 2;
+  const auto softmax = [&](auto most) {
+    constexpr int NP = decltype(most)::value;
+#pragma unroll 1
+    for (int rr = 0; rr < BR / 4; rr += 2) {
+      half2_t* row[2];
+      float2 x[2][NP];
+      float m[2] = {-INFINITY, -INFINITY}, sum[2] = {0.0f, 0.0f};
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        row[r] = reinterpret_cast<half2_t*>(Ss + (wave * (BR / 4) + rr + r) * SLD);
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+          x[r][j] = make_float2(-INFINITY, -INFINITY);
+          if (j * WAVE + lane < pairs) {
+            const half2_t v = row[r][j * WAVE + lane];
+            x[r][j] = make_float2((float)v.x, (float)v.y);
+          }
+          m[r] = fmaxf(m[r], fmaxf(x[r][j].x, x[r][j].y));
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        m[r] = wave_max_dpp(m[r]);
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+          x[r][j].x = exp_ieee_nonpositive(x[r][j].x - m[r]);
+          x[r][j].y = exp_ieee_nonpositive(x[r][j].y - m[r]);
+          if (j * WAVE + lane < pairs) sum[r] += x[r][j].x + x[r][j].y;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const float total = wave_sum(sum[r]), share = 1.0f / total;
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+          half2_t p;
+          p.x = round_f16(divide_by(x[r][j].x, total, share));
+          p.y = round_f16(divide_by(x[r][j].y, total, share));
+          if (j * WAVE + lane < pairs) row[r][j * WAVE + lane] = p;
+        }
+      }
     }
-    m = wave_max(m);
-    float s = 0.0f;
-    for (int i = lane; i < pairs; i += WAVE) {
-      const half2_t v = srow[i];
-      s += exp_ieee((float)v.x - m) + exp_ieee((float)v.y - m);
-    }
-    s = wave_sum(s);
-    for (int i = lane; i < pairs; i += WAVE) {
-      const half2_t v = srow[i];
-      half2_t p;
-      p.x = round_f16(exp_ieee((float)v.x - m) / s);
-      p.y = round_f16(exp_ieee((float)v.y - m) / s);
-      srow[i] = p;
+  };
+  if (pairs <= 2 * WAVE) {
+    softmax(std::integral_constant<int, 2>{});
+  } else if (pairs <= 4 * WAVE) {
+    softmax(std::integral_constant<int, 4>{});
+  } else if (pairs <= 8 * WAVE) {
+    softmax(std::integral_constant<int, 8>{});
+  } else {
+    for (int rr = 0; rr < BR / 4; ++rr) {
+      half2_t* srow = reinterpret_cast<half2_t*>(Ss + (wave * (BR / 4) + rr) * SLD);
+      float m = -INFINITY;
+      for (int i = lane; i < pairs; i += WAVE) {
+        const half2_t v = srow[i];
+        m = fmaxf(m, fmaxf((float)v.x, (float)v.y));
+      }
+      m = wave_max_dpp(m);
+      float s = 0.0f;
+      for (int i = lane; i < pairs; i += WAVE) {
+        const half2_t v = srow[i];
+        s += exp_ieee_nonpositive((float)v.x - m) + exp_ieee_nonpositive((float)v.y - m);
+      }
+      s = wave_sum(s);
+      const float share = 1.0f / s;
+      for (int i = lane; i < pairs; i += WAVE) {
+        const half2_t v = srow[i];
+        half2_t p;
+        p.x = round_f16(divide_by(exp_ieee_nonpositive((float)v.x - m), s, share));
+        p.y = round_f16(divide_by(exp_ieee_nonpositive((float)v.y - m), s, share));
+        srow[i] = p;
+      }
     }
   }
 
   // ---- out[BR][HD] = P . V: wave w owns output columns w*32 .. w*32+31 (two 16-wide tiles)
-  float4_t o[RT][2];
-#pragma unroll
-  for (int i = 0; i < RT; ++i) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) o[i][j] = (float4_t)(0.0f);
-  }
+  float4_t o[2] = {(float4_t)(0.0f), (float4_t)(0.0f)};
   // V chunks stay row-major in LDS, KVs[pos][d] (16-byte stores without bank conflicts); the
-  // matrix instruction wants 8 consecutive positions of one output column per lane, which are
-  // gathered with 2-byte reads: the 16 lanes of a fragment row group read 16 neighbouring columns
-  // (32 bytes), the four groups rows 8 positions apart.  A row is 272 bytes, so 8 rows apart is
-  // 128 bytes modulo the 256 bytes of the banks and groups 0 and 2 (1 and 3) would meet in the same
-  // banks; v_row() places position 8g + e of a 32-row block at row 4g + e % 4 + 16 (e / 4), which
-  // puts the four groups 64 bytes apart.
+  // matrix instruction wants 8 consecutive positions of one output column per lane.  ds_read_b64_tr_b16 turns them: of each sixteen
+  // lanes, lane l names 4 neighbouring columns of row l / 4, and lane c gets column c of the four rows (eight 2-byte reads to a fragment and
+  // their packing took 2 us more, n = T = 512).  Thirty-two lanes read eight rows of 32 bytes together: v_row() places positions 8g + e, e < 4, at
+  // rows 4g + e and e >= 4 sixteen rows on, and rows of 288 bytes put eight neighbouring ones in all banks.
   permute_rows = true;
+  const int v_at = (lane >> 4) * 4 + ((lane & 15) >> 2), v_col = wave * 32 + (lane & 3) * 4;
   for_chunks(v, [&](int c0) {
 #pragma unroll
     for (int ks = 0; ks < CW; ks += 32) {
-      half8_t fa[RT], fb[2];
-#pragma unroll
-      for (int i = 0; i < RT; ++i) fa[i] = *reinterpret_cast<const half8_t*>(&Ss[(i * 16 + frow) * SLD + c0 + ks + fk]);
+      const half8_t fa = *reinterpret_cast<const half8_t*>(&Ss[frow * SLD + c0 + ks + fk]);
+      half8_t fb[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const half_t* vcol = &KVs[(ks + fk / 2) * QLD + wave * 32 + j * 16 + frow];  // v_row(ks + fk + e) below
-#pragma unroll
-        for (int e = 0; e < 8; ++e) fb[j][e] = vcol[((e & 3) + 16 * (e >> 2)) * QLD];
+        const half_t* at = &KVs[(ks + v_at) * VLD + v_col + j * 16];
+        const half4_t lo = read_transposed(at), hi = read_transposed(at + 16 * VLD);
+        fb[j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       }
 #pragma unroll
-      for (int i = 0; i < RT; ++i) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) o[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[i], fb[j], o[i][j], 0, 0, 0);
-      }
+      for (int j = 0; j < 2; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb[j], o[j], 0, 0, 0);
     }
   });
 #pragma unroll
-  for (int i = 0; i < RT; ++i) {
+  for (int j = 0; j < 2; ++j) {
+    const int col = h * HD + wave * 32 + j * 16 + (lane & 15);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = h * HD + wave * 32 + j * 16 + (lane & 15);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int gr = r0 + i * 16 + (lane >> 4) * 4 + e;
-        if (gr < n_new) out[(size_t)gr * dim + col] = round_f16(o[i][j][e]);  // llama_cu.cu:529
-      }
+    for (int e = 0; e < 4; ++e) {
+      const int gr = r0 + (lane >> 4) * 4 + e;
+      if (gr < n_new) out[(size_t)gr * dim + col] = round_f16(o[j][e]);  // llama_cu.cu:529
     }
   }
 }
@@ -1311,10 +1352,7 @@ constexpr int STATIC_MAX_DEVICES = 16;
 static __device__ __align__(256) half_t scratch[MAX_HEADS * MAX_T_DECODE];
 static half_t* scratch_dev[STATIC_MAX_DEVICES] = {};
 
-size_t prefill_lds_bytes(int BR, int Tc) {
-  const size_t kv = (size_t)CW * QLD;
-  return ((size_t)BR * QLD + kv + (size_t)BR * (Tc + 8)) * sizeof(half_t);
-}
+size_t prefill_lds_bytes(int Tc) { return ((size_t)BR * QLD + (size_t)CW * VLD + (size_t)BR * (Tc + 8)) * sizeof(half_t); }
 
 }  // namespace
 
@@ -1367,14 +1405,16 @@ int lcu_attention(void* out_dev, const void* q_dev, const void* k_dev, const voi
   }
   LCU_REQUIRE(T <= MAX_T_PREFILL, "lcu_attention: T %d exceeds %d for n_new > 1", T, MAX_T_PREFILL);
   // Many scores: the kernel that computes them three times and stores none.  A wavefront of it walks all T columns
-  // alone, 3.75 us per 64 of them, while the kernel below shares a tile's columns among four wavefronts but is bound by
-  // what LDS holds from about 0.17 M scores per us on; the lines cross where the call has 11 000 scores per column
-  // (heads, n = T, us here against below: 32 heads 512 rows 35 / 25, 700 rows 46 / 47, 1024 rows 67 / 143, 1987 rows 155 / 502;
-  // 52 heads 512 rows 35 / 37; 4 heads 1500 rows 89 / 90; 32 heads 64 rows of 1000 62 / 38, 512 rows of 2048 122 / 214).
+  // alone, 4.1 us per 64 of them, while the kernel below shares a tile's columns among four wavefronts but does 0.23 M scores per us, and
+  // 0.15 M where LDS holds one strip only; the lines cross where the call has 17 000 and 9000 scores per column
+  // (heads, n = T, us here against below: 32 heads 512 rows 35 / 18, 800 rows 55 / 40, 1024 rows 70 / 69, 1200 rows 83 / 97, 1987 rows 167 / 433;
+  // 52 heads 600 rows 45 / 41, 700 rows 51 / 50, 900 rows 71 / 78; 16 heads 1500 rows 97 / 78, 2000 rows 129 / 223; 4 heads 2000 rows 117 / 62;
+  // 32 heads 512 rows of 1500 97 / 85, of 2048 129 / 202, 128 rows of 2000 120 / 58).
   // Its requests and stores are of 16 and 8 bytes: operands that are not so aligned stay with the kernel below.
   const double scores = (double)n_heads * n_new * (start_pos + 0.5 * n_new);
   const bool aligned = (((uintptr_t)q_dev | (uintptr_t)k_dev | (uintptr_t)v_dev) & 15) == 0 && ((uintptr_t)out_dev & 7) == 0;
-  if (scores >= 11000.0 * T && aligned) {
+  const size_t lds = prefill_lds_bytes((T + CW - 1) / CW * CW);
+  if (scores >= (2 * lds <= 160 * 1024 ? 17000.0 : 9000.0) * T && aligned) {
     // 128 rows to a workgroup read K and V half as often, if two workgroups per compute unit are left
     if ((long)((n_new + 127) / 128) * n_heads >= 512) {
       return launch_prompt_attention<8>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T,
@@ -1383,33 +1423,18 @@ int lcu_attention(void* out_dev, const void* q_dev, const void* k_dev, const voi
     return launch_prompt_attention<4>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T,
                                       start_pos, dim, n_heads, s);
   }
-  // 16-row tiles when 32-row tiles would leave the grid under four workgroups per compute unit
-  // and the rows are short (T <= 1024: 22 us against 29 us at n = T = 512, dim 4096); with long
-  // rows the per-chunk overhead of the extra workgroups costs more than the balance gains.
-  const long wgs32 = (long)((n_new + 31) / 32) * n_heads;
-  const int BR = ((wgs32 < 1024 && T <= 1024) || T > MAX_T_PREFILL_32) ? 16 : 32;
+  // (tiles of 32 rows, which read K and V half as often: 52 heads 600 rows 40 / 41 us, 32 heads 800 rows 38 / 40, elsewhere up to 1.7 times as long)
   const int n_tiles = (n_new + BR - 1) / BR;
-  const int Tc_max = (T + CW - 1) / CW * CW;
-  const size_t lds = prefill_lds_bytes(BR, Tc_max);
   static bool attr_set[16] = {};
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
   if (!attr_set[dev & 15]) {
-    LCU_HIP(hipFuncSetAttribute((const void*)prefill_attention_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)prefill_lds_bytes(16, MAX_T_PREFILL)));
-    LCU_HIP(hipFuncSetAttribute((const void*)prefill_attention_kernel<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)prefill_lds_bytes(32, MAX_T_PREFILL_32)));
+    LCU_HIP(hipFuncSetAttribute((const void*)prefill_attention_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)prefill_lds_bytes(MAX_T_PREFILL)));
     attr_set[dev & 15] = true;
   }
-  if (BR == 16) {
-    prefill_attention_kernel<16><<<n_tiles * n_heads, 256, lds, s>>>(
-        (half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T, start_pos, dim,
-        n_tiles);
-  } else {
-    prefill_attention_kernel<32><<<n_tiles * n_heads, 256, lds, s>>>(
-        (half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T, start_pos, dim,
-        n_tiles);
-  }
+  prefill_attention_kernel<<<n_tiles * n_heads, 256, lds, s>>>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev,
+                                                               n_new, T, start_pos, dim, n_tiles);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }

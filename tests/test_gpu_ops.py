@@ -842,6 +842,46 @@ def test_attention_of_many_scores_equals_portions(gpu):
     G.release()
 
 
+# the kernel that stores scores: a lane's pairs of a row in registers up to 128, 256, 512 and 1024 columns, on both sides of each, and in
+# LDS beyond; both sides of the line to the kernel above, with two strips and with one in a compute unit's LDS
+@pytest.mark.parametrize("heads,n,T", [(4, 17, 256), (4, 20, 257), (4, 33, 512), (3, 18, 513), (3, 16, 1024), (3, 31, 1025), (64, 500, 500), (64, 560, 560),
+                                       (17, 300, 1838), (14, 1250, 1990), (9, 1250, 1990)])
+def test_attention_of_scores_in_registers(gpu, heads, n, T):
+    test_attention_of_many_scores(gpu, heads, n, T)
+
+
+@pytest.mark.parametrize("heads,n", [(64, 560), (5, 150)])
+def test_attention_of_extreme_scores(gpu, heads, n):
+    """Both kernels for prompts against the oracle: equal scores, one that takes all, scores past fp16, products past fp32, NaN."""
+    G = gpu
+    dim = heads * 128
+    q, k, v = normal((n, dim), 0, 1040, 1.0), normal((n, dim), 0, 1041, 1.0), normal((n, dim), 0, 1042, 1.0)
+    q[:, :128] *= 0
+    q[:, 128:256] *= 60
+    k[100, 256:384] = 60000
+    q[:, 256:384] = 60000
+    k[60, 384], k[80, 512] = np.inf, np.nan
+    out_d = G.empty((n, dim))
+    G.B.check(G.L().lcu_attention(out_d.ptr, G.dev_keep(q).ptr, G.dev_keep(k).ptr, G.dev_keep(v).ptr, n, n, 0, dim, heads, None))
+    got = G.host(out_d, (n, dim))
+    assert G.ulp_mismatch(got[:, :256], O.attention_prefill_kernel_order(q[:, :256], k[:, :256], v[:, :256], 2, 0)) == 0.0
+    # a score of +infinity or NaN leaves a row of NaN; one of -infinity is a probability of 0
+    seen = np.tril(np.ones((n, n), bool))
+    with np.errstate(all="ignore"):
+        z = [np.float64(q[:, h * 128:h * 128 + 128]) @ np.float64(k[:, h * 128:h * 128 + 128]).T / 128 ** 0.5 for h in range(5)]
+        lost = [(seen & ~(np.float32(x).astype(np.float16) < np.inf)).any(1) for x in z]
+    assert lost[2][100:].all() and 0 < lost[3].sum() < n - 60 and lost[4].sum() == n - 80
+    for h in (2, 3, 4):
+        out = got[:, h * 128:h * 128 + 128]
+        assert (np.isnan(out) == lost[h][:, None]).all(), h
+        if h > 2:
+            x = np.where(seen, np.where(lost[h][:, None], 0.0, z[h]), -np.inf)
+            e = np.exp(x - x.max(1, keepdims=True))
+            want = e @ np.float64(v[:, h * 128:h * 128 + 128]) / e.sum(1, keepdims=True)
+            assert np.abs(out - want)[~lost[h]].max() < 1.6e-2  # values below 4: scores, probabilities and outputs in halves of 2^-11 each
+    G.release()
+
+
 def test_attention_decode_twice_reuses_workspace(gpu):
     # the split-T decode path keeps arrival counters in a workspace; back-to-back calls must agree
     G = gpu
