@@ -393,22 +393,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS <= 4 ? 2 : 1) void 
   int tn = logical / tiles_m;
   int e = 0;  // GROUPED: the group of this tile
   if constexpr (EP::GROUPED) {
-    // The launch has as many row tiles as the list can ever hold; those that are there are dealt to the XCDs in equal runs, group by
-    // group, a group's row tiles of the same columns side by side: an XCD's L2 then holds the rows of two or three experts, not of
-    // all sixteen (512 tokens, top 2 of 16 experts of 4096 x 5632 and 2816 x 4096: 199 -> 181 us, 101 -> 92; 2000 tokens 380 -> 347,
-    // 203 -> 193).  A run of the list is found among its 64 entries that hold the tile, so longer ones are cut there.
-    const int n_tiles = *ep.n_tiles, active = n_tiles * tiles_n, qa = active / NUM_XCD, ra = active % NUM_XCD;
-    if (idx >= qa + (xcd < ra ? 1 : 0)) return;
-    const int at = xcd * qa + min(xcd, ra) + idx, j = at / tiles_n, block = j & ~63;
-    const int mine = ep.tile_group[min(block + lane, n_tiles - 1)];
-    e = __builtin_amdgcn_readlane(mine, j - block);
-    const uint64_t others = ~__ballot(mine == e && block + lane < n_tiles);  // bits of the list's other groups
-    const uint64_t below = others & ((1ull << (j - block)) - 1), above = others >> (j - block);
-    const int first = below ? 64 - __builtin_clzll(below) : 0;
-    const int count = (above ? j - block + __builtin_ctzll(above) : 64) - first;
-    const int rest = at - (block + first) * tiles_n;
-    tm = block + first + rest % count;
-    tn = rest / count;
+    const group_tile_t at = group_tile(ep, tiles_n, bx);
+    if (at.group < 0) return;
+    e = at.group, tm = at.row_tile, tn = at.column_tile;
   }
   // which weight matrix this tile belongs to: chosen once, from kernel arguments (scalar selects)
   half_t* out = out0;
@@ -1789,11 +1776,17 @@ template int gemm_bf16<true>(linear_epilogue<false, true> const&, const void*, c
 
 // Products of groups of rows with one matrix each, from the tile list in ep (row tiles of ep.tile_rows rows, at
 // most max_tiles of them).
+// What bounds them is the weight stream, up to some 100 rows a group: 24 GB/s to a compute unit, those lines included that two row tiles of
+// a group both ask for.  So a group's rows go into one tile where they fit, and W's ring holds seven stages: 512 tokens, top 2 of 16 experts of
+// 4096 x 5632 and 2816 x 4096, tiles of 64 rows 176 and 103 us, of 128 160 and 88 (162 and 92 on gemm_dl_kernel), of 256 169 and 93; 320 tokens 148
+// and 74, 150 and 82, 167 and 88; 1000 tokens 223 and 122, 202 and 119, 179 and 107 (gemm_dl_kernel 235 and 123); 2000 tokens 361 and 195, 325 and 175,
+// 254 and 155 (286 and 171).
 template <bool GATED>
 int gemm_bf16_grouped(linear_epilogue<true, GATED> const& ep, const void* A, const void* W, int max_tiles, int K, int N,
                       hipStream_t st) {
-  if (ep.tile_rows == 256) return launch_bf16<256, 128, 4, 2, 1, 3>(ep, A, W, max_tiles, 0, K, N, st);
-  if (ep.tile_rows == 128) return launch_bf16<128, 128, 4, 2, 1, 3>(ep, A, W, max_tiles, 0, K, N, st);
+  const operands_t op = single_matrix(nullptr, W, nullptr);
+  if (ep.tile_rows == 256) return launch_tile<256, 128, 4, 2, 3, 3, false, false>(ep, op, A, max_tiles * 256, K, N, 0, 0.0f, st);
+  if (ep.tile_rows == 128) return launch_tile<128, 128, 2, 2, 3, 7, false, false>(ep, op, A, max_tiles * 128, K, N, 0, 0.0f, st);
   return launch_bf16<64, 128, 2, 2, 1, 3>(ep, A, W, max_tiles, 0, K, N, st);
 }
 template int gemm_bf16_grouped<false>(linear_epilogue<true, false> const&, const void*, const void*, int, int, int, hipStream_t);

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0, int block_shift,
     int M, int K, int N, float beta, int tiles_m, int tiles_n, int from, float* __restrict__ part, int splits, int step, more_matrices_t more, EP ep) {
   using shape = tile_shape<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP>;
-  static_assert(!EP::GROUPED, "one matrix for all rows");
+  static_assert(!EP::GROUPED || (!SPLIT && EP::BF16), "experts");
   constexpr int NW = shape::NW;
   constexpr int TM = shape::WR / 16, TN = shape::WC / 16;        // 16x16 tiles of a wavefront
   constexpr int A_BYTES = shape::A_BYTES, B_BYTES = shape::B_BYTES, W_BYTES = shape::W_BYTES, W_RING = NA * A_BYTES;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   const int bx = SPLIT ? blockIdx.x - split * nb : blockIdx.x;
   const int q = nb / 8, r = nb % 8, xcd = bx % 8;
   const int logical = xcd * q + min(xcd, r) + bx / 8;
-  const int tm = logical % tiles_m;
+  int tm = logical % tiles_m;
   int tn = logical / tiles_m;
   half_t* out = out0;
   const void* W = W0;
@@ -141,7 +141,16 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     if constexpr (U8) S = g == 0 ? S0 : (g == 1 ? more.S[0] : more.S[1]);
     if constexpr (SPLIT) part += (size_t)g * splits * M * N;  // each matrix has its own partial sums
   }
-  const int m0 = tm * BM, n0 = from + tn * BN;
+  int m0 = tm * BM;
+  if constexpr (EP::GROUPED) {
+    const group_tile_t at = group_tile(ep, tiles_n, bx);
+    if (at.group < 0) return;
+    m0 = ep.tile_row[at.row_tile];
+    M = ep.group_end[at.group];
+    tn = at.column_tile;
+    W = (const char*)W0 + (size_t)at.group * ep.group_stride;
+  }
+  const int n0 = from + tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave % WM) * shape::WR, wn = (wave / WM) * shape::WC;
 
@@ -160,7 +169,12 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 #pragma unroll
   for (int j = 0; j < PA; ++j) {
     const int c = (wave + j * NW) * 64 + lane, row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
-    a_off[j] = row_piece(m0 + row, M, (uint32_t)K * 2u, g);
+    if constexpr (EP::GROUPED) {
+      const int r = min(m0 + row, M - 1), from_row = ep.row_index ? ep.row_index[r] : r;
+      a_off[j] = row_piece(from_row, from_row + 1, (uint32_t)K * 2u, g);
+    } else {
+      a_off[j] = row_piece(m0 + row, M, (uint32_t)K * 2u, g);
+    }
   }
 #pragma unroll
   for (int j = 0; j < PB; ++j) {
@@ -182,7 +196,8 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 #pragma unroll
     for (int j = 0; j < TN; ++j) f_first[j] = (uint32_t)min(n0 + wn + j * 16 + (lane & 15), N - 1) * blocks;
   }
-  uint4_t ra = operand_resource(A, (uint32_t)M * (uint32_t)K * 2u), rw = operand_resource(W, (uint32_t)N * (uint32_t)K * (U8 ? 1u : 2u)), rs = ra;
+  // of gathered rows the list knows only which they are
+  uint4_t ra = operand_resource(A, EP::GROUPED ? 0xffffffffu : (uint32_t)M * (uint32_t)K * 2u), rw = operand_resource(W, (uint32_t)N * (uint32_t)K * (U8 ? 1u : 2u)), rs = ra;
   if constexpr (U8) rs = operand_resource(S, (uint32_t)N * ((uint32_t)K >> (6 + block_shift)) * 2u);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)tile_lds;
   // Inline assembly, so that the compiler does not know about the LDS writes: knowing, it waits for every LDS read
@@ -357,6 +372,14 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   typedef float4_t any_float4_t __attribute__((aligned(4)));
   const auto pass = [&](auto which) {
     constexpr int p = decltype(which)::value;
+    float scale[4][4];  // of the rows of gated experts
+    if constexpr (EP::GROUPED && EP::GATED) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int gm = m0 + wm + p * 64 + i / 4 * 16 + (lane >> 4) * 4 + i % 4;
+        scale[i / 4][i % 4] = ep.row_scale ? ep.row_scale[min(gm, M - 1)] : 1.0f;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
@@ -368,7 +391,11 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 #pragma unroll
           for (int j = 0; j < TN; j += 4) {
 #pragma unroll
-            for (int e = 0; e < 2; ++e) to[(j / 2 + e) * 16] = ep.gate(acc[p * 4 + i][j + e][v], acc[p * 4 + i][j + 2 + e][v]);
+            for (int e = 0; e < 2; ++e) {
+              float gate = acc[p * 4 + i][j + e][v], up = acc[p * 4 + i][j + 2 + e][v];
+              if constexpr (EP::GROUPED) gate *= scale[i][v], up *= scale[i][v];
+              to[(j / 2 + e) * 16] = ep.gate(gate, up);
+            }
           }
         } else {
 #pragma unroll

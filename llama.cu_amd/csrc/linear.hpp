@@ -44,6 +44,29 @@ struct row_groups<true> {
   int tile_rows;
 };
 
+// Which tile workgroup `bx` takes; group -1: none.  The launch has as many row tiles as the list can ever hold; those that are there are dealt to
+// the XCDs in equal runs, group by group, a group's row tiles of the same columns side by side: an XCD's L2 then holds the rows of two or
+// three experts, not of all sixteen (512 tokens, top 2 of 16 experts of 4096 x 5632 and 2816 x 4096, 64-row tiles: 199 -> 181 us, 101 -> 92; 2000
+// tokens 380 -> 347, 203 -> 193).  A run of the list is found among its 64 entries that hold the tile, so longer ones are cut there.
+struct group_tile_t {
+  int group, row_tile, column_tile;
+};
+__device__ __forceinline__ group_tile_t group_tile(const row_groups<true>& g, int columns, int bx) {
+  constexpr int XCDS = 8;
+  const int lane = threadIdx.x & 63, xcd = bx % XCDS, idx = bx / XCDS;
+  const int n_tiles = *g.n_tiles, active = n_tiles * columns, q = active / XCDS, r = active % XCDS;
+  if (idx >= q + (xcd < r ? 1 : 0)) return {-1, 0, 0};
+  const int at = xcd * q + min(xcd, r) + idx, j = at / columns, block = j & ~63;
+  const int mine = g.tile_group[min(block + lane, n_tiles - 1)];
+  const int group = __builtin_amdgcn_readlane(mine, j - block);
+  const uint64_t others = ~__ballot(mine == group && block + lane < n_tiles);  // bits of the list's other groups
+  const uint64_t below = others & ((1ull << (j - block)) - 1), above = others >> (j - block);
+  const int first = below ? 64 - __builtin_clzll(below) : 0;
+  const int count = (above ? j - block + __builtin_ctzll(above) : 64) - first;
+  const int rest = at - (block + first) * columns;
+  return {group, block + first + rest % count, rest / count};
+}
+
 // GATED: the matrix holds, in blocks of 64 rows, 32 gate rows and the 32 up rows of the same hidden columns.
 template <bool GROUPED_, bool GATED_>
 struct linear_epilogue : row_groups<GROUPED_> {

@@ -321,8 +321,8 @@ void layered_context_impl::embed(int n, void* w_next) {
 void layered_context_impl::experts(experts_weights const& w, experts_params const& p, int n) {
   layered_model_impl const& m = *model_;
   const int rows = n * p.top, W = m.shape.width;
-  // tiles of about half an expert's rows: larger ones multiply faster, but every expert ends in a part of one
-  plan_.tile_rows = m.dtype == LCU_F32 ? 32 : (rows >= 384 * p.experts ? 256 : rows >= 96 * p.experts ? 128 : 64);
+  // tiles that hold an expert's rows, or most of them: a second tile asks for its weights again (figures at gemm_bf16_grouped)
+  plan_.tile_rows = m.dtype == LCU_F32 ? 32 : (rows >= 104 * p.experts ? 256 : rows >= 52 * p.experts ? 128 : 64);
   plan_.max_tiles = rows / plan_.tile_rows + std::min(p.experts, rows);
   LCU_CHECK(lcu_router(t_choice_.data(), t_weight_.data(), p.shared_ff > 0 ? t_shared_gate_.data() : nullptr, t_h_.data(),
                        w.router.data(), p.experts, p.top, m.dtype, n, m.ld, stream_));

@@ -459,6 +459,36 @@ def test_experts_lists_of_many_tiles(gpu, n, K, ff, experts, top, tile):
     test_experts(gpu, BF16, n, K, ff, experts, top, tile)
 
 
+# one, some and many tiles to an expert, K and the hidden columns shorter and longer than W's ring of seven stages
+@pytest.mark.parametrize("n,K,ff,experts,top", [(700, 576, 500, 3, 2), (600, 64, 100, 5, 1), (50, 1024, 64, 9, 3)])
+def test_experts_in_tiles_of_any_height(gpu, n, K, ff, experts, top):
+    """Tiles of 64, 128 and 256 rows: the same sums in the same order, so the same bits."""
+    rng = np.random.default_rng(n)
+    N, ld, rows = 200, up64(ff), n * top
+    h = put(gpu, rounded(rng.standard_normal((n, K))), BF16)
+    gate, up = (rounded(rng.standard_normal((experts, ff, K)) / K ** 0.5) for _ in range(2))
+    packed = put(gpu, np.stack([pack_gated(gate[e], up[e], ld) for e in range(experts)]), BF16)
+    down = put(gpu, pad(rounded(rng.standard_normal((experts, N, ff)) / ff ** 0.5), ld), BF16)
+    choice = ints(gpu, np.stack([rng.permutation(experts)[:top] for _ in range(n)]))
+    weight, g = put(gpu, rng.random((n, top))), gpu.B.GateParams(0.8, 1.702, 1.0)
+    got = []
+    for tile in (64, 128, 256):
+        plan, keep, max_tiles = gpu.B.ExpertPlan(), {}, rows // tile + experts
+        for name, count in (("row_token", rows), ("row_weight", rows), ("inverse", rows), ("tile_expert", max_tiles), ("tile_row", max_tiles),
+                            ("expert_end", experts), ("n_tiles", 1)):
+            keep[name] = ints(gpu, np.zeros(count))
+            setattr(plan, name, keep[name].ptr)
+        plan.tile_rows, plan.max_tiles = tile, max_tiles
+        call(gpu, "lcu_experts_plan", C.byref(plan), choice, weight, n, top, experts)
+        hidden, out = zeros(gpu, (rows, ld), BF16), zeros(gpu, (rows, N))
+        call(gpu, "lcu_experts_up", hidden, ld, h, packed, 2 * ld * K * 2, C.byref(g), C.byref(plan), BF16, n, K, 2 * ld)
+        call(gpu, "lcu_experts_down", out, N, hidden, down, N * ld * 2, C.byref(plan), BF16, rows, ld, N)
+        got.append(get(gpu, out, (rows, N))[get_ints(gpu, keep["inverse"], (rows,))])
+    assert np.isfinite(got[0]).all() and np.abs(got[0]).max() > 0.1
+    assert (got[0] == got[1]).all() and (got[0] == got[2]).all()
+    gpu.release()
+
+
 @pytest.mark.parametrize("n", [1, 7, 640, 32000, 50257])
 def test_argmax_and_softmax(gpu, n):
     rng = np.random.default_rng(n)
