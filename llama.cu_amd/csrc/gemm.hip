@@ -951,7 +951,8 @@ struct large_tiles_t {
 // A last round that is nearly empty goes to smaller tiles: whole rounds of one width, then the columns that are left in those tiles that cost least
 // (us, the best single width / so: uint8 512 rows, K 6656, twice 17920 columns 254 / 234; fp16 K 4096, twice 11008 columns, 700 rows 143 / 136,
 // 1000 rows 164 / 158, 1987 rows 300 / 290).  The second launch costs 3 us more; below 1024 of K that is what it gains.
-// Gated outputs come in pairs of 32 columns and 32 columns behind them: no 96-column wavefronts there.
+// Gated outputs come in pairs of 32 columns and 32 columns behind them, so there 192 columns go to each of four wavefronts of 64 rows
+// (bfloat16, us with 128 and 256 columns only / so: 512x4096x22016 104 / 84, 1500 rows 260 / 236, 1987x2048x5632 57 / 46).
 // Up to 512 of K what a tile pays beside its stages counts: 256 columns leave by four wavefronts, and the rounds are no measure of
 // them (1441 rows of K 256, three times 2944 columns: 216 tiles of 256 20.1 us, 414 of 128 16.5; bfloat16 1027x512x11840 28.7 / 23.4),
 // and 192 no gain below 256.
@@ -966,7 +967,7 @@ large_tiles_t plan_large(int M, int K, int N, int n_mats, long cus, bool gated) 
     return {c256 < c128 ? 256 : 128, {}, {}, 0, 0};
   }
   const auto round = [&](int columns) -> long { return columns == 128 ? (U8 ? 59 : 57) : columns == 192 ? (U8 ? 79 : 73) : (U8 ? 104 : 94); };
-  const auto allowed = [&](int columns) { return columns == 128 || (columns == 192 ? K >= 256 && !gated : K >= 640); };
+  const auto allowed = [&](int columns) { return columns == 128 || (columns == 192 ? K >= (gated ? 640 : 256) : K >= 640); };
   large_tiles_t best{128, {}, {}, 0, 0};
   long least = rounds(tiles(256, 128, N) * n_mats) * round(128);
   for (int columns : {256, 192}) {
@@ -1005,8 +1006,8 @@ int launch_columns(EP const& ep, operands_t op, const void* A, int M, int K, int
     return launch_tile<256, 128, 1, 4, 3, 3, true, false>(ep, op, A, M, K, N, block, beta, st, 1, nullptr, which);
   } else {
     if (columns == 256) return launch_tile<256, 256, 2, 2, 2, 3, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
-    if constexpr (!EP::GATED) {
-      if (columns == 192) return launch_tile<256, 192, 2, 2, 2, 4, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
+    if (columns == 192) {
+      return launch_tile<256, 192, EP::GATED ? 4 : 2, EP::GATED ? 1 : 2, 2, 4, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
     }
     return launch_tile<256, 128, 4, 2, 3, 3, false, false>(ep, op, A, M, K, N, 0, beta, st, 1, nullptr, which);
   }

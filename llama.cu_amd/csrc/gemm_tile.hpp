@@ -98,7 +98,7 @@ struct tile_shape {
   static constexpr int NW = WM * WN, WR = BM / WM, WC = BN / WN;
   static constexpr int A_BYTES = BM * 128, B_BYTES = BN * (U8 ? 64 : 128), SW = (WC + 63) / 64 * 64, S_BYTES = U8 ? NW * SW * 4 : 0;
   static constexpr int W_BYTES = B_BYTES + S_BYTES;      // S: one word per column of every wavefront, of its own
-  static constexpr int OUT_LD = WC + 4;                  // floats per row of a wavefront's 64 output rows in LDS
+  static constexpr int OUT_LD = (EP::GATED ? WC / 2 : WC) + 4;  // floats per row of a wavefront's 64 output rows in LDS
   static constexpr int RING = NA * A_BYTES + NB * W_BYTES, OUT = NW * 64 * OUT_LD * 4;
   static constexpr int LDS = RING > OUT ? RING : OUT;
   static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 16 == 0, "tile");

@@ -94,6 +94,12 @@ def test_linear_columns_left_of_whole_rounds(gpu, M, K, N):
     test_gated_linear_large_tiles(gpu, M, K, N // 2)
 
 
+# gated outputs of 192 columns: one round of them, behind whole rounds of 256, ragged ends; the shortest K and one below
+@pytest.mark.parametrize("M,K,ff", [(300, 1024, 10900), (1990, 1024, 10980), (500, 640, 10920), (500, 576, 10920)])
+def test_gated_linear_192_columns(gpu, M, K, ff):
+    test_gated_linear_large_tiles(gpu, M, K, ff)
+
+
 @pytest.mark.parametrize("M,K,ff", [(1100, 1216, 1850), (1100, 1280, 1850), (1441, 640, 4400), (20, 512, 13000), (6, 2816, 1020)])
 def test_gated_linear_tiles_by_length(gpu, M, K, ff):
     test_gated_linear_large_tiles(gpu, M, K, ff)
