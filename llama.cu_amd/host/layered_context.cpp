@@ -379,8 +379,8 @@ void layered_context_impl::enqueue_rows(int n) {
 
 // One token: launches fused around the weight streams.  A recurrent layer's mixer takes three (projections
 // with the convolution, gates with the state, output product), an attention layer's too (projections with the
-// cache rows, attention, output product), a latent layer's five (projections; keys applied to the queries, with norm,
-// rotations and cache rows; scores; values; output product; two more with a queries' latent), a feed-forward two
+// cache rows, attention, output product), a latent layer's four (projections; keys applied to the queries, with norm,
+// rotations and cache rows; scores and values, two launches beyond SHORT_CONTEXT positions; output product; two more with a queries' latent), a feed-forward two
 // (first products, second products); between sublayers one launch adds the result, takes both norms and, in front of a feed-forward, routes.  The last
 // layer's norms end in the final one.
 void layered_context_impl::enqueue_one() {
