@@ -966,7 +966,12 @@ large_tiles_t plan_large(int M, int K, int N, int n_mats, long cus, bool gated) 
     const long c128 = rounds(tiles(128, 128, N) * n_mats) * (U8 ? 42 : 52), c256 = rounds(tiles(128, 256, N) * n_mats) * (U8 ? 62 : 66);
     return {c256 < c128 ? 256 : 128, {}, {}, 0, 0};
   }
-  const auto round = [&](int columns) -> long { return columns == 128 ? (U8 ? 59 : 57) : columns == 192 ? (U8 ? 79 : 73) : (U8 ? 104 : 94); };
+  // over a short K what a tile pays beside its stages makes the wider ones dearer (fp16, 192 / 128 columns: 1508x256x11087 45 / 29 us, 783x512x15510
+  // twice 71 / 51, 520x640x16509 three times 87 / 65)
+  const bool brief = !U8 && K < 1152;
+  const auto round = [&](int columns) -> long {
+    return columns == 128 ? (U8 ? 59 : 57) : columns == 192 ? (U8 ? 79 : brief ? 88 : 73) : (U8 ? 104 : brief ? 106 : 94);
+  };
   const auto allowed = [&](int columns) { return columns == 128 || (columns == 192 ? K >= (gated ? 640 : 256) : K >= 640); };
   large_tiles_t best{128, {}, {}, 0, 0};
   long least = rounds(tiles(256, 128, N) * n_mats) * round(128);
