@@ -112,7 +112,10 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   static_assert(!EP::GROUPED || (!SPLIT && EP::BF16), "experts");
   constexpr int NW = shape::NW;
   constexpr int TM = shape::WR / 16, TN = shape::WC / 16;        // 16x16 tiles of a wavefront
-  constexpr int A_BYTES = shape::A_BYTES, B_BYTES = shape::B_BYTES, W_BYTES = shape::W_BYTES, W_RING = NA * A_BYTES;
+  constexpr int A_BYTES = shape::A_BYTES, B_BYTES = shape::B_BYTES, W_BYTES = shape::W_BYTES;
+  // rings of one length: a stage's lhs and columns side by side, one slot for both (uint8 with two slots 5 to 7 % slower, 736x4096x4096 40 / 43 us)
+  constexpr bool JOINT = NA == NB;
+  constexpr int A_STEP = JOINT ? A_BYTES + W_BYTES : A_BYTES, W_STEP = JOINT ? A_STEP : W_BYTES, W_RING = JOINT ? A_BYTES : NA * A_BYTES;
   constexpr int PA = A_BYTES / 1024 / NW, PB = B_BYTES / 1024 / NW, PS = U8 ? shape::SW / 64 : 0;
   constexpr int PW = PB + PS, P = PA + PW;  // requests of a wavefront per stage
   constexpr int BEHIND = NB > NA ? PW : 0;  // of a stage's requests, those behind its lhs that lhs's turn need not wait for
@@ -210,13 +213,13 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   // request i of a wavefront's P: lhs of stage `a` into its ring's slot, then the columns (and scales) of stage `b` into theirs
   const auto issue = [&](int a, int a_slot, int b, int b_slot, int i) {
     if (i < PA) {
-      request(ra, stage_offset(ra[2], stage_of(a) * 128u), a_off[i], a_slot * A_BYTES + (wave + i * NW) * 1024);
+      request(ra, stage_offset(ra[2], stage_of(a) * 128u), a_off[i], a_slot * A_STEP + (wave + i * NW) * 1024);
     } else if (i < PA + PB) {
-      request(rw, stage_offset(rw[2], stage_of(b) * (U8 ? 64u : 128u)), b_off[i - PA], W_RING + b_slot * W_BYTES + (wave + (i - PA) * NW) * 1024);
+      request(rw, stage_offset(rw[2], stage_of(b) * (U8 ? 64u : 128u)), b_off[i - PA], W_RING + b_slot * W_STEP + (wave + (i - PA) * NW) * 1024);
     } else if constexpr (U8) {  // the word that holds the row's scale of this stage
       const uint32_t at = s_first[i - PA - PB] + (stage_of(b) >> block_shift);
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(scale_word(at)), "s"(rs),
-                   "s"(lds0 + W_RING + b_slot * W_BYTES + B_BYTES + wave * shape::SW * 4 + (i - PA - PB) * 256)
+                   "s"(lds0 + W_RING + b_slot * W_STEP + B_BYTES + wave * shape::SW * 4 + (i - PA - PB) * 256)
                    : "memory", "m0");
     }
   };
@@ -240,7 +243,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   // reads of half 0: (scales, codes,) W and lhs fragments of half 0(, codes of half 1); of half 1 the fragments that are left
   constexpr int READS0 = U8 ? 3 * TN + TM : TN + TM, READS1 = U8 ? TM : TN + TM, PRODUCTS = TM * TN;
   const auto read = [&](int a_slot, int b_slot, int h, int i) {
-    const unsigned char *pa = tile_lds + a_slot * A_BYTES + a_row, *pw = tile_lds + b_slot * W_BYTES;
+    const unsigned char *pa = tile_lds + a_slot * A_STEP + a_row, *pw = tile_lds + b_slot * W_STEP;
     if constexpr (U8) {
       const unsigned char* c = pw + W_RING + (wn + frag_row) * 64 + frag_chunk * 8;
       const int half_turn = (frag_row / 4) % 2 * 32;  // pieces turned by two: the halves change places
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   int a_slot = 0, b_slot = 0;
   for (int t = 0; t < nt - 1; ++t) {
     end_at(t + NA, t + NB);
-    const int a_next = a_slot + 1 == NA ? 0 : a_slot + 1, b_next = b_slot + 1 == NB ? 0 : b_slot + 1;
+    const int a_next = a_slot + 1 == NA ? 0 : a_slot + 1, b_next = JOINT ? a_next : b_slot + 1 == NB ? 0 : b_slot + 1;
     stage(t, a_slot, b_slot, a_next, b_next, std::true_type{});
     a_slot = a_next;
     b_slot = b_next;
