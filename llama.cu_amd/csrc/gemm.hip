@@ -972,7 +972,7 @@ large_tiles_t plan_large(int M, int K, int N, int n_mats, long cus, bool gated) 
   const auto round = [&](int columns) -> long {
     return columns == 128 ? (U8 ? 59 : 57) : columns == 192 ? (U8 ? 79 : brief ? 88 : 73) : (U8 ? 104 : brief ? 106 : 94);
   };
-  const auto allowed = [&](int columns) { return columns == 128 || (columns == 192 ? K >= (gated ? 640 : 256) : K >= 640); };
+  const auto allowed = [&](int columns) { return columns == 128 || (columns == 192 ? K >= (U8 || gated ? 640 : 256) : K >= 640); };  // uint8, K 512: 1772x17920 192 columns 65 us, 128 52
   large_tiles_t best{128, {}, {}, 0, 0};
   long least = rounds(tiles(256, 128, N) * n_mats) * round(128);
   for (int columns : {256, 192}) {
