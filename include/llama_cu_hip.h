@@ -549,6 +549,33 @@ int lcu_decode_residual_router(void* x_dev, void* h_dev, const void* out_f32_dev
                                int groups, float eps, const void* router_w_dev, int n_experts, int choose, void* expert_dev,
                                void* weight_dev, void* router_gate_dev, void* stream);
 
+/* The same products of a row that is not there yet: the launch itself adds what the sublayer before it left and takes both
+ * norms (lcu_decode_residual_router without a router), each workgroup for itself, while its weights are on their way.  The sum
+ * goes to x_out, which must not overlap x; the normed row goes to h only where the shape takes a launch of its own for it
+ * (rows of more than 2048 elements, matrices of more than 64 MB).  K is the row's ld.  Same bits as the two calls. */
+typedef struct lcu_step_row {
+  const void* x_dev; /* fp32 residual row */
+  void* x_out_dev;
+  void* h_dev;       /* bfloat16 */
+  const void* out_f32_dev;
+  const void* shared_f32_dev;
+  const void* shared_gate_dev;
+  const void* w_after_dev;
+  const void* w_next_dev; /* NULL: the sum itself, not its norm */
+  int top, width, ld, groups;
+  float eps;
+} lcu_step_row;
+int lcu_step_linear(void* out_f32_dev, const lcu_step_row* row, const void* w_dev, const void* bias_dev, int N, void* stream);
+int lcu_step_linear_bf16(void* out_dev, const lcu_step_row* row, const void* w_dev, int N, void* stream);
+int lcu_step_delta_in(void* u_dev, void* plain_dev, void* tail_f32_dev, void* conv_state_dev, const lcu_step_row* row, const void* w_dev,
+                      const void* conv_dev, int taps, int channels, int plain, int N, void* stream);
+int lcu_step_gated(void* hidden_dev, const lcu_step_row* row, const void* w_dev, const lcu_gate_params* gate, int ld, void* stream);
+int lcu_step_recurrent_in(void* y_dev, void* u_dev, void* conv_state_dev, const lcu_step_row* row, const void* w_dev, const void* bias_dev,
+                          const void* conv_dev, const void* conv_bias_dev, int taps, int ld, void* stream);
+int lcu_step_kv(void* q_out_dev, void* k_cache_dev, void* v_cache_dev, const lcu_step_row* row, const void* w_dev, const void* bias_dev,
+                int q_cols, int k_cols, int v_cols, void* v_first_dev, int v_mode, const void* lambda_dev, const void* pos_dev,
+                int max_positions, void* stream);
+
 /* pseudo-random matrix (synthetic weights): mean + std * N(0, 1) (the hash of lcu_fill_normal_f16) into
  * columns 0 .. cols - 1 of rows of ld elements */
 int lcu_fill_normal_matrix(void* out_dev, size_t rows, int cols, int ld, int dtype, uint64_t seed, uint64_t stream_id, float mean,

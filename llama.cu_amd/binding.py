@@ -134,6 +134,12 @@ SIGNATURES = {
     "lcu_decode_experts_up": (i32, [vp] * 6 + [sz, vp, vp, vp, i32, i32, i32, i32, vp]),
     "lcu_decode_experts_down": (i32, [vp, i32, vp, vp, vp, sz, i32, i32, vp, vp, i32, i32, vp]),
     "lcu_decode_residual_router": (i32, [vp, vp, vp, i32] + [vp] * 4 + [i32, i32, i32, f32, vp, i32, i32, vp, vp, vp, vp]),
+    "lcu_step_linear": (i32, [vp, vp, vp, vp, i32, vp]),
+    "lcu_step_linear_bf16": (i32, [vp, vp, vp, i32, vp]),
+    "lcu_step_delta_in": (i32, [vp] * 7 + [i32] * 4 + [vp]),
+    "lcu_step_gated": (i32, [vp, vp, vp, vp, i32, vp]),
+    "lcu_step_recurrent_in": (i32, [vp] * 8 + [i32, i32, vp]),
+    "lcu_step_kv": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, i32, vp, vp, i32, vp]),
     "lcu_fill_normal_matrix": (i32, [vp, sz, i32, i32, i32, u64, u64, f32, f32, vp]),
     # llama_cu_c.h
     "lcu_model_open": (vp, [C.c_char_p, i32, i32]),
@@ -247,6 +253,12 @@ class DeltaParams(C.Structure):
     """lcu_delta_params"""
     _fields_ = [(n, i32) for n in ("heads", "kv_heads", "dk", "dv", "dim", "vdim")] + [("eps", f32)] + \
         [(n, vp) for n in ("a_log", "dt_bias", "norm")]
+
+
+class StepRow(C.Structure):
+    """lcu_step_row"""
+    _fields_ = [(n, vp) for n in ("x", "x_out", "h", "out", "shared", "shared_gate", "w_after", "w_next")] + \
+        [(n, i32) for n in ("top", "width", "ld", "groups")] + [("eps", f32)]
 
 
 class DeviceBuffer:

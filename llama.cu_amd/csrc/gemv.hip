@@ -23,10 +23,12 @@
 // the instruction aligns and cuts its three addends in a way of its own, which the oracle's
 // kernel-order flavour restates from measured samples): the dequantisation arithmetic, not HBM,
 // is what bounds this kernel on large matrices.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
 #include "linear.hpp"
+#include "rownorm.hpp"
 
 using namespace lcu;
 
@@ -928,6 +930,162 @@ __global__ __launch_bounds__(GEMV_THREADS) void decode_experts_down_kernel(proje
   st.run(nullptr, 1.0f, part);
 }
 
+// ---- the same products of a row that the launch works out by itself ------------------------------
+// What stood between a sublayer and the next product was a launch of one workgroup whose result every workgroup of the product then
+// read: 3.0 us with its boundary.  Here every workgroup works the row out: it asks for the residual row, the sublayer's result and both
+// norms' weights first, then for as many weights as the compute unit's queue takes without a wait (64 KB; a wavefront that issues into a
+// full queue stalls, 128 KB made the norms 1 us later), and has the normed row in LDS when these arrive.  One workgroup of eight
+// wavefronts per compute unit (sixteen: the norms' reductions take twice as long); each takes an equal run of the tasks, a wavefront
+// whole rows of W, the next ones asked for ahead.  A wavefront adds a row's products up as the four wavefronts of stream_t would, four
+// sums that meet in their order: same bits.  K 2048, both launches -> this one, in a graph, weights from memory: N 1280 6.1 -> 5.2 us, 5696
+// 8.6 -> 7.2, 6176 9.0 -> 7.6, 5632 gated pairs 12.0 -> 11.1; 32000 rows 23.6 -> 23.6 (an equal share each streams slower than workgroups
+// that are dealt as others end: 14.5 against 19.3 for 11000 rows of 4096), so matrices above 64 MB and rows beyond 2048 keep two launches.
+// NC: 512-column pieces of a row; per: tasks of a workgroup, one more for the first `more`.
+constexpr int NORMED_THREADS = 512;
+template <int NC, int R, class Tasks>
+__global__ __launch_bounds__(NORMED_THREADS) void normed_rows_kernel(step_row s, Tasks tk, int per, int more, int sums_bytes) {
+  constexpr int TH = NORMED_THREADS, WAVES = TH / WAVE, CHUNK = 8 * WAVE, VW = GEMV_WAVES, NV = (NC * CHUNK + TH * 4 - 1) / (TH * 4);
+  constexpr int AHEAD = 8 / R < NC ? 8 / R : NC;  // pieces of the first task asked for before the norms
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  bf16_t* hs = reinterpret_cast<bf16_t*>(lds + sums_bytes);                     // the normed row
+  float4_t* done = reinterpret_cast<float4_t*>(lds + sums_bytes + NC * CHUNK * 2);  // [tasks of this workgroup][R][VW]: sums of 16 lanes
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), K = s.rs.ld;
+  const int first = blockIdx.x * per + min((int)blockIdx.x, more), end = first + per + ((int)blockIdx.x < more ? 1 : 0);
+  row_t<NV, TH> m, t, old, after, next;
+  load_row(after, s.w_after, s.rs);
+  load_row(next, s.w_next ? s.w_next : s.w_after, s.rs);
+  load_row(old, s.x, s.rs);
+  load_sum(m, t, s.src, 0, s.rs);
+  issue_order_fence();
+  const auto load = [&](uint4_t (&w)[NC][R], int task, auto from, auto to) {
+    const uint8_t* rows[R];
+    const half_t* none[R];
+    tk.rows(task, rows, none);
+#pragma unroll
+    for (int c = decltype(from)::value; c < decltype(to)::value; ++c) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        w[c][r] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>(rows[r] + (size_t)min(c * CHUNK + lane * 8, K - 8) * 2));
+      }
+    }
+  };
+  constexpr std::integral_constant<int, 0> begin{};
+  constexpr std::integral_constant<int, AHEAD> ahead{};
+  constexpr std::integral_constant<int, NC> all{};
+  uint4_t w[2][NC][R];
+  const int mine = min(first + wave, end - 1);  // a wavefront without a task asks for its neighbour's lines
+  load(w[0], mine, begin, ahead);
+  issue_order_fence();
+  float* sums = reinterpret_cast<float*>(lds);
+  scale_row(m, s.rs, sums, after);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) m.v[j] += old.v[j];
+  if (blockIdx.x == 0) store_row(s.x_out, m, s.rs);
+  if (s.w_next) scale_row(m, s.rs, sums, next);
+  store_row(hs, m, s.rs);
+  issue_order_fence();
+  load(w[0], mine, ahead, all);
+  issue_order_fence();
+  __syncthreads();
+  const auto step = [&](uint4_t (&w)[NC][R], uint4_t (&nw)[NC][R], int task) {
+    if (task + WAVES < end) load(nw, task + WAVES, begin, all);
+    float a0[R][VW] = {}, a1[R][VW] = {};
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int kk = c * CHUNK + lane * 8, v = c % VW;
+      if (kk < K) {
+        const uint4_t xw = *reinterpret_cast<const uint4_t*>(hs + kk);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            a0[r][v] = fmaf(__builtin_bit_cast(float, w[c][r][e] << 16), __builtin_bit_cast(float, xw[e] << 16), a0[r][v]);
+            a1[r][v] = fmaf(__builtin_bit_cast(float, w[c][r][e] & 0xffff0000u), __builtin_bit_cast(float, xw[e] & 0xffff0000u), a1[r][v]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+      for (int v = 0; v < VW; ++v) {
+        const float q = row16_sum(a0[r][v] + a1[r][v]);
+        if ((lane & 15) == 0) reinterpret_cast<float*>(&done[((task - first) * R + r) * VW + v])[lane / 16] = q;
+      }
+    }
+  };
+  for (int task = first + wave; task < end; task += 2 * WAVES) {
+    step(w[0], w[1], task);
+    if (task + WAVES < end) step(w[1], w[0], task + WAVES);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < end - first; i += TH) {
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      acc[r] = 0.0f;
+#pragma unroll
+      for (int v = 0; v < VW; ++v) {
+        const float4_t q = done[(i * R + r) * VW + v];
+        acc[r] += (q[0] + q[1]) + (q[2] + q[3]);  // as wave_sum does
+      }
+    }
+    tk.finish(first + i, acc);
+  }
+}
+
+constexpr int NORMED_ROW_MAX = 2048;               // elements of a row
+constexpr size_t NORMED_BYTES_MAX = 64u << 20;     // of the matrix
+constexpr int NORMED_SUMS_MAX = 512;               // results a workgroup keeps in LDS
+
+// tasks of R rows through normed_rows_kernel; false: the shape is not for it
+template <int R, class Tasks>
+bool launch_normed_rows(const step_row& s, const Tasks& tk, int tasks, hipStream_t st) {
+  const device_state* ds = current_device_state();
+  const int groups = std::min(ds && ds->compute_units > 0 ? ds->compute_units : 256, tasks);
+  const int per = tasks / groups, more = tasks % groups, kept = (per + (more > 0 ? 1 : 0)) * R;
+  if (s.rs.ld > NORMED_ROW_MAX || (size_t)tasks * R * s.rs.ld * 2 > NORMED_BYTES_MAX || kept > NORMED_SUMS_MAX) return false;
+  const int sums = (int)((row_lds_bytes(s.rs) + 15) / 16 * 16);
+  const auto go = [&](auto nc) {
+    constexpr int NC = decltype(nc)::value;
+    normed_rows_kernel<NC, R><<<groups, NORMED_THREADS, sums + NC * 8 * WAVE * 2 + kept * GEMV_WAVES * 16, st>>>(s, tk, per, more, sums);
+  };
+  if (s.rs.ld <= 1024) {
+    go(std::integral_constant<int, 2>{});
+  } else {
+    go(std::integral_constant<int, 4>{});
+  }
+  return true;
+}
+
+template <class Epilogue>
+int launch_decode_rows(const lcu_step_row* row, const void* W, int K, int N, Epilogue ep, hipStream_t st) {
+  const step_row s = as_step_row(row);
+  if (launch_normed_rows<2>(s, bf16_tasks<2, Epilogue>{(const bf16_t*)W, K, N, ep}, (N + 1) / 2, st)) {
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+  }
+  const int rc = residual_step(s, st);
+  return rc ? rc : launch_decode_rows((const void*)s.h, W, K, N, ep, st);
+}
+
+int dense_gated(void* hidden, const void* h, const void* w, const lcu_gate_params* gate, int ld, int K, hipStream_t st) {
+  const clamped_gate g{gate->limit, gate->alpha, gate->up_shift};
+  expert_slots p{};  // no chosen expert: the matrix takes the place of the shared one
+  p.shared_up = (const bf16_t*)w;
+  p.shared_hidden = (bf16_t*)hidden;
+  p.gate = p.shared_gate = g;
+  p.ld = p.shared_ld = ld;
+  p.K = K;
+  if (K > 2048) {
+    decode_experts_up_kernel<2><<<ld, GEMV_THREADS, 0, st>>>((const bf16_t*)h, p);
+  } else {
+    decode_experts_up_kernel<1><<<ld, GEMV_THREADS, 0, st>>>((const bf16_t*)h, p);
+  }
+  LCU_LAUNCH_CHECK();
+  return LCU_OK;
+}
+
 // calls f with the number of 16-byte pieces of x per thread (x_stage_t) that covers dim <= 24576
 template <class F>
 void with_x_pieces(int dim, F&& f) {
@@ -1213,20 +1371,7 @@ int lcu_decode_delta_in(void* u_dev, void* plain_dev, void* tail_f32_dev, void* 
 int lcu_decode_gated(void* hidden_dev, const void* h_dev, const void* w_dev, const lcu_gate_params* gate, int ld, int K, void* stream) {
   LCU_REQUIRE(hidden_dev && h_dev && w_dev && gate, "lcu_decode_gated: null pointer");
   LCU_REQUIRE(ld > 0 && ld % 32 == 0 && K > 0 && K % 64 == 0, "lcu_decode_gated: bad shape ld %d K %d", ld, K);
-  const clamped_gate g{gate->limit, gate->alpha, gate->up_shift};
-  expert_slots p{};  // no chosen expert: the matrix takes the place of the shared one
-  p.shared_up = (const bf16_t*)w_dev;
-  p.shared_hidden = (bf16_t*)hidden_dev;
-  p.gate = p.shared_gate = g;
-  p.ld = p.shared_ld = ld;
-  p.K = K;
-  if (K > 2048) {
-    decode_experts_up_kernel<2><<<ld, GEMV_THREADS, 0, as_stream(stream)>>>((const bf16_t*)h_dev, p);
-  } else {
-    decode_experts_up_kernel<1><<<ld, GEMV_THREADS, 0, as_stream(stream)>>>((const bf16_t*)h_dev, p);
-  }
-  LCU_LAUNCH_CHECK();
-  return LCU_OK;
+  return dense_gated(hidden_dev, h_dev, w_dev, gate, ld, K, as_stream(stream));
 }
 
 int lcu_decode_recurrent_in(void* y_dev, void* u_dev, void* conv_state_dev, const void* x_dev, const void* w_dev,
@@ -1295,6 +1440,76 @@ int lcu_decode_experts_down(void* out_f32_dev, int ldo, const void* hidden_dev, 
   }
   LCU_LAUNCH_CHECK();
   return LCU_OK;
+}
+
+// ---- the same of a row that the launch works out ----
+
+int lcu_step_linear(void* out_f32_dev, const lcu_step_row* row, const void* w_dev, const void* bias_dev, int N, void* stream) {
+  const int rc = check_step_row("lcu_step_linear", row);
+  if (rc) return rc;
+  LCU_REQUIRE(out_f32_dev && w_dev && N > 0, "lcu_step_linear: bad arguments");
+  return launch_decode_rows(row, w_dev, row->ld, N, store_f32_row{(float*)out_f32_dev, (const float*)bias_dev}, as_stream(stream));
+}
+
+int lcu_step_linear_bf16(void* out_dev, const lcu_step_row* row, const void* w_dev, int N, void* stream) {
+  const int rc = check_step_row("lcu_step_linear_bf16", row);
+  if (rc) return rc;
+  LCU_REQUIRE(out_dev && w_dev && N > 0, "lcu_step_linear_bf16: bad arguments");
+  return launch_decode_rows(row, w_dev, row->ld, N, store_bf16_row{(bf16_t*)out_dev}, as_stream(stream));
+}
+
+int lcu_step_delta_in(void* u_dev, void* plain_dev, void* tail_f32_dev, void* conv_state_dev, const lcu_step_row* row, const void* w_dev,
+                      const void* conv_dev, int taps, int channels, int plain, int N, void* stream) {
+  const int rc = check_step_row("lcu_step_delta_in", row);
+  if (rc) return rc;
+  LCU_REQUIRE(u_dev && plain_dev && tail_f32_dev && w_dev && conv_dev && (conv_state_dev || taps == 1) && taps >= 1 && channels > 0 &&
+                  plain >= 0 && N >= channels + plain,
+              "lcu_step_delta_in: bad arguments");
+  return launch_decode_rows(row, w_dev, row->ld, N,
+                            delta_in_row{(bf16_t*)u_dev, (bf16_t*)plain_dev, (float*)tail_f32_dev, (bf16_t*)conv_state_dev,
+                                         (const float*)conv_dev, taps, channels, plain},
+                            as_stream(stream));
+}
+
+int lcu_step_gated(void* hidden_dev, const lcu_step_row* row, const void* w_dev, const lcu_gate_params* gate, int ld, void* stream) {
+  int rc = check_step_row("lcu_step_gated", row);
+  if (rc) return rc;
+  LCU_REQUIRE(hidden_dev && w_dev && gate && ld > 0 && ld % 32 == 0, "lcu_step_gated: bad arguments");
+  const step_row s = as_step_row(row);
+  const expert_up_tasks<1> tk{(const bf16_t*)w_dev, (bf16_t*)hidden_dev, {gate->limit, gate->alpha, gate->up_shift}, 1.0f, row->ld};
+  if (launch_normed_rows<2>(s, tk, ld, as_stream(stream))) {
+    LCU_LAUNCH_CHECK();
+    return LCU_OK;
+  }
+  rc = residual_step(s, as_stream(stream));
+  return rc ? rc : dense_gated(hidden_dev, s.h, w_dev, gate, ld, row->ld, as_stream(stream));
+}
+
+int lcu_step_recurrent_in(void* y_dev, void* u_dev, void* conv_state_dev, const lcu_step_row* row, const void* w_dev, const void* bias_dev,
+                          const void* conv_dev, const void* conv_bias_dev, int taps, int ld, void* stream) {
+  const int rc = check_step_row("lcu_step_recurrent_in", row);
+  if (rc) return rc;
+  LCU_REQUIRE(y_dev && u_dev && w_dev && bias_dev && conv_dev && conv_bias_dev && (conv_state_dev || taps == 1) && taps >= 1 && ld > 0,
+              "lcu_step_recurrent_in: bad arguments");
+  return launch_decode_rows(row, w_dev, row->ld, 2 * ld,
+                            conv_step_row{(bf16_t*)y_dev, (bf16_t*)u_dev, (bf16_t*)conv_state_dev, (const float*)bias_dev,
+                                          (const float*)conv_dev, (const float*)conv_bias_dev, taps, ld},
+                            as_stream(stream));
+}
+
+int lcu_step_kv(void* q_out_dev, void* k_cache_dev, void* v_cache_dev, const lcu_step_row* row, const void* w_dev, const void* bias_dev,
+                int q_cols, int k_cols, int v_cols, void* v_first_dev, int v_mode, const void* lambda_dev, const void* pos_dev,
+                int max_positions, void* stream) {
+  const int rc = check_step_row("lcu_step_kv", row);
+  if (rc) return rc;
+  LCU_REQUIRE(q_out_dev && k_cache_dev && v_cache_dev && w_dev && bias_dev && pos_dev && (v_mode == 0 || v_first_dev) &&
+                  (v_mode != 2 || lambda_dev) && v_mode >= 0 && v_mode <= 2 && max_positions > 0 && q_cols + k_cols + v_cols > 0,
+              "lcu_step_kv: bad arguments");
+  return launch_decode_rows(row, w_dev, row->ld, q_cols + k_cols + v_cols,
+                            qkv_row{(bf16_t*)q_out_dev, (bf16_t*)k_cache_dev, (bf16_t*)v_cache_dev, (bf16_t*)v_first_dev,
+                                    (const float*)bias_dev, (const float*)lambda_dev, (const int*)pos_dev, q_cols, k_cols, v_cols,
+                                    v_mode, max_positions},
+                            as_stream(stream));
 }
 
 #ifdef LCU_PHASE_TIMELINE

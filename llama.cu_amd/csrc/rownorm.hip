@@ -41,27 +41,6 @@ __global__ __launch_bounds__(TH) void embed_pos_norm_kernel(float* __restrict__ 
   store_row(h + (size_t)r * rs.ld, row, rs);
 }
 
-// what sublayers left for row r: its rows of src.out, and the shared expert's row times its gate
-template <int NV, int TH>
-__device__ __forceinline__ void load_sum(row_t<NV, TH>& m, row_t<NV, TH>& t, const sublayer_rows& src, int r, const row_shape& rs) {
-  const auto from = [&](int k) {
-    const size_t at = (size_t)r * src.top + k;
-    return src.out + (src.inverse ? (size_t)src.inverse[at] : at) * rs.ld;
-  };
-  load_row(m, from(0), rs);
-  for (int k = 1; k < src.top; ++k) {
-    load_row(t, from(k), rs);
-#pragma unroll
-    for (int j = 0; j < NV; ++j) m.v[j] += t.v[j];
-  }
-  if (src.shared) {
-    const float f = src.shared_gate[r];
-    load_row(t, src.shared + (size_t)r * rs.ld, rs);
-#pragma unroll
-    for (int j = 0; j < NV; ++j) m.v[j] += f * t.v[j];
-  }
-}
-
 // m = the sublayer's result; x += norm(m) under w_after; h = x, its norm under w_next when given.
 template <class T, int NV, int TH>
 __global__ __launch_bounds__(TH) void residual_norm_kernel(float* __restrict__ x, T* __restrict__ h,
@@ -90,7 +69,7 @@ __global__ __launch_bounds__(TH) void residual_norm_kernel(float* __restrict__ x
 // takes rows of the router's matrix (its first two asked for before the norms are worked out), the first one
 // then chooses.
 template <int NV>
-__global__ __launch_bounds__(STEP_THREADS) void residual_step_kernel(float* __restrict__ x, bf16_t* __restrict__ h, sublayer_rows src,
+__global__ __launch_bounds__(STEP_THREADS) void residual_step_kernel(const float* x, float* x_out, bf16_t* __restrict__ h, sublayer_rows src,
                                                                      const float* __restrict__ w_after,
                                                                      const float* __restrict__ w_next, row_shape rs, router_step rt) {
   constexpr int TH = STEP_THREADS, AHEAD = 8;  // 16-byte pieces of a router row a lane asks for ahead: 4096 columns
@@ -114,7 +93,7 @@ __global__ __launch_bounds__(STEP_THREADS) void residual_step_kernel(float* __re
   scale_row(m, rs, lds, after);
 #pragma unroll
   for (int j = 0; j < NV; ++j) m.v[j] += old.v[j];
-  store_row(x, m, rs);
+  store_row(x_out, m, rs);
   if (!h) return;
   if (w_next) scale_row(m, rs, lds, next);
   store_row(h, m, rs);
@@ -281,6 +260,31 @@ int check_rows(const char* who, int dtype, int rows, const row_shape& rs) {
 
 }  // namespace
 
+namespace lcu {
+
+int check_step_row(const char* who, const lcu_step_row* r) {
+  LCU_REQUIRE(r && r->x_dev && r->x_out_dev && r->h_dev && r->out_f32_dev && r->w_after_dev && (!r->shared_f32_dev || r->shared_gate_dev),
+              "%s: null pointer", who);
+  LCU_REQUIRE(r->top >= 1, "%s: %d rows", who, r->top);
+  const int rc = check_rows(who, LCU_BF16, 1, row_shape{r->width, r->ld, r->groups, r->eps});
+  if (rc) return rc;
+  const char *x = (const char*)r->x_dev, *out = (const char*)r->x_out_dev;
+  const size_t bytes = (size_t)r->ld * 4;
+  LCU_REQUIRE(out + bytes <= x || x + bytes <= out, "%s: x_out overlaps x", who);
+  return LCU_OK;
+}
+
+int residual_step(const step_row& s, hipStream_t stream) {
+  with_step_pieces(s.rs.ld, [&](auto nv) {
+    residual_step_kernel<decltype(nv)::value><<<1, STEP_THREADS, row_lds_bytes(s.rs), stream>>>(s.x, s.x_out, s.h, s.src, s.w_after, s.w_next,
+                                                                                               s.rs, router_step{});
+  });
+  LCU_LAUNCH_CHECK();
+  return LCU_OK;
+}
+
+}  // namespace lcu
+
 extern "C" {
 
 int lcu_embed_pos_norm(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, const void* table_dev, int n_vocab,
@@ -368,7 +372,7 @@ int lcu_decode_residual_router(void* x_dev, void* h_dev, const void* out_f32_dev
   if (router_w_dev && lds < (size_t)ld * 2) lds = (size_t)ld * 2;
   with_step_pieces(ld, [&](auto nv) {
     residual_step_kernel<decltype(nv)::value><<<1, STEP_THREADS, lds, as_stream(stream)>>>(
-        (float*)x_dev, (bf16_t*)h_dev, src, (const float*)w_after_dev, (const float*)w_next_dev, rs, rt);
+        (const float*)x_dev, (float*)x_dev, (bf16_t*)h_dev, src, (const float*)w_after_dev, (const float*)w_next_dev, rs, rt);
   });
   LCU_LAUNCH_CHECK();
   return LCU_OK;

@@ -68,12 +68,74 @@ __device__ __forceinline__ void store_row(T* p, const row_t<NV, TH>& r, const ro
   }
 }
 
+// what sublayers left for row r: its rows of src.out, and the shared expert's row times its gate
+template <int NV, int TH>
+__device__ __forceinline__ void load_sum(row_t<NV, TH>& m, row_t<NV, TH>& t, const sublayer_rows& src, int r, const row_shape& rs) {
+  const auto from = [&](int k) {
+    const size_t at = (size_t)r * src.top + k;
+    return src.out + (src.inverse ? (size_t)src.inverse[at] : at) * rs.ld;
+  };
+  load_row(m, from(0), rs);
+  for (int k = 1; k < src.top; ++k) {
+    load_row(t, from(k), rs);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) m.v[j] += t.v[j];
+  }
+  if (src.shared) {
+    const float f = src.shared_gate[r];
+    load_row(t, src.shared + (size_t)r * rs.ld, rs);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) m.v[j] += f * t.v[j];
+  }
+}
+
+// The row between two sublayers of a one-token step: x_out = x + norm(src) under w_after; what follows reads its norm under
+// w_next (itself when NULL), in bfloat16.
+struct step_row {
+  const float* x;
+  float* x_out;  // x, or a row that does not overlap it
+  bf16_t* h;
+  sublayer_rows src;
+  const float* w_after;
+  const float* w_next;
+  row_shape rs;
+};
+int residual_step(const step_row& s, hipStream_t stream);  // a launch of one workgroup (rownorm.hip)
+int check_step_row(const char* who, const lcu_step_row* row);
+inline step_row as_step_row(const lcu_step_row* r) {
+  return {(const float*)r->x_dev, (float*)r->x_out_dev, (bf16_t*)r->h_dev,
+          {(const float*)r->out_f32_dev, nullptr, r->top, (const float*)r->shared_f32_dev, (const float*)r->shared_gate_dev},
+          (const float*)r->w_after_dev, (const float*)r->w_next_dev, {r->width, r->ld, r->groups, r->eps}};
+}
+
 // LDS a workgroup needs for scale_row
 inline size_t row_lds_bytes(const row_shape& rs) {
   const size_t quads = (size_t)rs.ld / 4;                        // general form: a partial sum per four columns ...
   const size_t pieces = (rs.ld + ROW_PIECE - 1) / ROW_PIECE;     // ... or one per piece of a wavefront
   const bool whole = rs.width % rs.groups == 0 && (rs.width / rs.groups) % ROW_PIECE == 0;
   return ((whole ? pieces : quads * 4) + rs.groups) * sizeof(float);
+}
+
+// p[0] + p[1] + ... in that order, sixteen (four) asked for at a time
+__device__ __forceinline__ float sum_of_pieces(const float* p, int count) {
+  float total = 0.0f;
+  int k = 0;
+  for (; k + 16 <= count; k += 16) {
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = p[k + i];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) total += v[i];
+  }
+  for (; k + 8 <= count; k += 8) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = p[k + i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) total += v[i];
+  }
+  for (; k < count; ++k) total += p[k];
+  return total;
 }
 
 // row <- row / sqrt(mean of its part's squares + eps) * w.  Parts that are whole pieces of a wavefront (256
@@ -97,8 +159,7 @@ __device__ __forceinline__ void scale_row(row_t<NV, TH>& r, const row_shape& rs,
     for (int j = 0; j < NV; ++j) {
       const int g = __builtin_amdgcn_readfirstlane((j * WAVES + wave) / per);
       if (g < rs.groups) {
-        float total = 0.0f;
-        for (int k = 0; k < per; ++k) total += piece[g * per + k];
+        const float total = sum_of_pieces(piece + g * per, per);
         r.v[j] *= (1.0f / sqrtf(total / (float)part + rs.eps)) * w.v[j];
       }
     }

@@ -94,6 +94,7 @@ layered_context_impl::layered_context_impl(layered_model_impl* model, int contex
   const size_t ld = m.ld;
   t_x_ = zeroed(R * ld * 4);
   t_h_ = zeroed(R * ld * e);
+  t_x_next_ = zeroed(ld * 4);
   t_m_ = zeroed(R * ld * 4);
   t_wide_ = zeroed(R * wide * e);
   t_u_ = zeroed(R * u * e);
@@ -167,7 +168,7 @@ size_t layered_context_impl::context_memory_usage() {
   size_t count = 0;
   for (layer_state const& s : state_) count += s.k.size() + s.v.size() + s.conv.size() + s.s.size();
   for (gpu_buffer const* b :
-       {&t_low_, &t_queries_, &t_latent_queries_, &t_keys_values_, &t_tail_, &t_x_, &t_h_, &t_m_, &t_wide_, &t_u_, &t_rec_, &t_scratch_, &t_hidden_, &t_shared_hidden_, &t_expert_out_, &t_shared_out_,
+       {&t_low_, &t_queries_, &t_latent_queries_, &t_keys_values_, &t_tail_, &t_x_, &t_x_next_, &t_h_, &t_m_, &t_wide_, &t_u_, &t_rec_, &t_scratch_, &t_hidden_, &t_shared_hidden_, &t_expert_out_, &t_shared_out_,
         &t_v_first_, &t_choice_, &t_weight_, &t_shared_gate_, &t_row_token_, &t_row_weight_, &t_inverse_, &t_tile_expert_,
         &t_tile_row_, &t_expert_end_, &t_n_tiles_, &t_arrived_, &t_step_, &t_want_, &t_head_in_, &t_logits_, &t_probs_, &t_index_}) {
     count += b->size();
@@ -209,7 +210,9 @@ void layered_context_impl::latent(latent_weights const& w, latent_params const& 
   layered_model_impl const& m = *model_;
   const lcu_latent_params lp = latent_shape(w, p);
   const auto product = [&](gpu_buffer& out, gpu_buffer const& x, gpu_buffer const& weight, int K, int N) {
-    if (fused) {
+    if (fused && &x == &t_h_ && row_.x_dev) {
+      LCU_CHECK(lcu_step_linear_bf16(out.data(), &row_, weight.data(), N, stream_));
+    } else if (fused) {
       LCU_CHECK(lcu_decode_linear_bf16(out.data(), x.data(), weight.data(), K, N, stream_));
     } else {
       LCU_CHECK(lcu_linear(out.data(), 0, N, x.data(), weight.data(), nullptr, 0, m.dtype, n, K, N, stream_));
@@ -297,8 +300,13 @@ void layered_context_impl::delta(delta_weights const& w, delta_params const& p, 
 void layered_context_impl::decode_delta(delta_weights const& w, delta_params const& p, layer_state& s) {
   layered_model_impl const& m = *model_;
   const lcu_delta_params d = delta_shape(w, p);
-  LCU_CHECK(lcu_decode_delta_in(t_u_.data(), t_wide_.data(), t_tail_.data(), s.conv.data(), t_h_.data(), w.in.data(), w.conv.data(), p.taps,
-                                m.ld, w.channels, w.plain, w.rows, stream_));
+  if (row_.x_dev) {
+    LCU_CHECK(lcu_step_delta_in(t_u_.data(), t_wide_.data(), t_tail_.data(), s.conv.data(), &row_, w.in.data(), w.conv.data(), p.taps,
+                                w.channels, w.plain, w.rows, stream_));
+  } else {
+    LCU_CHECK(lcu_decode_delta_in(t_u_.data(), t_wide_.data(), t_tail_.data(), s.conv.data(), t_h_.data(), w.in.data(), w.conv.data(),
+                                  p.taps, m.ld, w.channels, w.plain, w.rows, stream_));
+  }
   LCU_CHECK(lcu_decode_delta_step(t_rec_.data(), t_u_.data(), t_wide_.data(), t_tail_.data(), &d, s.s.data(), stream_));
   LCU_CHECK(lcu_decode_linear(t_m_.data(), t_rec_.data(), w.out.data(), nullptr, w.ldo, m.shape.width, stream_));
 }
@@ -379,17 +387,26 @@ void layered_context_impl::enqueue_rows(int n) {
   }
 }
 
+void layered_context_impl::pend_row(const void* out, int top, const void* shared, const void* shared_gate, const void* w_after,
+                                    const void* w_next) {
+  layered_params const& p = model_->shape;
+  void* x = row_.x_out_dev ? row_.x_out_dev : t_x_.data();  // the row that the last pending one became
+  row_ = lcu_step_row{x, x == t_x_.data() ? t_x_next_.data() : t_x_.data(), t_h_.data(), out, shared, shared_gate, w_after, w_next, top,
+                      p.width, model_->ld, p.norm_groups, p.norm_eps};
+}
+
 // One token: launches fused around the weight streams.  A recurrent layer's mixer takes three (projections
 // with the convolution, gates with the state, output product), an attention layer's too (projections with the
 // cache rows, attention, output product), a latent layer's four (projections; keys applied to the queries, with norm,
 // rotations and cache rows; scores and values, two launches beyond short_positions_; output product; two more with a queries' latent), a feed-forward two
-// (first products, second products); between sublayers one launch adds the result, takes both norms and, in front of a feed-forward, routes.  The last
-// layer's norms end in the final one.
+// (first products, second products).  Between sublayers the product that reads the row adds the result and takes both norms
+// by itself (row_); in front of experts, where the router needs the row, a launch does.  The last layer's norms end in the final one.
 void layered_context_impl::enqueue_one() {
   layered_model_impl const& m = *model_;
   layered_params const& p = m.shape;
   const size_t n_layers = m.layers.size();
   const auto norm_ahead = [&](size_t l) { return l < n_layers ? m.layers[l].norm1.data() : m.final_norm.data(); };
+  row_ = lcu_step_row{};
   embed(1, norm_ahead(0));
   for (size_t l = 0; l < n_layers; ++l) {
     layer_params const& q = p.layers[l];
@@ -397,8 +414,13 @@ void layered_context_impl::enqueue_one() {
     layer_state& s = state_[l];
     if (q.mixer == mixer_type::rglru) {
       recurrence_weights const& w = L.recurrence;
-      LCU_CHECK(lcu_decode_recurrent_in(t_wide_.data(), t_u_.data(), s.conv.data(), t_h_.data(), w.yx.data(), w.yx_bias.data(),
-                                        w.conv.data(), w.conv_bias.data(), q.recurrence.taps, m.ld, w.ld, stream_));
+      if (row_.x_dev) {
+        LCU_CHECK(lcu_step_recurrent_in(t_wide_.data(), t_u_.data(), s.conv.data(), &row_, w.yx.data(), w.yx_bias.data(), w.conv.data(),
+                                        w.conv_bias.data(), q.recurrence.taps, w.ld, stream_));
+      } else {
+        LCU_CHECK(lcu_decode_recurrent_in(t_wide_.data(), t_u_.data(), s.conv.data(), t_h_.data(), w.yx.data(), w.yx_bias.data(),
+                                          w.conv.data(), w.conv_bias.data(), q.recurrence.taps, m.ld, w.ld, stream_));
+      }
       LCU_CHECK(lcu_decode_recurrent_step(t_rec_.data(), t_u_.data(), t_wide_.data(), w.gate_r.data(), w.gate_i.data(), w.bias_r.data(),
                                           w.bias_i.data(), w.decay.data(), s.s.data(), w.channels, w.block, stream_));
       LCU_CHECK(lcu_decode_linear(t_m_.data(), t_rec_.data(), w.out.data(), nullptr, w.ld, p.width, stream_));
@@ -410,36 +432,40 @@ void layered_context_impl::enqueue_one() {
       attention_weights const& w = L.attention;
       attention_params const& a = q.attention;
       const lcu_window_params window{a.heads, a.kv_heads, w.dk, w.dv, a.window, a.keep_first, a.scale, w.r1.data(), w.r2.data()};
-      LCU_CHECK(lcu_decode_kv(t_wide_.data(), s.k.data(), s.v.data(), t_h_.data(), w.qkv.data(), w.qkv_bias.data(), w.q_cols, w.k_cols,
-                              w.v_cols, t_v_first_.data(), w.v_mode, w.v_mix.data(), start(), context_len_, m.ld, stream_));
+      if (row_.x_dev) {
+        LCU_CHECK(lcu_step_kv(t_wide_.data(), s.k.data(), s.v.data(), &row_, w.qkv.data(), w.qkv_bias.data(), w.q_cols, w.k_cols, w.v_cols,
+                              t_v_first_.data(), w.v_mode, w.v_mix.data(), start(), context_len_, stream_));
+      } else {
+        LCU_CHECK(lcu_decode_kv(t_wide_.data(), s.k.data(), s.v.data(), t_h_.data(), w.qkv.data(), w.qkv_bias.data(), w.q_cols, w.k_cols,
+                                w.v_cols, t_v_first_.data(), w.v_mode, w.v_mix.data(), start(), context_len_, m.ld, stream_));
+      }
       LCU_CHECK(lcu_attention_windowed_decode(t_rec_.data(), t_wide_.data(), s.k.data(), s.v.data(), start(), context_len_, &window,
                                               t_arrived_.data(), stream_));
       LCU_CHECK(lcu_decode_linear(t_m_.data(), t_rec_.data(), w.out.data(), w.out_bias.data(), w.ldo, p.width, stream_));
     }
-    experts_weights const& w = L.mlp;
-    const bool shared = q.has_mlp && q.mlp.shared_ff > 0;
-    LCU_CHECK(lcu_decode_residual_router(t_x_.data(), t_h_.data(), t_m_.data(), 1, nullptr, nullptr, L.norm1b.data(),
-                                         q.has_mlp ? L.norm2.data() : norm_ahead(l + 1), p.width, m.ld, p.norm_groups, p.norm_eps,
-                                         w.router.data(), q.mlp.experts, q.mlp.top, t_choice_.data(), t_weight_.data(),
-                                         shared ? t_shared_gate_.data() : nullptr, stream_));
+    pend_row(t_m_.data(), 1, nullptr, nullptr, L.norm1b.data(), q.has_mlp ? L.norm2.data() : norm_ahead(l + 1));
     if (q.dense.ff > 0) {
-      LCU_CHECK(lcu_decode_gated(t_shared_hidden_.data(), t_h_.data(), L.dense.up.data(), &q.dense.gate, L.dense.ld, m.ld, stream_));
+      LCU_CHECK(lcu_step_gated(t_shared_hidden_.data(), &row_, L.dense.up.data(), &q.dense.gate, L.dense.ld, stream_));
       LCU_CHECK(lcu_decode_linear(t_m_.data(), t_shared_hidden_.data(), L.dense.down.data(), nullptr, L.dense.ld, p.width, stream_));
-      LCU_CHECK(lcu_decode_residual_router(t_x_.data(), t_h_.data(), t_m_.data(), 1, nullptr, nullptr, L.norm2b.data(), norm_ahead(l + 1),
-                                           p.width, m.ld, p.norm_groups, p.norm_eps, nullptr, 0, 0, nullptr, nullptr, nullptr, stream_));
+      pend_row(t_m_.data(), 1, nullptr, nullptr, L.norm2b.data(), norm_ahead(l + 1));
     } else if (q.has_mlp) {
+      experts_weights const& w = L.mlp;
+      const bool shared = q.mlp.shared_ff > 0;
+      row_.x_out_dev = const_cast<void*>(row_.x_dev);  // this launch, of one workgroup, works in place
+      LCU_CHECK(lcu_decode_residual_router(row_.x_out_dev, t_h_.data(), t_m_.data(), 1, nullptr, nullptr, L.norm1b.data(), L.norm2.data(),
+                                           p.width, m.ld, p.norm_groups, p.norm_eps, w.router.data(), q.mlp.experts, q.mlp.top,
+                                           t_choice_.data(), t_weight_.data(), shared ? t_shared_gate_.data() : nullptr, stream_));
       LCU_CHECK(lcu_decode_experts_up(t_hidden_.data(), t_shared_hidden_.data(), t_h_.data(), t_choice_.data(), t_weight_.data(),
                                       w.up.data(), w.up_stride, &q.mlp.gate, w.shared_up.data(), &q.mlp.shared_gate, q.mlp.top, w.ld,
                                       w.shared_ld, m.ld, stream_));
       LCU_CHECK(lcu_decode_experts_down(t_expert_out_.data(), m.ld, t_hidden_.data(), t_choice_.data(), w.down.data(), w.down_stride,
                                         q.mlp.top, w.ld, t_shared_hidden_.data(), w.shared_down.data(), w.shared_ld, p.width, stream_));
       const float* shared_row = (float*)t_expert_out_.data() + (size_t)q.mlp.top * m.ld;
-      LCU_CHECK(lcu_decode_residual_router(t_x_.data(), t_h_.data(), t_expert_out_.data(), q.mlp.top, shared ? shared_row : nullptr,
-                                           shared ? t_shared_gate_.data() : nullptr, L.norm2b.data(), norm_ahead(l + 1), p.width, m.ld,
-                                           p.norm_groups, p.norm_eps, nullptr, 0, 0, nullptr, nullptr, nullptr, stream_));
+      pend_row(t_expert_out_.data(), q.mlp.top, shared ? shared_row : nullptr, shared ? t_shared_gate_.data() : nullptr, L.norm2b.data(),
+               norm_ahead(l + 1));
     }
   }
-  LCU_CHECK(lcu_decode_linear(t_logits_.data(), t_h_.data(), m.head.data(), nullptr, m.ld, p.vocab, stream_));
+  LCU_CHECK(lcu_step_linear(t_logits_.data(), &row_, m.head.data(), nullptr, p.vocab, stream_));
   LCU_CHECK(lcu_argmax_f32(t_index_.data(), t_logits_.data(), p.vocab, stream_));
 }
 

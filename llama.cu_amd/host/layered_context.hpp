@@ -42,6 +42,8 @@ struct layered_context_impl final : public llama_context {
   void embed(int n, void* w_next);
   lcu_delta_params delta_shape(delta_weights const& w, delta_params const& p) const;
   void enqueue_head(int n_rows);
+  // one-token steps: leaves a sublayer's result (the sum of `top` rows and a gated one) to the product that reads the row next
+  void pend_row(const void* out, int top, const void* shared, const void* shared_gate, const void* w_after, const void* w_next);
   void* next_norm(size_t layer) const;             // weights of the norm in front of layer `layer`, or NULL
 
   layered_model_impl* model_;
@@ -60,6 +62,8 @@ struct layered_context_impl final : public llama_context {
   float* last_logits() const { return (float*)t_logits_.data() + last_logits_row_ * model_->shape.vocab; }
   int want_cap_{0};
   lcu_expert_plan plan_{};
+  gpu_buffer t_x_next_;                            // one-token steps: the residual row goes to and fro between t_x_ and this
+  lcu_step_row row_{};                             // one-token steps: the pending row
   bool fused_step_{true};                          // one-token steps in bfloat16 take enqueue_one
   bool recording_{false};
   std::vector<std::vector<float>> residual_;

@@ -479,3 +479,45 @@ def test_unsupported_shapes_are_refused_before_any_launch(gpu):
     assert L.lcu_latent_attention(a, 64, a, a, 64, a, None, a, 8, a, None, None, 0, C.byref(p), a, 1, gpu.stream) == -2
     assert L.lcu_linear_tail(a, 64, a, 2, 64, a, a, 0, 1, 64, 64, gpu.stream) == -2              # no column is left for the tail
     gpu.release()
+
+
+@pytest.mark.parametrize("width,groups,N,top", [(40, 1, 1, 1), (192, 2, 70, 1), (512, 2, 513, 3), (1000, 8, 700, 1), (1024, 1, 2048, 2), (1088, 1, 300, 1),
+                                                (2048, 8, 1281, 1), (2048, 1, 8500, 1), (2048, 1, 16500, 1), (2112, 1, 90, 2)])
+def test_products_of_a_row_worked_out_on_the_way(gpu, width, groups, N, top):
+    """Residual, both norms and the product in one launch (two beyond its range): the bits of lcu_decode_residual_router and the
+    product by themselves, for every product that reads such a row, with all that it writes."""
+    rng = np.random.default_rng(width + N)
+    ld, eps, taps, rows = up64(width), 1e-6, 4, 2 * up64(N)
+    L32, third = up32(N), max(1, N // 3)
+    kc = (N - third) // 2
+    x0 = pad(rng.standard_normal(width), ld).astype(np.float32)
+    out, shared, gate = put(gpu, pad(rng.standard_normal((top, width)), ld)), put(gpu, pad(rng.standard_normal(width), ld)), put(gpu, np.array([0.7]))
+    more = (shared, gate) if top > 1 else (None, None)
+    w1, w2 = (put(gpu, pad(1 + 0.1 * rng.standard_normal(width), ld)) for _ in range(2))
+    w = put(gpu, pad(rng.standard_normal((509, width)) / width ** 0.5, ld)[np.arange(rows) % 509], BF16)
+    bias, conv, lam, pos = put(gpu, rng.standard_normal(rows)), put(gpu, rng.standard_normal((taps, rows))), put(gpu, np.array([0.3])), ints(gpu, [2])
+    gp = gpu.B.GateParams(7.0, 1.0, 0.0)
+    # the row and its length, if any, between what a product writes and the rest of its arguments
+    products = {"linear": lambda b, x, k: (b[0], x, w, bias, *k, N), "linear_bf16": lambda b, x, k: (b[0], x, w, *k, N),
+                "gated": lambda b, x, k: (b[0], x, w, C.byref(gp), L32, *k),
+                "delta_in": lambda b, x, k: (*b, x, w, conv, taps, *k, third, kc, N),
+                "recurrent_in": lambda b, x, k: (b[0], b[1], b[3], x, w, bias, conv, bias, taps, *k, N),
+                "kv": lambda b, x, k: (*b[:3], x, w, bias, third, kc, N - third - kc, b[3], 2, lam, pos, 3, *k)}
+    for name, arguments in products.items():
+        results = []
+        for step in (False, True):
+            buffers, x, x2, h = [zeros(gpu, (taps, rows)) for _ in range(4)], put(gpu, x0), put(gpu, x0), zeros(gpu, ld, BF16)
+            if step:
+                row = gpu.B.StepRow(x.ptr, x2.ptr, h.ptr, out.ptr, *(m and m.ptr for m in more), w1.ptr, w2.ptr, top, width, ld, groups, eps)
+                call(gpu, "lcu_step_" + name, *arguments(buffers, C.byref(row), ()))
+                assert (get(gpu, x, (ld,)) == x0).all()
+            else:
+                call(gpu, "lcu_decode_residual_router", x2, h, out, top, *more, w1, w2, width, ld, groups, eps, None, 0, 0, None, None, None)
+                call(gpu, "lcu_decode_" + name, *arguments(buffers, h, (ld,)))
+            gpu.B.check(gpu.L().lcu_sync(gpu.stream))
+            results.append([gpu.host(b, (taps, rows), np.uint32) for b in buffers] + [gpu.host(x2, (ld,), np.uint32)])
+        for got, want in zip(*results):
+            assert np.array_equal(got, want), name
+    row.x_out = x.ptr + 4 * (ld - 1)  # a workgroup would read what another has written
+    assert gpu.L().lcu_step_linear_bf16(h.ptr, C.byref(row), w.ptr, N, gpu.stream) == -2
+    gpu.release()
