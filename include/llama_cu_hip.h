@@ -53,6 +53,10 @@ int lcu_get_device(int* out_device);                                            
 int lcu_set_device(int device);
 int lcu_malloc(void** out_dev, size_t bytes);                                   /* gpu_buffer ctor, 712-715 */
 int lcu_free(void* dev);                                                        /* gpu_buffer dtor, 732-736 */
+/* page-locked host memory that kernels read and write; lcu_fetch: a launch copies `bytes` (a multiple of 4) of it to the device */
+int lcu_host_alloc(void** out_host, size_t bytes);
+int lcu_host_free(void* host);
+int lcu_fetch(void* dst_dev, const void* src_host, size_t bytes, void* stream);
 int lcu_memset(void* dev, int byte_value, size_t bytes, void* stream);          /* llama_cu.h:239-241 */
 /* the first `bytes` (a multiple of 16) of `count` buffers in one launch: buffers_dev is a device array of their
  * addresses, each on a 16-byte boundary */
@@ -151,6 +155,11 @@ int lcu_embed_u8(void* out_dev, const void* ids_dev, int n_ids, int dim, const v
 int lcu_embed_rmsnorm(void* x_out_dev, void* norm_out_dev, const void* ids_dev, int n_ids, int dim,
                       const void* table_dev, const void* scales_dev, int block, int n_vocab,
                       const void* weights_dev, float eps, void* stream);
+/* the same for a one-token step whose state (at most 1024 bytes, a multiple of 4) lies in page-locked memory, the token's id in it at
+ * id_host: the launch copies the state to state_dev as well */
+int lcu_step_embed_rmsnorm(void* state_dev, const void* state_host, size_t state_bytes, void* x_out_dev, void* norm_out_dev,
+                           const void* id_host, int dim, const void* table_dev, const void* scales_dev, int block, int n_vocab,
+                           const void* weights_dev, float eps, void* stream);
 /* the host argmax of llama_cu.cu:1205-1209 done on the device: index of the first maximum of n
  * fp16 values compared as float, written as int32 */
 int lcu_argmax_f16(void* out_index_dev, const void* values_dev, int n, void* stream);
@@ -391,6 +400,11 @@ int lcu_embed_pos_norm(void* x_dev, void* h_dev, const void* ids_i32_dev, int n_
                        const void* w_next_dev, int dtype, int width, int ld, int groups, float eps, void* stream);
 int lcu_embed_scaled(void* x_dev, void* h_dev, const void* ids_i32_dev, int n_ids, const void* table_dev, int n_vocab, float scale,
                      const void* w_next_dev, int dtype, int width, int ld, int groups, float eps, void* stream);
+/* lcu_embed_pos_norm (pos_table given; scale is ignored) or lcu_embed_scaled of one token whose int32 position and id lie in page-locked
+ * memory at state_host; the launch copies both to state_dev */
+int lcu_step_embed(void* state_dev, const void* state_host, void* x_dev, void* h_dev, const void* table_dev, int n_vocab, float scale,
+                   const void* pos_table_dev, int n_pos, const void* w_embed_dev, const void* w_next_dev, int dtype, int width, int ld,
+                   int groups, float eps, void* stream);
 int lcu_residual_norm(void* x_dev, void* h_dev, const void* out_f32_dev, const void* inverse_dev, int top,
                       const void* shared_f32_dev, const void* shared_gate_dev, const void* w_after_dev,
                       const void* w_next_dev, int dtype, int rows, int width, int ld, int groups, float eps, void* stream);

@@ -36,6 +36,9 @@ SIGNATURES = {
     "lcu_set_device": (i32, [i32]),
     "lcu_malloc": (i32, [C.POINTER(vp), sz]),
     "lcu_free": (i32, [vp]),
+    "lcu_host_alloc": (i32, [C.POINTER(vp), sz]),
+    "lcu_host_free": (i32, [vp]),
+    "lcu_fetch": (i32, [vp, vp, sz, vp]),
     "lcu_memset": (i32, [vp, i32, sz, vp]),
     "lcu_memset_many": (i32, [vp, i32, i32, sz, vp]),
     "lcu_h2d": (i32, [vp, vp, sz, vp]),
@@ -102,6 +105,8 @@ SIGNATURES = {
     "lcu_experts_plan": (i32, [vp, vp, vp, i32, i32, i32, vp]),
     "lcu_experts_up": (i32, [vp, i32, vp, vp, sz, vp, vp, i32, i32, i32, i32, vp]),
     "lcu_experts_down": (i32, [vp, i32, vp, vp, sz, vp, i32, i32, i32, i32, vp]),
+    "lcu_step_embed_rmsnorm": (i32, [vp, vp, sz, vp, vp, vp, i32, vp, vp, i32, i32, vp, f32, vp]),
+    "lcu_step_embed": (i32, [vp, vp, vp, vp, vp, i32, f32, vp, i32, vp, vp, i32, i32, i32, i32, f32, vp]),
     "lcu_embed_pos_norm": (i32, [vp, vp, vp, i32, vp, i32, vp, i32, vp, vp, vp, i32, i32, i32, i32, f32, vp]),
     "lcu_embed_scaled": (i32, [vp, vp, vp, i32, vp, i32, f32, vp, i32, i32, i32, i32, f32, vp]),
     "lcu_residual_norm": (i32, [vp, vp, vp, vp, i32, vp, vp, vp, vp, i32, i32, i32, i32, i32, f32, vp]),

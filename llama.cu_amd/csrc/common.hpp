@@ -80,6 +80,18 @@ constexpr int SYNC_WORDS = SYNC_EXCHANGE + (EXCH_PROJ + 4096) * 2;
 constexpr int SYNC_TIMEOUTS = SYNC_EXCHANGE - 1;  // word that counts bounded waits which ran out
 workspace_t workspace_for(hipStream_t stream);
 
+// What a one-token step takes from the host: the first launch of a step, which needs a word of it anyway, copies it out of page-locked
+// memory for the launches behind (a launch for that alone: 2.5 us of every step).  words 0: nothing.
+struct step_fetch {
+  uint32_t* dst;
+  const uint32_t* src;
+  int words;  // at most the threads of a workgroup
+  __device__ __forceinline__ void operator()() const {
+    if (blockIdx.x == 0 && (int)threadIdx.x < words) dst[threadIdx.x] = src[threadIdx.x];
+  }
+};
+constexpr size_t STEP_FETCH_MAX = 256 * 4;  // bytes
+
 // fp32 -> fp16, round to nearest even, as a separate step.  Written through an opaque register so
 // the compiler cannot merge the conversion into the preceding multiply or fused multiply-add
 // (v_fma_mixlo_f16 rounds the exact result once to fp16; the reference rounds to fp32 first, and a

@@ -534,10 +534,11 @@ __global__ __launch_bounds__(256) void embed_rmsnorm_kernel(half_t* __restrict__
                                                             const short* __restrict__ ids, int cols,
                                                             const void* __restrict__ table,
                                                             const half_t* __restrict__ scales, int block, int n_vocab,
-                                                            const half_t* __restrict__ weights, float eps) {
+                                                            const half_t* __restrict__ weights, float eps, step_fetch fetch) {
   extern __shared__ half_t xs[];
   __shared__ __attribute__((aligned(16))) float red[8];
   constexpr int P = 4;
+  fetch();
   half8_t wp[P];
 #pragma unroll
   for (int j = 0; j < P; ++j) {
@@ -1060,9 +1061,8 @@ int lcu_embed_u8(void* out_dev, const void* ids_dev, int n_ids, int dim, const v
   return LCU_OK;
 }
 
-int lcu_embed_rmsnorm(void* x_out_dev, void* norm_out_dev, const void* ids_dev, int n_ids, int dim,
-                      const void* table_dev, const void* scales_dev, int block, int n_vocab, const void* weights_dev,
-                      float eps, void* stream) {
+static int embed_rmsnorm(void* x_out_dev, void* norm_out_dev, const void* ids_dev, int n_ids, int dim, const void* table_dev,
+                         const void* scales_dev, int block, int n_vocab, const void* weights_dev, float eps, step_fetch fetch, void* stream) {
   LCU_REQUIRE(x_out_dev && norm_out_dev && ids_dev && table_dev && weights_dev, "lcu_embed_rmsnorm: null pointer");
   LCU_REQUIRE(n_ids >= 0 && dim > 0 && dim % 8 == 0 && dim <= 8192 && n_vocab > 0,
               "lcu_embed_rmsnorm: bad shape n %d dim %d (dim a multiple of 8, at most 8192)", n_ids, dim);
@@ -1073,14 +1073,29 @@ int lcu_embed_rmsnorm(void* x_out_dev, void* norm_out_dev, const void* ids_dev, 
   if (block > 0) {
     embed_rmsnorm_kernel<true><<<n_ids, 256, (size_t)dim * 2, as_stream(stream)>>>(
         (half_t*)x_out_dev, (half_t*)norm_out_dev, (const short*)ids_dev, dim, table_dev, (const half_t*)scales_dev, block,
-        n_vocab, (const half_t*)weights_dev, eps);
+        n_vocab, (const half_t*)weights_dev, eps, fetch);
   } else {
     embed_rmsnorm_kernel<false><<<n_ids, 256, (size_t)dim * 2, as_stream(stream)>>>(
         (half_t*)x_out_dev, (half_t*)norm_out_dev, (const short*)ids_dev, dim, table_dev, nullptr, 0, n_vocab,
-        (const half_t*)weights_dev, eps);
+        (const half_t*)weights_dev, eps, fetch);
   }
   LCU_LAUNCH_CHECK();
   return LCU_OK;
+}
+
+int lcu_embed_rmsnorm(void* x_out_dev, void* norm_out_dev, const void* ids_dev, int n_ids, int dim,
+                      const void* table_dev, const void* scales_dev, int block, int n_vocab, const void* weights_dev,
+                      float eps, void* stream) {
+  return embed_rmsnorm(x_out_dev, norm_out_dev, ids_dev, n_ids, dim, table_dev, scales_dev, block, n_vocab, weights_dev, eps, step_fetch{},
+                       stream);
+}
+
+int lcu_step_embed_rmsnorm(void* state_dev, const void* state_host, size_t state_bytes, void* x_out_dev, void* norm_out_dev,
+                           const void* id_host, int dim, const void* table_dev, const void* scales_dev, int block, int n_vocab,
+                           const void* weights_dev, float eps, void* stream) {
+  LCU_REQUIRE(state_dev && state_host && state_bytes % 4 == 0 && state_bytes <= STEP_FETCH_MAX, "lcu_step_embed_rmsnorm: bad state");
+  return embed_rmsnorm(x_out_dev, norm_out_dev, id_host, 1, dim, table_dev, scales_dev, block, n_vocab, weights_dev, eps,
+                       step_fetch{(uint32_t*)state_dev, (const uint32_t*)state_host, (int)(state_bytes / 4)}, stream);
 }
 
 int lcu_exp_f32(void* out_dev, const void* in_dev, size_t n, void* stream) {

@@ -19,9 +19,10 @@ __global__ __launch_bounds__(TH) void embed_pos_norm_kernel(float* __restrict__ 
                                                                      const int* __restrict__ ids, const T* __restrict__ table, float scale,
                                                                      const T* __restrict__ pos_table, const float* __restrict__ w0,
                                                                      const float* __restrict__ w1, const int* __restrict__ start,
-                                                                     int n_vocab, int n_pos, row_shape rs) {
+                                                                     int n_vocab, int n_pos, row_shape rs, step_fetch fetch) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int r = blockIdx.x;
+  fetch();
   const int id = min(max(ids[r], 0), n_vocab - 1);
   row_t<NV, TH> row, at, w, next;
   if (w0) load_row(w, w0, rs);
@@ -287,9 +288,9 @@ int residual_step(const step_row& s, hipStream_t stream) {
 
 extern "C" {
 
-int lcu_embed_pos_norm(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, const void* table_dev, int n_vocab,
-                       const void* pos_table_dev, int n_pos, const void* start_dev, const void* w_embed_dev,
-                       const void* w_next_dev, int dtype, int width, int ld, int groups, float eps, void* stream) {
+static int embed_pos_norm(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, const void* table_dev, int n_vocab,
+                          const void* pos_table_dev, int n_pos, const void* start_dev, const void* w_embed_dev, const void* w_next_dev,
+                          int dtype, int width, int ld, int groups, float eps, step_fetch fetch, void* stream) {
   LCU_REQUIRE(x_dev && ids_dev && table_dev && pos_table_dev && start_dev && w_embed_dev && (h_dev || !w_next_dev),
               "lcu_embed_pos_norm: null pointer");
   const row_shape rs{width, ld, groups, eps};
@@ -302,14 +303,14 @@ int lcu_embed_pos_norm(void* x_dev, void* h_dev, const void* ids_dev, int n_ids,
     using T = std::remove_pointer_t<decltype(kind)>;
     embed_pos_norm_kernel<T, decltype(nv)::value, decltype(th)::value><<<n_ids, decltype(th)::value, row_lds_bytes(rs), st>>>(
         (float*)x_dev, (T*)h_dev, (const int*)ids_dev, (const T*)table_dev, 1.0f, (const T*)pos_table_dev, (const float*)w_embed_dev,
-        (const float*)w_next_dev, (const int*)start_dev, n_vocab, n_pos, rs);
+        (const float*)w_next_dev, (const int*)start_dev, n_vocab, n_pos, rs, fetch);
   });
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
 
-int lcu_embed_scaled(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, const void* table_dev, int n_vocab, float scale,
-                     const void* w_next_dev, int dtype, int width, int ld, int groups, float eps, void* stream) {
+static int embed_scaled(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, const void* table_dev, int n_vocab, float scale,
+                        const void* w_next_dev, int dtype, int width, int ld, int groups, float eps, step_fetch fetch, void* stream) {
   LCU_REQUIRE(x_dev && ids_dev && table_dev && (h_dev || !w_next_dev), "lcu_embed_scaled: null pointer");
   const row_shape rs{width, ld, groups, eps};
   const int rc = check_rows("lcu_embed_scaled", dtype, n_ids, rs);
@@ -321,10 +322,36 @@ int lcu_embed_scaled(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, c
     using T = std::remove_pointer_t<decltype(kind)>;
     embed_pos_norm_kernel<T, decltype(nv)::value, decltype(th)::value><<<n_ids, decltype(th)::value, row_lds_bytes(rs), st>>>(
         (float*)x_dev, (T*)h_dev, (const int*)ids_dev, (const T*)table_dev, scale, nullptr, nullptr, (const float*)w_next_dev, nullptr,
-        n_vocab, 0, rs);
+        n_vocab, 0, rs, fetch);
   });
   LCU_LAUNCH_CHECK();
   return LCU_OK;
+}
+
+int lcu_embed_pos_norm(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, const void* table_dev, int n_vocab,
+                       const void* pos_table_dev, int n_pos, const void* start_dev, const void* w_embed_dev,
+                       const void* w_next_dev, int dtype, int width, int ld, int groups, float eps, void* stream) {
+  return embed_pos_norm(x_dev, h_dev, ids_dev, n_ids, table_dev, n_vocab, pos_table_dev, n_pos, start_dev, w_embed_dev, w_next_dev, dtype,
+                        width, ld, groups, eps, step_fetch{}, stream);
+}
+
+int lcu_embed_scaled(void* x_dev, void* h_dev, const void* ids_dev, int n_ids, const void* table_dev, int n_vocab, float scale,
+                     const void* w_next_dev, int dtype, int width, int ld, int groups, float eps, void* stream) {
+  return embed_scaled(x_dev, h_dev, ids_dev, n_ids, table_dev, n_vocab, scale, w_next_dev, dtype, width, ld, groups, eps, step_fetch{},
+                      stream);
+}
+
+int lcu_step_embed(void* state_dev, const void* state_host, void* x_dev, void* h_dev, const void* table_dev, int n_vocab, float scale,
+                   const void* pos_table_dev, int n_pos, const void* w_embed_dev, const void* w_next_dev, int dtype, int width, int ld,
+                   int groups, float eps, void* stream) {
+  LCU_REQUIRE(state_dev && state_host, "lcu_step_embed: null pointer");
+  const step_fetch fetch{(uint32_t*)state_dev, (const uint32_t*)state_host, 2};
+  const void* id = (const char*)state_host + 4;
+  if (pos_table_dev) {
+    return embed_pos_norm(x_dev, h_dev, id, 1, table_dev, n_vocab, pos_table_dev, n_pos, state_host, w_embed_dev, w_next_dev, dtype, width,
+                          ld, groups, eps, fetch, stream);
+  }
+  return embed_scaled(x_dev, h_dev, id, 1, table_dev, n_vocab, scale, w_next_dev, dtype, width, ld, groups, eps, fetch, stream);
 }
 
 int lcu_residual_norm(void* x_dev, void* h_dev, const void* out_f32_dev, const void* inverse_dev, int top,

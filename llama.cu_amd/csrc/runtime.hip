@@ -57,6 +57,11 @@ using namespace lcu;
 
 namespace {
 __global__ void add_u32_kernel(uint32_t* word, uint32_t count) { atomicAdd(word, count); }
+
+__global__ void fetch_kernel(uint32_t* dst, const uint32_t* src, int words) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < words) dst[i] = src[i];
+}
 }  // namespace
 
 extern "C" {
@@ -141,6 +146,29 @@ int lcu_free(void* dev) {
   if (dev) {
     LCU_HIP(hipFree(dev));
   }
+  return LCU_OK;
+}
+
+int lcu_host_alloc(void** out_host, size_t bytes) {
+  LCU_REQUIRE(out_host != nullptr && bytes > 0, "lcu_host_alloc: bad arguments");
+  *out_host = nullptr;
+  LCU_HIP(hipHostMalloc(out_host, bytes, hipHostMallocCoherent | hipHostMallocMapped));
+  return LCU_OK;
+}
+
+int lcu_host_free(void* host) {
+  if (host) {
+    LCU_HIP(hipHostFree(host));
+  }
+  return LCU_OK;
+}
+
+int lcu_fetch(void* dst_dev, const void* src_host, size_t bytes, void* stream) {
+  LCU_REQUIRE(dst_dev && src_host && bytes % 4 == 0 && bytes <= ((size_t)1 << 20), "lcu_fetch: bad arguments");
+  if (bytes == 0) return LCU_OK;
+  const int words = (int)(bytes / 4);
+  fetch_kernel<<<(words + 255) / 256, 256, 0, as_stream(stream)>>>((uint32_t*)dst_dev, (const uint32_t*)src_host, words);
+  LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
 

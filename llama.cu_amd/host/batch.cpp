@@ -34,8 +34,9 @@ struct llama_batch_context_impl final : public llama_batch_context {
     t_silu_ = gpu_buffer(B * ffn * 2);
     t_logits_ = gpu_buffer(B * vocab * 2);
     t_probs_ = gpu_buffer(B * vocab * 2);
-    t_argmax_ = gpu_buffer(B * sizeof(int));
-    t_step_ = gpu_buffer(B * (sizeof(int32_t) + sizeof(int16_t)));  // positions, then tokens
+    t_argmax_ = pinned_buffer(B * sizeof(int));
+    step_in_ = pinned_buffer(round_up(B * (sizeof(int32_t) + sizeof(int16_t)), 4));  // positions, then tokens
+    t_step_ = gpu_buffer(step_in_.size());
     t_cache_ptrs_ = gpu_buffer((size_t)p.n_layers * 2 * B * sizeof(void*));
     upload_cache_pointers();
   }
@@ -62,10 +63,10 @@ struct llama_batch_context_impl final : public llama_batch_context {
       count += s->context_memory_usage();
     }
     for (gpu_buffer const* b : {&t_x_, &t_norm_, &t_q_, &t_k_, &t_v_, &t_out_, &t_w1_, &t_w3_, &t_silu_, &t_logits_,
-                                &t_probs_, &t_argmax_, &t_step_, &t_cache_ptrs_}) {
+                                &t_probs_, &t_step_, &t_cache_ptrs_}) {
       count += b->size();
     }
-    return count;
+    return count + t_argmax_.size();
   }
 
   short next_token(int sequence, std::vector<short> const& new_tokens) override {
@@ -76,18 +77,17 @@ struct llama_batch_context_impl final : public llama_batch_context {
   std::vector<short> next_tokens(std::vector<short> const& tokens) override {
     const int B = (int)seqs_.size();
     assert((int)tokens.size() == B);
-    // positions and tokens go up in one copy; every kernel of the step reads them on the device,
+    // positions and tokens are fetched by the step's first launch; every other one reads them on the device,
     // so the step is captured once (on its second run) and replayed afterwards
-    std::vector<char> host((size_t)B * 6);
+    char* host = (char*)step_in_.data();  // nothing on the device reads it between two calls
     int max_T = 0;
     for (int b = 0; b < B; ++b) {
       assert(seqs_[b]->tokens_left() >= 1);
       const int32_t pos = seqs_[b]->start_pos();
-      memcpy(host.data() + (size_t)b * 4, &pos, 4);
-      memcpy(host.data() + (size_t)B * 4 + (size_t)b * 2, &tokens[b], 2);
+      memcpy(host + (size_t)b * 4, &pos, 4);
+      memcpy(host + (size_t)B * 4 + (size_t)b * 2, &tokens[b], 2);
       max_T = pos + 1 > max_T ? pos + 1 : max_T;
     }
-    LCU_CHECK(lcu_h2d(t_step_.data(), host.data(), host.size(), stream_));
     // the attention kernel is given a bound on the rows it may see; a graph is good while the
     // bound holds (bounds: 1024, then the context length)
     const int bound = (max_T <= 1024 && context_len_ > 1024) ? 1024 : context_len_;
@@ -109,8 +109,8 @@ struct llama_batch_context_impl final : public llama_batch_context {
         enqueue_step(bound);
       }
     }
-    std::vector<int> idx(B);
-    LCU_CHECK(lcu_d2h(idx.data(), t_argmax_.data(), (size_t)B * sizeof(int), stream_));  // blocks
+    LCU_CHECK(lcu_sync(stream_));
+    const int* idx = (const int*)t_argmax_.data();
     std::vector<short> out(B);
     for (int b = 0; b < B; ++b) {
       seqs_[b]->advance_one();
@@ -165,6 +165,7 @@ struct llama_batch_context_impl final : public llama_batch_context {
     const void* pos = t_step_.data();
     const void* ids = (char*)t_step_.data() + (size_t)B * 4;
     void* x = t_x_.data();
+    LCU_CHECK(lcu_fetch(t_step_.data(), step_in_.data(), step_in_.size(), stream_));
     if (model_->tok_embeddings.quantised) {  // llama_cu.cu:1087-1097
       LCU_CHECK(lcu_embed_u8(x, ids, B, dim, model_->tok_embeddings.data.data(), model_->tok_embeddings.scales.data(),
                              block, vocab, stream_));
@@ -206,7 +207,8 @@ struct llama_batch_context_impl final : public llama_batch_context {
   int context_len_;
   float temperature_;
   std::vector<std::unique_ptr<llama_context_impl>> seqs_;
-  gpu_buffer t_x_, t_norm_, t_q_, t_k_, t_v_, t_out_, t_w1_, t_w3_, t_silu_, t_logits_, t_probs_, t_argmax_;
+  gpu_buffer t_x_, t_norm_, t_q_, t_k_, t_v_, t_out_, t_w1_, t_w3_, t_silu_, t_logits_, t_probs_;
+  pinned_buffer t_argmax_, step_in_;  // written by a step's last launch, read by its first
   gpu_buffer t_step_;        // int32 positions [B], then int16 tokens [B]
   gpu_buffer t_cache_ptrs_;  // see upload_cache_pointers
   void* stream_{nullptr};

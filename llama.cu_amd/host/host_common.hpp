@@ -4,6 +4,7 @@
 #include <stdio.h>
 
 #include <mutex>
+#include <utility>
 
 #include "llama_cu_hip.h"
 #include "llama_cu_host.hpp"
@@ -37,6 +38,35 @@ inline std::recursive_mutex& device_structure_mutex() {
   return m;
 }
 using device_structure_lock = std::lock_guard<std::recursive_mutex>;
+
+// Page-locked memory that launches read and write: what a step takes from the host and gives back.  A copy of a few bytes costs
+// the host and the device more than a launch.
+class pinned_buffer {
+ public:
+  pinned_buffer() {}
+  explicit pinned_buffer(size_t size) : size_(size) {
+    device_structure_lock lock(device_structure_mutex());
+    LCU_CHECK(lcu_host_alloc(&ptr_, size));
+  }
+  pinned_buffer(pinned_buffer&& other) : ptr_(std::exchange(other.ptr_, nullptr)), size_(std::exchange(other.size_, 0)) {}
+  pinned_buffer& operator=(pinned_buffer&& other) {
+    std::swap(ptr_, other.ptr_);
+    std::swap(size_, other.size_);
+    return *this;
+  }
+  ~pinned_buffer() {
+    if (ptr_) {
+      device_structure_lock lock(device_structure_mutex());
+      LCU_CHECK(lcu_host_free(ptr_));
+    }
+  }
+  void* data() const { return ptr_; }
+  size_t size() const { return size_; }
+
+ private:
+  void* ptr_{nullptr};
+  size_t size_{0};
+};
 
 inline size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 inline size_t round_up(size_t a, size_t b) { return ceil_div(a, b) * b; }

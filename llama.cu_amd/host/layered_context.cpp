@@ -133,7 +133,8 @@ layered_context_impl::layered_context_impl(layered_model_impl* model, int contex
   t_arrived_ = zeroed(counters * 4);
   t_step_ = zeroed((1 + R) * 4);
   t_probs_ = zeroed((size_t)m.shape.vocab * 2);
-  t_index_ = zeroed(4);
+  t_index_ = pinned_buffer(4);
+  step_in_ = pinned_buffer(8);
   plan_ = lcu_expert_plan{t_row_token_.data(),   t_row_weight_.data(), t_inverse_.data(), t_tile_expert_.data(),
                           t_tile_row_.data(),    t_expert_end_.data(), t_n_tiles_.data(), 0, 0};
   LCU_CHECK(lcu_sync(stream_));
@@ -170,10 +171,10 @@ size_t layered_context_impl::context_memory_usage() {
   for (gpu_buffer const* b :
        {&t_low_, &t_queries_, &t_latent_queries_, &t_keys_values_, &t_tail_, &t_x_, &t_x_next_, &t_h_, &t_m_, &t_wide_, &t_u_, &t_rec_, &t_scratch_, &t_hidden_, &t_shared_hidden_, &t_expert_out_, &t_shared_out_,
         &t_v_first_, &t_choice_, &t_weight_, &t_shared_gate_, &t_row_token_, &t_row_weight_, &t_inverse_, &t_tile_expert_,
-        &t_tile_row_, &t_expert_end_, &t_n_tiles_, &t_arrived_, &t_step_, &t_want_, &t_head_in_, &t_logits_, &t_probs_, &t_index_}) {
+        &t_tile_row_, &t_expert_end_, &t_n_tiles_, &t_arrived_, &t_step_, &t_want_, &t_head_in_, &t_logits_, &t_probs_}) {
     count += b->size();
   }
-  return count;
+  return count + t_index_.size();
 }
 
 void* layered_context_impl::next_norm(size_t layer) const {
@@ -407,7 +408,10 @@ void layered_context_impl::enqueue_one() {
   const size_t n_layers = m.layers.size();
   const auto norm_ahead = [&](size_t l) { return l < n_layers ? m.layers[l].norm1.data() : m.final_norm.data(); };
   row_ = lcu_step_row{};
-  embed(1, norm_ahead(0));
+  const bool learned = p.learned_positions && p.embed_norm;
+  LCU_CHECK(lcu_step_embed(t_step_.data(), step_in_.data(), t_x_.data(), t_h_.data(), m.embed.data(), p.vocab, p.embed_scale,
+                           learned ? m.pos.data() : nullptr, learned ? p.max_positions : 0, learned ? m.embed_norm.data() : nullptr,
+                           norm_ahead(0), m.dtype, p.width, m.ld, p.norm_groups, p.norm_eps, stream_));
   for (size_t l = 0; l < n_layers; ++l) {
     layer_params const& q = p.layers[l];
     layer_weights const& L = m.layers[l];
@@ -552,7 +556,11 @@ int layered_context_impl::forward(const int32_t* tokens, int n, const int32_t* w
     if (at > 0) LCU_CHECK(lcu_sync(stream_));  // the host's copies of the previous pass are about to change
     host_step_.assign(1, start_pos_);
     host_step_.insert(host_step_.end(), tokens + at, tokens + at + count);
-    LCU_CHECK(lcu_h2d(t_step_.data(), host_step_.data(), host_step_.size() * 4, stream_));
+    if (fused) {
+      memcpy(step_in_.data(), host_step_.data(), step_in_.size());
+    } else {
+      LCU_CHECK(lcu_h2d(t_step_.data(), host_step_.data(), host_step_.size() * 4, stream_));
+    }
     if (!fused && !rows.empty()) {
       host_want_ = rows;
       LCU_CHECK(lcu_h2d(t_want_.data(), host_want_.data(), host_want_.size() * 4, stream_));
@@ -575,7 +583,8 @@ int layered_context_impl::forward(const int32_t* tokens, int n, const int32_t* w
         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
         LCU_CHECK(lcu_sample_row(t_index_.data(), t_probs_.data(), vocab, z ^ (z >> 31), nullptr, stream_));
       }
-      LCU_CHECK(lcu_d2h(&token, t_index_.data(), 4, stream_));
+      LCU_CHECK(lcu_sync(stream_));
+      memcpy(&token, t_index_.data(), 4);
     }
     for (size_t i = 0; i < slots.size(); ++i) {  // consecutive rows of logits
       const size_t row = fused ? 0 : i;

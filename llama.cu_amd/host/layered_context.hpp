@@ -53,7 +53,8 @@ struct layered_context_impl final : public llama_context {
   gpu_buffer t_low_, t_queries_, t_latent_queries_, t_keys_values_, t_tail_;  // latent attention, delta rule
   gpu_buffer t_v_first_, t_choice_, t_weight_, t_shared_gate_, t_row_token_, t_row_weight_, t_inverse_, t_tile_expert_,
       t_tile_row_, t_expert_end_, t_n_tiles_;
-  gpu_buffer t_step_, t_want_, t_head_in_, t_logits_, t_probs_, t_index_;
+  gpu_buffer t_step_, t_want_, t_head_in_, t_logits_, t_probs_;
+  pinned_buffer t_index_, step_in_;                // the token, written by a call's last launch; t_step_ of a one-token step, fetched by its first
   // t_step_: position of the pass's first token, then its ids (int32); the launches read both from here
   void* start() const { return t_step_.data(); }
   void* ids() const { return (char*)t_step_.data() + 4; }

@@ -287,7 +287,8 @@ void llama_context_impl::clear_tokens() {
     t_tokens_ = gpu_buffer(ctx * sizeof(short));
     t_logits_ = gpu_buffer((size_t)p.n_vocab * 2);
     t_probs_ = gpu_buffer((size_t)p.n_vocab * 2);
-    t_argmax_ = gpu_buffer(2 * sizeof(int));  // {token, count of hand-overs that did not arrive}
+    t_argmax_ = pinned_buffer(2 * sizeof(int));
+    step_in_ = pinned_buffer(sizeof(step_state));
     t_step_ = gpu_buffer(sizeof(step_state) + 2 * p.n_layers * sizeof(void*));  // and the addresses of the caches
   }
   std::vector<void*> caches;
@@ -313,10 +314,10 @@ size_t llama_context_impl::context_memory_usage() {
     count += kv.k.size() + kv.v.size();
   }
   for (gpu_buffer const* b : {&t_embed_, &t_norm_, &t_xq_, &t_out_, &t_w1_, &t_w3_, &t_silu_, &t_tokens_, &t_logits_,
-                              &t_probs_, &t_argmax_}) {
+                              &t_probs_}) {
     count += b->size();
   }
-  return count + sizeof(step_state);
+  return count + t_argmax_.size() + sizeof(step_state);
 }
 
 void llama_context_impl::matmul(void* out, const void* lhs, weight_tensor const& w, int M, float beta) {
@@ -508,7 +509,8 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
       ++host_step_.seq;
       LCU_CHECK(lcu_sync_reset(stream_));
     }
-    LCU_CHECK(lcu_h2d(t_step_.data(), &host_step_, sizeof(host_step_), stream_));
+    memcpy(step_in_.data(), &host_step_, sizeof(host_step_));  // nothing on the device reads it between two calls
+    if (n > 1) LCU_CHECK(lcu_fetch(t_step_.data(), step_in_.data(), sizeof(host_step_), stream_));
   }
   if (n == 1) {
     ids = (char*)t_step_.data() + offsetof(step_state, token);
@@ -519,13 +521,15 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
     // 1087-1097; a one-token step gathers the row and normalises it for the first layer (1129) in one launch
     const bool quantised = model_->tok_embeddings.quantised;
     if (n == 1 && dim % 8 == 0 && dim <= 8192 && (!quantised || block % 8 == 0) && !model_->layers.empty()) {
-      LCU_CHECK(lcu_embed_rmsnorm(x, t_norm_.data(), ids, 1, dim, model_->tok_embeddings.data.data(),
-                                  quantised ? model_->tok_embeddings.scales.data() : nullptr, quantised ? block : 0, vocab,
-                                  model_->layers[0].attn_norm.data(), model_->params.norm_eps, stream_));
+      LCU_CHECK(lcu_step_embed_rmsnorm(t_step_.data(), step_in_.data(), sizeof(host_step_), x, t_norm_.data(),
+                                       (char*)step_in_.data() + offsetof(step_state, token), dim, model_->tok_embeddings.data.data(),
+                                       quantised ? model_->tok_embeddings.scales.data() : nullptr, quantised ? block : 0, vocab,
+                                       model_->layers[0].attn_norm.data(), model_->params.norm_eps, stream_));
       enqueue_layers(n, true);
       enqueue_head(n);
       return;
     }
+    if (n == 1) LCU_CHECK(lcu_fetch(t_step_.data(), step_in_.data(), sizeof(host_step_), stream_));
     if (model_->tok_embeddings.quantised) {
       LCU_CHECK(lcu_embed_u8(x, ids, n, dim, model_->tok_embeddings.data.data(), model_->tok_embeddings.scales.data(),
                              block, vocab, stream_));
@@ -577,7 +581,11 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
     int token;
     unsigned timeouts;
   } result{0, 0};
-  LCU_CHECK(lcu_d2h(&result, t_argmax_.data(), sizeof(result), stream_));  // 1198-1200, blocks
+  const auto await_result = [&] {  // 1198-1200
+    LCU_CHECK(lcu_sync(stream_));
+    memcpy(&result, t_argmax_.data(), sizeof(result));
+  };
+  await_result();
   // The one-token launches hand results over between their workgroups with bounded waits, and a wait
   // that ran out went on with stale words: the count of such waits comes back with the token, and a
   // count that has moved means this step's token is not to be trusted.  It is never returned: the
@@ -597,7 +605,7 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
       hand_overs_ = false;
       drop_graph();
       enqueue_all();
-      LCU_CHECK(lcu_d2h(&result, t_argmax_.data(), sizeof(result), stream_));
+      await_result();
       timeouts_seen_ = result.timeouts;
     } else {
       fprintf(stderr, "llama_context: the stream's count of failed hand-overs moved by %u during a call that hands "

@@ -86,7 +86,8 @@ struct llama_context_impl final : public llama_context {
   void drop_graph();
   std::vector<kv_cache_layer> kv_;
   gpu_buffer t_embed_, t_norm_, t_xq_, t_out_, t_w1_, t_w3_, t_silu_;
-  gpu_buffer t_tokens_, t_logits_, t_probs_, t_argmax_;
+  gpu_buffer t_tokens_, t_logits_, t_probs_;
+  pinned_buffer t_argmax_;  // {token, count of hand-overs that did not arrive}, written by the last launch of a call
   // step state on the device: {int32 position, int16 token, 64 random bits, uint32 step counter};
   // the decode kernels and the sampler read it from here, so one captured graph replays for every
   // step (the counter differs from step to step: the epoch of the attention kernel's hand-over)
@@ -100,6 +101,7 @@ struct llama_context_impl final : public llama_context {
     uint32_t seq;     // counts the one-token steps of this context
     uint32_t pad2;
   } host_step_{};
+  pinned_buffer step_in_;  // host_step_ on its way: the first launch of a one-token step fetches it
   bool sampling_{false};
   uint64_t sample_seed_{0};
   uint64_t samples_drawn_{0};

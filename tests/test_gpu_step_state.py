@@ -1,0 +1,82 @@
+"""What a one-token step takes from the host: page-locked words that its first launch reads and copies to the device."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from layered_helpers import BF16, F32, call, get, gpu, put, rounded, up64, zeros  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def words(gpu):
+    """Page-locked memory as an array of 256 int32."""
+    p = C.c_void_p()
+    gpu.B.check(gpu.L().lcu_host_alloc(C.byref(p), 1024))
+    yield np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_int32)), (256,))
+    gpu.B.check(gpu.L().lcu_sync(gpu.stream))
+    gpu.B.check(gpu.L().lcu_host_free(p))
+
+
+@pytest.mark.parametrize("n", [1, 6, 255, 256])
+def test_fetched_words(gpu, words, n):
+    words[:] = np.random.default_rng(n).integers(-2**31, 2**31, 256)
+    out = zeros(gpu, 256)
+    call(gpu, "lcu_fetch", out, words.ctypes.data, 4 * n)
+    gpu.B.check(gpu.L().lcu_sync(gpu.stream))
+    assert np.array_equal(gpu.host(out, (256,), np.int32), np.where(np.arange(256) < n, words, 0))
+    assert gpu.L().lcu_fetch(out.ptr, words.ctypes.data, 6, gpu.stream) == -2
+    gpu.release()
+
+
+@pytest.mark.parametrize("dim,block,state", [(8, 0, 2), (512, 0, 6), (8192, 0, 256), (1024, 128, 6)])
+def test_embedding_with_the_steps_state(gpu, words, dim, block, state):
+    """The bits of lcu_embed_rmsnorm, and the state on the device."""
+    rng = np.random.default_rng(dim)
+    words[:] = rng.integers(-2**31, 2**31, 256)
+    words[1] = 5
+    ids, out = gpu.dev_keep(np.array([5], np.int16)), zeros(gpu, 256)
+    table = gpu.dev_keep(rng.integers(0, 256, (9, dim)).astype(np.uint8) if block else rng.standard_normal((9, dim)).astype(np.float16))
+    scales = gpu.dev_keep((0.01 * rng.random((9, max(1, dim // 128)))).astype(np.float16)) if block else None
+    w = gpu.dev_keep(rng.standard_normal(dim).astype(np.float16))
+    results = []
+    for step in (False, True):
+        x, h = (gpu.dev_keep(np.zeros(dim, np.float16)) for _ in range(2))
+        if step:
+            call(gpu, "lcu_step_embed_rmsnorm", out, words.ctypes.data, 4 * state, x, h, words.ctypes.data + 4, dim, table, scales, block, 9, w, 1e-6)
+        else:
+            call(gpu, "lcu_embed_rmsnorm", x, h, ids, 1, dim, table, scales, block, 9, w, 1e-6)
+        gpu.B.check(gpu.L().lcu_sync(gpu.stream))
+        results.append([gpu.host(b, (dim,), np.uint16) for b in (x, h)])
+    assert all(np.array_equal(a, b) for a, b in zip(*results))
+    assert np.array_equal(gpu.host(out, (256,), np.int32), np.where(np.arange(256) < state, words, 0))
+    assert gpu.L().lcu_step_embed_rmsnorm(out.ptr, words.ctypes.data, 1028, x.ptr, h.ptr, words.ctypes.data, dim, table.ptr,
+                                          scales.ptr if block else None, block, 9, w.ptr, 1e-6, gpu.stream) == -2
+    gpu.release()
+
+
+@pytest.mark.parametrize("width,learned", [(70, False), (4200, False), (960, True)])
+def test_layered_embedding_with_the_steps_state(gpu, words, width, learned):
+    """The bits of lcu_embed_scaled and lcu_embed_pos_norm at position 3, and position and id on the device."""
+    rng = np.random.default_rng(width)
+    ld = up64(width)
+    padded = lambda a: np.pad(a, [(0, 0)] * (a.ndim - 1) + [(0, ld - width)])
+    words[:2] = 3, 5
+    pair, out = gpu.dev_keep(words[:2].copy()), zeros(gpu, 2)
+    table, pos = (put(gpu, padded(rounded(rng.standard_normal((9, width)))), BF16) for _ in range(2))
+    w1, w2 = (put(gpu, padded(rng.standard_normal(width))) for _ in range(2))
+    shape = (w2, BF16, width, ld, 1, 1e-5)
+    results = []
+    for step in (False, True):
+        x, h = zeros(gpu, ld), zeros(gpu, ld, BF16)
+        if step:
+            call(gpu, "lcu_step_embed", out, words.ctypes.data, x, h, table, 9, 2.5, *((pos, 9, w1) if learned else (None, 0, None)), *shape)
+        elif learned:
+            call(gpu, "lcu_embed_pos_norm", x, h, pair.ptr + 4, 1, table, 9, pos, 9, pair, w1, *shape)
+        else:
+            call(gpu, "lcu_embed_scaled", x, h, pair.ptr + 4, 1, table, 9, 2.5, *shape)
+        results.append([get(gpu, x, (ld,), F32), get(gpu, h, (ld,), BF16)])
+    assert all(np.array_equal(a, b) for a, b in zip(*results))
+    assert np.array_equal(gpu.host(out, (2,), np.int32), words[:2])
+    gpu.release()
