@@ -79,6 +79,48 @@ def test_gated_linear_large_tiles(gpu, M, K, ff):
     gpu.release()
 
 
+# K dealt to several workgroups: tiles of 128 and of 64 rows, runs of unequal length, ragged rows and columns, fewer and more than 2^20 outputs
+SPLIT_PRODUCTS = [(65, 4096, 1530, (64, 11)), (65, 4096, 4096, (128, 6)), (129, 2880, 2045, (64, 5)), (300, 4096, 6146, (64, 2)), (513, 5632, 2061, (128, 3)),
+                  (900, 10752, 1030, (128, 3))]
+
+
+@pytest.mark.parametrize("M,K,N,plan", SPLIT_PRODUCTS)
+def test_linear_split(gpu, M, K, N, plan):
+    assert gemm_plan.bf16_split(M, K, N) == plan and gemm_plan.bf16_split(M, K, N, workspace=0) == (0, 0)
+    rng = np.random.default_rng(N)
+    x, w, bias = rounded(rng.standard_normal((M, K))), rounded(rng.standard_normal((N, K)) / K ** 0.5), rng.standard_normal(N)
+    xd, wd, bd = put(gpu, x, BF16), put(gpu, w, BF16), put(gpu, bias)
+    want = (x.astype(np.float32) @ w.T.astype(np.float32)).astype(np.float64)
+    for is_f32, gelu, tail, b in ((1, 0, 0, None), (0, N // 3, 0, bd), (0, 0, 19, None)):
+        ld, cut = N + 1, N - tail
+        out, rest = zeros(gpu, (M, ld), F32 if is_f32 else BF16), zeros(gpu, (M, max(tail, 1)))
+        if tail:
+            call(gpu, "lcu_linear_tail", out, ld, rest, tail, cut, xd, wd, BF16, M, K, N)
+        else:
+            call(gpu, "lcu_linear", out, is_f32, ld, xd, wd, b, gelu, BF16, M, K, N)
+        full = want + bias if b is not None else want.copy()
+        if gelu:
+            full[:, :gelu] = S.gelu_tanh(full[:, :gelu])
+        got = get(gpu, out, (M, ld), F32 if is_f32 else BF16)
+        close(got[:, :cut], full[:, :cut], F32 if is_f32 else BF16)
+        assert (got[:, cut:] == 0).all()
+        if tail:
+            close(get(gpu, rest, (M, tail)), full[:, cut:], F32)
+    # a stream of somebody else's: the tiles as they are
+    out = zeros(gpu, (M, N))
+    gpu.B.check(gpu.L().lcu_sync(gpu.stream))
+    gpu.B.check(gpu.L().lcu_linear(out.ptr, 1, N, xd.ptr, wd.ptr, None, 0, BF16, M, K, N, None))
+    gpu.B.check(gpu.L().lcu_sync(None))
+    close(get(gpu, out, (M, N)), want, F32)
+    gpu.release()
+
+
+@pytest.mark.parametrize("M,K,ff,plan", [(65, 4096, 740, (64, 11)), (100, 4096, 2020, (128, 5)), (700, 4096, 1020, (128, 2)), (640, 8192, 1700, (128, 3))])
+def test_gated_linear_split(gpu, M, K, ff, plan):
+    assert gemm_plan.bf16_split(M, K, 2 * up64(ff), gated=True) == plan
+    test_gated_linear_large_tiles(gpu, M, K, ff)
+
+
 # 128 columns over a short K; gated tiles of 128x128 that outnumber the compute units, on both sides of theirs
 @pytest.mark.parametrize("M,K,N", [(1441, 512, 8900), (1441, 640, 8900),
                                    (8, 512, 30000), (40, 640, 25000),  # few rows in two rounds of workgroups
