@@ -49,20 +49,18 @@ __global__ __launch_bounds__(TH) void residual_norm_kernel(float* __restrict__ x
                                                                     const float* __restrict__ w_next, row_shape rs) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int r = blockIdx.x;
-  row_t<NV, TH> m, t, old;
+  row_t<NV, TH> m, t, old, next;
   load_sum(m, t, src, r, rs);
   float* xr = x + (size_t)r * rs.ld;
   load_row(old, xr, rs);
   load_row(t, w_after, rs);
+  if (w_next) load_row(next, w_next, rs);
   scale_row(m, rs, lds, t);
 #pragma unroll
   for (int j = 0; j < NV; ++j) m.v[j] += old.v[j];
   store_row(xr, m, rs);
   if (!h) return;
-  if (w_next) {
-    load_row(t, w_next, rs);
-    scale_row(m, rs, lds, t);
-  }
+  if (w_next) scale_row(m, rs, lds, next);
   store_row(h + (size_t)r * rs.ld, m, rs);
 }
 

@@ -76,16 +76,20 @@ __device__ __forceinline__ void load_sum(row_t<NV, TH>& m, row_t<NV, TH>& t, con
     return src.out + (src.inverse ? (size_t)src.inverse[at] : at) * rs.ld;
   };
   load_row(m, from(0), rs);
+  if (src.top == 1 && !src.shared) return;
+  // two experts and the shared one: all three on their way before the first is added
+  row_t<NV, TH> u;
+  const float f = src.shared ? src.shared_gate[r] : 0.0f;
+  if (src.top > 1) load_row(t, from(1), rs);
+  if (src.shared) load_row(u, src.shared + (size_t)r * rs.ld, rs);
   for (int k = 1; k < src.top; ++k) {
-    load_row(t, from(k), rs);
+    if (k > 1) load_row(t, from(k), rs);
 #pragma unroll
     for (int j = 0; j < NV; ++j) m.v[j] += t.v[j];
   }
   if (src.shared) {
-    const float f = src.shared_gate[r];
-    load_row(t, src.shared + (size_t)r * rs.ld, rs);
 #pragma unroll
-    for (int j = 0; j < NV; ++j) m.v[j] += f * t.v[j];
+    for (int j = 0; j < NV; ++j) m.v[j] += f * u.v[j];
   }
 }
 
@@ -116,17 +120,10 @@ inline size_t row_lds_bytes(const row_shape& rs) {
   return ((whole ? pieces : quads * 4) + rs.groups) * sizeof(float);
 }
 
-// p[0] + p[1] + ... in that order, sixteen (four) asked for at a time
+// p[0] + p[1] + ... in that order, eight asked for at a time
 __device__ __forceinline__ float sum_of_pieces(const float* p, int count) {
   float total = 0.0f;
   int k = 0;
-  for (; k + 16 <= count; k += 16) {
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = p[k + i];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) total += v[i];
-  }
   for (; k + 8 <= count; k += 8) {
     float v[8];
 #pragma unroll
@@ -134,7 +131,12 @@ __device__ __forceinline__ float sum_of_pieces(const float* p, int count) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) total += v[i];
   }
-  for (; k < count; ++k) total += p[k];
+  for (; k + 2 <= count; k += 2) {
+    const float v = p[k], u = p[k + 1];
+    total += v;
+    total += u;
+  }
+  if (k < count) total += p[k];
   return total;
 }
 
@@ -155,6 +157,13 @@ __device__ __forceinline__ void scale_row(row_t<NV, TH>& r, const row_shape& rs,
     }
     __syncthreads();
     const int per = part / ROW_PIECE;
+    if (rs.groups == 1) {
+      const float scale = 1.0f / sqrtf(sum_of_pieces(piece, per) / (float)part + rs.eps);
+#pragma unroll
+      for (int j = 0; j < NV; ++j) r.v[j] *= scale * w.v[j];
+      __syncthreads();
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int g = __builtin_amdgcn_readfirstlane((j * WAVES + wave) / per);
