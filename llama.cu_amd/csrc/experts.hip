@@ -32,10 +32,12 @@ __global__ __launch_bounds__(256) void router_kernel(int* __restrict__ expert, f
   choose_experts(z, n_experts, top, expert + (size_t)t * top, weight + (size_t)t * top);
 }
 
-// The same for bfloat16 operands on the matrix cores: one workgroup takes 16 tokens and all rows of w, its eight
+// The same for bfloat16 operands on the matrix cores: one workgroup takes 16 tokens (or 4) and all rows of w, its eight
 // wavefronts an eighth of K each, four tiles of 16 rows of w at a time; the eighths meet in LDS and are added
-// in wavefront order, and every wavefront chooses for two of the tokens.
-constexpr int ROUTER_TOKENS = 16, ROUTER_WAVES = 8;
+// in wavefront order, and the wavefronts choose for the tokens in turn.
+// What bounds it is the compute unit's way to the operands, 64 bytes a row at a time, five clocks each (every load asked for at once: no
+// sooner).  So a workgroup takes four tokens, whose rows stand for the other twelve, as long as there is a compute unit for each.
+constexpr int ROUTER_TOKENS = 16, ROUTER_FEW = 4, ROUTER_WAVES = 8;
 template <int TILES>
 __device__ __forceinline__ void router_tiles(float4_t (&acc)[4], const bf16_t* a, const bf16_t* const (&b)[4], int s0, int s1) {
 #pragma unroll 8
@@ -51,14 +53,14 @@ __device__ __forceinline__ void router_tiles(float4_t (&acc)[4], const bf16_t* a
 
 __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_tile_kernel(int* __restrict__ expert, float* __restrict__ weight,
                                                           float* __restrict__ shared_gate, const bf16_t* __restrict__ h,
-                                                          const bf16_t* __restrict__ w, int n, int n_experts, int top, int K) {
+                                                          const bf16_t* __restrict__ w, int n, int n_experts, int top, int K, int tokens) {
   extern __shared__ float zs[];  // [ROUTER_TOKENS][ldz]
   __shared__ float part[ROUTER_WAVES][ROUTER_TOKENS][64 + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t0 = blockIdx.x * ROUTER_TOKENS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t0 = blockIdx.x * tokens;
   const int n_rows = n_experts + (shared_gate ? 1 : 0), ldz = (n_rows + 15) / 16 * 16 + 1;
   const int col = lane & 15, quad = lane >> 4;
   const int steps = K / 32, s0 = wave * steps / ROUTER_WAVES, s1 = (wave + 1) * steps / ROUTER_WAVES;
-  const bf16_t* a = h + (size_t)min(t0 + col, n - 1) * K + quad * 8;
+  const bf16_t* a = h + (size_t)min(t0 + min(col, tokens - 1), n - 1) * K + quad * 8;
   for (int e0 = 0; e0 < n_rows; e0 += 64) {
     float4_t acc[4];
     const bf16_t* b[4];
@@ -89,9 +91,7 @@ __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_tile_kernel(int* __r
     }
     __syncthreads();
   }
-  for (int k = 0; k < ROUTER_TOKENS / ROUTER_WAVES; ++k) {
-    const int t = t0 + wave * (ROUTER_TOKENS / ROUTER_WAVES) + k;
-    if (t >= n) continue;
+  for (int t = t0 + wave; t < min(t0 + tokens, n); t += ROUTER_WAVES) {
     float* z = zs + (t - t0) * ldz;
     if (shared_gate && lane == 0) shared_gate[t] = sigmoid_f32(z[n_experts]);
     choose_experts(z, n_experts, top, expert + (size_t)t * top, weight + (size_t)t * top);
@@ -162,8 +162,11 @@ int lcu_router(void* expert_dev, void* weight_dev, void* shared_gate_dev, const 
       LCU_HIP(hipFuncSetAttribute((const void*)router_tile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
       raised[dev & 15] = true;
     }
-    router_tile_kernel<<<(n + ROUTER_TOKENS - 1) / ROUTER_TOKENS, 64 * ROUTER_WAVES, lds, st>>>(
-        (int*)expert_dev, (float*)weight_dev, (float*)shared_gate_dev, (const bf16_t*)h_dev, (const bf16_t*)w_dev, n, n_experts, top, K);
+    const device_state* ds = current_device_state();
+    const int tokens = n <= ROUTER_FEW * (ds && ds->compute_units > 0 ? ds->compute_units : 256) ? ROUTER_FEW : ROUTER_TOKENS;
+    router_tile_kernel<<<(n + tokens - 1) / tokens, 64 * ROUTER_WAVES, lds, st>>>((int*)expert_dev, (float*)weight_dev, (float*)shared_gate_dev,
+                                                                                 (const bf16_t*)h_dev, (const bf16_t*)w_dev, n, n_experts, top, K,
+                                                                                 tokens);
   }
   LCU_LAUNCH_CHECK();
   return LCU_OK;

@@ -553,6 +553,22 @@ def test_experts_in_tiles_of_any_height(gpu, n, K, ff, experts, top):
     gpu.release()
 
 
+@pytest.mark.parametrize("K,experts,top", [(320, 16, 2), (64, 70, 3)])
+def test_router_tokens_to_a_workgroup(gpu, K, experts, top):
+    """1030 tokens, sixteen to a workgroup, choose as the first 1, 3, 4, 5, 1023 and 1024 of them, four to one, to the bit."""
+    rng = np.random.default_rng(K)
+    h, w = put(gpu, rounded(rng.standard_normal((1030, K))), BF16), put(gpu, rounded(rng.standard_normal((experts + 1, K)) / K ** 0.5), BF16)
+    results = {}
+    for n in (1030, 1, 3, 4, 5, 1023, 1024):
+        e, wt, sg = ints(gpu, np.full((n + 1, top), -7)), zeros(gpu, (n + 1, top)), zeros(gpu, n + 1)
+        call(gpu, "lcu_router", e, wt, sg, h, w, experts, top, BF16, n, K)
+        results[n] = get_ints(gpu, e, (n + 1, top)), get(gpu, wt, (n + 1, top)), get(gpu, sg, (n + 1,))
+        assert (results[n][0][n] == -7).all() and not results[n][1][n].any() and results[n][2][n] == 0
+        for got, want in zip(results[n], results[1030]):
+            assert (got[:n] == want[:n]).all()
+    gpu.release()
+
+
 @pytest.mark.parametrize("n", [1, 7, 640, 32000, 50257])
 def test_argmax_and_softmax(gpu, n):
     rng = np.random.default_rng(n)
