@@ -159,6 +159,34 @@ __host__ __device__ __forceinline__ float divide_by(float x, float d, float reci
   return fmaf(fmaf(-q, d, x), reciprocal, q);
 }
 
+// fp16(silu(a) * b), silu(a) = a / (1 + exp_ieee(-a)) in fp32 (llama_cu.cu:533-539), in two thirds of the instructions of exp_ieee and a
+// division, with the same result for all a and b.  exp_ieee's scaling in one step where 2^k is a normal number; the quotient from the
+// reciprocal by a Newton step and Markstein's correction, the divisor lying between 1 and 6.1e37.  Below -87 the quotient is
+// smaller than anything that times a finite b is not 0 in fp16; beyond 88.72283 the exponential is infinite and the quotient -0; above 80
+// the divisor is 1.  (Every a with b of all kinds: test_silu_of_every_half.)
+__device__ __forceinline__ half_t silu_mul(half_t a, half_t b) {
+  const float val = (float)a, x = fminf(-val, 87.0f);
+  const float magic = x * 1.44269504f + 12582912.0f;
+  const float kf = magic - 12582912.0f;
+  float r = fmaf(kf, -0.693359375f, x);
+  r = fmaf(kf, 2.12194440e-4f, r);
+  float p = 1.9875691500e-4f;
+  p = fmaf(p, r, 1.3981999507e-3f);
+  p = fmaf(p, r, 8.3334519073e-3f);
+  p = fmaf(p, r, 4.1665795894e-2f);
+  p = fmaf(p, r, 1.6666665459e-1f);
+  p = fmaf(p, r, 5.0000001201e-1f);
+  p = fmaf(p * r, r, r) + 1.0f;
+  const float d = 1.0f + p * __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, magic) << 23) + 0x3f800000u);
+  float inverse = __builtin_amdgcn_rcpf(d);
+  inverse = fmaf(fmaf(-d, inverse, 1.0f), inverse, inverse);
+  float q = val * inverse;
+  q = fmaf(-fmaf(d, q, -val), inverse, q);  // in this form -0 stays -0
+  q = val < -88.72283f ? val * 0.0f : q;
+  q = val > 80.0f ? val : q;
+  return round_f16(q * (float)b);
+}
+
 // ---- wavefront reductions (all 64 lanes end with the result) ----
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {

@@ -444,12 +444,6 @@ __global__ __launch_bounds__(1024) void softmax_argmax_kernel(half_t* __restrict
   }
 }
 
-// silu, llama_cu.cu:533-539
-__device__ __forceinline__ half_t silu_mul_one(half_t a, half_t b) {
-  const float val = (float)a;
-  return round_f16(val / (1.0f + exp_ieee(-val)) * (float)b);
-}
-
 // eight elements per thread with 16-byte accesses (VEC: every pointer 16-byte aligned), the tail
 // and unaligned buffers one by one
 template <bool VEC>
@@ -463,13 +457,13 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(half_t* out, const half_t
     half8_t r;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      r[e] = silu_mul_one(av[e], bv[e]);
+      r[e] = silu_mul(av[e], bv[e]);
     }
     *reinterpret_cast<half8_t*>(out + i) = r;
     return;
   }
   for (size_t j = i; j < min(i + 8, size); ++j) {
-    out[j] = silu_mul_one(a[j], b[j]);
+    out[j] = silu_mul(a[j], b[j]);
   }
 }
 

@@ -1300,10 +1300,9 @@ __global__ __launch_bounds__(256) void reduce_silu_kernel(half_t* __restrict__ o
   if (i >= mn) return;
   const float2 a = sum_pair(part, i, mn, splits);
   const float2 g = sum_pair(part + (size_t)splits * mn, i, mn, splits);
-  const float v0 = (float)round_f16(a.x), v1 = (float)round_f16(a.y);
   half2_t w;
-  w.x = round_f16(v0 / (1.0f + exp_ieee(-v0)) * (float)round_f16(g.x));
-  w.y = round_f16(v1 / (1.0f + exp_ieee(-v1)) * (float)round_f16(g.y));
+  w.x = silu_mul(round_f16(a.x), round_f16(g.x));
+  w.y = silu_mul(round_f16(a.y), round_f16(g.y));
   *reinterpret_cast<half2_t*>(out + i) = w;
 }
 
@@ -1988,6 +1987,12 @@ int lcu_batch_ffn_up(void* out_dev, void* w1_tmp_dev, void* w3_tmp_dev, const vo
     reduce_silu_kernel<<<(unsigned)((mn / 2 + 255) / 256), 256, 0, st>>>((half_t*)out_dev, ps.part, ps.splits, mn);
     LCU_LAUNCH_CHECK();
     return LCU_OK;
+  }
+  if (block == 0 && n_seq > 64 && dim % 128 == 0 && ffn % 16 == 0 && (size_t)n_seq * dim * 2 < ((size_t)1 << 32) &&
+      (size_t)ffn * dim * 2 < ((size_t)1 << 32) && ffn < 1 << 30 && tiles_of(n_seq, ffn, 256, 128) * 2 >= 160) {  // those of plan_rows' large tiles
+    operands_t op = single_matrix((half_t*)out_dev, w_dev[0], nullptr);
+    op.more.W[0] = w_dev[1];
+    return launch_large<false>(silu_epilogue{}, op, lhs_dev, n_seq, dim, 2 * ffn, 0, 0.0f, st);
   }
   const int rc = block ? lcu_gemm_f16u8_nt_multi(outs, lhs_dev, w_dev, scales_dev, 2, n_seq, dim, ffn, block, 0.0f, stream)
                        : lcu_gemm_f16_nt_multi(outs, lhs_dev, w_dev, 2, n_seq, dim, ffn, 0.0f, stream);

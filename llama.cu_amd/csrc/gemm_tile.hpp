@@ -37,15 +37,23 @@ struct more_matrices_t {
 };
 
 struct f16_epilogue {
-  static constexpr bool BF16 = false, GROUPED = false, GATED = false, ROTARY = false;
+  static constexpr bool BF16 = false, GROUPED = false, GATED = false, ROTARY = false, PAIRED = false;
 };
 // fp16 outputs whose first `matrices` matrices are rotated (llama_cu.cu:368-389): row r is at position first + r, head_dim a multiple of 8.
 // The rotation reads outputs as they would be stored, so the bits are those of lcu_rope_pair afterwards.  512 rows, three times 4096x4096: the
 // product 63.6 us and the rotation by itself 7.4 -> 65.7; 1987 rows 183 and 20.7 -> 186.
 struct rotary_epilogue {
-  static constexpr bool BF16 = false, GROUPED = false, GATED = false, ROTARY = true;
+  static constexpr bool BF16 = false, GROUPED = false, GATED = false, ROTARY = true, PAIRED = false;
   const float2* table;  // [positions][head_dim / 2] (cos, sin)
   int head_dim, first, matrices;
+};
+
+// fp16(silu(lhs W^T) * (lhs V^T)), llama_cu.cu:1180-1183: the columns alternate, sixteen of W (matrix 0) and the sixteen of V (matrix 1) that
+// they meet, so that a lane holds both; N counts both.  A wavefront requests columns of one matrix only.  Half the outputs and no launch that
+// reads them again: 512 rows, K 4096, twice 11008 columns 97.9 us in two launches, 90.2 here (95 with the general exponential and division: 96
+// outputs to a lane are 4 us of the tile), 1987 rows 329 and 318; K 2048, twice 5632 columns 38.3 and 33.3, 112 and 101.
+struct silu_epilogue {
+  static constexpr bool BF16 = false, GROUPED = false, GATED = false, ROTARY = false, PAIRED = true;
 };
 
 template <int N>
@@ -98,7 +106,7 @@ struct tile_shape {
   static constexpr int NW = WM * WN, WR = BM / WM, WC = BN / WN;
   static constexpr int A_BYTES = BM * 128, B_BYTES = BN * (U8 ? 64 : 128), SW = (WC + 63) / 64 * 64, S_BYTES = U8 ? NW * SW * 4 : 0;
   static constexpr int W_BYTES = B_BYTES + S_BYTES;      // S: one word per column of every wavefront, of its own
-  static constexpr int OUT_LD = (EP::GATED ? WC / 2 : WC) + 4;  // floats per row of a wavefront's 64 output rows in LDS
+  static constexpr int OUT_LD = (EP::GATED || EP::PAIRED ? WC / 2 : WC) + 4;  // floats per row of a wavefront's 64 output rows in LDS
   static constexpr int RING = NA * A_BYTES + NB * W_BYTES, OUT = NW * 64 * OUT_LD * 4;
   static constexpr int LDS = RING > OUT ? RING : OUT;
   static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 16 == 0, "tile");
@@ -121,6 +129,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   constexpr int BEHIND = NB > NA ? PW : 0;  // of a stage's requests, those behind its lhs that lhs's turn need not wait for
   static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0 && NA >= 2 && NB >= NA && PA * NA + PW * NB < 64, "requests");
   static_assert(!U8 || !EP::BF16, "codes");
+  static_assert(!EP::PAIRED || (!U8 && !SPLIT && NW % 4 == 0 && TN % 2 == 0), "pairs of columns");
   extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
 
   // consecutive workgroups go round the eight XCDs: each gets one run of the M-fastest tile sequence, so that
@@ -156,6 +165,9 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   const int n0 = from + tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave % WM) * shape::WR, wn = (wave / WM) * shape::WC;
+  // request j of a wavefront is rows (wave + j NW) 8 .. + 7 of the tile: of the same matrix for every j
+  if constexpr (EP::PAIRED) W = (wave >> 1) & 1 ? more.W[0] : W0;
+  const int matrix_n = EP::PAIRED ? N / 2 : N;
 
   // this workgroup's K stages
   const int nt_all = K / 64;
@@ -186,8 +198,8 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
       const int row = c / 4, g = (c % 4) ^ (2 * ((row / 4) % 2));
       b_off[j] = row_piece(n0 + row, N, (uint32_t)K, g);
     } else {
-      const int row = c / 8, g = (c % 8) ^ ((row / 2) % 8);
-      b_off[j] = row_piece(n0 + row, N, (uint32_t)K * 2u, g);
+      const int row = c / 8, g = (c % 8) ^ ((row / 2) % 8), n = n0 + row;
+      b_off[j] = row_piece(EP::PAIRED ? n / 32 * 16 + n % 16 : n, matrix_n, (uint32_t)K * 2u, g);
     }
   }
   // first scale of the rows whose scales this lane requests, and of those of its fragments
@@ -201,7 +213,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   }
   int lhs_rows = M;
   if constexpr (EP::GROUPED) lhs_rows = ep.lhs_rows;
-  uint4_t ra = operand_resource(A, (uint32_t)lhs_rows * (uint32_t)K * 2u), rw = operand_resource(W, (uint32_t)N * (uint32_t)K * (U8 ? 1u : 2u)), rs = ra;
+  uint4_t ra = operand_resource(A, (uint32_t)lhs_rows * (uint32_t)K * 2u), rw = operand_resource(W, (uint32_t)matrix_n * (uint32_t)K * (U8 ? 1u : 2u)), rs = ra;
   if constexpr (U8) rs = operand_resource(S, (uint32_t)N * ((uint32_t)K >> (6 + block_shift)) * 2u);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)tile_lds;
   // Inline assembly, so that the compiler does not know about the LDS writes: knowing, it waits for every LDS read
@@ -367,9 +379,10 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   // ---- epilogue, 64 rows of the wavefront's tile at a time.  Register v of lane l holds row 4 (l / 16) + v, column
   // l % 16 of a 16x16 tile.
   float* rows = reinterpret_cast<float*>(tile_lds) + wave * 64 * shape::OUT_LD;
-  constexpr int OC = EP::GATED ? shape::WC / 2 : shape::WC;  // output columns of the wavefront
+  constexpr bool HALVED = EP::GATED || EP::PAIRED;           // two columns to an output
+  constexpr int OC = HALVED ? shape::WC / 2 : shape::WC;     // output columns of the wavefront
   constexpr int PIECES = OC / 8;                             // pieces of eight columns per row, and per lane
-  const int out_n0 = EP::GATED ? (n0 + wn) / 2 : n0 + wn, out_n = EP::GATED ? N / 2 : N;
+  const int out_n0 = HALVED ? (n0 + wn) / 2 : n0 + wn, out_n = HALVED ? N / 2 : N;
   // Pieces of eight columns leave as 16 bytes wherever a row begins, its last ones one by one (fp16 1401x384x16515: 39 us so,
   // 75 with single stores for rows off 16 bytes).
   typedef half8_t any_half8_t __attribute__((aligned(2)));
@@ -401,6 +414,9 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
               to[(j / 2 + e) * 16] = ep.gate(gate, up);
             }
           }
+        } else if constexpr (EP::PAIRED) {  // both rounded as they would be stored
+#pragma unroll
+          for (int j = 0; j < TN; j += 2) to[j / 2 * 16] = (float)silu_mul(round_f16(acc[p * 4 + i][j][v]), round_f16(acc[p * 4 + i][j + 1][v]));
         } else {
 #pragma unroll
           for (int j = 0; j < TN; ++j) to[j * 16] = acc[p * 4 + i][j][v];
@@ -417,7 +433,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
 #pragma unroll
           for (int k = 0; k < AT_ONCE; ++k) {
             const int c = lane + 64 * (k0 + k), gm = m0 + wm + p * 64 + c / PIECES, gn = out_n0 + c % PIECES * 8;
-            if (gm < M && gn + 8 <= N) old[k] = *reinterpret_cast<const any_half8_t*>(out + (size_t)gm * N + gn);
+            if (gm < M && gn + 8 <= out_n) old[k] = *reinterpret_cast<const any_half8_t*>(out + (size_t)gm * out_n + gn);
           }
         }
       }
@@ -451,8 +467,8 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
         } else if constexpr (EP::BF16) {
           ep.store8(gm, gn, x, out_n);
         } else {
-          half_t* to = out + (size_t)gm * N + gn;
-          if (gn + 8 <= N) {  // llama_cu.cu:208-215: fp16(acc + beta * old)
+          half_t* to = out + (size_t)gm * out_n + gn;
+          if (gn + 8 <= out_n) {  // llama_cu.cu:208-215: fp16(acc + beta * old)
             half8_t y;
 #pragma unroll
             for (int e = 0; e < 8; ++e) y[e] = round_f16(beta != 0.0f ? fmaf(beta, (float)old[k][e], x[e]) : x[e]);
@@ -468,7 +484,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
             }
             *reinterpret_cast<any_half8_t*>(to) = y;
           } else {
-            for (int e = 0; e < 8 && gn + e < N; ++e) to[e] = round_f16(beta != 0.0f ? fmaf(beta, (float)to[e], x[e]) : x[e]);
+            for (int e = 0; e < 8 && gn + e < out_n; ++e) to[e] = round_f16(beta != 0.0f ? fmaf(beta, (float)to[e], x[e]) : x[e]);
           }
         }
       }

@@ -71,7 +71,7 @@ __device__ __forceinline__ group_tile_t group_tile(const row_groups<true>& g, in
 // GATED: the matrix holds, in blocks of 64 rows, 32 gate rows and the 32 up rows of the same hidden columns.
 template <bool GROUPED_, bool GATED_>
 struct linear_epilogue : row_groups<GROUPED_> {
-  static constexpr bool BF16 = true, GROUPED = GROUPED_, GATED = GATED_, ROTARY = false;
+  static constexpr bool BF16 = true, GROUPED = GROUPED_, GATED = GATED_, ROTARY = false, PAIRED = false;
   void* out;
   int ldo;
   bool out_f32;

@@ -3,6 +3,8 @@
 Bars: bit-exact for the quantiser's codes and scales, for dequantisation, embedding, RoPE and the
 argmax; max-abs-rel <= 1e-2 for every fp16 output that accumulates in fp32 (matmul, attention,
 softmax, norm, silu)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -631,6 +633,38 @@ def test_silu_mul(gpu):
         G.B.check(G.L().lcu_silu_mul(od.ptr + 2 * off, ad.ptr + 2 * off, bd.ptr + 2 * off, n2, None))
         got2 = G.host(od, (n2 + off,))[off:]
         assert (got2.view(np.uint16) == got[off:n2 + off].view(np.uint16)).all()
+    G.release()
+
+
+def test_silu_of_every_half(gpu):
+    """The short forms of exponential and division against the general ones: every a, with b of every kind."""
+    G = gpu
+    a = np.arange(65536, dtype=np.uint16).view(np.float16)
+    for value in (1.0, -0.37, 65504.0, 6e-8, -0.0, np.inf, np.nan):
+        b = np.full(65536, value, np.float16)
+        out = G.dev_keep(np.zeros(65536, np.float16))
+        G.B.check(G.L().lcu_silu_mul(out.ptr, G.dev_keep(a).ptr, G.dev_keep(b).ptr, 65536, None))
+        got, want = G.host(out, (65536,), np.float16), O.silu_mul(a, b)
+        assert (np.isnan(got) == np.isnan(want)).all()
+        assert (got.view(np.uint16) == want.view(np.uint16))[~np.isnan(want)].all(), value
+    G.release()
+
+
+@pytest.mark.parametrize("n,dim,ffn", [(65, 128, 10240), (100, 128, 16400), (129, 256, 10256), (300, 384, 5136), (512, 1024, 11008), (773, 2048, 6160), (1027, 2048, 6592), (1033, 2048, 6704), (1024, 1024, 13392)])
+def test_up_products_with_their_silu(gpu, n, dim, ffn):
+    """Large tiles whose columns alternate between W1 and W3: the bits of the two products and lcu_silu_mul, whatever is behind the last row
+    and column.  128, 192 and 256 columns, whole rounds and the rest, 128 rows."""
+    G, L = gpu, gpu.L()
+    rng = np.random.default_rng(n + ffn)
+    x = G.dev_keep(rng.standard_normal((n, dim)).astype(np.float16))
+    w = [G.dev_keep((rng.standard_normal((ffn, dim)) * 3 / dim ** 0.5).astype(np.float16)) for _ in range(2)]
+    t1, t3, want, got = (G.dev_keep(np.full((n + 1, ffn), -7, np.float16)) for _ in range(4))
+    ptrs = lambda bufs: (C.c_void_p * len(bufs))(*[b.ptr for b in bufs])
+    G.B.check(L.lcu_gemm_f16_nt_multi(ptrs([t1, t3]), x.ptr, ptrs(w), 2, n, dim, ffn, 0.0, None))
+    G.B.check(L.lcu_silu_mul(want.ptr, t1.ptr, t3.ptr, n * ffn, None))
+    G.B.check(L.lcu_batch_ffn_up(got.ptr, t1.ptr, t3.ptr, x.ptr, ptrs(w), None, 0, n, dim, ffn, None))
+    a, b = G.host(got, (n + 1, ffn), np.uint16), G.host(want, (n + 1, ffn), np.uint16)
+    assert (a == b).all() and (a[n] == np.float16(-7).view(np.uint16)).all()
     G.release()
 
 
