@@ -8,16 +8,15 @@
 // Four kernels:
 //   gemm_tile_kernel (gemm_tile.hpp): 256-row tiles of 128, 192 or 256 columns where these fill most of the
 //     chip, 256x128 with the K range split over workgroups, 128-row tiles of up to 128 rows and where only
-//     those of 128x128 fill most of the chip; fp16, uint8 (codes in blocks of 64 << n) and bfloat16 weights
+//     those of 128x128 fill most of the chip, else 128x64; fp16, uint8 (codes in blocks of 64 << n) and bfloat16 weights
 //   gemm_stream_kernel (gemm_stream.hpp): 2..64 rows, the K range split over workgroups
-//   gemm_dl_kernel (K a multiple of 128, every other shape of the model family): both operands travel
-//     from global memory straight into a ring of 2-3 LDS stages with global_load_lds_dwordx4 (no
-//     staging registers, no LDS store instructions); rows are unpadded and the 16-byte chunks of a
-//     row are permuted so that neither the requests nor the fragment reads meet in a bank; tiles
-//     of 128x64 (other blocks of codes: 256x128 and 128x128 too) with 4 or 8 wavefronts (a second group of four may take the
-//     other half of a 128-wide K stage), chosen by how many tiles the product has; uint8 weights
-//     add a ring of codes and of scales and are turned into fp16 -- exactly fp16((q - 127.5) *
-//     scale), llama_cu.cu:287-289 -- once per block tile
+//   gemm_dl_kernel (K a multiple of 128; a short K where 128x128 tiles fill the chip, other blocks of codes, splits of few rows,
+//     bfloat16 experts and small tiles): both operands travel from global memory straight into a ring of 2-3 LDS
+//     stages with global_load_lds_dwordx4 (no staging registers, no LDS store instructions); rows are
+//     unpadded and the 16-byte chunks of a row are permuted so that neither the requests nor the fragment
+//     reads meet in a bank; 4 or 8 wavefronts (a second group of four may take the other half of a 128-wide K
+//     stage), chosen by how many tiles the product has; uint8 weights add a ring of codes and of scales and are
+//     turned into fp16 -- exactly fp16((q - 127.5) * scale), llama_cu.cu:287-289 -- once per block tile
 //   Where the K range is split -- 2..64 rows, few large tiles and a long K -- a second launch adds the
 //     fp32 partial sums in split order (launch_skinny; large_tile_splits in gemm_plan.hpp)
 //   gemm_kernel (ragged K): global -> registers -> padded LDS with two LDS buffers and two
@@ -909,7 +908,7 @@ inline int block_shift(int block) {
 }
 
 // A launch of gemm_tile_kernel; splits > 1: the K stages of every tile dealt to that many workgroups, fp32 sums to part.
-template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP>
+template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP, int CHAINS = 1>
 int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits = 1,
                 float* part = nullptr, columns_t which = {}, int step = 1) {
   using shape = tile_shape<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP>;
@@ -917,7 +916,7 @@ int launch_tile(EP const& ep, operands_t op, const void* A, int M, int K, int N,
   if (which.from > 0) op = last_matrix(op);
   const int tiles_n_per = (N - which.from + BN - 1) / BN, tiles_n = which.tiles > 0 ? which.tiles : tiles_n_per * op.n_mats;
   op.more.tiles_n_per = op.n_mats > 1 ? tiles_n_per : 0;
-  auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP>;
+  auto kernel = gemm_tile_kernel<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP, CHAINS>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -1442,10 +1441,9 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
                   const rotary_epilogue* rotary = nullptr, bool* rotated = nullptr) {
   // Tile choice.  Large tiles read fewer operand bytes per multiply-add and pay per output for fewer
   // barriers.  So: tiles of 256 rows when those of 256x128 still give 160 workgroups, or with few of them
-  // and a long K the splits of each (large_tile_splits); 128x128 when these give 160; 128x64 with four
-  // wavefronts when there are more of them than compute units (two fit); else 128x64 with two groups of four
-  // wavefronts splitting the K stage, because then the grid cannot give a compute unit a second workgroup
-  // (512x4096x4096 29 us, with one group 34, on the register-staged kernel 36.5; 400x2048x2048 13.6, 17.5, 19.1).
+  // and a long K the splits of each (large_tile_splits); 128x128 when these give 160; 128x64 with a ring of
+  // three stages when there are more of them than compute units (two fit); else 128x64 with a longer ring, the
+  // even and the odd stages summed apart.
   // gemm_tile_kernel pays about 1 us more per tile before its first and behind its last stage than gemm_dl_kernel (a longer ring
   // to fill, outputs through LDS) and less per stage: over a short K the other kernels stay, by the lines below.
   // Several matrices of one shape (op.n_mats > 1) count as one product with n_mats * N columns; only uint8
@@ -1550,7 +1548,18 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
         return launch_tile<128, 128, 2, 2, 4, 4, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
       }
     } else {
-      if (plan.tiles == row_tiles::narrow) return launch_dl<128, 64, 2, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+      // More 128x64 tiles than compute units, two to a compute unit: against gemm_dl_kernel 40 drawn products of K 256 to 5000 take 0.98 of the time
+      // (0.92 to 1.02; 1038x4096x2048 37.5 / 34.8 us), uint8 0.78 (0.70 to 0.86; 559x1792x3352 25.6 / 18.0): every code converted once, not twice.
+      if (plan.tiles == row_tiles::narrow) {
+        if constexpr (!U8) return launch_tile<128, 64, 2, 2, 3, 3, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
+        if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 3, 3, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        return launch_dl<128, 64, 2, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+      }
+      // us, two groups of four wavefronts that halve the stages on gemm_dl_kernel / four that sum them in turn here: 512 rows of K 256, 512, 1024, 2048,
+      // 4096 (4096 columns; 2048) 6.3 / 5.2, 7.2 / 6.1, 10.9 / 9.7, 15.4 / 15.0, 28.9 / 29.3; 300x4096x4096 25.1 / 23.8, 1000x2048x2048 17.2 / 15.7; 70
+      // drawn products 0.91 of the time (0.82 to 1.03), 45 in uint8 0.84 (0.79 to 0.88).  24 KB a stage on their way into LDS bound it over a long K.
+      if constexpr (!U8) return launch_tile<128, 64, 2, 2, 4, 4, false, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
+      if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 4, 4, true, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
       return launch_dl<128, 64, 2, 2, 2, 3, U8>(op, A, M, K, N, block, beta, st);
     }
   }
@@ -1742,9 +1751,9 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     if (tm(128) * tn(64) > 128) return launch_bf16<128, 64, 4, 1, 1, 3>(ep, A, W, tm(128), M, K, N, st);
     return launch_bf16<64, 64, 2, 1, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   } else {
-    if (tm(128) * tn(64) > 256) return launch_bf16<128, 64, 2, 2, 1, 3>(ep, A, W, tm(128), M, K, N, st);
+    if (tm(128) * tn(64) > 256) return launch_tile<128, 64, 2, 2, 3, 3, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
     if (K % 128 == 0 && tm(128) * tn(64) > 128) {
-      return launch_bf16<128, 64, 2, 2, 2, 3>(ep, A, W, tm(128), M, K, N, st);
+      return launch_tile<128, 64, 2, 2, 4, 4, false, false, linear_epilogue<false, GATED>, 2>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
     }
     return launch_bf16<64, 64, 2, 2, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   }

@@ -35,7 +35,7 @@ enum class row_tiles {
   split_large,  // 256x128, K dealt to `splits` workgroups
   medium,       // 128x128
   narrow,       // 128x64, two to a compute unit
-  halves        // 128x64 with two groups of wavefronts, one to a compute unit
+  halves        // 128x64, one to a compute unit
 };
 struct row_plan_t {
   row_tiles tiles;

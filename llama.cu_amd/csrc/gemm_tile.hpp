@@ -112,7 +112,8 @@ struct tile_shape {
   static_assert(LDS <= 160 * 1024 && WR % 64 == 0 && WC % 16 == 0, "tile");
 };
 
-template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP>
+// CHAINS 2: the even and the odd stages of K are summed apart, and the two sums added (K a multiple of 128).
+template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP, int CHAINS = 1>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0, int block_shift,
     int M, int K, int N, float beta, int tiles_m, int tiles_n, int from, float* __restrict__ part, int splits, int step, more_matrices_t more, EP ep) {
@@ -237,11 +238,14 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
     }
   };
 
-  float4_t acc[TM][TN];
+  float4_t acc[TM][TN], odd[CHAINS == 2 ? TM : 1][CHAINS == 2 ? TN : 1];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = (float4_t)(0.0f);
+    for (int j = 0; j < TN; ++j) {
+      acc[i][j] = (float4_t)(0.0f);
+      if constexpr (CHAINS == 2) odd[i][j] = (float4_t)(0.0f);
+    }
   }
   const int frag_row = lane & 15, frag_chunk = lane >> 4, turn = (frag_row / 2) % 8;
   uint32_t pos[2];
@@ -293,23 +297,29 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
       fb[h][j][4 * w + 2 * high + 1] = y.y;
     }
   };
-  const auto multiply = [&](int h, int i) {
+  const auto multiply = [&](int h, int i, auto chain) {
     const int a = i / TN, b = (a & 1) ? TN - 1 - i % TN : i % TN;
-    if constexpr (EP::BF16) {
-      acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fa[h][a]), __builtin_bit_cast(bf16x8_t, fb[h][b]),
-                                                          acc[a][b], 0, 0, 0);
+    const auto add_to = [&](float4_t& sum) {
+      if constexpr (EP::BF16) {
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fa[h][a]), __builtin_bit_cast(bf16x8_t, fb[h][b]), sum, 0, 0, 0);
+      } else {
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[h][a], fb[h][b], sum, 0, 0, 0);
+      }
+    };
+    if constexpr (decltype(chain)::value == 1) {
+      add_to(odd[a][b]);
     } else {
-      acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[h][a], fb[h][b], acc[a][b], 0, 0, 0);
+      add_to(acc[a][b]);
     }
   };
   // the products of half h, with the reads spread over the first five eighths, the requests over all of them, and the
   // conversions of the next half (U8) over the last half (of half 1, whose codes are read first) or all (of half 0)
-  const auto half_stage = [&](int h, auto n_reads, auto&& do_read, auto n_requests, auto&& do_request, auto n_converts, int convert_stage) {
+  const auto half_stage = [&](int h, auto n_reads, auto&& do_read, auto n_requests, auto&& do_request, auto n_converts, int convert_stage, auto chain) {
     constexpr int NR = decltype(n_reads)::value, NQ = decltype(n_requests)::value, SPREAD = PRODUCTS * 5 / 8;
     constexpr int NC = decltype(n_converts)::value;
     static_for<PRODUCTS>([&](auto at) {
       constexpr int i = decltype(at)::value;
-      multiply(h, i);
+      multiply(h, i, chain);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (i < SPREAD) {
 #pragma unroll
@@ -329,20 +339,20 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   // requests of the next stage have landed the barrier says both for everybody.  Then the second half, with the next stage's first half
   // on its way and the stages NA and NB ahead requested into this one's slots.  Of a stage's requests the lhs goes first: when that of
   // stage t + 1 has to be there, the columns asked for behind it and all of the NA - 2 stages since may still be out.
-  const auto stage = [&](int t, int a_slot, int b_slot, int a_next, int b_next, auto more_follow) {
+  const auto stage = [&](int t, int a_slot, int b_slot, int a_next, int b_next, auto more_follow, auto chain) {
     constexpr bool MORE = decltype(more_follow)::value;
     half_stage(0, std::integral_constant<int, READS1>{}, [&](int k) { read(a_slot, b_slot, 1, k); }, std::integral_constant<int, 0>{}, [](int) {},
-               std::integral_constant<int, CONVERTS>{}, t);
+               std::integral_constant<int, CONVERTS>{}, t, chain);
     if constexpr (MORE) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       wait_vmcnt<(NA - 2) * P + BEHIND>();
       asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       half_stage(1, std::integral_constant<int, READS0>{}, [&](int k) { read(a_next, b_next, 0, k); }, std::integral_constant<int, P>{},
-                 [&](int k) { issue(t + NA, a_slot, t + NB, b_slot, k); }, std::integral_constant<int, CONVERTS>{}, t + 1);
+                 [&](int k) { issue(t + NA, a_slot, t + NB, b_slot, k); }, std::integral_constant<int, CONVERTS>{}, t + 1, chain);
     } else {
       half_stage(1, std::integral_constant<int, 0>{}, [](int) {}, std::integral_constant<int, 0>{}, [](int) {},
-                 std::integral_constant<int, 0>{}, 0);
+                 std::integral_constant<int, 0>{}, 0, chain);
     }
   };
 
@@ -365,14 +375,32 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   for (int k = 0; k < CONVERTS; ++k) convert(0, k, 0);
   __builtin_amdgcn_sched_barrier(0);
   int a_slot = 0, b_slot = 0;
-  for (int t = 0; t < nt - 1; ++t) {
+  constexpr std::integral_constant<int, 0> even_chain{};
+  constexpr std::integral_constant<int, CHAINS - 1> odd_chain{};
+  const auto step_on = [&](int t, auto chain) {
     end_at(t + NA, t + NB);
     const int a_next = a_slot + 1 == NA ? 0 : a_slot + 1, b_next = JOINT ? a_next : b_slot + 1 == NB ? 0 : b_slot + 1;
-    stage(t, a_slot, b_slot, a_next, b_next, std::true_type{});
+    stage(t, a_slot, b_slot, a_next, b_next, std::true_type{}, chain);
     a_slot = a_next;
     b_slot = b_next;
+  };
+  if constexpr (CHAINS == 2) {
+    for (int t = 0; t < nt - 2; t += 2) {
+      step_on(t, even_chain);
+      step_on(t + 1, odd_chain);
+    }
+    step_on(nt - 2, even_chain);
+  } else {
+    for (int t = 0; t < nt - 1; ++t) step_on(t, even_chain);
   }
-  stage(nt - 1, a_slot, b_slot, 0, 0, std::false_type{});
+  stage(nt - 1, a_slot, b_slot, 0, 0, std::false_type{}, odd_chain);
+  if constexpr (CHAINS == 2) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] += odd[i][j];
+    }
+  }
   wait_vmcnt<0>();  // the requests behind the last stage have written their zeros
   __syncthreads();  // LDS is free
 
