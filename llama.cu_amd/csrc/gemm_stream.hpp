@@ -8,7 +8,7 @@
 // as many wavefronts as give every compute unit one (stream_waves): 128-column tiles with a common ring left 288 workgroups
 // of Wq, Wk, Wv for 256 compute units.  (Loaded into registers as the matrix instructions want them, sixteen rows
 // per 16 lanes, a line takes four requests: slower for fp16 than the common ring.)
-// M = 8 with the launch that adds the splits, fp16 three times (4096, 4096) 26.0 -> 22.7 us, twice (N, K) = (11008, 4096) 45 -> 42,
+// M = 8 with a launch that adds the splits, fp16 three times (4096, 4096) 26.0 -> 22.7 us, twice (N, K) = (11008, 4096) 45 -> 42,
 // (4096, 4096) 12.1 -> 12.4; uint8 three times (6656, 6656) 61 -> 35, twice (17920, 6656) 104 -> 57, (6656, 17920) 62 -> 37.  Rows of
 // 8 KB meet in the same memory channels: K = 4224 takes a tenth less than 4096.
 #pragma once
@@ -44,11 +44,22 @@ __device__ __forceinline__ void wait_requests(int more) {
   }
 }
 
-template <int TM, bool U8, bool BF16>
+// JOIN: what becomes of the sums.  separate_sums: they go to part, and another launch adds them up.  Otherwise a workgroup has every split of its
+// columns (MATRICES 2: of those of both matrices), a wavefront each, and lhs lies in LDS whole; the sums meet in LDS, are added in the order of
+// the splits, and join(matrix, row, first of two columns, sums of the two [MATRICES]) makes outputs of them.  What bounded the second launch was its
+// start and its first loads, 2 to 4 us for a few hundred KB.  us, two launches / one, 8 rows: fp16 (K, N) = (4096, 4096) three times and the rotary
+// 24.4 / 21.0, (4096, 11008) twice and the SiLU 44.2 / 41.2, (2048, 2048) three times 12.3 / 8.2, uint8 (4096, 4096) three times 19.8 / 15.7; alone, fp16
+// 13x2048x6656 12.0 / 9.1, 40x256x16384 9.5 / 6.4, uint8 20x1408x6656 11.5 / 7.3; over 80 drawn shapes of 2 to 62 rows 12 to 58 % sooner where one launch does it.
+struct separate_sums {
+  static constexpr bool JOINED = false;
+  static constexpr int MATRICES = 1;
+};
+
+template <int TM, bool U8, bool BF16, class JOIN = separate_sums>
 __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kernel(const half_t* __restrict__ A, const void* __restrict__ W0,
                                                                                const half_t* __restrict__ S0, int block_shift, int M, int K,
                                                                                int N, int tiles, int kc, float* __restrict__ part, int splits,
-                                                                               more_matrices_t more) {
+                                                                               more_matrices_t more, JOIN join) {
   constexpr int RING = STREAM_RING, UNIT = stream_unit(U8), P = U8 ? 3 : 2;  // requests per unit
   constexpr int PER = U8 ? 2 : 1;                                           // stages per unit
   extern __shared__ __attribute__((aligned(16))) unsigned char stream_mem[];
@@ -57,13 +68,17 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
   // Tiles of one matrix, then of the next; the same for the next split.  Consecutive workgroups go round the eight XCDs: each
   // gets one run of the tiles, the same of every split, so that what adds the splits up may find them in one L2 (bfloat16,
   // 8 rows, 4096x2048, both launches: 11.9 us with the tiles dealt one by one, 8.3 so; fp16 4096x32000 66 / 61).
-  const int mats = more.tiles_n_per, nb = tiles * mats;
-  const int split = blockIdx.x / nb, bx = blockIdx.x - split * nb, xcd = bx % 8;
-  const int rest = xcd * (nb / 8) + min(xcd, nb % 8) + bx / 8, g = rest / tiles;
+  constexpr bool JOINED = JOIN::JOINED;
+  // JOINED: the sixteens of columns of all matrices are dealt, `groups` to a workgroup, `per` wavefronts to one of them.
+  const int sixteens = (N + 15) / 16, per = JOINED ? splits * JOIN::MATRICES : 1, groups = waves / per;
+  const int mats = more.tiles_n_per, nb = JOINED ? tiles : tiles * mats;
+  const int split = JOINED ? wave % splits : blockIdx.x / nb, bx = JOINED ? blockIdx.x : blockIdx.x - split * nb, xcd = bx % 8;
+  const int rest = xcd * (nb / 8) + min(xcd, nb % 8) + bx / 8, sixteen = rest * groups + wave / per;
+  const int g = !JOINED ? rest / tiles : JOIN::MATRICES == 2 ? wave % per / splits : sixteen / sixteens;
   const void* W = g == 0 ? W0 : (g == 1 ? more.W[0] : more.W[1]);
   const half_t* S = g == 0 ? S0 : (g == 1 ? more.S[0] : more.S[1]);
-  const int n0 = ((rest - g * tiles) * waves + wave) * 16;
-  const bool mine = n0 < N;
+  const int n0 = (JOINED ? (JOIN::MATRICES == 2 ? sixteen : sixteen - g * sixteens) : (rest - g * tiles) * waves + wave) * 16;
+  const bool mine = n0 < N && g < mats;
   const int nt_all = K / 64;
   const int stage0 = (int)((long)split * nt_all / splits), stage1 = (int)((long)(split + 1) * nt_all / splits);
   // stages are counted from an even one, so that units of two are whole lines of codes
@@ -78,7 +93,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
     const int pieces = kc / 8;
     for (int u = wave; u * 64 < M * pieces; u += waves) {
       const int piece = min(u * 64 + lane, M * pieces - 1), row = piece / pieces, at = piece - row * pieces;
-      const int k = min((base * 64 + chunk * kc) + ((at & ~15) | ((at ^ row) & 15)) * 8, K - 8);
+      const int k = min(((JOINED ? 0 : base * 64) + chunk * kc) + ((at & ~15) | ((at ^ row) & 15)) * 8, K - 8);
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(A + (size_t)row * K + k),
                    "s"(lds0 + (chunk & 1) * chunk_bytes + u * 1024)
                    : "memory", "m0");
@@ -150,7 +165,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
 #pragma unroll
       for (int h = 0; h < 2; ++h) w[h] = *reinterpret_cast<const half8_t*>(row + (((4 * h + group) ^ turn) << 4));
     }
-    const int chunk = s * 64 / kc, p0 = (s * 64 - chunk * kc) / 8;
+    const int chunk = JOINED ? 0 : s * 64 / kc, p0 = JOINED ? (base + s) * 8 : (s * 64 - chunk * kc) / 8;
     const unsigned char* lhs = stream_mem + (chunk & 1) * chunk_bytes;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -167,7 +182,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
     }
   };
 
-  const int chunk_units = kc / 64 / PER, u0 = first / PER;
+  const int chunk_units = JOINED ? units : kc / 64 / PER, u0 = first / PER;
   request_chunk(0);
   if (mine) {
 #pragma unroll
@@ -202,6 +217,36 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
         if (PER == 1 || (s >= first && s < end)) multiply(slot, s);
       }
     }
+  }
+  if constexpr (JOINED) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");  // everybody has read lhs, whose place the sums take: [wavefront][row][16]
+    float* sums = reinterpret_cast<float*>(stream_mem);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sums[(wave * TM * 16 + i * 16 + group * 4 + e) * 16 + col] = acc[i][e];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    for (int at = threadIdx.x; at < groups * M * 8; at += blockDim.x) {
+      const int c = at % 8 * 2, m = at / 8 % M, block = at / 8 / M, of = rest * groups + block;
+      const int matrix = JOIN::MATRICES == 2 ? 0 : of / sixteens, n = (of - matrix * sixteens) * 16 + c;
+      if (n >= N || matrix >= mats) continue;
+      float2 total[JOIN::MATRICES];
+#pragma unroll
+      for (int x = 0; x < JOIN::MATRICES; ++x) {
+        const float* from = sums + ((block * per + x * splits) * TM * 16 + m) * 16 + c;
+        total[x] = *reinterpret_cast<const float2*>(from);
+        for (int s = 1; s < splits; ++s) {
+          const float2 more_of_it = *reinterpret_cast<const float2*>(from + s * TM * 256);
+          total[x].x += more_of_it.x;
+          total[x].y += more_of_it.y;
+        }
+      }
+      join(matrix, m, n, total);
+    }
+    return;
   }
   if (!mine) return;
   // register e of a lane is row 4 group + e, column col of its tile

@@ -400,6 +400,35 @@ def test_gemm_f16_few_rows(gpu, M, K, N):
     G.release()
 
 
+# few rows whose splits are added up where they end: one to four row tiles, workgroups that hold the last columns of one matrix and the first of
+# the next, columns past the last whole sixteen, lhs that fills its place (64x512, 8x4096) and lhs that does not fit (9x4096)
+@pytest.mark.parametrize("M,K,N,mats,block", [(2, 512, 3000, 3, 0), (16, 2048, 1002, 3, 0), (17, 1920, 2034, 2, 0), (32, 1024, 1300, 3, 128), (33, 896, 3010, 3, 64),
+                                              (64, 512, 4098, 3, 0), (64, 512, 4098, 2, 256), (8, 4096, 1346, 3, 128), (9, 4096, 2050, 3, 0), (3, 8192, 1026, 1, 0)])
+def test_few_rows_added_up_where_they_end(gpu, M, K, N, mats, block):
+    G = gpu
+    check, L, VP = G.B.check, G.L(), G.B.vp
+    x, ws = normal((M, K), 0, 450, 1.0), [normal((N, K), 0, 451 + g, 0.02) for g in range(mats)]
+    codes = [O.quantize_absmax_u8(w, block) for w in ws] if block else []
+    refs = ([O.matmul_nt_kernel_order(x, codes=c, scales=s, block=block, n_mats=mats) for c, s in codes] if block else
+            [O.matmul_nt_kernel_order(x, w, n_mats=mats) for w in ws])
+    wd, sd = [G.dev_keep(c[0]) for c in codes] or [G.dev_keep(w) for w in ws], [G.dev_keep(c[1]) for c in codes]
+    w_arr, s_arr = (VP * mats)(*[w.ptr for w in wd]), (VP * mats)(*[s.ptr for s in sd]) if block else None
+    # lhs by itself, then inside the first output, which may only be written when all of lhs has been read
+    whole = np.zeros(M * max(K, N), dtype=np.float16)
+    whole[:M * K] = x.reshape(-1)
+    for same in (False, True):
+        lhs = G.dev_keep(whole)
+        outs = [lhs if same and g == 0 else G.empty((M, N)) for g in range(mats)]
+        o_arr = (VP * mats)(*[o.ptr for o in outs])
+        if block:
+            check(L.lcu_gemm_f16u8_nt_multi(o_arr, lhs.ptr, w_arr, s_arr, mats, M, K, N, block, 0.0, None))
+        else:
+            check(L.lcu_gemm_f16_nt_multi(o_arr, lhs.ptr, w_arr, mats, M, K, N, 0.0, None))
+        for o, ref in zip(outs, refs):
+            assert G.ulp_mismatch(G.host(o, (M, N)), ref) == 0.0, O.gemm_plan(M, K, N, block > 0, block or 128, mats)
+    G.release()
+
+
 # uint8 tiles of 256 rows at their edges: 128 and 256 columns, K split over workgroups, blocks of one, two and four K
 # stages, and a block that takes the other kernel
 @pytest.mark.parametrize("M,K,N,block", [(2049, 256, 4100, 64), (4096, 128, 4090, 128), (2300, 512, 6000, 256), (300, 5120, 1030, 128),
