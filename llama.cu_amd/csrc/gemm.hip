@@ -1146,9 +1146,9 @@ bool scale_words_ok(const operands_t& op, int K, int N, int block) {
   }
 }
 
-template <int TM, bool U8, class JOIN>
+template <int TM, bool U8, bool BF16, class JOIN>
 int launch_joined_rows(JOIN const& join, operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, int waves, int tiles) {
-  auto kernel = gemm_stream_kernel<TM, U8, false, JOIN>;
+  auto kernel = gemm_stream_kernel<TM, U8, BF16, JOIN>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -1161,6 +1161,13 @@ int launch_joined_rows(JOIN const& join, operands_t op, const half_t* A, int M, 
                                                                                          splits, op.more, join);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
+}
+
+template <bool U8, bool BF16, class JOIN>
+int launch_joined_shape(JOIN const& join, operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, stream_join_t shape) {
+  if (M <= 16) return launch_joined_rows<1, U8, BF16>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
+  if (M <= 32) return launch_joined_rows<2, U8, BF16>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
+  return launch_joined_rows<4, U8, BF16>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
 }
 
 inline bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
@@ -1187,21 +1194,14 @@ int launch_joined(JOIN const& join, operands_t op, const half_t* A, int M, int K
   if (plan.splits == 0) return LCU_OK;
   const stream_join_t shape = plan_stream_join(N, op.n_mats, JOIN::MATRICES, plan.splits, ds->compute_units, stream_max_waves(U8));
   if (shape.waves == 0) return LCU_OK;
-  int rc;
-  if (M <= 16) {
-    rc = launch_joined_rows<1, U8>(join, op, A, M, K, N, block, st, plan.splits, shape.waves, shape.tiles);
-  } else if (M <= 32) {
-    rc = launch_joined_rows<2, U8>(join, op, A, M, K, N, block, st, plan.splits, shape.waves, shape.tiles);
-  } else {
-    rc = launch_joined_rows<4, U8>(join, op, A, M, K, N, block, st, plan.splits, shape.waves, shape.tiles);
-  }
+  const int rc = launch_joined_shape<U8, false>(join, op, A, M, K, N, block, st, plan.splits, shape);
   *done = rc == LCU_OK;
   return rc;
 }
 
 // what splitk_reduce_kernel makes of the sums
 struct f16_join {
-  static constexpr bool JOINED = true;
+  static constexpr bool JOINED = true, GATED = false;
   static constexpr int MATRICES = 1;
   half_t* out[3];
   int N;
@@ -1388,7 +1388,7 @@ __global__ __launch_bounds__(256) void reduce_rope_store_kernel(half_t* __restri
 // the same, two products and SiLU, and the bare sums, where the product's workgroups have all the splits of their columns (gemm_stream_kernel)
 template <class ROWS>
 struct rope_join {
-  static constexpr bool JOINED = true;
+  static constexpr bool JOINED = true, GATED = false;
   static constexpr int MATRICES = 1;
   half_t* q_out;
   ROWS rows;
@@ -1402,7 +1402,7 @@ struct rope_join {
   }
 };
 struct silu_join {
-  static constexpr bool JOINED = true;
+  static constexpr bool JOINED = true, GATED = false;
   static constexpr int MATRICES = 2;
   half_t* out;
   int ffn;
@@ -1415,7 +1415,7 @@ struct silu_join {
 };
 
 struct sum_join {
-  static constexpr bool JOINED = true;
+  static constexpr bool JOINED = true, GATED = false;
   static constexpr int MATRICES = 1;
   float* part;
   int N;
@@ -1820,6 +1820,44 @@ int add_splits(linear_epilogue<false, GATED> const& ep, const float* part, int M
   return LCU_OK;
 }
 
+template <bool GATED_>
+struct linear_join {
+  static constexpr bool JOINED = true, GATED = GATED_;
+  static constexpr int MATRICES = GATED ? 2 : 1;
+  linear_epilogue<false, GATED> ep;
+  int N;
+  __device__ __forceinline__ void operator()(int, int row, int c, const float2 (&x)[MATRICES]) const {
+    if constexpr (GATED) {
+      ep.store_gated(row, c, x[0].x, x[1].x);
+      ep.store_gated(row, c + 1, x[0].y, x[1].y);
+    } else {
+      ep.store(row, c, x[0].x);
+      if (c + 1 < N) ep.store(row, c + 1, x[0].y);
+    }
+  }
+};
+
+// The same in one launch (launch_joined; us, two / one: 6x2048x2048 6.8 / 5.6, 13x2048x6656 12.5 / 9.2, 42x768x6656 11.4 / 7.4, 11x2048x256 7.7 / 4.9; 40
+// drawn shapes of 2 to 62 rows 7 to 71 % sooner where K is split).  *done = false, with nothing launched, where lhs does not fit LDS whole, the workgroups would take a
+// second round, or the outputs lie over lhs.
+template <bool GATED>
+int bf16_joined(linear_epilogue<false, GATED> const& ep, const void* A, const void* W, int M, int K, int N, int splits, long cus, hipStream_t st, bool* done) {
+  *done = false;
+  const size_t lhs_bytes = (size_t)M * K * 2;
+  const int outs = GATED ? N / 2 : N;
+  if (K % 128 != 0 || lhs_bytes > (size_t)STREAM_LHS || (GATED && outs % 32 != 0) ||
+      overlap(ep.out, ((size_t)(M - 1) * ep.ldo + outs) * (ep.out_f32 ? 4 : 2), A, lhs_bytes) ||
+      (ep.tail && overlap(ep.tail, ((size_t)(M - 1) * ep.ld_tail + (N - ep.tail_from)) * 4, A, lhs_bytes))) {
+    return LCU_OK;
+  }
+  const int mats = GATED ? 2 : 1;
+  const stream_join_t shape = plan_stream_join(outs, mats, mats, splits, cus, stream_max_waves(false));
+  if (shape.waves == 0) return LCU_OK;
+  const int rc = launch_joined_shape<false, true>(linear_join<GATED>{ep, N}, single_matrix(nullptr, W, nullptr), (const half_t*)A, M, K, N, 0, st, splits, shape);
+  *done = rc == LCU_OK;
+  return rc;
+}
+
 // Few rows: the weight stream is what counts (see launch_skinny).  *done = false when the shape gives no second
 // workgroup to a tile.
 template <bool GATED>
@@ -1832,8 +1870,9 @@ int bf16_skinny(linear_epilogue<false, GATED> const& ep, const void* A, const vo
   int splits = std::min((ds->compute_units + tiles - 1) / tiles, K / BK / 4);
   while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws.bytes) --splits;
   if (splits < 2) return LCU_OK;
+  int rc = bf16_joined<GATED>(ep, A, W, M, K, N, splits, ds->compute_units, st, done);
+  if (rc != LCU_OK || *done) return rc;
   float* part = (float*)ws.ptr;
-  int rc;
   if (streams(M, N, 1, splits, K / BK, (long)tiles * splits, ds->compute_units, false, true)) {
     rc = launch_stream<false, true>(single_matrix(nullptr, W, nullptr), A, M, K, N, 0, st, splits, part, ds->compute_units);
   } else {

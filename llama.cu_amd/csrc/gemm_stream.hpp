@@ -50,8 +50,9 @@ __device__ __forceinline__ void wait_requests(int more) {
 // start and its first loads, 2 to 4 us for a few hundred KB.  us, two launches / one, 8 rows: fp16 (K, N) = (4096, 4096) three times and the rotary
 // 24.4 / 21.0, (4096, 11008) twice and the SiLU 44.2 / 41.2, (2048, 2048) three times 12.3 / 8.2, uint8 (4096, 4096) three times 19.8 / 15.7; alone, fp16
 // 13x2048x6656 12.0 / 9.1, 40x256x16384 9.5 / 6.4, uint8 20x1408x6656 11.5 / 7.3; over 80 drawn shapes of 2 to 62 rows 12 to 58 % sooner where one launch does it.
+// GATED: the two are blocks of 32 columns of one matrix, a gate's and behind it an up block; the columns are those of the outputs.
 struct separate_sums {
-  static constexpr bool JOINED = false;
+  static constexpr bool JOINED = false, GATED = false;
   static constexpr int MATRICES = 1;
 };
 
@@ -70,15 +71,17 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
   // 8 rows, 4096x2048, both launches: 11.9 us with the tiles dealt one by one, 8.3 so; fp16 4096x32000 66 / 61).
   constexpr bool JOINED = JOIN::JOINED;
   // JOINED: the sixteens of columns of all matrices are dealt, `groups` to a workgroup, `per` wavefronts to one of them.
-  const int sixteens = (N + 15) / 16, per = JOINED ? splits * JOIN::MATRICES : 1, groups = waves / per;
+  const int outs = JOIN::GATED ? N / 2 : N, sixteens = (outs + 15) / 16, per = JOINED ? splits * JOIN::MATRICES : 1, groups = waves / per;
   const int mats = more.tiles_n_per, nb = JOINED ? tiles : tiles * mats;
   const int split = JOINED ? wave % splits : blockIdx.x / nb, bx = JOINED ? blockIdx.x : blockIdx.x - split * nb, xcd = bx % 8;
   const int rest = xcd * (nb / 8) + min(xcd, nb % 8) + bx / 8, sixteen = rest * groups + wave / per;
-  const int g = !JOINED ? rest / tiles : JOIN::MATRICES == 2 ? wave % per / splits : sixteen / sixteens;
+  const int x = wave % per / splits;  // MATRICES 2: which of them
+  const int g = !JOINED ? rest / tiles : JOIN::GATED ? 0 : JOIN::MATRICES == 2 ? x : sixteen / sixteens;
   const void* W = g == 0 ? W0 : (g == 1 ? more.W[0] : more.W[1]);
   const half_t* S = g == 0 ? S0 : (g == 1 ? more.S[0] : more.S[1]);
-  const int n0 = (JOINED ? (JOIN::MATRICES == 2 ? sixteen : sixteen - g * sixteens) : (rest - g * tiles) * waves + wave) * 16;
-  const bool mine = n0 < N && g < mats;
+  const int of_matrix = !JOINED ? (rest - g * tiles) * waves + wave : JOIN::MATRICES == 2 ? sixteen : sixteen - g * sixteens;
+  const int n0 = JOIN::GATED ? of_matrix / 2 * 64 + x * 32 + of_matrix % 2 * 16 : of_matrix * 16;
+  const bool mine = of_matrix < sixteens && g < mats;
   const int nt_all = K / 64;
   const int stage0 = (int)((long)split * nt_all / splits), stage1 = (int)((long)(split + 1) * nt_all / splits);
   // stages are counted from an even one, so that units of two are whole lines of codes
@@ -232,16 +235,16 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
     for (int at = threadIdx.x; at < groups * M * 8; at += blockDim.x) {
       const int c = at % 8 * 2, m = at / 8 % M, block = at / 8 / M, of = rest * groups + block;
       const int matrix = JOIN::MATRICES == 2 ? 0 : of / sixteens, n = (of - matrix * sixteens) * 16 + c;
-      if (n >= N || matrix >= mats) continue;
+      if (n >= outs || matrix >= mats) continue;
       float2 total[JOIN::MATRICES];
 #pragma unroll
-      for (int x = 0; x < JOIN::MATRICES; ++x) {
-        const float* from = sums + ((block * per + x * splits) * TM * 16 + m) * 16 + c;
-        total[x] = *reinterpret_cast<const float2*>(from);
+      for (int y = 0; y < JOIN::MATRICES; ++y) {
+        const float* from = sums + ((block * per + y * splits) * TM * 16 + m) * 16 + c;
+        total[y] = *reinterpret_cast<const float2*>(from);
         for (int s = 1; s < splits; ++s) {
           const float2 more_of_it = *reinterpret_cast<const float2*>(from + s * TM * 256);
-          total[x].x += more_of_it.x;
-          total[x].y += more_of_it.y;
+          total[y].x += more_of_it.x;
+          total[y].y += more_of_it.y;
         }
       }
       join(matrix, m, n, total);

@@ -121,6 +121,26 @@ def test_gated_linear_split(gpu, M, K, ff, plan):
     test_gated_linear_large_tiles(gpu, M, K, ff)
 
 
+# few rows whose splits are added up where they end: one to four row tiles, odd and ragged columns, lhs that just fits its place (16x2048, 64x512) and
+# that does not (17x2048), outputs over lhs, which may only be written when all of lhs has been read
+@pytest.mark.parametrize("M,K,N", [(1, 2048, 1531), (2, 512, 515), (16, 2048, 3071), (17, 2048, 1030), (31, 1024, 2047), (64, 512, 4100)])
+def test_linear_few_rows_in_one_launch(gpu, M, K, N):
+    test_linear_large_tiles(gpu, M, K, N)
+    rng = np.random.default_rng(N)
+    x, w = rounded(rng.standard_normal((M, K))), rounded(rng.standard_normal((N, K)) / K ** 0.5)
+    whole = np.zeros((1, M * max(K, N)))
+    whole[0, :M * K] = x.reshape(-1)
+    both = put(gpu, whole, BF16)
+    call(gpu, "lcu_linear", both, 0, N, both, put(gpu, w, BF16), None, 0, BF16, M, K, N)
+    close(get(gpu, both, (1, M * max(K, N)), BF16)[0, :M * N].reshape(M, N), (x.astype(np.float32) @ w.T.astype(np.float32)).astype(np.float64), BF16)
+    gpu.release()
+
+
+@pytest.mark.parametrize("M,K,ff", [(1, 1024, 1000), (16, 2048, 2816), (17, 1920, 700), (33, 896, 2030), (64, 512, 1990)])
+def test_gated_linear_few_rows_in_one_launch(gpu, M, K, ff):
+    test_gated_linear_large_tiles(gpu, M, K, ff)
+
+
 # 128 columns over a short K; gated tiles of 128x128 that outnumber the compute units, on both sides of theirs
 @pytest.mark.parametrize("M,K,N", [(1441, 512, 8900), (1441, 640, 8900),
                                    (8, 512, 30000), (40, 640, 25000),  # few rows in two rounds of workgroups
