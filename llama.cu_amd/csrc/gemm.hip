@@ -1044,17 +1044,21 @@ inline int stream_waves(int N, int n_mats, int splits, long cus, int most, long*
   return best;
 }
 
-// Workgroups that have every split of their columns: wavefronts of one (0: more than a round of them, or too few wavefronts for the splits)
+// Workgroups that have every split of their columns: wavefronts of one (0: more than a round of them, too few wavefronts for the splits, or no room for lhs)
 // and workgroups in all.  As few sixteens of columns as leave one round, four wavefronts at least.
 struct stream_join_t {
   int waves, tiles;
 };
-inline stream_join_t plan_stream_join(int N, int n_mats, int joined, int splits, long cus, int most) {
+inline stream_join_t plan_stream_join(int M, int K, int N, int n_mats, int joined, int splits, long cus, bool u8) {
   const int per = splits * joined;
   const long sixteens = (long)(N + 15) / 16 * (n_mats / joined);
-  for (int each = 1; each * per <= most; ++each) {
+  const int row_tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  if ((size_t)M * K * 2 > (size_t)STREAM_LDS) return {0, 0};
+  for (int each = 1; each * per <= stream_max_waves(u8); ++each) {
+    const int waves = each * per;
     const long tiles = (sixteens + each - 1) / each;
-    if (tiles <= cus && each * per >= 4) return {each * per, (int)tiles};
+    if (stream_joined_lhs(waves, row_tiles, M, K) + waves * STREAM_RING * stream_unit(u8) > STREAM_LDS) break;
+    if (tiles <= cus && waves >= 4) return {waves, (int)tiles};
   }
   return {0, 0};
 }
@@ -1153,11 +1157,12 @@ int launch_joined_rows(JOIN const& join, operands_t op, const half_t* A, int M, 
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
   if (!raised[dev & 15]) {
-    LCU_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, stream_lds(U8, stream_max_waves(U8))));
+    LCU_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS));
     raised[dev & 15] = true;
   }
   op.more.tiles_n_per = op.n_mats;
-  kernel<<<tiles, 64 * waves, stream_lds(U8, waves), st>>>(A, op.W, op.S, block_shift(block), M, K, N, tiles, K, nullptr,
+  const int lds = stream_joined_lhs(waves, TM, M, K) + waves * STREAM_RING * stream_unit(U8);
+  kernel<<<tiles, 64 * waves, lds, st>>>(A, op.W, op.S, block_shift(block), M, K, N, tiles, K, nullptr,
                                                                                          splits, op.more, join);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
@@ -1183,7 +1188,7 @@ int launch_joined(JOIN const& join, operands_t op, const half_t* A, int M, int K
   const device_state* ds = current_device_state();
   const workspace_t ws = workspace_for(st);
   const size_t lhs_bytes = (size_t)M * K * 2, out_bytes = (size_t)M * N * 2;
-  if (ds == nullptr || ws.ptr == nullptr || K % 128 != 0 || N % 2 != 0 || M < 2 || M > 64 || lhs_bytes > (size_t)STREAM_LHS ||
+  if (ds == nullptr || ws.ptr == nullptr || K % 128 != 0 || N % 2 != 0 || M < 2 || M > 64 ||
       (U8 && block_shift(block) < 0) || !scale_words_ok<U8>(op, K, N, block)) {
     return LCU_OK;
   }
@@ -1192,7 +1197,7 @@ int launch_joined(JOIN const& join, operands_t op, const half_t* A, int M, int K
   }
   const skinny_plan_t plan = plan_skinny<U8>(M <= 32 || U8 ? 32 : 64, M, K, N, op.n_mats, ds->compute_units, ws.bytes);
   if (plan.splits == 0) return LCU_OK;
-  const stream_join_t shape = plan_stream_join(N, op.n_mats, JOIN::MATRICES, plan.splits, ds->compute_units, stream_max_waves(U8));
+  const stream_join_t shape = plan_stream_join(M, K, N, op.n_mats, JOIN::MATRICES, plan.splits, ds->compute_units, U8);
   if (shape.waves == 0) return LCU_OK;
   const int rc = launch_joined_shape<U8, false>(join, op, A, M, K, N, block, st, plan.splits, shape);
   *done = rc == LCU_OK;
@@ -1845,13 +1850,13 @@ int bf16_joined(linear_epilogue<false, GATED> const& ep, const void* A, const vo
   *done = false;
   const size_t lhs_bytes = (size_t)M * K * 2;
   const int outs = GATED ? N / 2 : N;
-  if (K % 128 != 0 || lhs_bytes > (size_t)STREAM_LHS || (GATED && outs % 32 != 0) ||
+  if (K % 128 != 0 || (GATED && outs % 32 != 0) ||
       overlap(ep.out, ((size_t)(M - 1) * ep.ldo + outs) * (ep.out_f32 ? 4 : 2), A, lhs_bytes) ||
       (ep.tail && overlap(ep.tail, ((size_t)(M - 1) * ep.ld_tail + (N - ep.tail_from)) * 4, A, lhs_bytes))) {
     return LCU_OK;
   }
   const int mats = GATED ? 2 : 1;
-  const stream_join_t shape = plan_stream_join(outs, mats, mats, splits, cus, stream_max_waves(false));
+  const stream_join_t shape = plan_stream_join(M, K, outs, mats, mats, splits, cus, false);
   if (shape.waves == 0) return LCU_OK;
   const int rc = launch_joined_shape<false, true>(linear_join<GATED>{ep, N}, single_matrix(nullptr, W, nullptr), (const half_t*)A, M, K, N, 0, st, splits, shape);
   *done = rc == LCU_OK;

@@ -24,6 +24,11 @@ constexpr int STREAM_LHS = 64 * 1024;  // bytes of lhs in LDS: one chunk, or two
 constexpr int stream_unit(bool u8) { return 2048 + (u8 ? 256 : 0); }
 constexpr int stream_max_waves(bool u8) { return u8 ? 10 : 12; }  // LDS: 160 KB
 constexpr int stream_lds(bool u8, int waves) { return STREAM_LHS + waves * STREAM_RING * stream_unit(u8); }
+// JOINED: lhs whole, and behind the product the sums of every wavefront in its place, [wavefront][row][16]; the rest for the rings
+constexpr int stream_joined_lhs(int waves, int row_tiles, int M, int K) {
+  return std::max((M * K * 2 + 1023) / 1024 * 1024, waves * row_tiles * 1024);
+}
+constexpr int STREAM_LDS = 160 * 1024;
 // K extent of a chunk of lhs: the longest run, counted from the 128 of K that it begins in, or what two chunks leave
 inline int stream_chunk(int rows, int stages_in_all, int splits) {
   long longest = 0;
@@ -50,6 +55,8 @@ __device__ __forceinline__ void wait_requests(int more) {
 // start and its first loads, 2 to 4 us for a few hundred KB.  us, two launches / one, 8 rows: fp16 (K, N) = (4096, 4096) three times and the rotary
 // 24.4 / 21.0, (4096, 11008) twice and the SiLU 44.2 / 41.2, (2048, 2048) three times 12.3 / 8.2, uint8 (4096, 4096) three times 19.8 / 15.7; alone, fp16
 // 13x2048x6656 12.0 / 9.1, 40x256x16384 9.5 / 6.4, uint8 20x1408x6656 11.5 / 7.3; over 80 drawn shapes of 2 to 62 rows 12 to 58 % sooner where one launch does it.
+// The rings take only what their wavefronts need, so that lhs may have more than STREAM_LHS: 34x1408x4096 10.3 -> 7.8, 10 rows of 4096 three times and the
+// rotary 24.2 -> 21.3.
 // GATED: the two are blocks of 32 columns of one matrix, a gate's and behind it an up block; the columns are those of the outputs.
 struct separate_sums {
   static constexpr bool JOINED = false, GATED = false;
@@ -105,7 +112,8 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
   };
 
   // this wavefront's columns: rows of 128 bytes, 16-byte piece p of row r at p ^ (r / 2) % 8
-  const uint32_t ring0 = lds0 + STREAM_LHS + wave * RING * UNIT;
+  const uint32_t lhs_room = JOINED ? (uint32_t)stream_joined_lhs(waves, TM, M, K) : STREAM_LHS;
+  const uint32_t ring0 = lds0 + lhs_room + wave * RING * UNIT;
   uint4_t rw = operand_resource(W, (uint32_t)N * (uint32_t)K * (U8 ? 1u : 2u)), rs = rw;
   if constexpr (U8) rs = operand_resource(S, (uint32_t)N * ((uint32_t)K >> (6 + block_shift)) * 2u);
   uint32_t w_off[2], s_first = 0;
@@ -213,7 +221,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
       // unit u has landed, and the unit before it has been read: the ring may take another in its place
       wait_requests<P*(RING - 2)>(u - from < RING - 1 ? lhs_out : 0);
       request(u + RING - 1);
-      const unsigned char* slot = stream_mem + STREAM_LHS + (wave * RING + u % RING) * UNIT;
+      const unsigned char* slot = stream_mem + lhs_room + (wave * RING + u % RING) * UNIT;
 #pragma unroll
       for (int e = 0; e < PER; ++e) {
         const int s = u * PER + e;
@@ -223,7 +231,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
   }
   if constexpr (JOINED) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");  // everybody has read lhs, whose place the sums take: [wavefront][row][16]
+    asm volatile("s_barrier" ::: "memory");  // everybody has read lhs, whose place the sums take
     float* sums = reinterpret_cast<float*>(stream_mem);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {

@@ -121,9 +121,9 @@ def test_gated_linear_split(gpu, M, K, ff, plan):
     test_gated_linear_large_tiles(gpu, M, K, ff)
 
 
-# few rows whose splits are added up where they end: one to four row tiles, odd and ragged columns, lhs that just fits its place (16x2048, 64x512) and
-# that does not (17x2048), outputs over lhs, which may only be written when all of lhs has been read
-@pytest.mark.parametrize("M,K,N", [(1, 2048, 1531), (2, 512, 515), (16, 2048, 3071), (17, 2048, 1030), (31, 1024, 2047), (64, 512, 4100)])
+# few rows whose splits are added up where they end: one to four row tiles, odd and ragged columns, lhs that just fits beside the rings (24x2048) and
+# that does not (25x2048), outputs over lhs, which may only be written when all of lhs has been read
+@pytest.mark.parametrize("M,K,N", [(1, 2048, 1531), (2, 512, 515), (16, 2048, 3071), (24, 2048, 1000), (25, 2048, 1000), (31, 1024, 2047), (64, 512, 4100)])
 def test_linear_few_rows_in_one_launch(gpu, M, K, N):
     test_linear_large_tiles(gpu, M, K, N)
     rng = np.random.default_rng(N)

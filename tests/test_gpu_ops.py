@@ -401,9 +401,9 @@ def test_gemm_f16_few_rows(gpu, M, K, N):
 
 
 # few rows whose splits are added up where they end: one to four row tiles, workgroups that hold the last columns of one matrix and the first of
-# the next, columns past the last whole sixteen, lhs that fills its place (64x512, 8x4096) and lhs that does not fit (9x4096)
+# the next, columns past the last whole sixteen, lhs that fills what the rings leave (12x4096, codes 11x4096) and lhs that does not fit (13x4096, codes 12x4096)
 @pytest.mark.parametrize("M,K,N,mats,block", [(2, 512, 3000, 3, 0), (16, 2048, 1002, 3, 0), (17, 1920, 2034, 2, 0), (32, 1024, 1300, 3, 128), (33, 896, 3010, 3, 64),
-                                              (64, 512, 4098, 3, 0), (64, 512, 4098, 2, 256), (8, 4096, 1346, 3, 128), (9, 4096, 2050, 3, 0), (3, 8192, 1026, 1, 0)])
+                                              (64, 512, 4098, 3, 0), (64, 512, 4098, 2, 256), (11, 4096, 1346, 3, 128), (12, 4096, 1346, 3, 128), (12, 4096, 1346, 3, 0), (13, 4096, 1346, 3, 0), (3, 8192, 1026, 1, 0)])
 def test_few_rows_added_up_where_they_end(gpu, M, K, N, mats, block):
     G = gpu
     check, L, VP = G.B.check, G.L(), G.B.vp
