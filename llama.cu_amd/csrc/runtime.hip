@@ -149,17 +149,58 @@ int lcu_free(void* dev) {
   return LCU_OK;
 }
 
+// Page-locked memory comes in pages, some 50 us each to lock, and a context wants two pieces of a few bytes: pieces of up to 64 bytes share a page of their
+// device, whose first 64 bytes say which of it are taken.  A page goes back with its last piece.
+namespace {
+constexpr size_t HOST_PAGE = 4096, HOST_PIECE = 64;
+struct host_page {
+  host_page* next;
+  uint64_t taken;  // bit i: piece i; bit 0: this header
+  int device;
+};
+static_assert(sizeof(host_page) <= HOST_PIECE && HOST_PAGE / HOST_PIECE == 64, "a bit to a piece");
+std::mutex g_host_mutex;
+host_page* g_host_pages = nullptr;
+}  // namespace
+
 int lcu_host_alloc(void** out_host, size_t bytes) {
   LCU_REQUIRE(out_host != nullptr && bytes > 0, "lcu_host_alloc: bad arguments");
   *out_host = nullptr;
-  LCU_HIP(hipHostMalloc(out_host, bytes, hipHostMallocCoherent | hipHostMallocMapped));
+  if (bytes > HOST_PIECE) {
+    LCU_HIP(hipHostMalloc(out_host, bytes, hipHostMallocCoherent | hipHostMallocMapped));
+    return LCU_OK;
+  }
+  int device = 0;
+  LCU_HIP(hipGetDevice(&device));
+  std::lock_guard<std::mutex> lock(g_host_mutex);
+  host_page* page = g_host_pages;
+  while (page && (page->device != device || page->taken == ~(uint64_t)0)) page = page->next;
+  if (!page) {
+    LCU_HIP(hipHostMalloc((void**)&page, HOST_PAGE, hipHostMallocCoherent | hipHostMallocMapped));
+    *page = host_page{g_host_pages, 1, device};
+    g_host_pages = page;
+  }
+  const int piece = __builtin_ctzll(~page->taken);
+  page->taken |= (uint64_t)1 << piece;
+  *out_host = memset((char*)page + piece * HOST_PIECE, 0, HOST_PIECE);
   return LCU_OK;
 }
 
 int lcu_host_free(void* host) {
-  if (host) {
-    LCU_HIP(hipHostFree(host));
+  if (!host) return LCU_OK;
+  {
+    std::lock_guard<std::mutex> lock(g_host_mutex);
+    host_page** link = &g_host_pages;
+    const uintptr_t at = reinterpret_cast<uintptr_t>(host);
+    while (*link && at - reinterpret_cast<uintptr_t>(*link) >= HOST_PAGE) link = &(*link)->next;
+    if (host_page* page = *link) {
+      page->taken &= ~((uint64_t)1 << (at - reinterpret_cast<uintptr_t>(page)) / HOST_PIECE);
+      if (page->taken != 1) return LCU_OK;
+      *link = page->next;
+      host = page;
+    }
   }
+  LCU_HIP(hipHostFree(host));
   return LCU_OK;
 }
 

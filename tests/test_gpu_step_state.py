@@ -19,6 +19,39 @@ def words(gpu):
     gpu.B.check(gpu.L().lcu_host_free(p))
 
 
+def test_small_pieces_of_page_locked_memory(gpu):
+    """More than a page of them: apart, zero, written by the device one by one, and taken anew after some have gone back."""
+    L, check = gpu.L(), gpu.B.check
+
+    def take(n):
+        out = [C.c_void_p() for _ in range(n)]
+        for p in out:
+            check(L.lcu_host_alloc(C.byref(p), 64))
+        return out
+
+    def view(p):
+        return np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_int32)), (16,))
+
+    pieces, source = take(150), gpu.dev_keep(np.arange(150, dtype=np.float32))
+    for _ in range(2):
+        at = sorted(p.value for p in pieces)
+        assert all(b - a >= 64 for a, b in zip(at, at[1:])) and all(a % 64 == 0 for a in at)
+        assert all((view(p) == 0).all() for p in pieces)
+        for i, p in enumerate(pieces):
+            check(L.lcu_argmax_f32(p, source.ptr, i + 1, gpu.stream))
+        check(L.lcu_sync(gpu.stream))
+        assert all(view(p)[0] == i and (view(p)[1:] == 0).all() for i, p in enumerate(pieces))
+        for p in pieces[::2] + pieces[1:100:2]:
+            check(L.lcu_host_free(p))
+        kept = pieces[101::2]
+        for p in kept:
+            view(p)[:] = 0
+        pieces = take(150 - len(kept)) + kept
+    for p in pieces:
+        check(L.lcu_host_free(p))
+    gpu.release()
+
+
 @pytest.mark.parametrize("n", [1, 6, 255, 256])
 def test_fetched_words(gpu, words, n):
     words[:] = np.random.default_rng(n).integers(-2**31, 2**31, 256)
