@@ -9,7 +9,8 @@
 //   gemm_tile_kernel (gemm_tile.hpp): 256-row tiles of 128, 192 or 256 columns where these fill most of the
 //     chip, 256x128 with the K range split over workgroups, 128-row tiles of up to 128 rows and where only
 //     those of 128x128 fill most of the chip, else 128x64; fp16, uint8 (codes in blocks of 64 << n) and bfloat16 weights
-//   gemm_stream_kernel (gemm_stream.hpp): 2..64 rows, the K range split over workgroups
+//   gemm_stream_kernel (gemm_stream.hpp): 2..64 rows, the K range split over wavefronts that add up their sums and finish
+//     the outputs, or over workgroups
 //   gemm_dl_kernel (K a multiple of 128; a short K where 128x128 tiles fill the chip, other blocks of codes, splits of few rows,
 //     bfloat16 experts and small tiles): both operands travel from global memory straight into a ring of 2-3 LDS
 //     stages with global_load_lds_dwordx4 (no staging registers, no LDS store instructions); rows are
@@ -17,7 +18,7 @@
 //     reads meet in a bank; 4 or 8 wavefronts (a second group of four may take the other half of a 128-wide K
 //     stage), chosen by how many tiles the product has; uint8 weights add a ring of codes and of scales and are
 //     turned into fp16 -- exactly fp16((q - 127.5) * scale), llama_cu.cu:287-289 -- once per block tile
-//   Where the K range is split -- 2..64 rows, few large tiles and a long K -- a second launch adds the
+//   Where the K range is split over workgroups -- 2..64 rows, few large tiles and a long K -- a second launch adds the
 //     fp32 partial sums in split order (launch_skinny; large_tile_splits in gemm_plan.hpp)
 //   gemm_kernel (ragged K): global -> registers -> padded LDS with two LDS buffers and two
 //     register stages, uint8 weights dequantised between the load and the LDS store
@@ -1220,7 +1221,8 @@ struct f16_join {
 
 // Few rows (2 .. 64: short prompts, where the reference takes its 16-row tile, llama_cu.cu:1481-1484):
 // the K stages split as BM x 128 tiles would need to give every compute unit one workgroup; gemm_stream_kernel
-// walks the splits, in one launch with what follows (launch_joined) or for another to add up, or such tiles with four wavefronts do (`streams`; blocks of codes other than 64 << n).
+// walks the splits, in one launch with what follows (launch_joined) or for another to add up, or such tiles with four
+// wavefronts do (`streams`; blocks of codes other than 64 << n).
 // Returns LCU_OK with *done = false when the shape does not suit it.
 template <int BM, bool U8>
 int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st,
