@@ -1750,7 +1750,7 @@ int launch_bf16(EP const& ep, const void* A, const void* W, int tiles_m, int M, 
   return LCU_OK;
 }
 
-// The splits' sums in split order, then the epilogue; a thread per output.
+// the splits' sums in split order, then the epilogue; a thread per output
 template <bool GATED>
 __global__ __launch_bounds__(256) void splitk_epilogue_kernel(linear_epilogue<false, GATED> ep, const float* __restrict__ part, int M,
                                                               int N, int splits) {
@@ -1768,63 +1768,6 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(linear_epilogue<fa
   } else {
     ep.store(m, n, sum(n));
   }
-}
-// The same for a million outputs and more, eight neighbouring ones to a thread, two splits asked for at a time (512x4096x4096 in two splits, both
-// launches 34.3 -> 32.8 us; for fewer the threads become too few, 100x2048x2048 in eight 10.3 -> 13.0).
-template <bool GATED>
-__global__ __launch_bounds__(256) void splitk_epilogue8_kernel(linear_epilogue<false, GATED> ep, const float* __restrict__ part, int M,
-                                                               int N, int splits) {
-  typedef float4_t any_float4_t __attribute__((aligned(4)));
-  constexpr int RUNS = GATED ? 2 : 1;  // of eight columns of the product: gate and up rows
-  const int outs = GATED ? N / 2 : N, pieces = (outs + 7) / 8, i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= M * pieces) return;
-  const int m = i / pieces, n = (i - m * pieces) * 8, c = GATED ? n / 32 * 64 + n % 32 : n;
-  const bool whole = GATED || n + 8 <= N;
-  float4_t sum[RUNS][2] = {};
-  const size_t mn = (size_t)M * N, at = (size_t)m * N + c;
-  for (int k = 0; k < splits; k += 2) {
-    float4_t v[2][RUNS][2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const float* from = part + (size_t)min(k + u, splits - 1) * mn + at;
-#pragma unroll
-      for (int r = 0; r < RUNS; ++r) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (whole) {
-            v[u][r][h] = *reinterpret_cast<const any_float4_t*>(from + r * 32 + h * 4);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[u][r][h][e] = from[min(h * 4 + e, N - 1 - n)];
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (k + u >= splits) break;
-#pragma unroll
-      for (int r = 0; r < RUNS; ++r) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) sum[r][h] += v[u][r][h];
-      }
-    }
-  }
-  float x[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = GATED ? ep.gate(sum[0][e / 4][e % 4], sum[RUNS - 1][e / 4][e % 4]) : sum[0][e / 4][e % 4];
-  ep.store8(m, n, x, outs);
-}
-template <bool GATED>
-int add_splits(linear_epilogue<false, GATED> const& ep, const float* part, int M, int N, int splits, hipStream_t st) {
-  const int outs = GATED ? N / 2 : N;
-  if ((long)M * outs < 1 << 20) {
-    splitk_epilogue_kernel<GATED><<<(M * outs + 255) / 256, 256, 0, st>>>(ep, part, M, N, splits);
-  } else {
-    splitk_epilogue8_kernel<GATED><<<(M * ((outs + 7) / 8) + 255) / 256, 256, 0, st>>>(ep, part, M, N, splits);
-  }
-  LCU_LAUNCH_CHECK();
-  return LCU_OK;
 }
 
 template <bool GATED_>
@@ -1887,9 +1830,11 @@ int bf16_skinny(linear_epilogue<false, GATED> const& ep, const void* A, const vo
                  : launch_bf16<64, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part);
   }
   if (rc != LCU_OK) return rc;
-  rc = add_splits(ep, part, M, N, splits, st);
-  *done = rc == LCU_OK;
-  return rc;
+  const int outs = M * (GATED ? N / 2 : N);
+  splitk_epilogue_kernel<GATED><<<(outs + 255) / 256, 256, 0, st>>>(ep, part, M, N, splits);
+  LCU_LAUNCH_CHECK();
+  *done = true;
+  return LCU_OK;
 }
 
 }  // namespace
@@ -1909,18 +1854,6 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     return launch_bf16<64, 64, 2, GATED ? 1 : 2, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   }
   if (tm(256) * tn(128) >= 160) return launch_large<false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
-  const device_state* ds = current_device_state();
-  const workspace_t ws = workspace_for(st);
-  // sums through the workspace only where nobody else's launches use it
-  const bf16_split_t split = plan_bf16_split(GATED, M, K, N, ds && ds->compute_units > 0 ? ds->compute_units : 256, ws.ptr && ws.owned ? ws.bytes : 0);
-  if (split.splits > 1) {
-    float* part = (float*)ws.ptr;
-    const linear_epilogue<false, false> none{};
-    const int rc = split.rows == 128 ? launch_tile<128, 128, 2, 2, 4, 4, false, true>(none, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st,
-                                                                                      split.splits, part)
-                                     : launch_bf16<64, 128, 2, 2, 1, 3, true>(none, A, W, tm(64), M, K, N, st, split.splits, part);
-    return rc != LCU_OK ? rc : add_splits(ep, part, M, N, split.splits, st);
-  }
   if constexpr (GATED) {  // 1000 rows of 4608 columns, K 512, 1024, 2048: 17.2 us, 24.5, 43.1 with two workgroups per compute unit, else 17.8, 24.8, 39.7
     if (K < 1280 && tm(128) * tn(128) > 256) return launch_bf16<128, 128, 2, 2, 1, 2>(ep, A, W, tm(128), M, K, N, st);
   }

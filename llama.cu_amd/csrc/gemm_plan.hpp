@@ -148,55 +148,6 @@ inline left_sums_t plan_left_sums(bool u8, int M, int K, int N, long cus, size_t
   return {2, 2};
 }
 
-// A bfloat16 product of more than 64 rows whose tiles leave compute units idle: the K stages of every tile of 128x128 (one to a compute unit)
-// or 64x128 (two) dealt to `splits` workgroups, the sums added by a second launch (splits 0: the tiles as they are).  In between lay the products
-// of prompts of 65 to some 500 tokens: 100x4096x4096 29.4 -> 17 us, 100x10752x4096 69 -> 27, 100x5632x2048 37 -> 15, 192x4096x1536 28 -> 15, 512x5632x2048
-// 38 -> 28.  Costs in us: a fixed part, rounds of workgroups by their stages and by themselves, the work in them, W, the sums (both ways) and
-// the outputs by their bytes; fitted to 6800 drawn products with weights from memory, each tile as it is and in two to twelve splits.  Over these
-// the choice takes 0.86 of the time before, the best one would take 0.85; 0.5 % of them take more than 3 % longer (up to 11).
-struct bf16_split_t {
-  int rows, splits;
-};
-inline bf16_split_t plan_bf16_split(bool gated, int M, int K, int N, long cus, size_t workspace_bytes) {
-  struct cost_t {
-    int rows, columns, per_cu;  // workgroups to a compute unit
-    double fixed, stages, round, work, weights, sums, outputs;
-    double operator()(int M, int K, int N, long cus, int splits) const {
-      const double full = (double)tiles_of(M, N, rows, columns) * splits / (double)(per_cu * cus), rounds = std::ceil(full);
-      const double run = (double)((K / PLAN_STAGE + splits - 1) / splits) / 64, mn = 4e-6 * M * N;
-      return fixed + rounds * (stages * run + round) + work * full * run + weights * 2e-6 * N * K + (splits > 1 ? sums * splits * mn : 0) + outputs * mn;
-    }
-  };
-  constexpr cost_t wide{128, 128, 1, 0.57, 24.77, 5.05, 8.07, 0.057, 0, 0.132}, gated_tall{128, 64, 2, 4.06, 16.89, 0, 24.45, 0.101, 0, 0.067},
-      gated_small{64, 64, 3, 0, 23.51, 3.79, 4.47, 0.117, 0, 0.075}, tall{128, 64, 2, 2.55, 0, 0, 58.06, 0.176, 0, 0.483},
-      tall_halves{128, 64, 1, 5.03, 16.93, 0, 1.99, 0.09, 0, 0.29}, small{64, 64, 3, 0, 19.65, 2.73, 8.1, 0.139, 0, 0.178};
-  constexpr cost_t split_wide{128, 128, 1, 6.75, 25.66, 0.47, 0, 0.076, 0.582, 0}, split_low{64, 128, 2, 6.61, 20.74, 0, 16.23, 0.092, 0.493, 0.011};
-  if (M <= 64 || K % PLAN_STAGE != 0 || tiles_of(M, N, 256, 128) >= 160) return {0, 0};
-  const cost_t* now;  // the tiles of gemm_bf16
-  if (gated && K < 1280 && tiles_of(M, N, 128, 128) > 256) return {0, 0};
-  if (tiles_of(M, N, 128, 128) >= 160) {
-    now = &wide;
-  } else if (gated) {
-    now = tiles_of(M, N, 128, 64) > 128 ? &gated_tall : &gated_small;
-  } else if (tiles_of(M, N, 128, 64) > 256) {
-    now = &tall;
-  } else {
-    now = K % 128 == 0 && tiles_of(M, N, 128, 64) > 128 ? &tall_halves : &small;
-  }
-  double least = 0.93 * (*now)(M, K, N, cus, 1);  // what the fit may be wrong by
-  bf16_split_t best{0, 0};
-  for (const cost_t* tile : {&split_wide, &split_low}) {
-    for (int splits = 2; splits <= 16 && K / PLAN_STAGE / splits >= 4 && (size_t)splits * M * N * sizeof(float) <= workspace_bytes; ++splits) {
-      const double cost = (*tile)(M, K, N, cus, splits);
-      if (cost < least) {
-        least = cost;
-        best = {tile->rows, splits};
-      }
-    }
-  }
-  return best;
-}
-
 // Rows of a tile for the products of `rows` rows sorted by expert with matrices [2 ff][K] (gated) and [K][ff]: those whose tiles cost least.  An expert
 // that a tile does not hold asks for its weights once more, but larger tiles are fewer, and where the product has few of them compute units idle
 // (4 experts of 256 hidden columns, 4096 wide, 260 rows: 64-row tiles 37 us, 128 46; top 2 of 16 of 2816, 512 tokens 284, 238, of 256 rows 272, 1000

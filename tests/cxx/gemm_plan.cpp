@@ -30,13 +30,6 @@ void left_sums(int u8, int M, int K, int N, long cus, long workspace, int owned,
   out[1] = p.step;
 }
 
-// rows of a tile, splits (0: none)
-void bf16_split(int gated, int M, int K, int N, long cus, long workspace, int* out) {
-  const bf16_split_t p = plan_bf16_split(gated != 0, M, K, N, cus, (size_t)workspace);
-  out[0] = p.rows;
-  out[1] = p.splits;
-}
-
 int expert_rows(long rows, int experts, int K, int ff, long cus) { return plan_expert_rows(rows, experts, K, ff, cus); }
 
 int attention_again(int n_heads, int n_new, int start_pos, long cus) { return scores_again(n_heads, n_new, start_pos, cus); }

@@ -24,8 +24,7 @@ def _lib():
     lib.large.argtypes = [i, i, i, i, i, w, i, C.POINTER(i)]
     lib.attention_again.argtypes = [i, i, i, w]
     lib.expert_rows.argtypes = [w, i, i, i, w]
-    lib.bf16_split.argtypes = [i, i, i, i, w, w, C.POINTER(i)]
-    lib.bf16_split.restype = lib.rows.restype = lib.left_sums.restype = lib.large.restype = None
+    lib.rows.restype = lib.left_sums.restype = lib.large.restype = None
     os.unlink(path)
     os.rmdir(folder)
     return lib
@@ -49,13 +48,6 @@ def left_sums(M, K, N, u8=False, owned=True, cus=CUS, workspace=WORKSPACE):
     """(splits, step)"""
     out = (C.c_int * 2)()
     _lib().left_sums(int(u8), M, K, N, cus, workspace, int(owned), out)
-    return out[0], out[1]
-
-
-def bf16_split(M, K, N, gated=False, cus=CUS, workspace=WORKSPACE):
-    """(rows of a tile, splits)"""
-    out = (C.c_int * 2)()
-    _lib().bf16_split(int(gated), M, K, N, cus, workspace, out)
     return out[0], out[1]
 
 
