@@ -262,9 +262,11 @@ int lcu_attention_decode_batch(void* out_dev, const void* q_dev, const void* k_c
  * lcu_batch_proj_norm for more rows where their product is split, or, on a stream that owns its
  * workspace, sums the even and the odd stages of K apart; any other shape runs the separate operators
  * above).  w_dev / scales_dev: host arrays of device pointers (scales NULL
- * and block 0 for fp16 weights); *_tmp_dev: [n_seq][dim] / [n_seq][ffn] fp16 scratch.
- *   lcu_batch_qkv: Wq, Wk, Wv products of lhs [n_seq][dim], then lcu_rope_store_batch (1144-1156)
- *   lcu_batch_ffn_up: W1, W3 products, then fp16(silu(w1) * w3) (1180-1183)
+ * and block 0 for fp16 weights); *_tmp_dev: [n_seq][dim] / [n_seq][ffn] fp16 scratch, written only where a
+ * launch of their own goes on with the products.
+ *   lcu_batch_qkv: Wq, Wk, Wv products of lhs [n_seq][dim], then lcu_rope_store_batch (1144-1156); the caches do not overlap lhs
+ *   lcu_batch_ffn_up: W1, W3 products, then fp16(silu(w1) * w3) (1180-1183); out may overlap lhs (the products then go to the
+ *     temporaries first)
  *   lcu_batch_proj_norm: x += lhs [n_seq][K] * W^T (1174 / 1185), then norm_out = rms_norm(x) with
  *     norm_w (1176, or 1129 of the next layer, or 1191) */
 int lcu_batch_qkv(void* q_out_dev, void* k_tmp_dev, void* v_tmp_dev, const void* lhs_dev, const void* const* w_dev,

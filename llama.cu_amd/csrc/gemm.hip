@@ -2118,7 +2118,8 @@ int lcu_batch_ffn_up(void* out_dev, void* w1_tmp_dev, void* w3_tmp_dev, const vo
     return LCU_OK;
   }
   if (block == 0 && n_seq > 64 && dim % 128 == 0 && ffn % 16 == 0 && (size_t)n_seq * dim * 2 < ((size_t)1 << 32) &&
-      (size_t)ffn * dim * 2 < ((size_t)1 << 32) && ffn < 1 << 30 && tiles_of(n_seq, ffn, 256, 128) * 2 >= 160) {  // those of plan_rows' large tiles
+      (size_t)ffn * dim * 2 < ((size_t)1 << 32) && ffn < 1 << 30 && tiles_of(n_seq, ffn, 256, 128) * 2 >= 160 &&  // those of plan_rows' large tiles
+      !overlap(out_dev, (size_t)n_seq * ffn * 2, lhs_dev, (size_t)n_seq * dim * 2)) {  // other workgroups, or the launch for the rest, still read lhs
     operands_t op = single_matrix((half_t*)out_dev, w_dev[0], nullptr);
     op.more.W[0] = w_dev[1];
     return launch_large<false>(silu_epilogue{}, op, lhs_dev, n_seq, dim, 2 * ffn, 0, 0.0f, st);

@@ -697,6 +697,27 @@ def test_up_products_with_their_silu(gpu, n, dim, ffn):
     G.release()
 
 
+@pytest.mark.parametrize("n,dim,ffn,at", [(100, 128, 16400, 0), (512, 1024, 11008, 0), (512, 1024, 11008, 4000000), (1033, 2048, 6704, 0), (773, 2048, 6160, 773 * 6160 - 8)])
+def test_up_products_over_their_lhs(gpu, n, dim, ffn, at):
+    """Outputs in the buffer of lhs, from its first element on or with lhs at their element `at`: the products go to the temporaries first, as
+    the workgroups of one launch would still be reading lhs."""
+    G, L = gpu, gpu.L()
+    rng = np.random.default_rng(n + ffn + at)
+    x = rng.standard_normal((n, dim)).astype(np.float16)
+    w = [G.dev_keep((rng.standard_normal((ffn, dim)) * 3 / dim ** 0.5).astype(np.float16)) for _ in range(2)]
+    ptrs = lambda bufs: (C.c_void_p * len(bufs))(*[b.ptr for b in bufs])
+    t1, t3, want, u1, u3 = (G.dev_keep(np.full((n, ffn), -7, np.float16)) for _ in range(5))
+    G.B.check(L.lcu_gemm_f16_nt_multi(ptrs([t1, t3]), G.dev_keep(x).ptr, ptrs(w), 2, n, dim, ffn, 0.0, None))
+    G.B.check(L.lcu_silu_mul(want.ptr, t1.ptr, t3.ptr, n * ffn, None))
+    both = np.zeros(max(n * ffn, at + n * dim), np.float16)
+    both[at:at + n * dim] = x.reshape(-1)
+    both = G.dev_keep(both)
+    G.B.check(L.lcu_batch_ffn_up(both.ptr, u1.ptr, u3.ptr, both.ptr + 2 * at, ptrs(w), None, 0, n, dim, ffn, None))
+    for got, ref in ((both, want), (u1, t1), (u3, t3)):
+        assert (G.host(got, (n, ffn), np.uint16) == G.host(ref, (n, ffn), np.uint16)).all()
+    G.release()
+
+
 def test_exp_bit_exact(gpu):
     """the exponential of every softmax and SiLU: host restatement and kernel agree on every bit"""
     G = gpu
