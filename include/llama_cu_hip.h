@@ -567,8 +567,9 @@ int lcu_decode_residual_router(void* x_dev, void* h_dev, const void* out_f32_dev
 
 /* The same products of a row that is not there yet: the launch itself adds what the sublayer before it left and takes both
  * norms (lcu_decode_residual_router without a router), each workgroup for itself, while its weights are on their way.  The sum
- * goes to x_out, which must not overlap x; the normed row goes to h only where the shape takes a launch of its own for it
- * (rows of more than 2048 elements, matrices of more than 64 MB).  K is the row's ld.  Same bits as the two calls. */
+ * goes to x_out, which must not overlap x; the normed row goes to h only where it takes a launch of its own
+ * (rows of more than 2048 elements, matrices of more than 64 MB, outputs or x_out over what the row is worked out of, x_out
+ * over another operand).  Outputs must not overlap h.  K is the row's ld.  Same bits as the two calls. */
 typedef struct lcu_step_row {
   const void* x_dev; /* fp32 residual row */
   void* x_out_dev;

@@ -92,6 +92,11 @@ struct step_fetch {
 };
 constexpr size_t STEP_FETCH_MAX = 256 * 4;  // bytes
 
+inline bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + b_bytes && y < x + a_bytes;
+}
+
 // fp32 -> fp16, round to nearest even, as a separate step.  Written through an opaque register so
 // the compiler cannot merge the conversion into the preceding multiply or fused multiply-add
 // (v_fma_mixlo_f16 rounds the exact result once to fp16; the reference rounds to fp32 first, and a

@@ -1176,11 +1176,6 @@ int launch_joined_shape(JOIN const& join, operands_t op, const half_t* A, int M,
   return launch_joined_rows<4, U8, BF16>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
 }
 
-inline bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
-  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-  return x < y + b_bytes && y < x + a_bytes;
-}
-
 // A product of few rows and what follows it in one launch, with the splits of plan_skinny.  *done = false, with nothing launched, where lhs does not fit
 // LDS whole, the workgroups would take a second round, or an output (an operand's, or `out`) lies over lhs, which other workgroups still read.
 template <bool U8, class JOIN>

@@ -24,6 +24,7 @@
 // kernel-order flavour restates from measured samples): the dequantisation arithmetic, not HBM,
 // is what bounds this kernel on large matrices.
 #include <algorithm>
+#include <initializer_list>
 #include <type_traits>
 
 #include "common.hpp"
@@ -1038,13 +1039,49 @@ constexpr int NORMED_ROW_MAX = 2048;               // elements of a row
 constexpr size_t NORMED_BYTES_MAX = 64u << 20;     // of the matrix
 constexpr int NORMED_SUMS_MAX = 512;               // results a workgroup keeps in LDS
 
-// tasks of R rows through normed_rows_kernel; false: the shape is not for it
+// what a product writes, and what it reads besides the row
+struct operand_t {
+  const void* at;
+  size_t bytes;
+  bool written;
+};
+using operand_list = std::initializer_list<operand_t>;
+
+// Whether one launch may work the row out: every workgroup reads its sources at a time of its own, so that nothing which the launch writes may
+// lie over them, nor x_out over an operand.
+inline bool row_apart(const step_row& s, operand_list operands) {
+  const size_t bytes = (size_t)s.rs.ld * 4;
+  const operand_t sources[] = {{s.x, bytes, false},
+                               {s.src.out, s.src.top * bytes, false},
+                               {s.src.shared, bytes, false},
+                               {s.src.shared ? s.src.shared_gate : nullptr, 4, false},
+                               {s.w_after, bytes, false},
+                               {s.w_next, bytes, false}};
+  const auto apart = [](operand_t const& a, operand_t const& b) {
+    return !a.at || !b.at || a.bytes == 0 || b.bytes == 0 || !overlap(a.at, a.bytes, b.at, b.bytes);
+  };
+  const operand_t x_out{s.x_out, bytes, true};
+  for (operand_t const& from : sources) {
+    if (!apart(x_out, from)) return false;
+    for (operand_t const& o : operands) {
+      if (o.written && !apart(o, from)) return false;
+    }
+  }
+  for (operand_t const& o : operands) {
+    if (!apart(x_out, o)) return false;
+  }
+  return true;
+}
+
+// tasks of R rows through normed_rows_kernel; false: the shape is not for it, or the operands lie over the row
 template <int R, class Tasks>
-bool launch_normed_rows(const step_row& s, const Tasks& tk, int tasks, hipStream_t st) {
+bool launch_normed_rows(const step_row& s, const Tasks& tk, int tasks, operand_list operands, hipStream_t st) {
   const device_state* ds = current_device_state();
   const int groups = std::min(ds && ds->compute_units > 0 ? ds->compute_units : 256, tasks);
   const int per = tasks / groups, more = tasks % groups, kept = (per + (more > 0 ? 1 : 0)) * R;
-  if (s.rs.ld > NORMED_ROW_MAX || (size_t)tasks * R * s.rs.ld * 2 > NORMED_BYTES_MAX || kept > NORMED_SUMS_MAX) return false;
+  if (s.rs.ld > NORMED_ROW_MAX || (size_t)tasks * R * s.rs.ld * 2 > NORMED_BYTES_MAX || kept > NORMED_SUMS_MAX || !row_apart(s, operands)) {
+    return false;
+  }
   const int sums = (int)((row_lds_bytes(s.rs) + 15) / 16 * 16);
   const auto go = [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
@@ -1059,9 +1096,9 @@ bool launch_normed_rows(const step_row& s, const Tasks& tk, int tasks, hipStream
 }
 
 template <class Epilogue>
-int launch_decode_rows(const lcu_step_row* row, const void* W, int K, int N, Epilogue ep, hipStream_t st) {
+int launch_decode_rows(const lcu_step_row* row, const void* W, int K, int N, Epilogue ep, operand_list operands, hipStream_t st) {
   const step_row s = as_step_row(row);
-  if (launch_normed_rows<2>(s, bf16_tasks<2, Epilogue>{(const bf16_t*)W, K, N, ep}, (N + 1) / 2, st)) {
+  if (launch_normed_rows<2>(s, bf16_tasks<2, Epilogue>{(const bf16_t*)W, K, N, ep}, (N + 1) / 2, operands, st)) {
     LCU_LAUNCH_CHECK();
     return LCU_OK;
   }
@@ -1448,14 +1485,17 @@ int lcu_step_linear(void* out_f32_dev, const lcu_step_row* row, const void* w_de
   const int rc = check_step_row("lcu_step_linear", row);
   if (rc) return rc;
   LCU_REQUIRE(out_f32_dev && w_dev && N > 0, "lcu_step_linear: bad arguments");
-  return launch_decode_rows(row, w_dev, row->ld, N, store_f32_row{(float*)out_f32_dev, (const float*)bias_dev}, as_stream(stream));
+  return launch_decode_rows(row, w_dev, row->ld, N, store_f32_row{(float*)out_f32_dev, (const float*)bias_dev},
+                            {{out_f32_dev, (size_t)N * 4, true}, {w_dev, (size_t)N * row->ld * 2, false}, {bias_dev, (size_t)N * 4, false}},
+                            as_stream(stream));
 }
 
 int lcu_step_linear_bf16(void* out_dev, const lcu_step_row* row, const void* w_dev, int N, void* stream) {
   const int rc = check_step_row("lcu_step_linear_bf16", row);
   if (rc) return rc;
   LCU_REQUIRE(out_dev && w_dev && N > 0, "lcu_step_linear_bf16: bad arguments");
-  return launch_decode_rows(row, w_dev, row->ld, N, store_bf16_row{(bf16_t*)out_dev}, as_stream(stream));
+  return launch_decode_rows(row, w_dev, row->ld, N, store_bf16_row{(bf16_t*)out_dev},
+                            {{out_dev, (size_t)N * 2, true}, {w_dev, (size_t)N * row->ld * 2, false}}, as_stream(stream));
 }
 
 int lcu_step_delta_in(void* u_dev, void* plain_dev, void* tail_f32_dev, void* conv_state_dev, const lcu_step_row* row, const void* w_dev,
@@ -1468,6 +1508,12 @@ int lcu_step_delta_in(void* u_dev, void* plain_dev, void* tail_f32_dev, void* co
   return launch_decode_rows(row, w_dev, row->ld, N,
                             delta_in_row{(bf16_t*)u_dev, (bf16_t*)plain_dev, (float*)tail_f32_dev, (bf16_t*)conv_state_dev,
                                          (const float*)conv_dev, taps, channels, plain},
+                            {{u_dev, (size_t)channels * 2, true},
+                             {plain_dev, (size_t)plain * 2, true},
+                             {tail_f32_dev, (size_t)(N - channels - plain) * 4, true},
+                             {conv_state_dev, (size_t)(taps - 1) * channels * 2, true},
+                             {w_dev, (size_t)N * row->ld * 2, false},
+                             {conv_dev, (size_t)taps * channels * 4, false}},
                             as_stream(stream));
 }
 
@@ -1477,7 +1523,7 @@ int lcu_step_gated(void* hidden_dev, const lcu_step_row* row, const void* w_dev,
   LCU_REQUIRE(hidden_dev && w_dev && gate && ld > 0 && ld % 32 == 0, "lcu_step_gated: bad arguments");
   const step_row s = as_step_row(row);
   const expert_up_tasks<1> tk{(const bf16_t*)w_dev, (bf16_t*)hidden_dev, {gate->limit, gate->alpha, gate->up_shift}, 1.0f, row->ld};
-  if (launch_normed_rows<2>(s, tk, ld, as_stream(stream))) {
+  if (launch_normed_rows<2>(s, tk, ld, {{hidden_dev, (size_t)ld * 2, true}, {w_dev, (size_t)ld * row->ld * 4, false}}, as_stream(stream))) {
     LCU_LAUNCH_CHECK();
     return LCU_OK;
   }
@@ -1494,6 +1540,13 @@ int lcu_step_recurrent_in(void* y_dev, void* u_dev, void* conv_state_dev, const 
   return launch_decode_rows(row, w_dev, row->ld, 2 * ld,
                             conv_step_row{(bf16_t*)y_dev, (bf16_t*)u_dev, (bf16_t*)conv_state_dev, (const float*)bias_dev,
                                           (const float*)conv_dev, (const float*)conv_bias_dev, taps, ld},
+                            {{y_dev, (size_t)ld * 2, true},
+                             {u_dev, (size_t)ld * 2, true},
+                             {conv_state_dev, (size_t)(taps - 1) * ld * 2, true},
+                             {w_dev, (size_t)ld * row->ld * 4, false},
+                             {bias_dev, (size_t)ld * 8, false},
+                             {conv_dev, (size_t)taps * ld * 4, false},
+                             {conv_bias_dev, (size_t)ld * 4, false}},
                             as_stream(stream));
 }
 
@@ -1509,6 +1562,14 @@ int lcu_step_kv(void* q_out_dev, void* k_cache_dev, void* v_cache_dev, const lcu
                             qkv_row{(bf16_t*)q_out_dev, (bf16_t*)k_cache_dev, (bf16_t*)v_cache_dev, (bf16_t*)v_first_dev,
                                     (const float*)bias_dev, (const float*)lambda_dev, (const int*)pos_dev, q_cols, k_cols, v_cols,
                                     v_mode, max_positions},
+                            {{q_out_dev, (size_t)q_cols * 2, true},
+                             {k_cache_dev, (size_t)max_positions * k_cols * 2, true},
+                             {v_cache_dev, (size_t)max_positions * v_cols * 2, true},
+                             {v_mode ? v_first_dev : nullptr, (size_t)v_cols * 2, v_mode == 1},
+                             {w_dev, (size_t)(q_cols + k_cols + v_cols) * row->ld * 2, false},
+                             {bias_dev, (size_t)(q_cols + k_cols + v_cols) * 4, false},
+                             {v_mode == 2 ? lambda_dev : nullptr, 4, false},
+                             {pos_dev, 4, false}},
                             as_stream(stream));
 }
 

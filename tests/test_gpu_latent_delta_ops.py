@@ -2,6 +2,7 @@
 (plain_latent_delta.py), in both element types; the sizes are ragged.  Keys that matter are made to stand out: one
 score decides the output where the key is seen, and must leave no trace one token further."""
 import ctypes as C
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -520,4 +521,76 @@ def test_products_of_a_row_worked_out_on_the_way(gpu, width, groups, N, top):
             assert np.array_equal(got, want), name
     row.x_out = x.ptr + 4 * (ld - 1)  # a workgroup would read what another has written
     assert gpu.L().lcu_step_linear_bf16(h.ptr, C.byref(row), w.ptr, N, gpu.stream) == -2
+    gpu.release()
+
+
+@pytest.mark.parametrize("width,N", [(192, 70), (1000, 300), (2048, 1281), (2112, 90)])
+@pytest.mark.parametrize("over", ["nothing", "x_out out", "x_out out end", "x_out shared", "x_out bias", "product x", "product x end", "product out",
+                                  "product shared", "product w_after", "product x_out"])
+def test_products_over_the_row_they_are_worked_out_of(gpu, width, N, over):
+    """Where one launch would write what its other workgroups read, the row takes a launch of its own, which leaves the normed row in h:
+    the bits of the two calls on buffers apart, the product written last."""
+    if over == "x_out bias" and N < width:
+        N = up64(width)  # the bias is the row itself
+    rng = np.random.default_rng(width + N)
+    ld, top, eps = up64(width), 2, 1e-6
+    host = {"x": pad(rng.standard_normal(width), ld), "out": pad(rng.standard_normal((top, width)), ld), "shared": pad(rng.standard_normal(width), ld),
+            "w_after": pad(1 + 0.1 * rng.standard_normal(width), ld), "w_next": pad(1 + 0.1 * rng.standard_normal(width), ld)}
+    w, gate = put(gpu, pad(rng.standard_normal((N, width)) / width ** 0.5, ld), BF16), put(gpu, np.array([0.7]))
+    results = []
+    for step in (False, True):
+        b = {k: put(gpu, np.pad(v.ravel(), (0, N + ld))) for k, v in host.items()}  # room for the product, or the sum
+        at = {"x_out": zeros(gpu, ld + N).ptr, "product": zeros(gpu, N).ptr}
+        bias, h = put(gpu, np.pad(host["x"], (0, N))), zeros(gpu, ld, BF16)
+        bias_at = bias.ptr
+        if step and over != "nothing":
+            what, onto, *end = over.split()
+            if onto == "bias":
+                bias_at = at["x_out"]
+            else:
+                base, size = (at["x_out"], ld) if onto == "x_out" else (b[onto].ptr, top * ld if onto == "out" else ld)
+                at[what] = base + (4 * (size - 16) if end else 0)
+        if step:
+            row = gpu.B.StepRow(b["x"].ptr, at["x_out"], h.ptr, b["out"].ptr, b["shared"].ptr, gate.ptr, b["w_after"].ptr, b["w_next"].ptr, top, width, ld, 1, eps)
+            call(gpu, "lcu_step_linear", at["product"], C.byref(row), w, bias_at, N)
+        else:
+            if over == "x_out bias":
+                bias_at = b["x"].ptr
+            call(gpu, "lcu_decode_residual_router", b["x"], h, b["out"], top, b["shared"], gate, b["w_after"], b["w_next"], width, ld, 1, eps, None, 0, 0, None, None, None)
+            call(gpu, "lcu_decode_linear", at["product"], h, w, bias_at, ld, N)
+            at["x_out"] = b["x"].ptr
+        gpu.B.check(gpu.L().lcu_sync(gpu.stream))
+        take = lambda p, n: gpu.host(SimpleNamespace(ptr=p), (n,), np.uint32)
+        results.append((take(at["product"], N), None if over == "product x_out" else take(at["x_out"], ld), get(gpu, h, (ld,), BF16)))
+    (want, sum_want, h_want), (got, sum_got, h_got) = results
+    assert np.array_equal(got, want) and (sum_got is None or np.array_equal(sum_got, sum_want))
+    assert np.array_equal(h_got, h_want if over != "nothing" or width > 2048 else np.zeros(ld))
+    gpu.release()
+
+
+@pytest.mark.parametrize("product,written", [("linear_bf16", (0,)), ("gated", (0,)), ("delta_in", (0, 1, 2, 3)), ("recurrent_in", (0, 1, 3)), ("kv", (0, 1, 2, 3))])
+def test_whatever_a_product_writes_over_its_row(gpu, product, written):
+    """Each array that a product writes, on the last words of the residual row and of the second result: the row takes its own launch, whose normed row is in h."""
+    width, N, taps, top, eps = 192, 96, 3, 2, 1e-6
+    rng = np.random.default_rng(len(product))
+    x0, out0 = rng.standard_normal(width), rng.standard_normal((top, width))
+    w, ones, wide = put(gpu, rng.standard_normal((2 * N, width)), BF16), put(gpu, np.ones(width)), put(gpu, rng.standard_normal((taps, 2 * N)))
+    pos, gp, third = ints(gpu, [1]), gpu.B.GateParams(7.0, 1.0, 0.0), N // 3
+    arguments = {"linear_bf16": lambda b, x: (b[0], x, w, N), "gated": lambda b, x: (b[0], x, w, C.byref(gp), N),
+                 "delta_in": lambda b, x: (*b, x, w, wide, taps, third, third, N),
+                 "recurrent_in": lambda b, x: (b[0], b[1], b[3], x, w, wide, wide, wide, taps, N),
+                 "kv": lambda b, x: (*b[:3], x, w, wide, third, third, third, b[3], 1, None, pos, 2)}[product]
+    x, h = put(gpu, x0), zeros(gpu, width, BF16)
+    call(gpu, "lcu_decode_residual_router", x, h, put(gpu, out0), top, None, None, ones, ones, width, width, 1, eps, None, 0, 0, None, None, None)
+    want = get(gpu, h, (width,), BF16)
+    for at in (None, *written):
+        for source in ("x", "out"):
+            buffers = [zeros(gpu, taps * 2 * N).ptr for _ in range(4)]
+            b = {"x": put(gpu, np.pad(x0, (0, taps * 2 * N))), "out": put(gpu, np.pad(out0.ravel(), (0, taps * 2 * N)))}
+            if at is not None:
+                buffers[at] = b[source].ptr + 4 * ((top if source == "out" else 1) * width - 4)
+            h = zeros(gpu, width, BF16)
+            row = gpu.B.StepRow(b["x"].ptr, zeros(gpu, width).ptr, h.ptr, b["out"].ptr, None, None, ones.ptr, ones.ptr, top, width, width, 1, eps)
+            call(gpu, "lcu_step_" + product, *arguments(buffers, C.byref(row)))
+            assert np.array_equal(get(gpu, h, (width,), BF16), want if at is not None else np.zeros(width)), (at, source)
     gpu.release()
