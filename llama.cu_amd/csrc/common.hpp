@@ -168,7 +168,9 @@ __host__ __device__ __forceinline__ float divide_by(float x, float d, float reci
 // division, with the same result for all a and b.  exp_ieee's scaling in one step where 2^k is a normal number; the quotient from the
 // reciprocal by a Newton step and Markstein's correction, the divisor lying between 1 and 6.1e37.  Below -87 the quotient is
 // smaller than anything that times a finite b is not 0 in fp16; beyond 88.72283 the exponential is infinite and the quotient -0; above 80
-// the divisor is 1.  (Every a with b of all kinds: test_silu_of_every_half.)
+// the divisor is 1.  The correction gives the IEEE quotient from a reciprocal that is a unit off too, but for one divisor, 2 - 2^-23 of
+// a = 2^-23: there it needs the chip's reciprocal to round up, as it does (else b = 0.5, 2.5, 4.5 ..., whose products are ties among the
+// subnormals, would give other outputs).  (Every a with b of all kinds, these among them: test_silu_of_every_half.)
 __device__ __forceinline__ half_t silu_mul(half_t a, half_t b) {
   const float val = (float)a, x = fminf(-val, 87.0f);
   const float magic = x * 1.44269504f + 12582912.0f;
