@@ -1685,16 +1685,22 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
       // More 128x64 tiles than compute units, two to a compute unit: against gemm_dl_kernel 40 drawn products of K 256 to 5000 take 0.98 of the time
       // (0.92 to 1.02; 1038x4096x2048 37.5 / 34.8 us), uint8 0.78 (0.70 to 0.86; 559x1792x3352 25.6 / 18.0): every code converted once, not twice.
       if (plan.tiles == row_tiles::narrow) {
-        if constexpr (!U8) return launch_tile<128, 64, 2, 2, 3, 3, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
-        if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 3, 3, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
-        return launch_dl<128, 64, 2, 2, 1, 3, U8>(op, A, M, K, N, block, beta, st);
+        if constexpr (U8) {
+          if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 3, 3, true, false>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+          return launch_dl<128, 64, 2, 2, 1, 3, true>(op, A, M, K, N, block, beta, st);
+        } else {
+          return launch_tile<128, 64, 2, 2, 3, 3, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
+        }
       }
       // us, two groups of four wavefronts that halve the stages on gemm_dl_kernel / four that sum them in turn here: 512 rows of K 256, 512, 1024, 2048,
       // 4096 (4096 columns; 2048) 6.3 / 5.2, 7.2 / 6.1, 10.9 / 9.7, 15.4 / 15.0, 28.9 / 29.3; 300x4096x4096 25.1 / 23.8, 1000x2048x2048 17.2 / 15.7; 70
       // drawn products 0.91 of the time (0.82 to 1.03), 45 in uint8 0.84 (0.79 to 0.88).  24 KB a stage on their way into LDS bound it over a long K.
-      if constexpr (!U8) return launch_tile<128, 64, 2, 2, 4, 4, false, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
-      if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 4, 4, true, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
-      return launch_dl<128, 64, 2, 2, 2, 3, U8>(op, A, M, K, N, block, beta, st);
+      if constexpr (U8) {
+        if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 4, 4, true, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
+        return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);
+      } else {
+        return launch_tile<128, 64, 2, 2, 4, 4, false, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
+      }
     }
   }
   // ragged K: the register-staged kernel, one matrix per launch
