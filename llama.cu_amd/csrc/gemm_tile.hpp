@@ -167,7 +167,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave % WM) * shape::WR, wn = (wave / WM) * shape::WC;
   // request j of a wavefront is rows (wave + j NW) 8 .. + 7 of the tile: of the same matrix for every j
-  if constexpr (EP::PAIRED) W = (wave >> 1) & 1 ? more.W[0] : W0;
+  if constexpr (EP::PAIRED) W = paired_matrix(wave * 8) == 1 ? more.W[0] : W0;
   const int matrix_n = EP::PAIRED ? N / 2 : N;
 
   // this workgroup's K stages
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
       b_off[j] = row_piece(n0 + row, N, (uint32_t)K, g);
     } else {
       const int row = c / 8, g = (c % 8) ^ ((row / 2) % 8), n = n0 + row;
-      b_off[j] = row_piece(EP::PAIRED ? n / 32 * 16 + n % 16 : n, matrix_n, (uint32_t)K * 2u, g);
+      b_off[j] = row_piece(EP::PAIRED ? paired_row(n) : n, matrix_n, (uint32_t)K * 2u, g);
     }
   }
   // first scale of the rows whose scales this lane requests, and of those of its fragments

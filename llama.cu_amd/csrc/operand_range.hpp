@@ -11,6 +11,10 @@ constexpr uint32_t row_piece(int row, int rows, uint32_t row_bytes, int piece) {
   return (uint32_t)(row < rows ? row : rows - 1) * row_bytes + (uint32_t)piece * 16u;
 }
 
+// Columns that alternate between two matrices, sixteen of each: which of them column n is of, and its row there
+constexpr int paired_matrix(int n) { return n / 16 % 2; }
+constexpr int paired_row(int n) { return n / 32 * 16 + n % 16; }
+
 // scalar offset of a request for the stage that begins `along` bytes into a row.  Behind the last stage the resource's
 // length is 0, and the offset is 0 with it: such a request counts as any other and lies outside the length whichever
 // way a range check sets the scalar offset off against it.

@@ -1,7 +1,8 @@
 // Every buffer request that gemm_tile_kernel and gemm_stream_kernel make for a set of shapes, walked on the host with
 // the kernels' own arithmetic (csrc/operand_range.hpp) in the order of their loops: whatever a request may reach lies in
 // its operand, under either reading of a raw buffer's range check.  Argument "offset": the scalar offset stays when the
-// length becomes 0; the walk must then find requests past the end (and says so by its exit code).
+// length becomes 0; "columns": two matrices whose columns alternate are clamped at the columns of both.  The walk must then
+// find requests past the end (and says so by its exit code).
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
@@ -11,7 +12,7 @@
 
 namespace {
 
-bool plant = false;
+bool plant = false, plant_columns = false;
 long requests = 0, outside = 0;
 
 uint32_t along_of(uint32_t length, uint32_t along) { return plant ? along : lcu::stage_offset(length, along); }
@@ -69,6 +70,37 @@ void walk_tile(const shape& s, int BM, int BN, int NS, int NB = 0, int step = 1)
         for (int st = 0; st < NB; ++st) issue(st - (NB - NS), st);
         for (int t = 0; t < nt - 1; ++t) issue(t + NS, t + NB);
       }
+    }
+  }
+}
+
+// gemm_tile.hpp with the columns of two matrices of N rows in turn: tiles of BM x BN of WAVES wavefronts from column `from` on, each wavefront's requests
+// from one matrix
+void walk_paired(const shape& s, int BM, int BN, int waves, int NS, int NB, int from) {
+  const uint32_t K = s.K;
+  const uint64_t a_size = (uint64_t)s.M * K * 2, w_size = (uint64_t)s.N * K * 2;
+  const int nt = s.K / 64, columns = 2 * s.N, last = from + (columns - from - 1) / BN * BN, clamp = plant_columns ? columns : s.N;
+  for (int m0 : {0, (s.M - 1) / BM * BM}) {
+    for (int n0 : {from, last}) {
+      uint32_t la = (uint32_t)a_size, lw = (uint32_t)(plant_columns ? 2 * w_size : w_size);
+      const auto issue = [&](int a, int b) {
+        if (a == nt) la = 0;
+        if (b == nt) lw = 0;
+        const uint32_t along_a = along_of(la, (uint32_t)a * 128u), along_w = along_of(lw, (uint32_t)b * 128u);
+        for (int row = 0; a >= 0 && row < BM; ++row)
+          for (int g = 0; g < 8; ++g) request(la, lcu::row_piece(m0 + row, s.M, K * 2, g), along_a, 16, a_size);
+        for (int wave = 0; wave < waves; ++wave) {
+          for (int j = 0; j < BN / 8 / waves; ++j) {
+            for (int i = 0; i < 8; ++i) {
+              const int n = n0 + (wave + j * waves) * 8 + i;
+              if (lcu::paired_matrix(n) != lcu::paired_matrix(wave * 8)) ++outside;  // not in the wavefront's matrix
+              for (int g = 0; g < 8; ++g) request(lw, lcu::row_piece(lcu::paired_row(n), clamp, K * 2, g), along_w, 16, w_size);
+            }
+          }
+        }
+      };
+      for (int st = 0; st < NB; ++st) issue(st - (NB - NS), st);
+      for (int t = 0; t < nt - 1; ++t) issue(t + NS, t + NB);
     }
   }
 }
@@ -131,6 +163,7 @@ void walk_stream(const shape& s) {
 
 int main(int argc, char** argv) {
   plant = argc > 1 && !strcmp(argv[1], "offset");
+  plant_columns = argc > 1 && !strcmp(argv[1], "columns");
   // K of one to many stages, shorter than the ring too; rows and columns past the last whole tile; one and several scales per
   // row, the number of all of them even; operands just below 4 GiB
   const shape tiles[] = {{300, 64, 1030, 0, 1},   {65, 128, 20500, 0, 1},    {2049, 192, 4100, 0, 1},  {100, 5120, 1030, 0, 3},
@@ -145,6 +178,18 @@ int main(int argc, char** argv) {
     walk_tile(s, 256, 192, s.block ? 3 : 2, s.block ? 3 : 4);
     walk_tile(s, 256, 256, 2, 3);
     if (s.K % 128 == 0) walk_tile(s, 128, 128, 4, 4, 2);
+  }
+  // hidden columns a multiple of 16 and of no tile's width; all tiles, and those of a second launch over the columns that whole rounds leave
+  const shape pairs[] = {{65, 128, 10256, 0, 1}, {300, 384, 5136, 0, 1}, {1033, 2048, 6704, 0, 1}, {100, 64, 16400, 0, 1}, {129, 16384, 65520, 0, 1}};
+  for (const shape& s : pairs) {
+    for (int share : {0, 2}) {
+      const auto from = [&](int columns) { return share == 0 ? 0 : 2 * s.N / columns * (share - 1) / share * columns; };
+      walk_paired(s, 128, 256, 8, 3, 3, from(256));
+      walk_paired(s, 128, 128, 4, 4, 4, from(192));
+      walk_paired(s, 256, 256, 4, 2, 3, from(256));
+      walk_paired(s, 256, 192, 4, 2, 4, from(192));
+      walk_paired(s, 256, 128, 8, 3, 3, from(128));
+    }
   }
   const shape experts[] = {{512, 4096, 5632, 0, 1}, {700, 576, 1000, 0, 1}, {130, 64, 200, 0, 1}, {50, 1024, 128, 0, 1}, {300, 448, 130, 0, 1}};
   for (const shape& s : experts) {
