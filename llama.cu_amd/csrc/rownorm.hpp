@@ -160,7 +160,9 @@ __device__ __forceinline__ void scale_row(row_t<NV, TH>& r, const row_shape& rs,
     if (rs.groups == 1) {
       const float scale = 1.0f / sqrtf(sum_of_pieces(piece, per) / (float)part + rs.eps);
 #pragma unroll
-      for (int j = 0; j < NV; ++j) r.v[j] *= scale * w.v[j];
+      for (int j = 0; j < NV; ++j) {
+        if (j * WAVES + wave < per) r.v[j] *= scale * w.v[j];  // the padding stays zeros, also under a scale that is not finite
+      }
       __syncthreads();
       return;
     }

@@ -219,6 +219,23 @@ def test_grouped_norm_residual_and_embedding(gpu, dt, width, groups, rows):
     gpu.release()
 
 
+# a row that is not finite keeps its padding: parts of whole pieces of 256 columns with padding behind them, and a width that is none
+@BOTH
+@pytest.mark.parametrize("width,groups,ld", [(512, 1, 640), (256, 1, 1088), (1024, 2, 1152), (768, 1, 2112), (500, 1, 640)])
+@pytest.mark.parametrize("rows", [1, 3])
+def test_padding_of_rows_that_are_not_finite(gpu, dt, width, groups, ld, rows):
+    rng = np.random.default_rng(width)
+    out = rng.standard_normal((rows, width))
+    out[0, 3] = np.nan
+    ones = put(gpu, pad(np.ones(width), ld))
+    x, h = zeros(gpu, (rows, ld)), zeros(gpu, (rows, ld), dt)
+    call(gpu, "lcu_residual_norm", x, h, put(gpu, pad(out, ld)), None, 1, None, None, ones, ones, dt, rows, width, ld, groups, 1e-5)
+    for got in (get(gpu, x, (rows, ld)), get(gpu, h, (rows, ld), dt)):
+        assert np.isnan(got[0, :width // groups]).all() and np.isfinite(got[1:]).all()
+        assert (got[:, width:] == 0).all()
+    gpu.release()
+
+
 @pytest.mark.parametrize("width,groups,experts,top", [(96, 1, 5, 1), (320, 5, 12, 3), (1024, 2, 40, 2), (4352, 17, 70, 4), (9216, 9, 17, 2), (12288, 3, 512, 5), (11000, 1000, 20, 1)])
 def test_one_row_step_with_router(gpu, width, groups, experts, top):
     rng = np.random.default_rng(width)
