@@ -1651,9 +1651,10 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
     // three matrices 55 -> 41, 512x4096x5120 54 -> 39.
     if (plan.tiles == row_tiles::medium) {
       if constexpr (U8) {
-        // Several matrices, each with so few tiles that a call of its own would sum the half stages apart: so does their common
-        // launch, on the kernel that such a call takes (512 rows, three times 3072x3072: 86 us on the register-staged
-        // kernel, 75 in separate calls, 71 here; blocks of 32 96 / 77 / 73; 1000 rows, twice 2048 columns of K 4608 85 / 76 / 74).
+        // Several matrices, each with so few tiles that a call of its own would sum the even and the odd stages apart: so does their common
+        // launch, on gemm_dl_kernel.  us, weights from memory, separate calls / here: blocks of 32, which such calls take to the same kernel,
+        // 512 rows, three times 3072x3072 78 / 73, 1000 rows, twice 2048 columns of K 4608 74 / 73.  Blocks of 64 << n, which they take to the
+        // two chains of gemm_tile_kernel below, 67 / 73 and 63 / 72, 768 rows, three times 2048x2048 49 / 51: there this launch is behind.
         const bool one_chain = tiles128 < 256 || tiles128 / nm >= 256 || tiles64 / nm > 256;
         if (!one_chain) return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);
         // us, the older kernel / here, K 256, 512, 1024, 2048: 512 rows of 5120 columns 7.6 / 7.8, 10.5 / 9.8, 16.3 / 13.7; one matrix with
@@ -1692,9 +1693,10 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
           return launch_tile<128, 64, 2, 2, 3, 3, false, false>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
         }
       }
-      // us, two groups of four wavefronts that halve the stages on gemm_dl_kernel / four that sum them in turn here: 512 rows of K 256, 512, 1024, 2048,
-      // 4096 (4096 columns; 2048) 6.3 / 5.2, 7.2 / 6.1, 10.9 / 9.7, 15.4 / 15.0, 28.9 / 29.3; 300x4096x4096 25.1 / 23.8, 1000x2048x2048 17.2 / 15.7; 70
-      // drawn products 0.91 of the time (0.82 to 1.03), 45 in uint8 0.84 (0.79 to 0.88).  24 KB a stage on their way into LDS bound it over a long K.
+      // us, two groups of four wavefronts that halve the stages on gemm_dl_kernel / four that sum them in turn here: 300x4096x4096 25.1 / 23.8,
+      // 1000x2048x2048 17.2 / 15.7; 512 rows of 4096 columns, K 256, 512, 1024, 2048 6.3 / 5.2, 7.2 / 6.1, 10.9 / 9.7, 15.4 / 15.0, but K 4096 28.9 / 29.3:
+      // 24 KB a stage on their way into LDS bound it over a long K, and the rest is what it gains.  70 drawn products 0.91 of the time (0.82 to
+      // 1.03), 45 in uint8 0.84 (0.79 to 0.88).
       if constexpr (U8) {
         if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 4, 4, true, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
         return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);

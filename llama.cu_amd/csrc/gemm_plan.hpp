@@ -135,7 +135,9 @@ inline large_tiles_t plan_large(product_type type, int M, int K, int N, int n_ma
 // one the tiles do, in between both less (product, residual and norm, separate / here, us: fp16 80x4096x4096 30 / 24, 256 rows 33 / 29, 512 rows
 // 35.5 / 34.7, 1301x1408x512 15.7 / 17.3, 1096x1152x512 14.6 / 15.7; uint8 512x4096x4096 45 / 39, 700x2048x2048 25.1 / 23.1, 693x1408x2048
 // 20.2 / 22.0, 1290x768x512 14.9 / 16.3; of 7270 drawn products that these lines take 6 are more than 3 % slower so, on average they take 0.8 of
-// the time).
+// the time).  That was against separate products on gemm_dl_kernel.  On the 128x64 tiles of gemm_tile_kernel, which they take now, they are ahead of some
+// that these lines take (fp16 80x4096x4096 27.6 / 24.9, 256 rows 31.1 / 29.5, 400 rows 26.9 / 27.7, 512 rows 32.0 / 32.7, 200x2048x2048 16.2 / 16.6;
+// uint8 300x1152x1030 19.3 / 16.4, 512x4096x4096 34.3 / 35.4, 700x2048x2048 19.7 / 22.2).
 struct left_sums_t {
   int splits, step;
 };
