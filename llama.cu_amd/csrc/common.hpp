@@ -90,6 +90,8 @@ struct step_fetch {
     if (blockIdx.x == 0 && (int)threadIdx.x < words) dst[threadIdx.x] = src[threadIdx.x];
   }
 };
+// A word that the host may be watching in page-locked memory: written as a whole, past the caches.
+__device__ __forceinline__ void leave_word(int* at, int value) { __hip_atomic_store(at, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 constexpr size_t STEP_FETCH_MAX = 256 * 4;  // bytes
 
 inline bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {

@@ -361,8 +361,8 @@ __global__ __launch_bounds__(1024) void softmax_argmax_kernel(half_t* __restrict
           idx = sidx[w];
         }
       }
-      *index = idx == 0x7fffffff ? 0 : idx;
-      if (status_in) index[1] = (int)*status_in;
+      leave_word(index, idx == 0x7fffffff ? 0 : idx);
+      if (status_in) leave_word(index + 1, (int)*status_in);
     }
     return;
   }
@@ -439,8 +439,8 @@ __global__ __launch_bounds__(1024) void softmax_argmax_kernel(half_t* __restrict
         idx = sidx[w];
       }
     }
-    *index = idx == 0x7fffffff ? 0 : idx;
-    if (status_in) index[1] = (int)*status_in;
+    leave_word(index, idx == 0x7fffffff ? 0 : idx);
+    if (status_in) leave_word(index + 1, (int)*status_in);
   }
 }
 

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(1024) void argmax_f32_kernel(int* __restrict__ inde
   __syncthreads();
   if (tid == 0) {
     for (int w = 1; w < 16; ++w) take(sred[w], sidx[w]);
-    *index = idx == 0x7fffffff ? 0 : idx;
+    leave_word(index, idx == 0x7fffffff ? 0 : idx);
   }
 }
 

@@ -96,6 +96,8 @@ struct llama_batch_context_impl final : public llama_batch_context {
     }
     graph_bound_ = bound;
     ++calls_;
+    const awaited_words answers(t_argmax_, B);
+    answers.expect();
     {
       device_structure_lock lock(device_structure_mutex());  // capture, instantiation, launch: see host_common.hpp
       if (!graph_ && calls_ >= 2) {
@@ -109,7 +111,7 @@ struct llama_batch_context_impl final : public llama_batch_context {
         enqueue_step(bound);
       }
     }
-    LCU_CHECK(lcu_sync(stream_));
+    answers.await(stream_);
     const int* idx = (const int*)t_argmax_.data();
     std::vector<short> out(B);
     for (int b = 0; b < B; ++b) {
@@ -129,6 +131,7 @@ struct llama_batch_context_impl final : public llama_batch_context {
   void drop_graph() {
     if (graph_) {
       device_structure_lock lock(device_structure_mutex());
+      LCU_CHECK(lcu_sync(stream_));  // its last launch may still be ending
       LCU_CHECK(lcu_graph_destroy(graph_));
       graph_ = nullptr;
     }

@@ -496,6 +496,7 @@ void layered_context_impl::drop_graph() {
   for (auto& d : decode_) {
     if (d.graph) {
       device_structure_lock lock(device_structure_mutex());
+      LCU_CHECK(lcu_sync(stream_));  // its last launch may still be ending
       LCU_CHECK(lcu_graph_destroy(d.graph));
       d.graph = nullptr;
     }
@@ -534,6 +535,8 @@ int layered_context_impl::forward(const int32_t* tokens, int n, const int32_t* w
   if (recording_) residual_.assign(m.layers.size(), {});
   const bool fused = n == 1 && m.dtype == LCU_BF16 && fused_step_ && !recording_;
   int token = -1;
+  const awaited_words answer(t_index_, 1);
+  answer.expect();
   for (int at = 0; at < n; at += rows_) {
     const int count = std::min(rows_, n - at);
     const bool ends = at + count == n;
@@ -583,7 +586,11 @@ int layered_context_impl::forward(const int32_t* tokens, int n, const int32_t* w
         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
         LCU_CHECK(lcu_sample_row(t_index_.data(), t_probs_.data(), vocab, z ^ (z >> 31), nullptr, stream_));
       }
-      LCU_CHECK(lcu_sync(stream_));
+      if (sampling_) {
+        LCU_CHECK(lcu_sync(stream_));  // the sampler's launch writes the token once more
+      } else {
+        answer.await(stream_);
+      }
       memcpy(&token, t_index_.data(), 4);
     }
     for (size_t i = 0; i < slots.size(); ++i) {  // consecutive rows of logits

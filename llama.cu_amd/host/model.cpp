@@ -478,6 +478,7 @@ void llama_context_impl::greedy() {
 void llama_context_impl::drop_graph() {
   if (decode_graph_) {
     device_structure_lock lock(device_structure_mutex());
+    LCU_CHECK(lcu_sync(stream_));  // its last launch may still be ending
     LCU_CHECK(lcu_graph_destroy(decode_graph_));
     decode_graph_ = nullptr;
   }
@@ -548,6 +549,8 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
   if (n == 1) {
     one_step.lock();
   }
+  const awaited_words answer(t_argmax_, 2);
+  answer.expect();
   if (n == 1) {
     // A decode step is ~260 launches of a few microseconds each: the first one runs eagerly (and
     // loads the kernels), the second is captured into a HIP graph, every later one replays it.
@@ -556,6 +559,7 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
     const int bound = (start_pos_ + 1 <= 1024 && context_len_ > 1024) ? 1024 : (int)context_len_;
     device_structure_lock lock(device_structure_mutex());  // capture, instantiation, launch: see host_common.hpp
     if (decode_graph_ && bound != decode_bound_) {
+      LCU_CHECK(lcu_sync(stream_));  // its last launch may still be ending
       LCU_CHECK(lcu_graph_destroy(decode_graph_));
       decode_graph_ = nullptr;
     }
@@ -582,7 +586,11 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
     unsigned timeouts;
   } result{0, 0};
   const auto await_result = [&] {  // 1198-1200
-    LCU_CHECK(lcu_sync(stream_));
+    if (sampling_) {
+      LCU_CHECK(lcu_sync(stream_));  // the sampler's launch writes the token once more
+    } else {
+      answer.await(stream_);
+    }
     memcpy(&result, t_argmax_.data(), sizeof(result));
   };
   await_result();
@@ -604,6 +612,7 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
       ++hand_over_fallbacks_;
       hand_overs_ = false;
       drop_graph();
+      answer.expect();
       enqueue_all();
       await_result();
       timeouts_seen_ = result.timeouts;

@@ -113,3 +113,40 @@ def test_layered_embedding_with_the_steps_state(gpu, words, width, learned):
     assert all(np.array_equal(a, b) for a, b in zip(*results))
     assert np.array_equal(gpu.host(out, (2,), np.int32), words[:2])
     gpu.release()
+
+
+@pytest.mark.parametrize("kind", ["fp16", "uint8", "layered", "batch"])
+def test_a_calls_token_is_its_own(gpu, kind):
+    """What a call returns is read as soon as it is there: after every one of many calls, short prompts and captured steps in turn, it is the first
+    maximum of what that call left, and a context used again gives the same."""
+    P = gpu.P
+    if kind == "layered":
+        model = P.Model(config={"architecture": "Logivik", "vocab": 301, "width": 64, "embedding": {"scale": 8.0}, "norm": {"eps": 1e-5}, "layers": [
+            {"type": "latent_attention_2", "mlp": {"kind": "dense", "ff": 128},
+             "mixer": {"heads": 2, "dim": 32, "vdim": 32, "kv_rank": 32, "q_rank": 32, "scale": 0.2, "mask": {"size": 64}}}]}, seed=4)
+    else:
+        model = P.Model(dim=256, multiple_of=128, n_heads=2, n_layers=1, n_vocab=512, seed=5, weight_std=0.05, q_type=int(kind == "uint8"), qblock=128)
+    ctx = P.BatchContext(model, 3, context_len=96) if kind == "batch" else P.Context(model, context_len=96)
+    ids = np.random.default_rng(1).integers(0, 301, 200).astype(np.int16)
+    runs = []
+    for _ in range(2):
+        seen = []
+        for b in range(3):
+            ctx.clear_tokens(*([b] if kind == "batch" else []))
+            if kind == "batch":
+                ctx.next_token(b, ids[b:b + 2])
+        for step in range(30):
+            if kind == "batch":
+                token = list(ctx.next_tokens(ids[3 * step:3 * step + 3]))
+                rows = ctx.probs().reshape(3, -1)
+            else:
+                token = [ctx.next_token(ids[5 * step:5 * step + (3 if step % 7 == 3 else 1)])]
+                rows = ctx.probs().reshape(1, -1)
+            if kind != "layered":  # whose token is that of the fp32 logits: fp16 probabilities may tie
+                assert token == [int(i) for i in rows.argmax(1)]
+            assert all(rows[i, t] == rows[i].max() for i, t in enumerate(token))
+            seen.append(token)
+        runs.append(seen)
+    assert runs[0] == runs[1] and len({tuple(t) for t in runs[0]}) > 3
+    ctx.close()
+    model.close()
