@@ -865,6 +865,14 @@ __device__ __forceinline__ int v_row(int p) {
   return (p & ~31) + 4 * g + (e & 3) + 16 * (e >> 2);
 }
 
+// two scores less the maximum of their row, no lower than exp_ieee_above takes
+__device__ __forceinline__ void less_max(float (&d)[2], half2_t s, float m) {
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(d[0]) : "v"(s), "v"(m));
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d[1]) : "v"(s), "v"(m));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) d[i] = __builtin_amdgcn_fmed3f(d[i], EXP_LEAST, 0.0f);
+}
+
 __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restrict__ out, const half_t* __restrict__ q,
                                                                 const half_t* __restrict__ k, const half_t* __restrict__ v,
                                                                 int n_new, int T, int start_pos, int dim, int n_tiles) {
@@ -883,21 +891,13 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   const int Tc = (c_end + CW - 1) / CW * CW;
   const int SLD = Tc + 8;
 
-  half_t* Qs = reinterpret_cast<half_t*>(smem);             // [BR][QLD]
-  half_t* KVs = Qs + BR * QLD;                              // K chunk [CW][QLD] or V chunk [CW][VLD]
+  half_t* KVs = reinterpret_cast<half_t*>(smem);            // K chunk [CW][QLD] or V chunk [CW][VLD]
   half_t* Ss = KVs + CW * VLD;                              // [BR][SLD]
 
-  // Q tile
-  for (int c = tid; c < BR * HD / 8; c += 256) {
-    const int row = c >> 4, col = (c & 15) * 8;
-    const int gr = r0 + row;
-    half8_t val = (half8_t)(0.0f);
-    if (gr < n_new) val = *reinterpret_cast<const half8_t*>(q + (size_t)gr * dim + h * HD + col);
-    *reinterpret_cast<half8_t*>(&Qs[row * QLD + col]) = val;
-  }
-
-  const float denom = sqrtf((float)HD), inverse = 1.0f / denom;
   const int frow = lane & 15, fk = (lane >> 4) * 8;
+  half8_t qf[HD / 32];  // this lane's query; rows past the last one: the last one, whose outputs nobody stores twice
+#pragma unroll
+  for (int i = 0; i < HD / 32; ++i) qf[i] = *reinterpret_cast<const half8_t*>(q + (size_t)min(r0 + frow, n_new - 1) * dim + h * HD + i * 32 + fk);
   // A chunk of 64 cache rows is 64 x 128 halves = 4 x 16 bytes per thread.  The next chunk is
   // requested into registers before the current one is multiplied, so its latency hides behind
   // the matrix instructions instead of standing between two barriers.
@@ -952,24 +952,23 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   prefetch_first(k);
   for_chunks(k, [&](int c0) {
     float4_t acc = (float4_t)(0.0f);
+    half8_t kf[HD / 32];
 #pragma unroll
-    for (int ks = 0; ks < HD; ks += 32) {
-      const half8_t fb = *reinterpret_cast<const half8_t*>(&KVs[(wave * 16 + frow) * QLD + ks + fk]);
-      const half8_t fa = *reinterpret_cast<const half8_t*>(&Qs[frow * QLD + ks + fk]);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb, acc, 0, 0, 0);
-    }
+    for (int i = 0; i < HD / 32; ++i) kf[i] = *reinterpret_cast<const half8_t*>(&KVs[(wave * 16 + frow) * QLD + i * 32 + fk]);
+    __builtin_amdgcn_sched_barrier(0);  // all of them asked for before the first is waited for
+#pragma unroll
+    for (int i = 0; i < HD / 32; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qf[i], kf[i], acc, 0, 0, 0);
     // accumulator register e of lane l is (row 4*(l/16) + e, column l%16)
     const int col = c0 + wave * 16 + (lane & 15);
-    float size = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) size = fmaxf(size, fabsf(acc[e]));
-    const bool plain = __ballot(size > 3.402823466e38f) == 0;  // infinite products are divided the long way (divide_by)
+    for (int e = 0; e < 4; e += 2) {
+      const half2_t scores = round_f16_pair(score_of(acc[e]), score_of(acc[e + 1]));
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int row = (lane >> 4) * 4 + e;
-      const bool masked = col > r0 + row + start_pos || col >= T;  // llama_cu.cu:415
-      acc[e] = plain ? divide_by(acc[e], denom, inverse) : acc[e] / denom;
-      Ss[row * SLD + col] = masked ? (half_t)(-INFINITY) : round_f16(acc[e]);
+      for (int y = 0; y < 2; ++y) {
+        const int row = (lane >> 4) * 4 + e + y;
+        const bool masked = col > r0 + row + start_pos || col >= T;  // llama_cu.cu:415
+        Ss[row * SLD + col] = masked ? (half_t)(-INFINITY) : scores[y];
+      }
     }
   });
   // the first V chunks travel while the softmax runs
@@ -979,36 +978,70 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   // ---- softmax over each row of the strip (llama_cu.cu:433-499): wave w owns rows w * BR / 4 on, two at a time; the bits of
   // exp_ieee and a true division, as in every other softmax here.  Vector instructions are what it takes: up to 1024 columns a lane
   // keeps its pairs of neighbouring scores and takes each exponential once (32 heads, n = T = 512: 25.5 us with exponentials twice and
-  // general divisions, 19.8 so, 17.8 with V turned on its way out of LDS below).
+  // general divisions, 19.8 so, 17.8 with V turned on its way out of LDS below;
+  // 16.7 with the shorter forms of common.hpp, queries in registers and a chunk's fragments asked for together; 16 heads 1000 rows 35.4 -> 29.5, 52 heads
+  // 512 rows 26.2 -> 23.9).  The general forms where a maximum is not finite.
   const int pairs = Tc / 2;
+  const auto whole_row = [&](half2_t* srow) {
+    float m = -INFINITY;
+    for (int i = lane; i < pairs; i += WAVE) {
+      const half2_t v = srow[i];
+      m = fmaxf(m, fmaxf((float)v.x, (float)v.y));
+    }
+    m = wave_max_dpp(m);
+    float s = 0.0f;
+    for (int i = lane; i < pairs; i += WAVE) {
+      const half2_t v = srow[i];
+      s += exp_ieee_nonpositive((float)v.x - m) + exp_ieee_nonpositive((float)v.y - m);
+    }
+    s = wave_sum(s);
+    const float share = 1.0f / s;
+    for (int i = lane; i < pairs; i += WAVE) {
+      const half2_t v = srow[i];
+      half2_t p;
+      p.x = round_f16(divide_by(exp_ieee_nonpositive((float)v.x - m), s, share));
+      p.y = round_f16(divide_by(exp_ieee_nonpositive((float)v.y - m), s, share));
+      srow[i] = p;
+    }
+  };
   const auto softmax = [&](auto most) {
     constexpr int NP = decltype(most)::value;
 #pragma unroll 1
     for (int rr = 0; rr < BR / 4; rr += 2) {
       half2_t* row[2];
-      float2 x[2][NP];
-      float m[2] = {-INFINITY, -INFINITY}, sum[2] = {0.0f, 0.0f};
+      half2_t v[2][NP];
+      float m[2];
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
         row[r] = reinterpret_cast<half2_t*>(Ss + (wave * (BR / 4) + rr + r) * SLD);
+        half2_t top = {(half_t)-INFINITY, (half_t)-INFINITY};
 #pragma unroll
         for (int j = 0; j < NP; ++j) {
-          x[r][j] = make_float2(-INFINITY, -INFINITY);
-          if (j * WAVE + lane < pairs) {
-            const half2_t v = row[r][j * WAVE + lane];
-            x[r][j] = make_float2((float)v.x, (float)v.y);
-          }
-          m[r] = fmaxf(m[r], fmaxf(x[r][j].x, x[r][j].y));
+          v[r][j] = (half2_t){(half_t)-INFINITY, (half_t)-INFINITY};
+          if (j * WAVE + lane < pairs) v[r][j] = row[r][j * WAVE + lane];
+          top = __builtin_elementwise_maximum(top, v[r][j]);  // NaN stays NaN
         }
+        m[r] = wave_max_dpp(fmaxf((float)top.x, (float)top.y));
+        if (__ballot(!((float)top.x <= 65504.0f && (float)top.y <= 65504.0f)) != 0) m[r] = NAN;
       }
+      // a maximum that is finite, as it is for finite queries and keys: the short exponentials
+      const bool plain = fabsf(m[0]) <= 65504.0f && fabsf(m[1]) <= 65504.0f;
+      if (!plain) {
+        whole_row(row[0]);
+        whole_row(row[1]);
+        continue;
+      }
+      float2 x[2][NP];
+      float sum[2] = {0.0f, 0.0f};
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
-        m[r] = wave_max_dpp(m[r]);
 #pragma unroll
         for (int j = 0; j < NP; ++j) {
-          x[r][j].x = exp_ieee_nonpositive(x[r][j].x - m[r]);
-          x[r][j].y = exp_ieee_nonpositive(x[r][j].y - m[r]);
-          if (j * WAVE + lane < pairs) sum[r] += x[r][j].x + x[r][j].y;
+          float d[2], e[2];
+          less_max(d, v[r][j], m[r]);
+          exp_ieee_above(e, d);
+          x[r][j] = make_float2(e[0], e[1]);
+          if (j * WAVE + lane < pairs) sum[r] += e[0] + e[1];
         }
       }
 #pragma unroll
@@ -1016,9 +1049,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
         const float total = wave_sum(sum[r]), share = 1.0f / total;
 #pragma unroll
         for (int j = 0; j < NP; ++j) {
-          half2_t p;
-          p.x = round_f16(divide_by(x[r][j].x, total, share));
-          p.y = round_f16(divide_by(x[r][j].y, total, share));
+          const half2_t p = round_f16_pair(divide_by(x[r][j].x, total, share), divide_by(x[r][j].y, total, share));
           if (j * WAVE + lane < pairs) row[r][j * WAVE + lane] = p;
         }
       }
@@ -1031,29 +1062,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   } else if (pairs <= 8 * WAVE) {
     softmax(std::integral_constant<int, 8>{});
   } else {
-    for (int rr = 0; rr < BR / 4; ++rr) {
-      half2_t* srow = reinterpret_cast<half2_t*>(Ss + (wave * (BR / 4) + rr) * SLD);
-      float m = -INFINITY;
-      for (int i = lane; i < pairs; i += WAVE) {
-        const half2_t v = srow[i];
-        m = fmaxf(m, fmaxf((float)v.x, (float)v.y));
-      }
-      m = wave_max_dpp(m);
-      float s = 0.0f;
-      for (int i = lane; i < pairs; i += WAVE) {
-        const half2_t v = srow[i];
-        s += exp_ieee_nonpositive((float)v.x - m) + exp_ieee_nonpositive((float)v.y - m);
-      }
-      s = wave_sum(s);
-      const float share = 1.0f / s;
-      for (int i = lane; i < pairs; i += WAVE) {
-        const half2_t v = srow[i];
-        half2_t p;
-        p.x = round_f16(divide_by(exp_ieee_nonpositive((float)v.x - m), s, share));
-        p.y = round_f16(divide_by(exp_ieee_nonpositive((float)v.y - m), s, share));
-        srow[i] = p;
-      }
-    }
+    for (int rr = 0; rr < BR / 4; ++rr) whole_row(reinterpret_cast<half2_t*>(Ss + (wave * (BR / 4) + rr) * SLD));
   }
 
   // ---- out[BR][HD] = P . V: wave w owns output columns w*32 .. w*32+31 (two 16-wide tiles)
@@ -1066,18 +1075,22 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
   permute_rows = true;
   const int v_at = (lane >> 4) * 4 + ((lane & 15) >> 2), v_col = wave * 32 + (lane & 3) * 4;
   for_chunks(v, [&](int c0) {
+    half8_t pf[CW / 32], vf[CW / 32][2];
 #pragma unroll
-    for (int ks = 0; ks < CW; ks += 32) {
-      const half8_t fa = *reinterpret_cast<const half8_t*>(&Ss[frow * SLD + c0 + ks + fk]);
-      half8_t fb[2];
+    for (int i = 0; i < CW / 32; ++i) {
+      pf[i] = *reinterpret_cast<const half8_t*>(&Ss[frow * SLD + c0 + i * 32 + fk]);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const half_t* at = &KVs[(ks + v_at) * VLD + v_col + j * 16];
+        const half_t* at = &KVs[(i * 32 + v_at) * VLD + v_col + j * 16];
         const half4_t lo = read_transposed(at), hi = read_transposed(at + 16 * VLD);
-        fb[j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        vf[i][j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       }
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb[j], o[j], 0, 0, 0);
+    for (int i = 0; i < CW / 32; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf[i], vf[i][j], o[j], 0, 0, 0);
     }
   });
 #pragma unroll
@@ -1092,23 +1105,43 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(half_t* __restri
 }
 
 // ---- prompts -------------------------------------------------------------------------------------
-// Attention of many rows: NW wavefronts of 16 rows each share the K and V of their head in chunks of 64 cache rows,
-// which travel into a ring of four 16 KB LDS slots, three ahead.
+// Attention of many rows: four wavefronts of 16 rows each share the K and V of their head in chunks of 64 cache rows,
+// which travel into a ring of SLOTS LDS slots of 16 KB, all but one of them ahead.
 //
-// What bounds it is vector instructions: a score that is rounded to fp16, exponentiated and divided where the
-// reference does takes about 50 of them.  So scores are never stored: they are computed three times (the matrix
-// cores have room), for the maximum, for the sum and for the probabilities, and LDS holds no strip of scores, which at
-// 2000 rows left four wavefronts to a compute unit.  Scores are computed with cache rows as rows of the tile, in an
+// What bounds it is vector instructions and LDS reads in turn: a score that is rounded to fp16, exponentiated and divided where the
+// reference does takes 40 of the former, and every wavefront reads all of K three times and V once.  Scores are never stored: they are
+// computed three times (the matrix cores have room), for the maximum, for the sum and for the probabilities, and LDS holds no strip of
+// scores, which at 2000 rows left four wavefronts to a compute unit.  Scores are computed with cache rows as rows of the tile, in an
 // order that leaves a lane eight consecutive ones of its query: the operand of the product with V as it stands, V
 // itself being transposed on its way out of LDS.
 // The sums are those of a wavefront per row: pair p = (column % 128) / 2 adds its two exponentials per 128 columns, then the
 // 64 pairs meet as in wave_sum (llama_cu.cu:433-499); the products with V are a chain over ascending cache rows.
-// 32 heads, n = T = 1987: 502 -> 155 us, 512 rows of 2048: 214 -> 122 us; 52 heads, n = T = 2048: 839 -> 246 us.
-template <int NW>
-__global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_t* __restrict__ out, const half_t* __restrict__ q,
+// One vector instruction waits 8 clocks for the one it depends on, and an LDS read some 130: eight exponentials go side by side, fragments are asked
+// for four instructions ahead, and requests need no address arithmetic but the scalar base of a chunk.  32 heads, n = T: 1987 rows
+// 142 -> 118 us, 1500 rows 91 -> 74, 1024 rows 63 -> 52; 512 rows of 2000 118 -> 97; 52 heads, 1987 rows 212 -> 193.  (Eight wavefronts to a
+// workgroup read K and V half as often from L2: 145 us; 32 rows to a wavefront, which halves the LDS reads and leaves two of them to a SIMD: 156.)
+// Exponentials of N scores (products with a query) less the row's maximum m, which is a score.  In the short forms, for products
+// within +-7e5 (and MASKED_SHORT): the quotient by sqrt(128) in two instructions, which give its fp16 value for every finite product
+// (tests/cxx/kernel_arithmetic.hip); two rounded by one; the difference straight from the half; exp_ieee_nonpositive with the power of two added to the
+// exponent, which leaves e^-87.3 instead of 0 below that: too little to change a sum that has 1 in it, and 0 as a probability.
+template <int N, class SHORT>
+__device__ __forceinline__ void exponentials(float (&e)[N], const float (&x)[N], float m, SHORT short_forms) {
+  if constexpr (SHORT::value) {
+    float d[N / 2][2];
+#pragma unroll
+    for (int i = 0; i < N; i += 2) less_max(d[i / 2], round_f16_pair(score_of(x[i]), score_of(x[i + 1])), m);
+    exp_ieee_above(e, reinterpret_cast<const float(&)[N]>(d));
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) e[i] = exp_ieee_nonpositive((float)round_f16(score_of(x[i])) - m);
+  }
+}
+
+template <int SLOTS>
+__global__ __launch_bounds__(256, 160 / 16 / SLOTS) void prompt_attention_kernel(half_t* __restrict__ out, const half_t* __restrict__ q,
                                                                            const half_t* __restrict__ k, const half_t* __restrict__ v,
                                                                            int n_new, int T, int start_pos, int dim, int n_tiles) {
-  constexpr int ROWS = 16 * NW, SLOT = 64 * HD * 2, R = 16 / NW;  // rows of a workgroup, bytes of a chunk, requests per wavefront
+  constexpr int NW = 4, ROWS = 16 * NW, SLOT = 64 * HD * 2, R = 16 / NW;  // rows of a workgroup, bytes of a chunk, requests per wavefront
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // the tiles that see most columns first
   const int n_heads = gridDim.x / n_tiles;
@@ -1130,34 +1163,51 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
   const auto turn_k = [](int r) { return (r & 3) | (((r >> 3) & 3) << 2); };
   const auto turn_v = [](int r) { return ((r & 3) | (((r >> 3) & 1) << 2)) << 1; };
-  const auto issue = [&](int item) {
-    const bool is_v = item >= 2 * chunks && (item & 1) != 0;
-    const int c = item < chunks ? item : (item < 2 * chunks ? item - chunks : item / 2 - chunks);
-    const half_t* src = (is_v ? v : k) + h * HD;
+  // where this lane's pieces of a chunk lie, from its first row on
+  uint32_t k_from[R], v_from[R];
+  const auto places = [&](uint32_t (&from)[R], bool is_v, int rows) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       const int r = (wave + j * NW) * 4 + (lane >> 4);
-      const int piece = (lane & 15) ^ (is_v ? turn_v(r) : turn_k(r));
-      // rows past T are never used: their scores are masked, their probabilities 0
-      const half_t* from = src + (size_t)min(c * 64 + r, T - 1) * dim + piece * 8;
-      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from),
-                   "s"(lds0 + (item & 3) * SLOT + (wave + j * NW) * 1024)
-                   : "memory", "m0");
+      from[j] = (uint32_t)(min(r, rows - 1) * dim + ((lane & 15) ^ (is_v ? turn_v(r) : turn_k(r))) * 8) * 2;
     }
   };
-  // item i is there for everybody, and item i + 3 on its way into the slot of item i - 1, which everybody has read
-  const auto acquire = [&](int item) {
+  places(k_from, false, 64);
+  places(v_from, true, 64);
+  const auto issue = [&](int item) __attribute__((always_inline)) {
+    const bool is_v = item >= 2 * chunks && (item & 1) != 0;
+    const int c = item < chunks ? item : (item < 2 * chunks ? item - chunks : item / 2 - chunks);
+    const half_t* src = (is_v ? v : k) + h * HD + (size_t)c * 64 * dim;
+    const uint32_t to = lds0 + item % SLOTS * SLOT + wave * 1024;
+    const auto request = [&](const uint32_t (&from)[R]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from[j]), "s"(src), "s"(to + j * NW * 1024) : "memory", "m0");
+      }
+    };
+    if (c * 64 + 64 > T) {  // rows past T are never used: their scores are masked, their probabilities 0
+      uint32_t from[R];
+      places(from, is_v, T - c * 64);
+      request(from);
+    } else if (is_v) {
+      request(v_from);
+    } else {
+      request(k_from);
+    }
+  };
+  // item i is there for everybody, and item i + SLOTS - 1 on its way into the slot of item i - 1, which everybody has read
+  const auto acquire = [&](int item) __attribute__((always_inline)) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const int behind = items - 1 - item;
-    if (behind >= 2) {
+    if (SLOTS > 3 && behind >= 2) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * R) : "memory");
-    } else if (behind == 1) {
+    } else if (behind >= 1) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");
     } else {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     asm volatile("s_barrier" ::: "memory");
-    if (item + 3 < items) issue(item + 3);
+    if (item + SLOTS - 1 < items) issue(item + SLOTS - 1);
   };
 
   // scores of chunk c: s[b][t][e] is column 64 c + 32 b + 8 group + 4 t + e of the lane's query.  Row m of tile (b, t) is
@@ -1165,45 +1215,51 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_
   const int key_row = 8 * (row >> 2) + (row & 3);
   const uint32_t k_base = (uint32_t)key_row * 256;
   const int k_turn = turn_k(key_row);
-  const auto products = [&](float4_t (&s)[2][2], int item) {
-    const unsigned char* slot = smem + (item & 3) * SLOT + k_base;
-    // four sums in turn: each matrix instruction's result is wanted four instructions later
-    // (32 heads, n = T = 1024: 70 us with one sum after the other, 67 us so)
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
+  const auto products = [&](float4_t (&s)[2][2], int item) __attribute__((always_inline)) {
+    const unsigned char* slot = smem + item % SLOTS * SLOT + k_base;
+    // Four sums in turn: each matrix instruction's result is wanted four instructions later (32 heads, n = T = 1024: 70 us with one sum
+    // after the other, 67 us so).  Keys are asked for four instructions ahead: left to itself the compiler asks for one fragment, waits for it
+    // and multiplies it, here and below.
+    half8_t kf[2][4];
+    const auto fetch = [&](int d) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int b = i >> 1, t = i & 1;
-        const half8_t kf = *reinterpret_cast<const half8_t*>(slot + (32 * b + 4 * t) * 256 + (((d * 4 + group) ^ k_turn) * 16));
-        s[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[d], d == 0 ? (float4_t)(0.0f) : s[b][t], 0, 0, 0);
+        kf[d & 1][i] = *reinterpret_cast<const half8_t*>(slot + (32 * (i >> 1) + 4 * (i & 1)) * 256 + (((d * 4 + group) ^ k_turn) * 16));
       }
+    };
+    fetch(0);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      if (d < 3) fetch(d + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float4_t& to = s[i >> 1][i & 1];
+        to = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[d & 1][i], qf[d], d == 0 ? (float4_t)(0.0f) : to, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // the lowest finite value: scaled and rounded to fp16 it is the reference's -infinity
-  constexpr float MASKED = -3.402823466e38f;
-  const auto mask = [&](float4_t (&s)[2][2], int c) {
+  // the lowest finite value: scaled and rounded to fp16 it is the reference's -infinity; and what becomes the lowest finite half
+  constexpr float MASKED = -3.402823466e38f, MASKED_SHORT = -741093.0f;
+  const auto mask = [&](float4_t (&s)[2][2], int c, float masked) {
     if (c < masked_from) return;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (c * 64 + 32 * b + 8 * group + 4 * t + e > limit) s[b][t][e] = MASKED;
-        }
-      }
+    for (int i = 0; i < 16; ++i) {
+      const int b = i >> 3, t = (i >> 2) & 1, e = i & 3;
+      if (c * 64 + 32 * b + 8 * group + 4 * t + e > limit) s[b][t][e] = masked;
     }
   };
 
 #pragma unroll
-  for (int i = 0; i < 3; ++i) issue(i);  // a tile has four items at least
+  for (int i = 0; i < SLOTS - 1; ++i) issue(i);  // a tile has four items at least
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    qf[s] = *reinterpret_cast<const half8_t*>(q + (size_t)min(w0 + row, n_new - 1) * dim + h * HD + s * 32 + group * 8);
+  for (int d = 0; d < 4; ++d) {
+    qf[d] = *reinterpret_cast<const half8_t*>(q + (size_t)min(w0 + row, n_new - 1) * dim + h * HD + d * 32 + group * 8);
   }
   // arrived before the loops: a wait inside them would be for the chunks requested meanwhile too
 #pragma unroll
-  for (int s = 0; s < 4; ++s) asm volatile("" : "+v"(qf[s]));
+  for (int d = 0; d < 4; ++d) asm volatile("" : "+v"(qf[d]));
 
   // ---- maximum.  Rounding and division keep the order, so the largest product gives the largest score.
   float m = -INFINITY, size = 0.0f;
@@ -1212,58 +1268,43 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_
     if (c >= own_chunks) continue;
     float4_t s[2][2];
     products(s, c);
-    mask(s, c);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      m = fmaxf(m, s[i >> 3][(i >> 2) & 1][i & 3]);
-      size = fmaxf(size, fabsf(s[i >> 3][(i >> 2) & 1][i & 3]));
-    }
+    for (int i = 0; i < 16; ++i) size = __builtin_elementwise_maximum(size, fabsf(s[i >> 3][(i >> 2) & 1][i & 3]));  // NaN stays NaN
+    mask(s, c, MASKED);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) m = fmaxf(m, s[i >> 3][(i >> 2) & 1][i & 3]);
   }
+  // Products of all sizes but the largest, infinite and NaN ones: the short forms, whose scores are within +-62 000 and a masked one the lowest
+  // finite half.
+  const bool plain = __ballot(!(size <= 7e5f)) == 0;
   m = fmaxf(m, __shfl_xor(m, 16, WAVE));
-  m = fmaxf(m, __shfl_xor(m, 32, WAVE));
-  const float denom = sqrtf((float)HD), inverse = 1.0f / denom;
-  // an infinite product (infinite operands) would leave NaN in the remainder: such rows are divided the long way
-  const bool plain = __ballot(size > -MASKED) == 0;
-  const auto scaled = [&](float x) { return (float)round_f16(plain ? divide_by(x, denom, inverse) : x / denom); };
-  m = scaled(m);
-  const auto scale = [&](float4_t (&s)[2][2]) {  // products to scores, which are fp16 values; one branch for all of them
-    if (plain) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float4_t& x = s[i >> 3][(i >> 2) & 1];
-        x[i & 3] = (float)round_f16(divide_by(x[i & 3], denom, inverse));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float4_t& x = s[i >> 3][(i >> 2) & 1];
-        x[i & 3] = (float)round_f16(x[i & 3] / denom);
-      }
-    }
-  };
+  m = (float)round_f16(score_of(fmaxf(m, __shfl_xor(m, 32, WAVE))));
 
   // ---- sum
   float pairs[2][2][4] = {};  // [chunk & 1][b][pair]: pair index 32 (chunk & 1) + 16 b + 4 group + pair of 64
-  const auto add_chunk = [&](int c, float (&sum)[2][4]) {
+  const auto add_chunk = [&](int c, float (&sum)[2][4], auto short_forms) __attribute__((always_inline)) {
     acquire(chunks + c);
     if (c >= own_chunks) return;
     float4_t s[2][2];
     products(s, chunks + c);
-    mask(s, c);
-    scale(s);
+    mask(s, c, short_forms ? MASKED_SHORT : MASKED);
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
+      float e[8], of[8];
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const float4_t x = s[b][p >> 1];
-        sum[b][p] += exp_ieee_nonpositive(x[2 * (p & 1)] - m) + exp_ieee_nonpositive(x[2 * (p & 1) + 1] - m);
-      }
+      for (int y = 0; y < 8; ++y) of[y] = s[b][y >> 2][y & 3];
+      exponentials(e, of, m, short_forms);
+#pragma unroll
+      for (int p = 0; p < 4; ++p) sum[b][p] += e[2 * p] + e[2 * p + 1];
     }
   };
-  for (int c = 0; c < chunks; c += 2) {
-    add_chunk(c, pairs[0]);
-    if (c + 1 < chunks) add_chunk(c + 1, pairs[1]);
-  }
+  const auto add_all = [&](auto short_forms) __attribute__((always_inline)) {
+    for (int c = 0; c < chunks; c += 2) {
+      add_chunk(c, pairs[0], short_forms);
+      if (c + 1 < chunks) add_chunk(c + 1, pairs[1], short_forms);
+    }
+  };
+  plain ? add_all(std::true_type{}) : add_all(std::false_type{});
   float quarter[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
@@ -1283,40 +1324,63 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_
   const int v_row = 8 * group + (row >> 2), v_turn = turn_v(v_row);
   const uint32_t v_base = (uint32_t)v_row * 256 + (row & 1) * 8;
   typedef short short4_t __attribute__((ext_vector_type(4)));
-  for (int c = 0; c < chunks; ++c) {
-    const int item = 2 * chunks + 2 * c;
-    half8_t pf[2];
-    acquire(item);
-    if (c < own_chunks) {
-      float4_t s[2][2];
-      products(s, item);
-      mask(s, c);
-      scale(s);
+  const auto weigh_all = [&](auto short_forms) __attribute__((always_inline)) {
+    for (int c = 0; c < chunks; ++c) {
+      const int item = 2 * chunks + 2 * c;
+      half8_t pf[2];
+      acquire(item);
+      if (c < own_chunks) {
+        float4_t s[2][2];
+        products(s, item);
+        mask(s, c, short_forms ? MASKED_SHORT : MASKED);
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < 2; ++b) {
+          float e[8], of[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) pf[b][e] = round_f16(divide_by(exp_ieee_nonpositive(s[b][e >> 2][e & 3] - m), total, share));
+          for (int y = 0; y < 8; ++y) of[y] = s[b][y >> 2][y & 3];
+          exponentials(e, of, m, short_forms);
+#pragma unroll
+          for (int y = 0; y < 8; ++y) e[y] = divide_by(e[y], total, share);
+#pragma unroll
+          for (int y = 0; y < 8; y += 2) {
+            const half2_t two = round_f16_pair(e[y], e[y + 1]);
+            pf[b][y] = two.x;
+            pf[b][y + 1] = two.y;
+          }
+        }
       }
-    }
-    acquire(item + 1);
-    if (c < own_chunks) {
-      const unsigned char* slot = smem + ((item + 1) & 3) * SLOT + v_base;
+      acquire(item + 1);
+      if (c < own_chunks) {
+        const unsigned char* slot = smem + (item + 1) % SLOTS * SLOT + v_base;
+        union {
+          short4_t half[2];
+          half8_t all;
+        } vf[2][4];
+        const auto fetch = [&](int set) __attribute__((always_inline)) {
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
+          for (int i = 0; i < 4; ++i) {
+            const int b = set >> 1, d = (set & 1) * 4 + i;
+            const unsigned char* at = slot + 32 * b * 256 + (((2 * d + ((row >> 1) & 1)) ^ v_turn) * 16);
+            vf[set & 1][i].half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)at);
+            vf[set & 1][i].half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(at + 4 * 256));
+          }
+        };
+        fetch(0);
 #pragma unroll
-        for (int d = 0; d < HD / 16; ++d) {
-          const unsigned char* at = slot + 32 * b * 256 + (((2 * d + ((row >> 1) & 1)) ^ v_turn) * 16);
-          union {
-            short4_t half[2];
-            half8_t all;
-          } vf;
-          vf.half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)at);
-          vf.half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(at + 4 * 256));
-          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf.all, pf[b], o[d], 0, 0, 0);
+        for (int set = 0; set < 4; ++set) {
+          if (set < 3) fetch(set + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int d = (set & 1) * 4 + i;
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[set & 1][i].all, pf[set >> 1], o[d], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
-  }
+  };
+  plain ? weigh_all(std::true_type{}) : weigh_all(std::false_type{});
   if (w0 + row < n_new) {
     half_t* to = out + (size_t)(w0 + row) * dim + h * HD + 4 * group;
 #pragma unroll
@@ -1329,11 +1393,11 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void prompt_attention_kernel(half_
   }
 }
 
-template <int NW>
+template <int SLOTS>
 int launch_prompt_attention(half_t* out, const half_t* q, const half_t* k, const half_t* v, int n_new, int T, int start_pos, int dim,
                             int n_heads, hipStream_t s) {
-  const int n_tiles = (n_new + 16 * NW - 1) / (16 * NW);
-  prompt_attention_kernel<NW><<<n_tiles * n_heads, 64 * NW, 4 * 64 * HD * 2, s>>>(out, q, k, v, n_new, T, start_pos, dim, n_tiles);
+  const int n_tiles = (n_new + 63) / 64;
+  prompt_attention_kernel<SLOTS><<<n_tiles * n_heads, 256, SLOTS * 64 * HD * 2, s>>>(out, q, k, v, n_new, T, start_pos, dim, n_tiles);
   LCU_LAUNCH_CHECK();
   return LCU_OK;
 }
@@ -1401,14 +1465,14 @@ int lcu_attention(void* out_dev, const void* q_dev, const void* k_dev, const voi
   // many scores: the kernel that computes them three times and stores none (scores_again)
   // Its requests and stores are of 16 and 8 bytes: operands that are not so aligned stay with the kernel below.
   const bool aligned = (((uintptr_t)q_dev | (uintptr_t)k_dev | (uintptr_t)v_dev) & 15) == 0 && ((uintptr_t)out_dev & 7) == 0;
-  if (aligned && scores_again(n_heads, n_new, start_pos, st->compute_units > 0 ? st->compute_units : 256)) {
-    // 128 rows to a workgroup read K and V half as often, if two workgroups per compute unit are left
-    if ((long)((n_new + 127) / 128) * n_heads >= 512) {
-      return launch_prompt_attention<8>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T,
-                                        start_pos, dim, n_heads, s);
-    }
-    return launch_prompt_attention<4>((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev, (const half_t*)v_dev, n_new, T,
-                                      start_pos, dim, n_heads, s);
+  const int cus = st->compute_units > 0 ? st->compute_units : 256;
+  if (aligned && scores_again(n_heads, n_new, start_pos, cus)) {
+    // Two workgroups to a compute unit with three chunks ahead, or three with two: up to three of them in all the former, beyond it the
+    // latter (32 heads, n = T, two / three, us: 1024 rows 52 / 53, 1500 rows 74 / 79, 1987 rows 127 / 118, 4000 rows 455 / 425; 52 heads 700 rows
+    // 38.4 / 39.9, 1987 rows 204 / 193)
+    const bool few = (long)((n_new + 63) / 64) * n_heads <= 3L * cus;
+    return (few ? launch_prompt_attention<4> : launch_prompt_attention<3>)((half_t*)out_dev, (const half_t*)q_dev, (const half_t*)k_dev,
+                                                                            (const half_t*)v_dev, n_new, T, start_pos, dim, n_heads, s);
   }
   // (tiles of 32 rows, which read K and V half as often: 52 heads 600 rows 40 / 41 us, 32 heads 800 rows 38 / 40, elsewhere up to 1.7 times as long)
   const int n_tiles = (n_new + BR - 1) / BR;

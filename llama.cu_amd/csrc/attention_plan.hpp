@@ -7,12 +7,12 @@ namespace lcu {
 constexpr int HD = 128;        // head width
 constexpr int BR = 16;         // query rows per workgroup of the kernel that stores its scores
 constexpr int CW = 64;         // cache rows per staged chunk
-constexpr int QLD = HD + 8;    // LDS row stride (halves) of the Q and K tiles
+constexpr int QLD = HD + 8;    // LDS row stride (halves) of K chunks
 constexpr int VLD = HD + 16;   // and of V chunks
 
 inline size_t prefill_lds_bytes(int T) {
   const int Tc = (T + CW - 1) / CW * CW;
-  return ((size_t)BR * QLD + (size_t)CW * VLD + (size_t)BR * (Tc + 8)) * 2;
+  return ((size_t)CW * VLD + (size_t)BR * (Tc + 8)) * 2;
 }
 
 // Whether computing the scores three times and storing none (prompt_attention_kernel) is done sooner than keeping a strip of them in LDS
@@ -26,10 +26,11 @@ inline size_t prefill_lds_bytes(int T) {
 // others for the columns in front of the prompt, which every tile sees, while those of the prompt itself balance (tiles of later rows, which see
 // more of them, go first).  Of 1370 drawn calls 50 take more than 3 % longer than the other kernel so, 303 with the line at 17 000 and 442 at
 // 13 000 (40 heads 452 rows of 1712 104 / 128; 52 heads 306 rows of 1531 94 / 123; 24 heads 1019 rows of 1094 70 / 55).
+// Both take 6 to 18 % less since then (32 heads 1024 rows 63 -> 52, 800 rows 35.5 -> 32); the lines stand where they were.
 inline bool scores_again(int n_heads, int n_new, int start_pos, long cus) {
   const int T = start_pos + n_new;
   const double scores = (double)n_heads * n_new * (start_pos + 0.5 * n_new);
-  const size_t strips = (size_t)160 * 1024 / prefill_lds_bytes(T);
+  const size_t strips = (size_t)160 * 1024 / (prefill_lds_bytes(T) + BR * QLD * 2);  // the lines were measured with a tile of queries in LDS too
   if (strips != 2 || scores >= 17000.0 * T || scores < 11000.0 * T) return scores >= (strips >= 2 ? 17000.0 : 9000.0) * T;
   const long tiles = (long)((n_new + BR - 1) / BR) * n_heads, rounds = (tiles + 2 * cus - 1) / (2 * cus);
   const double kept = 0.0283 * (0.5 * n_new * tiles / (2 * cus) + (double)start_pos * rounds) + 1.4 * rounds + 2.7, again = 0.056 * T + 7.3;  // us

@@ -108,6 +108,13 @@ __device__ __forceinline__ half_t round_f16(float f) {
   return (half_t)f;
 }
 
+// the same for two, by one instruction
+__device__ __forceinline__ half2_t round_f16_pair(float a, float b) {
+  half2_t r;
+  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // e^x in fp32 from IEEE operations only (multiply, fused multiply-add, round to nearest even,
 // integer scaling), so that the host restatement of the same steps gives the same bits; within
 // one ulp of the true value, as the reference's expf is (llama_cu.cu:463, 497, 537 call CUDA's,
@@ -154,6 +161,37 @@ __host__ __device__ __forceinline__ float exp_ieee_nonpositive(float x) {
   const float scale = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, magic) << 23) + 0x3f800000u);
   return x < -87.33654f ? 0.0f : p * scale;
 }
+
+// exp_ieee_nonpositive for EXP_LEAST <= x <= 0: below that it is 0, so its results are normal numbers and the power of two can be added to their
+// exponent.  The same bits (tests/cxx/kernel_arithmetic.hip goes through all of them).
+constexpr float EXP_LEAST = -87.33654f;
+// Several at once: a step waits 8 clocks for the one before, and another wavefront's or another value's takes its place meanwhile.
+template <int N>
+__host__ __device__ __forceinline__ void exp_ieee_above(float (&e)[N], const float (&x)[N]) {
+  float magic[N], r[N], p[N];
+  const auto each = [](auto step) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) step(i);
+  };
+  each([&](int i) { magic[i] = x[i] * 1.44269504f; });
+  each([&](int i) { magic[i] += 12582912.0f; });
+  each([&](int i) { p[i] = magic[i] - 12582912.0f; });
+  each([&](int i) { r[i] = fmaf(p[i], -0.693359375f, x[i]); });
+  each([&](int i) { r[i] = fmaf(p[i], 2.12194440e-4f, r[i]); });
+  each([&](int i) { p[i] = fmaf(1.9875691500e-4f, r[i], 1.3981999507e-3f); });
+  each([&](int i) { p[i] = fmaf(p[i], r[i], 8.3334519073e-3f); });
+  each([&](int i) { p[i] = fmaf(p[i], r[i], 4.1665795894e-2f); });
+  each([&](int i) { p[i] = fmaf(p[i], r[i], 1.6666665459e-1f); });
+  each([&](int i) { p[i] = fmaf(p[i], r[i], 5.0000001201e-1f); });
+  each([&](int i) { p[i] = p[i] * r[i]; });
+  each([&](int i) { p[i] = fmaf(p[i], r[i], r[i]); });
+  each([&](int i) { p[i] = p[i] + 1.0f; });
+  each([&](int i) { e[i] = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, magic[i]) << 23) + __builtin_bit_cast(uint32_t, p[i])); });
+}
+
+// A product of a query and a key over sqrt(128), as good as the correctly rounded quotient once it is rounded to fp16: for every finite x the same half
+// (tests/cxx/kernel_arithmetic.hip), infinity and NaN as themselves.  The reciprocal of the rounded root in two parts.
+__host__ __device__ __forceinline__ float score_of(float x) { return fmaf(x, 0.0883883461f, x * 3.02540437e-9f); }
 
 // x / d from the correctly rounded reciprocal of d: quotient, remainder, correction (Markstein, "Computation of
 // elementary functions on the IBM RISC System/6000 processor", 1990).  Where the remainder is exact the result is

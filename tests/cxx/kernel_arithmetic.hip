@@ -82,6 +82,26 @@ int main() {
          }));
   printf("  (%ld smaller ones differ in fp32)\n", small.load());
 
+  // the same in two instructions, which is for halves only: every float but NaN; and the exponential whose power of two is added to its exponent
+  report("score_of, fp16", in_pieces(1ull << 32, [&](uint64_t a, uint64_t b) {
+           long n = 0;
+           for (uint64_t i = a; i < b; ++i) {
+             const float x = of_bits((uint32_t)i);
+             n += x == x && half_bits(lcu::score_of(x)) != half_bits(x / denom);
+           }
+           return n;
+         }));
+  report("exp of all x in [EXP_LEAST, 0] by its exponent", in_pieces((bits(lcu::EXP_LEAST) - 0x80000000u) / 4 + 1, [](uint64_t a, uint64_t b) {
+           long n = 0;
+           for (uint64_t i = a; i < b; ++i) {
+             float x[4], e[4];
+             for (uint32_t k = 0; k < 4; ++k) x[k] = fmaxf(of_bits(0x80000000u + 4 * (uint32_t)i + k), lcu::EXP_LEAST);
+             lcu::exp_ieee_above(e, x);
+             for (int k = 0; k < 4; ++k) n += bits(e[k]) != bits(lcu::exp_ieee_nonpositive(x[k])) || e[k] < 1e-38f;
+           }
+           return n;
+         }));
+
   // the quantiser: every pair of a normal fp16 scale and an fp16 value with a quotient of up to 300
   report("halves over fp16 scales", in_pieces(0x7c00 - 0x0400, [](uint64_t a, uint64_t b) {
            long n = 0;

@@ -965,6 +965,25 @@ def test_attention_of_scores_where_two_strips_fit(gpu, heads, n, T):
     test_attention_of_many_scores(gpu, heads, n, T)
 
 
+@pytest.mark.parametrize("heads,n", [(64, 900), (64, 560), (5, 150)])
+def test_attention_of_scores_at_both_ends_of_fp16(gpu, heads, n):
+    """Every kernel for prompts against the oracle to the bit: scores among the subnormals, and scores on both sides of 62 000, where some wavefronts take
+    the short forms and others do not."""
+    G = gpu
+    dim = heads * 128
+    q, k, v = normal((n, dim), 0, 1050, 1.0), normal((n, dim), 0, 1051, 1.0), normal((n, dim), 0, 1052, 1.0)
+    largest = lambda: np.abs(np.float64(q[:, 128:256]) @ np.float64(k[:, 128:256]).T).max(1)
+    for x in (q, k):
+        x[:, :128] *= np.float16(1e-3)
+        x[:, 128:256] *= np.float16(100)
+    q[:, 128:256] = (q[:, 128:256] * (7.3e5 / largest().max())).astype(np.float16)
+    assert (largest() < 6.9e5).any() and 7.2e5 < largest().max() < 7.4e5  # beyond 7.41e5 a score is infinite
+    out_d = G.empty((n, dim))
+    G.B.check(G.L().lcu_attention(out_d.ptr, G.dev_keep(q).ptr, G.dev_keep(k).ptr, G.dev_keep(v).ptr, n, n, 0, dim, heads, None))
+    assert G.ulp_mismatch(G.host(out_d, (n, dim))[:, :256], O.attention_prefill_kernel_order(q[:, :256], k[:, :256], v[:, :256], 2, 0)) == 0.0
+    G.release()
+
+
 @pytest.mark.parametrize("heads,n", [(64, 560), (5, 150)])
 def test_attention_of_extreme_scores(gpu, heads, n):
     """Both kernels for prompts against the oracle: equal scores, one that takes all, scores past fp16, products past fp32, NaN."""
