@@ -123,35 +123,48 @@ __global__ __launch_bounds__(256) void attention_row_kernel(T* __restrict__ out,
 // maximum and sum.  Key tiles that hold no visible key of any of the rows (between the kept tokens and the
 // windows) are not visited; the next tile is asked for while one is worked on.  Scores are computed with the keys as
 // rows, so that a lane holds sixteen of its own query row, which are the second operand of the product with the
-// transposed values as they are: keys of a block of 32 lie in LDS in the order in which lanes hold them.  Probabilities go
+// transposed values as they are.  Probabilities go
 // in as two bfloat16 terms (value and remainder), so that they keep 16 significant bits.  Workgroups of a head differ in id
 // by the number of heads: where that is a multiple of eight they share an L2, and long rows come first.
 constexpr int QT = 64, KT = 64;
 
-// where key r of a tile lies in a row of transposed values
-__device__ __forceinline__ int key_place(int r) { return (r & ~31) + ((r >> 2) & 3) * 8 + ((r >> 4) & 1) * 4 + (r & 3); }
+// four neighbouring values of four keys, turned: of sixteen lanes, lane l names 4 columns of key l / 4 and lane c gets column c of the four
+typedef short short4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ short4_t read_turned(const bf16_t* at) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)at);
+}
+// maximum over the four lanes that hold a row, sixteen apart
+__device__ __forceinline__ float row_max(float x) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, x);
+  const auto one = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const uint32_t y = __builtin_bit_cast(uint32_t, fmaxf(__builtin_bit_cast(float, (uint32_t)one[0]), __builtin_bit_cast(float, (uint32_t)one[1])));
+  const auto two = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)two[0]), __builtin_bit_cast(float, (uint32_t)two[1]));
+}
 
-// KP: 32-column pieces of a key.  With registers for keys of 256 whatever their size, one wavefront per SIMD was all that
-// fits at values of 128; two or three do now.  2048 tokens, 32 heads, values of 128: keys of 192 over all and keys of 128 in a window
-// of 1024 took 233 and 157 us, 134 and 80 now.
-// OCC: wavefronts per SIMD that the registers are cut to.  Asked for two, the compiler puts the sums among the other registers and may
-// fit another wavefront, but each takes longer for a tile: launch_tiles.
+// What bounds it is the chain of a tile (scores, maximum, exponentials, values) on the two wavefronts that a SIMD has registers for.  So fragments of keys and
+// values are asked for four products ahead (left to itself the compiler asks for one and waits for it), values lie in LDS as they come and are turned on
+// their way out (ds_read_b64_tr_b16; written turned they took sixteen 4-byte stores a thread), four maxima meet by register swaps and only when one
+// has grown, and sums go in four chains.  us, 32 heads, values of 128, before / now: keys of 192 over all, 2048 rows 132 / 94, 512 rows 29 / 20; keys of
+// 128 in a window of 1024, 2048 rows 77 / 62, 512 rows 25 / 16; with distance bias 512 rows 32 / 18, 2048 rows 136 / 76; keys and values of 64,
+// 2048 rows 56 / 42.  (Three wavefronts per SIMD spill and take 233 in place of 94.)
+// KP: 32-column pieces of a key; OCC: wavefronts per SIMD that the registers are cut to.
 template <int DV, bool BIAS, int KP, int OCC>
 __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                                                              const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, int n,
                                                              int start, window_args p) {
-  constexpr int NT = DV / 16, LDP = KT + 8, VP = (DV + 63) / 64;  // KP, VP: pieces of a tile per thread
+  constexpr int NT = DV / 16, LDV = DV + 16, VP = DV / 32;  // KP, VP: pieces of a tile per thread
   extern __shared__ __attribute__((aligned(16))) unsigned char attn_lds[];
   const int ldk = p.dk + 8;
   bf16_t* Ks = reinterpret_cast<bf16_t*>(attn_lds);   // [KT][ldk]
-  bf16_t* Vt = Ks + KT * ldk;                         // [DV][LDP]
+  bf16_t* Vs = Ks + KT * ldk;                         // [KT][LDV]: eight neighbouring rows of 32 bytes lie in all banks
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, quad = lane >> 4;
   const int h = blockIdx.x % p.heads, q0 = ((int)gridDim.x / p.heads - 1 - (int)blockIdx.x / p.heads) * QT;
   const int g = h / (p.heads / p.kv_heads), dk8 = p.dk / 8, own8 = (p.dk - p.dk_shared) / 8;
   const float r1 = BIAS ? p.r1[h] : 0.0f, r2 = BIAS ? p.r2[h] : 0.0f;
   const int first = start + q0, last = start + min(q0 + QT, n) - 1;  // positions of the tile's rows
   const int win_tile = window_begin(p, first) / KT, kept_tiles = (min(p.keep, first + QT) + KT - 1) / KT;
-  uint4_t kr[KP], vr[VP][2];
+  uint4_t kr[KP], vr[VP];
   int k_at[KP];  // row and piece of the keys
 #pragma unroll
   for (int x = 0; x < KP; ++x) {
@@ -169,13 +182,9 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
     }
 #pragma unroll
     for (int x = 0; x < VP; ++x) {
-      const int c = tid + x * 256, r = (c & 31) * 2, e = (c >> 5) * 8;
-      if (e >= DV) continue;
-#pragma unroll
-      for (int y = 0; y < 2; ++y) {
-        const size_t row = max(min(kt * KT + r + y, last) - p.base, 0);
-        vr[x][y] = *reinterpret_cast<const uint4_t*>(v + row * p.v_ld + (size_t)g * DV + e);
-      }
+      const int c = tid + x * 256, r = c / (DV / 8), e = c % (DV / 8) * 8;
+      const size_t row = max(min(kt * KT + r, last) - p.base, 0);
+      vr[x] = *reinterpret_cast<const uint4_t*>(v + row * p.v_ld + (size_t)g * DV + e);
     }
   };
   int kt = kept_tiles > 0 ? 0 : win_tile;
@@ -187,7 +196,11 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
     qf[c] = *reinterpret_cast<const bf16x8_t*>(q + (size_t)min(q0 + wave * 16 + col, n - 1) * p.ldq + (size_t)h * p.dk + c * 32 + quad * 8);
   }
   const int i = first + wave * 16 + col;             // position of this lane's row
-  float m = p.sink ? p.sink[h] : -1e30f;             // the sink counts as a key of value zero
+  // Scores and maxima count in powers of two.  A maximum is followed only when a score lies more than SLACK above it: sums and values grow by up
+  // to 2^SLACK, and nothing rounds differently for it.
+  constexpr float LOG2E = 1.44269504f, SLACK = 8.0f;
+  const float scale = p.scale * LOG2E;
+  float m = p.sink ? p.sink[h] * LOG2E : -1e30f;     // the sink counts as a key of value zero
   float l = p.sink && quad == 0 ? 1.0f : 0.0f;       // of this lane's keys
   float4_t o[NT];                                    // values t * 16 + quad * 4 .. + 3 of the row
 #pragma unroll
@@ -202,14 +215,8 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
     }
 #pragma unroll
     for (int x = 0; x < VP; ++x) {
-      const int c = tid + x * 256, at = key_place((c & 31) * 2), e = (c >> 5) * 8;
-      if (e >= DV) continue;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const uint32_t a = vr[x][0][w], b = vr[x][1][w];
-        *reinterpret_cast<uint32_t*>(Vt + (e + 2 * w) * LDP + at) = (a & 0xFFFFu) | b << 16;
-        *reinterpret_cast<uint32_t*>(Vt + (e + 2 * w + 1) * LDP + at) = a >> 16 | (b & 0xFFFF0000u);
-      }
+      const int c = tid + x * 256;
+      *reinterpret_cast<uint4_t*>(Vs + c / (DV / 8) * LDV + c % (DV / 8) * 8) = vr[x];
     }
     __syncthreads();
     ++kt;
@@ -218,21 +225,27 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
     float4_t s[4];  // element e of s[t]: key t * 16 + quad * 4 + e
 #pragma unroll
     for (int t = 0; t < 4; ++t) s[t] = (float4_t)(0.0f);
+    bf16x8_t kf[2][4];
+    const auto keys = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) kf[c & 1][t] = *reinterpret_cast<const bf16x8_t*>(Ks + (t * 16 + col) * ldk + c * 32 + quad * 8);
+    };
+    keys(0);
 #pragma unroll
     for (int c = 0; c < KP; ++c) {
       if (c * 32 >= p.dk) continue;
+      if (c + 1 < KP && (c + 1) * 32 < p.dk) keys(c + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            *reinterpret_cast<const bf16x8_t*>(Ks + (t * 16 + col) * ldk + c * 32 + quad * 8), qf[c], s[t], 0, 0, 0);
-      }
+      for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[c & 1][t], qf[c], s[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      s[t] *= p.scale;
+      s[t] *= scale;
       if constexpr (BIAS) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[t][e] -= r1 * __logf(1.0f + r2 * (float)max(i - (k0 + t * 16 + quad * 4 + e), 0));
+        for (int e = 0; e < 4; ++e) s[t][e] -= r1 * __builtin_amdgcn_logf(1.0f + r2 * (float)max(i - (k0 + t * 16 + quad * 4 + e), 0));
       }
     }
     const int lowest = first + wave * 16;  // of the wavefront's positions
@@ -246,34 +259,56 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
         }
       }
     }
-    float top = m;
+    float top = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 4; ++t) top = fmaxf(top, fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])));
-    top = fmaxf(top, __shfl_xor(top, 16, WAVE));
-    top = fmaxf(top, __shfl_xor(top, 32, WAVE));
-    if (__ballot(top != m) != 0) {
-      const float shrink = __expf(m - top);
+    if (__ballot(top > m + SLACK) != 0) {
+      top = fmaxf(m, row_max(top));
+      const float shrink = __builtin_amdgcn_exp2f(m - top);
       m = top;
       l *= shrink;
 #pragma unroll
       for (int t = 0; t < NT; ++t) o[t] *= shrink;
     }
+    float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8_t hi[KT / 32], rem[KT / 32];
 #pragma unroll
     for (int c = 0; c < KT / 32; ++c) {
-      bf16x8_t hi, rem;
+      float pr[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float pr = __expf(s[c * 2 + e / 4][e % 4] - m);
-        l += pr;
-        hi[e] = (bf16_t)pr;
-        rem[e] = (bf16_t)(pr - (float)hi[e]);
-      }
+      for (int e = 0; e < 8; ++e) pr[e] = __builtin_amdgcn_exp2f(s[c * 2 + e / 4][e % 4] - m);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(Vt + (t * 16 + col) * LDP + c * 32 + quad * 8);
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, rem, o[t], 0, 0, 0);
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, hi, o[t], 0, 0, 0);
+      for (int e = 0; e < 8; ++e) part[e & 3] += pr[e];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) hi[c][e] = (bf16_t)pr[e];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) rem[c][e] = (bf16_t)(pr[e] - (float)hi[c][e]);
+    }
+    l += (part[0] + part[1]) + (part[2] + part[3]);
+    union {
+      short4_t half[2];
+      bf16x8_t all;
+    } vf[2][2];
+    const bf16_t* v_at = Vs + (quad * 4 + (col >> 2)) * LDV + (col & 3) * 4;
+    const auto values = [&](int step) __attribute__((always_inline)) {  // two of the KT / 32 * NT fragments
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        const int c = (2 * step + y) / NT, t = (2 * step + y) % NT;
+        vf[step & 1][y].half[0] = read_turned(v_at + c * 32 * LDV + t * 16);
+        vf[step & 1][y].half[1] = read_turned(v_at + (c * 32 + 16) * LDV + t * 16);
       }
+    };
+    values(0);
+#pragma unroll
+    for (int step = 0; step < KT / 32 * NT / 2; ++step) {
+      if (step + 1 < KT / 32 * NT / 2) values(step + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const int c = (2 * step + (y & 1)) / NT, t = (2 * step + (y & 1)) % NT;
+        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[step & 1][y & 1].all, y < 2 ? rem[c] : hi[c], o[t], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   l += __shfl_xor(l, 16, WAVE);
@@ -295,7 +330,7 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
   }
 }
 
-size_t tile_lds(int dk, int dv) { return ((size_t)KT * (dk + 8) + (size_t)dv * (KT + 8)) * 2; }
+size_t tile_lds(int dk, int dv) { return (size_t)KT * (dk + 8 + dv + 16) * 2; }
 
 template <int DV, bool BIAS, int KP, int OCC>
 int launch_tiles_of(void* out, const void* q, const void* k, const void* v, int n, int start, const window_args& p, hipStream_t st) {
@@ -315,23 +350,11 @@ int launch_tiles_of(void* out, const void* q, const void* k, const void* v, int 
   return LCU_OK;
 }
 
-// us, registers cut to two wavefronts / to one, where more fit all the same.  Keys of 192 are done sooner with one at every size (32 heads,
-// values of 128, 100 rows behind 1500 109 / 90, 2048 rows 150 / 134; values of 64 92 / 73).  Keys of 128 with values of 128 fit three
-// wavefronts in place of two when cut, which pays where the grid has more than that for every SIMD (32 heads, 2048 rows in a window of
-// 1024 80 / 106, 3000 rows 196 / 245) and costs where it has not (32 heads, 100 rows behind 3000 185 / 151; 64 heads, 500 behind 1000
-// 89 / 78; 16 heads, 3000 rows 166 / 143).  With values of 64 keys of 64 gain by the cut (512 rows 16.6 / 17.4), keys of 128 lose (32
-// heads, 100 rows behind 3000 144 / 119).
+// Registers for two wavefronts per SIMD, where they do without memory: left to itself the compiler takes more, and one is all that fits.
 template <int DV, bool BIAS>
 int launch_tiles(void* out, const void* q, const void* k, const void* v, int n, int start, const window_args& p, hipStream_t st) {
-  if (p.dk <= 128) {
-    if constexpr (DV <= 128) {
-      device_state* ds = current_device_state();
-      const long cus = ds && ds->compute_units > 0 ? ds->compute_units : 256;
-      if (DV == 128 ? (long)((n + QT - 1) / QT) * p.heads > 3 * cus : p.dk <= 64) return launch_tiles_of<DV, BIAS, 4, 2>(out, q, k, v, n, start, p, st);
-    }
-    return launch_tiles_of<DV, BIAS, 4, 1>(out, q, k, v, n, start, p, st);
-  }
-  if (p.dk <= 192) return launch_tiles_of<DV, BIAS, 6, 1>(out, q, k, v, n, start, p, st);
+  if (p.dk <= 128) return launch_tiles_of<DV, BIAS, 4, 2>(out, q, k, v, n, start, p, st);
+  if (p.dk <= 192) return launch_tiles_of<DV, BIAS, 6, DV <= 128 ? 2 : 1>(out, q, k, v, n, start, p, st);
   return launch_tiles_of<DV, BIAS, 8, 1>(out, q, k, v, n, start, p, st);
 }
 

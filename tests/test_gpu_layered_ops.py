@@ -407,6 +407,20 @@ def test_windowed_attention_key_sizes(gpu, dim, vdim):
     gpu.release()
 
 
+# a maximum that grows from tile to tile by less than the kernel follows (2^8 in all but a few rows), by about as much, by far more, and one that falls
+@pytest.mark.parametrize("growth", [0.01, 0.08, 0.6, -0.3])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (192, 128)])
+def test_windowed_attention_of_growing_scores(gpu, dim, vdim, growth):
+    heads, kv, T, window, keep = 3, 3, 330, 400, 0
+    c = attention_case(gpu, BF16, heads, kv, dim, vdim, window, keep, T, dim)
+    c["q"][..., 0] = 8.0
+    c["k"][..., 0] = rounded(growth * np.arange(T) * dim ** 0.5 / 8.0 / 1.3)[:, None]  # a score grows by `growth` from key to key
+    r1, r2 = (gpu.B.from_device(b, (heads,), np.float32).astype(float) for b in last_two_vectors(gpu))
+    want = S.windowed_attention(c["q"][..., :dim], c["k"][..., :dim], c["v"][..., :vdim], c["wp"].scale, r1, r2, window, keep)
+    close(run_attention(gpu, c, BF16, (T,)), want, BF16, bf16=2.0 ** -7)
+    gpu.release()
+
+
 # 768 workgroups and more: the form that fits three to a compute unit
 @pytest.mark.parametrize("heads,T", [(128, 384), (112, 390), (112, 449)])
 def test_windowed_attention_many_workgroups(gpu, heads, T):
