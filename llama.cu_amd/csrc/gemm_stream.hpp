@@ -11,6 +11,10 @@
 // M = 8 with a launch that adds the splits, fp16 three times (4096, 4096) 26.0 -> 22.7 us, twice (N, K) = (11008, 4096) 45 -> 42,
 // (4096, 4096) 12.1 -> 12.4; uint8 three times (6656, 6656) 61 -> 35, twice (17920, 6656) 104 -> 57, (6656, 17920) 62 -> 37.  Rows of
 // 8 KB meet in the same memory channels: K = 4224 takes a tenth less than 4096.
+// W is read once and marked so (nt): 8 rows, twice 11008 columns of K 4096 36.8 -> 33.7 us (4.9 -> 5.35
+// TB/s), 16x4096x11008 22.4 -> 20.9, 60x6656x17920 53.6 -> 50.0; eight sequences of eight 7B layers, 45 + 16 tokens 23.4 -> 22.1 ms.  uint8 gains up to
+// 1.5 %.  Weights that the 256 MB cache holds from call to call lose what they gained there (60x6656x17920 again and again 45 -> 47.8 us), but a
+// model's do not come back before the cache has seen all of them.
 #pragma once
 #include <algorithm>
 
@@ -129,7 +133,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
     const uint32_t slot = ring0 + (u % RING) * UNIT, along = stage_offset(rw[2], (uint32_t)(base * (U8 ? 64 : 128) + u * 128));
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(w_off[j]), "s"(rw), "s"(along),
+      asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(w_off[j]), "s"(rw), "s"(along),
                    "s"(slot + j * 1024)
                    : "memory", "m0");
     }
