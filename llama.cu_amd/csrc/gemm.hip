@@ -1257,18 +1257,22 @@ int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block
   return rc;
 }
 
-// tiles of 256x128 (128x128 up to 128 rows or where `small`), sums of every split to part
+// Sums of every split to part, in tiles of 256x128 (128x128 up to 128 rows or where `small`), or of fewer where these leave compute units idle
+// (plan_tile_size).  us, those / so: fp16 66x11008x4096 33.5 / 27.2, 128 rows 38.8 / 32.8, 66x6656x6656 35.7 / 29.4, 200x5632x2048 42.1 / 19.1; uint8
+// 36.6 / 27.5, 41.9 / 34.2, 40.9 / 28.2, 49.0 / 21.7.
 template <bool U8>
-int launch_partial(operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, bool small, int step) {
-  if (small || M <= 128) {
-    return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, 4, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
-  }
-  return launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, 3, U8, true>(f16_epilogue{}, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+int launch_partial(operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, bool small, int step, long cus) {
+  const tile_size_t tile = plan_tile_size(M, N, splits * op.n_mats, small || M <= 128 ? tile_size_t{128, 128} : tile_size_t{256, 128}, false, cus);
+  const f16_epilogue ep{};
+  if (tile.rows == 64) return launch_tile<64, 64, 1, 4, 4, 4, U8, true>(ep, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+  if (tile.columns == 64) return launch_tile<128, 64, U8 ? 1 : 2, U8 ? 4 : 2, 4, 4, U8, true>(ep, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+  if (tile.rows == 128) return launch_tile<128, 128, U8 ? 1 : 2, U8 ? 4 : 2, 4, 4, U8, true>(ep, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
+  return launch_tile<256, 128, U8 ? 1 : 4, U8 ? 4 : 2, 3, 3, U8, true>(ep, op, A, M, K, N, block, 0.0f, st, splits, part, {}, step);
 }
 
 template <bool U8>
-int launch_large_split(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits, float* part) {
-  const int rc = launch_partial<U8>(op, A, M, K, N, block, st, splits, part, false, 1);
+int launch_large_split(operands_t op, const half_t* A, int M, int K, int N, int block, float beta, hipStream_t st, int splits, float* part, long cus) {
+  const int rc = launch_partial<U8>(op, A, M, K, N, block, st, splits, part, false, 1, cus);
   if (rc != LCU_OK) return rc;
   const size_t mn = (size_t)M * N;
   splitk_reduce_kernel<<<dim3((unsigned)((mn + 1023) / 1024), op.n_mats), 256, 0, st>>>(op.out, op.more.out[0], op.more.out[1], part, mn,
@@ -1304,9 +1308,10 @@ int many_rows_partial(operands_t op, const half_t* A, int M, int K, int N, int b
       (size_t)M * K * 2 >= (size_t)1 << 32 || (size_t)N * K * (U8 ? 1 : 2) >= (size_t)1 << 32) {
     return LCU_OK;
   }
-  const left_sums_t left = plan_left_sums(U8, M, K, N, ds->compute_units > 0 ? ds->compute_units : 256, ws.bytes, ws.owned);
+  const long cus = ds->compute_units > 0 ? ds->compute_units : 256;
+  const left_sums_t left = plan_left_sums(U8, M, K, N, cus, ws.bytes, ws.owned);
   if (left.splits == 0) return LCU_OK;
-  const int rc = launch_partial<U8>(op, A, M, K, N, block, st, left.splits, (float*)ws.ptr, left.step == 2, left.step);
+  const int rc = launch_partial<U8>(op, A, M, K, N, block, st, left.splits, (float*)ws.ptr, left.step == 2, left.step, cus);
   res->part = (float*)ws.ptr;
   res->splits = left.splits;
   *done = rc == LCU_OK;
@@ -1641,7 +1646,7 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
       if constexpr (U8) {
         if (block_shift(block) < 0) return launch_split<256, 128, 4, 2, U8>(op, A, M, K, N, block, beta, st, plan.splits, (float*)ws.ptr);
       }
-      return launch_large_split<U8>(op, A, M, K, N, block, beta, st, plan.splits, (float*)ws.ptr);
+      return launch_large_split<U8>(op, A, M, K, N, block, beta, st, plan.splits, (float*)ws.ptr, cus);
     }
     // Tiles of 128x128, the ring of four stages filled by address-free requests: us here against a two-stage ring with two
     // workgroups per compute unit (from 256 tiles up) or eight wavefronts and three stages (below), M x K x N: 256 tiles
@@ -1697,11 +1702,17 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
       // 1000x2048x2048 17.2 / 15.7; 512 rows of 4096 columns, K 256, 512, 1024, 2048 6.3 / 5.2, 7.2 / 6.1, 10.9 / 9.7, 15.4 / 15.0, but K 4096 28.9 / 29.3:
       // 24 KB a stage on their way into LDS bound it over a long K, and the rest is what it gains.  70 drawn products 0.91 of the time (0.82 to
       // 1.03), 45 in uint8 0.84 (0.79 to 0.88).
+      // Smaller ones where these would leave compute units idle: 90 rows of 2048 columns eight fp16 layers 0.90 -> 0.71 ms.
+      const tile_size_t tile = plan_tile_size(M, N, op.n_mats, {128, 64}, !U8, cus);
+      const f16_epilogue ep{};
       if constexpr (U8) {
-        if (block_shift(block) >= 0) return launch_tile<128, 64, 1, 4, 4, 4, true, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, block, beta, st);
-        return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);
+        if (block_shift(block) < 0) return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);
+        if (tile.rows == 64) return launch_tile<64, 64, 1, 4, 4, 4, true, false, f16_epilogue, 2>(ep, op, A, M, K, N, block, beta, st);
+        return launch_tile<128, 64, 1, 4, 4, 4, true, false, f16_epilogue, 2>(ep, op, A, M, K, N, block, beta, st);
       } else {
-        return launch_tile<128, 64, 2, 2, 4, 4, false, false, f16_epilogue, 2>(f16_epilogue{}, op, A, M, K, N, 0, beta, st);
+        if (tile.columns == 32) return launch_tile<64, 32, 1, 2, 4, 4, false, false, f16_epilogue, 2>(ep, op, A, M, K, N, 0, beta, st);
+        if (tile.rows == 64) return launch_tile<64, 64, 1, 4, 4, 4, false, false, f16_epilogue, 2>(ep, op, A, M, K, N, 0, beta, st);
+        return launch_tile<128, 64, 2, 2, 4, 4, false, false, f16_epilogue, 2>(ep, op, A, M, K, N, 0, beta, st);
       }
     }
   }
@@ -1850,6 +1861,8 @@ template <bool GATED>
 int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void* W, int M, int K, int N, hipStream_t st) {
   const auto tm = [&](int bm) { return (M + bm - 1) / bm; };
   const auto tn = [&](int bn) { return (long)((N + bn - 1) / bn); };
+  const device_state* ds = current_device_state();
+  const long cus = ds && ds->compute_units > 0 ? ds->compute_units : 256;
   if (M <= 64) {
     bool done = false;
     const int rc = bf16_skinny<GATED>(ep, A, W, M, K, N, st, &done);
@@ -1869,7 +1882,10 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     if (K % 128 == 0 && tm(128) * tn(64) > 128) {
       return launch_tile<128, 64, 2, 2, 4, 4, false, false, linear_epilogue<false, GATED>, 2>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
     }
-    return launch_bf16<64, 64, 2, 2, 1, 3>(ep, A, W, tm(64), M, K, N, st);
+    // us, on gemm_dl_kernel / here: 100x2048x2048 16.3 / 11.0, 200x4096x4096 29.4 / 20.9, 66x4096x8192 30.5 / 24.2
+    const operands_t op = single_matrix(nullptr, W, nullptr);
+    if (plan_tile_size(M, N, 1, {64, 64}, true, cus).columns == 32) return launch_tile<64, 32, 1, 2, 4, 4, false, false>(ep, op, A, M, K, N, 0, 0.0f, st);
+    return launch_tile<64, 64, 1, 4, 4, 4, false, false>(ep, op, A, M, K, N, 0, 0.0f, st);
   }
 }
 template int gemm_bf16<false>(linear_epilogue<false, false> const&, const void*, const void*, int, int, int, hipStream_t);

@@ -49,6 +49,25 @@ inline row_plan_t plan_rows(int M, int K, int N, int n_mats, long cus, size_t wo
   return {tiles_of(M, N, 128, 64) * n_mats > 256 ? row_tiles::narrow : row_tiles::halves, 1};
 }
 
+// Rows and columns of the tiles of a product that a round of 128x64 ones (row_tiles::halves) or a few large ones with K dealt to `splits`
+// workgroups each leave compute units idle with: the smallest that still come out as one round.  What bounds these is the bytes
+// that a compute unit brings into LDS for a stage, lhs and columns, 24 KB with 128x64, 16 KB with 64x64, 12 KB with 64x32 (`narrowest`; codes would be
+// converted once more: 200 rows of width 2048, eight uint8 layers 0.87 ms with 64x64, 0.90 so); with two to a compute unit they meet there again
+// (us with weights from memory, 128x64 / 64x64 / 64x32, workgroups in brackets: fp16 90x4096x4096 25.8 (64) / 20.0 (128) / 18.8 (256), 200 rows 27.7 (128) / 20.5 (256) /
+// 26.0 (512), 300 rows 28.3 (192) / 31.5 (320); uint8 200 rows 32.5 / 22.5, 300 rows 33.7 / 37.1).  The sums are those of larger tiles.
+// each: matrices times splits.
+struct tile_size_t {
+  int rows, columns;
+};
+inline tile_size_t plan_tile_size(int M, int N, int each, tile_size_t largest, bool narrowest, long cus) {
+  constexpr tile_size_t sizes[] = {{64, 32}, {64, 64}, {128, 64}, {128, 128}, {256, 128}};
+  for (tile_size_t t : sizes) {
+    if (t.columns == 32 && !narrowest) continue;
+    if ((t.rows == largest.rows && t.columns == largest.columns) || tiles_of(M, N, t.rows, t.columns) * each <= cus) return t;
+  }
+  return largest;
+}
+
 // Which columns of a product a launch of gemm_tile_kernel takes: the first `tiles` tiles along N, counted through the matrices
 // (0: all of them), or those from column `from` of the last matrix on.
 struct columns_t {
@@ -137,7 +156,8 @@ inline large_tiles_t plan_large(product_type type, int M, int K, int N, int n_ma
 // 20.2 / 22.0, 1290x768x512 14.9 / 16.3; of 7270 drawn products that these lines take 6 are more than 3 % slower so, on average they take 0.8 of
 // the time).  That was against separate products on gemm_dl_kernel.  On the 128x64 tiles of gemm_tile_kernel, which they take now, they are ahead of some
 // that these lines take (fp16 80x4096x4096 27.6 / 24.9, 256 rows 31.1 / 29.5, 400 rows 26.9 / 27.7, 512 rows 32.0 / 32.7, 200x2048x2048 16.2 / 16.6;
-// uint8 300x1152x1030 19.3 / 16.4, 512x4096x4096 34.3 / 35.4, 700x2048x2048 19.7 / 22.2).
+// uint8 300x1152x1030 19.3 / 16.4, 512x4096x4096 34.3 / 35.4, 700x2048x2048 19.7 / 22.2).  Where the tiles of either are smaller now (plan_tile_size) both
+// are sooner than these figures.
 struct left_sums_t {
   int splits, step;
 };

@@ -114,7 +114,7 @@ struct tile_shape {
 
 // CHAINS 2: the even and the odd stages of K are summed apart, and the two sums added (K a multiple of 128).
 template <int BM, int BN, int WM, int WN, int NA, int NB, bool U8, bool SPLIT, class EP, int CHAINS = 1>
-__global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_tile_kernel(
+__global__ __launch_bounds__(64 * WM * WN, (WM * WN + 3) / 4) void gemm_tile_kernel(
     half_t* __restrict__ out0, const half_t* __restrict__ A, const void* __restrict__ W0, const half_t* __restrict__ S0, int block_shift,
     int M, int K, int N, float beta, int tiles_m, int tiles_n, int from, float* __restrict__ part, int splits, int step, more_matrices_t more, EP ep) {
   using shape = tile_shape<BM, BN, WM, WN, NA, NB, U8, SPLIT, EP>;

@@ -30,6 +30,13 @@ void left_sums(int u8, int M, int K, int N, long cus, long workspace, int owned,
   out[1] = p.step;
 }
 
+// rows, columns
+void tile_size(int M, int N, int each, int largest_rows, int largest_columns, int narrowest, long cus, int* out) {
+  const tile_size_t t = plan_tile_size(M, N, each, {largest_rows, largest_columns}, narrowest != 0, cus);
+  out[0] = t.rows;
+  out[1] = t.columns;
+}
+
 int expert_rows(long rows, int experts, int K, int ff, long cus) { return plan_expert_rows(rows, experts, K, ff, cus); }
 
 int attention_again(int n_heads, int n_new, int start_pos, long cus) { return scores_again(n_heads, n_new, start_pos, cus); }

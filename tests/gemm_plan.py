@@ -21,10 +21,11 @@ def _lib():
     i, w = C.c_int, C.c_long
     lib.rows.argtypes = [i, i, i, i, w, w, C.POINTER(i)]
     lib.left_sums.argtypes = [i, i, i, i, w, w, i, C.POINTER(i)]
+    lib.tile_size.argtypes = [i, i, i, i, i, i, w, C.POINTER(i)]
     lib.large.argtypes = [i, i, i, i, i, w, i, C.POINTER(i)]
     lib.attention_again.argtypes = [i, i, i, w]
     lib.expert_rows.argtypes = [w, i, i, i, w]
-    lib.rows.restype = lib.left_sums.restype = lib.large.restype = None
+    lib.rows.restype = lib.left_sums.restype = lib.large.restype = lib.tile_size.restype = None
     os.unlink(path)
     os.rmdir(folder)
     return lib
@@ -49,6 +50,13 @@ def left_sums(M, K, N, u8=False, owned=True, cus=CUS, workspace=WORKSPACE):
     out = (C.c_int * 2)()
     _lib().left_sums(int(u8), M, K, N, cus, workspace, int(owned), out)
     return out[0], out[1]
+
+
+def tile_size(M, N, each, largest, narrowest, cus=CUS):
+    """(rows, columns) of the tiles of products that leave compute units idle"""
+    out = (C.c_int * 2)()
+    _lib().tile_size(M, N, each, *largest, int(narrowest), cus, out)
+    return tuple(out)
 
 
 def scores_again(heads, n, T, cus=CUS):

@@ -148,6 +148,13 @@ def test_linear_columns_left_of_whole_rounds(gpu, M, K, N, plan):
     test_linear_large_tiles(gpu, M, K, N)
 
 
+# tiles below 128x64, either side of where a round of the narrowest ends
+@pytest.mark.parametrize("M,K,N,tile", [(66, 64, 4096, (64, 32)), (300, 192, 1590, (64, 32)), (300, 128, 1640, (64, 64)), (129, 320, 4094, (64, 64))])
+def test_linear_smaller_tiles(gpu, M, K, N, tile):
+    assert gemm_plan.tile_size(M, N, 1, (64, 64), True) == tile and gemm_plan.rows(M, 128, N)[0] == "halves"
+    test_linear_large_tiles(gpu, M, K, N)
+
+
 @pytest.mark.parametrize("M,K,ff,plan", [(1030, 1024, 6560, (192, 51, 9792, 128, 128)), (1025, 1024, 6750, (192, 51, 9792, 256, 128)),
                                          (1282, 2048, 6752, (256, 42, 10752, 128, 128)), (1990, 1024, 10980, (256, 64, 16384, 256, 192))])
 def test_gated_linear_columns_left_of_whole_rounds(gpu, M, K, ff, plan):

@@ -579,6 +579,29 @@ def test_streams_own_their_workspace(gpu):
         assert results[t] is not None and (results[t].view(np.uint16) == cases[t][2].view(np.uint16)).all()
 
 
+# tiles below 128x64 and below those that K is dealt for, either side of where a round of them ends; ragged rows and columns, rows off 16 bytes
+@pytest.mark.parametrize("M,K,N,splits,tile", [(66, 256, 1001, 0, (64, 32)), (65, 384, 4096, 0, (64, 32)), (67, 128, 4100, 0, (64, 64)),
+                                               (130, 384, 5440, 0, (64, 64)), (130, 256, 5472, 0, (128, 64)), (193, 128, 2052, 0, (64, 64)),
+                                               (66, 5120, 2056, 2, (64, 64)), (66, 5120, 4169, 2, (128, 64)), (130, 5120, 1100, 2, (64, 64)),
+                                               (257, 5120, 2700, 2, (128, 128))])
+@pytest.mark.parametrize("u8", [False, True])
+def test_gemm_smaller_tiles_of_one_round(gpu, u8, M, K, N, splits, tile):
+    import gemm_plan
+    G = gpu
+    assert gemm_plan.rows(M, K, N) == (("split_large", splits) if splits else ("halves", 1))
+    largest = (128, 64) if not splits else (128, 128) if M <= 128 else (256, 128)
+    narrowest = not splits and not u8
+    assert gemm_plan.tile_size(M, N, max(splits, 1), largest, narrowest) == ((64, 64) if tile == (64, 32) and u8 else tile)
+    x, w, old = normal((M, K), 0, 450, 1.0), normal((N, K), 0, 451, 0.02), normal((M, N), 0, 452, 1.0)
+    if u8:
+        codes, scales = O.quantize_absmax_u8(w, 128)
+        assert G.ulp_mismatch(G.gemm_u8(x, codes, scales, 128), O.matmul_nt_u8(x, codes, scales, 128, flavour=2)) == 0.0
+    else:
+        assert G.ulp_mismatch(G.gemm_f16(x, w), O.matmul_nt(x, w, flavour=2)) == 0.0
+        assert G.ulp_mismatch(G.gemm_f16(x, w, beta=1.0, out=old), O.matmul_nt(x, w, beta=1.0, out=old, flavour=2)) == 0.0
+    G.release()
+
+
 def test_gemm_rejects_bad_shapes(gpu):
     G = gpu
     a = G.dev(np.zeros((4, 12), dtype=np.float16))
