@@ -156,42 +156,56 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
     lhs_row[i] = (uint32_t)row * row_bytes;
     lhs_turn[i] = row & 15;
   }
-  // stage s, whose columns lie in `slot` (U8: in its first or second half)
-  const auto multiply = [&](const unsigned char* slot, int s) {
-    half8_t w[2];
+  // Stage s of chunk c, whose columns lie in `slot` (U8: in its first or second half).  Every fragment is asked for before the first product: left to
+  // itself the compiler reads one, waits for it and multiplies it, eight times with 64 rows, and there are one or two wavefronts to a SIMD (us, so / here:
+  // uint8 60x6656x17920 83.5 / 72.5, 40 rows 74.6 / 65.3, 20x6656x17920 37.6 / 35.1, 14x4096x11008 19.1 / 17.8; fp16 60x6656x17920 50.2 / 49.2).
+  const auto multiply = [&](const unsigned char* slot, int s, int c) {
+    half8_t w[2], a[2][TM];
+    uint2_t codes[2];
+    uint32_t word = 0;
     const unsigned char* row = slot + col * 128;
     if constexpr (U8) {
-      const uint32_t at = s_first + ((uint32_t)(base + s) >> block_shift);
-      const uint32_t word = *reinterpret_cast<const uint32_t*>(slot + 2048 + lane * 4);
-      const half_t s2 = __builtin_bit_cast(half_t, (uint16_t)((at & 1) ? word >> 16 : word)) * (half_t)2.0f;
-      const half2_t s2v = {s2, s2};
+      word = *reinterpret_cast<const uint32_t*>(slot + 2048 + lane * 4);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int byte = (s & 1) * 64 + h * 32 + group * 8;
-        const uint2_t q = *reinterpret_cast<const uint2_t*>(row + (((byte >> 4) ^ turn) << 4) + (byte & 8));
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const half2_t lo = dequant2(__builtin_amdgcn_perm(0u, q[i], 0x0c010c00u), s2v);
-          const half2_t hi = dequant2(__builtin_amdgcn_perm(0u, q[i], 0x0c030c02u), s2v);
-          w[h][4 * i] = lo.x, w[h][4 * i + 1] = lo.y, w[h][4 * i + 2] = hi.x, w[h][4 * i + 3] = hi.y;
-        }
+        codes[h] = *reinterpret_cast<const uint2_t*>(row + (((byte >> 4) ^ turn) << 4) + (byte & 8));
       }
     } else {
 #pragma unroll
       for (int h = 0; h < 2; ++h) w[h] = *reinterpret_cast<const half8_t*>(row + (((4 * h + group) ^ turn) << 4));
     }
-    const int chunk = JOINED ? 0 : s * 64 / kc, p0 = JOINED ? (base + s) * 8 : (s * 64 - chunk * kc) / 8;
-    const unsigned char* lhs = stream_mem + (chunk & 1) * chunk_bytes;
+    const int p0 = JOINED ? (base + s) * 8 : (s * 64 - c * kc) / 8;
+    const unsigned char* lhs = stream_mem + (JOINED ? 0 : (c & 1) * chunk_bytes);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int p = p0 + 4 * h + group;
 #pragma unroll
+      for (int i = 0; i < TM; ++i) a[h][i] = *reinterpret_cast<const half8_t*>(lhs + lhs_row[i] + ((p & ~15) | ((p ^ lhs_turn[i]) & 15)) * 16);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (U8) {
+      const uint32_t at = s_first + ((uint32_t)(base + s) >> block_shift);
+      const half_t s2 = __builtin_bit_cast(half_t, (uint16_t)((at & 1) ? word >> 16 : word)) * (half_t)2.0f;
+      const half2_t s2v = {s2, s2};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const half2_t lo = dequant2(__builtin_amdgcn_perm(0u, codes[h][i], 0x0c010c00u), s2v);
+          const half2_t hi = dequant2(__builtin_amdgcn_perm(0u, codes[h][i], 0x0c030c02u), s2v);
+          w[h][4 * i] = lo.x, w[h][4 * i + 1] = lo.y, w[h][4 * i + 2] = hi.x, w[h][4 * i + 3] = hi.y;
+        }
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
       for (int i = 0; i < TM; ++i) {
-        const half8_t a = *reinterpret_cast<const half8_t*>(lhs + lhs_row[i] + ((p & ~15) | ((p ^ lhs_turn[i]) & 15)) * 16);
         if constexpr (BF16) {
-          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, w[h]), acc[i], 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[h][i]), __builtin_bit_cast(bf16x8_t, w[h]), acc[i], 0, 0, 0);
         } else {
-          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, w[h], acc[i], 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[h][i], w[h], acc[i], 0, 0, 0);
         }
       }
     }
@@ -229,7 +243,7 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
 #pragma unroll
       for (int e = 0; e < PER; ++e) {
         const int s = u * PER + e;
-        if (PER == 1 || (s >= first && s < end)) multiply(slot, s);
+        if (PER == 1 || (s >= first && s < end)) multiply(slot, s, c);
       }
     }
   }
