@@ -1065,23 +1065,23 @@ inline stream_join_t plan_stream_join(int M, int K, int N, int n_mats, int joine
 }
 
 // Whether a product of few rows is one of gemm_stream_kernel, or of BM x 128 tiles of four wavefronts.  Of those several share a
-// compute unit; a workgroup here has it alone, so that a second round fills lhs and ring again with nothing beside it.  us, tiles /
-// here, 8 and 32 rows: fp16 2048x32000 (two rounds) 27.7 / 33.9, 30.7 / 37.6, 4096x32000 56.0 / 56.4, 58.5 / 58.6, 5888x9664 three
-// times (three) 62 / 67, 67 / 77; one round 4096x11008 twice 43.8 / 41.9, 46.5 / 42.9 (45 rows).  uint8 gains more in a round: 4096x11008
-// twice (two) 36.6 / 32.7 with 16 rows, 37.6 / 40.4 with 32, 4096x32000 37.2 / 32.9, 39.8 / 42.8, 5888x9664 three times 56 / 61, 56 / 81;
-// over short runs it does not (15x512x10304 twice 10.3 / 11.4).
-// One round: fp16 gains where the tiles (`tiles` in all, with their splits) do not come out even, or up to 16 rows over runs of 8 stages and
-// more; else it is done no sooner with weights from memory and later with weights from a cache (tiles / here, memory and cache:
-// 10x1024x7304 8.6 / 9.2, 7.4 / 8.3; 24x4096x4096 12.4 / 12.7, 11.0 / 11.7; but 13x2048x2048 three times 12.0 / 11.6, 9.1 / 10.0, 27x17920x6656
-// 62 / 47).  bfloat16 gains at every count (4x512x3264 9.2 / 7.9, 46x17920x6656 68 / 50).  Neither does for more than 16 rows over the
-// shortest runs (28x512x16840 10.5 / 11.1, bfloat16 56x512x16576 13.8 / 14.8).
+// compute unit; a workgroup here has it alone, so that a second round fills lhs and ring again with nothing beside it, which a long enough run
+// of stages pays for.  us with weights from memory, tiles / here: two rounds, fp16 8 rows of 32000 columns, K 2048, 2560, 4096, 6656 29.4 / 32.7, 33.6 / 31.0,
+// 62.2 / 54.7, 79.1 / 71.0, 24 rows 30.8 / 35.4, 43.2 / 41.0 (K 3072), 66.9 / 60.9, 64 rows of K 4096 71.9 / 68.0; uint8 32 rows, K 4096, 6656
+// 46.3 / 44.0, 70.1 / 61.9, 48 rows 76.3 / 76.2, 16 rows of 4096x11008 twice 36.6 / 32.7; three rounds, 5888x9664 three times 62 / 67.
+// One round: uint8 gains, but over short runs (15x512x10304 twice 10.3 / 11.4); fp16 where the tiles (`tiles` in all, with their splits) do not come out
+// even (27x17920x6656 62 / 45), or over runs of some stages (10x1024x7304 8.6 / 9.2; 24x4096x4096 13.3 / 13.3, 24x6144x4096 16.4 / 15.7, 20x11008x4096
+// 23.6 / 22.2, 20x8192x8192 36.5 / 33.0; 50 rows 18.3 / 18.3, 8192x4096 20.9 / 21.2, 8192x8192 64 rows 39.5 / 35.1).  bfloat16 gains at every count (4x512x3264
+// 9.2 / 7.9, 46x17920x6656 68 / 50).  Neither does for more than 16 rows over the shortest runs (28x512x16840 10.5 / 11.1, bfloat16
+// 56x512x16576 13.8 / 14.8).  A product called again and again, its weights in the caches, is sooner in tiles (64x8192x8192 26.7 / 34.3); a model's are not.
 inline bool streams(int M, int N, int n_mats, int splits, int stages, long tiles, long cus, bool u8, bool bf16) {
   long rounds = 1;
   stream_waves(N, n_mats, splits, cus, stream_max_waves(u8), &rounds);
   const int run = stages / splits;
-  if (u8) return rounds == 1 || (M <= 16 && rounds == 2 && run >= 12);
+  if (u8) return rounds == 1 || (rounds == 2 && M <= 32 && run >= (M <= 16 ? 12 : 20));
   const bool short_runs = M > 16 && run <= 4;
-  return rounds == 1 && (bf16 ? !short_runs || 4 * tiles <= 3 * cus : (tiles > cus && !short_runs) || (M <= 16 && run >= 8));
+  if (bf16) return rounds == 1 && (!short_runs || 4 * tiles <= 3 * cus);
+  return rounds == 1 ? (tiles > cus && !short_runs) || run >= (M <= 16 ? 8 : M <= 32 ? 12 : 24) : rounds == 2 && run >= 20;
 }
 
 template <int TM, bool U8, bool BF16>
@@ -1875,6 +1875,8 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
   }
   if (tm(128) * tn(128) >= 160) return launch_tile<128, 128, 2, 2, 4, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
   if constexpr (GATED) {
+    // us, below / here: 100 rows of 11264 columns, K 1536, 1792, 2048 17.6 / 17.7, 19.4 / 18.6, 20.9 / 19.3, 100x4096x5632 32.7 / 29.4, 100x2048x2816 18.5 / 17.4
+    if (K >= 1792) return launch_tile<128, 64, 2, 1, 4, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
     if (tm(128) * tn(64) > 128) return launch_bf16<128, 64, 4, 1, 1, 3>(ep, A, W, tm(128), M, K, N, st);
     return launch_bf16<64, 64, 2, 1, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   } else {

@@ -162,6 +162,12 @@ def test_gated_linear_columns_left_of_whole_rounds(gpu, M, K, ff, plan):
     test_gated_linear_large_tiles(gpu, M, K, ff)
 
 
+# gated outputs of few 128x64 tiles, either side of K = 1792
+@pytest.mark.parametrize("M,K,ff", [(66, 1728, 1500), (66, 1792, 1500), (129, 1856, 2000), (200, 2048, 70)])
+def test_gated_linear_few_tiles(gpu, M, K, ff):
+    test_gated_linear_large_tiles(gpu, M, K, ff)
+
+
 # gated outputs of 192 columns: one round of them, ragged ends, a short K
 @pytest.mark.parametrize("M,K,ff", [(300, 1024, 10900), (500, 640, 10920), (500, 576, 10920)])
 def test_gated_linear_192_columns(gpu, M, K, ff):

@@ -378,7 +378,7 @@ def test_gemm_u8(gpu, M, K, N):
 # chunks, one and two scales in 128 codes, and a block that takes the other kernel
 @pytest.mark.parametrize("M,K,N,block", [(2, 1152, 520, 64), (16, 1152, 4100, 128), (17, 2560, 1000, 256), (33, 1152, 5000, 64),
                                          (64, 5888, 4100, 128), (64, 1152, 3000, 384), (7, 17920, 6656, 128),
-                                         (16, 512, 32000, 128), (17, 512, 32000, 64)])  # two rounds of workgroups, both kernels
+                                         (16, 512, 32000, 128), (17, 512, 32000, 64), (20, 2560, 31010, 128)])  # two rounds of workgroups, both kernels
 def test_gemm_u8_few_rows(gpu, M, K, N, block):
     G = gpu
     x, w = normal((M, K), 0, 430, 1.0), normal((N, K), 0, 431, 0.02)
@@ -391,7 +391,8 @@ def test_gemm_u8_few_rows(gpu, M, K, N, block):
 # few rows, fp16: odd runs, rows past the last whole tile, columns past the last whole wavefront, lhs in chunks
 @pytest.mark.parametrize("M,K,N", [(3, 1152, 520), (16, 1408, 4099), (31, 2944, 1000), (48, 5888, 4100), (64, 4096, 24000),
                                    (16, 5760, 4099), (31, 5760, 4099), (24, 4096, 4096), (28, 512, 16840),  # 264, 264, 256 and 264 tiles
-                                   (8, 512, 32000), (40, 640, 31000)])  # two rounds of workgroups: the other kernel
+                                   (8, 512, 32000), (40, 640, 31000),  # two rounds of workgroups: the other kernel
+                                   (20, 2560, 31010), (24, 6144, 4099)])  # two rounds of long runs, one of them: this one
 def test_gemm_f16_few_rows(gpu, M, K, N):
     G = gpu
     x, w, old = normal((M, K), 0, 440, 1.0), normal((N, K), 0, 441, 0.02), normal((M, N), 0, 442, 1.0)
