@@ -204,6 +204,13 @@ __host__ __device__ __forceinline__ float divide_by(float x, float d, float reci
   return fmaf(fmaf(-q, d, x), reciprocal, q);
 }
 
+// The same with one correction more: the first leaves a quotient that is less than a unit off, from which the second gives the correctly rounded one.
+// An infinite x over a finite d stays itself, -0 becomes 0.  (Every half over divisors of all kinds, tests/cxx/kernel_arithmetic.hip.)
+__host__ __device__ __forceinline__ float divide_rounded(float x, float d, float reciprocal) {
+  const float near = divide_by(x, d, reciprocal), q = fmaf(fmaf(-near, d, x), reciprocal, near);
+  return __builtin_fabsf(x) == __builtin_inff() ? x * reciprocal : q;
+}
+
 // fp16(silu(a) * b), silu(a) = a / (1 + exp_ieee(-a)) in fp32 (llama_cu.cu:533-539), in two thirds of the instructions of exp_ieee and a
 // division, with the same result for all a and b.  exp_ieee's scaling in one step where 2^k is a normal number; the quotient from the
 // reciprocal by a Newton step and Markstein's correction, the divisor lying between 1 and 6.1e37.  Below -87 the quotient is

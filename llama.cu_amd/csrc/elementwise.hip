@@ -278,23 +278,32 @@ __global__ __launch_bounds__(1024) void softmax_argmax_kernel(half_t* __restrict
   index += blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n8 = n / 8;
-  if (n % 8 == 0 && n8 <= 4 * 1024) {
+  if (n % 8 == 0 && n8 > 0 && n8 <= 4 * 1024) {
     // every vocabulary of the model family (n <= 32768): the row is read once and each element's
     // x / temp, then its exponential, stays in registers -- the same operations in the same order
-    // as the general path below, which reads the row three times and takes each exponential twice
+    // as the general path below, which reads the row three times and takes each exponential twice.
+    // What bounds it are the vector instructions of one compute unit: quotients from a reciprocal, exponentials in their shorter form for arguments
+    // up to 0, and nothing for wavefronts behind the row (us, before / so: 32000 columns 18.3 / 12.3, 1024 6.3 / 5.4).
     float t[4][8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = tid + j * 1024;
-      const half8_t v = c < n8 ? *reinterpret_cast<const half8_t*>(logits + (size_t)c * 8) : (half8_t)(0.0f);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) t[j][e] = c < n8 ? (float)v[e] / temp : -INFINITY;
-    }
+    const float inverse = 1.0f / temp;
+    const bool by_reciprocal = fabsf(temp) > 0x1p-40f && fabsf(temp) < 0x1p40f;  // quotients and remainders of halves are normal numbers
     float m = -INFINITY;
+    half8_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const half8_t*>(logits + (size_t)min(tid + j * 1024, n8 - 1) * 8);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      if (tid + j * 1024 < n8) {
+        if (by_reciprocal) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) m = fmaxf(m, t[j][e]);
+          for (int e = 0; e < 8; ++e) t[j][e] = divide_rounded((float)v[j][e], temp, inverse);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[j][e] = (float)v[j][e] / temp;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = fmaxf(m, t[j][e]);
+      }
     }
     m = wave_max(m);
     if (lane == 0) sred[wave] = m;
@@ -309,7 +318,7 @@ __global__ __launch_bounds__(1024) void softmax_argmax_kernel(half_t* __restrict
       if (tid + j * 1024 < n8) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          t[j][e] = exp_ieee(t[j][e] - m);
+          t[j][e] = exp_ieee_nonpositive(t[j][e] - m);
           s += t[j][e];
         }
       }
@@ -321,6 +330,7 @@ __global__ __launch_bounds__(1024) void softmax_argmax_kernel(half_t* __restrict
 #pragma unroll
     for (int w = 0; w < 16; ++w) total += sred[w];
     __syncthreads();
+    const float share = 1.0f / total;
     float best = -INFINITY;
     int idx = 0x7fffffff;
 #pragma unroll
@@ -330,7 +340,7 @@ __global__ __launch_bounds__(1024) void softmax_argmax_kernel(half_t* __restrict
         half8_t p;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          p[e] = round_f16(t[j][e] / total);
+          p[e] = round_f16(divide_rounded(t[j][e], total, share));
           const float f = (float)p[e];
           if (f > best) {  // ascending index within a thread: strict > keeps the first maximum
             best = f;

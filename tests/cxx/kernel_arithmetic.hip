@@ -116,6 +116,37 @@ int main() {
            return n;
          }));
 
+  // logits: every half over temperatures of all sizes (0 of either sign), and probabilities over the sums of a vocabulary
+  report("halves over temperatures", in_pieces(4096, [](uint64_t a, uint64_t b) {
+           long n = 0;
+           for (uint64_t t = a; t < b; ++t) {
+             std::mt19937 random((uint32_t)t);
+             float d = of_bits(((127 - 40 + random() % 80) << 23) + (t % 3 == 0 ? random() % 64 : t % 3 == 1 ? 0x7fffffu - random() % 64 : random() % (1u << 23)));
+             const float usual[4] = {0.8f, 1.0f, 0.1f, 1.5f};
+             if (t < 4) d = usual[t];
+             if (t % 7 == 6) d = -d;
+             const float inverse = 1.0f / d;
+             for (uint32_t h = 0; h < 0x10000; ++h) {
+               const float x = (float)__builtin_bit_cast(_Float16, (uint16_t)h), want = x / d, got = lcu::divide_rounded(x, d, inverse);
+               n += x == x ? got != want : got == got;
+             }
+           }
+           return n;
+         }));
+  report("samples of e / sum in [1, 32768], fp32 for e of 2^-100 and more, or fp16", in_pieces(4096, [](uint64_t a, uint64_t b) {
+           long n = 0;
+           for (uint64_t t = a; t < b; ++t) {
+             std::mt19937 random((uint32_t)t + 5);
+             const float s = of_bits(0x3f800000u + random() % (15u << 23)), share = 1.0f / s;
+             for (int i = 0; i < 50000; ++i) {
+               const float e = i == 0 ? 0.0f : of_bits(0x00800000u + random() % (0x3f800001u - 0x00800000u));
+               const float want = e / s, got = lcu::divide_rounded(e, s, share);
+               n += bits(got) != bits(want) && (e >= 0x1p-100f || half_bits(got) != half_bits(want));
+             }
+           }
+           return n;
+         }));
+
   // probabilities: exponentials (0 and 2^-126 .. 1) over sums in [1, 4096], with significands at both ends among the sums
   report("samples of e / sum, fp16, or fp32 for e of 2^-100 and more", in_pieces(4096, [](uint64_t a, uint64_t b) {
            long n = 0;
