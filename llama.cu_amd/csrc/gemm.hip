@@ -1084,12 +1084,12 @@ inline bool streams(int M, int N, int n_mats, int splits, int stages, long tiles
   return rounds == 1 ? (tiles > cus && !short_runs) || run >= (M <= 16 ? 8 : M <= 32 ? 12 : 24) : rounds == 2 && run >= 20;
 }
 
-template <int TM, bool U8, bool BF16>
+template <int TM, bool U8, bool BF16, bool ONCE>
 int launch_stream_rows(operands_t op, const void* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, long cus) {
   long rounds = 1;
   const int waves = stream_waves(N, op.n_mats, splits, cus, stream_max_waves(U8), &rounds), tiles = ((N + 15) / 16 + waves - 1) / waves;
   op.more.tiles_n_per = op.n_mats;
-  auto kernel = gemm_stream_kernel<TM, U8, BF16>;
+  auto kernel = gemm_stream_kernel<TM, U8, BF16, ONCE>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -1107,9 +1107,13 @@ int launch_stream_rows(operands_t op, const void* A, int M, int K, int N, int bl
 // 1 .. 64 rows, K a multiple of 64: fp32 sums of every split's K stages to part[matrix][split][M][N]
 template <bool U8, bool BF16>
 int launch_stream(operands_t op, const void* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, long cus) {
-  if (M <= 16) return launch_stream_rows<1, U8, BF16>(op, A, M, K, N, block, st, splits, part, cus);
-  if (M <= 32) return launch_stream_rows<2, U8, BF16>(op, A, M, K, N, block, st, splits, part, cus);
-  return launch_stream_rows<4, U8, BF16>(op, A, M, K, N, block, st, splits, part, cus);
+  const auto rows = [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    if (M <= 16) return launch_stream_rows<1, U8, BF16, ONCE>(op, A, M, K, N, block, st, splits, part, cus);
+    if (M <= 32) return launch_stream_rows<2, U8, BF16, ONCE>(op, A, M, K, N, block, st, splits, part, cus);
+    return launch_stream_rows<4, U8, BF16, ONCE>(op, A, M, K, N, block, st, splits, part, cus);
+  };
+  return stream_once(N, K, op.n_mats, U8) ? rows(std::true_type{}) : rows(std::false_type{});
 }
 
 // How many workgroups the K stages of BM x 128 tiles are dealt to, and the workgroups in all; splits 0: too few of them, or no room for the sums.
@@ -1151,9 +1155,9 @@ bool scale_words_ok(const operands_t& op, int K, int N, int block) {
   }
 }
 
-template <int TM, bool U8, bool BF16, class JOIN>
+template <int TM, bool U8, bool BF16, bool ONCE, class JOIN>
 int launch_joined_rows(JOIN const& join, operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, int waves, int tiles) {
-  auto kernel = gemm_stream_kernel<TM, U8, BF16, JOIN>;
+  auto kernel = gemm_stream_kernel<TM, U8, BF16, ONCE, JOIN>;
   static bool raised[16] = {};  // per device, once
   int dev = 0;
   LCU_HIP(hipGetDevice(&dev));
@@ -1171,9 +1175,13 @@ int launch_joined_rows(JOIN const& join, operands_t op, const half_t* A, int M, 
 
 template <bool U8, bool BF16, class JOIN>
 int launch_joined_shape(JOIN const& join, operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, stream_join_t shape) {
-  if (M <= 16) return launch_joined_rows<1, U8, BF16>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
-  if (M <= 32) return launch_joined_rows<2, U8, BF16>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
-  return launch_joined_rows<4, U8, BF16>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
+  const auto rows = [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    if (M <= 16) return launch_joined_rows<1, U8, BF16, ONCE>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
+    if (M <= 32) return launch_joined_rows<2, U8, BF16, ONCE>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
+    return launch_joined_rows<4, U8, BF16, ONCE>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
+  };
+  return stream_once(N, K, op.n_mats, U8) ? rows(std::true_type{}) : rows(std::false_type{});
 }
 
 // A product of few rows and what follows it in one launch, with the splits of plan_skinny.  *done = false, with nothing launched, where lhs does not fit

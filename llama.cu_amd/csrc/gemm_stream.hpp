@@ -11,10 +11,10 @@
 // M = 8 with a launch that adds the splits, fp16 three times (4096, 4096) 26.0 -> 22.7 us, twice (N, K) = (11008, 4096) 45 -> 42,
 // (4096, 4096) 12.1 -> 12.4; uint8 three times (6656, 6656) 61 -> 35, twice (17920, 6656) 104 -> 57, (6656, 17920) 62 -> 37.  Rows of
 // 8 KB meet in the same memory channels: K = 4224 takes a tenth less than 4096.
-// W is read once and marked so (nt): 8 rows, twice 11008 columns of K 4096 36.8 -> 33.7 us (4.9 -> 5.35
-// TB/s), 16x4096x11008 22.4 -> 20.9, 60x6656x17920 53.6 -> 50.0; eight sequences of eight 7B layers, 45 + 16 tokens 23.4 -> 22.1 ms.  uint8 gains up to
-// 1.5 %.  Weights that the 256 MB cache holds from call to call lose what they gained there (60x6656x17920 again and again 45 -> 47.8 us), but a
-// model's do not come back before the cache has seen all of them.
+// Matrices from 64 MB up are marked as read once (nt), which keeps their lines out of the 256 MB cache in front of memory: 8 rows, twice 11008 columns
+// of K 4096 36.8 -> 33.7 us (4.9 -> 5.35 TB/s), 16x4096x11008 22.4 -> 20.9, 60x6656x17920 53.6 -> 50.0; eight sequences of eight 7B layers, 45 + 16 tokens
+// 23.4 -> 22.1 ms.  A model of smaller ones may come back from that cache step after step, and would lose by it (weights of 67 MB in the cache 13.1 / 18.2 us
+// with the mark; uint8 5x6656x6656 12.3 / 13.7, from memory 14.9 / 14.3).
 #pragma once
 #include <algorithm>
 
@@ -26,6 +26,7 @@ constexpr int STREAM_RING = 4;
 constexpr int STREAM_LHS = 64 * 1024;  // bytes of lhs in LDS: one chunk, or two of half of it
 // a unit is 16 rows of 128 bytes; uint8: and a word with the scales of each row
 constexpr int stream_unit(bool u8) { return 2048 + (u8 ? 256 : 0); }
+inline bool stream_once(int N, int K, int n_mats, bool u8) { return (size_t)N * K * n_mats * (u8 ? 1 : 2) >= (size_t)64 << 20; }
 constexpr int stream_max_waves(bool u8) { return u8 ? 10 : 12; }  // LDS: 160 KB
 constexpr int stream_lds(bool u8, int waves) { return STREAM_LHS + waves * STREAM_RING * stream_unit(u8); }
 // JOINED: lhs whole, and behind the product the sums of every wavefront in its place, [wavefront][row][16]; the rest for the rings
@@ -67,7 +68,7 @@ struct separate_sums {
   static constexpr int MATRICES = 1;
 };
 
-template <int TM, bool U8, bool BF16, class JOIN = separate_sums>
+template <int TM, bool U8, bool BF16, bool ONCE, class JOIN = separate_sums>
 __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kernel(const half_t* __restrict__ A, const void* __restrict__ W0,
                                                                                const half_t* __restrict__ S0, int block_shift, int M, int K,
                                                                                int N, int tiles, int kc, float* __restrict__ part, int splits,
@@ -131,11 +132,20 @@ __global__ __launch_bounds__(64 * stream_max_waves(U8), 3) void gemm_stream_kern
   const auto request = [&](int u) {
     if (u == units) rw[2] = rs[2] = 0;  // behind the last unit: requests that count and touch no memory (stage_offset)
     const uint32_t slot = ring0 + (u % RING) * UNIT, along = stage_offset(rw[2], (uint32_t)(base * (U8 ? 64 : 128) + u * 128));
+    if constexpr (ONCE) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(w_off[j]), "s"(rw), "s"(along),
-                   "s"(slot + j * 1024)
-                   : "memory", "m0");
+      for (int j = 0; j < 2; ++j) {
+        asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(w_off[j]), "s"(rw), "s"(along),
+                     "s"(slot + j * 1024)
+                     : "memory", "m0");
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(w_off[j]), "s"(rw), "s"(along),
+                     "s"(slot + j * 1024)
+                     : "memory", "m0");
+      }
     }
     if constexpr (U8) {  // the word that holds the row's scales of both stages
       const uint32_t at = s_first + ((uint32_t)(base + 2 * u) >> block_shift);
