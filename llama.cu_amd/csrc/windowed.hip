@@ -142,12 +142,22 @@ __device__ __forceinline__ float row_max(float x) {
   return fmaxf(__builtin_bit_cast(float, (uint32_t)two[0]), __builtin_bit_cast(float, (uint32_t)two[1]));
 }
 
+// ln x of an x that is no subnormal, as 1 + y never is: log2 x times ln 2 in two parts.  The bits of __logf, without its steps for subnormals
+// (2048 rows with distance bias 100 / 90 us).
+__device__ __forceinline__ float log_of_sum(float x) {
+  constexpr float LN2 = 0x1.62e42ep-1f, LN2_REST = 0x1.efa39ep-25f;  // ln 2 rounded down, and what that leaves
+  const float y = __builtin_amdgcn_logf(x), z = y * LN2;
+  return fabsf(y) < INFINITY ? z + fmaf(y, LN2_REST, fmaf(y, LN2, -z)) : y;
+}
+
 // What bounds it is the chain of a tile (scores, maximum, exponentials, values) on the two wavefronts that a SIMD has registers for.  So fragments of keys and
 // values are asked for four products ahead (left to itself the compiler asks for one and waits for it), values lie in LDS as they come and are turned on
-// their way out (ds_read_b64_tr_b16; written turned they took sixteen 4-byte stores a thread), four maxima meet by register swaps and only when one
-// has grown, and sums go in four chains.  us, 32 heads, values of 128, before / now: keys of 192 over all, 2048 rows 132 / 94, 512 rows 29 / 20; keys of
-// 128 in a window of 1024, 2048 rows 77 / 62, 512 rows 25 / 16; with distance bias 512 rows 32 / 18, 2048 rows 136 / 76; keys and values of 64,
-// 2048 rows 56 / 42.  (Three wavefronts per SIMD spill and take 233 in place of 94.)
+// their way out (ds_read_b64_tr_b16; written turned they took sixteen 4-byte stores a thread), and four maxima meet by register swaps and only when one
+// has grown.  us, 32 heads, values of 128, before / now: keys of 192 over all, 2048 rows 129 / 98, 512 rows 29 / 19.5; keys of
+// 128 in a window of 1024, 2048 rows 75 / 66, 512 rows 25 / 17; with distance bias 512 rows 32 / 20, 2048 rows 136 / 85; keys and values of 64,
+// 2048 rows 56 / 45; keys of 128, values of 256, 2048 rows 220 / 111.  (Three wavefronts per SIMD spill and take 233 in place of 98.)  Maxima, exponentials
+// and sums are those of a running softmax to base e, in the order of the keys: the bits are those from before.  (Scores in powers of two, a maximum
+// followed from 2^8 on and sums in four chains take 4 % less, 14 % with distance bias, and round otherwise.)
 // KP: 32-column pieces of a key; OCC: wavefronts per SIMD that the registers are cut to.
 template <int DV, bool BIAS, int KP, int OCC>
 __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
@@ -196,11 +206,7 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
     qf[c] = *reinterpret_cast<const bf16x8_t*>(q + (size_t)min(q0 + wave * 16 + col, n - 1) * p.ldq + (size_t)h * p.dk + c * 32 + quad * 8);
   }
   const int i = first + wave * 16 + col;             // position of this lane's row
-  // Scores and maxima count in powers of two.  A maximum is followed only when a score lies more than SLACK above it: sums and values grow by up
-  // to 2^SLACK, and nothing rounds differently for it.
-  constexpr float LOG2E = 1.44269504f, SLACK = 8.0f;
-  const float scale = p.scale * LOG2E;
-  float m = p.sink ? p.sink[h] * LOG2E : -1e30f;     // the sink counts as a key of value zero
+  float m = p.sink ? p.sink[h] : -1e30f;             // the sink counts as a key of value zero; any finite one stays finite
   float l = p.sink && quad == 0 ? 1.0f : 0.0f;       // of this lane's keys
   float4_t o[NT];                                    // values t * 16 + quad * 4 .. + 3 of the row
 #pragma unroll
@@ -242,10 +248,10 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      s[t] *= scale;
+      s[t] *= p.scale;
       if constexpr (BIAS) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[t][e] -= r1 * __builtin_amdgcn_logf(1.0f + r2 * (float)max(i - (k0 + t * 16 + quad * 4 + e), 0));
+        for (int e = 0; e < 4; ++e) s[t][e] -= r1 * log_of_sum(1.0f + r2 * (float)max(i - (k0 + t * 16 + quad * 4 + e), 0));
       }
     }
     const int lowest = first + wave * 16;  // of the wavefront's positions
@@ -262,29 +268,27 @@ __global__ __launch_bounds__(256, OCC) void attention_tile_kernel(bf16_t* __rest
     float top = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 4; ++t) top = fmaxf(top, fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])));
-    if (__ballot(top > m + SLACK) != 0) {
+    if (__ballot(top > m) != 0) {
       top = fmaxf(m, row_max(top));
-      const float shrink = __builtin_amdgcn_exp2f(m - top);
+      const float shrink = __expf(m - top);
       m = top;
       l *= shrink;
 #pragma unroll
       for (int t = 0; t < NT; ++t) o[t] *= shrink;
     }
-    float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     bf16x8_t hi[KT / 32], rem[KT / 32];
 #pragma unroll
     for (int c = 0; c < KT / 32; ++c) {
       float pr[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) pr[e] = __builtin_amdgcn_exp2f(s[c * 2 + e / 4][e % 4] - m);
+      for (int e = 0; e < 8; ++e) pr[e] = __expf(s[c * 2 + e / 4][e % 4] - m);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) part[e & 3] += pr[e];
+      for (int e = 0; e < 8; ++e) l += pr[e];
 #pragma unroll
       for (int e = 0; e < 8; ++e) hi[c][e] = (bf16_t)pr[e];
 #pragma unroll
       for (int e = 0; e < 8; ++e) rem[c][e] = (bf16_t)(pr[e] - (float)hi[c][e]);
     }
-    l += (part[0] + part[1]) + (part[2] + part[3]);
     union {
       short4_t half[2];
       bf16x8_t all;

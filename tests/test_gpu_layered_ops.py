@@ -420,7 +420,7 @@ def test_windowed_attention_key_sizes(gpu, dim, vdim):
     gpu.release()
 
 
-# a maximum that grows from tile to tile by less than the kernel follows (2^8 in all but a few rows), by about as much, by far more, and one that falls
+# a maximum that grows from tile to tile by little (e in 100 keys), by more, by e^38, and one that falls
 @pytest.mark.parametrize("growth", [0.01, 0.08, 0.6, -0.3])
 @pytest.mark.parametrize("dim,vdim", [(64, 64), (192, 128)])
 def test_windowed_attention_of_growing_scores(gpu, dim, vdim, growth):
@@ -431,6 +431,33 @@ def test_windowed_attention_of_growing_scores(gpu, dim, vdim, growth):
     r1, r2 = (gpu.B.from_device(b, (heads,), np.float32).astype(float) for b in last_two_vectors(gpu))
     want = S.windowed_attention(c["q"][..., :dim], c["k"][..., :dim], c["v"][..., :vdim], c["wp"].scale, r1, r2, window, keep)
     close(run_attention(gpu, c, BF16, (T,)), want, BF16, bf16=2.0 ** -7)
+    gpu.release()
+
+
+@BOTH
+@pytest.mark.parametrize("sink", [float(np.finfo(np.float32).min), -3e38, -2.4e38, -1e30])
+def test_windowed_attention_of_sinks_that_are_switched_off(gpu, dt, sink):
+    """A sink at the lowest float is no sink, also for rows whose window begins behind the first tile that their workgroup visits."""
+    for heads, kv, dim, vdim, window, T in [(3, 3, 64, 64, 10, 128), (4, 2, 192, 128, 70, 200)]:
+        c = attention_case(gpu, dt, heads, kv, dim, vdim, window, 0, T, dim)
+        c["wp"].sink = put(gpu, np.full(heads, sink)).ptr
+        close(run_attention(gpu, c, dt, (T,)), c["want"], dt, bf16=2.0 ** -7)
+    gpu.release()
+
+
+def test_windowed_attention_of_lowest_scores(gpu):
+    """Scores down to -1e30, where a running maximum begins: the largest of a row takes all."""
+    heads, T = 2, 130
+    c = attention_case(gpu, BF16, heads, heads, 32, 32, T, 0, T, 5)
+    c["wp"].scale, c["wp"].r1, c["wp"].r2 = 2.0 ** 96, None, None
+    c["q"][:] = 0.0
+    c["k"][:] = 0.0
+    c["q"][..., 0] = 1.0
+    c["k"][..., 0] = rounded(-np.random.default_rng(6).permutation(np.linspace(9.0, 12.5, T)))[:, None]  # scores of -7.1e29 to -9.9e29
+    got, scores = run_attention(gpu, c, BF16, (T,)), c["k"][:, 0, 0]
+    for i in range(T):
+        first = np.flatnonzero(scores[:i + 1] == scores[:i + 1].max())
+        assert np.allclose(got[i], c["v"][first].mean(0), rtol=2.0 ** -7, atol=0), i
     gpu.release()
 
 
