@@ -71,7 +71,9 @@ struct llama_batch_context_impl final : public llama_batch_context {
 
   short next_token(int sequence, std::vector<short> const& new_tokens) override {
     LCU_CHECK(lcu_sync(stream_));
-    return seqs_[sequence]->next_token(new_tokens);
+    const short token = seqs_[sequence]->next_token(new_tokens);
+    LCU_CHECK(lcu_sync(seqs_[sequence]->stream()));  // the token may be there first; the next step reads the keys and values on stream_
+    return token;
   }
 
   std::vector<short> next_tokens(std::vector<short> const& tokens) override {

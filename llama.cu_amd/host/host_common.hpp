@@ -71,8 +71,9 @@ class pinned_buffer {
 
 // What a call's last launch leaves in page-locked memory, none of it ever -1, is watched for instead of waiting for the stream: expect() before
 // the launch, await() for the words.  hipStreamSynchronize returns 5 to 10 us after the word is there (a graph of 11 small launches
-// 36.7 us with it and 26.5 so, of 36 launches 76.5 and 68.6).  Whoever reads what other launches of the call wrote does so behind them on
-// the same stream; what they read (page-locked input, a graph's arguments) is released or freed behind a wait for the stream itself.
+// 36.7 us with it and 26.5 so, of 36 launches 76.5 and 68.6).  The words say nothing of what else the call's launches wrote: that is read behind
+// them on the same stream, or on another behind a wait for this one; what they read (page-locked input, a graph's arguments) is released or
+// freed behind such a wait too.
 // A launch that takes longer than `patience`, or failed, is left to the stream's own wait and its error.
 class awaited_words {
  public:
