@@ -586,8 +586,8 @@ int layered_context_impl::forward(const int32_t* tokens, int n, const int32_t* w
         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
         LCU_CHECK(lcu_sample_row(t_index_.data(), t_probs_.data(), vocab, z ^ (z >> 31), nullptr, stream_));
       }
-      if (sampling_) {
-        LCU_CHECK(lcu_sync(stream_));  // the sampler's launch writes the token once more
+      if (n > 1 || sampling_) {
+        LCU_CHECK(lcu_sync(stream_));  // sampling: another launch writes the token once more
       } else {
         answer.await(stream_);
       }

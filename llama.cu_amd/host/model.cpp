@@ -586,8 +586,8 @@ short llama_context_impl::next_token(std::vector<short> const& new_tokens) {
     unsigned timeouts;
   } result{0, 0};
   const auto await_result = [&] {  // 1198-1200
-    if (sampling_) {
-      LCU_CHECK(lcu_sync(stream_));  // the sampler's launch writes the token once more
+    if (n > 1 || sampling_) {
+      LCU_CHECK(lcu_sync(stream_));  // sampling: another launch writes the token once more
     } else {
       answer.await(stream_);
     }

@@ -24,3 +24,43 @@ result += [("step", None)] + calls()
     for stream in prompts:
         last = max(i for i, (name, s) in enumerate(before) if s == stream and name != "lcu_sync")
         assert ["lcu_sync", stream] in before[last:]
+
+
+STEP = {"context": "context.next_token([1])", "batch": "batch.next_tokens([1, 2])[0]"}
+CONTEXTS = """
+model = tiny_model()
+context, batch = P.Context(model, context_len=64), P.BatchContext(model, 2, context_len=64)
+def names():
+    return [name for name, _ in calls()]
+"""
+
+
+def test_a_prompt_waits_for_its_stream():
+    """A call of several tokens has nothing to gain by looking for its token: it takes no processor time while it waits, however long."""
+    tokens, seconds, seen = recorded_calls.run(CONTEXTS + """
+stand_in.recorded_lateness(30000)
+tokens, began = [], time.thread_time()
+for _ in range(8):
+    tokens.append(context.next_token([1, 2, 3]))
+result = tokens, time.thread_time() - began, names()
+""")
+    assert tokens == [7] * 8 and seconds < 0.03 and seen[-1] == "lcu_sync"  # of 0.24 s in all
+
+
+@pytest.mark.parametrize("kind", STEP)
+def test_a_step_that_outlasts_the_watch_is_waited_for(kind):
+    """The token of a quick step is taken as it comes, that of a slow one behind a wait for its stream."""
+    tokens, quick, late, again = recorded_calls.run(CONTEXTS + f"""
+step = lambda: {STEP[kind]}
+tokens = [step() for _ in range(3)]
+names(); tokens.append(step())
+quick = names()
+stand_in.recorded_lateness(1000)
+tokens += [step(), step()]
+late = names()
+stand_in.recorded_lateness(-1)
+tokens.append(step())
+result = tokens, quick, late, names()
+""")
+    assert tokens == [7] * 7 and late == 2 * ["lcu_graph_launch", "lcu_sync"]
+    assert quick == again == ["lcu_graph_launch"]
