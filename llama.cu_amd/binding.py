@@ -45,6 +45,7 @@ SIGNATURES = {
     "lcu_d2h": (i32, [vp, vp, sz, vp]),
     "lcu_d2d": (i32, [vp, vp, sz, vp]),
     "lcu_stream_create": (i32, [C.POINTER(vp)]),
+    "lcu_stream_weights": (i32, [vp, sz]),
     "lcu_stream_destroy": (i32, [vp]),
     "lcu_sync": (i32, [vp]),
     "lcu_event_create": (i32, [C.POINTER(vp)]),

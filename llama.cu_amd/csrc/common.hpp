@@ -68,6 +68,7 @@ struct workspace_t {
   uint32_t* sync = nullptr;
   // true for the workspace of a stream made by lcu_stream_create: nobody else's launches use it
   bool owned = false;
+  size_t weights = 0;  // lcu_stream_weights
 };
 constexpr int SYNC_EXCHANGE = 2048;
 // offsets (in 8-byte words) of the hand-over areas: decode attention scores (64 heads x 4096), then

@@ -981,6 +981,11 @@ int launch_large(EP const& ep, operands_t op, const void* A, int M, int K, int N
   }
 }
 
+template <bool U8>
+size_t weight_bytes(const operands_t& op, int K, int N) {
+  return (size_t)N * K * (U8 ? 1 : 2) * op.n_mats;
+}
+
 // where a split-K launch left its partial sums: part[matrix][split][M][N] fp32
 struct partial_sums_t {
   const float* part;
@@ -1026,25 +1031,6 @@ int launch_split(operands_t op, const half_t* A, int M, int K, int N, int block,
   return LCU_OK;
 }
 
-// Wavefronts (of 16 columns) per workgroup of gemm_stream_kernel: one workgroup runs per compute unit, so the longest
-// compute unit has rounds * wavefronts of them to stream; below four a compute unit has too little in flight (8 rows, three
-// times 2048x2048: nine rounds of single wavefronts 19.6 us, one of ten 10.7).  *rounds: how many they are.
-inline int stream_waves(int N, int n_mats, int splits, long cus, int most, long* rounds) {
-  const long groups = (N + 15) / 16;
-  int best = 1;
-  long least = 0;
-  for (int w = 1; w <= most; ++w) {
-    const long wgs = (groups + w - 1) / w * n_mats * splits;
-    const long cost = (wgs + cus - 1) / cus * std::max(w, 4);
-    if (w == 1 || cost <= least) {
-      least = cost;
-      best = w;
-      *rounds = (wgs + cus - 1) / cus;
-    }
-  }
-  return best;
-}
-
 // Workgroups that have every split of their columns: wavefronts of one (0: more than a round of them, too few wavefronts for the splits, or no room for lhs)
 // and workgroups in all.  As few sixteens of columns as leave one round, four wavefronts at least.
 struct stream_join_t {
@@ -1062,26 +1048,6 @@ inline stream_join_t plan_stream_join(int M, int K, int N, int n_mats, int joine
     if (tiles <= cus && waves >= 4) return {waves, (int)tiles};
   }
   return {0, 0};
-}
-
-// Whether a product of few rows is one of gemm_stream_kernel, or of BM x 128 tiles of four wavefronts.  Of those several share a
-// compute unit; a workgroup here has it alone, so that a second round fills lhs and ring again with nothing beside it, which a long enough run
-// of stages pays for.  us with weights from memory, tiles / here: two rounds, fp16 8 rows of 32000 columns, K 2048, 2560, 4096, 6656 29.4 / 32.7, 33.6 / 31.0,
-// 62.2 / 54.7, 79.1 / 71.0, 24 rows 30.8 / 35.4, 43.2 / 41.0 (K 3072), 66.9 / 60.9, 64 rows of K 4096 71.9 / 68.0; uint8 32 rows, K 4096, 6656
-// 46.3 / 44.0, 70.1 / 61.9, 48 rows 76.3 / 76.2, 16 rows of 4096x11008 twice 36.6 / 32.7; three rounds, 5888x9664 three times 62 / 67.
-// One round: uint8 gains, but over short runs (15x512x10304 twice 10.3 / 11.4); fp16 where the tiles (`tiles` in all, with their splits) do not come out
-// even (27x17920x6656 62 / 45), or over runs of some stages (10x1024x7304 8.6 / 9.2; 24x4096x4096 13.3 / 13.3, 24x6144x4096 16.4 / 15.7, 20x11008x4096
-// 23.6 / 22.2, 20x8192x8192 36.5 / 33.0; 50 rows 18.3 / 18.3, 8192x4096 20.9 / 21.2, 8192x8192 64 rows 39.5 / 35.1).  bfloat16 gains at every count (4x512x3264
-// 9.2 / 7.9, 46x17920x6656 68 / 50).  Neither does for more than 16 rows over the shortest runs (28x512x16840 10.5 / 11.1, bfloat16
-// 56x512x16576 13.8 / 14.8).  A product called again and again, its weights in the caches, is sooner in tiles (64x8192x8192 26.7 / 34.3); a model's are not.
-inline bool streams(int M, int N, int n_mats, int splits, int stages, long tiles, long cus, bool u8, bool bf16) {
-  long rounds = 1;
-  stream_waves(N, n_mats, splits, cus, stream_max_waves(u8), &rounds);
-  const int run = stages / splits;
-  if (u8) return rounds == 1 || (rounds == 2 && M <= 32 && run >= (M <= 16 ? 12 : 20));
-  const bool short_runs = M > 16 && run <= 4;
-  if (bf16) return rounds == 1 && (!short_runs || 4 * tiles <= 3 * cus);
-  return rounds == 1 ? (tiles > cus && !short_runs) || run >= (M <= 16 ? 8 : M <= 32 ? 12 : 24) : rounds == 2 && run >= 20;
 }
 
 template <int TM, bool U8, bool BF16, bool ONCE>
@@ -1106,32 +1072,14 @@ int launch_stream_rows(operands_t op, const void* A, int M, int K, int N, int bl
 
 // 1 .. 64 rows, K a multiple of 64: fp32 sums of every split's K stages to part[matrix][split][M][N]
 template <bool U8, bool BF16>
-int launch_stream(operands_t op, const void* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, long cus) {
+int launch_stream(operands_t op, const void* A, int M, int K, int N, int block, hipStream_t st, int splits, float* part, long cus, bool memory) {
   const auto rows = [&](auto once) {
     constexpr bool ONCE = decltype(once)::value;
     if (M <= 16) return launch_stream_rows<1, U8, BF16, ONCE>(op, A, M, K, N, block, st, splits, part, cus);
     if (M <= 32) return launch_stream_rows<2, U8, BF16, ONCE>(op, A, M, K, N, block, st, splits, part, cus);
     return launch_stream_rows<4, U8, BF16, ONCE>(op, A, M, K, N, block, st, splits, part, cus);
   };
-  return stream_once(N, K, op.n_mats, U8) ? rows(std::true_type{}) : rows(std::false_type{});
-}
-
-// How many workgroups the K stages of BM x 128 tiles are dealt to, and the workgroups in all; splits 0: too few of them, or no room for the sums.
-struct skinny_plan_t {
-  int splits;
-  long tiles;
-};
-template <bool U8>
-skinny_plan_t plan_skinny(int BM, int M, int K, int N, int n_mats, int cus, size_t workspace_bytes) {
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + 127) / 128 * n_mats, nt_all = K / BK;
-  // one workgroup per compute unit and at least four stages each: more, shorter splits only add
-  // partial sums (512 workgroups: 16 against 13 us at N = K = 4096)
-  int splits = (cus + tiles_m * tiles_n - 1) / (tiles_m * tiles_n);
-  splits = max(1, min(splits, nt_all / 4));
-  const size_t each = (size_t)M * N * n_mats * sizeof(float);
-  while (splits > 1 && splits * each > workspace_bytes) --splits;
-  if (splits * each > workspace_bytes || (long)tiles_m * tiles_n * splits < cus / 2) return {0, 0};
-  return {splits, (long)tiles_m * tiles_n * splits};
+  return stream_once(memory, weight_bytes<U8>(op, K, N)) ? rows(std::true_type{}) : rows(std::false_type{});
 }
 
 // The direct-to-LDS kernels fetch a thread's fp16 scale as the aligned 4-byte word that holds it:
@@ -1174,14 +1122,15 @@ int launch_joined_rows(JOIN const& join, operands_t op, const half_t* A, int M, 
 }
 
 template <bool U8, bool BF16, class JOIN>
-int launch_joined_shape(JOIN const& join, operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, stream_join_t shape) {
+int launch_joined_shape(JOIN const& join, operands_t op, const half_t* A, int M, int K, int N, int block, hipStream_t st, int splits, stream_join_t shape,
+                        bool memory) {
   const auto rows = [&](auto once) {
     constexpr bool ONCE = decltype(once)::value;
     if (M <= 16) return launch_joined_rows<1, U8, BF16, ONCE>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
     if (M <= 32) return launch_joined_rows<2, U8, BF16, ONCE>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
     return launch_joined_rows<4, U8, BF16, ONCE>(join, op, A, M, K, N, block, st, splits, shape.waves, shape.tiles);
   };
-  return stream_once(N, K, op.n_mats, U8) ? rows(std::true_type{}) : rows(std::false_type{});
+  return stream_once(memory, weight_bytes<U8>(op, K, N)) ? rows(std::true_type{}) : rows(std::false_type{});
 }
 
 // A product of few rows and what follows it in one launch, with the splits of plan_skinny.  *done = false, with nothing launched, where lhs does not fit
@@ -1199,11 +1148,11 @@ int launch_joined(JOIN const& join, operands_t op, const half_t* A, int M, int K
   for (const void* o : {(const void*)op.out, (const void*)op.more.out[0], (const void*)op.more.out[1], out}) {
     if (o != nullptr && overlap(o, out_bytes, A, lhs_bytes)) return LCU_OK;
   }
-  const skinny_plan_t plan = plan_skinny<U8>(M <= 32 || U8 ? 32 : 64, M, K, N, op.n_mats, ds->compute_units, ws.bytes);
+  const skinny_plan_t plan = plan_skinny(M <= 32 || U8 ? 32 : 64, M, K, N, op.n_mats, ds->compute_units, ws.bytes);
   if (plan.splits == 0) return LCU_OK;
   const stream_join_t shape = plan_stream_join(M, K, N, op.n_mats, JOIN::MATRICES, plan.splits, ds->compute_units, U8);
   if (shape.waves == 0) return LCU_OK;
-  const int rc = launch_joined_shape<U8, false>(join, op, A, M, K, N, block, st, plan.splits, shape);
+  const int rc = launch_joined_shape<U8, false>(join, op, A, M, K, N, block, st, plan.splits, shape, from_memory(ws.weights, weight_bytes<U8>(op, K, N)));
   *done = rc == LCU_OK;
   return rc;
 }
@@ -1243,16 +1192,17 @@ int launch_skinny(operands_t op, const half_t* A, int M, int K, int N, int block
     rc = launch_joined<U8>(f16_join{{op.out, op.more.out[0], op.more.out[1]}, N, beta}, op, A, M, K, N, block, st, nullptr, done);
     if (rc != LCU_OK || *done) return rc;
   }
-  const skinny_plan_t plan = plan_skinny<U8>(BM, M, K, N, op.n_mats, ds->compute_units, ws.bytes);
+  const skinny_plan_t plan = plan_skinny(BM, M, K, N, op.n_mats, ds->compute_units, ws.bytes);
   if (plan.splits == 0) return LCU_OK;
   const int splits = plan.splits;
   const size_t mn = (size_t)M * N;
-  if ((U8 && block_shift(block) < 0) || !streams(M, N, op.n_mats, splits, K / BK, plan.tiles, ds->compute_units, U8, false)) {
+  const bool memory = from_memory(ws.weights, weight_bytes<U8>(op, K, N));
+  if ((U8 && block_shift(block) < 0) || !streams(M, N, op.n_mats, splits, K / BK, plan.tiles, ds->compute_units, U8, false, memory)) {
     rc = launch_split<BM, BN, 1, 4, U8>(op, A, M, K, N, block, beta, st, splits, (float*)ws.ptr, leave);
     *done = rc == LCU_OK;
     return rc;
   }
-  rc = launch_stream<U8, false>(op, A, M, K, N, block, st, splits, (float*)ws.ptr, ds->compute_units);
+  rc = launch_stream<U8, false>(op, A, M, K, N, block, st, splits, (float*)ws.ptr, ds->compute_units, memory);
   if (rc == LCU_OK && leave) {
     leave->part = (float*)ws.ptr;
     leave->splits = splits;
@@ -1813,7 +1763,8 @@ struct linear_join {
 // drawn shapes of 2 to 62 rows 7 to 71 % sooner where K is split).  *done = false, with nothing launched, where lhs does not fit LDS whole, the workgroups would take a
 // second round, or the outputs lie over lhs.
 template <bool GATED>
-int bf16_joined(linear_epilogue<false, GATED> const& ep, const void* A, const void* W, int M, int K, int N, int splits, long cus, hipStream_t st, bool* done) {
+int bf16_joined(linear_epilogue<false, GATED> const& ep, const void* A, const void* W, int M, int K, int N, int splits, long cus, bool memory,
+                hipStream_t st, bool* done) {
   *done = false;
   const size_t lhs_bytes = (size_t)M * K * 2;
   const int outs = GATED ? N / 2 : N;
@@ -1825,7 +1776,8 @@ int bf16_joined(linear_epilogue<false, GATED> const& ep, const void* A, const vo
   const int mats = GATED ? 2 : 1;
   const stream_join_t shape = plan_stream_join(M, K, outs, mats, mats, splits, cus, false);
   if (shape.waves == 0) return LCU_OK;
-  const int rc = launch_joined_shape<false, true>(linear_join<GATED>{ep, N}, single_matrix(nullptr, W, nullptr), (const half_t*)A, M, K, N, 0, st, splits, shape);
+  const int rc = launch_joined_shape<false, true>(linear_join<GATED>{ep, N}, single_matrix(nullptr, W, nullptr), (const half_t*)A, M, K, N, 0, st, splits, shape,
+                                                memory);
   *done = rc == LCU_OK;
   return rc;
 }
@@ -1842,11 +1794,12 @@ int bf16_skinny(linear_epilogue<false, GATED> const& ep, const void* A, const vo
   int splits = std::min((ds->compute_units + tiles - 1) / tiles, K / BK / 4);
   while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ws.bytes) --splits;
   if (splits < 2) return LCU_OK;
-  int rc = bf16_joined<GATED>(ep, A, W, M, K, N, splits, ds->compute_units, st, done);
+  const bool memory = from_memory(ws.weights, (size_t)N * K * 2);
+  int rc = bf16_joined<GATED>(ep, A, W, M, K, N, splits, ds->compute_units, memory, st, done);
   if (rc != LCU_OK || *done) return rc;
   float* part = (float*)ws.ptr;
-  if (streams(M, N, 1, splits, K / BK, (long)tiles * splits, ds->compute_units, false, true)) {
-    rc = launch_stream<false, true>(single_matrix(nullptr, W, nullptr), A, M, K, N, 0, st, splits, part, ds->compute_units);
+  if (streams(M, N, 1, splits, K / BK, (long)tiles * splits, ds->compute_units, false, true, memory)) {
+    rc = launch_stream<false, true>(single_matrix(nullptr, W, nullptr), A, M, K, N, 0, st, splits, part, ds->compute_units, memory);
   } else {
     rc = M <= 32 ? launch_bf16<32, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part)
                  : launch_bf16<64, 128, 1, 4, 1, 3, true>(ep, A, W, 1, M, K, N, st, splits, part);

@@ -1,4 +1,4 @@
-// Which tiles a product of more than 64 rows takes, and into how many chains its sums are cut (gemm.hip).  Plain arithmetic, apart from
+// Which tiles a product of more than 64 rows takes, and into how many chains its sums are cut (gemm.hip); which kernel one of fewer takes.  Plain arithmetic, apart from
 // the kernels, so that it can be checked on the host.
 #pragma once
 #include <algorithm>
@@ -187,6 +187,81 @@ inline int plan_expert_rows(long rows, int experts, int K, int ff, long cus) {
   };
   const double c64 = cost(64, 17.4, 3, 53, 2), c128 = cost(128, 24.8, 3.8, 19, 1), c256 = cost(256, 34.3, 5.1, 19, 1);
   return c64 <= c128 && c64 <= c256 ? 64 : c128 <= c256 ? 128 : 256;
+}
+
+// ---- 2 to 64 rows (gemm_stream.hpp) ----
+constexpr int stream_max_waves(bool u8) { return u8 ? 10 : 12; }  // LDS: 160 KB
+
+// Whether weights come from memory: a program goes through `known` bytes of them before it is back at the same ones (lcu_stream_weights), or one launch
+// through `bytes`, and the 256 MB cache in front of memory holds neither.  Other weights may lie there, and what is right for them is another
+// matter (streams, stream_once).  One product again and again, us as from a cache / as from memory: fp16 of 273 MB 8 rows 43.7 / 44.0, 40 rows 46.6 / 50.3,
+// 328 MB 8 rows 62.8 / 56.9, 426 MB 24 rows 79.4 / 73.7, uint8 of 321 MB 40 rows 187 / 161.
+constexpr size_t FROM_MEMORY = (size_t)320 << 20;
+inline bool from_memory(size_t known, size_t bytes) { return std::max(known, bytes) > FROM_MEMORY; }
+
+// Whether a launch of `bytes` of weights marks them as read once, which keeps their lines out of that cache.  us, unmarked / marked, weights from memory:
+// fp16 8x6656x6656 21.9 / 20.3, 24x4096x11008 22.9 / 21.6, 8x6656x17920 48.4 / 43.5; the same ones again and again 19.6 / 18.7, 19.8 / 20.4,
+// 40.5 / 42.5, 60 rows 42.5 / 48.1, 60x6656x6656 22.7 / 24.7.  Smaller launches' weights may stay there beside marked ones: eight fp16 layers of width 4096, 20 sequences, 1007 us a step with
+// Wo unmarked, 1024 with it marked (at width 2048, where nearly all are smaller, three layers 255 / 242).
+inline bool stream_once(bool memory, size_t bytes) { return memory && bytes >= (size_t)64 << 20; }
+
+// Wavefronts (of 16 columns) per workgroup of gemm_stream_kernel: one workgroup runs per compute unit, so the longest
+// compute unit has rounds * wavefronts of them to stream; below four a compute unit has too little in flight (8 rows, three
+// times 2048x2048: nine rounds of single wavefronts 19.6 us, one of ten 10.7).  *rounds: how many they are.
+inline int stream_waves(int N, int n_mats, int splits, long cus, int most, long* rounds) {
+  const long groups = (N + 15) / 16;
+  int best = 1;
+  long least = 0;
+  for (int w = 1; w <= most; ++w) {
+    const long wgs = (groups + w - 1) / w * n_mats * splits;
+    const long cost = (wgs + cus - 1) / cus * std::max(w, 4);
+    if (w == 1 || cost <= least) {
+      least = cost;
+      best = w;
+      *rounds = (wgs + cus - 1) / cus;
+    }
+  }
+  return best;
+}
+
+// How many workgroups the K stages of BM x 128 tiles are dealt to, and the workgroups in all; splits 0: too few of them, or no room for the sums.
+struct skinny_plan_t {
+  int splits;
+  long tiles;
+};
+inline skinny_plan_t plan_skinny(int BM, int M, int K, int N, int n_mats, int cus, size_t workspace_bytes) {
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + 127) / 128 * n_mats, nt_all = K / PLAN_STAGE;
+  // one workgroup per compute unit and at least four stages each: more, shorter splits only add
+  // partial sums (512 workgroups: 16 against 13 us at N = K = 4096)
+  int splits = (cus + tiles_m * tiles_n - 1) / (tiles_m * tiles_n);
+  splits = std::max(1, std::min(splits, nt_all / 4));
+  const size_t each = (size_t)M * N * n_mats * sizeof(float);
+  while (splits > 1 && splits * each > workspace_bytes) --splits;
+  if (splits * each > workspace_bytes || (long)tiles_m * tiles_n * splits < cus / 2) return {0, 0};
+  return {splits, (long)tiles_m * tiles_n * splits};
+}
+
+// Whether a product of few rows is one of gemm_stream_kernel, or of BM x 128 tiles of four wavefronts.  Of those several share a
+// compute unit; a workgroup here has it alone, so that a second round fills lhs and ring again with nothing beside it, which a long enough run
+// of stages pays for.  us with weights from memory, tiles / here: two rounds, fp16 8 rows of 32000 columns, K 2048, 2560, 4096, 6656 29.4 / 32.7, 33.6 / 31.0,
+// 62.2 / 54.7, 79.1 / 71.0, 24 rows 30.8 / 35.4, 43.2 / 41.0 (K 3072), 66.9 / 60.9, 64 rows of K 4096 71.9 / 68.0; uint8 32 rows, K 4096, 6656
+// 46.3 / 44.0, 70.1 / 61.9, 48 rows 76.3 / 76.2, 16 rows of 4096x11008 twice 36.6 / 32.7; three rounds, 5888x9664 three times 62 / 67.
+// One round: uint8 gains, but over short runs (15x512x10304 twice 10.3 / 11.4); fp16 where the tiles (`tiles` in all, with their splits) do not come out
+// even (27x17920x6656 62 / 45), or over runs of some stages (10x1024x7304 8.6 / 9.2; 24x4096x4096 13.3 / 13.3, 24x6144x4096 16.4 / 15.7, 20x11008x4096
+// 23.6 / 22.2, 20x8192x8192 36.5 / 33.0; 50 rows 18.3 / 18.3, 8192x4096 20.9 / 21.2, 8192x8192 64 rows 39.5 / 35.1).  bfloat16 gains at every count (4x512x3264
+// 9.2 / 7.9, 46x17920x6656 68 / 50).  Neither does for more than 16 rows over the shortest runs (28x512x16840 10.5 / 11.1, bfloat16
+// 56x512x16576 13.8 / 14.8).  Weights that may lie in a cache keep the lines that are right for them there (tiles / here from a cache: 64x8192x8192 26.6 / 34.0,
+// 20x8192x8192 23.7 / 30.8, 8x4096x32000 44.0 / 48.8; up to 16 rows of one round 10x1024x7304 7.4 / 8.3, 13x2048x2048 three times
+// 9.1 / 10.0).
+inline bool streams(int M, int N, int n_mats, int splits, int stages, long tiles, long cus, bool u8, bool bf16, bool memory) {
+  long rounds = 1;
+  stream_waves(N, n_mats, splits, cus, stream_max_waves(u8), &rounds);
+  const int run = stages / splits;
+  if (u8) return rounds == 1 || (rounds == 2 && (M <= 16 ? run >= 12 : memory && M <= 32 && run >= 20));
+  const bool short_runs = M > 16 && run <= 4;
+  if (bf16) return rounds == 1 && (!short_runs || 4 * tiles <= 3 * cus);
+  if (rounds == 1) return (tiles > cus && !short_runs) || (M <= 16 ? run >= 8 : memory && run >= (M <= 32 ? 12 : 24));
+  return memory && rounds == 2 && run >= 20;
 }
 
 }  // namespace lcu

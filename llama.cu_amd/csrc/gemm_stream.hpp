@@ -11,13 +11,13 @@
 // M = 8 with a launch that adds the splits, fp16 three times (4096, 4096) 26.0 -> 22.7 us, twice (N, K) = (11008, 4096) 45 -> 42,
 // (4096, 4096) 12.1 -> 12.4; uint8 three times (6656, 6656) 61 -> 35, twice (17920, 6656) 104 -> 57, (6656, 17920) 62 -> 37.  Rows of
 // 8 KB meet in the same memory channels: K = 4224 takes a tenth less than 4096.
-// Matrices from 64 MB up are marked as read once (nt), which keeps their lines out of the 256 MB cache in front of memory: 8 rows, twice 11008 columns
+// ONCE: weights that come from memory, 64 MB of them and more in a launch, are marked as read once (nt; stream_once).  8 rows, twice 11008 columns
 // of K 4096 36.8 -> 33.7 us (4.9 -> 5.35 TB/s), 16x4096x11008 22.4 -> 20.9, 60x6656x17920 53.6 -> 50.0; eight sequences of eight 7B layers, 45 + 16 tokens
-// 23.4 -> 22.1 ms.  A model of smaller ones may come back from that cache step after step, and would lose by it (weights of 67 MB in the cache 13.1 / 18.2 us
-// with the mark; uint8 5x6656x6656 12.3 / 13.7, from memory 14.9 / 14.3).
+// 23.4 -> 22.1 ms.
 #pragma once
 #include <algorithm>
 
+#include "gemm_plan.hpp"
 #include "gemm_tile.hpp"
 
 namespace lcu {
@@ -26,8 +26,6 @@ constexpr int STREAM_RING = 4;
 constexpr int STREAM_LHS = 64 * 1024;  // bytes of lhs in LDS: one chunk, or two of half of it
 // a unit is 16 rows of 128 bytes; uint8: and a word with the scales of each row
 constexpr int stream_unit(bool u8) { return 2048 + (u8 ? 256 : 0); }
-inline bool stream_once(int N, int K, int n_mats, bool u8) { return (size_t)N * K * n_mats * (u8 ? 1 : 2) >= (size_t)64 << 20; }
-constexpr int stream_max_waves(bool u8) { return u8 ? 10 : 12; }  // LDS: 160 KB
 constexpr int stream_lds(bool u8, int waves) { return STREAM_LHS + waves * STREAM_RING * stream_unit(u8); }
 // JOINED: lhs whole, and behind the product the sums of every wavefront in its place, [wavefront][row][16]; the rest for the rings
 constexpr int stream_joined_lhs(int waves, int row_tiles, int M, int K) {

@@ -40,7 +40,7 @@ workspace_t workspace_for(hipStream_t stream) {
   if (st == nullptr || !st->ready) {
     return workspace_t{};
   }
-  return workspace_t{st->workspace, st->workspace_bytes, st->workspace_sync, false};
+  return workspace_t{st->workspace, st->workspace_bytes, st->workspace_sync, false, 0};
 }
 
 device_state* current_device_state() {
@@ -282,6 +282,14 @@ int lcu_stream_destroy(void* stream) {
       LCU_HIP(hipFree(ws.ptr));
     }
   }
+  return LCU_OK;
+}
+
+int lcu_stream_weights(void* stream, size_t bytes) {
+  std::lock_guard<std::mutex> lock(g_stream_mutex);
+  auto it = g_stream_workspaces.find(as_stream(stream));
+  LCU_REQUIRE(stream != nullptr && it != g_stream_workspaces.end(), "lcu_stream_weights: not a stream of lcu_stream_create");
+  it->second.weights = bytes;
   return LCU_OK;
 }
 

@@ -18,6 +18,7 @@ struct llama_batch_context_impl final : public llama_batch_context {
     LCU_CHECK(lcu_init(0));
     device_structure_lock lock(device_structure_mutex());
     LCU_CHECK(lcu_stream_create(&stream_));
+    LCU_CHECK(lcu_stream_weights(stream_, model_->weight_bytes()));
     for (int b = 0; b < n_sequences; ++b) {
       seqs_.push_back(std::make_unique<llama_context_impl>(model, context_len, temperature));
     }

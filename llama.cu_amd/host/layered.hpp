@@ -148,6 +148,7 @@ struct layered_model_impl : public llama_model {
   layered_model_impl(layered_params const& p, element_type type);
   std::unique_ptr<llama_context> make_context(int context_len, float temperature) override;
   int max_context() const override;
+  size_t weight_bytes() const;  // of the matrices that a call goes through, every expert's among them
 
   layered_params shape;
   int dtype;        // LCU_BF16 or LCU_F32

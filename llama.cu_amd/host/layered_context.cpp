@@ -28,6 +28,7 @@ layered_context_impl::layered_context_impl(layered_model_impl* model, int contex
   device_structure_lock lock(device_structure_mutex());
   LCU_CHECK(lcu_init(0));
   LCU_CHECK(lcu_stream_create(&stream_));
+  LCU_CHECK(lcu_stream_weights(stream_, model_->weight_bytes()));
   layered_model_impl const& m = *model_;
   const size_t R = rows_, e = m.elem, ctx = context_len_;
   size_t low = 0, queries = 0, latent_queries = 0, keys_values = 0, tail = 0;

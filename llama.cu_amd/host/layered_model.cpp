@@ -453,6 +453,18 @@ bool layered_model_impl::shapes_supported() const {
   return true;
 }
 
+size_t layered_model_impl::weight_bytes() const {
+  size_t count = head.size();
+  for (layer_weights const& l : layers) {
+    for (gpu_buffer const* b : {&l.recurrence.yx, &l.recurrence.gate_r, &l.recurrence.gate_i, &l.recurrence.out, &l.attention.qkv, &l.attention.out,
+                                &l.latent.in, &l.latent.uq, &l.latent.ukv, &l.latent.out, &l.delta.in, &l.delta.out, &l.dense.up, &l.dense.down,
+                                &l.mlp.router, &l.mlp.up, &l.mlp.down, &l.mlp.shared_up, &l.mlp.shared_down}) {
+      count += b->size();
+    }
+  }
+  return count;
+}
+
 int layered_model_impl::max_context() const {
   // the fp32 attention kernel keeps the scores of every visible key
   if (dtype == LCU_F32) {

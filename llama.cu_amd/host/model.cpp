@@ -165,6 +165,14 @@ void llama_model_impl::synthesize(uint64_t seed, float std) {
   LCU_CHECK(lcu_sync(nullptr));
 }
 
+size_t llama_model_impl::weight_bytes() const {
+  size_t count = output.data.size() + output.scales.size();
+  for (llama_layer const& l : layers) {
+    for (weight_tensor const* t : {&l.wq, &l.wk, &l.wv, &l.wo, &l.w1, &l.w2, &l.w3}) count += t->data.size() + t->scales.size();
+  }
+  return count;
+}
+
 weight_tensor const* llama_model_impl::tensor_by_stream(uint64_t stream_id) const {
   if (stream_id == 1) return &tok_embeddings;
   if (stream_id == 2) return &output;
@@ -238,6 +246,7 @@ llama_context_impl::llama_context_impl(llama_model* model, int context_len, floa
   device_structure_lock lock(device_structure_mutex());
   LCU_CHECK(lcu_init(0));
   LCU_CHECK(lcu_stream_create(&stream_));
+  LCU_CHECK(lcu_stream_weights(stream_, model_->weight_bytes()));
   lcu_device_props props;
   LCU_CHECK(lcu_device_get_props(0, &props));
   compute_units_ = props.compute_units;

@@ -36,6 +36,7 @@ struct llama_model_impl : public llama_model {
   weight_tensor const* tensor_by_stream(uint64_t stream_id) const;
   std::unique_ptr<llama_context> make_context(int context_len, float temperature) override;
   int max_context() const override { return LLAMA_CU_MAX_CONTEXT; }
+  size_t weight_bytes() const;  // of the matrices that every call goes through
   weight_tensor tok_embeddings;
   weight_tensor output;
   gpu_buffer norm;

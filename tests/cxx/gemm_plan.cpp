@@ -37,6 +37,17 @@ void tile_size(int M, int N, int each, int largest_rows, int largest_columns, in
   out[1] = t.columns;
 }
 
+// 2 to 64 rows: splits, whether gemm_stream_kernel takes it, whether its weights are marked as read once
+void few_rows(int u8, int bf16, int M, int K, int N, int n_mats, long known, long cus, long workspace, int* out) {
+  const int tile = M <= 32 || u8 != 0 ? 32 : 64;
+  skinny_plan_t p = plan_skinny(tile, M, K, N, n_mats, (int)cus, (size_t)workspace);
+  const size_t bytes = (size_t)N * K * n_mats * (u8 != 0 ? 1 : 2);
+  const bool memory = from_memory((size_t)known, bytes);
+  out[0] = p.splits;
+  out[1] = p.splits > 0 && streams(M, N, n_mats, p.splits, K / PLAN_STAGE, p.tiles, cus, u8 != 0, bf16 != 0, memory);
+  out[2] = out[1] && stream_once(memory, bytes);
+}
+
 int expert_rows(long rows, int experts, int K, int ff, long cus) { return plan_expert_rows(rows, experts, K, ff, cus); }
 
 int attention_again(int n_heads, int n_new, int start_pos, long cus) { return scores_again(n_heads, n_new, start_pos, cus); }

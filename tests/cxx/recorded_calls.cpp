@@ -5,7 +5,7 @@
 #include <string.h>
 #include <unistd.h>
 
-#include <string>
+#include <map>
 #include <utility>
 #include <vector>
 
@@ -20,6 +20,7 @@ std::vector<noted> calls;
 std::vector<std::pair<int*, int>> answers, of_graph;
 bool capturing = false;
 long lateness = -1;
+std::map<void*, size_t> weights;
 size_t next_address = 4096;
 
 int note(const char* name, void* stream) {
@@ -45,6 +46,8 @@ int recorded_count() { return (int)calls.size(); }
 const char* recorded_name(int i) { return calls[i].name; }
 void* recorded_stream(int i) { return calls[i].stream; }
 
+size_t recorded_weights(void* stream) { return weights.count(stream) ? weights[stream] : 0; }
+
 const char* lcu_last_error(void) { return ""; }
 int lcu_malloc(void** out, size_t bytes) {
   *out = (void*)next_address;
@@ -63,6 +66,10 @@ int lcu_stream_create(void** out) { return lcu_malloc(out, 1); }
 int lcu_device_get_props(int, lcu_device_props* p) {
   memset(p, 0, sizeof(*p));
   p->compute_units = 256;
+  return 0;
+}
+int lcu_stream_weights(void* stream, size_t bytes) {
+  weights[stream] = bytes;
   return 0;
 }
 int lcu_sync_timeouts(void*, unsigned* out) {

@@ -22,10 +22,11 @@ def _lib():
     lib.rows.argtypes = [i, i, i, i, w, w, C.POINTER(i)]
     lib.left_sums.argtypes = [i, i, i, i, w, w, i, C.POINTER(i)]
     lib.tile_size.argtypes = [i, i, i, i, i, i, w, C.POINTER(i)]
+    lib.few_rows.argtypes = [i, i, i, i, i, i, w, w, w, C.POINTER(i)]
     lib.large.argtypes = [i, i, i, i, i, w, i, C.POINTER(i)]
     lib.attention_again.argtypes = [i, i, i, w]
     lib.expert_rows.argtypes = [w, i, i, i, w]
-    lib.rows.restype = lib.left_sums.restype = lib.large.restype = lib.tile_size.restype = None
+    lib.rows.restype = lib.left_sums.restype = lib.large.restype = lib.tile_size.restype = lib.few_rows.restype = None
     os.unlink(path)
     os.rmdir(folder)
     return lib
@@ -57,6 +58,13 @@ def tile_size(M, N, each, largest, narrowest, cus=CUS):
     out = (C.c_int * 2)()
     _lib().tile_size(M, N, each, *largest, int(narrowest), cus, out)
     return tuple(out)
+
+
+def few_rows(kind, M, K, N, n_mats=1, known=0, cus=CUS, workspace=WORKSPACE):
+    """(splits, whether gemm_stream_kernel takes it, whether it marks its weights as read once); known: bytes of weights that a program goes through"""
+    out = (C.c_int * 3)()
+    _lib().few_rows(kind == "u8", kind == "bf16", M, K, N, n_mats, known, cus, workspace, out)
+    return out[0], bool(out[1]), bool(out[2])
 
 
 def scores_again(heads, n, T, cus=CUS):

@@ -17,6 +17,7 @@ sys.path.insert(0, {tests!r})
 stand_in = C.CDLL({library!r}, os.RTLD_GLOBAL | os.RTLD_NOW)
 stand_in.recorded_name.restype = C.c_char_p
 stand_in.recorded_stream.restype = C.c_void_p
+stand_in.recorded_weights.argtypes, stand_in.recorded_weights.restype = [C.c_void_p], C.c_size_t
 import lcu
 P = lcu.package()
 def calls():

@@ -79,6 +79,30 @@ def test_gated_linear_large_tiles(gpu, M, K, ff):
     gpu.release()
 
 
+# few rows of weights that come from memory, marked as read once: one launch with what follows (6 and 5 rows) and two, one to four row tiles, ragged columns
+@pytest.mark.parametrize("gated,M,K,N", [(False, 6, 4096, 8301), (False, 16, 4096, 8300), (False, 30, 4096, 8300), (False, 60, 4096, 8300), (False, 9, 1024, 33000),
+                                         (True, 5, 4096, 4160), (True, 15, 4096, 4160), (True, 31, 2048, 8320), (True, 50, 4096, 4224)])
+def test_linear_of_weights_from_memory(gpu, gated, M, K, N):
+    known, outs = 13 << 30, up64(N)
+    assert gemm_plan.few_rows("bf16", M, K, 2 * outs if gated else N, known=known)[1:] == (True, True)
+    rng = np.random.default_rng(M)
+    x = rounded(rng.standard_normal((M, K)))
+    ws = [rounded(rng.standard_normal((N, K)) / K ** 0.5) for _ in range(2 if gated else 1)]
+    xd, wd, gate = put(gpu, x, BF16), put(gpu, pack_gated(*ws, outs) if gated else ws[0], BF16), gpu.B.GateParams(7.0, 1.702, 1.0)
+    results = []
+    for bytes_known in (known, 0):
+        gpu.B.check(gpu.L().lcu_stream_weights(gpu.stream, bytes_known))
+        out = zeros(gpu, (M, outs), BF16 if gated else F32)
+        if gated:
+            call(gpu, "lcu_linear_gated", out, outs, xd, wd, C.byref(gate), BF16, M, K, 2 * outs)
+        else:
+            call(gpu, "lcu_linear", out, 1, outs, xd, wd, None, 0, BF16, M, K, N)
+        results.append(get(gpu, out, (M, outs), BF16 if gated else F32)[:, :N])
+    assert (results[0] == results[1]).all()
+    close(results[0], S.expert(x, *ws, np.eye(N), 7.0) if gated else x @ ws[0].T, BF16 if gated else F32)
+    gpu.release()
+
+
 # products of 65 and more rows with few tiles over a long K, whose K is never split: a layer's roundings decide which experts a token takes, so the
 # order of the sums hangs neither on the stream nor on its workspace
 @pytest.mark.parametrize("gated", [False, True])

@@ -378,7 +378,7 @@ def test_gemm_u8(gpu, M, K, N):
 # chunks, one and two scales in 128 codes, and a block that takes the other kernel
 @pytest.mark.parametrize("M,K,N,block", [(2, 1152, 520, 64), (16, 1152, 4100, 128), (17, 2560, 1000, 256), (33, 1152, 5000, 64),
                                          (64, 5888, 4100, 128), (64, 1152, 3000, 384), (7, 17920, 6656, 128),
-                                         (16, 512, 32000, 128), (17, 512, 32000, 64), (20, 2560, 31010, 128)])  # two rounds of workgroups, both kernels
+                                         (16, 512, 32000, 128), (17, 512, 32000, 64), (20, 2560, 31010, 128)])  # two rounds of workgroups
 def test_gemm_u8_few_rows(gpu, M, K, N, block):
     G = gpu
     x, w = normal((M, K), 0, 430, 1.0), normal((N, K), 0, 431, 0.02)
@@ -392,13 +392,99 @@ def test_gemm_u8_few_rows(gpu, M, K, N, block):
 @pytest.mark.parametrize("M,K,N", [(3, 1152, 520), (16, 1408, 4099), (31, 2944, 1000), (48, 5888, 4100), (64, 4096, 24000),
                                    (16, 5760, 4099), (31, 5760, 4099), (24, 4096, 4096), (28, 512, 16840),  # 264, 264, 256 and 264 tiles
                                    (8, 512, 32000), (40, 640, 31000),  # two rounds of workgroups: the other kernel
-                                   (20, 2560, 31010), (24, 6144, 4099)])  # two rounds of long runs, one of them: this one
+                                   (20, 2560, 31010), (24, 6144, 4099)])  # two rounds of long runs, one of them: weights from memory decide
 def test_gemm_f16_few_rows(gpu, M, K, N):
     G = gpu
     x, w, old = normal((M, K), 0, 440, 1.0), normal((N, K), 0, 441, 0.02), normal((M, N), 0, 442, 1.0)
     assert G.ulp_mismatch(G.gemm_f16(x, w), O.matmul_nt(x, w, flavour=2)) == 0.0, O.gemm_plan(M, K, N)
     assert G.ulp_mismatch(G.gemm_f16(x, w, beta=1.0, out=old), O.matmul_nt(x, w, beta=1.0, out=old, flavour=2)) == 0.0
     G.release()
+
+
+MODEL = 13 << 30  # bytes of weights between two uses of the same ones
+
+
+@pytest.fixture
+def model_stream(gpu):
+    """A stream whose weights come from memory."""
+    stream = gpu.B.vp()
+    gpu.B.check(gpu.L().lcu_stream_create(C.byref(stream)))
+    gpu.B.check(gpu.L().lcu_stream_weights(stream, MODEL))
+    yield stream
+    gpu.B.check(gpu.L().lcu_stream_destroy(stream))
+
+
+# weights marked as read once, on a model's stream, against the oracle and against a stream that says nothing: one to four row tiles with a ragged last one, columns
+# past the last whole sixteen, sums that are added up where they end and sums that are not, two rounds of workgroups
+@pytest.mark.parametrize("kind,M,K,N,mats", [("f16", 3, 4096, 8300, 1), ("f16", 16, 5760, 6001, 1), ("f16", 24, 6144, 5500, 1), ("f16", 31, 2944, 11500, 1),
+                                             ("f16", 40, 8192, 4101, 1), ("f16", 63, 4096, 8300, 1), ("f16", 20, 2560, 31010, 1), ("f16", 7, 4096, 2902, 3),
+                                             ("f16", 45, 4096, 4104, 2), ("u8", 5, 6656, 10102, 1), ("u8", 20, 6656, 10102, 1), ("u8", 33, 6656, 10102, 1),
+                                             ("u8", 60, 17920, 4006, 1), ("u8", 64, 5888, 11502, 1), ("u8", 9, 4096, 5502, 3), ("u8", 48, 6656, 5102, 2),
+                                             ("u8", 17, 2560, 31010, 1)])
+def test_few_rows_of_weights_from_memory(gpu, model_stream, kind, M, K, N, mats):
+    import gemm_plan
+    G = gpu
+    check, L, VP = G.B.check, G.L(), G.B.vp
+    assert gemm_plan.few_rows(kind, M, K, N, mats, known=MODEL)[1:] == (True, True) and not gemm_plan.few_rows(kind, M, K, N, mats)[2]
+    x, ws = normal((M, K), 0, 460, 1.0), [normal((N, K), 0, 461 + g, 0.02) for g in range(mats)]
+    codes = [O.quantize_absmax_u8(w, 128) for w in ws] if kind == "u8" else []
+    xd, wd = G.dev_keep(x), [G.dev_keep(c[0]) for c in codes] or [G.dev_keep(w) for w in ws]
+    sd, results = [G.dev_keep(c[1]) for c in codes], []
+    for stream in (model_stream, None):
+        outs = [G.empty((M, N)) for _ in range(mats)]
+        arr = lambda items: (VP * mats)(*[i.ptr for i in items])
+        if codes:
+            check(L.lcu_gemm_f16u8_nt_multi(arr(outs), xd.ptr, arr(wd), arr(sd), mats, M, K, N, 128, 0.0, stream))
+        else:
+            check(L.lcu_gemm_f16_nt_multi(arr(outs), xd.ptr, arr(wd), mats, M, K, N, 0.0, stream))
+        check(L.lcu_sync(stream))
+        results.append([G.host(o, (M, N)) for o in outs])
+        for o in outs:
+            o.free()
+    for g in range(mats):
+        want = O.matmul_nt_kernel_order(x, codes=codes[g][0], scales=codes[g][1], block=128, n_mats=mats) if codes else \
+            O.matmul_nt_kernel_order(x, ws[g], n_mats=mats)
+        assert G.ulp_mismatch(results[0][g], want) == 0.0
+        assert (results[0][g].view(np.uint16) == results[1][g].view(np.uint16)).all()
+    G.release()
+
+
+@pytest.mark.parametrize("B,u8", [(2, False), (9, False), (20, False), (50, False), (9, True), (40, True)])
+def test_batch_steps_of_weights_from_memory(gpu, model_stream, B, u8):
+    """The fused steps of a batch, their weights marked as read once, against the same on a stream that says nothing, bit for bit."""
+    G = gpu
+    check, L, VP = G.B.check, G.L(), G.B.vp
+    dim, heads, ffn, ctx, block = (4992, 39, 13568, 8, 128) if u8 else (4096, 32, 8320, 8, 0)
+    table = VP()
+    check(L.lcu_rope_table_create(G.B.C.byref(table), ctx, dim // heads, 10000.0))
+
+    def weights(rows, cols, stream):
+        w = normal((rows, cols), 0, stream, 0.02)
+        return [G.dev_keep(a) for a in (O.quantize_absmax_u8(w, block) if u8 else (w,))]
+
+    qkv, up, w2 = [weights(dim, dim, 470 + g) for g in range(3)], [weights(ffn, dim, 480 + g) for g in range(2)], weights(dim, ffn, 490)
+    arr = lambda items, at=0: (VP * len(items))(*[i[at].ptr for i in items])
+    x, h, nw = normal((B, dim), 0, 491, 1.0), G.dev_keep(normal((B, ffn), 0, 492, 0.5)), G.dev_keep(normal((dim,), 0, 493, 1.0))
+    xd, pos, results = G.dev_keep(x), G.dev_keep(np.arange(B, dtype=np.int32) % ctx), []
+    for stream in (model_stream, None):
+        kc, vc = [G.dev_keep(np.zeros((ctx, dim), np.float16)) for _ in range(B)], [G.dev_keep(np.zeros((ctx, dim), np.float16)) for _ in range(B)]
+        kp, vp = (G.dev_keep(np.array([c.ptr for c in cs], dtype=np.uint64)) for cs in (kc, vc))
+        q, k, v, t1, t3, act, norm, res = [G.dev_keep(np.zeros((B, n), np.float16)) for n in (dim, dim, dim, ffn, ffn, ffn, dim)] + [G.dev_keep(x)]
+        check(L.lcu_batch_qkv(q.ptr, k.ptr, v.ptr, xd.ptr, arr(qkv), arr(qkv, 1) if u8 else None, block, B, dim, heads, kp.ptr, vp.ptr, pos.ptr, table, ctx, stream))
+        check(L.lcu_batch_ffn_up(act.ptr, t1.ptr, t3.ptr, xd.ptr, arr(up), arr(up, 1) if u8 else None, block, B, dim, ffn, stream))
+        check(L.lcu_batch_proj_norm(res.ptr, norm.ptr, h.ptr, w2[0].ptr, w2[1].ptr if u8 else None, block, B, ffn, dim, nw.ptr, 1e-6, stream))
+        check(L.lcu_sync(stream))
+        results.append([G.host(q, (B, dim)), G.host(act, (B, ffn)), G.host(res, (B, dim)), G.host(norm, (B, dim))] + [G.host(c, (ctx, dim)) for c in kc + vc])
+    for a, b in zip(*results):
+        assert (a.view(np.uint16) == b.view(np.uint16)).all() and np.abs(a.astype(np.float32)).max() > 0
+    G.release()
+    L.lcu_free(table)
+
+
+def test_only_streams_of_the_library_take_a_size_of_weights(gpu, model_stream):
+    L = gpu.L()
+    assert L.lcu_stream_weights(None, 1) != 0 and b"lcu_stream_weights" in L.lcu_last_error()
+    assert L.lcu_stream_weights(model_stream, 0) == 0
 
 
 # few rows whose splits are added up where they end: one to four row tiles, workgroups that hold the last columns of one matrix and the first of

@@ -64,3 +64,22 @@ result = tokens, quick, late, names()
 """)
     assert tokens == [7] * 7 and late == 2 * ["lcu_graph_launch", "lcu_sync"]
     assert quick == again == ["lcu_graph_launch"]
+
+
+def test_contexts_say_what_their_models_hold():
+    """Every stream of a context or a batch knows the bytes of the matrices that a call goes through, before its first launch."""
+    weights = recorded_calls.run("""
+model = tiny_model()
+context, batch = P.Context(model, context_len=64), P.BatchContext(model, 2, context_len=64)
+calls()
+context.next_token([1, 2]); batch.next_token(0, [1, 2]); batch.next_token(1, [1, 2]); batch.next_tokens([1, 2])
+of_llama = sorted({s for name, s in calls() if name.startswith("lcu_softmax")})
+layered = P.Model(config={"architecture": "Logivik", "vocab": 301, "width": 64, "embedding": {"scale": 8.0}, "norm": {"eps": 1e-5}, "layers": [
+    {"type": "latent_attention_2", "mlp": {"kind": "dense", "ff": 128},
+     "mixer": {"heads": 2, "dim": 32, "vdim": 32, "kv_rank": 32, "q_rank": 32, "scale": 0.2, "mask": {"size": 64}}}]}, seed=4)
+other = P.Context(layered, context_len=96)
+result = [stand_in.recorded_weights(s) for s in of_llama], stand_in.recorded_weights(P.lib().lcu_context_stream(other.h))
+""")
+    dim, ffn = 256, 768
+    assert weights[0] == 4 * [2 * (2 * (4 * dim * dim + 3 * dim * ffn) + 512 * dim)]
+    assert weights[1] > 2 * (301 * 64 + 3 * 64 * 128)
