@@ -1873,9 +1873,19 @@ int gemm_bf16_grouped(linear_epilogue<true, GATED> const& ep, const void* A, con
     if (few && ep.tile_rows == 256 && K <= 512) return launch_bf16<256, 128, 4, 2, 1, 3>(ep, A, W, max_tiles, 0, K, N, st);
     if (few && ep.tile_rows == 128 && K <= 2048) return launch_bf16<128, 128, 4, 2, 1, 3>(ep, A, W, max_tiles, 0, K, N, st);
   }
-  if (ep.tile_rows == 256) return launch_tile<256, 128, 4, 2, 3, 3, false, false>(ep, op, A, max_tiles * 256, K, N, 0, 0.0f, st);
-  if (ep.tile_rows == 128) return launch_tile<128, 128, 2, 2, 4, 4, false, false>(ep, op, A, max_tiles * 128, K, N, 0, 0.0f, st);
-  return launch_bf16<64, 128, 2, 2, 1, 3>(ep, A, W, max_tiles, 0, K, N, st);
+  if (ep.tile_rows == 64) return launch_bf16<64, 128, 2, 2, 1, 3>(ep, A, W, max_tiles, 0, K, N, st);
+  const auto tiles = [&](auto const& e) {
+    if (ep.tile_rows == 256) return launch_tile<256, 128, 4, 2, 3, 3, false, false>(e, op, A, max_tiles * 256, K, N, 0, 0.0f, st);
+    return launch_tile<128, 128, 2, 2, 4, 4, false, false>(e, op, A, max_tiles * 128, K, N, 0, 0.0f, st);
+  };
+  // Weights that come from memory are marked as read once, whatever the rows to an expert: one that takes two row tiles asks for its lines in both at the same
+  // time.  us, both products, unmarked / marked, from memory: top 2 of 16 of 2816, 4096 wide, 512 tokens 240 / 230, 1000 291 / 285, 2010 412 / 395, 4000 (500
+  // rows to an expert) 636 / 617; top 4 of 64 of 704, 2048 wide, 1000 161 / 151, 4000 259 / 248.  Those that may lie in the cache are not: top 2 of 8 of 512,
+  // 1024 wide (25 MB), again and again 1000 27.0 / 28.5, 2010 35.3 / 37.4, 4000 65 / 70.
+  if (!from_memory(workspace_for(st).weights, 0)) return tiles(ep);
+  read_once<GATED> marked;
+  static_cast<linear_epilogue<true, GATED>&>(marked) = ep;
+  return tiles(marked);
 }
 template int gemm_bf16_grouped<false>(linear_epilogue<true, false> const&, const void*, const void*, int, int, int, hipStream_t);
 template int gemm_bf16_grouped<true>(linear_epilogue<true, true> const&, const void*, const void*, int, int, int, hipStream_t);

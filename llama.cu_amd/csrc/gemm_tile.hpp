@@ -224,8 +224,8 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN + 3) / 4) void gemm_tile_ker
                  "s"(lds0 + at)
                  : "memory", "m0");
   };
-  // Lines that hardly another tile asks for: the columns of experts, whose rows mostly fit one tile (512 tokens, top 2 of 16 of 4096 x 5632, six layers
-  // of Rirulix 3335 -> 3225 us).  Other products' columns stay in the caches: 7B prompts gain 0.5 %, a product called again loses a third.
+  // marked as read once: the columns of experts that come from memory (read_once).  Other products' columns stay in the caches: 7B prompts gain 0.5 %, a product
+  // called again loses a third.
   const auto request_once = [&](uint4_t resource, uint32_t stage_bytes, uint32_t offset, uint32_t at) {
     asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(offset), "s"(resource), "s"(stage_bytes),
                  "s"(lds0 + at)
@@ -237,7 +237,11 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN + 3) / 4) void gemm_tile_ker
       request(ra, stage_offset(ra[2], stage_of(a) * 128u), a_off[i], a_slot * A_STEP + (wave + i * NW) * 1024);
     } else if (i < PA + PB) {
       const uint32_t along = stage_offset(rw[2], stage_of(b) * (U8 ? 64u : 128u)), at = W_RING + b_slot * W_STEP + (wave + (i - PA) * NW) * 1024;
-      if constexpr (EP::GROUPED) {
+      constexpr bool ONCE = [] {
+        if constexpr (EP::GROUPED) return EP::ONCE;
+        return false;
+      }();
+      if constexpr (ONCE) {
         request_once(rw, along, b_off[i - PA], at);
       } else {
         request(rw, along, b_off[i - PA], at);

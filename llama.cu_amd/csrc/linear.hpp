@@ -71,7 +71,7 @@ __device__ __forceinline__ group_tile_t group_tile(const row_groups<true>& g, in
 // GATED: the matrix holds, in blocks of 64 rows, 32 gate rows and the 32 up rows of the same hidden columns.
 template <bool GROUPED_, bool GATED_>
 struct linear_epilogue : row_groups<GROUPED_> {
-  static constexpr bool BF16 = true, GROUPED = GROUPED_, GATED = GATED_, ROTARY = false, PAIRED = false;
+  static constexpr bool BF16 = true, GROUPED = GROUPED_, GATED = GATED_, ROTARY = false, PAIRED = false, ONCE = false;
   void* out;
   int ldo;
   bool out_f32;
@@ -140,6 +140,12 @@ struct linear_epilogue : row_groups<GROUPED_> {
     }
     put(m, n, gate(g, u));
   }
+};
+
+// experts whose weights come from memory: their lines are marked as read once (gemm_bf16_grouped)
+template <bool GATED>
+struct read_once : linear_epilogue<true, GATED> {
+  static constexpr bool ONCE = true;
 };
 
 // gemm.hip

@@ -635,7 +635,8 @@ def test_experts_in_tiles_of_any_height(gpu, n, K, ff, experts, top):
     choice = ints(gpu, np.stack([rng.permutation(experts)[:top] for _ in range(n)]))
     weight, g = put(gpu, rng.random((n, top))), gpu.B.GateParams(0.8, 1.702, 1.0)
     got = []
-    for tile in (64, 128, 256):
+    for tile, known in ((64, 0), (128, 0), (256, 0), (128, 13 << 30), (256, 13 << 30)):  # with weights from memory they are marked as read once
+        gpu.B.check(gpu.L().lcu_stream_weights(gpu.stream, known))
         plan, keep, max_tiles = gpu.B.ExpertPlan(), {}, rows // tile + experts
         for name, count in (("row_token", rows), ("row_weight", rows), ("inverse", rows), ("tile_expert", max_tiles), ("tile_row", max_tiles),
                             ("expert_end", experts), ("n_tiles", 1)):
@@ -648,7 +649,8 @@ def test_experts_in_tiles_of_any_height(gpu, n, K, ff, experts, top):
         call(gpu, "lcu_experts_down", out, N, hidden, down, N * ld * 2, C.byref(plan), BF16, rows, ld, N)
         got.append(get(gpu, out, (rows, N))[get_ints(gpu, keep["inverse"], (rows,))])
     assert np.isfinite(got[0]).all() and np.abs(got[0]).max() > 0.1
-    assert (got[0] == got[1]).all() and (got[0] == got[2]).all()
+    gpu.B.check(gpu.L().lcu_stream_weights(gpu.stream, 0))
+    assert all((got[0] == g).all() for g in got[1:])
     gpu.release()
 
 
