@@ -1836,8 +1836,9 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
   }
   if (tm(128) * tn(128) >= 160) return launch_tile<128, 128, 2, 2, 4, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
   if constexpr (GATED) {
-    // us, below / here: 100 rows of 11264 columns, K 1536, 1792, 2048 17.6 / 17.7, 19.4 / 18.6, 20.9 / 19.3, 100x4096x5632 32.7 / 29.4, 100x2048x2816 18.5 / 17.4
-    if (K >= 1792) return launch_tile<128, 64, 2, 1, 4, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
+    if (gated_on_tiles(M, K, N, cus, from_memory(workspace_for(st).weights, (size_t)N * K * 2))) {
+      return launch_tile<128, 64, 2, 1, 4, 4, false, false>(ep, single_matrix(nullptr, W, nullptr), A, M, K, N, 0, 0.0f, st);
+    }
     if (tm(128) * tn(64) > 128) return launch_bf16<128, 64, 4, 1, 1, 3>(ep, A, W, tm(128), M, K, N, st);
     return launch_bf16<64, 64, 2, 1, 1, 3>(ep, A, W, tm(64), M, K, N, st);
   } else {

@@ -68,6 +68,13 @@ inline tile_size_t plan_tile_size(int M, int N, int each, tile_size_t largest, b
   return largest;
 }
 
+// Whether a gated product of less than 160 tiles of 128x128 takes 128x64 tiles of gemm_tile_kernel or smaller ones of gemm_dl_kernel.  The former's ring of four
+// stages hides the way from memory over a long K, but leaves a compute unit one workgroup: weights that may lie in a cache, and more tiles than one
+// round, are sooner with the latter.  us, gemm_dl_kernel / gemm_tile_kernel, from memory: 100 rows of 11264 columns, K 1536, 1792, 2048 17.6 / 17.7, 19.4 / 18.6,
+// 20.9 / 19.3, 258x4096x768 30.7 / 28.0, 133x8192x6656 60.7 / 51.1, 71x17920x5504 124 / 104; 327x3072x5632 (264 tiles) 30.5 / 43.8, 637x1792x3456 (270) 20.0 /
+// 30.1.  The same weights again and again 258x4096x768 24.7 / 27.9, 134x5632x3200 32.6 / 36.6, 378x8192x4096 49.6 / 53.3, 309x2048x5632 (264) 21.6 / 33.9.
+inline bool gated_on_tiles(int M, int K, int N, long cus, bool memory) { return memory && K >= 1792 && tiles_of(M, N, 128, 64) <= cus; }
+
 // Which columns of a product a launch of gemm_tile_kernel takes: the first `tiles` tiles along N, counted through the matrices
 // (0: all of them), or those from column `from` of the last matrix on.
 struct columns_t {

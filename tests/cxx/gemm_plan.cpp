@@ -48,6 +48,9 @@ void few_rows(int u8, int bf16, int M, int K, int N, int n_mats, long known, lon
   out[2] = out[1] && stream_once(memory, bytes);
 }
 
+// whether weights of which a program goes through `known` bytes are those of a gated product on gemm_tile_kernel
+int gated_tiles(int M, int K, int N, long known, long cus) { return gated_on_tiles(M, K, N, cus, from_memory((size_t)known, (size_t)N * K * 2)); }
+
 int expert_rows(long rows, int experts, int K, int ff, long cus) { return plan_expert_rows(rows, experts, K, ff, cus); }
 
 int attention_again(int n_heads, int n_new, int start_pos, long cus) { return scores_again(n_heads, n_new, start_pos, cus); }

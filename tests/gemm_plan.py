@@ -23,6 +23,7 @@ def _lib():
     lib.left_sums.argtypes = [i, i, i, i, w, w, i, C.POINTER(i)]
     lib.tile_size.argtypes = [i, i, i, i, i, i, w, C.POINTER(i)]
     lib.few_rows.argtypes = [i, i, i, i, i, i, w, w, w, C.POINTER(i)]
+    lib.gated_tiles.argtypes = [i, i, i, w, w]
     lib.large.argtypes = [i, i, i, i, i, w, i, C.POINTER(i)]
     lib.attention_again.argtypes = [i, i, i, w]
     lib.expert_rows.argtypes = [w, i, i, i, w]
@@ -65,6 +66,11 @@ def few_rows(kind, M, K, N, n_mats=1, known=0, cus=CUS, workspace=WORKSPACE):
     out = (C.c_int * 3)()
     _lib().few_rows(kind == "u8", kind == "bf16", M, K, N, n_mats, known, cus, workspace, out)
     return out[0], bool(out[1]), bool(out[2])
+
+
+def gated_tiles(M, K, N, known=0, cus=CUS):
+    """Whether a gated product of less than 160 tiles of 128x128 takes gemm_tile_kernel; known: as above"""
+    return bool(_lib().gated_tiles(M, K, N, known, cus))
 
 
 def scores_again(heads, n, T, cus=CUS):

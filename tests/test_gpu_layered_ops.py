@@ -186,10 +186,16 @@ def test_gated_linear_columns_left_of_whole_rounds(gpu, M, K, ff, plan):
     test_gated_linear_large_tiles(gpu, M, K, ff)
 
 
-# gated outputs of few 128x64 tiles, either side of K = 1792
+# gated outputs of few 128x64 tiles, either side of K = 1792 where weights come from memory, and where they may not
+@pytest.mark.parametrize("known", [0, 13 << 30])
 @pytest.mark.parametrize("M,K,ff", [(66, 1728, 1500), (66, 1792, 1500), (129, 1856, 2000), (200, 2048, 70)])
-def test_gated_linear_few_tiles(gpu, M, K, ff):
-    test_gated_linear_large_tiles(gpu, M, K, ff)
+def test_gated_linear_few_tiles(gpu, M, K, ff, known):
+    assert gemm_plan.gated_tiles(M, K, 2 * up64(ff), known) == (K >= 1792 and known > 0)
+    gpu.B.check(gpu.L().lcu_stream_weights(gpu.stream, known))
+    try:
+        test_gated_linear_large_tiles(gpu, M, K, ff)
+    finally:
+        gpu.B.check(gpu.L().lcu_stream_weights(gpu.stream, 0))
 
 
 # gated outputs of 192 columns: one round of them, ragged ends, a short K
