@@ -986,6 +986,20 @@ size_t weight_bytes(const operands_t& op, int K, int N) {
   return (size_t)N * K * (U8 ? 1 : 2) * op.n_mats;
 }
 
+// whether an output lies over lhs
+inline bool over_lhs(const operands_t& op, const void* A, int M, int K, int N) {
+  for (const void* o : {(const void*)op.out, (const void*)op.more.out[0], (const void*)op.more.out[1]}) {
+    if (o != nullptr && overlap(o, (size_t)M * N * 2, A, (size_t)M * K * 2)) return true;
+  }
+  return false;
+}
+template <bool GATED>
+bool over_lhs(linear_epilogue<false, GATED> const& ep, const void* A, int M, int K, int N) {
+  const size_t lhs_bytes = (size_t)M * K * 2, row = GATED ? N / 2 : N;
+  return overlap(ep.out, ((size_t)(M - 1) * ep.ldo + row) * (ep.out_f32 ? 4 : 2), A, lhs_bytes) ||
+         (ep.tail && overlap(ep.tail, ((size_t)(M - 1) * ep.ld_tail + (N - ep.tail_from)) * 4, A, lhs_bytes));
+}
+
 // where a split-K launch left its partial sums: part[matrix][split][M][N] fp32
 struct partial_sums_t {
   const float* part;
@@ -1140,14 +1154,11 @@ int launch_joined(JOIN const& join, operands_t op, const half_t* A, int M, int K
   *done = false;
   const device_state* ds = current_device_state();
   const workspace_t ws = workspace_for(st);
-  const size_t lhs_bytes = (size_t)M * K * 2, out_bytes = (size_t)M * N * 2;
   if (ds == nullptr || ws.ptr == nullptr || K % 128 != 0 || N % 2 != 0 || M < 2 || M > 64 ||
       (U8 && block_shift(block) < 0) || !scale_words_ok<U8>(op, K, N, block)) {
     return LCU_OK;
   }
-  for (const void* o : {(const void*)op.out, (const void*)op.more.out[0], (const void*)op.more.out[1], out}) {
-    if (o != nullptr && overlap(o, out_bytes, A, lhs_bytes)) return LCU_OK;
-  }
+  if (over_lhs(op, A, M, K, N) || (out != nullptr && overlap(out, (size_t)M * N * 2, A, (size_t)M * K * 2))) return LCU_OK;
   const skinny_plan_t plan = plan_skinny(M <= 32 || U8 ? 32 : 64, M, K, N, op.n_mats, ds->compute_units, ws.bytes);
   if (plan.splits == 0) return LCU_OK;
   const stream_join_t shape = plan_stream_join(M, K, N, op.n_mats, JOIN::MATRICES, plan.splits, ds->compute_units, U8);
@@ -1661,7 +1672,8 @@ int dispatch_gemm(operands_t op, const half_t* A, int M, int K, int N, int block
       // 24 KB a stage on their way into LDS bound it over a long K, and the rest is what it gains.  70 drawn products 0.91 of the time (0.82 to
       // 1.03), 45 in uint8 0.84 (0.79 to 0.88).
       // Smaller ones where these would leave compute units idle: 90 rows of 2048 columns eight fp16 layers 0.90 -> 0.71 ms.
-      const tile_size_t tile = plan_tile_size(M, N, op.n_mats, {128, 64}, !U8, cus);
+      // Outputs over lhs keep the tiles whose workgroup, where all columns are one tile, has read its rows before it stores them.
+      const tile_size_t tile = over_lhs(op, A, M, K, N) ? tile_size_t{128, 64} : plan_tile_size(M, N, op.n_mats, {128, 64}, !U8, cus);
       const f16_epilogue ep{};
       if constexpr (U8) {
         if (block_shift(block) < 0) return launch_dl<128, 64, 2, 2, 2, 3, true>(op, A, M, K, N, block, beta, st);
@@ -1766,13 +1778,8 @@ template <bool GATED>
 int bf16_joined(linear_epilogue<false, GATED> const& ep, const void* A, const void* W, int M, int K, int N, int splits, long cus, bool memory,
                 hipStream_t st, bool* done) {
   *done = false;
-  const size_t lhs_bytes = (size_t)M * K * 2;
   const int outs = GATED ? N / 2 : N;
-  if (K % 128 != 0 || (GATED && outs % 32 != 0) ||
-      overlap(ep.out, ((size_t)(M - 1) * ep.ldo + outs) * (ep.out_f32 ? 4 : 2), A, lhs_bytes) ||
-      (ep.tail && overlap(ep.tail, ((size_t)(M - 1) * ep.ld_tail + (N - ep.tail_from)) * 4, A, lhs_bytes))) {
-    return LCU_OK;
-  }
+  if (K % 128 != 0 || (GATED && outs % 32 != 0) || over_lhs(ep, A, M, K, N)) return LCU_OK;
   const int mats = GATED ? 2 : 1;
   const stream_join_t shape = plan_stream_join(M, K, outs, mats, mats, splits, cus, false);
   if (shape.waves == 0) return LCU_OK;
@@ -1848,7 +1855,8 @@ int gemm_bf16(linear_epilogue<false, GATED> const& ep, const void* A, const void
     }
     // us, on gemm_dl_kernel / here: 100x2048x2048 16.3 / 11.0, 200x4096x4096 29.4 / 20.9, 66x4096x8192 30.5 / 24.2
     const operands_t op = single_matrix(nullptr, W, nullptr);
-    if (plan_tile_size(M, N, 1, {64, 64}, true, cus).columns == 32) return launch_tile<64, 32, 1, 2, 4, 4, false, false>(ep, op, A, M, K, N, 0, 0.0f, st);
+    const tile_size_t tile = over_lhs(ep, A, M, K, N) ? tile_size_t{64, 64} : plan_tile_size(M, N, 1, {64, 64}, true, cus);  // over lhs: as in dispatch_gemm
+    if (tile.columns == 32) return launch_tile<64, 32, 1, 2, 4, 4, false, false>(ep, op, A, M, K, N, 0, 0.0f, st);
     return launch_tile<64, 64, 1, 4, 4, 4, false, false>(ep, op, A, M, K, N, 0, 0.0f, st);
   }
 }

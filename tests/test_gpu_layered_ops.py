@@ -179,6 +179,19 @@ def test_linear_smaller_tiles(gpu, M, K, N, tile):
     test_linear_large_tiles(gpu, M, K, N)
 
 
+# columns of one tile: the workgroup that stores rows has read them, so outputs may lie over lhs
+@pytest.mark.parametrize("M", [65, 300])
+def test_linear_of_few_columns_over_lhs(gpu, M):
+    rng = np.random.default_rng(M)
+    x, w = rounded(rng.standard_normal((M, 64))), rounded(rng.standard_normal((64, 64)) / 8)
+    xd, wd, out = put(gpu, x, BF16), put(gpu, w, BF16), zeros(gpu, (M, 64), BF16)
+    call(gpu, "lcu_linear", out, 0, 64, xd, wd, None, 0, BF16, M, 64, 64)
+    call(gpu, "lcu_linear", xd, 0, 64, xd, wd, None, 0, BF16, M, 64, 64)
+    assert np.array_equal(get(gpu, xd, (M, 64), BF16), get(gpu, out, (M, 64), BF16))
+    close(get(gpu, out, (M, 64), BF16), x @ w.T, BF16)
+    gpu.release()
+
+
 @pytest.mark.parametrize("M,K,ff,plan", [(1030, 1024, 6560, (192, 51, 9792, 128, 128)), (1025, 1024, 6750, (192, 51, 9792, 256, 128)),
                                          (1282, 2048, 6752, (256, 42, 10752, 128, 128)), (1990, 1024, 10980, (256, 64, 16384, 256, 192))])
 def test_gated_linear_columns_left_of_whole_rounds(gpu, M, K, ff, plan):

@@ -689,6 +689,25 @@ def test_gemm_smaller_tiles_of_one_round(gpu, u8, M, K, N, splits, tile):
     G.release()
 
 
+# products whose columns fit one tile of 64: the workgroup that stores rows has read them, so outputs may lie over lhs
+@pytest.mark.parametrize("M,K,N,at", [(100, 128, 64, 0), (128, 256, 64, 0), (65, 384, 33, 128), (90, 128, 50, 4096), (128, 512, 64, 65536)])
+@pytest.mark.parametrize("u8", [False, True])
+def test_gemm_of_few_columns_over_lhs(gpu, u8, M, K, N, at):
+    G = gpu
+    x, w = normal((M, K), 0, 460, 1.0), normal((N, K), 0, 461, 0.02)
+    if u8:
+        codes, scales = O.quantize_absmax_u8(w, 64)
+        want, args = G.gemm_u8(x, codes, scales, 64), (G.dev_keep(codes).ptr, G.dev_keep(scales).ptr)
+    else:
+        want, args = G.gemm_f16(x, w), (G.dev_keep(w).ptr,)
+    held = G.dev_keep(x)
+    call, tail = (G.L().lcu_gemm_f16u8_nt, (64, 0.0, None)) if u8 else (G.L().lcu_gemm_f16_nt, (0.0, None))
+    G.B.check(call(held.ptr + at, held.ptr, *args, M, K, N, *tail))
+    got = G.host(held, (M, K)).reshape(-1)[at // 2:at // 2 + M * N]
+    assert np.array_equal(got.view(np.uint16), want.reshape(-1).view(np.uint16))
+    G.release()
+
+
 def test_gemm_rejects_bad_shapes(gpu):
     G = gpu
     a = G.dev(np.zeros((4, 12), dtype=np.float16))
