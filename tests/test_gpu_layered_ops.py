@@ -463,6 +463,18 @@ def test_windowed_attention_key_sizes(gpu, dim, vdim):
     gpu.release()
 
 
+# values of 256 behind keys of up to 128, whose registers are cut to two wavefronts per SIMD, with and without a distance bias
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("dim,window,T", [(32, 90, 150), (64, 300, 193), (96, 10, 128), (128, 65, 257)])
+def test_windowed_attention_of_wide_values(gpu, dim, window, T, bias):
+    c = attention_case(gpu, BF16, 4, 2, dim, 200, window, 3, T, dim)
+    if not bias:
+        c["wp"].r1 = c["wp"].r2 = None
+        c["want"] = S.windowed_attention(c["q"][..., :dim], c["k"][..., :dim], c["v"][..., :200], c["wp"].scale, np.zeros(4), np.zeros(4), window, 3)
+    close(run_attention(gpu, c, BF16, (T,)), c["want"], BF16, bf16=2.0 ** -7)
+    gpu.release()
+
+
 # a maximum that grows from tile to tile by little (e in 100 keys), by more, by e^38, and one that falls
 @pytest.mark.parametrize("growth", [0.01, 0.08, 0.6, -0.3])
 @pytest.mark.parametrize("dim,vdim", [(64, 64), (192, 128)])
@@ -504,7 +516,7 @@ def test_windowed_attention_of_lowest_scores(gpu):
     gpu.release()
 
 
-# 768 workgroups and more: the form that fits three to a compute unit
+# more workgroups than the chip holds at once, 768 and beyond of rows that fill their tiles and rows that do not
 @pytest.mark.parametrize("heads,T", [(128, 384), (112, 390), (112, 449)])
 def test_windowed_attention_many_workgroups(gpu, heads, T):
     c = attention_case(gpu, BF16, heads, 4, 120, 128, 90, 3, T, heads)
