@@ -73,9 +73,9 @@ class pinned_buffer {
 // What the last launch of a one-token step leaves in page-locked memory, none of it ever -1, is watched for instead of waiting for the stream: expect()
 // before the launch, await() for the words.  hipStreamSynchronize returns 5 to 10 us after the word is there (a graph of 11 small launches
 // 36.7 us with it and 26.5 so, of 36 launches 76.5 and 68.6).  Calls of several tokens wait for the stream: whoever waits for it again afterwards, as
-// clear_tokens does, pays for that wait then (requests of one prompt of 512 tokens, width 512, 174 us with the watch, 150 without).  The words say nothing of what else the call's launches wrote: that is read behind
-// them on the same stream, or on another behind a wait for this one; what they read (page-locked input, a graph's arguments) is released or
-// freed behind such a wait too.
+// clear_tokens does, pays for that wait then (requests of one prompt of 512 tokens, width 512, 174 us with the watch, 150 without).  The words say
+// nothing of what else the call's launches wrote: that is read behind them on the same stream, or on another behind a wait for this one; what they
+// read (page-locked input, a graph's arguments) is released or freed behind such a wait too.
 // A watching thread is as busy as one in hipStreamSynchronize, which looks at the stream's signal all the while (1.2 cores either way), but gives its
 // core up to any other thread between two looks.  A launch that takes longer than `patience`, or failed, is left to the stream's own wait and its error.
 class awaited_words {
