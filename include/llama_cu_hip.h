@@ -67,8 +67,8 @@ int lcu_d2d(void* dst_dev, const void* src_dev, size_t bytes, void* stream);
 int lcu_stream_create(void** out_stream);
 int lcu_stream_destroy(void* stream);
 /* What a program knows and a single call cannot: the bytes of weights that the launches on a stream of lcu_stream_create go through before they
- * come to the same ones again (0, as it begins: unknown).  Products of few rows and of experts choose by it how weights are read, with the same
- * results; the contexts say what their models hold.  No counterpart in the reference. */
+ * come to the same ones again (0, as it begins: unknown).  Products of few rows, of experts and gated ones of few tiles choose by it how weights
+ * are read, with the same results; the contexts say what their models hold.  No counterpart in the reference. */
 int lcu_stream_weights(void* stream, size_t bytes);
 /* bounded in-launch waits that ran out on this stream's workspace so far (0 in any healthy run) */
 int lcu_sync_timeouts(void* stream, unsigned* out_count);
